@@ -133,6 +133,11 @@ int orx_arg_kind(orx_fn f, int index);
 int orx_launch(orx_fn f, const uint32_t grid[3], const uint32_t block[3], uint32_t shared_bytes,
                void* hip_stream, void** args);
 
+/* orx_launch with the geometry that orx_geometry() gives for the live rows, for a caller that launches from
+ * the handle and holds no record to be validated (one call per launch, the geometry worked out once).  Same
+ * checks of the arguments and rows, same results and error codes. */
+int orx_enqueue(orx_fn f, void* hip_stream, void** args);
+
 /* Size of the library's own scratch, one copy per device for the life of the process. */
 #define ORX_STATIC_SCRATCH_BYTES (64u << 20)
 

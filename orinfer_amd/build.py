@@ -1,7 +1,9 @@
-"""Builds liborx.so (HIP kernels + C ABI) for gfx950 with hipcc.  Usage: python -m orinfer_amd.build"""
+"""Builds liborx.so (HIP kernels + C ABI) for gfx950 with hipcc and _launcher.so (the launch path of lib.py) with g++.
+Usage: python -m orinfer_amd.build"""
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -18,6 +20,7 @@ FLAGS = [
     "-ffp-contract=off",
     "-Wall", "-Wno-unused-function", "-Wno-unknown-attributes", "-Wno-unused-command-line-argument",
 ]
+LAUNCHER = HERE / "_launcher.so"
 FIXTURE_RUNNER = HERE / "orx_run_fixture"
 
 
@@ -48,6 +51,11 @@ def build(verbose=True):
     if verbose:
         print(" ".join(link), flush=True)
     subprocess.check_call(link)
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f"-I{sysconfig.get_paths()['include']}",
+           str(CSRC / "launcher.cpp"), "-o", str(LAUNCHER), f"-L{HERE}", "-lorx", "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.check_call(cmd)
     runner_src = CSRC / "orx_run_fixture.cpp"
     if runner_src.exists():
         cmd = [hipcc(), "--offload-arch=gfx950", "-O2", "-std=c++17", "-x", "hip",

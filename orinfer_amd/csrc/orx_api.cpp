@@ -447,10 +447,9 @@ int resolve(const char* symbol, const char* variant_json, orx_fn* out) {
     return ORX_OK;
 }
 
-// Validates a launch against the record and returns the row count and geometry it runs with.
-int check_launch(const orx_function* f, const uint32_t grid[3], const uint32_t block[3], uint32_t shared_bytes,
-                 void** args, bool workspace_from_caller, int* rows_out, Geometry* want) {
-    if (f == nullptr || grid == nullptr || block == nullptr || args == nullptr) {
+// Checks a launch's arguments and rows and returns the row count and geometry it runs with.
+int check_arguments(const orx_function* f, void** args, bool workspace_from_caller, int* rows_out, Geometry* want) {
+    if (f == nullptr || args == nullptr) {
         set_error("orx_launch: null handle, geometry or argument list");
         return ORX_ERR_BAD_ARGUMENT;
     }
@@ -483,14 +482,25 @@ int check_launch(const orx_function* f, const uint32_t grid[3], const uint32_t b
             return ORX_ERR_ROWS;
         }
     }
-    int code = f->geometry(*f, rows, want);
+    *rows_out = rows;
+    return f->geometry(*f, rows, want);
+}
+
+// The same, and the record's geometry against the one the kernel needs.
+int check_launch(const orx_function* f, const uint32_t grid[3], const uint32_t block[3], uint32_t shared_bytes,
+                 void** args, bool workspace_from_caller, int* rows_out, Geometry* want) {
+    if (grid == nullptr || block == nullptr) {
+        set_error("orx_launch: null handle, geometry or argument list");
+        return ORX_ERR_BAD_ARGUMENT;
+    }
+    const int code = check_arguments(f, args, workspace_from_caller, rows_out, want);
     if (code != ORX_OK) return code;
     for (int i = 0; i < 3; ++i) {
         if (grid[i] != want->grid[i] || block[i] != want->block[i]) {
             set_error("launch %s: geometry grid(%u,%u,%u) block(%u,%u,%u) does not fit the kernel, which needs "
                       "grid(%u,%u,%u) block(%u,%u,%u) for %d rows",
                       f->symbol.c_str(), grid[0], grid[1], grid[2], block[0], block[1], block[2], want->grid[0],
-                      want->grid[1], want->grid[2], want->block[0], want->block[1], want->block[2], rows);
+                      want->grid[1], want->grid[2], want->block[0], want->block[1], want->block[2], *rows_out);
             return ORX_ERR_BAD_GEOMETRY;
         }
     }
@@ -498,7 +508,6 @@ int check_launch(const orx_function* f, const uint32_t grid[3], const uint32_t b
         set_error("launch %s: dynamic shared bytes %u, kernel needs %u", f->symbol.c_str(), shared_bytes, want->shared);
         return ORX_ERR_BAD_GEOMETRY;
     }
-    *rows_out = rows;
     return ORX_OK;
 }
 
@@ -525,6 +534,17 @@ void** expand_args(const orx_function* f, void** args, void** storage) {
 
 uint64_t workspace_need(const orx_function* f, int rows) {
     return f->takes_workspace && f->workspace_need != nullptr ? f->workspace_need(*f, rows) : 0;
+}
+
+// A checked launch with the Workspace the caller gave.
+int launch_checked(const orx_function* f, int rows, const Geometry& want, void* hip_stream, void** args) {
+    const uint64_t need = workspace_need(f, rows);
+    if (need != 0 && *reinterpret_cast<uint64_t*>(args[f->workspace_arg]) == 0) {
+        set_error("launch %s: %d rows need a Workspace of %llu bytes (orx_workspace_bytes), the buffer is null",
+                  f->symbol.c_str(), rows, (unsigned long long)need);
+        return (int)ORX_ERR_WORKSPACE;
+    }
+    return f->launch(*f, rows, want, reinterpret_cast<hipStream_t>(hip_stream), args);
 }
 
 }  // namespace
@@ -673,14 +693,18 @@ int orx_launch(orx_fn f, const uint32_t grid[3], const uint32_t block[3], uint32
         void* full[64];
         args = expand_args(f, args, full);
         const int code = check_launch(f, grid, block, shared_bytes, args, true, &rows, &want);
-        if (code != ORX_OK) return code;
-        const uint64_t need = workspace_need(f, rows);
-        if (need != 0 && *reinterpret_cast<uint64_t*>(args[f->workspace_arg]) == 0) {
-            set_error("launch %s: %d rows need a Workspace of %llu bytes (orx_workspace_bytes), the buffer is null",
-                      f->symbol.c_str(), rows, (unsigned long long)need);
-            return (int)ORX_ERR_WORKSPACE;
-        }
-        return f->launch(*f, rows, want, reinterpret_cast<hipStream_t>(hip_stream), args);
+        return code != ORX_OK ? code : launch_checked(f, rows, want, hip_stream, args);
+    });
+}
+
+int orx_enqueue(orx_fn f, void* hip_stream, void** args) {
+    return guard("orx_enqueue", [&, args]() mutable {
+        int rows = 0;
+        Geometry want;
+        void* full[64];
+        args = expand_args(f, args, full);
+        const int code = check_arguments(f, args, true, &rows, &want);
+        return code != ORX_OK ? code : launch_checked(f, rows, want, hip_stream, args);
     });
 }
 

@@ -11,7 +11,7 @@ import numpy as np
 import torch
 
 from . import codebook
-from .lib import ORX_ERR_BAD_VARIANT, Kernel, OrxError
+from .lib import ORX_ERR_BAD_VARIANT, Kernel, OrxError, current_stream
 
 
 def _dev(array):
@@ -55,6 +55,7 @@ class QuantizedLinear:
         else:
             self.projection = Kernel("int8_projection", **variant)
         self.workspace = self.projection.workspace()
+        self._live = self.out  # the rows of `out` that the last launch wrote (slicing costs 1 us of a 7 us call)
 
     def quantize(self, x16, stream=None):
         rows = x16.shape[0]
@@ -68,9 +69,14 @@ class QuantizedLinear:
         else:
             self.projection(stream=stream, A=self.a_q, Output=self.out, TokenScale=self.a_s, Weight=self.weight,
                             WeightScale=self.scales, Workspace=self.workspace, m=rows)
-        return self.out[:rows]
+        live = self._live
+        if live.shape[0] != rows:
+            live = self._live = self.out[:rows]
+        return live
 
     def run(self, x16, stream=None):
+        if stream is None:
+            stream = current_stream()
         return self.project(self.quantize(x16, stream), stream)
 
 
@@ -170,7 +176,7 @@ class MoeLayer:
         self.k_combine = Kernel("moe_combine", H=hidden, slots=assignments, **common)
 
     def run(self, x16, logits, stream=None):
-        s = stream
+        s = current_stream() if stream is None else stream
         if self.fused_stages:
             return self._run_fused(x16, logits, s)
         self.k_router(stream=s, IDs=self.ids, Logits=logits, Prob=self.prob)
@@ -271,7 +277,7 @@ class MoeTokenLayer:
                     raise
 
     def run(self, x16, logits, stream=None):
-        s = stream
+        s = current_stream() if stream is None else stream
         if self.fused:
             self.k_gate_up_routing(stream=s, A=x16, AS=self.a_s, Book=self.book, C=self.gate_up_out, IDs=self.ids,
                                    Logits=logits, P=self.w1, Prob=self.prob, WS=self.s1)

@@ -205,6 +205,23 @@ def test_launch_record_is_validated_before_anything_is_enqueued():
         assert err.value.code == lib.ORX_ERR_ROWS
 
 
+@pytest.mark.parametrize("values, code", [
+    (dict(m=0), "ORX_ERR_ROWS"), (dict(m=5), "ORX_ERR_ROWS"), (dict(m=-1), "ORX_ERR_ROWS"), (dict(m=2**32 + 5), "ORX_ERR_ROWS"),
+    (dict(A=None), "ORX_ERR_BAD_ARGUMENT"), (dict(W=257), "ORX_ERR_BAD_ARGUMENT"), (dict(Q=256), "ORX_ERR_BAD_ARGUMENT"),
+])
+def test_a_named_launch_is_checked_before_anything_is_enqueued(values, code):
+    """Kernel.__call__ goes through orx_enqueue: the argument, row and name checks of the record launch."""
+    kernel = lib.Kernel("e8p_q4_projection", M=4, N=256, K=256, dynamic_rows=True)
+    named = {**{name: 256 for name in kernel.arg_names}, "m": 4, **values}
+    with pytest.raises(lib.OrxError) as err:
+        kernel(stream=0, **named)
+    assert err.value.code == getattr(lib, code)
+    with pytest.raises(lib.OrxError) as err:
+        kernel(stream=0, **{k: v for k, v in named.items() if k != "A"})
+    assert err.value.code == lib.ORX_ERR_BAD_ARGUMENT
+    assert lib.library().orx_enqueue(None, None, None) == lib.ORX_ERR_BAD_ARGUMENT
+
+
 def test_handles_own_no_device_memory_and_say_what_workspace_they_need():
     """orx_resolve allocates nothing: scratch is a `Workspace` buffer the engine sizes from
     orx_workspace_bytes (AGENTS.md:41: the engine owns every buffer).  A thousand handles resolve in
