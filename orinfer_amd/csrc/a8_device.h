@@ -51,13 +51,35 @@ __device__ __forceinline__ uint32_t quantise4(const float (&value)[4], float sca
     return low | (high << 16);
 }
 
-// fp16(silu(gate) * up) in fp32 with a stable sigmoid (kernels/cuda/operators/op04_swiglu.py:6-17).
+// A stable sigmoid in fp32: e = exp(-|gate|), (gate >= 0 ? 1 : e) / (1 + e).  exp(x) = 2^(x log2 e): the hardware
+// exponential of the rounded product, corrected to first order by what the rounding took off (one fused multiply-add
+// recovers it: x - t ln 2), so it is good to one unit in the last place.  The quotient is the reciprocal with one Newton step
+// and one residual correction (Markstein's division): correctly rounded up to rare ties, for a denominator in
+// [1, 2].  Below -87 the exponential would leave the normal numbers and no product with two fp16 values of it rounds
+// to anything but 0, so the argument stops there.  Fifteen instructions, two of them transcendental, where the library
+// exponential and quotient took about thirty (8192 rows of 17408 values were bound by them).
+__device__ __forceinline__ float sigmoid_value(float gate) {
+    const float x = fmaxf(-fabsf(gate), -87.f);
+    const float t = x * 1.44269502162933349609375f;                       // fp32(log2 e)
+    const float rest = __builtin_fmaf(-t, 0.693147182464599609375f, x);   // fp32(ln 2)
+    const float power = __builtin_amdgcn_exp2f(t);
+    const float e = __builtin_fmaf(power, rest, power);
+    const float denominator = 1.0f + e, numerator = gate >= 0.f ? 1.0f : e;
+    const float guess = __builtin_amdgcn_rcpf(denominator);
+    const float reciprocal = __builtin_fmaf(__builtin_fmaf(-denominator, guess, 1.0f), guess, guess);
+    const float quotient = numerator * reciprocal;
+    return __builtin_fmaf(__builtin_fmaf(-denominator, quotient, numerator), reciprocal, quotient);
+}
+
+// fp16(silu(gate) * up) (kernels/cuda/operators/op04_swiglu.py:6-17).
 __device__ __forceinline__ float swiglu_value(__half gate, __half up) {
     const float g = __half2float(gate), u = __half2float(up);
-    const float e = expf(-fabsf(g));
-    const float sigmoid = __fdiv_rn(g >= 0.f ? 1.0f : e, 1.0f + e);  // one division serves both signs of the gate
-    // one fp16 rounding here: the value a downstream quantiser sees is the materialised fp16
-    return __half2float(__float2half_rn((g * sigmoid) * u));
+    float value = (g * sigmoid_value(g)) * u;
+    // opaque: the fp32 product rounds, then the fp16 cast does (a fused multiply-convert rounds once, and which of the
+    // two the compiler takes would differ between the kernels that share this)
+    asm("" : "+v"(value));
+    // the value a downstream quantiser sees is the materialised fp16
+    return __half2float(__float2half_rn(value));
 }
 
 // ---- nibble planes ------------------------------------------------------------------------------

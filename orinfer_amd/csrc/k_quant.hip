@@ -5,7 +5,7 @@
 // code = clamp(rint(x / fp32(scale)), -127, 127) with a correctly rounded divide and
 // ties-to-even (:14-18, :49-65, contract text :71-78).  `fused` quantises
 // fp16(silu(gate)*up) read from X[rows, 2K] (:43-46, op04_swiglu.py:6-17).
-// The kernel is memory-bound: one fp16 read (twice, second pass from L2) and one int8 write.
+// The kernel is memory-bound: one fp16 read and one int8 write.
 //
 // rotate_activation_a8 follows kernels/cuda/model/rotation_a8.py:188-224,369-383: x * sign, seven
 // butterfly stages inside every block of 128 channels in fp32, one multiply by fp32(128^-1/2), an
@@ -50,86 +50,116 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
     return r;
 }
 
-// grid (rows, groups), 256 threads.  STAGED (dynamic LDS of one group of fp16 values): a thread keeps
-// the 16-byte pieces it read for the maximum in LDS and quantises them from there.  With many rows
-// of long groups in flight the second read no longer hits the L2 cache (8192 rows of 17408: every
-// CU holds 8 rows of 34 KB), so it would cost HBM traffic a second time.
-template <bool FUSED, bool MASKED, int THREADS = 256, bool STAGED = false>
-__global__ __launch_bounds__(THREADS) void a8_kernel(const __half* __restrict__ x, const uint8_t* __restrict__ mask,
-                                                     int8_t* __restrict__ q, __half* __restrict__ s, int k, int group,
-                                                     int groups) {
-    extern __shared__ __align__(16) uint4 staged[];
-    __shared__ float scratch[THREADS / 64];
+// Masked rows and groups longer than the held form takes: two passes over the group, grid (rows, groups).
+template <bool FUSED, bool MASKED>
+__global__ __launch_bounds__(256) void a8_kernel(const __half* __restrict__ x, const uint8_t* __restrict__ mask,
+                                                 int8_t* __restrict__ q, __half* __restrict__ s, int k, int group,
+                                                 int groups) {
+    __shared__ float scratch[4];
     const int row = blockIdx.x, g = blockIdx.y;
     const int first = g * group;
     const int width = min(group, k - first);
     const int64_t in_base = (int64_t)row * (FUSED ? 2 * k : k);
     const int64_t out_base = (int64_t)row * k;
-    // 8 halves per thread per step when everything is 16-byte aligned and unmasked/unfused
-    const bool vector = !FUSED && !MASKED && (k % 8 == 0) && (group % 8 == 0) &&
-                        ((reinterpret_cast<uintptr_t>(x) & 15) == 0) && ((reinterpret_cast<uintptr_t>(q) & 7) == 0);
     float amax = 0.f;
-    typedef _Float16 half_pair __attribute__((ext_vector_type(2)));
-    half_pair amax2 = {(_Float16)0.f, (_Float16)0.f};  // largest magnitudes so far as two fp16 lanes: comparing needs no conversion
-    // a group of at most one 16-byte piece per thread stays in registers between the two passes
-    // (only in the 16-wave form: carrying the piece through the loops costs the 4-wave form its
-    // overlap of loads, 28 -> 48 us at 8192 x 5120)
-    const bool held = THREADS == 1024 && vector && width / 8 <= THREADS;
-    uint4 kept = make_uint4(0u, 0u, 0u, 0u);
-    if (STAGED && vector) {
-        // four pieces per thread leave together (clamped, so unconditional): a long group would
-        // otherwise cost one load latency per piece
-        const uint4* src = reinterpret_cast<const uint4*>(x + in_base + first);
-        const int pieces = width / 8;
-        for (int base = threadIdx.x; base < pieces; base += 4 * THREADS) {
-            uint4 raw[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) raw[u] = src[min(base + u * THREADS, pieces - 1)];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int i = base + u * THREADS;
-                if (i < pieces) staged[i] = raw[u];  // read back below by this thread only
-                const uint32_t words[4] = {raw[u].x, raw[u].y, raw[u].z, raw[u].w};
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    amax2 = __builtin_elementwise_max(amax2, __builtin_bit_cast(half_pair, words[j] & 0x7FFF7FFFu));
-            }
-        }
-        amax = fmaxf((float)amax2[0], (float)amax2[1]);
-    } else if (vector) {
-        const uint4* src = reinterpret_cast<const uint4*>(x + in_base + first);
-        for (int i = threadIdx.x; i < width / 8; i += blockDim.x) {
-            const uint4 raw = src[i];
-            if (THREADS == 1024) kept = raw;
-            const uint32_t words[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                amax2 = __builtin_elementwise_max(amax2, __builtin_bit_cast(half_pair, words[j] & 0x7FFF7FFFu));
-        }
-        amax = fmaxf((float)amax2[0], (float)amax2[1]);
-    } else {
-        for (int i = threadIdx.x; i < width; i += blockDim.x)
-            amax = fmaxf(amax, fabsf(load_value<FUSED, MASKED>(x, mask, in_base, k, first + i)));
-    }
+    for (int i = threadIdx.x; i < width; i += 256)
+        amax = fmaxf(amax, fabsf(load_value<FUSED, MASKED>(x, mask, in_base, k, first + i)));
     amax = block_max(amax, scratch);
-    const float raw_scale = fmaxf(__fdiv_rn(amax, 127.0f), 5.9604644775390625e-08f);
-    const __half stored = amax > 0.f ? __float2half_rn(raw_scale) : __float2half_rn(1.0f);
+    const __half stored = a8_scale(amax);
     if (threadIdx.x == 0) s[(int64_t)row * groups + g] = stored;
     const float scale = __half2float(stored);
     const float inverse = __frcp_rn(scale);
+    for (int i = threadIdx.x; i < width; i += 256)
+        q[out_base + first + i] = quantise(load_value<FUSED, MASKED>(x, mask, in_base, k, first + i), scale, inverse);
+}
+
+// One pass: WAVES waves hold a (row, group) in registers as 16-byte pieces of eight fp16 values, PIECES to a lane,
+// between the maximum and the codes; FUSED values are fp16(silu(gate) * up), computed once.  All loads of a wave leave
+// together.  One wave needs no barrier (four groups to a workgroup then); more waves meet once, for the maximum.
+// What bounds it: memory with many rows (8192 x 4096: 28.1 -> 20.7 us, 4.9 TB/s; the two-pass kernel read every row twice),
+// the vector ALU beside it in the FUSED form (8192 x 17408: 416 -> 148 us; the two-pass kernel also computed every value
+// twice), the latency of one row's loads and reductions with few (FUSED, one row of 17408: 43 -> 6.3 us).
+template <bool FUSED, int WAVES, int PIECES>
+__global__ __launch_bounds__(WAVES == 1 ? 256 : 64 * WAVES) void a8_held_kernel(const __half* __restrict__ x,
+                                                                                int8_t* __restrict__ q,
+                                                                                __half* __restrict__ s, int k, int group,
+                                                                                int groups, int rows) {
+    constexpr int kLanes = 64 * WAVES;
+    typedef _Float16 half_pair __attribute__((ext_vector_type(2)));
+    typedef uint32_t word4 __attribute__((ext_vector_type(4)));
+    __shared__ float scratch[WAVES];
+    const int lane = WAVES == 1 ? threadIdx.x & 63 : threadIdx.x;
+    const int unit = WAVES == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;  // wave-uniform
+    if (unit >= rows * groups) return;  // only with one wave to a unit: nothing below waits for it
+    const int row = unit / groups, g = unit % groups;
+    const int first = g * group;
+    const int width = min(group, k - first);
+    const int64_t in_base = (int64_t)row * (FUSED ? 2 * k : k);
+    const int64_t out_base = (int64_t)row * k;
+    const bool vector = (k % 8 == 0) && (group % 8 == 0) && ((reinterpret_cast<uintptr_t>(x) & 15) == 0) &&
+                        ((reinterpret_cast<uintptr_t>(q) & 7) == 0);
+    word4 held[PIECES];
+    const int pieces = width / 8;
+    float amax = 0.f;
     if (vector) {
-        const uint4* src = reinterpret_cast<const uint4*>(x + in_base + first);
+        const word4* src = reinterpret_cast<const word4*>(x + in_base + first);
+        word4 up[FUSED ? PIECES : 1];
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) {  // clamped, so unconditional
+            const int i = min(lane + p * kLanes, pieces - 1);
+            held[p] = src[i];
+            if (FUSED) up[p] = *reinterpret_cast<const word4*>(x + in_base + k + first + 8 * i);
+        }
+        half_pair largest = {(_Float16)0.f, (_Float16)0.f};  // magnitudes as two fp16 lanes: comparing needs no conversion
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) {
+            if (lane + p * kLanes < pieces) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (FUSED) {
+                        const __half2 gate = __builtin_bit_cast(__half2, (uint32_t)held[p][j]);
+                        const __half2 value = __builtin_bit_cast(__half2, (uint32_t)up[p][j]);
+                        const half_pair pair = {(_Float16)swiglu_value(__low2half(gate), __low2half(value)),
+                                                (_Float16)swiglu_value(__high2half(gate), __high2half(value))};
+                        held[p][j] = __builtin_bit_cast(uint32_t, pair);
+                    }
+                    largest = __builtin_elementwise_max(largest, __builtin_bit_cast(half_pair, held[p][j] & 0x7FFF7FFFu));
+                }
+            }
+        }
+        amax = fmaxf((float)largest[0], (float)largest[1]);
+    } else {
+        for (int i = lane; i < width; i += kLanes)
+            amax = fmaxf(amax, fabsf(load_value<FUSED, false>(x, nullptr, in_base, k, first + i)));
+    }
+    if (WAVES == 1) {
+#pragma unroll
+        for (int offset = 32; offset > 0; offset >>= 1) amax = fmaxf(amax, __shfl_xor(amax, offset, 64));
+    } else {
+        amax = block_max(amax, scratch);
+    }
+    const __half stored = a8_scale(amax);
+    if (lane == 0) s[(int64_t)row * groups + g] = stored;
+    const float scale = __half2float(stored);
+    const float inverse = __frcp_rn(scale);
+    if (vector) {
         uint2* dst = reinterpret_cast<uint2*>(q + out_base + first);
-        for (int i = threadIdx.x; i < width / 8; i += blockDim.x) {
-            const uint4 raw = held ? kept : STAGED ? staged[i] : src[i];
-            const __half* h = reinterpret_cast<const __half*>(&raw);
-            const float low[4] = {__half2float(h[0]), __half2float(h[1]), __half2float(h[2]), __half2float(h[3])};
-            const float high[4] = {__half2float(h[4]), __half2float(h[5]), __half2float(h[6]), __half2float(h[7])};
-            dst[i] = make_uint2(quantise4(low, scale, inverse), quantise4(high, scale, inverse));
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) {
+            if (lane + p * kLanes < pieces) {
+                float value[8];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const half_pair pair = __builtin_bit_cast(half_pair, (uint32_t)held[p][j]);
+                    value[2 * j] = (float)pair[0], value[2 * j + 1] = (float)pair[1];
+                }
+                const float low[4] = {value[0], value[1], value[2], value[3]}, high[4] = {value[4], value[5], value[6], value[7]};
+                dst[lane + p * kLanes] = make_uint2(quantise4(low, scale, inverse), quantise4(high, scale, inverse));
+            }
         }
     } else {
-        for (int i = threadIdx.x; i < width; i += blockDim.x)
-            q[out_base + first + i] = quantise(load_value<FUSED, MASKED>(x, mask, in_base, k, first + i), scale, inverse);
+        for (int i = lane; i < width; i += kLanes)
+            q[out_base + first + i] = quantise(load_value<FUSED, false>(x, nullptr, in_base, k, first + i), scale, inverse);
     }
 }
 
@@ -193,58 +223,6 @@ __device__ __forceinline__ void quantise_row(const __half* rotated, float amax, 
         const __half* h = reinterpret_cast<const __half*>(&raw);
         const float values[4] = {__half2float(h[0]), __half2float(h[1]), __half2float(h[2]), __half2float(h[3])};
         *reinterpret_cast<uint32_t*>(q + (int64_t)row * k + 4 * i) = quantise4(values, scale, inverse);
-    }
-}
-
-// Short groups (at most 512 values): one wave per (row, group), four per workgroup, a lane holds one
-// 16-byte piece; the maximum is a wave reduction, so there is no barrier and no second read.
-template <bool FUSED>
-__global__ __launch_bounds__(256) void a8_wave_kernel(const __half* __restrict__ x, int8_t* __restrict__ q,
-                                                      __half* __restrict__ s, int k, int group, int groups, int rows) {
-    const int lane = threadIdx.x & 63;
-    const int unit = blockIdx.x * 4 + (threadIdx.x >> 6);  // wave-uniform
-    if (unit >= rows * groups) return;
-    const int row = unit / groups, g = unit % groups;
-    const int first = g * group;
-    const int width = min(group, k - first);
-    const int64_t in_base = (int64_t)row * (FUSED ? 2 * k : k);
-    const int64_t out_base = (int64_t)row * k;
-    const bool vector = (k % 8 == 0) && (group % 8 == 0) && ((reinterpret_cast<uintptr_t>(x) & 15) == 0) &&
-                        ((reinterpret_cast<uintptr_t>(q) & 7) == 0);
-    float value[8];
-    float amax = 0.f;
-    if (vector) {
-        const bool live = lane < width / 8;
-        const int piece = live ? lane : 0;
-        const uint4 raw = *reinterpret_cast<const uint4*>(x + in_base + first + 8 * piece);
-        uint4 raw_up = make_uint4(0u, 0u, 0u, 0u);
-        if (FUSED) raw_up = *reinterpret_cast<const uint4*>(x + in_base + k + first + 8 * piece);
-        const __half* h = reinterpret_cast<const __half*>(&raw);
-        const __half* up = reinterpret_cast<const __half*>(&raw_up);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            value[j] = FUSED ? swiglu_value(h[j], up[j]) : __half2float(h[j]);
-            if (live) amax = fmaxf(amax, fabsf(value[j]));
-        }
-    } else {
-        for (int i = lane; i < width; i += 64) amax = fmaxf(amax, fabsf(load_value<FUSED, false>(x, nullptr, in_base, k, first + i)));
-    }
-#pragma unroll
-    for (int offset = 32; offset > 0; offset >>= 1) amax = fmaxf(amax, __shfl_xor(amax, offset, 64));
-    const float raw_scale = fmaxf(__fdiv_rn(amax, 127.0f), 5.9604644775390625e-08f);
-    const __half stored = amax > 0.f ? __float2half_rn(raw_scale) : __float2half_rn(1.0f);
-    if (lane == 0) s[(int64_t)row * groups + g] = stored;
-    const float scale = __half2float(stored);
-    const float inverse = __frcp_rn(scale);
-    if (vector) {
-        if (lane < width / 8) {
-            const float low[4] = {value[0], value[1], value[2], value[3]}, high[4] = {value[4], value[5], value[6], value[7]};
-            *reinterpret_cast<uint2*>(q + out_base + first + 8 * lane) =
-                make_uint2(quantise4(low, scale, inverse), quantise4(high, scale, inverse));
-        }
-    } else {
-        for (int i = lane; i < width; i += 64)
-            q[out_base + first + i] = quantise(load_value<FUSED, false>(x, nullptr, in_base, k, first + i), scale, inverse);
     }
 }
 
@@ -482,35 +460,46 @@ __global__ __launch_bounds__(256) void rotate_kernel(const __half* __restrict__ 
     }
 }
 
+template <int WAVES>
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
 #pragma unroll
     for (int offset = 32; offset > 0; offset >>= 1) v += __shfl_xor(v, offset, 64);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (lane == 0) scratch[wave] = v;
     __syncthreads();
-    return (scratch[0] + scratch[1]) + (scratch[2] + scratch[3]);
+    float part[WAVES];
+#pragma unroll
+    for (int i = 0; i < WAVES; ++i) part[i] = scratch[i];
+#pragma unroll
+    for (int half = 1; half < WAVES; half *= 2)
+#pragma unroll
+        for (int i = 0; i < WAVES; i += 2 * half) part[i] += part[i + half];
+    return part[0];
 }
 
 // Residual add + RMSNorm in front of the rotation, one workgroup per row, same lane layout as
 // rotate_a8_kernel.  First pass: RO = fp32(X) + R, sum of squares.  Second pass: the fp32 sum (kept
 // in registers, or read back by the thread that wrote it where the row is longer than the registers
 // hold), Y = fp16((sum * rsqrt(mean + eps)) * (W + offset)), and that fp16 value goes through signs,
-// butterflies and A8 as if rotate_a8_kernel had read Y.
-__global__ __launch_bounds__(256) void residual_norm_rotate_a8_kernel(
+// butterflies and A8 as if rotate_a8_kernel had read Y.  4 waves (16 when rows are few, as in rotate_a8_kernel: one row
+// of 5120 then takes 4.8 us instead of 7.0, twenty 5.1 instead of 7.7).
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void residual_norm_rotate_a8_kernel(
     const __half* __restrict__ x, const float* __restrict__ r, const __half* __restrict__ w, __half* __restrict__ y,
     float* __restrict__ ro, const int8_t* __restrict__ signs, int8_t* __restrict__ q, __half* __restrict__ s, int k,
     float epsilon, float weight_offset) {
     extern __shared__ __align__(16) __half rotated[];  // k halves
-    __shared__ float scratch[4], sum_scratch[4];
+    constexpr int kWaves = THREADS / 64;
+    __shared__ float scratch[kWaves], sum_scratch[kWaves];
     const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int half_wave = lane >> 5, l32 = lane & 31;
     const int blocks = k / 128;  // even: k is a multiple of 256
     const int64_t base = (int64_t)row * k;
     float squares = 0.f;
-    // The first kHeld steps of a wave (all of them up to K = 5120): every load of both passes leaves
+    // The first kHeld steps of a wave (all of them up to K = 5120, 8192 with 16 waves): every load of both passes leaves
     // at once, and the fp32 sums stay in registers for the second pass.  Longer rows go on in the
     // loops below, which read their sums back.
-    constexpr int kHeld = 5;
+    constexpr int kHeld = THREADS == 256 ? 5 : 2;
     float4 kept[kHeld];
     uint2 held_w[kHeld];
     uint32_t held_sign[kHeld];
@@ -519,7 +508,7 @@ __global__ __launch_bounds__(256) void residual_norm_rotate_a8_kernel(
         float4 residual[kHeld];
 #pragma unroll
         for (int u = 0; u < kHeld; ++u) {  // clamped, so unconditional (blocks is even: a pair is live or not as a whole)
-            const int first = (min(2 * (wave + 4 * u), blocks - 2) + half_wave) * 128 + 4 * l32;
+            const int first = (min(2 * (wave + kWaves * u), blocks - 2) + half_wave) * 128 + 4 * l32;
             raw[u] = *reinterpret_cast<const uint2*>(x + base + first);
             residual[u] = *reinterpret_cast<const float4*>(r + base + first);
             held_w[u] = *reinterpret_cast<const uint2*>(w + first);
@@ -527,8 +516,8 @@ __global__ __launch_bounds__(256) void residual_norm_rotate_a8_kernel(
         }
 #pragma unroll
         for (int u = 0; u < kHeld; ++u) {
-            if (2 * (wave + 4 * u) >= blocks) break;  // wave-uniform
-            const int first = (2 * (wave + 4 * u) + half_wave) * 128 + 4 * l32;
+            if (2 * (wave + kWaves * u) >= blocks) break;  // wave-uniform
+            const int first = (2 * (wave + kWaves * u) + half_wave) * 128 + 4 * l32;
             const __half* h = reinterpret_cast<const __half*>(&raw[u]);
             float4 sum;
             sum.x = __half2float(h[0]) + residual[u].x;
@@ -543,7 +532,7 @@ __global__ __launch_bounds__(256) void residual_norm_rotate_a8_kernel(
             squares += sum.w * sum.w;
         }
     }
-    for (int pair = wave + 4 * kHeld; 2 * pair < blocks; pair += 4) {
+    for (int pair = wave + kWaves * kHeld; 2 * pair < blocks; pair += kWaves) {
         const int first = (2 * pair + half_wave) * 128 + 4 * l32;
         const uint2 raw = *reinterpret_cast<const uint2*>(x + base + first);
         const __half* h = reinterpret_cast<const __half*>(&raw);
@@ -559,7 +548,7 @@ __global__ __launch_bounds__(256) void residual_norm_rotate_a8_kernel(
         squares += sum.z * sum.z;
         squares += sum.w * sum.w;
     }
-    const float total = block_sum(squares, sum_scratch);
+    const float total = block_sum<kWaves>(squares, sum_scratch);
     const float inverse = rsqrtf(__fdiv_rn(total, (float)k) + epsilon);
     float amax = 0.f;
     auto second_pass = [&](int first, const float4& sum, const uint2& raw_w, uint32_t sign_word) {
@@ -583,10 +572,10 @@ __global__ __launch_bounds__(256) void residual_norm_rotate_a8_kernel(
     };
 #pragma unroll
     for (int u = 0; u < kHeld; ++u) {
-        if (2 * (wave + 4 * u) >= blocks) break;  // wave-uniform
-        second_pass((2 * (wave + 4 * u) + half_wave) * 128 + 4 * l32, kept[u], held_w[u], held_sign[u]);
+        if (2 * (wave + kWaves * u) >= blocks) break;  // wave-uniform
+        second_pass((2 * (wave + kWaves * u) + half_wave) * 128 + 4 * l32, kept[u], held_w[u], held_sign[u]);
     }
-    for (int pair = wave + 4 * kHeld; 2 * pair < blocks; pair += 4) {
+    for (int pair = wave + kWaves * kHeld; 2 * pair < blocks; pair += kWaves) {
         const int first = (2 * pair + half_wave) * 128 + 4 * l32;
         const float4 sum = *reinterpret_cast<const float4*>(ro + base + first);  // written above by this thread
         const uint2 raw_w = *reinterpret_cast<const uint2*>(w + first);
@@ -664,26 +653,51 @@ __global__ __launch_bounds__(256) void swiglu_kernel(const __half* __restrict__ 
 
 // ---- host side -----------------------------------------------------------------------------
 // slots used: K, group, flags (bit0 masked, bit1 fused), capacity
-// few rows of long groups (decode): 16 waves per group, one 16-byte piece per thread
-bool a8_wide(const orx_function& f, int rows) { return f.flags == 0 && rows <= 256 && f.group >= 4096; }
-// short groups, no mask: one wave per group
-bool a8_per_wave(const orx_function& f) { return !(f.flags & 1) && f.group <= 512; }
-// many rows of long groups: the pieces wait in LDS between the two passes (9 to 48 KiB per group: at least three of the four pieces a thread requests at once are real)
-bool a8_staged(const orx_function& f, int rows) {
-    return f.flags == 0 && !a8_wide(f, rows) && f.group % 8 == 0 && f.group >= 4608 && f.group <= 24576;
+// The forms of a8_held_kernel: waves to a group, pieces of eight values to a lane.
+struct HeldForm {
+    int waves, pieces;
+    const void *plain, *fused;
+};
+const HeldForm* held_forms(int* count) {
+#define ORX_HELD(W, P)                                                                                             \
+    {W, P, reinterpret_cast<const void*>(&a8_held_kernel<false, W, P>), reinterpret_cast<const void*>(&a8_held_kernel<true, W, P>)}
+    static const HeldForm forms[] = {ORX_HELD(1, 1), ORX_HELD(1, 2), ORX_HELD(1, 4), ORX_HELD(4, 1), ORX_HELD(4, 2),
+                                     ORX_HELD(4, 3), ORX_HELD(4, 4), ORX_HELD(4, 6), ORX_HELD(8, 1), ORX_HELD(8, 2),
+                                     ORX_HELD(8, 3), ORX_HELD(8, 5), ORX_HELD(8, 8)};
+#undef ORX_HELD
+    *count = (int)(sizeof forms / sizeof forms[0]);
+    return forms;
+}
+
+// The form a launch takes, or null for the general kernel (a mask, groups beyond 32768 values).  Measured (us, FUSED in
+// brackets), 1 / 4 / 8 waves to a row: 8192 rows of 1024 7.3 / 10.9 / 19.7, of 2048 11.7 / 13.4 / 21.6 (with so many
+// rows the rate at which workgroups start is the limit, so a wave takes a whole row as long as four pieces to a
+// lane hold it), of 5120 - / 23 / 30 (- / 45 / 51); 4096 rows of 17408 - / 37 / 37 (- / 80 / 75); one row of 17408 - / 4.6 / 3.8
+// (- / 7.4 / 6.3); 200 rows of 5120 - / 3.8 / 3.6.  Sixteen waves were nowhere more than 0.1 us better.
+const HeldForm* held_form(const orx_function& f, int rows) {
+    if (f.flags & 1) return nullptr;
+    const int pieces = (f.group + 7) / 8;
+    const int64_t units = (int64_t)rows * ((f.K + f.group - 1) / f.group);
+    const int waves = pieces <= 64 || (pieces <= 256 && units >= 2048) ? 1
+                      : pieces > 1536 || (pieces > 256 && units <= 512) ? 8 : 4;
+    int count = 0;
+    const HeldForm* forms = held_forms(&count);
+    for (int i = 0; i < count; ++i)
+        if (forms[i].waves == waves && forms[i].pieces * 64 * waves >= pieces) return &forms[i];
+    return nullptr;
 }
 
 int a8_geometry(const orx_function& f, int rows, Geometry* g) {
     const uint32_t groups = ceil_div((uint32_t)f.K, (uint32_t)f.group);
-    if (a8_per_wave(f)) {
-        g->grid[0] = ceil_div((uint32_t)rows * groups, 4u);
-        g->block[0] = 256;
+    if (const HeldForm* form = held_form(f, rows)) {
+        const uint32_t waves = (uint32_t)form->waves, units = (uint32_t)rows * groups;
+        g->grid[0] = waves == 1 ? ceil_div(units, 4u) : units;
+        g->block[0] = waves == 1 ? 256 : 64 * waves;
         return ORX_OK;
     }
     g->grid[0] = (uint32_t)rows;
     g->grid[1] = groups;
-    g->block[0] = a8_wide(f, rows) ? 1024 : 256;
-    g->shared = a8_staged(f, rows) ? (uint32_t)f.group * 2u : 0u;
+    g->block[0] = 256;
     return ORX_OK;
 }
 
@@ -692,19 +706,14 @@ int a8_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t st
     int8_t* q = pointer_arg<int8_t>(args, 1);
     __half* s = pointer_arg<__half>(args, 2);
     const __half* x = pointer_arg<const __half>(args, 3);
-    const dim3 grid(g.grid[0], g.grid[1]), block(256);
+    const dim3 grid(g.grid[0], g.grid[1]), block(g.block[0]);
     const int groups = (int)ceil_div((uint32_t)f.K, (uint32_t)f.group);
     const bool masked = f.flags & 1, fused = f.flags & 2;
-    if (a8_per_wave(f)) {
-        if (fused)
-            ORX_LAUNCH((a8_wave_kernel<true>), grid, block, 0, stream, x, q, s, f.K, f.group, groups, rows);
-        else
-            ORX_LAUNCH((a8_wave_kernel<false>), grid, block, 0, stream, x, q, s, f.K, f.group, groups, rows);
-    } else if (g.block[0] == 1024)
-        ORX_LAUNCH((a8_kernel<false, false, 1024>), grid, dim3(1024), 0, stream, x, mask, q, s, f.K, f.group, groups);
-    else if (g.shared > 0)
-        ORX_LAUNCH((a8_kernel<false, false, 256, true>), grid, block, g.shared, stream, x, mask, q, s, f.K, f.group, groups);
-    else if (fused && masked)
+    if (const HeldForm* form = held_form(f, rows)) {
+        typedef void (*Held)(const __half*, int8_t*, __half*, int, int, int, int);
+        const Held kernel = reinterpret_cast<Held>(const_cast<void*>(fused ? form->fused : form->plain));
+        ORX_LAUNCH(kernel, grid, block, 0, stream, x, q, s, f.K, f.group, groups, rows);
+    } else if (fused && masked)
         ORX_LAUNCH((a8_kernel<true, true>), grid, block, 0, stream, x, mask, q, s, f.K, f.group, groups);
     else if (fused)
         ORX_LAUNCH((a8_kernel<true, false>), grid, block, 0, stream, x, mask, q, s, f.K, f.group, groups);
@@ -738,7 +747,7 @@ int make_a8(const Variant& v, orx_function* f) {
     // Mask may be null unless masked (the reference ignores it then, op30:75-76)
     f->args = {{"Mask", ArgPointer, masked ? 1u : 0x80000001u}, {"Q", ArgPointer, 1}, {"S", ArgPointer, 2},
                {"X", ArgPointer, 2}, {"rows", ArgI32, 4}};
-    f->device_function = nullptr;  // kernels with 256 and 1024 threads serve this symbol
+    f->device_function = nullptr;  // the kernel follows the rows and the group
     f->geometry = a8_geometry;
     f->launch = a8_launch;
     return ORX_OK;
@@ -946,7 +955,7 @@ int make_rotate(const Variant& v, orx_function* f) {
 // slots used: K, flags (bit0: weights stored zero-centred), capacity
 int residual_rotate_geometry(const orx_function& f, int rows, Geometry* g) {
     g->grid[0] = (uint32_t)rows;
-    g->block[0] = 256;
+    g->block[0] = rows <= kRotateWideRows && f.K >= 2048 ? 1024 : 256;
     g->shared = (uint32_t)f.K * 2;
     return ORX_OK;
 }
@@ -962,8 +971,13 @@ int residual_rotate_launch(const orx_function& f, int rows, const Geometry& g, h
     const __half* w = pointer_arg<const __half>(args, 5);
     const __half* x = pointer_arg<const __half>(args, 6);
     __half* y = pointer_arg<__half>(args, 7);
-    ORX_LAUNCH(residual_norm_rotate_a8_kernel, dim3(g.grid[0]), dim3(256), g.shared, stream, x, r, w, y, ro, signs,
-                       q, s, f.K, 1e-6f, (f.flags & 1) ? 1.0f : 0.0f);
+    const float offset = (f.flags & 1) ? 1.0f : 0.0f;
+    if (g.block[0] == 1024)
+        ORX_LAUNCH(residual_norm_rotate_a8_kernel<1024>, dim3(g.grid[0]), dim3(1024), g.shared, stream, x, r, w, y, ro, signs,
+                   q, s, f.K, 1e-6f, offset);
+    else
+        ORX_LAUNCH(residual_norm_rotate_a8_kernel<256>, dim3(g.grid[0]), dim3(256), g.shared, stream, x, r, w, y, ro, signs,
+                   q, s, f.K, 1e-6f, offset);
     return hip_check(hipGetLastError(), "launch residual_norm_rotate_a8");
 }
 
@@ -1072,7 +1086,7 @@ int make_residual_rotate(const Variant& v, orx_function* f) {
     f->args = {{"Q", ArgPointer, 4},     {"R", ArgPointer, 16}, {"RO", ArgPointer, 16}, {"S", ArgPointer, 2},
                {"Signs", ArgPointer, 4}, {"W", ArgPointer, 8},  {"X", ArgPointer, 8},   {"Y", ArgPointer, 8}};
     if (f->dynamic_rows) f->args.push_back({"m", ArgI32, 4});
-    f->device_function = reinterpret_cast<const void*>(&residual_norm_rotate_a8_kernel);
+    f->device_function = nullptr;  // kernels with 256 and 1024 threads serve this symbol
     f->geometry = residual_rotate_geometry;
     f->launch = residual_rotate_launch;
     return ORX_OK;

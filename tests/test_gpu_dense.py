@@ -107,6 +107,29 @@ def test_a8_many_rows_of_long_groups(rows, k, group):
     np.testing.assert_array_equal(gu.host(q), wq)
 
 
+@pytest.mark.parametrize("fused", [False, True], ids=["rows", "swiglu"])
+@pytest.mark.parametrize("rows,k,group", [
+    (2049, 1016, 1016), (2048, 2048, 2048), (1023, 1536, 768),          # one wave to a group, units that do not divide by four
+    (3, 520, 520), (5, 2048, 2048), (600, 2056, 2056), (514, 12288, 12288),   # four waves, at both ends of their pieces
+    (2, 2056, 2056), (513, 12296, 12296), (1, 32768, 32768),            # eight waves
+    (1, 32776, 32776), (2, 2060, 2060), (2049, 1020, 1020),             # too long to hold; rows that are not 16-byte aligned
+])
+def test_a8_held_forms(rows, k, group, fused):
+    """The waves and pieces that hold a row follow its length and the row count; codes and scales do not."""
+    rng = np.random.default_rng(orc.SEED + rows + k + fused)
+    x = (rng.normal(size=(rows, 2 * k if fused else k)) * 2).astype(np.float16)
+    x[0, -1] = 300
+    q, s = gu.a8(gu.dev(x), group=group, fused=fused)
+    values = x
+    if fused:  # the device's own fp16 values (the exponential may differ from libm in the last place)
+        y = torch.empty((rows, k), dtype=torch.float16, device=gu.DEV)
+        gu.kernel("swiglu", I=k)(X=gu.dev(x), Y=y, rows=rows)
+        values = gu.host(y)
+    wq, ws = orc.a8(values, group)
+    np.testing.assert_array_equal(gu.host(s), ws)
+    np.testing.assert_array_equal(gu.host(q), wq)
+
+
 def test_a8_masked_columns():
     rng = np.random.default_rng(orc.SEED)
     x = rng.normal(size=(9, 512)).astype(np.float16)
@@ -203,7 +226,7 @@ def ulps_fp16(a, b):
 
 
 @pytest.mark.parametrize("m,k,zero_centered", [(1, 256, True), (3, 1536, True), (5, 5120, True), (2, 5120, False),
-                                               (1, 17408, True)])
+                                               (1, 17408, True), (2, 2048, True), (256, 2304, True), (257, 2304, True)])
 def test_residual_norm_rotate_a8_matches_oracle(m, k, zero_centered):
     rng = np.random.default_rng(orc.SEED + 3 * m + k)
     x = rng.normal(size=(m, k)).astype(np.float16)
