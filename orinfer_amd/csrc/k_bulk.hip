@@ -1,0 +1,461 @@
+// Routed single-stage (Q2) expert projections of long prompts: 128-row tiles, codes decoded into MFMA operands.
+//
+// Reference counterpart: the routed decode kernels/cuda/model/e8p_decode.py:36-245 over the tile list of
+// kernels/cuda/model/routing.py.  Arithmetic: exact int32 over the full K, (float(acc) * ws) * as, rounded to fp16 once.
+//
+// With hundreds of rows per expert the projection is a matrix product: 4096 tokens x top-8 of 128 experts are 137 GOP in
+// gate_up and 69 GOP in down, which the 32-row tiles of the weight-streaming kernels ran at 460 TOP/s, decoding every code
+// once per 32 rows.
+//  * A unit is (tile of up to 128 slots, 256 output channels), a workgroup four waves, two workgroups to a CU, so that the
+//    set-up and the epilogue of one run beside the K loop of the other.
+//  * A wave owns 64 channels and all rows of the tile, 8 x 4 blocks of v_mfma_i32_16x16x64_i8 (128 accumulator
+//    registers).  Its codes go from memory into registers (8 bytes per lane, block of 16 channels and 128 of K) and through
+//    the byte tables straight into the weight operands: no decoded weight passes through LDS, and a code is
+//    decoded once per 128 rows.  Per 64 of K a wave then asks LDS for 8 fragments of 1 KiB and 16 lookups of 512 bytes while
+//    it multiplies 32 times.  Tiles of at most 64 or 32 rows take 4 or 2 row blocks.
+//  * Token rows come through LDS by direct loads in whole cache lines (K chunks of 128, two slots of 16 KiB); with GATHER
+//    the rows are those of the slots' tokens, so no launch copies a token's row top_k times.
+//  * Entry i of both tables lies in 128 bytes, eight copies of the basis entry in front of eight of the mask entry; of 16
+//    neighbouring lanes eight read one table and eight the other, each its own copy, so they never collide (two tables of eight
+//    copies, read one after the other: half as many conflict cycles again; sixteen copies of each leave room for one
+//    workgroup per CU).
+// Measured at 4096 tokens x top-8 of 128 experts (H = 2048, I = 512; popularity of the experts like 1 / rank^1.1):
+// gate_up 296 -> 100 us, down 215 -> 86 us.  What bounds it now: no pipe is full (LDS 42 %, vector ALU 40 %, matrix pipe
+// 30 % of the cycles); the two waves of a SIMD wait for each other's LDS reads and barriers in a third of theirs.
+// One persistent workgroup of eight waves per CU that requests the next unit's chunks early measured 118 and 75 us.
+//  * SWIGLU: a wave owns 32 gate and the 32 matching up channels, so gate and up of one (slot, channel) meet in one
+//    lane; the epilogue writes fp16(silu(gate) * up) and, where asked, gate | up and the slots' largest magnitudes.
+#include <hip/hip_fp16.h>
+
+#include <algorithm>
+#include <type_traits>
+
+#include "a8_device.h"
+#include "e8p_device.h"
+#include "orx_internal.h"
+
+namespace orx {
+namespace {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef unsigned int v2u __attribute__((ext_vector_type(2)));
+
+constexpr int kThreads = 256;
+constexpr int kTileRows = 128;
+constexpr int kSpan = 256;  // output channels of a unit (SWIGLU: 128 gate + 128 up)
+constexpr uint32_t kTokens = 256 * 128;  // behind the tables: 256 entries of 8 copies of basis, 8 of mask
+constexpr uint32_t kSlot = kTileRows * 128;
+constexpr uint32_t kTokenScale = kTokens + 2 * kSlot;
+constexpr uint32_t kChannelScale = kTokenScale + kTileRows * 4;
+constexpr uint32_t kLds = kChannelScale + kSpan * 4;
+
+struct BulkParams {
+    const int8_t* a;        // (slots, K), or (tokens, K) when gathered
+    const __half* as;
+    const int* slot_token;  // GATHER: token of every slot
+    const uint8_t* w;       // (E, K/128, N, 16) u16
+    const uint32_t* book;
+    const __half* ws;       // (E, N)
+    __half* out;            // (slots, N); may be null with SWIGLU
+    __half* act;            // SWIGLU: (slots, N/2)
+    int* row_max;           // SWIGLU: raised to the fp32 bits of the slot's largest |act|; may be null
+    const int* counts;
+    const int* offsets;
+    const int* tile_expert;
+    const int* tile_row;
+    const int* tile_count;
+    int n, k, tile_capacity, spans;
+};
+
+__device__ __forceinline__ int swizzle(int row) { return (row >> 1) & 7; }
+__device__ __forceinline__ uint32_t lds_address_of(const void* pointer) {
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)pointer;
+}
+__device__ __forceinline__ void direct_load_16(const void* global, void* lds_wave_base) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)global,
+                                     (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, 0);
+}
+// LDS and code reads from asm statements, waited for by hand: the compiler waits for every direct-to-LDS load in flight in
+// front of an LDS read it can see.
+template <int OFFSET>
+__device__ __forceinline__ void lds_read_16(v4i& value, uint32_t address) {
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(value) : "v"(address), "n"(OFFSET));
+}
+template <int OFFSET>
+__device__ __forceinline__ void lds_read_8(v2u& value, uint32_t address) {
+    asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(value) : "v"(address), "n"(OFFSET));
+}
+template <int OFFSET>
+__device__ __forceinline__ void load_8(v2u& value, uint32_t lane_offset, const uint8_t* uniform_base) {
+    asm volatile("global_load_dwordx2 %0, %1, %2 offset:%3"
+                 : "=v"(value)
+                 : "v"(lane_offset), "s"(uniform_base), "n"(OFFSET)
+                 : "memory");
+}
+__device__ __forceinline__ uint32_t pack2(__half low, __half high) {
+    return (uint32_t)__half_as_ushort(low) | (uint32_t)__half_as_ushort(high) << 16;
+}
+template <typename T>
+__device__ __forceinline__ T* uniform_pointer(T* pointer) {
+    const uint64_t bits = reinterpret_cast<uint64_t>(pointer);
+    const uint32_t low = __builtin_amdgcn_readfirstlane((uint32_t)bits), high = __builtin_amdgcn_readfirstlane((uint32_t)(bits >> 32));
+    return reinterpret_cast<T*>((uint64_t)high << 32 | low);
+}
+
+template <bool GATHER, bool SWIGLU>
+__global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+    // ---- unit: workgroups 8 apart (one XCD) take the spans of one tile, whose rows that XCD's L2 then holds ----
+    const int b = (int)blockIdx.x, region = 8 * p.spans;
+    const int tile = (b / region) * 8 + b % 8, span = (b / 8) % p.spans;
+    if (tile >= p.tile_capacity || tile >= p.tile_count[0]) return;
+    const uint32_t selector = p.book[tid];
+    const int expert = __builtin_amdgcn_readfirstlane(p.tile_expert[tile]);
+    const int first = __builtin_amdgcn_readfirstlane(p.tile_row[tile]);
+    const int rows = __builtin_amdgcn_readfirstlane(min(kTileRows, p.counts[expert] - first));
+    if (rows <= 0) return;
+    const int row0 = __builtin_amdgcn_readfirstlane(p.offsets[expert] + first);
+    const int inner = p.n / 2;
+    const int chunks = p.k / 128;
+
+    // ---- this wave's channels: plain n0 .. n0 + 63; SWIGLU gate n0 .. n0 + 31 and up inner + n0 .. ----
+    const int group = span * 4 + wave;
+    const int limit = SWIGLU ? inner / 32 : p.n / 64;
+    const bool live_wave = group < limit;  // the others help with the token rows
+    const int n0 = (live_wave ? group : 0) * (SWIGLU ? 32 : 64);
+    const uint8_t* const codes_base = uniform_pointer(p.w + (int64_t)expert * p.n * (p.k / 4));
+    const uint32_t chunk_stride = (uint32_t)p.n * 32;
+    const uint32_t code_offset = (uint32_t)(n0 + (lane & 15)) * 32 + (uint32_t)(lane >> 4) * 8;
+    const uint32_t code_offset_up = code_offset + (SWIGLU ? (uint32_t)inner * 32 : 1024u);
+    const int8_t* const a_base = uniform_pointer(p.a);
+
+    auto run = [&](auto blocks_tag) {
+        constexpr int NB = decltype(blocks_tag)::value;  // 16-row blocks
+        constexpr int LOADS = NB / 2;                    // 16 NB rows are 2 NB requests of 8 rows, over four waves
+        constexpr int PHASES = NB >= 4 ? 4 : 2;          // a step of 64 in phases of RB row blocks,
+        constexpr int RB = NB / PHASES, LB = 4 / PHASES; // each looking up LB of the next step's four weight blocks
+        // ---- token rows: request b of this wave brings rows 8 (LOADS wave + b) .. +7 of a chunk, 128 bytes each.  The
+        // quarter q of a wave multiplies K bytes [32 q, +32) of a chunk in two steps of 16, so piece c = 2 q + s of row r sits
+        // at position (q + 4 s) ^ swizzle(r): a fragment read touches four neighbouring positions of 16 rows ----
+        uint32_t row_offset[LOADS];
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            const int row = (wave * LOADS + i) * 8 + (lane >> 3);
+            const int slot = row0 + min(row, rows - 1);
+            const int position = (lane & 7) ^ swizzle(row);
+            const int piece = ((position & 3) << 1) | (position >> 2);
+            row_offset[i] = (uint32_t)(GATHER ? p.slot_token[slot] : slot) * (uint32_t)p.k + (uint32_t)piece * 16;
+        }
+        auto issue_tokens = [&](int chunk, int slot) {
+            const int8_t* base = a_base + min(chunk, chunks - 1) * 128;
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) {
+                uint32_t offset = row_offset[i];
+                asm volatile("" : "+v"(offset));  // 32 bits beside a uniform base, not a 64-bit address kept per request
+                direct_load_16(base + (uint64_t)offset, lds + kTokens + (uint32_t)slot * kSlot + (uint32_t)(wave * LOADS + i) * 1024);
+            }
+        };
+        // two register sets of codes, by the parity of the chunk: four blocks of 16 channels, 8 bytes to a lane
+        v2u codes[2][4];
+        auto issue_codes = [&](int chunk, auto set_tag) {
+            constexpr int SET = decltype(set_tag)::value;
+            const uint8_t* base = codes_base + (uint64_t)min(chunk, chunks - 1) * chunk_stride;
+            load_8<0>(codes[SET][0], code_offset, base);
+            load_8<512>(codes[SET][1], code_offset, base);
+            load_8<0>(codes[SET][2], code_offset_up, base);
+            load_8<512>(codes[SET][3], code_offset_up, base);
+        };
+        std::integral_constant<int, 0> zero;
+        std::integral_constant<int, 1> one;
+        issue_codes(0, zero);
+        issue_tokens(0, 0);
+        issue_codes(1, one);
+        issue_tokens(1, 1);
+
+        // ---- tables, scales (beside the first loads) ----
+        {
+            const uint2 basis = byte_basis_signed(selector), mask = byte_mask_signed((uint32_t)tid);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                *reinterpret_cast<uint4*>(lds + tid * 128 + 16 * i) = make_uint4(basis.x, basis.y, basis.x, basis.y);
+                *reinterpret_cast<uint4*>(lds + tid * 128 + 64 + 16 * i) = make_uint4(mask.x, mask.y, mask.x, mask.y);
+            }
+            if (tid < kTileRows) {
+                const int slot = row0 + min(tid, rows - 1);
+                reinterpret_cast<float*>(lds + kTokenScale)[tid] = __half2float(p.as[GATHER ? p.slot_token[slot] : slot]);
+            }
+            // channel scale `lane` of each wave, in the order of its four blocks
+            const int channel = SWIGLU && lane >= 32 ? inner + n0 + lane - 32 : n0 + lane;
+            reinterpret_cast<float*>(lds + kChannelScale)[tid] = __half2float(p.ws[(int64_t)expert * p.n + channel]);
+        }
+
+        v4i acc[NB][4];
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[i][j] = v4i{0, 0, 0, 0};
+
+        // ---- LDS reads ----
+        const uint32_t lds_base = lds_address_of(lds);
+        // Lookups: half of the lanes read the basis entry of a code while the others read its mask entry, then the other
+        // way round (the two are XORed, so it does not matter which came first).
+        const uint32_t other = (uint32_t)(lane >> 3) & 1;
+        const uint32_t first_table = lds_base + (uint32_t)(lane & 7) * 8 + other * 64, second_table = first_table ^ 64u;
+        const uint32_t first_bit = 8 - 8 * other, second_bit = 8 - first_bit;  // byte of a code that indexes it
+        const uint32_t frag = lds_base + kTokens + (uint32_t)(lane & 15) * 128 + (uint32_t)(((lane >> 4) ^ swizzle(lane & 15)) * 16);
+        v4i token[2][RB];  // fragments of even and odd phases
+        auto read_tokens = [&](auto phase_tag, uint32_t address) {
+            constexpr int PHASE = decltype(phase_tag)::value;
+            lds_read_16<PHASE * RB * 2048>(token[PHASE & 1][0], address);
+            if constexpr (RB > 1) lds_read_16<PHASE * RB * 2048 + 2048>(token[PHASE & 1][1], address);
+        };
+        v2u looked[4 * LB];
+        auto lookup = [&](int at, uint32_t word) {  // both entries of two codes
+            lds_read_8<0>(looked[4 * at + 0], (__builtin_amdgcn_ubfe(word, first_bit, 8) << 7) + first_table);
+            lds_read_8<0>(looked[4 * at + 1], (__builtin_amdgcn_ubfe(word, second_bit, 8) << 7) + second_table);
+            lds_read_8<0>(looked[4 * at + 2], (__builtin_amdgcn_ubfe(word, first_bit + 16, 8) << 7) + first_table);
+            lds_read_8<0>(looked[4 * at + 3], (__builtin_amdgcn_ubfe(word, second_bit + 16, 8) << 7) + second_table);
+        };
+        auto combine = [&](int at) {
+            const v2u* e = looked + 4 * at;
+            return v4i{(int)(e[0][0] ^ e[1][0]), (int)(e[0][1] ^ e[1][1]), (int)(e[2][0] ^ e[3][0]), (int)(e[2][1] ^ e[3][1])};
+        };
+        auto wait_reads = [&]() {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int i = 0; i < 4 * LB; ++i) asm volatile("" : "+v"(looked[i]));
+#pragma unroll
+            for (int i = 0; i < RB; ++i) asm volatile("" : "+v"(token[0][i]), "+v"(token[1][i]));
+        };
+        v4i weight[2][4];  // of a chunk's two steps
+        // Phase PHASE of step STEP: its multiplies (one operand changing between consecutive ones), and behind the first of them
+        // the fragments of the phase after it and LB blocks of the next step's codes; all of these have come when it ends.
+        auto phase = [&](auto step_tag, auto phase_tag, uint32_t next_fragments, const v2u(&next_codes)[4], auto requests) {
+            constexpr int STEP = decltype(step_tag)::value, PHASE = decltype(phase_tag)::value;
+            constexpr int NEXT = (PHASE + 1) % PHASES;
+#pragma unroll
+            for (int i = 0; i < RB; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int jj = (i & 1) ? 3 - j : j;
+                    v4i& sum = acc[PHASE * RB + i][jj];
+                    sum = __builtin_amdgcn_mfma_i32_16x16x64_i8(weight[STEP][jj], token[PHASE & 1][i], sum, 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (i == 0 && j == 0) read_tokens(std::integral_constant<int, NEXT>{}, next_fragments);
+                    if (i == 0 && j >= 1 && j - 1 < LB) lookup(j - 1, next_codes[PHASE * LB + j - 1][1 - STEP]);
+                    if (i == 0 && j == 3) requests();
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            wait_reads();
+#pragma unroll
+            for (int l = 0; l < LB; ++l) weight[1 - STEP][PHASE * LB + l] = combine(l);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto nothing = [] {};
+        std::integral_constant<int, 2> two;
+        std::integral_constant<int, 3> three;
+
+        // ---- prologue: chunk 0 in LDS, the weights of its first step decoded, its first fragments read ----
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)"
+                     : "+v"(codes[0][0]), "+v"(codes[0][1]), "+v"(codes[0][2]), "+v"(codes[0][3]), "+v"(codes[1][0]), "+v"(codes[1][1]),
+                       "+v"(codes[1][2]), "+v"(codes[1][3])
+                     :
+                     : "memory");
+        __syncthreads();
+        read_tokens(zero, frag);
+        read_tokens(one, frag);
+#pragma unroll
+        for (int j = 0; j < 4; j += LB) {
+#pragma unroll
+            for (int l = 0; l < LB; ++l) lookup(l, codes[0][j + l][0]);
+            wait_reads();
+#pragma unroll
+            for (int l = 0; l < LB; ++l) weight[0][j + l] = combine(l);
+        }
+
+        // One chunk: two steps of 64.  In front of its last phase the workgroup meets once: chunk t + 1 has landed,
+        // everybody has read chunk t, and the requests of chunk t + 2 go out into its slot and its code registers.
+        auto chunk_step = [&](int t, auto set_tag) {
+            constexpr int SET = decltype(set_tag)::value;
+            const uint32_t here = frag + (uint32_t)SET * kSlot, there = frag + (uint32_t)(1 - SET) * kSlot;
+            auto meet = [&]() {
+                asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            auto request = [&]() { issue_codes(t + 2, set_tag), issue_tokens(t + 2, SET); };
+            if constexpr (PHASES == 4) {
+                phase(zero, zero, here, codes[SET], nothing);
+                phase(zero, one, here, codes[SET], nothing);
+                phase(zero, two, here, codes[SET], nothing);
+                phase(zero, three, here ^ 64u, codes[SET], nothing);
+            } else {
+                phase(zero, zero, here, codes[SET], nothing);
+                phase(zero, one, here ^ 64u, codes[SET], nothing);
+            }
+            // the codes of chunk t + 1 are older than its token rows
+            asm volatile("s_waitcnt vmcnt(%4)"
+                         : "+v"(codes[1 - SET][0]), "+v"(codes[1 - SET][1]), "+v"(codes[1 - SET][2]), "+v"(codes[1 - SET][3])
+                         : "n"(LOADS));
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (PHASES == 4) {
+                phase(one, zero, here ^ 64u, codes[1 - SET], nothing);
+                phase(one, one, here ^ 64u, codes[1 - SET], nothing);
+                phase(one, two, here ^ 64u, codes[1 - SET], nothing);
+                meet();
+                phase(one, three, there, codes[1 - SET], request);
+            } else {
+                phase(one, zero, here ^ 64u, codes[1 - SET], nothing);
+                meet();
+                phase(one, one, there, codes[1 - SET], request);
+            }
+        };
+        int t = 0;
+        for (; t + 1 < chunks; t += 2) {
+            chunk_step(t, zero);
+            chunk_step(t + 1, one);
+        }
+        if (t < chunks) chunk_step(t, zero);
+        // requests of chunks that do not exist (clamped): their registers stay named until they have landed
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)"
+                     : "+v"(codes[0][0]), "+v"(codes[0][1]), "+v"(codes[0][2]), "+v"(codes[0][3]), "+v"(codes[1][0]), "+v"(codes[1][1]),
+                       "+v"(codes[1][2]), "+v"(codes[1][3])
+                     :
+                     : "memory");
+
+        // ---- epilogue: a lane holds four consecutive channels of one slot in every block.  One swap of the odd rows of 16
+        // lanes of block j with the even rows of block j + 1 leaves a lane with 16 contiguous bytes of one output row ----
+        if (!live_wave) return;
+        int own = threadIdx.x & 63;
+        asm volatile("" : "+v"(own));  // nothing of the addresses below is carried through the K loop
+        const int quarter = own >> 4;
+        const float* const token_scales = reinterpret_cast<const float*>(lds + kTokenScale);
+        const float* const channel_scales = reinterpret_cast<const float*>(lds + kChannelScale) + wave * 64;
+        auto store_pair = [&](bool live, __half* row_out, const uint32_t (&first_words)[2], const uint32_t (&second_words)[2]) {
+            const v2u l = __builtin_amdgcn_permlane16_swap(first_words[0], second_words[0], false, false);
+            const v2u h = __builtin_amdgcn_permlane16_swap(first_words[1], second_words[1], false, false);
+            if (!live) return;
+            row_out += (quarter & 1) * 16 + (quarter >> 1) * 8;
+            const uint4 piece = make_uint4(l[0], h[0], l[1], h[1]);
+            if ((reinterpret_cast<uintptr_t>(row_out) & 15) == 0) {
+                *reinterpret_cast<uint4*>(row_out) = piece;
+            } else {  // an output buffer may be aligned to its elements only
+                const uint32_t words[4] = {piece.x, piece.y, piece.z, piece.w};
+#pragma unroll
+                for (int e = 0; e < 8; ++e) row_out[e] = __ushort_as_half((unsigned short)(words[e >> 1] >> (16 * (e & 1))));
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const int local = i * 16 + (own & 15);
+            const bool live = local < rows;
+            const float token_scale = token_scales[local];
+            const int64_t slot = row0 + local;
+            auto value = [&](int j, int r) {
+                return __float2half_rn(rescale(acc[i][j][r], channel_scales[j * 16 + 4 * quarter + r], token_scale));
+            };
+            if constexpr (!SWIGLU) {
+#pragma unroll
+                for (int pair = 0; pair < 2; ++pair) {
+                    uint32_t words[2][2];
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+                        words[e][0] = pack2(value(2 * pair + e, 0), value(2 * pair + e, 1)),
+                        words[e][1] = pack2(value(2 * pair + e, 2), value(2 * pair + e, 3));
+                    store_pair(live, p.out + slot * p.n + n0 + 32 * pair, words[0], words[1]);
+                }
+            } else {
+                uint32_t words[2][2];
+                const bool maxima = p.row_max != nullptr;
+                float amax = 0.f;
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    __half gate[4], up[4], product[4];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        gate[r] = value(e, r), up[r] = value(e + 2, r);
+                        const float v = swiglu_value(gate[r], up[r]);
+                        product[r] = __float2half_rn(v);
+                        if (maxima) amax = fmaxf(amax, fabsf(v));
+                    }
+                    words[e][0] = pack2(product[0], product[1]), words[e][1] = pack2(product[2], product[3]);
+                    if (live && p.out != nullptr) {
+                        __half* dst = p.out + slot * p.n + n0 + 16 * e + 4 * quarter;
+                        *reinterpret_cast<uint2*>(dst) = make_uint2(pack2(gate[0], gate[1]), pack2(gate[2], gate[3]));
+                        *reinterpret_cast<uint2*>(dst + inner) = make_uint2(pack2(up[0], up[1]), pack2(up[2], up[3]));
+                    }
+                }
+                store_pair(live, p.act + slot * inner + n0, words[0], words[1]);
+                if (maxima) {
+                    amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
+                    amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+                    if (live && quarter == 0) atomicMax(p.row_max + slot, __float_as_int(amax));
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    if (rows > 64)
+        run(std::integral_constant<int, 8>{});
+    else if (rows > 32)
+        run(std::integral_constant<int, 4>{});
+    else
+        run(std::integral_constant<int, 2>{});
+}
+
+}  // namespace
+
+// What the kernel takes: K-major codes, tiles of 128 rows, whole 64-channel groups per wave, row offsets of 32 bits.
+bool grouped_bulk_eligible(int n, int k, int block_m, int packed_k, int64_t rows) {
+    return block_m == kTileRows && packed_k == 128 && k % 128 == 0 && n % 64 == 0 && rows * k < (1ll << 31) &&
+           (int64_t)n * 32 < (1ll << 31);
+}
+
+void grouped_bulk_geometry(int n, int tiles, bool swiglu, Geometry* g) {
+    const uint32_t spans = swiglu ? ceil_div((uint32_t)n / 2, kSpan / 2) : ceil_div((uint32_t)n, kSpan);
+    g->grid[0] = ceil_div((uint32_t)tiles, 8u) * 8u * spans;
+    g->grid[1] = g->grid[2] = 1;
+    g->block[0] = kThreads;
+    g->shared = kLds;
+}
+
+int grouped_bulk_launch(const GroupedBuffers& b, int n, int k, int tiles, bool gather, bool swiglu, hipStream_t stream) {
+    static DeviceOnce opted_in;  // dynamic LDS above 64 KiB needs an opt-in per kernel and device
+    const int ready = opted_in.run([] {
+        for (const void* kernel : {reinterpret_cast<const void*>(&grouped_bulk_kernel<false, false>),
+                                   reinterpret_cast<const void*>(&grouped_bulk_kernel<true, false>),
+                                   reinterpret_cast<const void*>(&grouped_bulk_kernel<false, true>),
+                                   reinterpret_cast<const void*>(&grouped_bulk_kernel<true, true>)}) {
+            const int code = hip_check(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds),
+                                       "hipFuncSetAttribute");
+            if (code != ORX_OK) return code;
+        }
+        return (int)ORX_OK;
+    });
+    if (ready != ORX_OK) return ready;
+    Geometry g;
+    grouped_bulk_geometry(n, tiles, swiglu, &g);
+    BulkParams p = {};
+    p.a = reinterpret_cast<const int8_t*>(b.a), p.as = reinterpret_cast<const __half*>(b.as), p.slot_token = b.slot_token;
+    p.w = reinterpret_cast<const uint8_t*>(b.w), p.book = b.book, p.ws = reinterpret_cast<const __half*>(b.ws);
+    p.out = reinterpret_cast<__half*>(b.out), p.act = reinterpret_cast<__half*>(b.act);
+    p.row_max = swiglu ? const_cast<int*>(b.row_max) : nullptr;
+    p.counts = b.counts, p.offsets = b.offsets, p.tile_expert = b.tile_expert, p.tile_row = b.tile_row;
+    p.tile_count = b.tile_count;
+    p.n = n, p.k = k, p.tile_capacity = tiles;
+    p.spans = (int)(swiglu ? ceil_div((uint32_t)n / 2, kSpan / 2) : ceil_div((uint32_t)n, kSpan));
+    const dim3 grid(g.grid[0]), block(kThreads);
+    if (gather && swiglu)
+        ORX_LAUNCH((grouped_bulk_kernel<true, true>), grid, block, g.shared, stream, p);
+    else if (gather)
+        ORX_LAUNCH((grouped_bulk_kernel<true, false>), grid, block, g.shared, stream, p);
+    else if (swiglu)
+        ORX_LAUNCH((grouped_bulk_kernel<false, true>), grid, block, g.shared, stream, p);
+    else
+        ORX_LAUNCH((grouped_bulk_kernel<false, false>), grid, block, g.shared, stream, p);
+    return hip_check(hipGetLastError(), "launch routed projection (bulk)");
+}
+
+}  // namespace orx

@@ -56,6 +56,9 @@ bool grouped_resident_preferred(int rows, int experts, int n);
 void grouped_resident_geometry(int k, int input, int epilogue, int slots, Geometry* g);
 int grouped_resident_launch(const GroupedBuffers& b, int n, int k, int tiles, int packed_k, int input, int epilogue,
                             int slots, hipStream_t stream);
+bool grouped_bulk_eligible(int n, int k, int block_m, int packed_k, int64_t rows);
+void grouped_bulk_geometry(int n, int tiles, bool swiglu, Geometry* g);
+int grouped_bulk_launch(const GroupedBuffers& b, int n, int k, int tiles, bool gather, bool swiglu, hipStream_t stream);
 int stream_grouped_launch(const int8_t* a, const void* w, const uint32_t* book, const __half* ws, const __half* as,
                           void* out, const int* counts, const int* offsets, const int* tile_expert, const int* tile_row,
                           const int* tile_count, int n, int k, int tiles, int block_m, int packed_k,
@@ -1545,8 +1548,14 @@ int make_int8_swiglu(const Variant& v, orx_function* f) {
 // bits 4-5: the BookForm of the general decode
 enum GroupedForm { kGeneralDecode = 1, kPatched = 2, kExpertTables = 4, kTakesPatch = 8, kBookFormShift = 4 };
 
+// The bulk kernel: every list of 128-row tiles that it takes (`algorithm=mfma` keeps the generic tiles).
+bool grouped_uses_bulk(const orx_function& f) {
+    return !(f.H & kGeneralDecode) && f.algorithm == kAuto && (f.flags2 & 3) != 2 &&
+           grouped_bulk_eligible(f.N, f.K, f.block_m, f.packed_k, f.capacity);
+}
+
 bool grouped_uses_resident(const orx_function& f) {
-    if (f.H & kGeneralDecode) return false;
+    if ((f.H & kGeneralDecode) || grouped_uses_bulk(f)) return false;
     if (f.algorithm == kResident || f.flags2 != 0) return true;
     return f.algorithm == kAuto && grouped_resident_eligible(f.N, f.K, f.block_m, f.tiles, 0, 0, f.capacity) &&
            grouped_resident_preferred(f.capacity, f.E, f.N);
@@ -1554,6 +1563,10 @@ bool grouped_uses_resident(const orx_function& f) {
 
 int grouped_geometry(const orx_function& f, int rows, Geometry* g) {
     (void)rows;
+    if (grouped_uses_bulk(f)) {
+        grouped_bulk_geometry(f.N, f.tiles, (f.flags2 >> 2) == 1, g);
+        return ORX_OK;
+    }
     if (grouped_uses_resident(f)) {
         grouped_resident_geometry(f.K, f.flags2 & 3, f.flags2 >> 2, f.capacity, g);
         return ORX_OK;
@@ -1590,6 +1603,8 @@ int grouped_launch(const orx_function& f, int rows, const Geometry& g, hipStream
     b.tile_row = reinterpret_cast<const int*>(buffer("TileRow")), b.ws = buffer("WS");
     b.slot_token = reinterpret_cast<const int*>(buffer("SlotToken"));
     b.row_max = reinterpret_cast<const int*>(buffer("RowMax")), b.act = buffer("Act"), b.q = buffer("Q");
+    if (grouped_uses_bulk(f))
+        return grouped_bulk_launch(b, f.N, f.K, f.tiles, (f.flags2 & 3) == 1, (f.flags2 >> 2) == 1, stream);
     if (grouped_uses_resident(f))
         return grouped_resident_launch(b, f.N, f.K, f.tiles, f.packed_k, f.flags2 & 3, f.flags2 >> 2, f.capacity, stream);
     GemmParams p = {};
@@ -1713,8 +1728,10 @@ int make_q2_grouped(const Variant& v, orx_function* f) {
     // fp16(silu(gate) * up), RowMax (slots, zero before the launch) is raised to the fp32 bits of every slot's
     // largest |Act|, and C may be null.  input_dtype=float16: A holds such fp16 rows and RowMax their maxima; the
     // rows are quantised by the A8 rule while staged, and AS and Q (either may be null) receive scales and codes.
-    // All three are forms of the resident kernel: served where `auto` picks it, or by name.
-    if (f->flags2 != 0) {
+    // All three are forms of the resident kernel: served where `auto` picks it, or by name.  Lists of 128-row tiles have the
+    // first two on the bulk kernel, which needs no RowMax (it may be null: the rows are quantised by a launch of their own).
+    const bool bulk = grouped_uses_bulk(*f);
+    if (f->flags2 != 0 && !bulk) {
         if ((f->algorithm != kAuto && f->algorithm != kResident) ||
             !grouped_resident_eligible(f->N, f->K, f->block_m, f->tiles, f->flags2 & 3, f->flags2 >> 2, f->capacity) ||
             (f->algorithm == kAuto && !grouped_resident_preferred(f->capacity, f->E, f->N))) {
@@ -1729,7 +1746,7 @@ int make_q2_grouped(const Variant& v, orx_function* f) {
         f->args.clear();
         f->args.push_back({"A", ArgPointer, 16});
         f->args.push_back({"AS", ArgPointer, rows16 ? nullable | 2u : 2u});
-        if (swiglu) f->args.push_back({"Act", ArgPointer, 8});
+        if (swiglu) f->args.push_back({"Act", ArgPointer, bulk ? 16u : 8u});
         f->args.push_back({"Book", ArgPointer, 4});
         f->args.push_back({"C", ArgPointer, swiglu ? nullable | 8u : 2u});
         f->args.push_back({"Counts", ArgPointer, 4});
@@ -1738,7 +1755,7 @@ int make_q2_grouped(const Variant& v, orx_function* f) {
         // (E, K/128, N) u16 when patched; the reference binds a one-element dummy otherwise: never read, may be null
         if (vq) f->args.push_back({"Patch", ArgPointer, patched ? 2u : nullable | 2u});
         if (rows16) f->args.push_back({"Q", ArgPointer, nullable | 8u});
-        if (rows16 || swiglu) f->args.push_back({"RowMax", ArgPointer, 4});
+        if (rows16 || swiglu) f->args.push_back({"RowMax", ArgPointer, bulk ? nullable | 4u : 4u});
         if (gathered) f->args.push_back({"SlotToken", ArgPointer, 4});
         f->args.push_back({"TileCount", ArgPointer, 4});
         f->args.push_back({"TileExpert", ArgPointer, 4});

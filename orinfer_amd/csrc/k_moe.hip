@@ -440,6 +440,99 @@ __global__ __launch_bounds__(kMetaThreads) void route_metadata_kernel(
     }
 }
 
+// The same metadata for assignment lists of any length, in two launches of one workgroup per segment of 1024 assignments
+// (one workgroup walks 16384 of them in 20 us; the reference's histogram, one workgroup per expert over the whole list, took
+// 68 us for 32768 and 128 experts).  Every wave ranks 64 assignments.
+// rank:  RelativeSlot[i] = rank of assignment i among those of its expert in its segment, Segments[s][e] = their number.
+// place: every workgroup adds up the segments in front of its own and scans the experts; the tile list is dealt to all.
+// (Whole tiles in front of the rests, so that a projection ends on short units, made it 4 % slower: a CU runs a long and a
+// short unit together better than two of a kind.)
+constexpr int kSegment = kMetaThreads;
+__global__ __launch_bounds__(kMetaThreads) void segment_rank_kernel(const int* __restrict__ ids, int* __restrict__ relative,
+                                                                    int* __restrict__ segments, int assignments, int experts) {
+    extern __shared__ int counters[];  // [kMetaWaves][experts]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int at = blockIdx.x * kSegment + tid;
+    const bool valid = at < assignments;
+    const int id = valid ? ids[at] : 0;
+    for (int i = tid; i < kMetaWaves * experts; i += kMetaThreads) counters[i] = 0;
+    // the lanes of this wave that hold the same expert, found one id bit at a time
+    const int id_bits = 32 - __builtin_clz(max(experts - 1, 1));
+    unsigned long long same = __ballot(valid);
+    for (int bit = 0; bit < id_bits; ++bit) {
+        const bool set = (id >> bit) & 1;
+        const unsigned long long with = __ballot(valid && set);
+        same &= set ? with : ~with;
+    }
+    const int rank = __popcll(same & ((1ull << lane) - 1ull)), group = __popcll(same);
+    __syncthreads();
+    if (valid && rank == group - 1) counters[wave * experts + id] = group;
+    __syncthreads();
+    if (tid < experts) {  // exclusive prefix over the waves, total of the segment
+        int count[kMetaWaves], before = 0;
+#pragma unroll
+        for (int w = 0; w < kMetaWaves; ++w) count[w] = counters[w * experts + tid];
+#pragma unroll
+        for (int w = 0; w < kMetaWaves; ++w) counters[w * experts + tid] = before, before += count[w];
+        segments[(int64_t)blockIdx.x * experts + tid] = before;
+    }
+    __syncthreads();
+    if (valid) relative[at] = counters[wave * experts + id] + rank;
+}
+
+__global__ __launch_bounds__(kMetaThreads) void segment_place_kernel(
+    const int* __restrict__ ids, const int* __restrict__ segments, int* __restrict__ counts, int* __restrict__ relative,
+    int* __restrict__ row_offsets, int* __restrict__ tile_count, int* __restrict__ tile_expert, int* __restrict__ tile_offsets,
+    int* __restrict__ tile_row, int* __restrict__ slot_map, int* __restrict__ slot_token, int* __restrict__ row_max,
+    int assignments, int experts, int top_k, int block_m) {
+    __shared__ int in_front[kMetaThreads], first_row[kMetaThreads], wave_rows[kMetaWaves], wave_tiles[kMetaWaves];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int segment = blockIdx.x, total_segments = gridDim.x;
+    const int at = segment * kSegment + tid;
+    const bool valid = at < assignments;
+    const int id = valid ? ids[at] : 0, local = valid ? relative[at] : 0;
+    int count = 0, before = 0;
+    if (tid < experts) {
+#pragma unroll 8
+        for (int s = 0; s < total_segments; ++s) {
+            const int c = segments[(int64_t)s * experts + tid];
+            before += s < segment ? c : 0;
+            count += c;
+        }
+        in_front[tid] = before;
+    }
+    const int tiles = (count + block_m - 1) / block_m;
+    int row_scan = count, tile_scan = tiles;
+#pragma unroll
+    for (int offset = 1; offset < 64; offset <<= 1) {
+        const int r = __shfl_up(row_scan, offset, 64), t = __shfl_up(tile_scan, offset, 64);
+        if (lane >= offset) row_scan += r, tile_scan += t;
+    }
+    if (lane == 63) wave_rows[wave] = row_scan, wave_tiles[wave] = tile_scan;
+    __syncthreads();
+    int row_base = 0, tile_base = 0, tile_total = 0;
+    for (int w = 0; w < kMetaWaves; ++w) {
+        if (w < wave) row_base += wave_rows[w], tile_base += wave_tiles[w];
+        tile_total += wave_tiles[w];
+    }
+    if (tid < experts) {
+        const int row = row_base + row_scan - count, tile = tile_base + tile_scan - tiles;
+        first_row[tid] = row;
+        if (segment == 0) counts[tid] = count, row_offsets[tid] = row, tile_offsets[tid] = tile;
+        for (int t = segment; t < tiles; t += total_segments) tile_expert[tile + t] = tid, tile_row[tile + t] = t * block_m;
+    }
+    if (segment == 0 && tid == 0) tile_count[0] = tile_total;
+    __syncthreads();
+    if (!valid) return;
+    const int in_expert = in_front[id] + local;
+    relative[at] = in_expert;
+    const int slot = first_row[id] + in_expert;
+    slot_map[at] = slot;
+    slot_token[slot] = at / top_k;
+    if (row_max != nullptr) row_max[at] = 0;
+}
+
 // One token: every selected expert owns one row and one tile, in expert-id order
 // (moe.py:659-709; ids distinct and inside [0, E), as router_topk leaves them).  One workgroup;
 // thread e counts the ids equal to and below e, thread rank places its id.  Tiles from top_k on
@@ -895,7 +988,18 @@ int make_tiles(const Variant& v, orx_function* f) {
     return ORX_OK;
 }
 
-int metadata_geometry(const orx_function& f, int, Geometry* g) {
+// flags: bit0 slot_maps, bit1 segments (workspace=true: any number of assignments, two launches)
+enum { kSlotMaps = 1, kSegments = 2 };
+uint64_t metadata_workspace(const orx_function& f, int rows) {
+    return (uint64_t)ceil_div((uint32_t)rows * (uint32_t)f.top_k, (uint32_t)kSegment) * (uint32_t)f.E * sizeof(int);
+}
+int metadata_geometry(const orx_function& f, int rows, Geometry* g) {
+    if (f.flags & kSegments) {
+        g->grid[0] = ceil_div((uint32_t)rows * (uint32_t)f.top_k, (uint32_t)kSegment);
+        g->block[0] = kMetaThreads;
+        g->shared = (uint32_t)(kMetaWaves * f.E * sizeof(int));
+        return ORX_OK;
+    }
     g->grid[0] = 1;
     g->block[0] = kMetaThreads;
     // counters, scan totals, wave-local slot and expert of every assignment the variant can hold
@@ -907,13 +1011,27 @@ int metadata_geometry(const orx_function& f, int, Geometry* g) {
 int metadata_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t s, void** args) {
     static DeviceOnce opted_in;  // 64 KiB of counters at E = 1024 needs the LDS opt-in
     const int ready = opted_in.run([] {
-        return hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(&route_metadata_kernel),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024),
-                         "hipFuncSetAttribute");
+        for (const void* kernel : {reinterpret_cast<const void*>(&route_metadata_kernel), reinterpret_cast<const void*>(&segment_rank_kernel)}) {
+            const int code = hip_check(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024),
+                                       "hipFuncSetAttribute");
+            if (code != ORX_OK) return code;
+        }
+        return (int)ORX_OK;
     });
     if (ready != ORX_OK) return ready;
-    const bool maps = f.flags & 1;
+    const bool maps = f.flags & kSlotMaps;
     const int offsets_at = maps ? 4 : 3, tiles_at = maps ? 7 : 4;
+    if (f.flags & kSegments) {
+        const int* ids = pointer_arg<const int>(args, 1);
+        int *relative = pointer_arg<int>(args, 2), *segments = pointer_arg<int>(args, f.workspace_arg);
+        ORX_LAUNCH(segment_rank_kernel, dim3(g.grid[0]), dim3(kMetaThreads), g.shared, s, ids, relative, segments, rows * f.top_k, f.E);
+        ORX_LAUNCH(segment_place_kernel, dim3(g.grid[0]), dim3(kMetaThreads), 0, s, ids, segments, pointer_arg<int>(args, 0),
+                   relative, pointer_arg<int>(args, offsets_at), pointer_arg<int>(args, tiles_at),
+                   pointer_arg<int>(args, tiles_at + 1), pointer_arg<int>(args, tiles_at + 2), pointer_arg<int>(args, tiles_at + 3),
+                   pointer_arg<int>(args, 5), pointer_arg<int>(args, 6), pointer_arg<int>(args, 3), rows * f.top_k, f.E, f.top_k,
+                   f.block_m);
+        return hip_check(hipGetLastError(), "launch route_metadata");
+    }
     ORX_LAUNCH(route_metadata_kernel, dim3(1), dim3(kMetaThreads), g.shared, s, pointer_arg<const int>(args, 1),
                        pointer_arg<int>(args, 0), pointer_arg<int>(args, 2), pointer_arg<int>(args, offsets_at),
                        pointer_arg<int>(args, tiles_at), pointer_arg<int>(args, tiles_at + 1),
@@ -927,26 +1045,34 @@ int make_metadata(const Variant& v, orx_function* f) {
     bool bad = false;
     f->block_m = (int)v.integer("block_m", 8, &bad);  // moe.py:714
     if (bad) return ORX_ERR_BAD_VARIANT;
+    const bool slot_maps = v.boolean("slot_maps", false, &bad);
+    // workspace=true (with slot_maps): the list in segments, two launches; Workspace holds the segments' counts
+    f->takes_workspace = v.boolean("workspace", false, &bad);
+    if (bad) return ORX_ERR_BAD_VARIANT;
+    if (f->takes_workspace && (!slot_maps || (int64_t)f->M * f->top_k > (1ll << 30))) {
+        set_error("route_metadata: workspace=true goes with slot_maps=true and at most 2^30 assignments");
+        return ORX_ERR_BAD_VARIANT;
+    }
     // one expert per thread, one route per lane; the reference's own form is decode-only (M <= 1024)
     if (f->M <= 0 || f->E <= 0 || f->E > kMetaThreads || f->top_k <= 0 || f->top_k > f->E || !valid_block_m(f->block_m) ||
-        (size_t)(kMetaWaves * f->E + 2 * kMetaWaves + 2 * (size_t)f->M * f->top_k) * sizeof(int) > 160 * 1024) {
+        (!f->takes_workspace && (size_t)(kMetaWaves * f->E + 2 * kMetaWaves + 2 * (size_t)f->M * f->top_k) * sizeof(int) > 160 * 1024)) {
         set_error("route_metadata: need E <= 1024, top_k <= E, a valid block_m and M*top_k small enough for LDS");
         return ORX_ERR_BAD_VARIANT;
     }
-    const bool slot_maps = v.boolean("slot_maps", false, &bad);
-    if (bad) return ORX_ERR_BAD_VARIANT;
-    f->flags = slot_maps ? 1 : 0;
+    f->flags = (slot_maps ? kSlotMaps : 0) | (f->takes_workspace ? kSegments : 0);
     f->args = {{"Counts", ArgPointer, 4}, {"IDs", ArgPointer, 4}, {"RelativeSlot", ArgPointer, 4}};
-    if (slot_maps) f->args.push_back({"RowMax", ArgPointer, 4});
+    if (slot_maps) f->args.push_back({"RowMax", ArgPointer, f->takes_workspace ? 0x80000004u : 4u});
     f->args.push_back({"RowOffsets", ArgPointer, 4});
     if (slot_maps) f->args.push_back({"SlotMap", ArgPointer, 4}), f->args.push_back({"SlotToken", ArgPointer, 4});
     for (const ArgSpec& a : std::initializer_list<ArgSpec>{{"TileCount", ArgPointer, 4}, {"TileExpert", ArgPointer, 4},
                                                            {"TileOffsets", ArgPointer, 4}, {"TileRow", ArgPointer, 4}})
         f->args.push_back(a);
+    if (f->takes_workspace) f->args.push_back({"Workspace", ArgPointer, 256u | 0x80000000u}), f->workspace_need = metadata_workspace;
     if (f->dynamic_rows) f->args.push_back({"m", ArgI32, 4});
     f->geometry = metadata_geometry;
     f->launch = metadata_launch;
-    f->device_function = reinterpret_cast<const void*>(&route_metadata_kernel);
+    f->device_function = f->takes_workspace ? reinterpret_cast<const void*>(&segment_rank_kernel)
+                                            : reinterpret_cast<const void*>(&route_metadata_kernel);
     return ORX_OK;
 }
 
@@ -1154,7 +1280,7 @@ const Registration* moe_registrations(int* count) {
      "IDs,Offsets,Slots[,m]"},
     {"expert_offsets", make_offsets, "E=512, block_m=16", "Counts,RowOffsets,TileCount,TileOffsets"},
     {"expert_tiles", make_tiles, "M, E=512, top_k=10, block_m=16", "Counts,TileExpert,TileOffsets,TileRow"},
-    {"route_metadata", make_metadata, "M, E=512, top_k=10, block_m=8, dynamic_rows=false, slot_maps=false",
+    {"route_metadata", make_metadata, "M, E=512, top_k=10, block_m=8, dynamic_rows=false, slot_maps=false, workspace=false",
      "Counts,IDs,RelativeSlot[,RowMax],RowOffsets[,SlotMap,SlotToken],TileCount,TileExpert,TileOffsets,TileRow[,m]"},
     {"single_route_metadata", make_single_metadata, "E=512, top_k=10, capacity=11",
      "Counts,IDs,Offsets,Relative,TileCount,TileExpert,TileOffsets,TileRow"},

@@ -80,6 +80,13 @@ class QuantizedLinear:
         return self.project(self.quantize(x16, stream), stream)
 
 
+BULK_ROWS = 128  # tile height of the routed projections of long prompts
+# Routed rows per expert from which they beat the 32-row tiles of the seven-launch order (us, seven launches against six):
+# 64 experts x top-6, H 3072, I 256: 73 / 76 at 24 rows, 87 / 85 at 48, 136 / 99 at 96; 16 x top-2, H 4096, I 1536: 85 / 88 at 32,
+# 121 / 93 at 64, 325 / 171 at 256.  The five-launch order is kept wherever it applies (up to 8192 routed rows).
+BULK_ROWS_PER_EXPERT = 48
+
+
 class MoeLayer:
     """Q2A8 expert layer: token-sort, grouped gate_up, SwiGLU->A8, grouped down, weighted combine."""
 
@@ -173,12 +180,38 @@ class MoeLayer:
             except OrxError as error:
                 if fused_stages or error.code != ORX_ERR_BAD_VARIANT:
                     raise
+        # Long prompts: six launches over tiles of 128 rows (`block_m` is the tile height of the orders above).
+        #   router top-k + A8 of every token's row, metadata in segments (two launches),
+        #   gate_up that gathers the token rows and writes fp16(silu(gate) * up), A8, down, combine.
+        self.bulk = False
+        if (not self.fused_stages and fused_stages is None and not keep_intermediates and signs is None and hidden % 8 == 0
+                and packed_k == 128 and experts <= 1024 and grouped_algorithm == "auto" and assignments >= BULK_ROWS_PER_EXPERT * experts):
+            try:
+                tiles = (assignments + BULK_ROWS - 1) // BULK_ROWS + min(experts, assignments)
+                bulk = dict(rows=assignments, E=experts, tiles=tiles, block_m=BULK_ROWS)
+                self.k_router_a8 = Kernel("router_topk", renormalize=True, quantize_hidden=hidden, **common)
+                self.k_metadata_slots = Kernel("route_metadata", block_m=BULK_ROWS, slot_maps=True, workspace=True, **common)
+                self.k_gate_up_bulk = Kernel("e8p_decode_grouped", N=2 * intermediate, K=hidden, gather=True,
+                                             epilogue="swiglu", **bulk)
+                self.k_act_a8 = Kernel("activation_quantization", K=intermediate)
+                self.k_down_bulk = Kernel("e8p_decode_grouped", N=hidden, K=intermediate, **bulk)
+                self.segments = self.k_metadata_slots.workspace()
+                self.slot_token = torch.empty(assignments, **i32)
+                self.act = torch.empty((assignments, intermediate), **f16)
+                if tiles > self.tile_capacity:
+                    self.tile_expert, self.tile_row = torch.empty(tiles, **i32), torch.empty(tiles, **i32)
+                self.bulk = True
+            except OrxError as error:
+                if error.code != ORX_ERR_BAD_VARIANT:
+                    raise
         self.k_combine = Kernel("moe_combine", H=hidden, slots=assignments, **common)
 
     def run(self, x16, logits, stream=None):
         s = current_stream() if stream is None else stream
         if self.fused_stages:
             return self._run_fused(x16, logits, s)
+        if self.bulk:
+            return self._run_bulk(x16, logits, s)
         self.k_router(stream=s, IDs=self.ids, Logits=logits, Prob=self.prob)
         if self.k_metadata is not None:
             self.k_metadata(stream=s, Counts=self.counts, IDs=self.ids, RelativeSlot=self.relative,
@@ -210,6 +243,21 @@ class MoeLayer:
                        SlotMap=self.slot_map)
         return self.out
 
+    def _run_bulk(self, x16, logits, s):
+        self.k_router_a8(stream=s, IDs=self.ids, Logits=logits, Prob=self.prob, Q=self.a_q, S=self.a_s, X=x16)
+        self.k_metadata_slots(stream=s, Counts=self.counts, IDs=self.ids, RelativeSlot=self.relative, RowMax=None,
+                              RowOffsets=self.row_offsets, SlotMap=self.slot_map, SlotToken=self.slot_token,
+                              TileCount=self.tile_count, TileExpert=self.tile_expert, TileOffsets=self.tile_offsets,
+                              TileRow=self.tile_row, Workspace=self.segments)
+        routed = dict(Book=self.book, Counts=self.counts, Offsets=self.row_offsets, TileCount=self.tile_count,
+                      TileExpert=self.tile_expert, TileRow=self.tile_row)
+        self.k_gate_up_bulk(stream=s, A=self.a_q, AS=self.a_s, Act=self.act, C=None, P=self.w1, RowMax=None,
+                            SlotToken=self.slot_token, WS=self.s1, **routed)
+        self.k_act_a8(stream=s, Mask=None, Q=self.h_q, S=self.h_s, X=self.act, rows=self.assignments)
+        self.k_down_bulk(stream=s, A=self.h_q, AS=self.h_s, C=self.down_out, P=self.w2, WS=self.s2, **routed)
+        self.k_combine(stream=s, Expert=self.down_out, Output=self.out, Prob=self.prob, Shared=None, SharedGate=None,
+                       SlotMap=self.slot_map)
+        return self.out
 
     def _run_fused(self, x16, logits, s):
         keep = self.keep_intermediates

@@ -111,6 +111,40 @@ def test_route_metadata_one_launch(m, e, k, bm, repeats):
     np.testing.assert_array_equal(gu.host(out["TileRow"]), want_tr)
 
 
+@pytest.mark.parametrize("m,e,k,bm", [(1, 3, 1, 128), (128, 128, 8, 128), (129, 128, 8, 32), (700, 1024, 3, 8), (5000, 7, 2, 128),
+                                      (4096, 64, 6, 128)])
+def test_route_metadata_in_segments(m, e, k, bm):
+    """workspace=True: the same metadata from segments of 1024 assignments, live rows below the capacity, repeated routes."""
+    rng = np.random.default_rng(orc.SEED + m + e)
+    ids_np = rng.integers(0, e, (m, k)).astype(np.int32)
+    ids_np[:, 0] = np.minimum(ids_np[:, 0], e // 2)
+    cap_rows = m + 3
+    kern = gu.kernel("route_metadata", M=cap_rows, E=e, top_k=k, block_m=bm, dynamic_rows=True, slot_maps=True, workspace=True)
+    padded = np.zeros((cap_rows, k), np.int32)
+    padded[:m] = ids_np
+    cap = orc.tile_capacity(cap_rows * k, e, bm)
+    out = {name: torch.full(shape, -1, **I32) for name, shape in
+           (("Counts", (e,)), ("RelativeSlot", (cap_rows, k)), ("RowOffsets", (e,)), ("TileCount", (1,)),
+            ("TileExpert", (cap,)), ("TileOffsets", (e,)), ("TileRow", (cap,)), ("SlotMap", (cap_rows, k)),
+            ("SlotToken", (cap_rows * k,)), ("RowMax", (cap_rows * k,)))}
+    kern(IDs=gu.dev(padded), m=m, **out)
+    want_counts, want_rel = orc.expert_histogram(ids_np, e)
+    want_rows, want_tiles, want_total = orc.expert_offsets(want_counts, bm)
+    want_te, want_tr = orc.expert_tiles(want_counts, want_tiles, bm, cap)
+    slots = want_rows[ids_np] + want_rel
+    token_of = np.empty(m * k, np.int32)
+    token_of[slots.ravel()] = np.repeat(np.arange(m), k)
+    for name, want in (("Counts", want_counts), ("RowOffsets", want_rows), ("TileOffsets", want_tiles), ("TileCount", want_total),
+                       ("TileExpert", want_te), ("TileRow", want_tr)):
+        np.testing.assert_array_equal(gu.host(out[name]), want, err_msg=name)
+    for name, want in (("RelativeSlot", want_rel), ("SlotMap", slots)):
+        np.testing.assert_array_equal(gu.host(out[name])[:m], want, err_msg=name)
+        assert (gu.host(out[name])[m:] == -1).all()
+    np.testing.assert_array_equal(gu.host(out["SlotToken"])[: m * k], token_of)
+    assert (gu.host(out["RowMax"])[: m * k] == 0).all() and (gu.host(out["RowMax"])[m * k :] == -1).all()
+    kern(IDs=gu.dev(padded), m=m, **{**out, "RowMax": None})
+
+
 @pytest.mark.parametrize("algorithm", ["auto", "mfma"])
 @pytest.mark.parametrize("packed_k", [128, 64, 0])
 @pytest.mark.parametrize("bm", [32, 64, 128])
@@ -229,6 +263,60 @@ def test_grouped_q2_resident_kernel(case, packed_k):
     assert (got[lo:hi] == 55).all()
     np.testing.assert_array_equal(got[:lo], want[:lo])
     np.testing.assert_array_equal(got[hi:rows], want[hi:])
+
+
+@pytest.mark.parametrize("form", ["plain", "swiglu"])
+@pytest.mark.parametrize("n,k,counts", [
+    (128, 128, [0, 1, 16, 17, 33, 65, 0, 2]),                   # one K chunk, every number of row blocks, a wave without channels
+    (320, 384, [128, 129, 64, 0, 300, 32]),                     # an odd number of chunks, remainders behind whole tiles
+    (576, 256, [127, 31, 257, 5, 96]), (2176, 512, [48, 0, 130]),   # more than one span of channels
+])
+def test_grouped_q2_bulk_kernel(n, k, counts, form):
+    """Lists of 128-row tiles: rows in slot order, or gathered by slot with the SwiGLU epilogue, bit for bit."""
+    rng = np.random.default_rng(orc.SEED + n + k)
+    e, bm, swiglu = len(counts), 128, form == "swiglu"
+    counts_np = np.array(counts, np.int32)
+    rows, tokens = int(counts_np.sum()), 37
+    codes = rng.integers(0, 65536, (e, n, k // 8), dtype=np.uint16)
+    ws = rng.uniform(0.5, 1.5, (e, n)).astype(np.float16) * np.float16(0.05 / np.sqrt(k))
+    source = rng.integers(0, tokens, rows).astype(np.int32) if swiglu else np.arange(rows, dtype=np.int32)
+    a_q = rng.integers(-127, 128, (tokens if swiglu else rows, k), dtype=np.int8)
+    a_q[0, :2] = [-128, 127]
+    a_s = rng.uniform(0.01, 0.03, len(a_q)).astype(np.float16)
+    offsets_np, tile_offsets, total = orc.expert_offsets(counts_np, bm)
+    cap = orc.tile_capacity(rows, e, bm) + 3  # more room than tiles, as a layer has
+    te, tr = orc.expert_tiles(counts_np, tile_offsets, bm, cap)
+    w = np.stack([orc.q2_integers(c, TABLE) for c in codes])
+    want = orc.grouped_project(a_q[source], a_s[source][:, None], w, ws, counts_np, offsets_np)
+    out = torch.full((rows + 1, n), 55.0, dtype=torch.float16, device=gu.DEV)
+    args = dict(A=gu.dev(a_q), AS=gu.dev(a_s), Book=gu.book(), C=out, Counts=gu.dev(counts_np), Offsets=gu.dev(offsets_np),
+                P=gu.dev(np.stack([orc.q2_pack_k128(c) for c in codes])), TileCount=gu.dev(total), TileExpert=gu.dev(te),
+                TileRow=gu.dev(tr), WS=gu.dev(ws))
+    variant = dict(rows=rows, E=e, tiles=cap, N=n, K=k, block_m=bm)
+    if not swiglu:
+        kern = gu.kernel("e8p_decode_grouped", **variant)
+        kern(**args)
+        np.testing.assert_array_equal(gu.host(out)[:rows], want)
+        shifted = torch.full(((rows + 1) * n + 1,), 55.0, dtype=torch.float16, device=gu.DEV)[1:].view(rows + 1, n)
+        kern(**{**args, "C": shifted})  # an output aligned to its elements only
+        assert torch.equal(shifted, out) and bool((out[rows] == 55).all())
+        args["TileCount"].zero_()
+        out.fill_(7)
+        kern(**args)
+        assert bool((out == 7).all())
+        return
+    kern = gu.kernel("e8p_decode_grouped", gather=True, epilogue="swiglu", **variant)
+    act = torch.full((rows + 1, n // 2), 55.0, dtype=torch.float16, device=gu.DEV)
+    row_max = torch.zeros(rows + 1, dtype=torch.int32, device=gu.DEV)
+    kern(Act=act, RowMax=row_max, SlotToken=gu.dev(source), **args)
+    np.testing.assert_array_equal(gu.host(out)[:rows], want)
+    product = torch.empty((rows, n // 2), dtype=torch.float16, device=gu.DEV)
+    gu.kernel("swiglu", I=n // 2)(X=out, Y=product, rows=rows)  # the device's own SwiGLU of the fp16 gate | up rows
+    assert torch.equal(act[:rows], product) and bool((act[rows] == 55).all()) and bool((out[rows] == 55).all())
+    np.testing.assert_array_equal(gu.host(row_max)[:rows].view(np.float32), gu.host(product.abs().amax(1)).astype(np.float32))
+    lean = torch.full_like(act, 55.0)
+    kern(Act=lean, RowMax=None, SlotToken=gu.dev(source), **{**args, "C": None})
+    assert torch.equal(lean, act)
 
 
 def test_grouped_resident_rejects_shapes_it_cannot_take():
@@ -1022,6 +1110,27 @@ def test_five_launches_at_the_largest_gathered_batch_give_the_bits_of_seven():
     layer = programs.MoeLayer(1025, bigger["experts"], bigger["top_k"], bigger["hidden"], bigger["intermediate"],
                               bigger["gate_up"], bigger["gate_up_scales"], bigger["down"], bigger["down_scales"], block_m=32)
     assert not layer.fused_stages
+
+
+def test_long_prompt_program_gives_the_bits_of_seven_launches():
+    """From 8193 slots on the layer runs over 128-row tiles (six launches), eagerly and replayed."""
+    c = workloads.config3(tokens=1025)
+    x, logits = gu.dev(c["x"]), gu.dev(c["logits"])
+    args = (1025, c["experts"], c["top_k"], c["hidden"], c["intermediate"], c["gate_up"], c["gate_up_scales"], c["down"], c["down_scales"])
+    seven, six = programs.MoeLayer(*args, fused_stages=False), programs.MoeLayer(*args)
+    assert six.bulk and not seven.bulk
+    want = seven.run(x, logits).clone()
+    assert torch.equal(six.run(x, logits), want)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    gu.sync()
+    with torch.cuda.graph(graph, stream=stream):
+        six.run(x, logits, stream=stream.cuda_stream)
+    for _ in range(3):
+        six.out.fill_(float("nan"))
+        six.counts.fill_(-7)
+        graph.replay()
+        gu.sync()
+        assert torch.equal(six.out, want)
 
 
 # The selector decoder's whole domain, after tests/cuda/operators/e8p_selector.py:23-94: tables drawn from
