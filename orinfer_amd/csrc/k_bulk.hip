@@ -15,10 +15,8 @@
 //    it multiplies 32 times.  Tiles of at most 64 or 32 rows take 4 or 2 row blocks.
 //  * Token rows come through LDS by direct loads in whole cache lines (K chunks of 128, two slots of 16 KiB); with GATHER
 //    the rows are those of the slots' tokens, so no launch copies a token's row top_k times.
-//  * Entry i of both tables lies in 128 bytes, eight copies of the basis entry in front of eight of the mask entry; of 16
-//    neighbouring lanes eight read one table and eight the other, each its own copy, so they never collide (two tables of eight
-//    copies, read one after the other: half as many conflict cycles again; sixteen copies of each leave room for one
-//    workgroup per CU).
+//  * The two tables share 32 KiB without conflicts (PairedLookup); two tables of eight copies, read one after the other, had half
+//    as many conflict cycles again, and sixteen copies of each leave room for one workgroup per CU.
 // Measured at 4096 tokens x top-8 of 128 experts (H = 2048, I = 512; popularity of the experts like 1 / rank^1.1):
 // gate_up 296 -> 100 us, down 215 -> 86 us.  What bounds it now: no pipe is full (LDS 42 %, vector ALU 40 %, matrix pipe
 // 30 % of the cycles); the two waves of a SIMD wait for each other's LDS reads and barriers in a third of theirs.
@@ -32,18 +30,18 @@
 
 #include "a8_device.h"
 #include "e8p_device.h"
+#include "lds_asm.h"
 #include "orx_internal.h"
 
 namespace orx {
 namespace {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef unsigned int v2u __attribute__((ext_vector_type(2)));
+using namespace lds_asm;
 
 constexpr int kThreads = 256;
 constexpr int kTileRows = 128;
 constexpr int kSpan = 256;  // output channels of a unit (SWIGLU: 128 gate + 128 up)
-constexpr uint32_t kTokens = 256 * 128;  // behind the tables: 256 entries of 8 copies of basis, 8 of mask
+constexpr uint32_t kTokens = kPairedTableBytes;
 constexpr uint32_t kSlot = kTileRows * 128;
 constexpr uint32_t kTokenScale = kTokens + 2 * kSlot;
 constexpr uint32_t kChannelScale = kTokenScale + kTileRows * 4;
@@ -67,41 +65,9 @@ struct BulkParams {
     int n, k, tile_capacity, spans;
 };
 
-__device__ __forceinline__ int swizzle(int row) { return (row >> 1) & 7; }
-__device__ __forceinline__ uint32_t lds_address_of(const void* pointer) {
-    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)pointer;
-}
-__device__ __forceinline__ void direct_load_16(const void* global, void* lds_wave_base) {
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)global,
-                                     (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, 0);
-}
-// LDS and code reads from asm statements, waited for by hand: the compiler waits for every direct-to-LDS load in flight in
-// front of an LDS read it can see.
-template <int OFFSET>
-__device__ __forceinline__ void lds_read_16(v4i& value, uint32_t address) {
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(value) : "v"(address), "n"(OFFSET));
-}
-template <int OFFSET>
-__device__ __forceinline__ void lds_read_8(v2u& value, uint32_t address) {
-    asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(value) : "v"(address), "n"(OFFSET));
-}
-template <int OFFSET>
-__device__ __forceinline__ void load_8(v2u& value, uint32_t lane_offset, const uint8_t* uniform_base) {
-    asm volatile("global_load_dwordx2 %0, %1, %2 offset:%3"
-                 : "=v"(value)
-                 : "v"(lane_offset), "s"(uniform_base), "n"(OFFSET)
-                 : "memory");
-}
 __device__ __forceinline__ uint32_t pack2(__half low, __half high) {
     return (uint32_t)__half_as_ushort(low) | (uint32_t)__half_as_ushort(high) << 16;
 }
-template <typename T>
-__device__ __forceinline__ T* uniform_pointer(T* pointer) {
-    const uint64_t bits = reinterpret_cast<uint64_t>(pointer);
-    const uint32_t low = __builtin_amdgcn_readfirstlane((uint32_t)bits), high = __builtin_amdgcn_readfirstlane((uint32_t)(bits >> 32));
-    return reinterpret_cast<T*>((uint64_t)high << 32 | low);
-}
-
 template <bool GATHER, bool SWIGLU>
 __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p) {
     extern __shared__ __align__(16) uint8_t lds[];
@@ -177,12 +143,8 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
 
         // ---- tables, scales (beside the first loads) ----
         {
-            const uint2 basis = byte_basis_signed(selector), mask = byte_mask_signed((uint32_t)tid);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                *reinterpret_cast<uint4*>(lds + tid * 128 + 16 * i) = make_uint4(basis.x, basis.y, basis.x, basis.y);
-                *reinterpret_cast<uint4*>(lds + tid * 128 + 64 + 16 * i) = make_uint4(mask.x, mask.y, mask.x, mask.y);
-            }
+            write_paired_entry(lds, tid, false, byte_basis_signed(selector));
+            write_paired_entry(lds, tid, true, byte_mask_signed((uint32_t)tid));
             if (tid < kTileRows) {
                 const int slot = row0 + min(tid, rows - 1);
                 reinterpret_cast<float*>(lds + kTokenScale)[tid] = __half2float(p.as[GATHER ? p.slot_token[slot] : slot]);
@@ -200,11 +162,7 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
 
         // ---- LDS reads ----
         const uint32_t lds_base = lds_address_of(lds);
-        // Lookups: half of the lanes read the basis entry of a code while the others read its mask entry, then the other
-        // way round (the two are XORed, so it does not matter which came first).
-        const uint32_t other = (uint32_t)(lane >> 3) & 1;
-        const uint32_t first_table = lds_base + (uint32_t)(lane & 7) * 8 + other * 64, second_table = first_table ^ 64u;
-        const uint32_t first_bit = 8 - 8 * other, second_bit = 8 - first_bit;  // byte of a code that indexes it
+        const PairedLookup tables(lds_base, lane);
         const uint32_t frag = lds_base + kTokens + (uint32_t)(lane & 15) * 128 + (uint32_t)(((lane >> 4) ^ swizzle(lane & 15)) * 16);
         v4i token[2][RB];  // fragments of even and odd phases
         auto read_tokens = [&](auto phase_tag, uint32_t address) {
@@ -212,21 +170,20 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
             lds_read_16<PHASE * RB * 2048>(token[PHASE & 1][0], address);
             if constexpr (RB > 1) lds_read_16<PHASE * RB * 2048 + 2048>(token[PHASE & 1][1], address);
         };
-        v2u looked[4 * LB];
+        v2u looked[LB][2][2];
         auto lookup = [&](int at, uint32_t word) {  // both entries of two codes
-            lds_read_8<0>(looked[4 * at + 0], (__builtin_amdgcn_ubfe(word, first_bit, 8) << 7) + first_table);
-            lds_read_8<0>(looked[4 * at + 1], (__builtin_amdgcn_ubfe(word, second_bit, 8) << 7) + second_table);
-            lds_read_8<0>(looked[4 * at + 2], (__builtin_amdgcn_ubfe(word, first_bit + 16, 8) << 7) + first_table);
-            lds_read_8<0>(looked[4 * at + 3], (__builtin_amdgcn_ubfe(word, second_bit + 16, 8) << 7) + second_table);
+            tables.read<0>(looked[at][0], word);
+            tables.read<1>(looked[at][1], word);
         };
         auto combine = [&](int at) {
-            const v2u* e = looked + 4 * at;
-            return v4i{(int)(e[0][0] ^ e[1][0]), (int)(e[0][1] ^ e[1][1]), (int)(e[2][0] ^ e[3][0]), (int)(e[2][1] ^ e[3][1])};
+            const v2u first = looked[at][0][0] ^ looked[at][0][1], second = looked[at][1][0] ^ looked[at][1][1];
+            return v4i{(int)first[0], (int)first[1], (int)second[0], (int)second[1]};
         };
         auto wait_reads = [&]() {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-            for (int i = 0; i < 4 * LB; ++i) asm volatile("" : "+v"(looked[i]));
+            for (int l = 0; l < LB; ++l)
+                asm volatile("" : "+v"(looked[l][0][0]), "+v"(looked[l][0][1]), "+v"(looked[l][1][0]), "+v"(looked[l][1][1]));
 #pragma unroll
             for (int i = 0; i < RB; ++i) asm volatile("" : "+v"(token[0][i]), "+v"(token[1][i]));
         };

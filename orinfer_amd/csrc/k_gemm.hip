@@ -47,6 +47,11 @@ bool dense_resident_eligible(int n, int k, int packed_k);
 void dense_resident_geometry(int rows, int n, int k, int packed_k, Geometry* g);
 int dense_resident_launch(const int8_t* a, const void* w, const uint32_t* book, const __half* ws, const __half* as,
                           void* out, int rows, int n, int k, int stride, int packed_k, bool out_f32, hipStream_t stream);
+bool runs_eligible(int codec, int rows, int n, int k);
+int runs_rounds(int codec, int rows, int n, int* tile_rows);
+void runs_geometry(int codec, int rows, int n, Geometry* g);
+int runs_launch(int codec, const int8_t* a, const void* w, const uint32_t* book, const __half* ws, const __half* as, void* out,
+                int rows, int n, int k, int stride, int packed_k, bool out_f32, hipStream_t stream);
 bool dense_wide_eligible(int n, int k, int packed_k);
 void dense_wide_geometry(int n, Geometry* g);
 int dense_wide_launch(const int8_t* a, const void* w, const uint32_t* book, const __half* ws, const __half* as, void* out,
@@ -83,7 +88,7 @@ typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
 enum Codec { kQ4 = 0, kQ2 = 1, kW8 = 2, kS4 = 3 };  // kS4: row-scaled scalar Q4 nibbles (q4_projection.py)
-enum Algorithm { kAuto = 0, kGemv = 1, kMfma = 2, kStream = 3, kResident = 4, kWide = 5, kTall = 6 };
+enum Algorithm { kAuto = 0, kGemv = 1, kMfma = 2, kStream = 3, kResident = 4, kWide = 5, kTall = 6, kRuns = 7 };
 // orx_function::flags2 of a projection.  kPreferGemv / kNoGemv: the reference's schedule names as hints among the
 // library's own kernels (algorithm=dp4a: its dot-product schedule for few rows; tensor_core: its matrix-unit one).
 enum Flags2 { kNoSplit = 1, kNoExpand = 2, kPreferGemv = 4, kNoGemv = 8 };
@@ -692,6 +697,35 @@ int tile_for(const orx_function& f, int rows) {
     return f.tile_hint && rows <= f.tile_hint ? f.tile_hint : 0;
 }
 
+// Channel runs with K split over the waves (k_runs.hip), `algorithm=runs` by name, and by `auto` from two rows on while the
+// workgroups fit one round of the CUs (up to 64 rows: any number, the tiles are low).  Measured against what `auto` launched
+// before (us, N x K, 256 CUs):
+//   int8: 5120 x 17408 24 / 64 / 96 / 128 rows 32 -> 23, 45 -> 32, 46 -> 41, 47 -> 49; 17408 x 5120 24 / 64 rows 32 -> 21, 48 -> 27;
+//     4096 x 4096 32 / 96 / 256 rows 9.8 -> 7.3, 19 -> 11, 22 -> 14; 1024 x 17408 16 / 64 rows three times faster; level
+//     with the streaming kernel where that has a whole number of workgroups per CU (8192 x 8192, 4-16 rows: 0.92-0.96) or
+//     little to stream (1024 x 1024 up to 32 rows: 0.92-0.98): left there.
+//   two-stage codes: 48 / 64 rows 17408 x 5120 31 -> 21, 31 -> 23, 7168 x 5120 12.7 -> 11.1, 14.8 -> 12.3; 96 / 128 / 200 / 256
+//     rows 7168 x 5120 22 -> 17, 25 -> 21, 36 -> 28, 36 -> 31; 4096 x 8192 200 rows 1.4, 1024 x 1024 200 rows 2.9 times faster; wider
+//     matrices go to the channel runs over all rows (11008 x 4096 at 128 / 256 rows 0.96 / 0.87).  Up to 32 rows the
+//     batched-decode kernels are faster where they take K (17408 x 5120: 0.8-0.9), and slower where the
+//     streaming kernel stands in for them (2560 x 9728 and 2048 x 16384: 1.1-2.4).
+// Above 128 rows K = 1024 and row tiles of more than 120 rows stay with the split tiles, whose callers provide a Workspace.
+bool use_runs(const orx_function& f, int rows) {
+    if (f.algorithm == kRuns) return runs_eligible(f.flags, rows, f.N, f.K);
+    if (f.algorithm != kAuto || tile_for(f, rows) != 0 || rows < 2 || f.K % kBK != 0 || !runs_eligible(f.flags, rows, f.N, f.K)) return false;
+    if ((f.flags2 & kPreferGemv) && f.block_m > 0 && rows <= 4) return false;  // the dot-product family wherever it serves the rows
+    const int64_t weights = (int64_t)f.N * f.K;
+    if (rows > 64) {
+        int tile_rows = 0;
+        if (runs_rounds(f.flags, rows, f.N, &tile_rows) != 1 || (f.flags2 & kNoSplit)) return false;
+        if (rows > 128 && (f.K <= 1024 || tile_rows > 120)) return false;
+        return f.flags == kW8 ? rows <= 112 || f.K <= 8192 : f.N <= 32 * device_compute_units();
+    }
+    if (f.flags == kW8) return rows > 32 || (weights >= (1 << 22) && (rows > 16 || f.N % (32 * device_compute_units()) != 0));
+    if (rows > 32) return weights >= (1 << 22);
+    return f.K > 5120 && f.N <= 32 * device_compute_units();
+}
+
 // Channel runs per CU over the whole K (k_wide.hip): two-stage codes, `algorithm=wide` by name, and by
 // `auto` at 65..128 rows (33..64 rows of large matrices) while K is short enough.  Its time is 10 us + 0.4..0.55 us per K step of 128 whatever
 // N is (up to 96 channels per CU), where the split 128 x 128 tiles pay for N K: measured at 65-128 rows,
@@ -883,6 +917,7 @@ uint64_t big_rest_workspace(const orx_function& f, int rows) {
 // two-stage launch on the 256-row tiles (and behind them the partial slots of the channels that the
 // persistent launch leaves to the split tiles).
 uint64_t projection_workspace(const orx_function& f, int rows) {
+    if (use_runs(f, rows)) return 0;
     if (use_wide(f, rows) || use_tall(f, rows)) return 0;
     if (use_gemv(f, rows) || use_resident(f, rows) || use_stream(f, rows)) return 0;
     if (use_expand(f, rows)) return (uint64_t)f.N * f.K + big_rest_workspace(f, rows);
@@ -902,6 +937,10 @@ int launch_split(const GemmParams& p, int groups, hipStream_t stream) {
 }
 
 int projection_geometry(const orx_function& f, int rows, Geometry* g) {
+    if (use_runs(f, rows)) {
+        runs_geometry(f.flags, rows, f.N, g);
+        return ORX_OK;
+    }
     if (use_wide(f, rows)) {
         dense_wide_geometry(f.N, g);
         return ORX_OK;
@@ -969,6 +1008,8 @@ int q4_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t st
     p.w = pointer_arg<const void>(args, f.rotate_input ? 6 : 5);
     void* workspace = f.takes_workspace ? pointer_arg<void>(args, f.workspace_arg) : nullptr;
     p.n = f.N, p.k = f.K, p.stride = f.stride, p.m = rows, p.packed_k = f.packed_k, p.out_f32 = f.out_f32;
+    if (use_runs(f, rows))
+        return runs_launch(kQ4, p.a, p.w, p.book, p.ws, p.as, p.out, rows, f.N, f.K, f.stride, f.packed_k, f.out_f32, stream);
     if (use_wide(f, rows))
         return dense_wide_launch(p.a, p.w, p.book, p.ws, p.as, p.out, rows, f.N, f.K, f.stride, f.packed_k, f.out_f32, g, stream);
     if (use_tall(f, rows))
@@ -1019,6 +1060,8 @@ int w8_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t st
     p.book = nullptr;
     void* workspace = f.takes_workspace ? pointer_arg<void>(args, f.workspace_arg) : nullptr;
     p.n = f.N, p.k = f.K, p.stride = f.stride, p.m = rows, p.packed_k = 0, p.out_f32 = f.out_f32;
+    if (use_runs(f, rows))
+        return runs_launch(kW8, p.a, p.w, nullptr, p.ws, p.as, p.out, rows, f.N, f.K, f.stride, 0, f.out_f32, stream);
     if (use_gemv(f, rows)) return gemv_launch(f, rows, g, stream, p.a, p.w, p.book, p.ws, p.as, p.out);
     if (use_stream(f, rows)) {
         for (int first = 0; first < rows; first += 64) {
@@ -1101,14 +1144,19 @@ int make_projection(const Variant& v, orx_function* f, int codec) {
                    : algorithm == "resident" ? kResident
                    : algorithm == "wide"     ? kWide
                    : algorithm == "tall"     ? kTall
+                   : algorithm == "runs"     ? kRuns
                    : algorithm == "auto"     ? kAuto
                                              : -1;
     if (f->algorithm < 0) {
-        set_error("%s: algorithm must be auto, gemv, stream, resident, wide, tall or mfma", name);
+        set_error("%s: algorithm must be auto, gemv, stream, resident, wide, tall, runs or mfma", name);
         return ORX_ERR_BAD_VARIANT;
     }
     if (f->algorithm == kTall && (codec != kQ4 || f->K % 128 != 0 || f->K < 256)) {
         set_error("%s: algorithm=tall serves two-stage codes with K a multiple of 128, at least 256", name);
+        return ORX_ERR_BAD_VARIANT;
+    }
+    if (f->algorithm == kRuns && (f->K % 128 != 0 || !runs_eligible(codec, f->capacity, f->N, f->K))) {
+        set_error("%s: algorithm=runs serves up to 512 rows, K a multiple of 128", name);
         return ORX_ERR_BAD_VARIANT;
     }
     if (f->algorithm == kWide && (codec != kQ4 || !dense_wide_eligible(f->N, f->K, f->packed_k))) {

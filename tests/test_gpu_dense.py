@@ -1428,3 +1428,47 @@ def test_scalar_q4_other_magnitudes_extremes_and_unpack():
     gu.kernel("unpack_q4", N=n, K=k, magnitudes=magnitudes)(Output=unpacked, W=gu.dev(words))
     np.testing.assert_array_equal(gu.host(unpacked)[:n], weights)
     assert bool((unpacked[n] == 55).all())
+
+
+# ---- channel runs with K split over the waves -------------------------------------------------------------------
+# Token blocks of 16 (1 to 8 to a tile, up to four tiles), channel blocks (1 to 5 to a run, partly filled, a short last run),
+# fewer K chunks than waves and remainders of the ring.
+@pytest.mark.parametrize("rows,n,k", [(1, 16, 128), (2, 40, 256), (16, 1000, 1152), (17, 5120, 384), (33, 4112, 640), (48, 12288, 256),
+                                      (63, 20480, 128), (64, 768, 2304), (65, 7168, 384), (96, 2048, 1280), (112, 5136, 256),
+                                      (113, 300, 896), (128, 1024, 1152), (131, 2560, 1408), (200, 7168, 256), (257, 1000, 384),
+                                      (512, 520, 256)])
+@pytest.mark.parametrize("packed_k", [128, 64, 0])
+def test_channel_runs_two_stage_codes(rows, n, k, packed_k):
+    rng = np.random.default_rng(orc.SEED + rows + n + k)
+    packed = rng.integers(0, 2**32, (n, k // 8), dtype=np.uint32)
+    a_q = rng.integers(-127, 128, (rows, k), dtype=np.int8)
+    a_q[0, :2] = [-128, 127]
+    a_s = rng.uniform(0.005, 0.02, rows).astype(np.float16)
+    ws = rng.uniform(0.005, 0.02, n).astype(np.float16)
+    stored = packed if packed_k == 0 else orc.q4_pack_k(packed, packed_k)
+    got = gu.q4_project(gu.dev(a_q), gu.dev(a_s), gu.dev(stored), gu.dev(ws), packed_k=packed_k, algorithm="runs")
+    np.testing.assert_array_equal(gu.host(got), orc.project(a_q, a_s, orc.q4_integers(packed, TABLE), ws))
+
+
+@pytest.mark.parametrize("rows,n,k", [(1, 16, 128), (2, 40, 256), (16, 1000, 1152), (17, 5120, 384), (33, 4112, 640), (48, 12288, 256),
+                                      (63, 20480, 128), (64, 768, 2304), (65, 7168, 384), (96, 2048, 1280), (112, 5136, 256),
+                                      (128, 1024, 1152), (131, 2560, 1408), (200, 7168, 256), (257, 1000, 384), (512, 520, 256)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32], ids=["fp16", "fp32-strided"])
+def test_channel_runs_int8_weights(rows, n, k, dtype):
+    rng = np.random.default_rng(orc.SEED + rows + n + k)
+    weight = rng.integers(-128, 128, (n, k), dtype=np.int8)
+    a_q = rng.integers(-127, 128, (rows, k), dtype=np.int8)
+    a_s = rng.uniform(0.005, 0.02, rows).astype(np.float16)
+    ws = rng.uniform(0.005, 0.02, n).astype(np.float16)
+    stride = n if dtype == torch.float16 else n + 3
+    out = torch.full((rows + 1, stride), 91, dtype=dtype, device=gu.DEV)
+    gu.w8_project(gu.dev(a_q), gu.dev(a_s), gu.dev(weight), gu.dev(ws), out=out, rows=rows, stride=stride, dtype=dtype, algorithm="runs")
+    want = orc.project(a_q, a_s, weight, ws, out_dtype=np.float16 if dtype == torch.float16 else np.float32)
+    np.testing.assert_array_equal(gu.host(out)[:rows, :n], want)
+    assert (gu.host(out)[rows] == 91).all() and (gu.host(out)[:, n:] == 91).all()
+
+
+def test_channel_runs_refuse_what_they_do_not_serve():
+    for bad in (dict(M=513), dict(K=192)):
+        with pytest.raises(gu.lib.OrxError):
+            gu.kernel("int8_projection", **{**dict(M=8, N=256, K=256, algorithm="runs"), **bad})
