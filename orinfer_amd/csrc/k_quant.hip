@@ -460,29 +460,24 @@ __global__ __launch_bounds__(256) void rotate_kernel(const __half* __restrict__ 
     }
 }
 
-template <int WAVES>
+// Sum over the first four waves, known to all.
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
 #pragma unroll
     for (int offset = 32; offset > 0; offset >>= 1) v += __shfl_xor(v, offset, 64);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (lane == 0) scratch[wave] = v;
+    if (lane == 0 && wave < 4) scratch[wave] = v;
     __syncthreads();
-    float part[WAVES];
-#pragma unroll
-    for (int i = 0; i < WAVES; ++i) part[i] = scratch[i];
-#pragma unroll
-    for (int half = 1; half < WAVES; half *= 2)
-#pragma unroll
-        for (int i = 0; i < WAVES; i += 2 * half) part[i] += part[i + half];
-    return part[0];
+    return (scratch[0] + scratch[1]) + (scratch[2] + scratch[3]);
 }
 
 // Residual add + RMSNorm in front of the rotation, one workgroup per row, same lane layout as
 // rotate_a8_kernel.  First pass: RO = fp32(X) + R, sum of squares.  Second pass: the fp32 sum (kept
 // in registers, or read back by the thread that wrote it where the row is longer than the registers
 // hold), Y = fp16((sum * rsqrt(mean + eps)) * (W + offset)), and that fp16 value goes through signs,
-// butterflies and A8 as if rotate_a8_kernel had read Y.  4 waves (16 when rows are few, as in rotate_a8_kernel: one row
-// of 5120 then takes 4.8 us instead of 7.0, twenty 5.1 instead of 7.7).
+// butterflies and A8 as if rotate_a8_kernel had read Y.  4 waves, or 16 when rows are few, as in rotate_a8_kernel: one row
+// of 5120 then takes 5.0 us instead of 7.0, twenty 5.3 instead of 7.7.  The order of the fp32 sum is that of the 4 waves
+// for both (a code that flips in a row's largest value moves the whole row): the 16 leave their squares in LDS, and the
+// first four add them up as they would have come along.
 template <int THREADS>
 __global__ __launch_bounds__(THREADS) void residual_norm_rotate_a8_kernel(
     const __half* __restrict__ x, const float* __restrict__ r, const __half* __restrict__ w, __half* __restrict__ y,
@@ -490,13 +485,19 @@ __global__ __launch_bounds__(THREADS) void residual_norm_rotate_a8_kernel(
     float epsilon, float weight_offset) {
     extern __shared__ __align__(16) __half rotated[];  // k halves
     constexpr int kWaves = THREADS / 64;
-    __shared__ float scratch[kWaves], sum_scratch[kWaves];
+    __shared__ float scratch[kWaves], sum_scratch[4];
     const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int half_wave = lane >> 5, l32 = lane & 31;
     const int blocks = k / 128;  // even: k is a multiple of 256
     const int64_t base = (int64_t)row * k;
     float squares = 0.f;
-    // The first kHeld steps of a wave (all of them up to K = 5120, 8192 with 16 waves): every load of both passes leaves
+    auto add_squares = [&](const float4& v) {
+        squares += v.x * v.x;
+        squares += v.y * v.y;
+        squares += v.z * v.z;
+        squares += v.w * v.w;
+    };
+    // The first kHeld steps of a wave (all of them up to K = 5120, and always with 16 waves: K <= 8192): every load of both passes leaves
     // at once, and the fp32 sums stay in registers for the second pass.  Longer rows go on in the
     // loops below, which read their sums back.
     constexpr int kHeld = THREADS == 256 ? 5 : 2;
@@ -526,10 +527,10 @@ __global__ __launch_bounds__(THREADS) void residual_norm_rotate_a8_kernel(
             sum.w = __half2float(h[3]) + residual[u].w;
             *reinterpret_cast<float4*>(ro + base + first) = sum;
             kept[u] = sum;
-            squares += sum.x * sum.x;
-            squares += sum.y * sum.y;
-            squares += sum.z * sum.z;
-            squares += sum.w * sum.w;
+            if constexpr (kWaves == 4)
+                add_squares(sum);
+            else
+                reinterpret_cast<float4*>(rotated)[(wave + kWaves * u) * 64 + lane] = sum;
         }
     }
     for (int pair = wave + kWaves * kHeld; 2 * pair < blocks; pair += kWaves) {
@@ -543,12 +544,14 @@ __global__ __launch_bounds__(THREADS) void residual_norm_rotate_a8_kernel(
         sum.z = __half2float(h[2]) + residual.z;
         sum.w = __half2float(h[3]) + residual.w;
         *reinterpret_cast<float4*>(ro + base + first) = sum;
-        squares += sum.x * sum.x;
-        squares += sum.y * sum.y;
-        squares += sum.z * sum.z;
-        squares += sum.w * sum.w;
+        add_squares(sum);
     }
-    const float total = block_sum<kWaves>(squares, sum_scratch);
+    if constexpr (kWaves > 4) {
+        __syncthreads();
+        if (wave < 4)
+            for (int pair = wave; 2 * pair < blocks; pair += 4) add_squares(reinterpret_cast<const float4*>(rotated)[pair * 64 + lane]);
+    }
+    const float total = block_sum(squares, sum_scratch);  // its barrier also ends the reads of the sums in LDS
     const float inverse = rsqrtf(__fdiv_rn(total, (float)k) + epsilon);
     float amax = 0.f;
     auto second_pass = [&](int first, const float4& sum, const uint2& raw_w, uint32_t sign_word) {
@@ -955,8 +958,9 @@ int make_rotate(const Variant& v, orx_function* f) {
 // slots used: K, flags (bit0: weights stored zero-centred), capacity
 int residual_rotate_geometry(const orx_function& f, int rows, Geometry* g) {
     g->grid[0] = (uint32_t)rows;
-    g->block[0] = rows <= kRotateWideRows && f.K >= 2048 ? 1024 : 256;
-    g->shared = (uint32_t)f.K * 2;
+    const bool wide = rows <= kRotateWideRows && f.K >= 2048 && f.K <= 8192;
+    g->block[0] = wide ? 1024 : 256;
+    g->shared = (uint32_t)f.K * (wide ? 4 : 2);  // the rotated fp16 row; before it, where 16 waves share a row, its fp32 sums
     return ORX_OK;
 }
 
