@@ -16,8 +16,12 @@
 //    (rows padded by 16 bytes, so the per-lane 16-byte fragment reads do not collide); fetching
 //    them per lane from L1 costs one cache access per lane and instruction and was the limit of the
 //    streaming kernel this one replaces for large routed batches.
-//  * The two 8-byte table lookups per code are random; each table entry is stored 16 times (entry i
-//    for lane l at byte i*128 + (l%16)*8) so the lanes of one access group never share a bank.
+//  * The two 8-byte table lookups per code are random.  LDS serves 32 lanes of such a read per cycle: entry i of both
+//    tables lies in bytes 256 i, 16 copies of the basis entry and 16 of the mask entry, and of 32 neighbouring lanes 16
+//    read one table while the others read the other, each its own copy, so nothing collides; the second read goes the
+//    other way round (the two are XORed).  One v_perm_b32 builds an address.  (16 copies at 128 i in two tables, all lanes
+//    reading the same one, met in pairs and took twice the cycles.
+//    Gate|up of 256 tokens x top-8, 128 experts, 2048 x 1024: 22.1 -> 20.4 us.)
 //  * Units are dealt to workgroups in contiguous runs (a run mostly stays inside one tile, so the
 //    staged rows are reused).  What does not divide evenly is finished in a second phase where a
 //    32-channel block is split over K between the waves and summed with LDS integer atomics
@@ -38,6 +42,7 @@
 
 #include "a8_device.h"
 #include "e8p_device.h"
+#include "lds_asm.h"
 #include "orx_internal.h"
 
 namespace orx {
@@ -50,8 +55,7 @@ typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 constexpr int kWaves = 16;
 constexpr int kThreads = kWaves * 64;
 constexpr int kSpan = kWaves * 32;             // output channels of one unit
-constexpr uint32_t kBasisBase = 0;             // 256 entries x 16 copies x 8 bytes
-constexpr uint32_t kMaskBase = 32768;
+constexpr uint32_t kMaskOffset = 128;          // 256 entries x (16 copies of basis, 16 of mask) x 8 bytes
 constexpr uint32_t kInfoBase = 65536;          // (expert, first row, rows) of every routed tile
 constexpr int kMaxTiles = 1024;
 constexpr uint32_t kRowStatBase = kInfoBase + kMaxTiles * 12;  // fp16 rows quantised while staged: the scale of every staged row
@@ -144,11 +148,7 @@ __global__ __launch_bounds__(kThreads) void grouped_resident_kernel(GroupedParam
     if (wave < 8) {
         const int entry = tid & 255;
         const uint2 value = wave < 4 ? byte_basis_signed(selector) : byte_mask_signed((uint32_t)entry);
-        const uint4 pair = make_uint4(value.x, value.y, value.x, value.y);
-        // the slot order turns with the entry, or all lanes of a wave would write to the same banks: 2 us of a launch, 0.3 us so
-        uint8_t* dst = lds + (wave < 4 ? kBasisBase : kMaskBase) + entry * 128;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) *reinterpret_cast<uint4*>(dst + 16 * (i ^ (entry & 7))) = pair;
+        lds_asm::write_paired_entry<8>(lds, entry, wave >= 4, value);
     }
     if (kPhaseTwo)
         for (int i = tid; i < split.per_pass * kSumBlock; i += kThreads) sums[i] = 0;
@@ -196,14 +196,18 @@ __global__ __launch_bounds__(kThreads) void grouped_resident_kernel(GroupedParam
     auto fetch = [&](const uint8_t* base, int kb) { return *reinterpret_cast<const uint4*>(base + kb * kb_step); };
 
     // ---- decode ------------------------------------------------------------------------------
-    const uint32_t copy = (uint32_t)(lane & 15) * 8;
-    auto lookup = [&](uint32_t byte) { return *reinterpret_cast<const uint2*>(lds + byte); };
+    // address byte 0: this lane's copy, in the half of an entry it reads first or second; byte 1: the code byte that goes with it
+    const uint32_t copy = (uint32_t)(lane & 15) * 8, other = (uint32_t)(lane >> 4) & 1;
+    const uint32_t columns = (copy | other * kMaskOffset) | (copy | (other ^ 1) * kMaskOffset) << 8;
+    const uint32_t first_low = 0x0C0C0500u - (other << 8), second_low = 0x0C0C0401u + (other << 8);
+    const uint32_t first_high = first_low + 0x200u, second_high = second_low + 0x200u;
+    auto lookup = [&](uint32_t word, uint32_t selector) {
+        return *reinterpret_cast<const uint2*>(lds + __builtin_amdgcn_perm(word, columns, selector));
+    };
     auto decode_pair = [&](uint32_t word) -> v4i {  // two codes -> the 16 weights of one MFMA sub-step
-        const uint2 b0 = lookup(kBasisBase + (((word & 0xFF00u) >> 1) | copy));
-        const uint2 m0 = lookup(kMaskBase + (((word & 0xFFu) << 7) | copy));
-        const uint2 b1 = lookup(kBasisBase + (((word >> 17) & 0x7F80u) | copy));
-        const uint2 m1 = lookup(kMaskBase + (((word >> 9) & 0x7F80u) | copy));
-        return v4i{(int)(b0.x ^ m0.x), (int)(b0.y ^ m0.y), (int)(b1.x ^ m1.x), (int)(b1.y ^ m1.y)};
+        const uint2 a0 = lookup(word, first_low), b0 = lookup(word, second_low);
+        const uint2 a1 = lookup(word, first_high), b1 = lookup(word, second_high);
+        return v4i{(int)(a0.x ^ b0.x), (int)(a0.y ^ b0.y), (int)(a1.x ^ b1.x), (int)(a1.y ^ b1.y)};
     };
 
     // ---- staging of a tile's token rows ------------------------------------------------------
@@ -213,6 +217,11 @@ __global__ __launch_bounds__(kThreads) void grouped_resident_kernel(GroupedParam
     int held_max[INPUT == kInputAct ? kMaxHalfPieces : 1];
     const int row_pieces = p.k / 16;
     const int half_pieces = p.k / 8;  // kInputAct: pieces of 8 fp16 values per row
+    // row of a piece: floor(piece / pieces per row) as piece * ceil(2^20 / d) >> 20, exact while piece * d < 2^20 (32 d^2 here,
+    // d <= 160): two instructions where the division is about twenty, up to 2 x kMaxPieces times per thread and tile
+    const uint32_t per_row = (uint32_t)(INPUT == kInputAct ? half_pieces : row_pieces);
+    const uint32_t magic = __builtin_amdgcn_readfirstlane(((1u << 20) + per_row - 1) / per_row);
+    auto row_of = [&](int piece) { return (int)(__umul24((uint32_t)piece, magic) >> 20); };
     auto stage_load = [&](const Tile& t) {
         // unconditional loads of clamped pieces, so that all of them are in flight together
         const int first_row = t.rows > 0 ? t.row0 : 0;
@@ -226,7 +235,7 @@ __global__ __launch_bounds__(kThreads) void grouped_resident_kernel(GroupedParam
 #pragma unroll
             for (int i = 0; i < kMaxPieces; ++i) {
                 const int piece = min(tid + i * kThreads, last_piece);
-                const int row = piece / row_pieces, col = piece - row * row_pieces;
+                const int row = row_of(piece), col = piece - row * row_pieces;
                 const int64_t token = slot_tokens[first_row + row];
                 held[i] = *reinterpret_cast<const v4u*>(p.a + token * p.k + col * 16);
             }
@@ -235,7 +244,7 @@ __global__ __launch_bounds__(kThreads) void grouped_resident_kernel(GroupedParam
 #pragma unroll
             for (int i = 0; i < kMaxHalfPieces; ++i) {
                 const int piece = min(tid + i * kThreads, last_piece);
-                const int row = piece / half_pieces;
+                const int row = row_of(piece);
                 held[i] = reinterpret_cast<const v4u*>(p.x + (int64_t)first_row * p.k)[piece];
                 held_max[i] = p.row_max_in[first_row + row];
             }
@@ -250,7 +259,7 @@ __global__ __launch_bounds__(kThreads) void grouped_resident_kernel(GroupedParam
             for (int i = 0; i < kMaxPieces; ++i) {
                 const int piece = tid + i * kThreads;
                 if (piece < pieces) {
-                    const int row = piece / row_pieces, col = piece - row * row_pieces;
+                    const int row = row_of(piece), col = piece - row * row_pieces;
                     *reinterpret_cast<v4u*>(lds + tile_base + row * tile_stride + col * 16) = held[i];
                 }
             }
@@ -260,7 +269,7 @@ __global__ __launch_bounds__(kThreads) void grouped_resident_kernel(GroupedParam
             for (int i = 0; i < kMaxHalfPieces; ++i) {
                 const int piece = tid + i * kThreads;
                 if (piece < pieces) {
-                    const int row = piece / half_pieces, col = piece - row * half_pieces;
+                    const int row = row_of(piece), col = piece - row * half_pieces;
                     const __half stored = a8_scale(__int_as_float(held_max[i]));
                     const float scale = __half2float(stored), inverse = __frcp_rn(scale);
                     const __half* h = reinterpret_cast<const __half*>(&held[i]);
