@@ -25,7 +25,7 @@ namespace orx {
 // from k_gemv.hip
 int gemv_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t stream, const int8_t* a,
                 const void* w, const uint32_t* book, const __half* ws, const __half* as, void* out,
-                const int8_t* signs = nullptr);
+                const int8_t* signs = nullptr, int8_t* codes = nullptr);
 int gemv_geometry_for(const orx_function& f, int rows, Geometry* g);
 int gemv_configure(orx_function* f, int codec, int passes_override);
 int gemv_prepare_device();
@@ -1003,9 +1003,11 @@ int q4_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t st
     p.as = pointer_arg<const __half>(args, 1);
     p.book = pointer_arg<const uint32_t>(args, 2);
     p.out = pointer_arg<void>(args, 3);
-    p.ws = pointer_arg<const __half>(args, 4);
-    const int8_t* signs = f.rotate_input ? pointer_arg<const int8_t>(args, 5) : nullptr;
-    p.w = pointer_arg<const void>(args, f.rotate_input ? 6 : 5);
+    int next = 4;  // the optional buffers of the fp16-input form stand between the others, in the order of their names
+    int8_t* codes = f.publish_codes ? pointer_arg<int8_t>(args, next++) : nullptr;
+    p.ws = pointer_arg<const __half>(args, next++);
+    const int8_t* signs = f.rotate_input ? pointer_arg<const int8_t>(args, next++) : nullptr;
+    p.w = pointer_arg<const void>(args, next);
     void* workspace = f.takes_workspace ? pointer_arg<void>(args, f.workspace_arg) : nullptr;
     p.n = f.N, p.k = f.K, p.stride = f.stride, p.m = rows, p.packed_k = f.packed_k, p.out_f32 = f.out_f32;
     if (use_runs(f, rows))
@@ -1014,7 +1016,7 @@ int q4_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t st
         return dense_wide_launch(p.a, p.w, p.book, p.ws, p.as, p.out, rows, f.N, f.K, f.stride, f.packed_k, f.out_f32, g, stream);
     if (use_tall(f, rows))
         return gemm_tall_launch(p.a, p.w, p.book, p.ws, p.as, p.out, rows, f.N, f.K, f.stride, f.packed_k, f.out_f32, g, stream);
-    if (use_gemv(f, rows)) return gemv_launch(f, rows, g, stream, p.a, p.w, p.book, p.ws, p.as, p.out, signs);
+    if (use_gemv(f, rows)) return gemv_launch(f, rows, g, stream, p.a, p.w, p.book, p.ws, p.as, p.out, signs, codes);
     if (use_resident(f, rows)) {
         for (int first = 0; first < rows; first += 32) {
             const size_t out_offset = (size_t)first * f.stride * (f.out_f32 ? 4 : 2);
@@ -1247,8 +1249,15 @@ int make_q4_projection(const Variant& v, orx_function* f) {
         set_error("e8p_q4_projection: rotate=true needs input_dtype=float16");
         return ORX_ERR_BAD_VARIANT;
     }
-    f->args = {{"A", ArgPointer, 16}, {"AS", ArgPointer, 2}, {"Book", ArgPointer, 4},
-               {"Out", ArgPointer, 2}, {"S", ArgPointer, 2}};
+    // codes=true (fp16 input only): Q joins the buffers and receives the int8 codes, as A8 quantiser and projection leave them
+    f->publish_codes = v.boolean("codes", false, &bad);
+    if (bad || (f->publish_codes && !f->input_f16)) {
+        set_error("e8p_q4_projection: codes=true needs input_dtype=float16");
+        return ORX_ERR_BAD_VARIANT;
+    }
+    f->args = {{"A", ArgPointer, 16}, {"AS", ArgPointer, 2}, {"Book", ArgPointer, 4}, {"Out", ArgPointer, 2}};
+    if (f->publish_codes) f->args.push_back({"Q", ArgPointer, 8});
+    f->args.push_back({"S", ArgPointer, 2});
     if (f->rotate_input) f->args.push_back({"Signs", ArgPointer, 8});
     f->args.push_back({"W", ArgPointer, 16});
     if (f->takes_workspace) f->args.push_back({"Workspace", ArgPointer, 256u | 0x80000000u});  // null where no launch needs it
@@ -2057,7 +2066,7 @@ const Registration* gemm_registrations(int* count) {
     static const Registration rows[] = {
     {"e8p_q4_projection", make_q4_projection,
      "M, N, K, dynamic_rows=false, algorithm=auto|gemv|stream|resident|wide|mfma, packed_k=0|64|128, output_dtype=float16|float32, "
-     "input_dtype=int8|float16, rotate=false, workspace=false, split_k=true, "
+     "input_dtype=int8|float16, rotate=false, codes=false, workspace=false, split_k=true, "
      "output_stride=N, block_m=0|32|64|128|256, gemv_passes=0, decode_in_gemm=false",
      "A,AS,Book,Out,S[,Signs],W[,Workspace][,m]"},
     {"int8_projection", make_w8_projection,

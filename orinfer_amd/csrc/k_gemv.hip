@@ -322,12 +322,12 @@ constexpr int kKMajorLayout = 64;
 // X16 (one activation row, K up to 8192): `a` holds the row as fp16 and the kernel quantises it
 // itself during set-up, by the rule of the activation quantiser (row maximum over 127, fp16 scale,
 // round to nearest even); every workgroup does so for itself, the first one also writes the scale
-// to `as`.  That saves the separate launch in front of a single-row projection.
+// to `as` (and the codes to `codes`, unless that is null).  That saves the separate launch in front of a single-row projection.
 template <int CODEC, int MR, int D, int LAYOUT, bool HOLD, bool X16 = false>
 __global__ __launch_bounds__(kBankedThreads) void gemv_banked_kernel(
     const int8_t* __restrict__ a, const uint4* __restrict__ w, const uint32_t* __restrict__ book,
     const __half* __restrict__ ws, const __half* __restrict__ as, void* __restrict__ out, int n, int k, int stride,
-    int m, int flags, const int8_t* __restrict__ signs) {
+    int m, int flags, const int8_t* __restrict__ signs, int8_t* __restrict__ codes) {
     extern __shared__ __align__(16) uint32_t lds[];
     const bool out_f32 = flags & 1;  // bit 1: K-major blocks of 64 instead of 128
     constexpr int LPR = LAYOUT & (kKMajorLayout - 1);
@@ -555,6 +555,7 @@ __global__ __launch_bounds__(kBankedThreads) void gemv_banked_kernel(
                                (__builtin_amdgcn_perm(word[4 * half + 3], word[4 * half + 2], 0x0C0C0400u) << 16);
         }
         raw[0] = make_uint2(packed[0], packed[1]);
+        if (codes != nullptr && blockIdx.x == 0 && tid < groups) *reinterpret_cast<uint2*>(codes + 8 * tid) = raw[0];
     }
     int wave_total[MR];  // sum of this wave's activations, valid in lane 63
 #pragma unroll
@@ -750,9 +751,10 @@ int gemv_geometry(const orx_function& f, int rows, Geometry* g) {
     return ORX_OK;
 }
 
-// Sign vector of the rotation that the fp16-input form applies in front of its quantiser (null: none);
+// The fp16-input form: sign vector of the rotation in front of its quantiser and where its codes go (null: none);
 // set by gemv_launch for the launch it is about to make on this thread.
 static thread_local const int8_t* pending_signs = nullptr;
+static thread_local int8_t* pending_codes = nullptr;
 
 template <int D, int LPR>  // LPR: the kernel's LAYOUT (lanes per row, + 64 for K-major codes)
 int gemv_launch_banked(const orx_function& f, int rows, const Geometry& g, hipStream_t stream, const int8_t* a,
@@ -763,24 +765,24 @@ int gemv_launch_banked(const orx_function& f, int rows, const Geometry& g, hipSt
         case 1:
             if (f.input_f16 && hold)
                 ORX_LAUNCH((gemv_banked_kernel<kQ4, 1, D, LPR, true, true>), grid, block, g.shared, stream, a, w,
-                                   book, ws, as, out, f.N, f.K, f.stride, rows, (int)f.out_f32 | (f.packed_k == 64 ? 2 : 0), pending_signs);
+                                   book, ws, as, out, f.N, f.K, f.stride, rows, (int)f.out_f32 | (f.packed_k == 64 ? 2 : 0), pending_signs, pending_codes);
             else if (f.input_f16)
                 ORX_LAUNCH((gemv_banked_kernel<kQ4, 1, D, LPR, false, true>), grid, block, g.shared, stream, a, w,
-                                   book, ws, as, out, f.N, f.K, f.stride, rows, (int)f.out_f32 | (f.packed_k == 64 ? 2 : 0), pending_signs);
+                                   book, ws, as, out, f.N, f.K, f.stride, rows, (int)f.out_f32 | (f.packed_k == 64 ? 2 : 0), pending_signs, pending_codes);
             else if (hold)
                 ORX_LAUNCH((gemv_banked_kernel<kQ4, 1, D, LPR, true>), grid, block, g.shared, stream, a, w, book,
-                                   ws, as, out, f.N, f.K, f.stride, rows, (int)f.out_f32 | (f.packed_k == 64 ? 2 : 0), pending_signs);
+                                   ws, as, out, f.N, f.K, f.stride, rows, (int)f.out_f32 | (f.packed_k == 64 ? 2 : 0), pending_signs, pending_codes);
             else
                 ORX_LAUNCH((gemv_banked_kernel<kQ4, 1, D, LPR, false>), grid, block, g.shared, stream, a, w, book,
-                                   ws, as, out, f.N, f.K, f.stride, rows, (int)f.out_f32 | (f.packed_k == 64 ? 2 : 0), pending_signs);
+                                   ws, as, out, f.N, f.K, f.stride, rows, (int)f.out_f32 | (f.packed_k == 64 ? 2 : 0), pending_signs, pending_codes);
             break;
         case 2:
             ORX_LAUNCH((gemv_banked_kernel<kQ4, 2, D, LPR, false>), grid, block, g.shared, stream, a, w, book, ws,
-                               as, out, f.N, f.K, f.stride, rows, (int)f.out_f32 | (f.packed_k == 64 ? 2 : 0), pending_signs);
+                               as, out, f.N, f.K, f.stride, rows, (int)f.out_f32 | (f.packed_k == 64 ? 2 : 0), pending_signs, pending_codes);
             break;
         default:
             ORX_LAUNCH((gemv_banked_kernel<kQ4, 4, D, LPR, false>), grid, block, g.shared, stream, a, w, book, ws,
-                               as, out, f.N, f.K, f.stride, rows, (int)f.out_f32 | (f.packed_k == 64 ? 2 : 0), pending_signs);
+                               as, out, f.N, f.K, f.stride, rows, (int)f.out_f32 | (f.packed_k == 64 ? 2 : 0), pending_signs, pending_codes);
             break;
     }
     return hip_check(hipGetLastError(), "launch projection (gemv, replicated tables)");
@@ -1152,11 +1154,12 @@ bool gemv_serves_k_major(const orx_function& f, int rows) {
 // Launchers used by the projection factories.  Argument order is the caller's business:
 // they pass already-unmarshalled pointers.
 int gemv_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t stream, const int8_t* a,
-                const void* w, const uint32_t* book, const __half* ws, const __half* as, void* out, const int8_t* signs) {
+                const void* w, const uint32_t* book, const __half* ws, const __half* as, void* out, const int8_t* signs, int8_t* codes) {
     // LDS opt-in needs a device, so it happens at the first launch rather than at resolve time
     const int ready = gemv_prepare_device();
     if (ready != ORX_OK) return ready;
     pending_signs = f.input_f16 ? signs : nullptr;
+    pending_codes = f.input_f16 ? codes : nullptr;
     if (f.packed_k != 0 && !gemv_serves_k_major(f, rows)) {
         set_error("%s: the gemv algorithm does not serve this K-major shape for %d rows", f.symbol.c_str(), rows);
         return ORX_ERR_BAD_VARIANT;

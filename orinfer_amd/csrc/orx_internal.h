@@ -74,6 +74,7 @@ struct orx_function {
     int tile_hint = 0;  // projections: row tile preferred while the live rows fit one such tile (0 = none)
     bool out_f32 = false;
     bool input_f16 = false;  // single-row projection that quantises its fp16 activations itself
+    bool publish_codes = false; // ... and writes their int8 codes (takes a Q buffer)
     bool rotate_input = false;  // ... after the signed block-128 rotation (takes a Signs buffer)
     const void* device_function = nullptr;  // for hipFuncGetAttributes
     // The handle owns no device memory.  A kernel that needs scratch beyond its inputs and outputs

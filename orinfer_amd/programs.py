@@ -54,6 +54,16 @@ class QuantizedLinear:
             self.projection = Kernel("e8p_q4_projection", **variant)
         else:
             self.projection = Kernel("int8_projection", **variant)
+        # one row of two-stage codes, where the GEMV serves the shape: it quantises the fp16 row itself, one launch instead of two
+        # (9728 x 2560: 8.7 -> 6.4 us)
+        self.single = None
+        if codec == "q4" and algorithm in ("auto", "gemv") and not block_m:
+            try:
+                self.single = Kernel("e8p_q4_projection", M=1, N=self.n, K=self.k, algorithm=algorithm, packed_k=packed_k,
+                                     input_dtype="float16", codes=True)
+            except OrxError as error:
+                if error.code != ORX_ERR_BAD_VARIANT:
+                    raise
         self.workspace = self.projection.workspace()
         self._live = self.out  # the rows of `out` that the last launch wrote (slicing costs 1 us of a 7 us call)
 
@@ -69,6 +79,9 @@ class QuantizedLinear:
         else:
             self.projection(stream=stream, A=self.a_q, Output=self.out, TokenScale=self.a_s, Weight=self.weight,
                             WeightScale=self.scales, Workspace=self.workspace, m=rows)
+        return self._rows(rows)
+
+    def _rows(self, rows):
         live = self._live
         if live.shape[0] != rows:
             live = self._live = self.out[:rows]
@@ -77,6 +90,9 @@ class QuantizedLinear:
     def run(self, x16, stream=None):
         if stream is None:
             stream = current_stream()
+        if self.single is not None and x16.shape[0] == 1 and x16.data_ptr() % 16 == 0:  # (the quantiser takes any fp16 address)
+            self.single(stream=stream, A=x16, AS=self.a_s, Book=self.book, Out=self.out, Q=self.a_q, S=self.scales, W=self.weight)
+            return self._rows(1)
         return self.project(self.quantize(x16, stream), stream)
 
 

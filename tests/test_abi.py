@@ -55,6 +55,8 @@ ABI = {
     ("e8p_q4_projection", (("M", 1), ("N", 9728), ("K", 2560))): ["A", "AS", "Book", "Out", "S", "W"],
     ("e8p_q4_projection", (("M", 1), ("N", 9728), ("K", 2560), ("input_dtype", "float16"), ("rotate", True))):
         ["A", "AS", "Book", "Out", "S", "Signs", "W"],
+    ("e8p_q4_projection", (("M", 1), ("N", 9728), ("K", 2560), ("input_dtype", "float16"), ("codes", True), ("rotate", True))):
+        ["A", "AS", "Book", "Out", "Q", "S", "Signs", "W"],
     ("e8p_q4_projection", (("M", 64), ("N", 256), ("K", 256), ("dynamic_rows", True))):
         ["A", "AS", "Book", "Out", "S", "W", "m"],
     ("int8_projection", (("M", 8192), ("N", 4096), ("K", 4096))):

@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from oracle import reference as orc
-from orinfer_amd import codebook, workloads
+from orinfer_amd import codebook, programs, workloads
 
 from . import gpu_util as gu
 
@@ -402,6 +402,28 @@ def test_q4_gemv_rotates_and_quantises_fp16_input(n, k, packed_k):
         assert float(gu.host(a_scale)[1]) == 7.0 and (gu.host(out)[1] == 9).all()
     with pytest.raises(Exception):
         gu.kernel("e8p_q4_projection", M=1, N=n, K=k, rotate=True)
+
+
+@pytest.mark.parametrize("n,k,packed_k,single", [(200, 1024, 0, True), (136, 2048, 128, True), (48, 8192, 0, True), (40, 8704, 0, False), (64, 1152, 128, False)])
+def test_one_row_program_gives_the_bits_of_two_launches(n, k, packed_k, single):
+    """One launch quantises the row, publishes its codes and projects; shapes and addresses it does not take keep the two launches."""
+    rng = np.random.default_rng(orc.SEED + n + k)
+    packed = rng.integers(0, 2**32, (n, k // 8), dtype=np.uint32)
+    scales = rng.uniform(0.005, 0.02, n).astype(np.float16)
+    linear = programs.QuantizedLinear("q4", packed, scales, 4, packed_k=packed_k)
+    assert (linear.single is not None) == single
+    weights = orc.q4_integers(packed, TABLE)
+    for offset in (0, 1):  # the second row starts at an odd fp16
+        padded = torch.zeros(k + 8, dtype=torch.float16, device=gu.DEV)
+        x = padded[offset : offset + k].view(1, k)
+        x.copy_(torch.from_numpy((rng.normal(size=(1, k)) * 3).astype(np.float16)))
+        linear.a_q.fill_(99)
+        out = gu.host(linear.run(x)).copy()
+        a_q, a_s = orc.a8(gu.host(x))
+        np.testing.assert_array_equal(gu.host(linear.a_q)[:1], a_q)
+        assert (gu.host(linear.a_q)[1:] == 99).all()
+        np.testing.assert_array_equal(gu.host(linear.a_s)[:1], a_s)
+        np.testing.assert_array_equal(out, orc.project(a_q, a_s, weights, scales))
 
 
 def test_q4_fp16_input_is_refused_where_no_kernel_serves_it():
