@@ -34,7 +34,6 @@ typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 // Tables: entry i of the basis table ((h ^ 8) per coordinate) at byte i*256 + copy*8, entry u of the
 // sign/parity mask table at u*256 + 128 + copy*8, 16 copies each.  With the entry index in the
 // address's second byte, one v_perm_b32 builds a lookup address from a byte of the code.
-constexpr uint32_t kMaskOffset = 128;
 constexpr uint32_t kSumBase = 65536;      // two sets of kMaxHeld buffers of 16 channels x 33 ints
 constexpr int kSumStride = 33;
 constexpr int kSumBuffer = 16 * kSumStride;
@@ -125,18 +124,14 @@ __global__ __launch_bounds__(W * 64) void dense_resident_kernel(DenseParams p) {
 #pragma unroll
     for (int slot = 1; slot < P; ++slot) load_codes(ring[slot], min(slot, blocks - 1));
 
-    // byte 0: this lane's copy in the basis half of an entry, byte 1: in the mask half
-    const uint32_t copy = (uint32_t)(lane & 15) * 8;
-    const uint32_t columns = copy | (kMaskOffset | copy) << 8;
-    // selectors of v_perm_b32(code, columns): address byte 0 = a byte of `columns`, byte 1 = a byte of the code
-    constexpr uint32_t kBasisLow = 0x0C0C0500u, kMaskLow = 0x0C0C0401u, kBasisHigh = 0x0C0C0700u, kMaskHigh = 0x0C0C0601u;
+    const lds_asm::WidePairedLookup tables(lane);
     auto lookup = [&](uint32_t code, uint32_t selector) {
-        return *reinterpret_cast<const uint2*>(lds + __builtin_amdgcn_perm(code, columns, selector));
+        return *reinterpret_cast<const uint2*>(lds + tables.address(code, selector));
     };
     // one u32 two-stage code -> 8 int8 weights: w + 128 = 8 (v0 + 8) + 2 (v1 + 8) + 53 in every byte
     auto decode = [&](uint32_t code) {
-        const uint2 b0 = lookup(code, kBasisLow), m0 = lookup(code, kMaskLow);
-        const uint2 b1 = lookup(code, kBasisHigh), m1 = lookup(code, kMaskHigh);
+        const uint2 b0 = lookup(code, tables.first_low), m0 = lookup(code, tables.second_low);
+        const uint2 b1 = lookup(code, tables.first_high), m1 = lookup(code, tables.second_high);
         uint2 w;
         w.x = ((((b0.x ^ m0.x) << 3) + ((b1.x ^ m1.x) << 1)) + 0x35353535u) ^ 0x80808080u;
         w.y = ((((b0.y ^ m0.y) << 3) + ((b1.y ^ m1.y) << 1)) + 0x35353535u) ^ 0x80808080u;
@@ -325,14 +320,12 @@ __global__ __launch_bounds__(kSpecThreads) void dense_specialized_kernel(DensePa
     for (int i = tid; i < 2 * kSumBuffer; i += kDecoders * 64) sums[i] = 0;
     __syncthreads();
 
-    const uint32_t copy = (uint32_t)(lane & 15) * 8;
-    const uint32_t columns = copy | (kMaskOffset | copy) << 8;
-    constexpr uint32_t kBasisLow = 0x0C0C0500u, kMaskLow = 0x0C0C0401u, kBasisHigh = 0x0C0C0700u, kMaskHigh = 0x0C0C0601u;
+    const lds_asm::WidePairedLookup tables(lane);
     // The tables start at LDS address 0 (the kernel has no static LDS), so the permuted bytes are the
     // address itself.
     typedef const __attribute__((address_space(3))) v2u* TableEntry;
     auto lookup = [&](uint32_t code, uint32_t selector_bytes) {
-        return *reinterpret_cast<TableEntry>((uintptr_t)__builtin_amdgcn_perm(code, columns, selector_bytes));
+        return *reinterpret_cast<TableEntry>((uintptr_t)tables.address(code, selector_bytes));
     };
     // All lookups of a group of codes are requested before the first is used: with two decoder waves
     // per SIMD there is little else to hide the LDS latency behind.
@@ -340,7 +333,7 @@ __global__ __launch_bounds__(kSpecThreads) void dense_specialized_kernel(DensePa
         v2u b0, m0, b1, m1;
     };
     auto request = [&](uint32_t code) {
-        return Looked{lookup(code, kBasisLow), lookup(code, kMaskLow), lookup(code, kBasisHigh), lookup(code, kMaskHigh)};
+        return Looked{lookup(code, tables.first_low), lookup(code, tables.second_low), lookup(code, tables.first_high), lookup(code, tables.second_high)};
     };
     // one u32 two-stage code -> 8 int8 weights: w + 128 = 8 (v0 + 8) + 2 (v1 + 8) + 53 in every byte
     auto combine = [&](const Looked& l) {

@@ -50,7 +50,6 @@ constexpr int kStep = 128;      // K per step
 constexpr int kChannels = 96;   // channels per pass: three MFMA blocks
 constexpr int kMfmaWaves = 4, kDecoderWaves = 8;
 constexpr int kThreads = (kMfmaWaves + kDecoderWaves) * 64;
-constexpr uint32_t kMaskOffset = 128;            // tables: entry i at i*256 (basis) and i*256 + 128 (mask), 16 copies of 8 bytes
 constexpr uint32_t kTableBytes = 65536;
 constexpr int kWeightStages = 2;
 constexpr uint32_t kWeightStage = kChannels * kStep;  // 12 KiB
@@ -100,15 +99,13 @@ __global__ __launch_bounds__(kThreads) void wide_kernel(WideParams p) {
     }
 
     // decode of one u32 two-stage code to 8 int8 weights: w + 128 = 8 (v0 + 8) + 2 (v1 + 8) + 53 in every byte
-    const uint32_t copy = (uint32_t)(lane & 15) * 8;
-    const uint32_t columns = copy | (kMaskOffset | copy) << 8;
-    constexpr uint32_t kBasisLow = 0x0C0C0500u, kMaskLow = 0x0C0C0401u, kBasisHigh = 0x0C0C0700u, kMaskHigh = 0x0C0C0601u;
+    const lds_asm::WidePairedLookup tables(lane);
     auto lookup = [&](uint32_t code, uint32_t selector) {
-        return *reinterpret_cast<const uint2*>(lds + __builtin_amdgcn_perm(code, columns, selector));
+        return *reinterpret_cast<const uint2*>(lds + tables.address(code, selector));
     };
     auto decode = [&](uint32_t code) {
-        const uint2 b0 = lookup(code, kBasisLow), m0 = lookup(code, kMaskLow);
-        const uint2 b1 = lookup(code, kBasisHigh), m1 = lookup(code, kMaskHigh);
+        const uint2 b0 = lookup(code, tables.first_low), m0 = lookup(code, tables.second_low);
+        const uint2 b1 = lookup(code, tables.first_high), m1 = lookup(code, tables.second_high);
         uint2 w;
         w.x = ((((b0.x ^ m0.x) << 3) + ((b1.x ^ m1.x) << 1)) + 0x35353535u) ^ 0x80808080u;
         w.y = ((((b0.y ^ m0.y) << 3) + ((b1.y ^ m1.y) << 1)) + 0x35353535u) ^ 0x80808080u;

@@ -66,6 +66,20 @@ struct PairedLookup {
     }
 };
 constexpr uint32_t kPairedTableBytes = 256 * 128;
+// The same in entries of 256 bytes, 16 copies of either table: of 32 neighbouring lanes 16 read one table and 16 the other.
+// Byte 0 of an address is the lane's column, byte 1 a byte of the code: one v_perm_b32 of (code, columns) and a selector.
+struct WidePairedLookup {
+    uint32_t columns, first_low, second_low, first_high, second_high;
+    __device__ __forceinline__ explicit WidePairedLookup(int lane) {
+        const uint32_t copy = (uint32_t)(lane & 15) * 8, other = (uint32_t)(lane >> 4) & 1;
+        columns = (copy | other * 128) | (copy | (other ^ 1) * 128) << 8;
+        first_low = 0x0C0C0500u - (other << 8), second_low = 0x0C0C0401u + (other << 8);
+        first_high = first_low + 0x200u, second_high = second_low + 0x200u;
+    }
+    __device__ __forceinline__ uint32_t address(uint32_t code, uint32_t selector) const {
+        return __builtin_amdgcn_perm(code, columns, selector);
+    }
+};
 // One half of a paired entry: SLOTS 16-byte slots of two copies each.  Every lane of a wave writes its own entry, so the slot
 // order turns with the entry: in the same order for all, the lanes, whole entries apart, would write to the same banks (the
 // 16-wave kernels spent 2 us of every launch on 64 KB of tables that way, 0.3 us now).
