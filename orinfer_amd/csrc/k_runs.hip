@@ -28,6 +28,9 @@ namespace {
 
 using namespace lds_asm;
 
+// a step is one stretch of code: a lambda left as a call would keep the fragments in scratch memory
+#define ORX_INLINE __attribute__((always_inline))
+
 enum RunsCodec { kRunsQ4 = 0, kRunsW8 = 2 };
 
 struct RunsParams {
@@ -48,7 +51,7 @@ template <int CODEC, int TB, int CB>
 constexpr uint32_t runs_stage() { return 2048u * (TB + (CODEC == kRunsW8 ? CB : 0)); }
 template <int CODEC, int TB, int CB, int WAVES, int D>
 constexpr uint32_t runs_lds() {
-    const uint32_t rings = runs_stage<CODEC, TB, CB>() * WAVES * D, sums = CB * 16 * (TB * 16 + 4) * 4;  // the sums follow the rings
+    const uint32_t rings = runs_stage<CODEC, TB, CB>() * WAVES * D, sums = (CB * 16 * (TB * 16 + 4) + 128 + CB * 16) * 4;  // sums and scales follow the rings
     return runs_tables<CODEC>() + (rings > sums ? rings : sums);
 }
 
@@ -77,6 +80,9 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
     const int chunks = p.k / 128;
     const int begin = chunks * wave / WAVES, count = chunks * (wave + 1) / WAVES - begin, last = max(begin + count - 1, begin);
 
+    // token scales of the tile (threads 0-127) and scales of the run's channels: read here, used behind the K loop
+    uint32_t scale_bits = reinterpret_cast<const unsigned short*>(tid < 128 ? p.as + first_row : p.ws + first_channel)
+        [tid < 128 ? min(tid, rows - 1) : min(tid - 128, channels - 1)];
     uint32_t selector = 0;
     if constexpr (CODEC == kRunsQ4)
         if (tid < 256) selector = p.book[tid];
@@ -99,7 +105,7 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
     uint8_t* const ring = lds + runs_tables<CODEC>() + (uint32_t)wave * (D * kStage);
     const int8_t* const a_base = uniform_pointer(p.a + (int64_t)first_row * p.k);
     const uint8_t* const w_base = uniform_pointer(p.w + (int64_t)first_channel * p.row_stride);
-    auto request_rows = [&](const void* base, const Rows& r, auto blocks_tag, uint8_t* to) {
+    auto request_rows = [&](const void* base, const Rows& r, auto blocks_tag, uint8_t* to) ORX_INLINE {
         constexpr int BLOCKS = decltype(blocks_tag)::value;
 #pragma unroll
         for (int i = 0; i < 2 * BLOCKS; ++i) {
@@ -115,7 +121,7 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
     for (int j = 0; j < CB; ++j)
         code_offset[j] = (uint32_t)min(16 * j + column, channels - 1) * p.row_stride + (uint32_t)(quarter >> 1) * p.half_stride + (uint32_t)(quarter & 1) * 16;
     v4u codes[CODEC == kRunsQ4 ? D : 1][CB];
-    auto request = [&](int index, auto slot_tag) {  // chunk begin + index of this wave's slice
+    auto request = [&](int index, auto slot_tag) ORX_INLINE {  // chunk begin + index of this wave's slice
         constexpr int SLOT = decltype(slot_tag)::value;
         const int chunk = min(begin + index, last);
         const uint8_t* const weights = w_base + (uint64_t)chunk * p.chunk_stride;
@@ -128,7 +134,7 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
         }
         request_rows(a_base + (uint64_t)chunk * 128, token_rows, std::integral_constant<int, TB>{}, ring + SLOT * kStage);
     };
-    auto name_codes = [&]() {
+    auto name_codes = [&]() ORX_INLINE {
         if constexpr (CODEC == kRunsQ4) {
 #pragma unroll
             for (int d = 0; d < D; ++d)
@@ -137,7 +143,7 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
         }
     };
     // waits until at most `CHUNKS` of the youngest chunks requested are still on their way
-    auto wait_requests = [&](auto chunks_tag) {
+    auto wait_requests = [&](auto chunks_tag) ORX_INLINE {
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(chunks_tag)::value * kRequests) : "memory");
         name_codes();
     };
@@ -161,41 +167,42 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
         for (int j = 0; j < CB; ++j) acc[i][j] = v4i{0, 0, 0, 0};
     const uint32_t lds_base = lds_address_of(lds);
     const uint32_t frag = lds_address_of(ring) + (uint32_t)column * 128 + (uint32_t)((quarter ^ swizzle(column)) * 16);
-    auto read_fragment = [&](v4i& to, auto block_tag, uint32_t address) { lds_read_16<decltype(block_tag)::value * 2048>(to, address); };
+    auto read_fragment = [&](v4i& to, auto block_tag, uint32_t address) ORX_INLINE { lds_read_16<decltype(block_tag)::value * 2048>(to, address); };
 
     if constexpr (CODEC == kRunsQ4) {
         const PairedLookup tables(lds_base, lane);
-        v4i token[TB], weight[CB];
-        v2u looked[2][2][2];  // of two codes: stages, basis and mask entries
-        auto lookup = [&](const v4u& words, auto step_tag) {
-            constexpr int STEP = decltype(step_tag)::value;
-            tables.read<0>(looked[0][0], words[2 * STEP]);
-            tables.read<1>(looked[0][1], words[2 * STEP]);
-            tables.read<0>(looked[1][0], words[2 * STEP + 1]);
-            tables.read<1>(looked[1][1], words[2 * STEP + 1]);
+        // Two sets each: the fragments of a step and of the next, the lookups of a block and of the block before it.
+        constexpr int SETS = CB > 1 ? 2 : 1;
+        v4i token[SETS][TB], weight[CB];
+        v2u looked[SETS][2][2][2];  // of two codes: stages, basis and mask entries
+        auto lookup = [&](auto set_tag, const v4u& words, auto step_tag) ORX_INLINE {
+            constexpr int SET = decltype(set_tag)::value % SETS, STEP = decltype(step_tag)::value;
+            tables.read<0>(looked[SET][0][0], words[2 * STEP]);
+            tables.read<1>(looked[SET][0][1], words[2 * STEP]);
+            tables.read<0>(looked[SET][1][0], words[2 * STEP + 1]);
+            tables.read<1>(looked[SET][1][1], words[2 * STEP + 1]);
         };
-        auto combine = [&]() {  // w + 128 = 8 (v0 + 8) + 2 (v1 + 8) + 53 in every byte
-            v4i w;
-#pragma unroll
-            for (int c = 0; c < 2; ++c)
-#pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                    const uint32_t coarse = looked[c][0][0][e] ^ looked[c][0][1][e], fine = looked[c][1][0][e] ^ looked[c][1][1][e];
-                    w[2 * c + e] = (int)(((((coarse << 2) + fine) << 1) + 0x35353535u) ^ 0x80808080u);
-                }
-            return w;
+        auto combine = [&](auto set_tag, v4i& w, int word) ORX_INLINE {  // w + 128 = 8 (v0 + 8) + 2 (v1 + 8) + 53 in every byte
+            constexpr int SET = decltype(set_tag)::value % SETS;
+            const int c = word >> 1, e = word & 1;
+            const uint32_t coarse = looked[SET][c][0][0][e] ^ looked[SET][c][0][1][e], fine = looked[SET][c][1][0][e] ^ looked[SET][c][1][1][e];
+            w[word] = (int)(((((coarse << 2) + fine) << 1) + 0x35353535u) ^ 0x80808080u);
         };
-        auto wait_reads = [&]() {
-            asm volatile("s_waitcnt lgkmcnt(0)"
-                         : "+v"(looked[0][0][0]), "+v"(looked[0][0][1]), "+v"(looked[0][1][0]), "+v"(looked[0][1][1]),
-                           "+v"(looked[1][0][0]), "+v"(looked[1][0][1]), "+v"(looked[1][1][0]), "+v"(looked[1][1][1])
-                         :
-                         : "memory");
+        auto wait_reads = [&]() ORX_INLINE {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-            for (int i = 0; i < TB; ++i) asm volatile("" : "+v"(token[i]));
+            for (int set = 0; set < SETS; ++set) {
+#pragma unroll
+                for (int c = 0; c < 2; ++c)
+                    asm volatile("" : "+v"(looked[set][c][0][0]), "+v"(looked[set][c][0][1]), "+v"(looked[set][c][1][0]), "+v"(looked[set][c][1][1]));
+#pragma unroll
+                for (int i = 0; i < TB; ++i) asm volatile("" : "+v"(token[set][i]));
+            }
         };
-        auto read_token = [&](auto i_tag, uint32_t address) { read_fragment(token[decltype(i_tag)::value], i_tag, address); };
-        auto for_tokens = [&](auto body) {
+        auto read_token = [&](auto set_tag, auto i_tag, uint32_t address) ORX_INLINE {
+            read_fragment(token[decltype(set_tag)::value % SETS][decltype(i_tag)::value], i_tag, address);
+        };
+        auto for_tokens = [&](auto body) ORX_INLINE {
             body(std::integral_constant<int, 0>{});
             if constexpr (TB > 1) body(std::integral_constant<int, 1>{});
             if constexpr (TB > 2) body(std::integral_constant<int, 2>{});
@@ -205,42 +212,68 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
             if constexpr (TB > 6) body(std::integral_constant<int, 6>{});
             if constexpr (TB > 7) body(std::integral_constant<int, 7>{});
         };
-        // The multiplies of a step of 64, a block of channels at a time; under them the lookups of that block's next
-        // weights, and under the last block's the next fragments, each asked for when its last multiply is out.
-        auto step = [&](uint32_t next_fragments, const v4u(&next_codes)[CB], auto next_step_tag) {
-#pragma unroll
-            for (int j = 0; j < CB; ++j) {
-                for_tokens([&](auto i_tag) {
+        auto for_blocks = [&](auto body) ORX_INLINE {
+            body(std::integral_constant<int, 0>{});
+            if constexpr (CB > 1) body(std::integral_constant<int, 1>{});
+            if constexpr (CB > 2) body(std::integral_constant<int, 2>{});
+            if constexpr (CB > 3) body(std::integral_constant<int, 3>{});
+            if constexpr (CB > 4) body(std::integral_constant<int, 4>{});
+        };
+        // The multiplies of a step of 64 (HALF: which of the chunk), a block of channels at a time.  Under a block's multiplies:
+        // the lookups of its next weights go out, the lookups of the block before it (a whole block old, so that nothing
+        // waits for them) are combined, and all blocks but the last ask for their share of the next fragments (so those
+        // have returned when the step ends).  With one wave to a SIMD nothing else would fill these waits.
+        auto step = [&](auto half_tag, uint32_t next_fragments, const v4u(&next_codes)[CB], auto next_step_tag) ORX_INLINE {
+            constexpr int HALF = decltype(half_tag)::value;
+            for_blocks([&](auto j_tag) ORX_INLINE {
+                constexpr int j = decltype(j_tag)::value, before = (j + CB - 1) % CB;
+                std::integral_constant<int, HALF * CB + j> lookups;            // set parity of this block's lookups
+                std::integral_constant<int, HALF * CB + j + 2 * CB - 1> held;  // and of the block's before it
+                std::integral_constant<int, HALF + 1> next;
+                if constexpr (CB > 1) wait_reads();
+                for_tokens([&](auto i_tag) ORX_INLINE {
                     constexpr int i = decltype(i_tag)::value;
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(weight[j], token[i], acc[i][j], 0, 0, 0);
+                    acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(weight[j], token[HALF % SETS][i], acc[i][j], 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
-                    if (i == 0) lookup(next_codes[j], next_step_tag);
-                    if (j == CB - 1) read_token(i_tag, next_fragments);
+                    if constexpr (i == 0) lookup(lookups, next_codes[j], next_step_tag);
+                    if constexpr (CB == 1 || (j < CB - 1 && i % (CB - 1) == j)) read_token(next, i_tag, next_fragments);
+                    if constexpr (CB > 1) {
+#pragma unroll
+                        for (int word = 0; word < 4; ++word)
+                            if (word * TB / 4 == i) combine(held, weight[before], word);
+                    }
                     __builtin_amdgcn_sched_barrier(0);
                 });
-                wait_reads();
-                weight[j] = combine();
+                if constexpr (CB == 1) {
+                    wait_reads();
+#pragma unroll
+                    for (int word = 0; word < 4; ++word) combine(lookups, weight[0], word);
+                }
                 __builtin_amdgcn_sched_barrier(0);
-            }
+            });
         };
         std::integral_constant<int, 0> zero;
         std::integral_constant<int, 1> one;
         if (count > 0) {
             wait_requests(std::integral_constant<int, D - 1>{});
-            for_tokens([&](auto i_tag) { read_token(i_tag, frag); });
+            for_tokens([&](auto i_tag) ORX_INLINE { read_token(zero, i_tag, frag); });
+            for_blocks([&](auto j_tag) ORX_INLINE {  // (the last block's lookups are combined under the first multiplies)
+                constexpr int j = decltype(j_tag)::value;
+                std::integral_constant<int, CB + j> set;
+                lookup(set, codes[0][j], zero);
+                if constexpr (j < CB - 1 || CB == 1) {
+                    wait_reads();
 #pragma unroll
-            for (int j = 0; j < CB; ++j) {
-                lookup(codes[0][j], zero);
-                wait_reads();
-                weight[j] = combine();
-            }
-            auto chunk_step = [&](int t, auto slot_tag) {
+                    for (int word = 0; word < 4; ++word) combine(set, weight[j], word);
+                }
+            });
+            auto chunk_step = [&](int t, auto slot_tag) ORX_INLINE {
                 constexpr int SLOT = decltype(slot_tag)::value, NEXT = (SLOT + 1) % D;
-                step((frag + SLOT * kStage) ^ 64u, codes[SLOT], one);
+                step(zero, (frag + SLOT * kStage) ^ 64u, codes[SLOT], one);
                 wait_requests(std::integral_constant<int, D - 2>{});  // chunk t + 1 is here, and nobody reads chunk t any more
                 request(t + D, slot_tag);
                 __builtin_amdgcn_sched_barrier(0);
-                step(frag + NEXT * kStage, codes[NEXT], zero);
+                step(one, frag + NEXT * kStage, codes[NEXT], zero);
             };
             int t = 0;
             for (; t + D <= count; t += D) {
@@ -254,6 +287,7 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
                 if (t + 1 < count) chunk_step(t + 1, std::integral_constant<int, 1>{});
             if constexpr (D > 3)
                 if (t + 2 < count) chunk_step(t + 2, std::integral_constant<int, 2>{});
+            wait_reads();
         }
     } else {
         v4i token[2][TB], weight[2][CB];
@@ -306,6 +340,10 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
     // ---- the slices are added where the rings were: wave 0 stores, the others add ----
     // accumulator register r of a lane: channel 4 quarter + r of the block, token `column`
     int* const sums = reinterpret_cast<int*>(lds + runs_tables<CODEC>());
+    float* const token_scales = reinterpret_cast<float*>(sums + CB * 16 * kPitch);
+    float* const channel_scales = token_scales + 128;
+    asm volatile("" : "+v"(scale_bits));  // converted here, not where it was read
+    if (tid < 128 + CB * 16) token_scales[tid] = __half2float(__ushort_as_half((unsigned short)scale_bits));
     int own = threadIdx.x & 63;
     asm volatile("" : "+v"(own));
     int* const mine = sums + 4 * (own >> 4) * kPitch + (own & 15);
@@ -327,16 +365,38 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
                 for (int r = 0; r < 4; ++r) atomicAdd(mine + (16 * j + r) * kPitch + 16 * i, acc[i][j][r]);
     }
     __syncthreads();
-    for (int e = tid; e < rows * CB * 16; e += kThreads) {
-        const int local = e / (CB * 16), channel = e % (CB * 16);
+    // four channels of a row per thread and store
+    const int element = p.out_f32 ? 4 : 2;
+#pragma unroll 2
+    for (int e = tid; e < rows * CB * 4; e += kThreads) {
+        const int local = e / (CB * 4), channel = e % (CB * 4) * 4;
         if (channel >= channels) continue;
-        const int64_t row = first_row + local;
-        const int col = first_channel + channel;
-        const float value = rescale(sums[channel * kPitch + local], __half2float(p.ws[col]), __half2float(p.as[row]));
-        if (p.out_f32)
-            reinterpret_cast<float*>(p.out)[row * p.stride + col] = value;
-        else
-            reinterpret_cast<__half*>(p.out)[row * p.stride + col] = __float2half_rn(value);
+        const float token_scale = token_scales[local];
+        const float4 ws = *reinterpret_cast<const float4*>(channel_scales + channel);
+        const int* cell = sums + channel * kPitch + local;
+        const float value[4] = {rescale(cell[0], ws.x, token_scale), rescale(cell[kPitch], ws.y, token_scale),
+                                rescale(cell[2 * kPitch], ws.z, token_scale), rescale(cell[3 * kPitch], ws.w, token_scale)};
+        char* const dst = static_cast<char*>(p.out) + ((int64_t)(first_row + local) * p.stride + first_channel + channel) * element;
+        const bool whole = channel + 3 < channels && (reinterpret_cast<uintptr_t>(dst) & (uintptr_t)(4 * element - 1)) == 0;
+        if (p.out_f32) {
+            if (whole) {
+                *reinterpret_cast<float4*>(dst) = make_float4(value[0], value[1], value[2], value[3]);
+            } else {
+                for (int i = 0; i < 4; ++i)
+                    if (channel + i < channels) reinterpret_cast<float*>(dst)[i] = value[i];
+            }
+        } else {
+            __half h[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) h[i] = __float2half_rn(value[i]);
+            if (whole) {
+                *reinterpret_cast<uint2*>(dst) = make_uint2((uint32_t)__half_as_ushort(h[0]) | (uint32_t)__half_as_ushort(h[1]) << 16,
+                                                            (uint32_t)__half_as_ushort(h[2]) | (uint32_t)__half_as_ushort(h[3]) << 16);
+            } else {
+                for (int i = 0; i < 4; ++i)
+                    if (channel + i < channels) reinterpret_cast<__half*>(dst)[i] = h[i];
+            }
+        }
     }
 }
 
