@@ -890,18 +890,40 @@ __global__ __launch_bounds__(kRouteThreads) void route_gemv_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int route = blockIdx.y;
     const int routes = (int)gridDim.y;
+    // What does not wait for the routes is requested first: the logits or the route's expert, the table entry and the row of `a`
+    // (fp16: the pieces of 8 values that this thread quantises; K <= 16384 is up to four).
+    const bool swiglu_rows = x16 == 2;
+    constexpr int kSelected = LOCAL == 0 ? 1 : LOCAL;
+    float route_logits[kSelected];
+    if (LOCAL > 0 && wave == 0) load_route_logits<kSelected>(route_logits, logits, experts, lane);
     int expert = LOCAL > 0 ? 0 : ids[route];
+    const uint2 entry = reinterpret_cast<const uint2*>(book)[tid & 255];
+    const __half* x = reinterpret_cast<const __half*>(a) + (swiglu_rows ? (int64_t)route * 2 * k : 0);
+    uint4 kept[4], up_kept[4];
+    if (x16) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int i = tid + j * kRouteThreads;
+            kept[j] = up_kept[j] = make_uint4(0u, 0u, 0u, 0u);
+            if (i < k / 8) {
+                kept[j] = reinterpret_cast<const uint4*>(x)[i];
+                if (swiglu_rows) up_kept[j] = reinterpret_cast<const uint4*>(x + k)[i];
+            }
+        }
+    }
     if (LOCAL == 0 && (unsigned)expert >= (unsigned)experts) return;  // nothing to index: the row stays as it was
     const int row = shared_input ? 0 : route;
     const int blocks = k / 128;
     const int channel = blockIdx.x * kRouteChannels + (lane >> 1);
     const int half = lane & 1;
     const bool live = channel < n;
-    // codes of this lane: 16 bytes per K block, K blocks wave, wave + 8, ...; the first kRouteDepth
-    // loads leave before anything else (once the expert is known)
+    // codes of this lane: 16 bytes per K block, K blocks wave, wave + 8, ...; the first kRouteDepth loads leave as soon as the
+    // expert is known, and with them the scale of the channel that this thread stores at the end
     const int64_t block_stride = (int64_t)n * 2;  // uint4 per K block
     const uint4* codes = nullptr;
     uint4 held[kRouteDepth];
+    unsigned short scale_bits = 0;
+    const int out_channel = blockIdx.x * kRouteChannels + (tid & (kRouteChannels - 1));
     auto request_codes = [&]() {
         codes = reinterpret_cast<const uint4*>(p + (((int64_t)expert * blocks) * n + (live ? channel : 0)) * 16) + half;
 #pragma unroll
@@ -909,11 +931,13 @@ __global__ __launch_bounds__(kRouteThreads) void route_gemv_kernel(
             const int kb = wave + d * kRouteWaves;
             held[d] = kb < blocks ? codes[kb * block_stride] : make_uint4(0u, 0u, 0u, 0u);
         }
+        scale_bits = reinterpret_cast<const unsigned short*>(ws)[(int64_t)expert * n + min(out_channel, n - 1)];
     };
     if (LOCAL == 0) request_codes();
-    if (LOCAL > 0 && wave == 0) select_routes<LOCAL == 0 ? 1 : LOCAL>(logits, selected_ids, selected_prob, 0, experts, routes, renormalize, lane);
+    if (LOCAL > 0 && wave == 0)  // (one workgroup writes the probabilities)
+        select_routes<kSelected>(route_logits, selected_ids, blockIdx.x == 0 && blockIdx.y == 0 ? selected_prob : nullptr, experts,
+                                 routes, renormalize, lane);
     if (tid < 256) {
-        const uint2 entry = reinterpret_cast<const uint2*>(book)[tid];
         table[tid] = make_uint4(entry.x, entry.y, negate_bytes(entry.x), negate_bytes(entry.y));
     } else {
         const uint32_t u = tid - 256;
@@ -935,22 +959,14 @@ __global__ __launch_bounds__(kRouteThreads) void route_gemv_kernel(
         // `a` is an fp16 row (the shared token row, or with x16 == 2 this route's gate|up row, which
         // first becomes fp16(silu(gate) * up)): every workgroup quantises it by the A8 rule (row maximum
         // over 127, fp16 scale, round to nearest even) on its way into LDS; the first one also writes
-        // the scale.  Up to 4 pieces of 8 values per thread (K <= 16384) stay in registers between the
-        // two passes.
-        const bool swiglu_rows = x16 == 2;
-        const __half* x = reinterpret_cast<const __half*>(a) + (swiglu_rows ? (int64_t)route * 2 * k : 0);
-        uint4 kept[4];
+        // the scale.
         float amax = 0.f;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int i = tid + j * kRouteThreads;
-            kept[j] = make_uint4(0u, 0u, 0u, 0u);
-            if (i < k / 8) {
-                kept[j] = reinterpret_cast<const uint4*>(x)[i];
-                if (swiglu_rows) {
-                    const uint4 up_bits = reinterpret_cast<const uint4*>(x + k)[i];
-                    __half* gate = reinterpret_cast<__half*>(&kept[j]);
-                    const __half* up = reinterpret_cast<const __half*>(&up_bits);
+            if (swiglu_rows) {  // (pieces past the row are zeros and stay zeros)
+                __half* gate = reinterpret_cast<__half*>(&kept[j]);
+                const __half* up = reinterpret_cast<const __half*>(&up_kept[j]);
+                if (tid + j * kRouteThreads < k / 8) {
 #pragma unroll
                     for (int e = 0; e < 8; ++e) gate[e] = __float2half_rn(swiglu_value(gate[e], up[e]));
                 }
@@ -1034,16 +1050,13 @@ __global__ __launch_bounds__(kRouteThreads) void route_gemv_kernel(
     acc += __shfl_xor(acc, 1, 64);
     if (half == 0) partial[wave * kRouteChannels + (lane >> 1)] = acc;
     __syncthreads();
-    if (tid < kRouteChannels) {
-        const int out_channel = blockIdx.x * kRouteChannels + tid;
-        if (out_channel < n) {
-            int total = 0;
+    if (tid < kRouteChannels && out_channel < n) {
+        int total = 0;
 #pragma unroll
-            for (int w = 0; w < kRouteWaves; ++w) total += partial[w * kRouteChannels + tid];
-            const float token_scale = x16 ? row_scale : __half2float(as[row]);
-            const float scaled = ((float)total * __half2float(ws[(int64_t)expert * n + out_channel])) * token_scale;
-            c[(int64_t)route * n + out_channel] = __float2half_rn(scaled);
-        }
+        for (int w = 0; w < kRouteWaves; ++w) total += partial[w * kRouteChannels + tid];
+        const float token_scale = x16 ? row_scale : __half2float(as[row]);
+        const float scaled = ((float)total * __half2float(__ushort_as_half(scale_bits))) * token_scale;
+        c[(int64_t)route * n + out_channel] = __float2half_rn(scaled);
     }
 }
 

@@ -27,30 +27,34 @@ __device__ __forceinline__ void wave_quantise_row(const __half* __restrict__ x, 
     uint4 held[kHeldPieces];
 #pragma unroll
     for (int i = 0; i < kHeldPieces; ++i) held[i] = row_pieces[min(lane + 64 * i, pieces - 1)];
-    auto piece_at = [&](int i) { return i < kHeldPieces ? held[i] : row_pieces[lane + 64 * i]; };
+    // (the held pieces are counted at compile time: an array indexed by a loop's counter lives in scratch memory)
     float amax = 0.f;
-    for (int i = 0; lane + 64 * i < pieces; ++i) {
-        const uint4 raw = piece_at(i);
+    auto raise = [&](const uint4& raw) {
         const __half2* pairs = reinterpret_cast<const __half2*>(&raw);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const float2 f = __half22float2(pairs[j]);
             amax = fmaxf(amax, fmaxf(fabsf(f.x), fabsf(f.y)));
         }
-    }
+    };
+#pragma unroll
+    for (int i = 0; i < kHeldPieces; ++i) raise(held[i]);  // (repeats of the last piece among them)
+    for (int at = lane + 64 * kHeldPieces; at < pieces; at += 64) raise(row_pieces[at]);
 #pragma unroll
     for (int offset = 32; offset > 0; offset >>= 1) amax = fmaxf(amax, __shfl_xor(amax, offset, 64));
     const __half stored = a8_scale(amax);
     if (lane == 0) s[row] = stored;
     const float scale = __half2float(stored), inverse = __frcp_rn(scale);
-    for (int i = 0; lane + 64 * i < pieces; ++i) {
-        const uint4 raw = piece_at(i);
+    auto quantise = [&](const uint4& raw, int at) {
         const __half* v = reinterpret_cast<const __half*>(&raw);
         const float low[4] = {__half2float(v[0]), __half2float(v[1]), __half2float(v[2]), __half2float(v[3])};
         const float high[4] = {__half2float(v[4]), __half2float(v[5]), __half2float(v[6]), __half2float(v[7])};
-        reinterpret_cast<uint2*>(q + (int64_t)row * h)[lane + 64 * i] =
-            make_uint2(quantise4(low, scale, inverse), quantise4(high, scale, inverse));
-    }
+        reinterpret_cast<uint2*>(q + (int64_t)row * h)[at] = make_uint2(quantise4(low, scale, inverse), quantise4(high, scale, inverse));
+    };
+#pragma unroll
+    for (int i = 0; i < kHeldPieces; ++i)
+        if (lane + 64 * i < pieces) quantise(held[i], lane + 64 * i);
+    for (int at = lane + 64 * kHeldPieces; at < pieces; at += 64) quantise(row_pieces[at], at);
 }
 
 // QUANT (quantize_hidden): four more waves per workgroup quantise the same four tokens' hidden rows
@@ -73,7 +77,9 @@ __global__ __launch_bounds__((router_threads<LOCAL, QUANT>())) void router_topk_
         wave_quantise_row(x, q, s, row, h, lane);
         return;
     }
-    select_routes<LOCAL>(logits, ids, prob, row, e, top_k, renormalize, lane);
+    float values[LOCAL];
+    load_route_logits<LOCAL>(values, logits + (int64_t)row * e, e, lane);
+    select_routes<LOCAL>(values, ids + (int64_t)row * top_k, prob + (int64_t)row * top_k, e, top_k, renormalize, lane);
     if (QUANT && !kQuantiserWaves) wave_quantise_row(x, q, s, row, h, lane);
 }
 

@@ -367,7 +367,6 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
     __syncthreads();
     // four channels of a row per thread and store
     const int element = p.out_f32 ? 4 : 2;
-#pragma unroll 2
     for (int e = tid; e < rows * CB * 4; e += kThreads) {
         const int local = e / (CB * 4), channel = e % (CB * 4) * 4;
         if (channel >= channels) continue;

@@ -19,30 +19,22 @@ __device__ __forceinline__ float key_value(uint32_t ordered) {
     return __uint_as_float((ordered & 0x80000000u) ? ordered ^ 0x80000000u : ~ordered);
 }
 
-// Maximum of a 64-bit key over the wave with data-parallel-primitive moves only (no LDS round
-// trips: the selection loop below is a chain of top_k dependent reductions).  Quad swaps, half-row
-// and row mirrors give every lane its row's maximum; two broadcasts carry it across rows into
-// lane 63, which is then read back as a scalar.
+// Maximum of a 32-bit key over the wave with data-parallel-primitive moves only (no LDS round trips: the selection loop below
+// is a chain of top_k dependent reductions).  Quad swaps, half-row and row mirrors give every lane its row's maximum; two
+// broadcasts carry it across rows into lane 63, which is then read back as a scalar.
 template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ void dpp_max_step(uint32_t& hi, uint32_t& lo) {
+__device__ __forceinline__ uint32_t dpp_max_step(uint32_t v) {
     // lanes outside ROW_MASK receive their own value back
-    const uint32_t other_hi = (uint32_t)__builtin_amdgcn_update_dpp((int)hi, (int)hi, CTRL, ROW_MASK, 0xF, false);
-    const uint32_t other_lo = (uint32_t)__builtin_amdgcn_update_dpp((int)lo, (int)lo, CTRL, ROW_MASK, 0xF, false);
-    const bool take = other_hi > hi || (other_hi == hi && other_lo > lo);
-    hi = take ? other_hi : hi;
-    lo = take ? other_lo : lo;
+    return max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, ROW_MASK, 0xF, false));
 }
-__device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v) {
-    uint32_t hi = (uint32_t)(v >> 32), lo = (uint32_t)v;
-    dpp_max_step<0xB1, 0xF>(hi, lo);   // quad_perm [1,0,3,2]
-    dpp_max_step<0x4E, 0xF>(hi, lo);   // quad_perm [2,3,0,1]
-    dpp_max_step<0x141, 0xF>(hi, lo);  // row_half_mirror
-    dpp_max_step<0x140, 0xF>(hi, lo);  // row_mirror
-    dpp_max_step<0x142, 0xA>(hi, lo);  // row_bcast:15 into rows 1 and 3
-    dpp_max_step<0x143, 0xC>(hi, lo);  // row_bcast:31 into rows 2 and 3
-    const uint32_t top_hi = (uint32_t)__builtin_amdgcn_readlane((int)hi, 63);
-    const uint32_t top_lo = (uint32_t)__builtin_amdgcn_readlane((int)lo, 63);
-    return ((unsigned long long)top_hi << 32) | top_lo;
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+    v = dpp_max_step<0xB1, 0xF>(v);   // quad_perm [1,0,3,2]
+    v = dpp_max_step<0x4E, 0xF>(v);   // quad_perm [2,3,0,1]
+    v = dpp_max_step<0x141, 0xF>(v);  // row_half_mirror
+    v = dpp_max_step<0x140, 0xF>(v);  // row_mirror
+    v = dpp_max_step<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
+    v = dpp_max_step<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
@@ -50,54 +42,63 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
-// The routes of one row, by one wave: each lane keeps LOCAL = ceil(E/64) keys (rounded up to a power
-// of two) in registers.  Key = ordered score in the high word, (E - id) in the low word, so one max
-// picks the score and the lowest id on ties.  Lane `rank` writes ids[row, rank] and prob[row, rank].
+// The logits of one row as one wave holds them: LOCAL = ceil(E/64) (rounded up to a power of two) per lane.
 template <int LOCAL>
-__device__ __forceinline__ void select_routes(const float* __restrict__ logits, int* ids, float* prob, int row, int e,
-                                              int top_k, int renormalize, int lane) {
-    unsigned long long keys[LOCAL];
-    float all_exp = 0.f;
+__device__ __forceinline__ void load_route_logits(float (&values)[LOCAL], const float* __restrict__ logits, int e, int lane) {
+#pragma unroll
+    for (int j = 0; j < LOCAL; ++j) values[j] = logits[min(j * 64 + lane, e - 1)];
+}
+
+// The routes of one row, by one wave: the largest score first, the lowest id on ties.  A rank is one maximum of 32-bit keys and
+// one ballot per held key for the lowest id that has it; what depends on the score alone waits for the end.  (64-bit keys of
+// score and id, with the exponential inside the loop, took 0.3 us a rank.)  Lane `rank` writes ids[rank] and, where `prob` is
+// not null, prob[rank].
+template <int LOCAL>
+__device__ __forceinline__ void select_routes(const float (&values)[LOCAL], int* ids, float* prob, int e, int top_k, int renormalize,
+                                              int lane) {
+    uint32_t keys[LOCAL];
+    uint32_t open = 0;  // bit j: key j is there and not taken yet
     float local_max = -INFINITY;
 #pragma unroll
     for (int j = 0; j < LOCAL; ++j) {
-        const int id = j * 64 + lane;
-        keys[j] = 0ull;
-        if (id < e) {
-            const float v = logits[(int64_t)row * e + id];
-            keys[j] = ((unsigned long long)ordered_key(v) << 32) | (unsigned long long)(uint32_t)(e - id);
-            local_max = fmaxf(local_max, v);
-        }
+        const bool live = j * 64 + lane < e;
+        keys[j] = live ? ordered_key(values[j]) : 0u;
+        open |= live ? 1u << j : 0u;
+        if (live) local_max = fmaxf(local_max, values[j]);
     }
+    int my_id = e;
+    uint32_t my_key = 0;  // of rank == lane
+    for (int rank = 0; rank < top_k; ++rank) {
+        uint32_t best = keys[0];
+#pragma unroll
+        for (int j = 1; j < LOCAL; ++j) best = max(best, keys[j]);
+        best = wave_max_u32(best);
+        int id = e;  // (never more ranks than ids)
+#pragma unroll
+        for (int j = LOCAL - 1; j >= 0; --j) {
+            const unsigned long long having = __ballot(keys[j] == best && (open >> j & 1u));
+            if (having != 0) id = j * 64 + __builtin_ctzll(having);
+        }
+#pragma unroll
+        for (int j = 0; j < LOCAL; ++j)
+            if (j * 64 + lane == id) keys[j] = 0u, open &= ~(1u << j);
+        if (lane == rank) my_id = id, my_key = best;
+    }
+    if (lane < top_k) ids[lane] = my_id;
+    if (prob == nullptr) return;
     float global_max = local_max;
 #pragma unroll
     for (int offset = 32; offset > 0; offset >>= 1) global_max = fmaxf(global_max, __shfl_xor(global_max, offset, 64));
+    float all_exp = 0.f;
     if (!renormalize) {
 #pragma unroll
-        for (int j = 0; j < LOCAL; ++j) {
-            const int id = j * 64 + lane;
-            if (id < e) all_exp += expf(logits[(int64_t)row * e + id] - global_max);
-        }
+        for (int j = 0; j < LOCAL; ++j)
+            if (j * 64 + lane < e) all_exp += expf(values[j] - global_max);
         all_exp = wave_sum(all_exp);
     }
-    float mine = 0.f;  // numerator of rank == lane
-    for (int rank = 0; rank < top_k; ++rank) {
-        unsigned long long best = 0ull;
-#pragma unroll
-        for (int j = 0; j < LOCAL; ++j) best = keys[j] > best ? keys[j] : best;
-        best = wave_max_u64(best);
-        const int id = e - (int)(uint32_t)(best & 0xFFFFFFFFull);
-        const float score = key_value((uint32_t)(best >> 32));
-#pragma unroll
-        for (int j = 0; j < LOCAL; ++j)
-            if (j * 64 + lane == id) keys[j] = 0ull;
-        if (lane == rank) {
-            ids[(int64_t)row * top_k + rank] = id;
-            mine = expf(score - global_max);
-        }
-    }
-    const float selected_sum = wave_sum(lane < top_k ? mine : 0.f);
-    if (lane < top_k) prob[(int64_t)row * top_k + lane] = __fdiv_rn(mine, renormalize ? selected_sum : all_exp);
+    const float mine = lane < top_k ? expf(key_value(my_key) - global_max) : 0.f;
+    const float selected_sum = wave_sum(mine);
+    if (lane < top_k) prob[lane] = __fdiv_rn(mine, renormalize ? selected_sum : all_exp);
 }
 
 }  // namespace orx
