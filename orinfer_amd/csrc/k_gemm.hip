@@ -697,13 +697,16 @@ int tile_for(const orx_function& f, int rows) {
     return f.tile_hint && rows <= f.tile_hint ? f.tile_hint : 0;
 }
 
-// Channel runs with K split over the waves (k_runs.hip), `algorithm=runs` by name, and by `auto` from two rows on while the
+// Channel runs with K split over the waves (k_runs.hip), `algorithm=runs` by name, and by `auto` (int8 from one row on, codes from two) while the
 // workgroups fit one round of the CUs (up to 64 rows: any number, the tiles are low).  Measured against what `auto` launched
 // before (us, N x K, 256 CUs):
 //   int8: 5120 x 17408 24 / 64 / 96 / 128 rows 32 -> 23, 45 -> 32, 46 -> 41, 47 -> 49; 17408 x 5120 24 / 64 rows 32 -> 21, 48 -> 27;
 //     4096 x 4096 32 / 96 / 256 rows 9.8 -> 7.3, 19 -> 11, 22 -> 14; 1024 x 17408 16 / 64 rows three times faster; level
 //     with the streaming kernel where that has a whole number of workgroups per CU (8192 x 8192, 4-16 rows: 0.92-0.96) or
 //     little to stream (1024 x 1024 up to 32 rows: 0.92-0.98): left there.
+//     One row, against the GEMV, whose workgroups own 32 channels and leave CUs idle or half a round empty: 5120 x 17408 20.5 ->
+//     17.9, 17408 x 5120 19.6 -> 18.3, 8192 x 8192 16.8 -> 14.3, 4096 x 4096 7.2 -> 6.4, 2048 x 2048 3.5 -> 3.4; where the runs take
+//     two rounds (34816 x 5120: 33.0 against 33.8) or below 4 M weights (1024 x 2048: 3.5 against 3.9) it stays.
 //   two-stage codes: 48 / 64 rows 17408 x 5120 31 -> 21, 31 -> 23, 7168 x 5120 12.7 -> 11.1, 14.8 -> 12.3; 96 / 128 / 200 / 256
 //     rows 7168 x 5120 22 -> 17, 25 -> 21, 36 -> 28, 36 -> 31; 4096 x 8192 200 rows 1.4, 1024 x 1024 200 rows 2.9 times faster; wider
 //     matrices go to the channel runs over all rows (11008 x 4096 at 128 / 256 rows 0.96 / 0.87).  Up to 32 rows the
@@ -712,7 +715,7 @@ int tile_for(const orx_function& f, int rows) {
 // Above 128 rows K = 1024 and row tiles of more than 120 rows stay with the split tiles, whose callers provide a Workspace.
 bool use_runs(const orx_function& f, int rows) {
     if (f.algorithm == kRuns) return runs_eligible(f.flags, rows, f.N, f.K);
-    if (f.algorithm != kAuto || tile_for(f, rows) != 0 || rows < 2 || f.K % kBK != 0 || !runs_eligible(f.flags, rows, f.N, f.K)) return false;
+    if (f.algorithm != kAuto || tile_for(f, rows) != 0 || rows < (f.flags == kW8 ? 1 : 2) || f.K % kBK != 0 || !runs_eligible(f.flags, rows, f.N, f.K)) return false;
     if ((f.flags2 & kPreferGemv) && f.block_m > 0 && rows <= 4) return false;  // the dot-product family wherever it serves the rows
     const int64_t weights = (int64_t)f.N * f.K;
     if (rows > 64) {
@@ -721,6 +724,7 @@ bool use_runs(const orx_function& f, int rows) {
         if (rows > 128 && (f.K <= 1024 || tile_rows > 120)) return false;
         return f.flags == kW8 ? rows <= 112 || f.K <= 8192 : f.N <= 32 * device_compute_units();
     }
+    if (f.flags == kW8 && rows == 1) return weights >= (1 << 22) && f.N <= 80 * device_compute_units();
     if (f.flags == kW8) return rows > 32 || (weights >= (1 << 22) && (rows > 16 || f.N % (32 * device_compute_units()) != 0));
     if (rows > 32) return weights >= (1 << 22);
     return f.K > 5120 && f.N <= 32 * device_compute_units();

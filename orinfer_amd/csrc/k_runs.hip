@@ -87,7 +87,11 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
     if constexpr (CODEC == kRunsQ4)
         if (tid < 256) selector = p.book[tid];
 
-    // ---- requests: eight rows of 128 bytes each.  Requests behind the one that holds the last row repeat that one ----
+    // ---- requests: eight rows of 128 bytes each.  Requests behind the one that holds the last row repeat that one, so that every
+    // chunk counts the same.  int8: where the last request of a tile or a run would be such a repeat it is left out of every
+    // chunk (what its rows hold in LDS reaches no stored sum): 5120 x 17408 of 24 rows, 20 channels to a CU, has six requests
+    // a chunk instead of eight, 24.7 -> 24.1 us with the quantiser, of one row 18.7 -> 17.9 without it.  (Codes: the branch
+    // costs the step between the chunks more than a request: 17408 x 5120 of 48 rows 21.7 -> 25.3.) ----
     struct Rows {
         uint32_t even, odd, last;  // lane offsets in an even and an odd request, and in the last one
         int last_request;
@@ -102,6 +106,7 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
         return r;
     };
     const Rows token_rows = rows_of(rows), weight_rows = rows_of(channels);
+    const int left_out = CODEC == kRunsW8 ? (token_rows.last_request < 2 * TB - 1) + (weight_rows.last_request < 2 * CB - 1) : 0;
     uint8_t* const ring = lds + runs_tables<CODEC>() + (uint32_t)wave * (D * kStage);
     const int8_t* const a_base = uniform_pointer(p.a + (int64_t)first_row * p.k);
     const uint8_t* const w_base = uniform_pointer(p.w + (int64_t)first_channel * p.row_stride);
@@ -109,6 +114,7 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
         constexpr int BLOCKS = decltype(blocks_tag)::value;
 #pragma unroll
         for (int i = 0; i < 2 * BLOCKS; ++i) {
+            if (CODEC == kRunsW8 && i == 2 * BLOCKS - 1 && r.last_request < i) break;  // uniform
             const bool tail = i >= r.last_request;  // uniform
             uint32_t offset = tail ? r.last : i & 1 ? r.odd : r.even;
             asm volatile("" : "+v"(offset));  // 32 bits beside a uniform base
@@ -144,7 +150,13 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
     };
     // waits until at most `CHUNKS` of the youngest chunks requested are still on their way
     auto wait_requests = [&](auto chunks_tag) ORX_INLINE {
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(chunks_tag)::value * kRequests) : "memory");
+        constexpr int CHUNKS = decltype(chunks_tag)::value;
+        if (CHUNKS == 0 || left_out == 0)
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(CHUNKS * kRequests) : "memory");
+        else if (left_out == 1)
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(CHUNKS * (kRequests - 1)) : "memory");
+        else
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(CHUNKS * (kRequests - 2)) : "memory");
         name_codes();
     };
     request(0, std::integral_constant<int, 0>{});
@@ -432,6 +444,28 @@ const RunsForm* runs_forms(int* count) {
     return forms;
 }
 
+// the forms of a codec and a tile height, widest last: they follow one another in the list (every call of a handle asks several
+// times, so the list is not searched each time)
+struct RunsFormRange {
+    const RunsForm* first;
+    int count;
+};
+RunsFormRange runs_forms_of(int codec, int tb) {
+    struct Index {
+        RunsFormRange of[2][9] = {};
+        Index() {
+            int count = 0;
+            const RunsForm* forms = runs_forms(&count);
+            for (int i = 0; i < count; ++i) {
+                RunsFormRange& range = of[forms[i].codec == kRunsW8][forms[i].tb];
+                if (range.count++ == 0) range.first = &forms[i];
+            }
+        }
+    };
+    static const Index index;
+    return index.of[codec == kRunsW8][tb];
+}
+
 constexpr int kRunsMaxRows = 512;
 
 // How a launch is cut: rows into tiles of up to 128, channels into runs so that the workgroups fill whole rounds of the CUs.
@@ -440,15 +474,12 @@ struct RunsShape {
     int row_tiles, tile_rows, runs, run;
 };
 RunsShape runs_shape(int codec, int rows, int n) {
-    int count = 0;
-    const RunsForm* forms = runs_forms(&count);
     RunsShape s = {};
     s.row_tiles = (rows + 127) / 128;
     s.tile_rows = (rows + s.row_tiles - 1) / s.row_tiles;
     const int blocks = (s.tile_rows + 15) / 16;
-    int most = 0;
-    for (int i = 0; i < count; ++i)
-        if (forms[i].codec == codec && forms[i].tb == blocks) most = std::max(most, forms[i].cb);
+    const RunsFormRange forms = runs_forms_of(codec, blocks);
+    const int most = forms.first[forms.count - 1].cb;
     const int cus = device_compute_units();
     const int column_blocks = (n + 15) / 16;
     // fewest rounds of the CUs whose runs fit the widest form, then the runs as even as whole rounds make them
@@ -457,10 +488,8 @@ RunsShape runs_shape(int codec, int rows, int n) {
     s.runs = std::max(least_runs, rounds * cus / s.row_tiles);
     s.run = (n + s.runs - 1) / s.runs;
     s.runs = (n + s.run - 1) / s.run;
-    for (int i = 0; i < count; ++i)
-        if (forms[i].codec == codec && forms[i].tb == blocks && 16 * forms[i].cb >= s.run &&
-            (s.form == nullptr || forms[i].cb < s.form->cb))
-            s.form = &forms[i];
+    for (int i = forms.count - 1; i >= 0; --i)
+        if (16 * forms.first[i].cb >= s.run) s.form = &forms.first[i];
     return s;
 }
 

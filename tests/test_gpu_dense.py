@@ -1494,3 +1494,20 @@ def test_channel_runs_refuse_what_they_do_not_serve():
     for bad in (dict(M=513), dict(K=192)):
         with pytest.raises(gu.lib.OrxError):
             gu.kernel("int8_projection", **{**dict(M=8, N=256, K=256, algorithm="runs"), **bad})
+
+
+# The last request of a tile (8 rows) or of a run (8 channels) is left out where it would hold no row; a short last tile or run
+# beside full ones; rows of fp16 outputs that start at odd elements.
+@pytest.mark.parametrize("rows,n", [(1, 5120), (7, 6144), (8, 5120), (9, 6144), (24, 5130), (25, 6400), (40, 2048), (137, 2600)])
+@pytest.mark.parametrize("algorithm", ["auto", "runs"])
+def test_channel_runs_int8_weights_short_requests(rows, n, algorithm):
+    k = 2176  # 17 chunks: two to a wave, three to the last
+    rng = np.random.default_rng(orc.SEED + rows * n)
+    weight = rng.integers(-128, 128, (n, k), dtype=np.int8)
+    a_q = rng.integers(-127, 128, (rows, k), dtype=np.int8)
+    a_s = rng.uniform(0.005, 0.02, rows).astype(np.float16)
+    ws = rng.uniform(0.005, 0.02, n).astype(np.float16)
+    out = torch.full((rows + 1, n + 1), 91, dtype=torch.float16, device=gu.DEV)
+    gu.w8_project(gu.dev(a_q), gu.dev(a_s), gu.dev(weight), gu.dev(ws), out=out, rows=rows, stride=n + 1, algorithm=algorithm)
+    np.testing.assert_array_equal(gu.host(out)[:rows, :n], orc.project(a_q, a_s, weight, ws))
+    assert (gu.host(out)[rows] == 91).all() and (gu.host(out)[:, n] == 91).all()
