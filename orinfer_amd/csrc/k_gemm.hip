@@ -712,7 +712,15 @@ int tile_for(const orx_function& f, int rows) {
 //     matrices go to the channel runs over all rows (11008 x 4096 at 128 / 256 rows 0.96 / 0.87).  Up to 32 rows the
 //     batched-decode kernels are faster where they take K (17408 x 5120: 0.8-0.9), and slower where the
 //     streaming kernel stands in for them (2560 x 9728 and 2048 x 16384: 1.1-2.4).
-// Above 128 rows K = 1024 and row tiles of more than 120 rows stay with the split tiles, whose callers provide a Workspace.
+//     Rows of K = 5120 from 17 on: 20 / 32 rows 7168 x 5120 10.6 -> 9.8, 11.9 -> 10.8, 2048 x 5120 7.6 -> 6.8 at 24; level or slower at
+//     K <= 4096 (4096 x 4096 7.0 / 7.1 at 20 rows).  66 / 80 rows of up to 48 channels to a CU, against one pass over all rows:
+//     11008 x 4096 20.5 -> 17.9, 20.2 -> 18.0, 12288 x 3072 17.0 -> 15.7, 17.1 -> 15.9; slower at 68 channels (17408 x 5120 30.8 / 38.5).
+//   129 to 512 rows, against split tiles and decode-once with their scratch: codes 256 rows 4096 x 4096 27.4 -> 17.4, 2560 x 9728 33.6 ->
+//     28.6, 512 rows 4096 x 4096 32 -> 26, 2048 x 1024 24 -> 9, 136 / 200 rows 11008 x 4096 40.9 -> 32.4, 41.4 -> 38.1 in two rounds;
+//     int8 256 rows 4096 x 4096 23.6 -> 14.8, 2048 x 1024 20.3 -> 7.5, 136 / 200 rows 5120 x 17408 49.8 -> 38.6, 50.4 -> 45.7.  Two
+//     rounds of more than 200 rows lose (11008 x 4096 at 300 / 512 rows 47 / 55, 50 / 72; int8 5120 x 5120 at 512 41 / 47).  Row
+//     tiles of more than 120 rows and K up to 1024 go to the runs up to 16 channels to a CU only: handles of wider matrices say
+//     that they need scratch for these launches, and the split tiles that use it stay (7168 x 5120 at 256 rows 38.6, the runs 30.4).
 bool use_runs(const orx_function& f, int rows) {
     if (f.algorithm == kRuns) return runs_eligible(f.flags, rows, f.N, f.K);
     if (f.algorithm != kAuto || tile_for(f, rows) != 0 || rows < (f.flags == kW8 ? 1 : 2) || f.K % kBK != 0 || !runs_eligible(f.flags, rows, f.N, f.K)) return false;
@@ -720,14 +728,17 @@ bool use_runs(const orx_function& f, int rows) {
     const int64_t weights = (int64_t)f.N * f.K;
     if (rows > 64) {
         int tile_rows = 0;
-        if (runs_rounds(f.flags, rows, f.N, &tile_rows) != 1 || (f.flags2 & kNoSplit)) return false;
-        if (rows > 128 && (f.K <= 1024 || tile_rows > 120)) return false;
-        return f.flags == kW8 ? rows <= 112 || f.K <= 8192 : f.N <= 32 * device_compute_units();
+        const int rounds = runs_rounds(f.flags, rows, f.N, &tile_rows), cus = device_compute_units();
+        if (f.flags2 & kNoSplit) return false;
+        if (rows > 128 && (f.K <= 1024 || tile_rows > 120)) return rounds == 1 && f.K <= 10240 && f.N <= 16 * cus;
+        if (f.flags == kW8) return rounds == 1 && (rows <= 112 || f.K <= 8192 || (rows > 128 && tile_rows <= 100));
+        if (rows <= 80 || (rows > 128 && rows <= 200)) return rounds <= (rows <= 80 || f.K <= 1024 ? 1 : 2) && f.N <= 48 * cus;
+        return rounds == 1 && f.N <= 32 * cus;
     }
     if (f.flags == kW8 && rows == 1) return weights >= (1 << 22) && f.N <= 80 * device_compute_units();
     if (f.flags == kW8) return rows > 32 || (weights >= (1 << 22) && (rows > 16 || f.N % (32 * device_compute_units()) != 0));
     if (rows > 32) return weights >= (1 << 22);
-    return f.K > 5120 && f.N <= 32 * device_compute_units();
+    return (f.K > 5120 || (f.K == 5120 && rows > 16)) && f.N <= 32 * device_compute_units();
 }
 
 // Channel runs per CU over the whole K (k_wide.hip): two-stage codes, `algorithm=wide` by name, and by

@@ -1511,3 +1511,29 @@ def test_channel_runs_int8_weights_short_requests(rows, n, algorithm):
     gu.w8_project(gu.dev(a_q), gu.dev(a_s), gu.dev(weight), gu.dev(ws), out=out, rows=rows, stride=n + 1, algorithm=algorithm)
     np.testing.assert_array_equal(gu.host(out)[:rows, :n], orc.project(a_q, a_s, weight, ws))
     assert (gu.host(out)[rows] == 91).all() and (gu.host(out)[:, n] == 91).all()
+
+
+# Row counts at which `auto` hands a projection to the channel runs: handles with a Workspace and without, both codecs, either side
+# of a row tile, one and two rounds of the CUs.
+@pytest.mark.parametrize("rows,n,k", [(17, 1040, 5120), (80, 8208, 1152), (81, 8208, 1152), (129, 8208, 1152), (200, 8208, 1152), (201, 8208, 1152),
+                                      (240, 4096, 1152), (256, 4096, 1152), (257, 1040, 1024), (512, 1040, 1152)])
+def test_auto_rows_around_the_channel_runs(rows, n, k):
+    rng = np.random.default_rng(orc.SEED + 3 * rows + n)
+    packed = rng.integers(0, 2**32, (n, k // 8), dtype=np.uint32)
+    weight = rng.integers(-128, 128, (n, k), dtype=np.int8)
+    a_q = rng.integers(-127, 128, (rows, k), dtype=np.int8)
+    a_s = rng.uniform(0.005, 0.02, rows).astype(np.float16)
+    ws = rng.uniform(0.005, 0.02, n).astype(np.float16)
+    want4 = orc.project(a_q, a_s, orc.q4_integers(packed, TABLE), ws)
+    want8 = orc.project(a_q, a_s, weight, ws)
+    for scratch in (False, True):
+        variant = dict(M=rows, N=n, K=k, dynamic_rows=True, workspace=scratch)
+        q4, w8 = gu.lib.Kernel("e8p_q4_projection", **variant), gu.lib.Kernel("int8_projection", **variant)
+        out = torch.full((rows, n), 9.0, dtype=torch.float16, device=gu.DEV)
+        extra = {"Workspace": q4.workspace()} if scratch else {}
+        q4(A=gu.dev(a_q), AS=gu.dev(a_s), Book=gu.book(), Out=out, S=gu.dev(ws), W=gu.dev(packed), m=rows, **extra)
+        np.testing.assert_array_equal(gu.host(out), want4)
+        out.fill_(9.0)
+        extra = {"Workspace": w8.workspace()} if scratch else {}
+        w8(A=gu.dev(a_q), Output=out, TokenScale=gu.dev(a_s), Weight=gu.dev(weight), WeightScale=gu.dev(ws), m=rows, **extra)
+        np.testing.assert_array_equal(gu.host(out), want8)
