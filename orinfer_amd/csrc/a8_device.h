@@ -8,6 +8,29 @@
 
 namespace orx {
 
+// Maximum of a 32-bit key over the wave with data-parallel-primitive moves only: a shuffle is an LDS round trip, and the few-row
+// kernels wait for every one of them.  Quad swaps, half-row and row mirrors give every lane its row's maximum; two
+// broadcasts carry it across rows into lane 63, which is then read back as a scalar.
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ uint32_t dpp_max_step(uint32_t v) {
+    // lanes outside ROW_MASK receive their own value back
+    return max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, ROW_MASK, 0xF, false));
+}
+__device__ __forceinline__ uint32_t row_max_u32(uint32_t v) {  // over each row of 16 lanes, known to the row
+    v = dpp_max_step<0xB1, 0xF>(v);      // quad_perm [1,0,3,2]
+    v = dpp_max_step<0x4E, 0xF>(v);      // quad_perm [2,3,0,1]
+    v = dpp_max_step<0x141, 0xF>(v);     // row_half_mirror
+    return dpp_max_step<0x140, 0xF>(v);  // row_mirror
+}
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+    v = row_max_u32(v);
+    v = dpp_max_step<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
+    v = dpp_max_step<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+// of magnitudes (never NaN, never -0): their bits order as they do
+__device__ __forceinline__ float wave_max_magnitude(float v) { return __uint_as_float(wave_max_u32(__float_as_uint(v))); }
+
 // fp16 scale of a group from its largest magnitude: max(amax / 127, 2^-24), or 1 for an all-zero group.
 __device__ __forceinline__ __half a8_scale(float amax) {
     const float raw_scale = fmaxf(__fdiv_rn(amax, 127.0f), 5.9604644775390625e-08f);

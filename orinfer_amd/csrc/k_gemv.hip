@@ -512,8 +512,7 @@ __global__ __launch_bounds__(kBankedThreads) void gemv_banked_kernel(
 #pragma unroll
         for (int j = 0; j < 8; ++j)
             if (tid < groups) amax = fmaxf(amax, fabsf(value[j]));
-#pragma unroll
-        for (int offset = 32; offset > 0; offset >>= 1) amax = fmaxf(amax, __shfl_xor(amax, offset, 64));
+        amax = wave_max_magnitude(amax);
         if (lane == 0) wave_max[wave] = amax;
         __syncthreads();
         // the 16 wave maxima, one per lane of a row, reduced with lane controls (no LDS round trips):
@@ -978,8 +977,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_gemv_kernel(
                 amax = fmaxf(amax, fmaxf(fabsf(f.x), fabsf(f.y)));
             }
         }
-#pragma unroll
-        for (int offset = 32; offset > 0; offset >>= 1) amax = fmaxf(amax, __shfl_xor(amax, offset, 64));
+        amax = wave_max_magnitude(amax);
         if (lane == 0) route_wave_max[wave] = amax;
         __syncthreads();
         routes_published();

@@ -40,8 +40,7 @@ __device__ __forceinline__ void wave_quantise_row(const __half* __restrict__ x, 
 #pragma unroll
     for (int i = 0; i < kHeldPieces; ++i) raise(held[i]);  // (repeats of the last piece among them)
     for (int at = lane + 64 * kHeldPieces; at < pieces; at += 64) raise(row_pieces[at]);
-#pragma unroll
-    for (int offset = 32; offset > 0; offset >>= 1) amax = fmaxf(amax, __shfl_xor(amax, offset, 64));
+    amax = wave_max_magnitude(amax);
     const __half stored = a8_scale(amax);
     if (lane == 0) s[row] = stored;
     const float scale = __half2float(stored), inverse = __frcp_rn(scale);
@@ -623,8 +622,7 @@ __global__ __launch_bounds__(256) void quantize_dispatch_kernel(const __half* __
             amax = fmaxf(amax, fmaxf(fabsf(f.x), fabsf(f.y)));
         }
     }
-#pragma unroll
-    for (int offset = 32; offset > 0; offset >>= 1) amax = fmaxf(amax, __shfl_xor(amax, offset, 64));
+    amax = wave_max_magnitude(amax);
     if ((tid & 63) == 0) wave_max[tid >> 6] = amax;
     __syncthreads();
     amax = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));

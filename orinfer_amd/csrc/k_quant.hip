@@ -39,15 +39,12 @@ __device__ __forceinline__ float load_value(const __half* __restrict__ x, const 
 }
 
 __device__ __forceinline__ float block_max(float v, float* scratch) {
-#pragma unroll
-    for (int offset = 32; offset > 0; offset >>= 1) v = fmaxf(v, __shfl_xor(v, offset, 64));
+    v = wave_max_magnitude(v);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (lane == 0) scratch[wave] = v;
     __syncthreads();
-    const int waves = (blockDim.x + 63) >> 6;
-    float r = scratch[0];
-    for (int i = 1; i < waves; ++i) r = fmaxf(r, scratch[i]);
-    return r;
+    const int waves = (blockDim.x + 63) >> 6;  // 16 at most
+    return __uint_as_float(row_max_u32(__float_as_uint(scratch[min(lane & 15, waves - 1)])));
 }
 
 // Masked rows and groups longer than the held form takes: two passes over the group, grid (rows, groups).
@@ -133,8 +130,7 @@ __global__ __launch_bounds__(WAVES == 1 ? 256 : 64 * WAVES) void a8_held_kernel(
             amax = fmaxf(amax, fabsf(load_value<FUSED, false>(x, nullptr, in_base, k, first + i)));
     }
     if (WAVES == 1) {
-#pragma unroll
-        for (int offset = 32; offset > 0; offset >>= 1) amax = fmaxf(amax, __shfl_xor(amax, offset, 64));
+        amax = wave_max_magnitude(amax);
     } else {
         amax = block_max(amax, scratch);
     }

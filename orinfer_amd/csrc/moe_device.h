@@ -7,6 +7,8 @@
 #include <cmath>
 #include <cstdint>
 
+#include "a8_device.h"
+
 namespace orx {
 
 // Total order on finite fp32 with -0 == +0 (moe.py:449-465): larger key = larger score.
@@ -19,23 +21,6 @@ __device__ __forceinline__ float key_value(uint32_t ordered) {
     return __uint_as_float((ordered & 0x80000000u) ? ordered ^ 0x80000000u : ~ordered);
 }
 
-// Maximum of a 32-bit key over the wave with data-parallel-primitive moves only (no LDS round trips: the selection loop below
-// is a chain of top_k dependent reductions).  Quad swaps, half-row and row mirrors give every lane its row's maximum; two
-// broadcasts carry it across rows into lane 63, which is then read back as a scalar.
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ uint32_t dpp_max_step(uint32_t v) {
-    // lanes outside ROW_MASK receive their own value back
-    return max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, ROW_MASK, 0xF, false));
-}
-__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-    v = dpp_max_step<0xB1, 0xF>(v);   // quad_perm [1,0,3,2]
-    v = dpp_max_step<0x4E, 0xF>(v);   // quad_perm [2,3,0,1]
-    v = dpp_max_step<0x141, 0xF>(v);  // row_half_mirror
-    v = dpp_max_step<0x140, 0xF>(v);  // row_mirror
-    v = dpp_max_step<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
-    v = dpp_max_step<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
-    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
-}
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
     for (int offset = 32; offset > 0; offset >>= 1) v += __shfl_xor(v, offset, 64);
