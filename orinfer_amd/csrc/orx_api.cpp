@@ -48,7 +48,19 @@ int current_device() {
     return device;
 }
 
+// The CU count of one call on this thread.  Choosing a kernel asks for it ten to twenty times a row count, and asking the
+// runtime for the current device each time was most of what orx_workspace_bytes(0) took (8192 row counts: 7 to 12 ms).
+static thread_local int t_held_units = 0;
+struct HeldUnits {
+    const bool outermost;
+    HeldUnits() : outermost(t_held_units == 0) { t_held_units = device_compute_units(); }
+    ~HeldUnits() { if (outermost) t_held_units = 0; }
+    HeldUnits(const HeldUnits&) = delete;
+    HeldUnits& operator=(const HeldUnits&) = delete;
+};
+
 int device_compute_units() {
+    if (t_held_units != 0) return t_held_units;
     static std::atomic<int> cached[64];
     const int slot = current_device() & 63;
     int units = cached[slot].load(std::memory_order_relaxed);
@@ -666,6 +678,7 @@ int orx_workspace_bytes(orx_fn f, int32_t rows, uint64_t* bytes) {
             return (int)ORX_OK;
         }
         // rows <= 0 on a dynamic kernel: what the engine allocates once, the largest need of any row count
+        const HeldUnits held;
         uint64_t most = 0;
         for (int r = 1; r <= f->capacity; ++r) most = std::max(most, workspace_need(f, r));
         *bytes = most;
@@ -699,6 +712,7 @@ int orx_launch(orx_fn f, const uint32_t grid[3], const uint32_t block[3], uint32
 
 int orx_enqueue(orx_fn f, void* hip_stream, void** args) {
     return guard("orx_enqueue", [&, args]() mutable {
+        const HeldUnits held;
         int rows = 0;
         Geometry want;
         void* full[64];
