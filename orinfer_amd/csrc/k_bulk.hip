@@ -21,6 +21,10 @@
 // gate_up 296 -> 100 us, down 215 -> 86 us.  What bounds it now: no pipe is full (LDS 42 %, vector ALU 40 %, matrix pipe
 // 30 % of the cycles); the two waves of a SIMD wait for each other's LDS reads and barriers in a third of theirs.
 // One persistent workgroup of eight waves per CU that requests the next unit's chunks early measured 118 and 75 us.
+// Down without its stores takes 14 us less, without the K loop 55, without either 42 (K = 512: four chunks between set-up and
+// epilogue).  A workgroup that takes 2, 4 or 8 spans of a tile in a row, the next one's chunks requested in the last steps, and 512
+// persistent workgroups of this form with even shares both measured level or slower (whole layer 227 / 241 / 247 and 243 against
+// 226 us): what the set-up saves, the uneven ends lose.
 //  * SWIGLU: a wave owns 32 gate and the 32 matching up channels, so gate and up of one (slot, channel) meet in one
 //    lane; the epilogue writes fp16(silu(gate) * up) and, where asked, gate | up and the slots' largest magnitudes.
 #include <hip/hip_fp16.h>

@@ -10,8 +10,9 @@
 //  * K is split over the decoding waves.  A wave keeps the token fragments of its K slice in
 //    registers for the whole kernel (they are the same for every channel block), so activations are
 //    read once per CU.
-//  * Codes are decoded with two 8-byte lookups per stage in tables stored 16 times (one copy per
-//    lane of an access group, so lanes never share a bank; the address is one v_perm_b32); the two
+//  * Codes are decoded with two 8-byte lookups per stage in tables stored 16 times; of 32 neighbouring lanes half
+//    read one table and half the other, so no two meet in a bank (all lanes in the same table met in pairs: 17408 x 5120 of
+//    8 rows, quantiser included, 16.5 -> 15.9 us; a layer's three at 20 rows 1 us).  The address is one v_perm_b32; the two
 //    stages share one pair of tables (values v+8, shifted by the stage's weight when combined).
 //  * The K-slice partial sums of a block are added with LDS integer atomics (exact in any order);
 //    after a barrier 16 x M threads rescale and store the block while the others decode the next.
