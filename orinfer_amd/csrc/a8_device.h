@@ -76,17 +76,18 @@ __device__ __forceinline__ uint32_t quantise4(const float (&value)[4], float sca
 
 // A stable sigmoid in fp32: e = exp(-|gate|), (gate >= 0 ? 1 : e) / (1 + e).  exp(x) = 2^(x log2 e): the hardware
 // exponential of the rounded product, corrected to first order by what the rounding took off (one fused multiply-add
-// recovers it: x - t ln 2), so it is good to one unit in the last place.  The quotient is the reciprocal with one Newton step
-// and one residual correction (Markstein's division): correctly rounded up to rare ties, for a denominator in
-// [1, 2].  Below -87 the exponential would leave the normal numbers and no product with two fp16 values of it rounds
-// to anything but 0, so the argument stops there.  Fifteen instructions, two of them transcendental, where the library
-// exponential and quotient took about thirty (8192 rows of 17408 values were bound by them).
+// recovers it: x - t ln 2).  The hardware exponential gives 0 instead of subnormal numbers, so the whole power of two goes
+// on at the end: e is subnormal below -87.4 and 0 from -104 on (2^-150), where the argument stops, as the fp32 formula
+// has it; a gate of minus infinity thus gives -inf * 0 = NaN, which a quantiser's maximum drops, and not an infinity that
+// would be the row's scale.  The quotient is the reciprocal with one Newton step and one residual correction (Markstein's
+// division): correctly rounded up to rare ties, for a denominator in [1, 2].
 __device__ __forceinline__ float sigmoid_value(float gate) {
-    const float x = fmaxf(-fabsf(gate), -87.f);
+    const float x = fmaxf(-fabsf(gate), -104.f);
     const float t = x * 1.44269502162933349609375f;                       // fp32(log2 e)
     const float rest = __builtin_fmaf(-t, 0.693147182464599609375f, x);   // fp32(ln 2)
-    const float power = __builtin_amdgcn_exp2f(t);
-    const float e = __builtin_fmaf(power, rest, power);
+    const float whole = rintf(t);
+    const float power = __builtin_amdgcn_exp2f(t - whole);
+    const float e = __builtin_amdgcn_ldexpf(__builtin_fmaf(power, rest, power), (int)whole);
     const float denominator = 1.0f + e, numerator = gate >= 0.f ? 1.0f : e;
     const float guess = __builtin_amdgcn_rcpf(denominator);
     const float reciprocal = __builtin_fmaf(__builtin_fmaf(-denominator, guess, 1.0f), guess, guess);

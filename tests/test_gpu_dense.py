@@ -130,6 +130,59 @@ def test_a8_held_forms(rows, k, group, fused):
     np.testing.assert_array_equal(gu.host(q), wq)
 
 
+def test_swiglu_gates_without_a_finite_sigmoid_product():
+    """Gates at and beyond the ends of the exponential against the formula in fp32: a gate of minus infinity has no value
+    (-inf * 0), the gates down to -104 keep a sigmoid above zero, and what the products make of infinities is theirs."""
+    inf, nan = np.inf, np.nan
+    gates = np.array([-inf, inf, nan, -65504, -104.0625, -104, -103.9375, -90, -87.5, -87, -20, -0.0, 0, 1, 88, 65504], np.float16)
+    ups = np.array([1, -3, 65504, inf, -inf, nan, 0, -0.0], np.float16)
+    g, u = (a.reshape(1, -1) for a in np.meshgrid(gates, ups))
+    x = np.concatenate([g, u], axis=1)
+    y = torch.empty(g.shape, dtype=torch.float16, device=gu.DEV)
+    gu.kernel("swiglu", I=g.shape[1])(X=gu.dev(x), Y=y, rows=1)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = orc.swiglu_fp16(x)
+    got = gu.host(y)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(np.isinf(got), np.isinf(want))
+    known = ~np.isnan(want)
+    np.testing.assert_array_equal(np.signbit(got[known]), np.signbit(want[known]))
+    finite = np.isfinite(want)
+    np.testing.assert_allclose(got[finite].astype(np.float32), want[finite].astype(np.float32), rtol=1e-3, atol=6e-8)
+
+
+@pytest.mark.parametrize("rows,k", [
+    (2048, 512), (4, 512),     # one wave to a row
+    (4, 2048), (513, 12288),   # four waves
+    (4, 12296),                # eight waves
+    (4, 32776), (4, 2060),     # too long to hold; rows that are not 16-byte aligned
+])
+def test_a8_of_gates_without_a_value(rows, k):
+    """A gate that gives no number (minus infinity, NaN) leaves the row's scale and its other codes alone; an infinite value
+    is the row's largest: the scale is infinite and every finite value's code is 0."""
+    rng = np.random.default_rng(orc.SEED + rows + k)
+    x = (rng.normal(size=(rows, 2 * k)) * 2).astype(np.float16)
+    at = k // 2 + 3
+    for row, gate in ((0, -np.inf), (1, np.nan), (2, np.inf), (3, -np.inf)):
+        x[row, at] = gate
+    x[3, at + 1] = np.inf  # both in one row: the infinity decides
+    x[:, k + at] = 0.5
+    x[:, k + at + 1] = 0.25
+    y = torch.empty((rows, k), dtype=torch.float16, device=gu.DEV)
+    gu.kernel("swiglu", I=k)(X=gu.dev(x), Y=y, rows=rows)
+    values = gu.host(y)
+    assert np.isnan(values[[0, 1, 3], at]).all() and values[2, at] == np.inf and values[3, at + 1] == np.inf
+    for q, s in (gu.a8(gu.dev(x), fused=True), gu.a8(y)):
+        q, s = gu.host(q), gu.host(s)
+        plain = np.where(np.isfinite(values), values, np.float16(0))
+        wq, ws = orc.a8(plain)
+        live = np.isfinite(values)
+        keep = [r for r in range(rows) if r not in (2, 3)]
+        np.testing.assert_array_equal(s[keep], ws[keep])
+        np.testing.assert_array_equal(q[keep][live[keep]], wq[keep][live[keep]])
+        assert np.isinf(s[2:4]).all() and (q[2:4][live[2:4]] == 0).all()
+
+
 def test_a8_masked_columns():
     rng = np.random.default_rng(orc.SEED)
     x = rng.normal(size=(9, 512)).astype(np.float16)
