@@ -74,23 +74,28 @@ __device__ __forceinline__ uint32_t quantise4(const float (&value)[4], float sca
     return low | (high << 16);
 }
 
-// A stable sigmoid in fp32: e = exp(-|gate|), (gate >= 0 ? 1 : e) / (1 + e).  exp(x) = 2^(x log2 e): the hardware
-// exponential of the rounded product, corrected to first order by what the rounding took off (one fused multiply-add
-// recovers it: x - t ln 2).  The hardware exponential gives 0 instead of subnormal numbers, so the whole power of two goes
-// on at the end: e is subnormal below -87.4 and 0 from -104 on (2^-150), where the argument stops, as the fp32 formula
-// has it; a gate of minus infinity thus gives -inf * 0 = NaN, which a quantiser's maximum drops, and not an infinity that
-// would be the row's scale.  The quotient is the reciprocal with one Newton step and one residual correction (Markstein's
-// division): correctly rounded up to rare ties, for a denominator in [1, 2].
+// A stable sigmoid in fp32: e = exp(-|gate|), (gate >= 0 ? 1 : e) / (1 + e).
+// exp(x) = 2^whole 2^part, whole = rint(x log2 e) (the sum with 1.5 * 2^23 has it in its low bits), part = x log2 e - whole by
+// two fused multiply-adds over log2 e as a pair of fp32 numbers: |part| is at most a half, so its rounding is below that of
+// the hardware exponential, and one fp32 log2 e alone would cost 1.3e-8 * |x|.  The power of two goes on last because the
+// hardware exponential gives 0 instead of subnormal numbers: e is subnormal below -87.4 and 0 from -104 on (2^-150), where
+// the argument stops, as the fp32 formula has it; a gate of minus infinity thus gives -inf * 0 = NaN, which a quantiser's
+// maximum drops, and not an infinity that would be the row's scale.
+// The quotient is the product with the hardware reciprocal and one residual correction: the product is within two units in the
+// last place, so the residual is exact and the correction leaves half a unit and a 2^-22 part of one.
+// With a correctly rounded exponential of part the largest relative error over all fp16 gates is 1.06e-7 from -1 up, 1.55e-7 in
+// [-20, -1) and 6.4e-8 below, as that of a correctly rounded exp and quotient (1.04e-7, 1.55e-7, 5.7e-8); the hardware exponential's
+// own unit in the last place comes on top.  Sixteen instructions, two of them transcendental, where the library exponential and
+// quotient took about thirty (8192 rows of 17408 values were bound by them).
 __device__ __forceinline__ float sigmoid_value(float gate) {
     const float x = fmaxf(-fabsf(gate), -104.f);
-    const float t = x * 1.44269502162933349609375f;                       // fp32(log2 e)
-    const float rest = __builtin_fmaf(-t, 0.693147182464599609375f, x);   // fp32(ln 2)
-    const float whole = rintf(t);
-    const float power = __builtin_amdgcn_exp2f(t - whole);
-    const float e = __builtin_amdgcn_ldexpf(__builtin_fmaf(power, rest, power), (int)whole);
+    const float shifted = __builtin_fmaf(x, 1.44269502162933349609375f, 12582912.0f);  // fp32(log2 e)
+    const float whole = shifted - 12582912.0f;
+    const float rest = __builtin_fmaf(x, 1.44269502162933349609375f, -whole);
+    const float part = __builtin_fmaf(x, 1.925963033500011e-08f, rest);  // fp32(log2 e - fp32(log2 e))
+    const float e = __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(part), __float_as_int(shifted) - 0x4B400000);
     const float denominator = 1.0f + e, numerator = gate >= 0.f ? 1.0f : e;
-    const float guess = __builtin_amdgcn_rcpf(denominator);
-    const float reciprocal = __builtin_fmaf(__builtin_fmaf(-denominator, guess, 1.0f), guess, guess);
+    const float reciprocal = __builtin_amdgcn_rcpf(denominator);
     const float quotient = numerator * reciprocal;
     return __builtin_fmaf(__builtin_fmaf(-denominator, quotient, numerator), reciprocal, quotient);
 }

@@ -183,6 +183,24 @@ def test_a8_of_gates_without_a_value(rows, k):
         assert np.isinf(s[2:4]).all() and (q[2:4][live[2:4]] == 0).all()
 
 
+def test_swiglu_rounds_as_an_unbiased_exponential_does():
+    """Share of fp16 results that differ from the correctly rounded product, where the exponential's argument is large: the
+    fp32 roundings alone (sigmoid within 1.6e-7, two products) cost 0.85e-4 of them there, an exponential that is off by the
+    error of one fp32 ln 2 times its argument 1.1e-4."""
+    rng = np.random.default_rng(orc.SEED + 77)
+    rows, k = 1024, 16384
+    gate = rng.uniform(-18, -10, (rows, k)).astype(np.float16)
+    up = np.exp2(rng.uniform(8, 15.9, (rows, k))).astype(np.float16)
+    y = torch.empty((rows, k), dtype=torch.float16, device=gu.DEV)
+    gu.kernel("swiglu", I=k)(X=gu.dev(np.concatenate([gate, up], axis=1)), Y=y, rows=rows)
+    g = gate.astype(np.float64)
+    want = (g / (1.0 + np.exp(-g)) * up).astype(np.float16)
+    normal = np.abs(want) > 2.0**-14
+    share = ((gu.host(y) != want) & normal).sum() / normal.sum()
+    print("share of results rounded the other way:", share)
+    assert share < 1.0e-4
+
+
 def test_a8_masked_columns():
     rng = np.random.default_rng(orc.SEED)
     x = rng.normal(size=(9, 512)).astype(np.float16)
