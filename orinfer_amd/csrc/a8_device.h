@@ -51,7 +51,8 @@ __device__ __forceinline__ int8_t quantise(float value, float scale, float inver
 // Four codes packed into one word; one test (and, rarely, four exact quotients) for the four.
 // A product's distance from its rounded value is at most 0.5, so "within 2^-14 of a tie" is
 // "farther than 0.5 - 2^-14 from the rounded value".  The clamped integer plus 1.5 * 2^23 has the
-// integer in its low mantissa bits in two's complement: the low byte of that word is the int8 code.
+// integer in its low mantissa bits in two's complement: the low byte of that word is the int8 code.  The hint keeps
+// the quotients behind their branch: executed for every value they cost a one-piece form a fifth of its time.
 __device__ __forceinline__ uint32_t quantise4(const float (&value)[4], float scale, float inverse) {
     float r[4];
     float farthest = 0.f;
@@ -61,7 +62,7 @@ __device__ __forceinline__ uint32_t quantise4(const float (&value)[4], float sca
         r[j] = rintf(guess);
         farthest = fmaxf(farthest, fabsf(guess - r[j]));
     }
-    if (farthest > 0.49993896484375f) {
+    if (__builtin_expect(farthest > 0.49993896484375f, 0)) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) r[j] = rintf(__fdiv_rn(value[j], scale));
     }

@@ -26,16 +26,9 @@
 namespace orx {
 namespace {
 
-template <bool FUSED, bool MASKED>
-__device__ __forceinline__ float load_value(const __half* __restrict__ x, const uint8_t* __restrict__ mask,
-                                            int64_t row_base, int k, int col) {
-    float v;
-    if (FUSED)
-        v = swiglu_value(x[row_base + col], x[row_base + k + col]);
-    else
-        v = __half2float(x[row_base + col]);
-    if (MASKED && mask[col] != 0) v = 0.f;
-    return v;
+template <bool FUSED>
+__device__ __forceinline__ float load_value(const __half* __restrict__ x, int64_t row_base, int k, int col) {
+    return FUSED ? swiglu_value(x[row_base + col], x[row_base + k + col]) : __half2float(x[row_base + col]);
 }
 
 __device__ __forceinline__ float block_max(float v, float* scratch) {
@@ -47,43 +40,72 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
     return __uint_as_float(row_max_u32(__float_as_uint(scratch[min(lane & 15, waves - 1)])));
 }
 
-// Masked rows and groups longer than the held form takes: two passes over the group, grid (rows, groups).
-template <bool FUSED, bool MASKED>
-__global__ __launch_bounds__(256) void a8_kernel(const __half* __restrict__ x, const uint8_t* __restrict__ mask,
-                                                 int8_t* __restrict__ q, __half* __restrict__ s, int k, int group,
-                                                 int groups) {
+// Masked rows: two passes over the group, grid (rows, groups).
+template <bool FUSED>
+__global__ __launch_bounds__(256) void a8_masked_kernel(const __half* __restrict__ x, const uint8_t* __restrict__ mask,
+                                                        int8_t* __restrict__ q, __half* __restrict__ s, int k, int group,
+                                                        int groups) {
     __shared__ float scratch[4];
     const int row = blockIdx.x, g = blockIdx.y;
     const int first = g * group;
     const int width = min(group, k - first);
     const int64_t in_base = (int64_t)row * (FUSED ? 2 * k : k);
     const int64_t out_base = (int64_t)row * k;
+    auto value = [&](int col) { return mask[col] != 0 ? 0.f : load_value<FUSED>(x, in_base, k, col); };
     float amax = 0.f;
-    for (int i = threadIdx.x; i < width; i += 256)
-        amax = fmaxf(amax, fabsf(load_value<FUSED, MASKED>(x, mask, in_base, k, first + i)));
+    for (int i = threadIdx.x; i < width; i += 256) amax = fmaxf(amax, fabsf(value(first + i)));
     amax = block_max(amax, scratch);
     const __half stored = a8_scale(amax);
     if (threadIdx.x == 0) s[(int64_t)row * groups + g] = stored;
     const float scale = __half2float(stored);
     const float inverse = __frcp_rn(scale);
-    for (int i = threadIdx.x; i < width; i += 256)
-        q[out_base + first + i] = quantise(load_value<FUSED, MASKED>(x, mask, in_base, k, first + i), scale, inverse);
+    for (int i = threadIdx.x; i < width; i += 256) q[out_base + first + i] = quantise(value(first + i), scale, inverse);
+}
+
+typedef _Float16 half_pair __attribute__((ext_vector_type(2)));
+typedef uint32_t word4 __attribute__((ext_vector_type(4)));  // eight fp16 values
+
+// Eight values of a row as the quantiser sees them (FUSED: fp16(silu(gate) * up), eight of each) and their magnitudes, as two
+// fp16 lanes: comparing needs no conversion.
+template <bool FUSED>
+__device__ __forceinline__ void take_piece(word4& piece, word4 ups, half_pair& largest) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        if (FUSED) {
+            const __half2 gate = __builtin_bit_cast(__half2, (uint32_t)piece[j]), up = __builtin_bit_cast(__half2, (uint32_t)ups[j]);
+            const half_pair pair = {(_Float16)swiglu_value(__low2half(gate), __low2half(up)),
+                                    (_Float16)swiglu_value(__high2half(gate), __high2half(up))};
+            piece[j] = __builtin_bit_cast(uint32_t, pair);
+        }
+        largest = __builtin_elementwise_max(largest, __builtin_bit_cast(half_pair, (uint32_t)(piece[j] & 0x7FFF7FFFu)));
+    }
+}
+__device__ __forceinline__ uint2 quantise_piece(word4 piece, float scale, float inverse) {
+    float value[8];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const half_pair pair = __builtin_bit_cast(half_pair, (uint32_t)piece[j]);
+        value[2 * j] = (float)pair[0], value[2 * j + 1] = (float)pair[1];
+    }
+    const float low[4] = {value[0], value[1], value[2], value[3]}, high[4] = {value[4], value[5], value[6], value[7]};
+    return make_uint2(quantise4(low, scale, inverse), quantise4(high, scale, inverse));
 }
 
 // One pass: WAVES waves hold a (row, group) in registers as 16-byte pieces of eight fp16 values, PIECES to a lane,
 // between the maximum and the codes; FUSED values are fp16(silu(gate) * up), computed once.  All loads of a wave leave
 // together.  One wave needs no barrier (four groups to a workgroup then); more waves meet once, for the maximum.
+// LONG: what lies beyond the held pieces is read for the maximum and again for the codes, four pieces of a lane at a time
+// (us, against two passes with 16-byte loads, FUSED in brackets: 1 x 40960 12.7 -> 5.0 (81 -> 10.8), 2048 x 40960 77.5 -> 53.7
+// (263 -> 103), 512 x 131072 86 -> 49.5 (562 -> 115); four pieces held instead of eight: 5.9 (16.0), 59.5 (130), 52 (114)).
 // What bounds it: memory with many rows (8192 x 4096: 28.1 -> 20.7 us, 4.9 TB/s; the two-pass kernel read every row twice),
-// the vector ALU beside it in the FUSED form (8192 x 17408: 416 -> 148 us; the two-pass kernel also computed every value
-// twice), the latency of one row's loads and reductions with few (FUSED, one row of 17408: 43 -> 6.3 us).
-template <bool FUSED, int WAVES, int PIECES>
+// the vector ALU beside it in the FUSED form (8192 x 17408: 416 -> 146 us; the two-pass kernel also computed every value
+// twice), the latency of one row's loads and reductions with few (FUSED, one row of 17408: 43 -> 5.9 us).
+template <bool FUSED, int WAVES, int PIECES, bool LONG>
 __global__ __launch_bounds__(WAVES == 1 ? 256 : 64 * WAVES) void a8_held_kernel(const __half* __restrict__ x,
                                                                                 int8_t* __restrict__ q,
                                                                                 __half* __restrict__ s, int k, int group,
                                                                                 int groups, int rows) {
-    constexpr int kLanes = 64 * WAVES;
-    typedef _Float16 half_pair __attribute__((ext_vector_type(2)));
-    typedef uint32_t word4 __attribute__((ext_vector_type(4)));
+    constexpr int kLanes = 64 * WAVES, kTail = 4;
     __shared__ float scratch[WAVES];
     const int lane = WAVES == 1 ? threadIdx.x & 63 : threadIdx.x;
     const int unit = WAVES == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;  // wave-uniform
@@ -95,39 +117,40 @@ __global__ __launch_bounds__(WAVES == 1 ? 256 : 64 * WAVES) void a8_held_kernel(
     const int64_t out_base = (int64_t)row * k;
     const bool vector = (k % 8 == 0) && (group % 8 == 0) && ((reinterpret_cast<uintptr_t>(x) & 15) == 0) &&
                         ((reinterpret_cast<uintptr_t>(q) & 7) == 0);
+    const word4* src = reinterpret_cast<const word4*>(x + in_base + first);
+    const word4* src_up = reinterpret_cast<const word4*>(x + in_base + k + first);
     word4 held[PIECES];
     const int pieces = width / 8;
     float amax = 0.f;
     if (vector) {
-        const word4* src = reinterpret_cast<const word4*>(x + in_base + first);
-        word4 up[FUSED ? PIECES : 1];
+        word4 up[FUSED ? PIECES : 1] = {};
 #pragma unroll
         for (int p = 0; p < PIECES; ++p) {  // clamped, so unconditional
             const int i = min(lane + p * kLanes, pieces - 1);
             held[p] = src[i];
-            if (FUSED) up[p] = *reinterpret_cast<const word4*>(x + in_base + k + first + 8 * i);
+            if (FUSED) up[p] = src_up[i];
         }
-        half_pair largest = {(_Float16)0.f, (_Float16)0.f};  // magnitudes as two fp16 lanes: comparing needs no conversion
+        half_pair largest = {(_Float16)0.f, (_Float16)0.f};
 #pragma unroll
         for (int p = 0; p < PIECES; ++p) {
-            if (lane + p * kLanes < pieces) {
+            if (lane + p * kLanes < pieces) take_piece<FUSED>(held[p], up[FUSED ? p : 0], largest);
+        }
+        if (LONG) {
+            for (int base = lane + PIECES * kLanes; base < pieces; base += kTail * kLanes) {
+                word4 more[kTail], more_up[FUSED ? kTail : 1] = {};
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    if (FUSED) {
-                        const __half2 gate = __builtin_bit_cast(__half2, (uint32_t)held[p][j]);
-                        const __half2 value = __builtin_bit_cast(__half2, (uint32_t)up[p][j]);
-                        const half_pair pair = {(_Float16)swiglu_value(__low2half(gate), __low2half(value)),
-                                                (_Float16)swiglu_value(__high2half(gate), __high2half(value))};
-                        held[p][j] = __builtin_bit_cast(uint32_t, pair);
-                    }
-                    largest = __builtin_elementwise_max(largest, __builtin_bit_cast(half_pair, held[p][j] & 0x7FFF7FFFu));
+                for (int u = 0; u < kTail; ++u) {  // clamped: a repeated last piece does not change the maximum
+                    const int i = min(base + u * kLanes, pieces - 1);
+                    more[u] = src[i];
+                    if (FUSED) more_up[u] = src_up[i];
                 }
+#pragma unroll
+                for (int u = 0; u < kTail; ++u) take_piece<FUSED>(more[u], more_up[FUSED ? u : 0], largest);
             }
         }
         amax = fmaxf((float)largest[0], (float)largest[1]);
     } else {
-        for (int i = lane; i < width; i += kLanes)
-            amax = fmaxf(amax, fabsf(load_value<FUSED, false>(x, nullptr, in_base, k, first + i)));
+        for (int i = lane; i < width; i += kLanes) amax = fmaxf(amax, fabsf(load_value<FUSED>(x, in_base, k, first + i)));
     }
     if (WAVES == 1) {
         amax = wave_max_magnitude(amax);
@@ -141,21 +164,30 @@ __global__ __launch_bounds__(WAVES == 1 ? 256 : 64 * WAVES) void a8_held_kernel(
     if (vector) {
         uint2* dst = reinterpret_cast<uint2*>(q + out_base + first);
 #pragma unroll
-        for (int p = 0; p < PIECES; ++p) {
-            if (lane + p * kLanes < pieces) {
-                float value[8];
+        for (int p = 0; p < PIECES; ++p)
+            if (lane + p * kLanes < pieces) dst[lane + p * kLanes] = quantise_piece(held[p], scale, inverse);
+        if (LONG) {
+            for (int base = lane + PIECES * kLanes; base < pieces; base += kTail * kLanes) {
+                word4 more[kTail], more_up[FUSED ? kTail : 1] = {};
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const half_pair pair = __builtin_bit_cast(half_pair, (uint32_t)held[p][j]);
-                    value[2 * j] = (float)pair[0], value[2 * j + 1] = (float)pair[1];
+                for (int u = 0; u < kTail; ++u) {
+                    const int i = min(base + u * kLanes, pieces - 1);
+                    more[u] = src[i];
+                    if (FUSED) more_up[u] = src_up[i];
                 }
-                const float low[4] = {value[0], value[1], value[2], value[3]}, high[4] = {value[4], value[5], value[6], value[7]};
-                dst[lane + p * kLanes] = make_uint2(quantise4(low, scale, inverse), quantise4(high, scale, inverse));
+#pragma unroll
+                for (int u = 0; u < kTail; ++u) {
+                    if (base + u * kLanes < pieces) {
+                        half_pair unused = {(_Float16)0.f, (_Float16)0.f};
+                        take_piece<FUSED>(more[u], more_up[FUSED ? u : 0], unused);
+                        dst[base + u * kLanes] = quantise_piece(more[u], scale, inverse);
+                    }
+                }
             }
         }
     } else {
         for (int i = lane; i < width; i += kLanes)
-            q[out_base + first + i] = quantise(load_value<FUSED, false>(x, nullptr, in_base, k, first + i), scale, inverse);
+            q[out_base + first + i] = quantise(load_value<FUSED>(x, in_base, k, first + i), scale, inverse);
     }
 }
 
@@ -659,20 +691,22 @@ struct HeldForm {
 };
 const HeldForm* held_forms(int* count) {
 #define ORX_HELD(W, P)                                                                                             \
-    {W, P, reinterpret_cast<const void*>(&a8_held_kernel<false, W, P>), reinterpret_cast<const void*>(&a8_held_kernel<true, W, P>)}
+    {W, P, reinterpret_cast<const void*>(&a8_held_kernel<false, W, P, (W > 8)>),                                   \
+     reinterpret_cast<const void*>(&a8_held_kernel<true, W, P, (W > 8)>)}
     static const HeldForm forms[] = {ORX_HELD(1, 1), ORX_HELD(1, 2), ORX_HELD(1, 4), ORX_HELD(4, 1), ORX_HELD(4, 2),
                                      ORX_HELD(4, 3), ORX_HELD(4, 4), ORX_HELD(4, 6), ORX_HELD(8, 1), ORX_HELD(8, 2),
-                                     ORX_HELD(8, 3), ORX_HELD(8, 5), ORX_HELD(8, 8)};
+                                     ORX_HELD(8, 3), ORX_HELD(8, 5), ORX_HELD(8, 8), ORX_HELD(16, 8)};
 #undef ORX_HELD
     *count = (int)(sizeof forms / sizeof forms[0]);
     return forms;
 }
 
-// The form a launch takes, or null for the general kernel (a mask, groups beyond 32768 values).  Measured (us, FUSED in
+// The form a launch takes, or null for the two-pass kernel (a mask).  Measured (us, FUSED in
 // brackets), 1 / 4 / 8 waves to a row: 8192 rows of 1024 7.3 / 10.9 / 19.7, of 2048 11.7 / 13.4 / 21.6 (with so many
 // rows the rate at which workgroups start is the limit, so a wave takes a whole row as long as four pieces to a
 // lane hold it), of 5120 - / 23 / 30 (- / 45 / 51); 4096 rows of 17408 - / 37 / 37 (- / 80 / 75); one row of 17408 - / 4.6 / 3.8
-// (- / 7.4 / 6.3); 200 rows of 5120 - / 3.8 / 3.6.  Sixteen waves were nowhere more than 0.1 us better.
+// (- / 7.4 / 6.3); 200 rows of 5120 - / 3.8 / 3.6.  Sixteen waves were nowhere more than 0.1 us better up to 32768 values, the
+// most that eight hold; they take every longer group.
 const HeldForm* held_form(const orx_function& f, int rows) {
     if (f.flags & 1) return nullptr;
     const int pieces = (f.group + 7) / 8;
@@ -683,7 +717,7 @@ const HeldForm* held_form(const orx_function& f, int rows) {
     const HeldForm* forms = held_forms(&count);
     for (int i = 0; i < count; ++i)
         if (forms[i].waves == waves && forms[i].pieces * 64 * waves >= pieces) return &forms[i];
-    return nullptr;
+    return &forms[count - 1];
 }
 
 int a8_geometry(const orx_function& f, int rows, Geometry* g) {
@@ -707,19 +741,15 @@ int a8_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t st
     const __half* x = pointer_arg<const __half>(args, 3);
     const dim3 grid(g.grid[0], g.grid[1]), block(g.block[0]);
     const int groups = (int)ceil_div((uint32_t)f.K, (uint32_t)f.group);
-    const bool masked = f.flags & 1, fused = f.flags & 2;
+    const bool fused = f.flags & 2;
     if (const HeldForm* form = held_form(f, rows)) {
         typedef void (*Held)(const __half*, int8_t*, __half*, int, int, int, int);
         const Held kernel = reinterpret_cast<Held>(const_cast<void*>(fused ? form->fused : form->plain));
         ORX_LAUNCH(kernel, grid, block, 0, stream, x, q, s, f.K, f.group, groups, rows);
-    } else if (fused && masked)
-        ORX_LAUNCH((a8_kernel<true, true>), grid, block, 0, stream, x, mask, q, s, f.K, f.group, groups);
-    else if (fused)
-        ORX_LAUNCH((a8_kernel<true, false>), grid, block, 0, stream, x, mask, q, s, f.K, f.group, groups);
-    else if (masked)
-        ORX_LAUNCH((a8_kernel<false, true>), grid, block, 0, stream, x, mask, q, s, f.K, f.group, groups);
+    } else if (fused)
+        ORX_LAUNCH((a8_masked_kernel<true>), grid, block, 0, stream, x, mask, q, s, f.K, f.group, groups);
     else
-        ORX_LAUNCH((a8_kernel<false, false>), grid, block, 0, stream, x, mask, q, s, f.K, f.group, groups);
+        ORX_LAUNCH((a8_masked_kernel<false>), grid, block, 0, stream, x, mask, q, s, f.K, f.group, groups);
     return hip_check(hipGetLastError(), "launch activation_quantization");
 }
 

@@ -224,6 +224,16 @@ def test_a_named_launch_is_checked_before_anything_is_enqueued(values, code):
     assert lib.library().orx_enqueue(None, None, None) == lib.ORX_ERR_BAD_ARGUMENT
 
 
+@pytest.mark.parametrize("fused", [False, True])
+def test_groups_too_long_for_eight_waves_take_sixteen(fused):
+    """Unmasked groups beyond 32768 values keep the wide loads: sixteen waves to a group, one workgroup to a (row, group)."""
+    for k, group, rows in ((32776, 32776, 1), (40960, 40960, 300), (1 << 20, 65536, 3)):
+        kernel = lib.Kernel("activation_quantization", K=k, group_size=group, fused=fused)
+        assert kernel.geometry(rows) == ((rows * (k // group), 1, 1), (1024, 1, 1), 0)
+    held = lib.Kernel("activation_quantization", K=32768, fused=fused)
+    assert held.geometry(1) == ((1, 1, 1), (512, 1, 1), 0)
+
+
 def test_handles_own_no_device_memory_and_say_what_workspace_they_need():
     """orx_resolve allocates nothing: scratch is a `Workspace` buffer the engine sizes from
     orx_workspace_bytes (AGENTS.md:41: the engine owns every buffer).  A thousand handles resolve in

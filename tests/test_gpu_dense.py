@@ -112,7 +112,8 @@ def test_a8_many_rows_of_long_groups(rows, k, group):
     (2049, 1016, 1016), (2048, 2048, 2048), (1023, 1536, 768),          # one wave to a group, units that do not divide by four
     (3, 520, 520), (5, 2048, 2048), (600, 2056, 2056), (514, 12288, 12288),   # four waves, at both ends of their pieces
     (2, 2056, 2056), (513, 12296, 12296), (1, 32768, 32768),            # eight waves
-    (1, 32776, 32776), (2, 2060, 2060), (2049, 1020, 1020),             # too long to hold; rows that are not 16-byte aligned
+    (1, 32776, 32776), (3, 65536 + 4096, 65536 + 4096), (2, 90000, 45000),    # sixteen waves, longer than they hold
+    (2, 2060, 2060), (2049, 1020, 1020), (2, 40004, 40004),             # rows that are not 16-byte aligned
 ])
 def test_a8_held_forms(rows, k, group, fused):
     """The waves and pieces that hold a row follow its length and the row count; codes and scales do not."""
@@ -155,7 +156,7 @@ def test_swiglu_gates_without_a_finite_sigmoid_product():
     (2048, 512), (4, 512),     # one wave to a row
     (4, 2048), (513, 12288),   # four waves
     (4, 12296),                # eight waves
-    (4, 32776), (4, 2060),     # too long to hold; rows that are not 16-byte aligned
+    (4, 32776), (4, 2060),     # sixteen waves; rows that are not 16-byte aligned
 ])
 def test_a8_of_gates_without_a_value(rows, k):
     """A gate that gives no number (minus infinity, NaN) leaves the row's scale and its other codes alone; an infinite value
