@@ -709,12 +709,18 @@ const HeldForm* held_forms(int* count) {
 // most that eight hold; they take every longer group.
 const HeldForm* held_form(const orx_function& f, int rows) {
     if (f.flags & 1) return nullptr;
-    const int pieces = (f.group + 7) / 8;
-    const int64_t units = (int64_t)rows * ((f.K + f.group - 1) / f.group);
-    const int waves = pieces <= 64 || (pieces <= 256 && units >= 2048) ? 1
-                      : pieces > 1536 || (pieces > 256 && units <= 512) ? 8 : 4;
     int count = 0;
     const HeldForm* forms = held_forms(&count);
+    const int pieces = (f.group + 7) / 8;
+    const int64_t units = (int64_t)rows * ((f.K + f.group - 1) / f.group);
+    // Rows that are never 16-byte aligned go value by value, a value to a lane and step: more lanes to a row shorten the chain of
+    // its loads while rows are few or one wave would take more than 1024 values (one wave against four: 4096 x 2044 19.6 -> 15.3,
+    // fused 29.0 -> 19.7, but 8192 x 1020 15.8 / 17.3; eight against sixteen: 8 x 9004 6.1 -> 5.1, fused 9.4 -> 6.7, 1 x 4100 3.5 / 3.5,
+    // but fused 600 x 17404 32.4 / 36.3)
+    const bool values = f.K % 8 != 0 || f.group % 8 != 0;
+    if (values && pieces > 1024 && units <= 256) return &forms[count - 1];
+    const int waves = pieces <= 64 || (pieces <= (values ? 128 : 256) && units >= 2048) ? 1
+                      : pieces > 1536 || (pieces > 256 && units <= 512) ? 8 : 4;
     for (int i = 0; i < count; ++i)
         if (forms[i].waves == waves && forms[i].pieces * 64 * waves >= pieces) return &forms[i];
     return &forms[count - 1];

@@ -234,6 +234,15 @@ def test_groups_too_long_for_eight_waves_take_sixteen(fused):
     assert held.geometry(1) == ((1, 1, 1), (512, 1, 1), 0)
 
 
+def test_rows_that_go_value_by_value_take_more_waves():
+    """K or group not a multiple of 8: the quantiser reads single values, so one wave takes 1024 of them at most and few long
+    groups take sixteen."""
+    for k, group, rows, want in ((2044, 2044, 4096, ((4096, 1, 1), 256)), (1020, 1020, 8192, ((2048, 1, 1), 256)), (9004, 9004, 8, ((8, 1, 1), 1024)),
+                                 (9004, 9004, 8192, ((8192, 1, 1), 256)), (8400, 8397, 8, ((16, 1, 1), 1024)), (2048, 2048, 4096, ((1024, 1, 1), 256))):
+        grid, block, _ = lib.Kernel("activation_quantization", K=k, group_size=group).geometry(rows)
+        assert (grid, block[0]) == want, (k, group, rows)
+
+
 def test_handles_own_no_device_memory_and_say_what_workspace_they_need():
     """orx_resolve allocates nothing: scratch is a `Workspace` buffer the engine sizes from
     orx_workspace_bytes (AGENTS.md:41: the engine owns every buffer).  A thousand handles resolve in
