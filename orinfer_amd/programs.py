@@ -146,6 +146,7 @@ class MoeLayer:
         common = dict(M=tokens, E=experts, top_k=top_k)
         # one launch for all routing metadata where the fused kernel applies (kernels/cuda/model/moe.py:713-764),
         # the three-kernel form otherwise
+        one_launch_refused = fused_metadata is False
         if fused_metadata is None:
             fused_metadata = experts <= 1024 and (16 * experts + 32 + 2 * tokens * top_k) * 4 <= 160 * 1024
         self.k_metadata = Kernel("route_metadata", block_m=block_m, **common) if fused_metadata else None
@@ -199,9 +200,10 @@ class MoeLayer:
         # Long prompts: six launches over tiles of 128 rows (`block_m` is the tile height of the orders above).
         #   router top-k + A8 of every token's row, metadata in segments (two launches),
         #   gate_up that gathers the token rows and writes fp16(silu(gate) * up), A8, down, combine.
+        # A caller who asked for the quantiser and the dispatch, or the metadata, as launches of their own gets them.
         self.bulk = False
-        if (not self.fused_stages and fused_stages is None and not keep_intermediates and signs is None and hidden % 8 == 0
-                and packed_k == 128 and experts <= 1024 and grouped_algorithm == "auto" and assignments >= BULK_ROWS_PER_EXPERT * experts):
+        if (not self.fused_stages and fused_stages is None and not keep_intermediates and signs is None and self.fused_dispatch
+                and not one_launch_refused and packed_k == 128 and experts <= 1024 and grouped_algorithm == "auto" and assignments >= BULK_ROWS_PER_EXPERT * experts):
             try:
                 tiles = (assignments + BULK_ROWS - 1) // BULK_ROWS + min(experts, assignments)
                 bulk = dict(rows=assignments, E=experts, tiles=tiles, block_m=BULK_ROWS)

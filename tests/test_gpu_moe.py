@@ -1133,6 +1133,32 @@ def test_long_prompt_program_gives_the_bits_of_seven_launches():
         assert torch.equal(six.out, want)
 
 
+def test_long_prompts_keep_the_launches_a_caller_asked_for():
+    """fused_dispatch=False and fused_metadata=False hold whatever the row count is, and with the quantiser as a launch of its
+    own the hidden rows may start at any fp16 address."""
+    rng = np.random.default_rng(orc.SEED + 9)
+    tokens, experts, top_k, hidden, inter = 4100, 4, 2, 256, 128  # more slots than the five-launch order takes
+    bank = (rng.integers(0, 65536, (experts, 2 * inter, hidden // 8), dtype=np.uint16),
+            rng.uniform(0.0005, 0.002, (experts, 2 * inter)).astype(np.float16),
+            rng.integers(0, 65536, (experts, hidden, inter // 8), dtype=np.uint16),
+            rng.uniform(0.0005, 0.002, (experts, hidden)).astype(np.float16))
+    x = gu.dev(rng.normal(size=(tokens, hidden)).astype(np.float16))
+    logits = gu.dev(rng.normal(size=(tokens, experts)).astype(np.float32))
+    shape = (tokens, experts, top_k, hidden, inter) + bank
+    plain = programs.MoeLayer(*shape)
+    assert plain.bulk
+    want = plain.run(x, logits).clone()
+    shifted = torch.empty(tokens * hidden + 1, dtype=torch.float16, device=gu.DEV)[1:].view(tokens, hidden)
+    shifted.copy_(x)
+    assert shifted.data_ptr() % 16 != 0
+    split = programs.MoeLayer(*shape, fused_metadata=False)
+    assert not split.bulk and split.k_metadata is None
+    assert torch.equal(split.run(x, logits), want)
+    apart = programs.MoeLayer(*shape, fused_dispatch=False)
+    assert not apart.bulk and not apart.fused_dispatch
+    assert torch.equal(apart.run(shifted, logits), want)
+
+
 # The selector decoder's whole domain, after tests/cuda/operators/e8p_selector.py:23-94: tables drawn from
 # {0, +-2, +-6, +-10} (zero coordinates included), one table per expert or one for all, patch words on or
 # off (with the word that test plants: valid, value -128, last position), tile lists of 8 to 64 rows with
