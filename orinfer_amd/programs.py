@@ -136,9 +136,6 @@ class MoeLayer:
         self.slot_map = torch.empty((tokens, top_k), **i32)
         self.a_q = torch.empty((tokens, hidden), **i8)
         self.a_s = torch.empty((tokens, 1), **f16)
-        self.d = torch.empty((assignments, hidden), **i8)
-        self.ds = torch.empty((assignments, 1), **f16)
-        self.gate_up_out = torch.empty((assignments, 2 * intermediate), **f16)
         self.h_q = torch.empty((assignments, intermediate), **i8)
         self.h_s = torch.empty((assignments, 1), **f16)
         self.down_out = torch.empty((assignments, hidden), **f16)
@@ -222,6 +219,12 @@ class MoeLayer:
             except OrxError as error:
                 if error.code != ORX_ERR_BAD_VARIANT:
                     raise
+        # the dispatched rows and the gate | up outputs, which the order for long prompts does without
+        self.d = self.ds = self.gate_up_out = None
+        if not self.bulk:
+            self.d = torch.empty((assignments, hidden), **i8)
+            self.ds = torch.empty((assignments, 1), **f16)
+            self.gate_up_out = torch.empty((assignments, 2 * intermediate), **f16)
         self.k_combine = Kernel("moe_combine", H=hidden, slots=assignments, **common)
 
     def run(self, x16, logits, stream=None):

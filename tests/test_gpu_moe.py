@@ -1119,6 +1119,7 @@ def test_long_prompt_program_gives_the_bits_of_seven_launches():
     args = (1025, c["experts"], c["top_k"], c["hidden"], c["intermediate"], c["gate_up"], c["gate_up_scales"], c["down"], c["down_scales"])
     seven, six = programs.MoeLayer(*args, fused_stages=False), programs.MoeLayer(*args)
     assert six.bulk and not seven.bulk
+    assert six.d is None and six.ds is None and six.gate_up_out is None  # (tokens * top_k) rows of H and 2 I values it never writes
     want = seven.run(x, logits).clone()
     assert torch.equal(six.run(x, logits), want)
     stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
