@@ -498,6 +498,24 @@ def test_one_row_program_gives_the_bits_of_two_launches(n, k, packed_k, single):
         np.testing.assert_array_equal(out, orc.project(a_q, a_s, weights, scales))
 
 
+@pytest.mark.parametrize("codec", ["q4", "w8"])
+def test_a_result_of_a_linear_is_the_callers_own_tensor(codec):
+    """What a caller does to the shape of one result leaves the next one, and `out`, as they are."""
+    rng = np.random.default_rng(orc.SEED + 5)
+    weight = rng.integers(0, 2**32, (256, 64), dtype=np.uint32) if codec == "q4" else rng.integers(-127, 128, (256, 512), dtype=np.int8)
+    linear = programs.QuantizedLinear(codec, weight, rng.uniform(0.005, 0.02, 256).astype(np.float16), 4)
+    for rows in (1, 3, 4):
+        x = gu.dev(rng.normal(size=(rows, 512)).astype(np.float16))
+        first = linear.run(x)
+        want = first.clone()
+        first.t_()
+        second = linear.run(x)
+        assert second.shape == (rows, 256) and torch.equal(second, want) and second.data_ptr() == linear.out.data_ptr()
+        second.resize_((1, 2))
+        third = linear.project(rows)
+        assert third.shape == (rows, 256) and torch.equal(third, want) and linear.out.shape == (4, 256)
+
+
 def test_q4_fp16_input_is_refused_where_no_kernel_serves_it():
     for variant in (dict(M=2, N=256, K=1024), dict(M=1, N=256, K=1024, algorithm="mfma"), dict(M=1, N=256, K=16384),
                     dict(M=1, N=256, K=1024, input_dtype="bfloat16")):
