@@ -480,6 +480,9 @@ bool dense_resident_eligible(int n, int k, int packed_k) {
     return packed_k == 0 && k % 1024 == 0 && k / 1024 <= 8 && lds_bytes(n, device_compute_units()) <= kLdsLimit;
 }
 
+// the loader-wave kernel among them
+bool dense_loader_eligible(int n, int k, int packed_k) { return specialized_fits(n, k, packed_k); }
+
 void dense_resident_geometry(int rows, int n, int k, int packed_k, Geometry* g) {
     const int chunk = rows < 32 ? rows : 32;  // rows per launch
     g->grid[1] = g->grid[2] = 1;

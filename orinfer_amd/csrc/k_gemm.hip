@@ -44,6 +44,7 @@ int row_q4_gemv_launch(const int8_t* a, const void* w, uint32_t low, uint32_t hi
                        int rows, int n, int k, int stride, bool out_f32, const Geometry& g, hipStream_t stream);
 void stream_grouped_geometry(int n, int tiles, Geometry* g);
 bool dense_resident_eligible(int n, int k, int packed_k);
+bool dense_loader_eligible(int n, int k, int packed_k);
 void dense_resident_geometry(int rows, int n, int k, int packed_k, Geometry* g);
 int dense_resident_launch(const int8_t* a, const void* w, const uint32_t* book, const __half* ws, const __half* as,
                           void* out, int rows, int n, int k, int stride, int packed_k, bool out_f32, hipStream_t stream);
@@ -697,6 +698,38 @@ int tile_for(const orx_function& f, int rows) {
     return f.tile_hint && rows <= f.tile_hint ? f.tile_hint : 0;
 }
 
+// Two-stage codes of 2 to 32 rows: batched-decode kernels, channel runs or the streaming kernel.  All of them give a CU whole
+// pieces of the channels, so what counts is how many blocks of 16 a CU gets: the runs take one, two or three, a workgroup of the
+// streaming kernel always 32 channels.  With an odd count the streaming kernel leaves half of the CUs idle in a round; with two
+// it has the chip full and reads a token row once for 32 channels.  Measured over matrices that together do not stay in
+// cache (us; N x K, K-major / row-major codes); in cache the relations are the same unless a number says otherwise:
+//   one block, runs against the streaming kernel: 2048 x 4224 at 2 rows 6.8 to 7.0 / 7.0 to 7.2, 16 rows 7.0 to 7.2 / 7.3 to 8.3, 32 rows 7.5 to 8.7 / 7.8 to 10.2;
+//     K = 17408 at 16 rows 0.72 / 0.57 of its time; up to 16 rows level or slower below K = 4096 (2048 x 2560 5.4 to 5.0 / 5.5 to 5.1), above 16 rows
+//     faster from K = 3072 on (2048 x 3584 at 32 rows 6.9 to 7.5);
+//   two blocks: 7168 x 5376 at 2 rows 9.8 to 8.3 / 10.3 to 8.7, 24 rows 10.8 to 9.2 / 12.2 to 10.9; the runs get there with rows times K: 7168 x 17408 at 16 rows
+//     1.06 / 0.97 of its time, 32 rows 0.93 / 0.84; 7168 x 5120 row-major at 24 / 32 rows 1.06 / 0.98;
+//   three blocks: 9728 x 6144 at 8 rows 0.94 / 0.89 of its time, 24 rows 0.81 / 0.78; K = 4224 at 2 rows 1.06 / 1.02, 24 rows of K = 3200 1.04; two rows stay with
+//     the GEMV (9728 x 9728 18.7 to 17.0 / row-major).
+// The batched-decode kernels where they take the shape: the one with loader waves (K up to 5120) is the fastest up to 16
+// rows in one and three blocks (K = 5120, 16 rows: 0.85-0.97 of the runs, 0.72-0.9 of the streaming kernel); with one block and
+// more rows the runs pass it at 20 K-major and 24 row-major rows of K = 5120 (2048 x 5120 at 32 rows 7.9 to 8.8 / 8.3 to 8.8, 1024 x 4096 6.5 to 7.2);
+// with two blocks the streaming kernel does (use_resident).  The other one (row-major, K to 8192) is slower than the runs with one
+// block (4096 x 8192 at 8 / 24 rows: the runs 0.81 / 0.74 of it), and with three from rows times K = 160 K on (9728 x 8192 at 8 / 24 rows 1.05 /
+// 0.86, 12288 x 6144 at 17 / 32 rows 1.09 / 0.99).
+int channel_blocks_per_cu(int n) { return (int)ceil_div(ceil_div((uint32_t)n, 16u), (uint32_t)device_compute_units()); }
+bool runs_for_few_rows(const orx_function& f, int rows) {
+    const int blocks = channel_blocks_per_cu(f.N);
+    const int64_t work = (int64_t)rows * f.K;
+    if (blocks > 3) return false;
+    const bool loader = dense_loader_eligible(f.N, f.K, f.packed_k);
+    if (blocks == 1 && loader) return rows > 16 && work >= (f.packed_k != 0 ? 20 : 24) * 5120;
+    if (blocks == 1) return f.K >= (rows > 16 ? 3072 : 4096);
+    if (blocks == 2) return work >= (f.packed_k != 0 ? 32 * 12288 : 20 * 8192);
+    if (loader || rows <= 2) return false;
+    if (dense_resident_eligible(f.N, f.K, f.packed_k)) return work >= 20 * 8192;
+    return f.K >= (rows > 16 ? 4096 : 6144);
+}
+
 // Channel runs with K split over the waves (k_runs.hip), `algorithm=runs` by name, and by `auto` (int8 from one row on, codes from two) while the
 // workgroups fit one round of the CUs (up to 64 rows: any number, the tiles are low).  Measured against what `auto` launched
 // before (us, N x K, 256 CUs):
@@ -709,11 +742,8 @@ int tile_for(const orx_function& f, int rows) {
 //     two rounds (34816 x 5120: 33.0 against 33.8) or below 4 M weights (1024 x 2048: 3.5 against 3.9) it stays.
 //   two-stage codes: 48 / 64 rows 17408 x 5120 31 -> 21, 31 -> 23, 7168 x 5120 12.7 -> 11.1, 14.8 -> 12.3; 96 / 128 / 200 / 256
 //     rows 7168 x 5120 22 -> 17, 25 -> 21, 36 -> 28, 36 -> 31; 4096 x 8192 200 rows 1.4, 1024 x 1024 200 rows 2.9 times faster; wider
-//     matrices go to the channel runs over all rows (11008 x 4096 at 128 / 256 rows 0.96 / 0.87).  Up to 32 rows the
-//     batched-decode kernels are faster where they take K (17408 x 5120: 0.8-0.9), and slower where the
-//     streaming kernel stands in for them (2560 x 9728 and 2048 x 16384: 1.1-2.4).
-//     Rows of K = 5120 from 17 on: 20 / 32 rows 7168 x 5120 10.6 -> 9.8, 11.9 -> 10.8, 2048 x 5120 7.6 -> 6.8 at 24; level or slower at
-//     K <= 4096 (4096 x 4096 7.0 / 7.1 at 20 rows).  66 / 80 rows of up to 48 channels to a CU, against one pass over all rows:
+//     matrices go to the channel runs over all rows (11008 x 4096 at 128 / 256 rows 0.96 / 0.87).  Up to 32 rows: runs_for_few_rows.
+//     66 / 80 rows of up to 48 channels to a CU, against one pass over all rows:
 //     11008 x 4096 20.5 -> 17.9, 20.2 -> 18.0, 12288 x 3072 17.0 -> 15.7, 17.1 -> 15.9; slower at 68 channels (17408 x 5120 30.8 / 38.5).
 //   129 to 512 rows, against split tiles and decode-once with their scratch: codes 256 rows 4096 x 4096 27.4 -> 17.4, 2560 x 9728 33.6 ->
 //     28.6, 512 rows 4096 x 4096 32 -> 26, 2048 x 1024 24 -> 9, 136 / 200 rows 11008 x 4096 40.9 -> 32.4, 41.4 -> 38.1 in two rounds;
@@ -738,7 +768,7 @@ bool use_runs(const orx_function& f, int rows) {
     if (f.flags == kW8 && rows == 1) return weights >= (1 << 22) && f.N <= 80 * device_compute_units();
     if (f.flags == kW8) return rows > 32 || (weights >= (1 << 22) && (rows > 16 || f.N % (32 * device_compute_units()) != 0));
     if (rows > 32) return weights >= (1 << 22);
-    return (f.K > 5120 || (f.K == 5120 && rows > 16)) && f.N <= 32 * device_compute_units();
+    return runs_for_few_rows(f, rows);
 }
 
 // Channel runs per CU over the whole K (k_wide.hip): two-stage codes, `algorithm=wide` by name, and by
@@ -794,6 +824,14 @@ bool use_gemv(const orx_function& f, int rows) {
     if (f.flags2 & kNoGemv) return false;  // the matrix-unit kernels were asked for: streaming / batched-decode from row 1
     if ((f.flags2 & kPreferGemv) && f.block_m > 0 && f.tiles == 0)  // the dot-product family wherever it serves the rows
         return rows <= (f.flags == kW8 ? 2 : 4) && (f.packed_k == 0 || (rows <= 2 && gemv_serves_k_major(f, rows)));
+    // Two to four rows of codes: the GEMV's dot products grow with the rows and its workgroups with N, so the streaming kernel takes
+    // them (us, GEMV / streaming kernel): row-major up to three blocks of 16 channels to a CU, 2 / 4 rows of 2048 x 1280 5.2 / 4.2 and 7.1 / 4.3,
+    // 7168 x 5376 10.5 / 8.7 and 14.3 / 8.8, 9728 x 4224 1.2 times at 2 rows; K-major (2 rows) up to two, 7168 x 2560 6.8 / 5.5, 4096 x 4352 10.5 / 7.0,
+    // but 11008 x 4608 10.4 / 10.9, 17408 x 3584 11.8 / 13.4
+    if (f.flags == kQ4 && rows > 1) {
+        const int blocks = channel_blocks_per_cu(f.N);
+        if (blocks <= 2 || (blocks == 3 && f.packed_k == 0 && (rows > 2 || f.K < 6144))) return false;
+    }
     // K-major codes: 1 row (13.4 us at N=17408, K=5120; the streaming kernel takes 17.2), and 2 rows
     // (16.4 us) where the batched-decode kernel (15.4 us) does not take the shape
     if (f.packed_k != 0) return rows <= 2 && gemv_serves_k_major(f, rows) && !use_resident(f, rows);
@@ -827,6 +865,15 @@ bool use_resident(const orx_function& f, int rows) {
     // (the second launch pays for itself only on large matrices: N = 17408, K = 5120 at 48 rows 33 us
     // against 39 us for the streaming kernel, but N = K = 5120 20 against 14.5 us)
     const int limit = (int64_t)f.N * f.K >= ((int64_t)1 << 26) ? 64 : 32;
+    // Two blocks of 16 channels to a CU fill the streaming kernel's workgroups of 32 channels.  Against the loader-wave
+    // kernel (us, N = 7168): K-major codes 16 rows of K = 3072 / 4096 / 5120 6.4 / 7.6 / 9.0 -> 6.0 / 6.8 / 7.9, 24 rows 7.5 / 8.7 / 10.7 ->
+    // 6.6 / 7.5 / 8.9, 2 / 8 rows of K = 5120 7.9 / 8.4 -> 7.5 / 7.8 (weights in cache: 0.96 / 0.99 of its speed), of K = 4096 6.8 / 7.1 -> 6.6 / 6.7 (0.95 / 1.0), K = 2048
+    // 5.7 -> 5.5; row-major codes the loader-wave kernel is level (24 rows of K = 4096 / 5120 8.7 / 10.9 to 8.4 / 11.1; in
+    // cache 1.07 / 1.09 of the time) until the runs take over.  Against the other one (K = 6144) 2 / 16 / 24 rows 9.8 / 11.2 / 13.1 -> 9.2 / 10.5 / 11.8
+    if (f.algorithm == kAuto && channel_blocks_per_cu(f.N) == 2) {
+        if (!dense_loader_eligible(f.N, f.K, f.packed_k)) return false;
+        if (f.packed_k != 0 && f.K >= 3072 && (rows > 8 || f.K > 4096)) return false;
+    }
     return f.algorithm == kAuto && tile_for(f, rows) == 0 && rows > 1 && rows <= limit;
 }
 

@@ -243,6 +243,28 @@ def test_rows_that_go_value_by_value_take_more_waves():
         assert (grid, block[0]) == want, (k, group, rows)
 
 
+# 256 CUs: 4096 channels are one block of 16 to a CU, 8192 two, 12288 three
+@pytest.mark.parametrize("packed_k, n, k, rows, algorithm", [
+    (128, 2048, 4224, 2, "runs"), (128, 2048, 4224, 16, "runs"), (0, 4096, 4224, 4, "runs"), (128, 2048, 3968, 16, "stream"),
+    (0, 1024, 3200, 24, "runs"), (128, 1024, 2944, 24, "stream"), (0, 2048, 1280, 3, "stream"), (64, 2048, 4224, 8, "runs"),
+    (128, 7168, 5376, 8, "stream"), (0, 7168, 5376, 3, "stream"), (0, 7168, 6144, 16, "stream"), (0, 5120, 10240, 16, "runs"), (128, 5120, 10240, 16, "stream"),
+    (128, 5120, 12288, 32, "runs"), (0, 9728, 6400, 8, "runs"), (128, 12288, 4096 + 128, 24, "runs"), (128, 9728, 5376, 8, "stream"), (0, 9728, 9728, 2, "gemv"),
+    (0, 9728, 8192, 16, "resident"), (0, 9728, 8192, 24, "runs"), (0, 16384, 3200, 8, "stream"),
+    (128, 2048, 5120, 16, "resident"), (128, 2048, 5120, 24, "runs"), (0, 1024, 4096, 30, "runs"), (0, 1024, 4608, 24, "resident"),
+    (128, 7168, 5120, 8, "stream"), (128, 7168, 4096, 8, "resident"), (128, 7168, 4096, 9, "stream"), (128, 7168, 2048, 24, "resident"),
+    (0, 7168, 5120, 24, "resident"), (0, 7168, 5120, 32, "runs"), (0, 7168, 4608, 32, "resident"), (128, 17408, 5120, 32, "resident"),
+])
+def test_two_to_32_rows_of_codes_go_by_blocks_of_channels(packed_k, n, k, rows, algorithm):
+    """`auto` at 2 to 32 rows: which kernel follows from the blocks of 16 channels that a CU gets, from K and from the rows."""
+    shape = dict(M=32, N=n, K=k, dynamic_rows=True, packed_k=packed_k)
+    auto = lib.Kernel("e8p_q4_projection", **shape)
+    if algorithm in ("gemv", "resident"):
+        shape["M"] = rows
+    assert auto.geometry(rows) == lib.Kernel("e8p_q4_projection", algorithm=algorithm, **shape).geometry(rows)
+    others = [a for a in ("stream", "runs") if a != algorithm]
+    assert all(auto.geometry(rows) != lib.Kernel("e8p_q4_projection", algorithm=a, **shape).geometry(rows) for a in others)
+
+
 def test_handles_own_no_device_memory_and_say_what_workspace_they_need():
     """orx_resolve allocates nothing: scratch is a `Workspace` buffer the engine sizes from
     orx_workspace_bytes (AGENTS.md:41: the engine owns every buffer).  A thousand handles resolve in

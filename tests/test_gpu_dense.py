@@ -1580,6 +1580,22 @@ def test_channel_runs_int8_weights(rows, n, k, dtype):
     assert (gu.host(out)[rows] == 91).all() and (gu.host(out)[:, n:] == 91).all()
 
 
+# Either side of the lines where `auto` changes between the batched-decode kernels, the channel runs and the streaming kernel
+@pytest.mark.parametrize("packed_k,n,k", [(128, 1000, 3968), (128, 1000, 4096 + 128), (0, 1000, 3200), (0, 1000, 4224), (64, 1000, 4224), (128, 4112, 3072),
+                                          (128, 4112, 4608), (0, 4112, 6144), (128, 8208, 4224), (0, 8208, 6272)])
+def test_two_to_32_rows_of_codes_on_either_side_of_a_rule(packed_k, n, k):
+    rng = np.random.default_rng(orc.SEED + n + k)
+    a_q, a_s, packed, scales = q4_case(rng, 32, n, k)
+    a_q[0, :2] = [-128, 127]
+    want = orc.project(a_q, a_s, orc.q4_integers(packed, TABLE), scales)
+    stored = gu.dev(packed if packed_k == 0 else orc.q4_pack_k(packed, packed_k))
+    for rows in (2, 3, 4, 8, 9, 16, 17, 24, 32):
+        out = torch.full((33, n), 55, dtype=torch.float16, device=gu.DEV)
+        gu.q4_project(gu.dev(a_q), gu.dev(a_s), stored, gu.dev(scales), out=out, rows=rows, dynamic=True, capacity=32, packed_k=packed_k)
+        np.testing.assert_array_equal(gu.host(out)[:rows], want[:rows], err_msg=str(rows))
+        assert (gu.host(out)[rows:] == 55).all()
+
+
 def test_channel_runs_refuse_what_they_do_not_serve():
     for bad in (dict(M=513), dict(K=192)):
         with pytest.raises(gu.lib.OrxError):
