@@ -730,45 +730,64 @@ bool runs_for_few_rows(const orx_function& f, int rows) {
     return f.K >= (rows > 16 ? 4096 : 6144);
 }
 
-// Channel runs with K split over the waves (k_runs.hip), `algorithm=runs` by name, and by `auto` (int8 from one row on, codes from two) while the
-// workgroups fit one round of the CUs (up to 64 rows: any number, the tiles are low).  Measured against what `auto` launched
-// before (us, N x K, 256 CUs):
-//   int8: 5120 x 17408 24 / 64 / 96 / 128 rows 32 -> 23, 45 -> 32, 46 -> 41, 47 -> 49; 17408 x 5120 24 / 64 rows 32 -> 21, 48 -> 27;
-//     4096 x 4096 32 / 96 / 256 rows 9.8 -> 7.3, 19 -> 11, 22 -> 14; 1024 x 17408 16 / 64 rows three times faster; level
-//     with the streaming kernel where that has a whole number of workgroups per CU (8192 x 8192, 4-16 rows: 0.92-0.96) or
-//     little to stream (1024 x 1024 up to 32 rows: 0.92-0.98): left there.
-//     One row, against the GEMV, whose workgroups own 32 channels and leave CUs idle or half a round empty: 5120 x 17408 20.5 ->
-//     17.9, 17408 x 5120 19.6 -> 18.3, 8192 x 8192 16.8 -> 14.3, 4096 x 4096 7.2 -> 6.4, 2048 x 2048 3.5 -> 3.4; where the runs take
-//     two rounds (34816 x 5120: 33.0 against 33.8) or below 4 M weights (1024 x 2048: 3.5 against 3.9) it stays.
-//   two-stage codes: 48 / 64 rows 17408 x 5120 31 -> 21, 31 -> 23, 7168 x 5120 12.7 -> 11.1, 14.8 -> 12.3; 96 / 128 / 200 / 256
-//     rows 7168 x 5120 22 -> 17, 25 -> 21, 36 -> 28, 36 -> 31; 4096 x 8192 200 rows 1.4, 1024 x 1024 200 rows 2.9 times faster; wider
-//     matrices go to the channel runs over all rows (11008 x 4096 at 128 / 256 rows 0.96 / 0.87).  Up to 32 rows: runs_for_few_rows.
-//     66 / 80 rows of up to 48 channels to a CU, against one pass over all rows:
-//     11008 x 4096 20.5 -> 17.9, 20.2 -> 18.0, 12288 x 3072 17.0 -> 15.7, 17.1 -> 15.9; slower at 68 channels (17408 x 5120 30.8 / 38.5).
-//   129 to 512 rows, against split tiles and decode-once with their scratch: codes 256 rows 4096 x 4096 27.4 -> 17.4, 2560 x 9728 33.6 ->
-//     28.6, 512 rows 4096 x 4096 32 -> 26, 2048 x 1024 24 -> 9, 136 / 200 rows 11008 x 4096 40.9 -> 32.4, 41.4 -> 38.1 in two rounds;
-//     int8 256 rows 4096 x 4096 23.6 -> 14.8, 2048 x 1024 20.3 -> 7.5, 136 / 200 rows 5120 x 17408 49.8 -> 38.6, 50.4 -> 45.7.  Two
-//     rounds of more than 200 rows lose (11008 x 4096 at 300 / 512 rows 47 / 55, 50 / 72; int8 5120 x 5120 at 512 41 / 47).  Row
-//     tiles of more than 120 rows and K up to 1024 go to the runs up to 16 channels to a CU only: handles of wider matrices say
-//     that they need scratch for these launches, and the split tiles that use it stay (7168 x 5120 at 256 rows 38.6, the runs 30.4).
+// int8 rows up to 32: channel runs against the streaming kernel, whose workgroups of 32 channels make the same difference as above
+// (one row: against the GEMV, which has them too).  Runs / streaming kernel, us: one block 4096 x 1024 at 8 rows 4.0 / 3.9, 2048 x 2048 3.8 / 5.0,
+// 512 x 5120 4.0 / 8.4; two 7168 x 2048 6.1 / 5.2, 5120 x 3584 6.5 / 7.2, 7168 x 5120 9.9 / 10.4; three 9728 x 1024 5.4 / 5.3, x 2048 6.8 / 7.7; five 17408 x 256 / 512
+// level, x 1024 6.6 / 7.3; N a whole number of workgroups per CU (8192, 16384) at 8 rows of K = 3584 / 5120 / 8192 1.0-1.08 / 0.92-1.0 / 1.0-1.14 of its time,
+// above 16 rows from K = 3584 on 0.78-1.03.  One row, GEMV: 4096 x 1024 4.0 / 3.8, 2048 x 2048 3.8 / 4.3, 7168 x 2048 6.1 / 5.3, x 3584 7.6 / 7.7, 5120 x 17408 17.9 / 20.5,
+// 17408 x 256 / 1024 4.4 / 5.7, 6.6 / 7.1; above 80 channels to a CU the runs take two rounds (24576 x 5120 25.7 / 22.4).
+bool runs_for_few_int8_rows(const orx_function& f, int rows) {
+    const int blocks = channel_blocks_per_cu(f.N);
+    if (rows == 1 ? blocks > 5 : rows <= 16 && f.N % (32 * device_compute_units()) == 0) return false;
+    return blocks == 5 || f.K >= (blocks % 2 == 1 ? 2048 : 3072);
+}
+
+// 33 to 64 rows, against the streaming kernel and the 64-row tiles (runs / the better one): two blocks of codes, K = 1024 1.05-1.17, K = 2048
+// 0.95-1.05; one block K = 512 / 768 / 1024 1.03-1.15 / 0.96-1.03 / 0.93-1.0; three K = 256 / 512 0.98-1.11 / 0.89-1.02; int8, two blocks K = 512 / 1024 / 2048
+// 1.1 / 0.96-1.09 / 0.82-0.97, one block K = 256 / 512 1.05-1.26 / 0.94-1.04, three K = 256 0.80-0.84.  Wider, K = 5120 codes: 17408 channels at 48 / 64 rows 31 -> 21,
+// 31 -> 23 us.
+bool runs_for_33_to_64_rows(const orx_function& f) {
+    const int blocks = channel_blocks_per_cu(f.N);
+    if (blocks == 2 || blocks == 4) return f.K >= 2048;
+    return blocks > 1 || f.K >= (f.flags == kQ4 ? 1024 : 512);
+}
+
+// 65 to 512 rows, against all other kernels (with scratch), runs / the best of them:
+//   codes, 65 to 128 rows in one round: up to 32 channels to a CU 0.56-1.06 (K from 1024; 0.8 at 4096); 33 to 48 channels, where the runs over all
+//     rows are the other kernel, 65-80 rows 0.80-0.98, 96-128 rows K = 4096 0.95-1.02, K = 5120 0.93-0.96, K = 8192 (split tiles there) 0.85-0.91; slower
+//     at 68 channels (17408 x 5120 38.5 / 30.8 us);
+//   int8, 65 to 128 rows in one round: 0.1-0.9, except long K: 128 rows of K = 8192 / 10240 / 12288 up to 16 channels to a CU 0.84-0.88 / 0.98-1.03 / 1.04-1.08 (112 rows
+//     0.76-0.82 / 0.91-0.94 / 0.96-0.99), 17 to 32 channels 0.80-0.86 / 0.84-0.97 / 0.85-1.01;
+//   129 to 512 rows, in row tiles of up to 120 rows: codes at 129-200 rows 0.37-0.97 in one round, 33 to 48 channels in two rounds 0.81-1.02 (1.08 at K =
+//     10240, 200 rows); beyond, one round of up to 32 channels 0.41-1.0, two rounds 0.95-1.76; int8 in one round:
+//     K = 8192 / 10240 / 12288 in tiles of 120 rows 0.70-0.77 / 0.89-0.94 / 0.93-0.96, K = 17408 1.08-1.12, of 100 rows 0.84-0.9 and 0.9-1.0;
+//     two rounds of int8 rows 0.6-1.6;
+//   row tiles of 121 to 128 rows, and K up to 1024: up to 16 channels to a CU only (codes of any K 0.5-1.0 but for three row tiles of 4096 x 12288 and longer,
+//     1.06-1.16; int8 K = 10240 / 12288 / 17408 at 256 rows 0.93-0.96 / 0.96-1.0 / 1.10-1.15).  Handles of wider matrices declare scratch for these launches, and what
+//     they declare they use: the split tiles stay although the runs are faster (7168 x 5120 at 256 rows 38.6 us, the runs 30.4; K = 1024 about half the time).
+bool runs_for_many_rows(const orx_function& f, int rows) {
+    int tile_rows = 0;
+    const int rounds = runs_rounds(f.flags, rows, f.N, &tile_rows), cus = device_compute_units();
+    if (rows <= 128) {
+        if (f.flags == kW8) return rounds == 1 && (rows <= 112 || f.K <= 8192 || f.N > 16 * cus);
+        return rounds == 1 && f.N <= (rows <= 80 || f.K > 4096 ? 48 : 32) * cus;
+    }
+    if (tile_rows > 120 || f.K <= 1024)
+        return rounds == 1 && f.N <= 16 * cus && (f.K <= 10240 || (f.flags == kQ4 && (f.N <= 8 * cus || rows <= 256 || rows > 384)));
+    if (f.flags == kW8) return rounds == 1 && (f.K <= 8192 || tile_rows <= 100);
+    if (rows <= 200) return rounds <= 2 && f.N <= 48 * cus;
+    return rounds == 1 && f.N <= 32 * cus;
+}
+
+// Channel runs with K split over the waves (k_runs.hip): `algorithm=runs` by name, and by `auto` from one int8 row and two rows of codes
+// on.  The figures beside the rules are of 256 CUs and matrices that together do not stay in cache.
 bool use_runs(const orx_function& f, int rows) {
     if (f.algorithm == kRuns) return runs_eligible(f.flags, rows, f.N, f.K);
     if (f.algorithm != kAuto || tile_for(f, rows) != 0 || rows < (f.flags == kW8 ? 1 : 2) || f.K % kBK != 0 || !runs_eligible(f.flags, rows, f.N, f.K)) return false;
     if ((f.flags2 & kPreferGemv) && f.block_m > 0 && rows <= 4) return false;  // the dot-product family wherever it serves the rows
-    const int64_t weights = (int64_t)f.N * f.K;
-    if (rows > 64) {
-        int tile_rows = 0;
-        const int rounds = runs_rounds(f.flags, rows, f.N, &tile_rows), cus = device_compute_units();
-        if (f.flags2 & kNoSplit) return false;
-        if (rows > 128 && (f.K <= 1024 || tile_rows > 120)) return rounds == 1 && f.K <= 10240 && f.N <= 16 * cus;
-        if (f.flags == kW8) return rounds == 1 && (rows <= 112 || f.K <= 8192 || (rows > 128 && tile_rows <= 100));
-        if (rows <= 80 || (rows > 128 && rows <= 200)) return rounds <= (rows <= 80 || f.K <= 1024 ? 1 : 2) && f.N <= 48 * cus;
-        return rounds == 1 && f.N <= 32 * cus;
-    }
-    if (f.flags == kW8 && rows == 1) return weights >= (1 << 22) && f.N <= 80 * device_compute_units();
-    if (f.flags == kW8) return rows > 32 || (weights >= (1 << 22) && (rows > 16 || f.N % (32 * device_compute_units()) != 0));
-    if (rows > 32) return weights >= (1 << 22);
-    return runs_for_few_rows(f, rows);
+    if (rows <= 32) return f.flags == kW8 ? runs_for_few_int8_rows(f, rows) : runs_for_few_rows(f, rows);
+    if (rows <= 64) return runs_for_33_to_64_rows(f);
+    return (f.flags2 & kNoSplit) == 0 && runs_for_many_rows(f, rows);
 }
 
 // Channel runs per CU over the whole K (k_wide.hip): two-stage codes, `algorithm=wide` by name, and by
@@ -828,9 +847,11 @@ bool use_gemv(const orx_function& f, int rows) {
     // them (us, GEMV / streaming kernel): row-major up to three blocks of 16 channels to a CU, 2 / 4 rows of 2048 x 1280 5.2 / 4.2 and 7.1 / 4.3,
     // 7168 x 5376 10.5 / 8.7 and 14.3 / 8.8, 9728 x 4224 1.2 times at 2 rows; K-major (2 rows) up to two, 7168 x 2560 6.8 / 5.5, 4096 x 4352 10.5 / 7.0,
     // but 11008 x 4608 10.4 / 10.9, 17408 x 3584 11.8 / 13.4
-    if (f.flags == kQ4 && rows > 1) {
+    // Two int8 rows likewise up to four blocks: 4096 x 1024 4.2 / 3.8, 8192 x 5120 11.5 / 10.2, 16384 x 8192 35.7 / 27.8, but 24576 x 3584 17.2 / 20.4.
+    if (rows > 1) {
         const int blocks = channel_blocks_per_cu(f.N);
-        if (blocks <= 2 || (blocks == 3 && f.packed_k == 0 && (rows > 2 || f.K < 6144))) return false;
+        if (f.flags == kW8 && blocks <= 4) return false;
+        if (f.flags == kQ4 && (blocks <= 2 || (blocks == 3 && f.packed_k == 0 && (rows > 2 || f.K < 6144)))) return false;
     }
     // K-major codes: 1 row (13.4 us at N=17408, K=5120; the streaming kernel takes 17.2), and 2 rows
     // (16.4 us) where the batched-decode kernel (15.4 us) does not take the shape

@@ -265,6 +265,29 @@ def test_two_to_32_rows_of_codes_go_by_blocks_of_channels(packed_k, n, k, rows, 
     assert all(auto.geometry(rows) != lib.Kernel("e8p_q4_projection", algorithm=a, **shape).geometry(rows) for a in others)
 
 
+@pytest.mark.parametrize("codec, n, k, rows, algorithm", [
+    ("w8", 1024, 2048, 4, "runs"), ("w8", 4096, 1024, 8, "stream"), ("w8", 7168, 2048, 8, "stream"), ("w8", 7168, 3072, 8, "runs"), ("w8", 8192, 5120, 16, "stream"),
+    ("w8", 8192, 5120, 2, "stream"), ("w8", 8192, 5120, 17, "runs"), ("w8", 17408, 256, 2, "runs"), ("w8", 24576, 3584, 2, "gemv"), ("w8", 1024, 2048, 1, "runs"),
+    ("w8", 7168, 2048, 1, "gemv"), ("w8", 24576, 5120, 1, "gemv"), ("w8", 8192, 1024, 48, "stream"), ("w8", 4096, 512, 48, "runs"), ("w8", 4096, 256, 48, "stream"),
+    ("q4", 1024, 2048, 48, "runs"), ("q4", 7168, 1024, 48, "stream"), ("q4", 7168, 2048, 48, "runs"), ("q4", 4096, 512, 48, "stream"), ("q4", 12288, 256, 48, "runs"),
+    ("q4", 12288, 8192, 96, "runs"), ("q4", 12288, 4096, 80, "runs"), ("q4", 12288, 4096, 96, "wide"), ("w8", 7168, 12288, 128, "runs"), ("w8", 4096, 8192, 128, "runs"),
+    ("q4", 4096, 12288, 256, "runs"), ("q4", 4096, 10240, 384, "runs"), ("q4", 2048, 12288, 384, "runs"), ("w8", 4096, 10240, 256, "runs"),
+])
+def test_which_rows_the_channel_runs_take(codec, n, k, rows, algorithm):
+    """Either side of the lines between the channel runs and the kernels beside them, int8 rows and codes, without scratch."""
+    symbol, shape = {"q4": "e8p_q4_projection", "w8": "int8_projection"}[codec], dict(M=rows, N=n, K=k)
+    auto = lib.Kernel(symbol, **shape)
+    assert auto.geometry(rows) == lib.Kernel(symbol, algorithm=algorithm, **shape).geometry(rows)
+    if algorithm != "runs":
+        assert auto.geometry(rows) != lib.Kernel(symbol, algorithm="runs", **shape).geometry(rows)
+
+
+@pytest.mark.parametrize("codec, n, k, rows", [("w8", 4096, 12288, 128), ("w8", 4096, 12288, 256), ("q4", 4096, 12288, 384), ("q4", 7168, 1024, 130)])
+def test_which_rows_the_channel_runs_leave(codec, n, k, rows):
+    symbol, shape = {"q4": "e8p_q4_projection", "w8": "int8_projection"}[codec], dict(M=rows, N=n, K=k, workspace=True)
+    assert lib.Kernel(symbol, **shape).geometry(rows) != lib.Kernel(symbol, algorithm="runs", **shape).geometry(rows)
+
+
 def test_handles_own_no_device_memory_and_say_what_workspace_they_need():
     """orx_resolve allocates nothing: scratch is a `Workspace` buffer the engine sizes from
     orx_workspace_bytes (AGENTS.md:41: the engine owns every buffer).  A thousand handles resolve in

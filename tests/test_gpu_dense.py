@@ -1596,6 +1596,21 @@ def test_two_to_32_rows_of_codes_on_either_side_of_a_rule(packed_k, n, k):
         assert (gu.host(out)[rows:] == 55).all()
 
 
+@pytest.mark.parametrize("n,k", [(512, 2048), (4112, 3072), (4112, 2944), (8192, 1152), (17400, 256)])
+def test_few_int8_rows_on_either_side_of_a_rule(n, k):
+    rng = np.random.default_rng(orc.SEED + n + k)
+    weight = rng.integers(-128, 128, (n, k), dtype=np.int8)
+    a_q = rng.integers(-127, 128, (64, k), dtype=np.int8)
+    a_s = rng.uniform(0.005, 0.02, 64).astype(np.float16)
+    ws = rng.uniform(0.005, 0.02, n).astype(np.float16)
+    want = orc.project(a_q, a_s, weight, ws)
+    for rows in (1, 2, 3, 16, 17, 33, 64):
+        out = torch.full((65, n), 55, dtype=torch.float16, device=gu.DEV)
+        gu.w8_project(gu.dev(a_q), gu.dev(a_s), gu.dev(weight), gu.dev(ws), out=out, rows=rows, dynamic=True, capacity=64)
+        np.testing.assert_array_equal(gu.host(out)[:rows], want[:rows], err_msg=str(rows))
+        assert (gu.host(out)[rows:] == 55).all()
+
+
 def test_channel_runs_refuse_what_they_do_not_serve():
     for bad in (dict(M=513), dict(K=192)):
         with pytest.raises(gu.lib.OrxError):
