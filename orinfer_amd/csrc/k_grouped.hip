@@ -55,8 +55,7 @@ typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 constexpr int kWaves = 16;
 constexpr int kThreads = kWaves * 64;
 constexpr int kSpan = kWaves * 32;             // output channels of one unit
-constexpr uint32_t kMaskOffset = 128;          // 256 entries x (16 copies of basis, 16 of mask) x 8 bytes
-constexpr uint32_t kInfoBase = 65536;          // (expert, first row, rows) of every routed tile
+constexpr uint32_t kInfoBase = 65536;          // behind 256 entries x (16 copies of basis, 16 of mask) x 8 bytes: (expert, first row, rows) of every routed tile
 constexpr int kMaxTiles = 1024;
 constexpr uint32_t kRowStatBase = kInfoBase + kMaxTiles * 12;  // fp16 rows quantised while staged: the scale of every staged row
 constexpr uint32_t kSumBase = kRowStatBase + 256;          // phase-two sums, then the staged token rows
@@ -196,17 +195,13 @@ __global__ __launch_bounds__(kThreads) void grouped_resident_kernel(GroupedParam
     auto fetch = [&](const uint8_t* base, int kb) { return *reinterpret_cast<const uint4*>(base + kb * kb_step); };
 
     // ---- decode ------------------------------------------------------------------------------
-    // address byte 0: this lane's copy, in the half of an entry it reads first or second; byte 1: the code byte that goes with it
-    const uint32_t copy = (uint32_t)(lane & 15) * 8, other = (uint32_t)(lane >> 4) & 1;
-    const uint32_t columns = (copy | other * kMaskOffset) | (copy | (other ^ 1) * kMaskOffset) << 8;
-    const uint32_t first_low = 0x0C0C0500u - (other << 8), second_low = 0x0C0C0401u + (other << 8);
-    const uint32_t first_high = first_low + 0x200u, second_high = second_low + 0x200u;
+    const lds_asm::WidePairedLookup paired(lane);
     auto lookup = [&](uint32_t word, uint32_t selector) {
-        return *reinterpret_cast<const uint2*>(lds + __builtin_amdgcn_perm(word, columns, selector));
+        return *reinterpret_cast<const uint2*>(lds + paired.address(word, selector));
     };
     auto decode_pair = [&](uint32_t word) -> v4i {  // two codes -> the 16 weights of one MFMA sub-step
-        const uint2 a0 = lookup(word, first_low), b0 = lookup(word, second_low);
-        const uint2 a1 = lookup(word, first_high), b1 = lookup(word, second_high);
+        const uint2 a0 = lookup(word, paired.first_low), b0 = lookup(word, paired.second_low);
+        const uint2 a1 = lookup(word, paired.first_high), b1 = lookup(word, paired.second_high);
         return v4i{(int)(a0.x ^ b0.x), (int)(a0.y ^ b0.y), (int)(a1.x ^ b1.x), (int)(a1.y ^ b1.y)};
     };
 
