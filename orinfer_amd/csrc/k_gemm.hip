@@ -2148,12 +2148,12 @@ int make_q2_unpack(const Variant& v, orx_function* f) { return make_unpack(v, f,
 const Registration* gemm_registrations(int* count) {
     static const Registration rows[] = {
     {"e8p_q4_projection", make_q4_projection,
-     "M, N, K, dynamic_rows=false, algorithm=auto|gemv|stream|resident|wide|mfma, packed_k=0|64|128, output_dtype=float16|float32, "
+     "M, N, K, dynamic_rows=false, algorithm=auto|gemv|stream|resident|wide|tall|runs|mfma, packed_k=0|64|128, output_dtype=float16|float32, "
      "input_dtype=int8|float16, rotate=false, codes=false, workspace=false, split_k=true, "
      "output_stride=N, block_m=0|32|64|128|256, gemv_passes=0, decode_in_gemm=false",
-     "A,AS,Book,Out,S[,Signs],W[,Workspace][,m]"},
+     "A,AS,Book,Out[,Q],S[,Signs],W[,Workspace][,m]"},
     {"int8_projection", make_w8_projection,
-     "M, N, K, dynamic_rows=false, algorithm=auto|gemv|stream|mfma, output_dtype=float16|float32, output_stride=N, "
+     "M, N, K, dynamic_rows=false, algorithm=auto|gemv|stream|runs|mfma, output_dtype=float16|float32, output_stride=N, "
      "block_m=0|32|64|128|256, workspace=false, split_k=true",
      "A,Output,TokenScale,Weight,WeightScale[,Workspace][,m]"},
     {"int8_small_projection", make_w8_small_projection,

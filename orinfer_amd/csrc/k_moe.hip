@@ -1285,7 +1285,7 @@ const Registration* moe_registrations(int* count) {
     {"expert_offsets", make_offsets, "E=512, block_m=16", "Counts,RowOffsets,TileCount,TileOffsets"},
     {"expert_tiles", make_tiles, "M, E=512, top_k=10, block_m=16", "Counts,TileExpert,TileOffsets,TileRow"},
     {"route_metadata", make_metadata, "M, E=512, top_k=10, block_m=8, dynamic_rows=false, slot_maps=false, workspace=false",
-     "Counts,IDs,RelativeSlot[,RowMax],RowOffsets[,SlotMap,SlotToken],TileCount,TileExpert,TileOffsets,TileRow[,m]"},
+     "Counts,IDs,RelativeSlot[,RowMax],RowOffsets[,SlotMap,SlotToken],TileCount,TileExpert,TileOffsets,TileRow[,Workspace][,m]"},
     {"single_route_metadata", make_single_metadata, "E=512, top_k=10, capacity=11",
      "Counts,IDs,Offsets,Relative,TileCount,TileExpert,TileOffsets,TileRow"},
     {"expert_partition_offsets", make_partition_offsets, "experts, hot_m, cold_m, cold_rows",

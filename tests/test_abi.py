@@ -42,6 +42,28 @@ def test_catalog_lists_every_symbol_and_resolves():
         assert needed in symbols
 
 
+def test_catalog_names_every_algorithm_and_argument():
+    """The catalog's key list names each algorithm that the factory takes by name, and its argument pattern matches the
+    lists of the variants with every optional buffer."""
+    entries = {entry["symbol"]: entry for entry in lib.catalog()["kernels"]}
+    shape = dict(M=4, N=1024, K=1024)
+    for symbol, names in (("e8p_q4_projection", ("auto", "gemv", "stream", "resident", "wide", "tall", "runs", "mfma")),
+                          ("int8_projection", ("auto", "gemv", "stream", "runs", "mfma"))):
+        listed = re.search(r"algorithm=([a-z|]+)", entries[symbol]["variant_keys"]).group(1).split("|")
+        assert sorted(listed) == sorted(names)
+        for name in names:
+            lib.Kernel(symbol, **dict(shape, M=2 if symbol == "int8_projection" else 4), algorithm=name)
+    metadata = dict(M=64, E=16, top_k=2)
+    for symbol, variant in (("e8p_q4_projection", dict(shape, M=1, input_dtype="float16", codes=True)),
+                            ("e8p_q4_projection", dict(shape, M=1, input_dtype="float16", codes=True, rotate=True)),
+                            ("e8p_q4_projection", dict(shape, dynamic_rows=True, workspace=True)),
+                            ("int8_projection", dict(shape, dynamic_rows=True, workspace=True)),
+                            ("route_metadata", dict(metadata, slot_maps=True, workspace=True, dynamic_rows=True)),
+                            ("route_metadata", dict(metadata, slot_maps=True)), ("route_metadata", metadata)):
+        pattern = re.sub(r"\[([A-Za-z,]+)\]", r"(?:\1)?", entries[symbol]["arguments"])
+        assert re.fullmatch(pattern, ",".join(lib.Kernel(symbol, **variant).arg_names)), (symbol, variant)
+
+
 ABI = {
     # symbol, variant -> expected argument order (buffers in ASCII order, scalars, m last)
     ("activation_quantization", (("K", 2560),)): ["Mask", "Q", "S", "X", "rows"],
