@@ -1160,6 +1160,32 @@ def test_long_prompts_keep_the_launches_a_caller_asked_for():
     assert torch.equal(apart.run(shifted, logits), want)
 
 
+@pytest.mark.parametrize("tokens,order", [(256, "five"), (256, "seven"), (4097, "six"), (1, "token")])
+def test_gates_that_overflow_downwards_cost_their_own_value_only(tokens, order):
+    """A gate that leaves fp16 downwards has no SwiGLU value (-inf * 0): the row's scale and its other codes are as without it,
+    in each order of launches; the same channel upwards is an infinity and takes its row along."""
+    c = workloads.config3(tokens=tokens, top_k=2)
+    scales = np.array(c["gate_up_scales"])
+    scales[:, 5] = 60000.0  # one gate channel of every expert
+    bank = (c["gate_up"], scales, c["down"], c["down_scales"])
+    x, logits = gu.dev(c["x"]), gu.dev(c["logits"])
+    shape = (c["experts"], c["top_k"], c["hidden"], c["intermediate"])
+    plain = programs.MoeLayer(tokens, *shape, *bank, fused_stages=False)
+    plain.run(x, logits)
+    with np.errstate(invalid="ignore", over="ignore"):
+        value = orc.swiglu_fp16(gu.host(plain.gate_up_out)[:, [5, c["intermediate"] + 5]])[:, 0][gu.host(plain.slot_map)]  # (tokens, top_k)
+    lost = np.isinf(value).any(axis=1)
+    assert tokens == 1 or 0.5 < lost.mean() < 0.9 and np.isnan(value)[~lost].mean() > 0.9
+    layer = plain if order == "seven" else programs.MoeTokenLayer(*shape, *bank) if order == "token" else programs.MoeLayer(tokens, *shape, *bank)
+    if order in ("five", "six"):
+        assert layer.fused_stages == (order == "five") and layer.bulk == (order == "six")
+    out = gu.host(layer.run(x, logits))
+    whole = np.isfinite(out).all(axis=1)
+    np.testing.assert_array_equal(whole, ~lost)
+    if order != "seven":
+        np.testing.assert_array_equal(out[whole], gu.host(plain.out)[whole])
+
+
 # The selector decoder's whole domain, after tests/cuda/operators/e8p_selector.py:23-94: tables drawn from
 # {0, +-2, +-6, +-10} (zero coordinates included), one table per expert or one for all, patch words on or
 # off (with the word that test plants: valid, value -128, last position), tile lists of 8 to 64 rows with
