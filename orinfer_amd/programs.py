@@ -65,7 +65,6 @@ class QuantizedLinear:
                 if error.code != ORX_ERR_BAD_VARIANT:
                     raise
         self.workspace = self.projection.workspace()
-        self._live = self.out  # the rows of `out` that the last launch wrote
 
     def quantize(self, x16, stream=None):
         rows = x16.shape[0]
@@ -82,12 +81,9 @@ class QuantizedLinear:
         return self._rows(rows)
 
     def _rows(self, rows):
-        """A tensor of the caller's own over the first rows of `out`: what it does to its shape stays with it.  (detach() makes
-        one in 0.5 us, slicing in 1.4 us of a 6 us call.)"""
-        live = self._live
-        if live.shape[0] != rows:
-            live = self._live = self.out[:rows]
-        return live.detach()
+        """A tensor of the caller's own over the first rows of `out`: what it does to its shape stays with it.  (One view, 1.0 us of
+        host time beside the launch, slicing 1.4; a kept slice and detach() take 0.5, but 12 more on a first call.)"""
+        return self.out.as_strided((rows, self.n), (self.n, 1))
 
     def run(self, x16, stream=None):
         if stream is None:
