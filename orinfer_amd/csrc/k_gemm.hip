@@ -862,8 +862,7 @@ bool use_gemv(const orx_function& f, int rows) {
 
 // weight-streaming kernel for up to 64 rows.  Two-stage codes of 65..128 rows go to the 128x128
 // MFMA tiles with the decode inside (measured at N=17408, K=5120, 128 rows: 59 us against 91 us for
-// two streaming launches and 118 us for the 256x256 kernel).  W8 leaves the streaming kernel above
-// 16 rows: the 32/64/128-row tiles measure 27 / 31 / 40 us at 32 / 48 / 128 rows against 29 / 43 / 94.
+// two streaming launches and 118 us for the 256x256 kernel).
 bool use_stream(const orx_function& f, int rows) {
     if (f.algorithm == kStream) return rows <= 64;
     if (f.algorithm != kAuto || tile_for(f, rows) != 0) return false;

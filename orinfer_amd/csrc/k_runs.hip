@@ -13,7 +13,7 @@
 //  * Codes go from memory into registers, 16 bytes per lane, block of channels and chunk, and through the paired tables into
 //    the weight operands; the lookups of a block for the next step of 64 run under the multiplies of that block, and are
 //    combined under those of the block after it.
-//  What bounds it (7168 x 5120 codes of 200 rows, 28.5 us): LDS, at about half its rate, with one wave to a SIMD to keep it busy;
+//  What bounds it (7168 x 5120 codes of 200 rows, 28.5 us): latency, with one wave to a SIMD and the LDS at about half its rate;
 //  without the token requests, the lookups or the stores it takes 3.6, 4.6 or 2.3 us less.  int8, 24 rows of 5120 x 17408: the stream, 4.6 TB/s.
 //  * Quarter q of a wave multiplies bytes [32 q, +32) of a chunk, 16 in each of two steps: piece c = 2 q + s of row r sits at
 //    position (q + 4 s) ^ swizzle(r).
