@@ -791,23 +791,19 @@ bool use_runs(const orx_function& f, int rows) {
 }
 
 // Channel runs per CU over the whole K (k_wide.hip): two-stage codes, `algorithm=wide` by name, and by
-// `auto` at 65..128 rows (33..64 rows of large matrices) while K is short enough.  Its time is 10 us + 0.4..0.55 us per K step of 128 whatever
+// `auto` at 65..128 rows while K is short enough.  Its time is 10 us + 0.4..0.55 us per K step of 128 whatever
 // N is (up to 96 channels per CU), where the split 128 x 128 tiles pay for N K: measured at 65-128 rows,
 // K-major and row-major alike, K = 1024: 9 against 23 us (N = 1024); 2560: 16-17 against 26-28 (N = 9728);
 // 4096: 20-23 against 29 (N = 11008), 17-20 against 23 (N = 4096); 5120: 31-32 against 40 (N = 17408),
 // 21-25 against 27-30 (N = 5120, 7168), 55-62 against 62-63 (N = 34816); 8192: 30-36 against 32 (N = 8192),
 // 70-83 against 72-74 (N = 28672); 9728 and up: slower (N = 5120, K = 17408: 56-69 against 41).  Below 65
-// rows the batched-decode kernels are as fast or faster except at N = 17408 (30 against 31-34 us), above 128
+// rows the runs over part of the rows are faster (N = 17408 at 64 rows 23 against 30 us), above 128
 // rows a second pass doubles the time (58-62 against 57 us at 160-256 rows).
 bool use_wide(const orx_function& f, int rows) {
     if (f.flags != kQ4 || !dense_wide_eligible(f.N, f.K, f.packed_k)) return false;
     if (f.algorithm == kWide) return true;
     if (f.algorithm != kAuto || tile_for(f, rows) != 0 || f.K > 6144) return false;
-    if (rows >= 65 && rows <= 128) return true;
-    // 33..64 rows of a large matrix would be two batched-decode launches: one pass here is faster while a CU's
-    // run fits one channel pass (N = 17408, K = 5120: 29.9 / 30.2 / 30.4 us at 33 / 48 / 64 rows against 31.2 / 31.8 /
-    // 34.3; N = 34816, two channel passes: 51-53 against 49-54, left alone)
-    return rows >= 33 && rows <= 64 && (int64_t)f.N * f.K >= ((int64_t)1 << 26) && f.N <= 96 * device_compute_units();
+    return rows >= 65 && rows <= 128;
 }
 
 // Two-stage codes on 512 rows x channel runs with the decode in the K loop (k_gemm_big.hip): `algorithm=tall` by
@@ -866,25 +862,17 @@ bool use_gemv(const orx_function& f, int rows) {
 bool use_stream(const orx_function& f, int rows) {
     if (f.algorithm == kStream) return rows <= 64;
     if (f.algorithm != kAuto || tile_for(f, rows) != 0) return false;
-    if (f.flags == kQ4) return rows <= 64;
-    // W8 with weights that do not stay in cache: up to 32 rows (N = 17408, K = 5120 at 32 rows: 34.8 us
-    // against 39.0 us for the 32-row tiles; at 48 rows 49.0 against 42.5), up to 64 rows for matrices of
-    // at most 32 M weights (N = K = 4096 at 64 rows: 14.7 against 19.5 us)
-    return rows <= 32 || (rows <= 64 && (int64_t)f.N * f.K <= (int64_t)1 << 25);
+    // what the channel runs leave: matrices with little to stream, and 2^31 weights and more, where int8 rows above 32 are faster
+    // on the 64-row tiles (17408 x 5120 at 48 rows 42.5 to 49.0)
+    return rows <= 32 || (rows <= 64 && (f.flags == kQ4 || (int64_t)f.N * f.K < ((int64_t)1 << 31)));
 }
 
-// Resident two-stage kernel (32 rows per launch) where the streaming kernel would run and the shape
-// fits; `algorithm=resident` asks for it by name.
+// Resident two-stage kernel (up to 32 rows; by name several launches of 32) where the streaming kernel would run and the shape fits.
 bool use_resident(const orx_function& f, int rows) {
     if (f.flags != kQ4 || !dense_resident_eligible(f.N, f.K, f.packed_k)) return false;
     if (f.algorithm == kResident) return rows <= 128;
     // from 2 rows: the GEMV's dot products grow with the row count (16.4 us at 2 rows, 23 us at 3 and 4
     // rows of N=17408, K=5120), this kernel's MFMAs do not (15.6 us from 2 to 16 rows)
-    // up to 64 rows as two launches of 32 (36 and 39 us at 48 and 64 rows against 42 and 48 us for
-    // the streaming kernel)
-    // (the second launch pays for itself only on large matrices: N = 17408, K = 5120 at 48 rows 33 us
-    // against 39 us for the streaming kernel, but N = K = 5120 20 against 14.5 us)
-    const int limit = (int64_t)f.N * f.K >= ((int64_t)1 << 26) ? 64 : 32;
     // Two blocks of 16 channels to a CU fill the streaming kernel's workgroups of 32 channels.  Against the loader-wave
     // kernel (us, N = 7168): K-major codes 16 rows of K = 3072 / 4096 / 5120 6.4 / 7.6 / 9.0 -> 6.0 / 6.8 / 7.9, 24 rows 7.5 / 8.7 / 10.7 ->
     // 6.6 / 7.5 / 8.9, 2 / 8 rows of K = 5120 7.9 / 8.4 -> 7.5 / 7.8 (weights in cache: 0.96 / 0.99 of its speed), of K = 4096 6.8 / 7.1 -> 6.6 / 6.7 (0.95 / 1.0), K = 2048
@@ -894,7 +882,7 @@ bool use_resident(const orx_function& f, int rows) {
         if (!dense_loader_eligible(f.N, f.K, f.packed_k)) return false;
         if (f.packed_k != 0 && f.K >= 3072 && (rows > 8 || f.K > 4096)) return false;
     }
-    return f.algorithm == kAuto && tile_for(f, rows) == 0 && rows > 1 && rows <= limit;
+    return f.algorithm == kAuto && tile_for(f, rows) == 0 && rows > 1 && rows <= 32;
 }
 
 // 256x256 tiles once there are enough rows to fill them (or when block_m = 256 is forced)
