@@ -65,51 +65,45 @@ __device__ __forceinline__ uint32_t nibble_mask_word(uint32_t u) {
 // "biased nibble" form: byte j = ((h_j ^ 8) & 15) << shift and mask_j << shift.  XOR of a basis
 // entry and a mask entry is (v_j + 8) << shift, an unsigned value that never carries out of
 // its byte for shift <= 3.
+// The four nibbles at bits 16 HALF .. of a selector word, one to a byte and without their top bit.
+template <int HALF>
+__device__ __forceinline__ uint32_t spread_nibbles(uint32_t selector) {
+    uint32_t x = HALF ? selector >> 16 : selector & 0xFFFFu;
+    x = (x | x << 8) & 0x00FF00FFu;
+    return (x | x << 4) & 0x07070707u;
+}
+// Sign bits of coordinates 0..3 (HALF 0) or 4..7 of a low byte without its parity, as 0 or 1 in the four bytes.
+template <int HALF>
+__device__ __forceinline__ uint32_t spread_signs(uint32_t m) {
+    m >>= 2 * HALF;  // coordinate j of a half: bits 0, 4, 1, 5
+    return (m & 1u) | (m & 0x10u) << 4 | (m & 2u) << 15 | (m & 0x20u) << 19;
+}
+// Entries are made by every workgroup in front of its first lookup, a thread an entry: the eight bytes of a selector word are
+// picked out of a palette of eight by two v_perm_b32 (about a dozen instructions where a coordinate at a time took a hundred).
 __device__ __forceinline__ uint2 byte_basis_biased(uint32_t selector, int shift) {
-    uint32_t lo = 0, hi = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        lo |= ((((uint32_t)selector_half(selector, j) ^ 8u) & 15u) << shift) << (8 * j);
-        hi |= ((((uint32_t)selector_half(selector, j + 4) ^ 8u) & 15u) << shift) << (8 * j);
-    }
-    return make_uint2(lo, hi);
+    constexpr uint32_t kLow = 0x080D0B09u, kHigh = 0x08030507u;  // (h ^ 8) & 15 of ids 0..3 and of their negatives
+    return make_uint2(__builtin_amdgcn_perm(kHigh, kLow, spread_nibbles<0>(selector)) << shift,
+                      __builtin_amdgcn_perm(kHigh, kLow, spread_nibbles<1>(selector)) << shift);
 }
 
 __device__ __forceinline__ uint2 byte_mask_biased(uint32_t u, int shift) {
-    const uint32_t p = __popc(u) & 1u;
-    const uint32_t m = u ^ p;
-    uint32_t lo = 0, hi = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        lo |= (((sign_bit(m, j) ? 0xEu : 0u) ^ p) << shift) << (8 * j);
-        hi |= (((sign_bit(m, j + 4) ? 0xEu : 0u) ^ p) << shift) << (8 * j);
-    }
-    return make_uint2(lo, hi);
+    const uint32_t p = __popc(u) & 1u, m = u ^ p, parity = p * 0x01010101u;
+    const uint32_t lo = spread_signs<0>(m), hi = spread_signs<1>(m);
+    return make_uint2((((lo << 4) - (lo << 1)) ^ parity) << shift, (((hi << 4) - (hi << 1)) ^ parity) << shift);
 }
 
 // "signed byte" form (single-stage Q2): byte j = t_j and mask3_j; XOR is q_j itself.
 __device__ __forceinline__ uint2 byte_basis_signed(uint32_t selector) {
-    uint32_t lo = 0, hi = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        lo |= ((uint32_t)(2 * selector_half(selector, j)) & 255u) << (8 * j);
-        hi |= ((uint32_t)(2 * selector_half(selector, j + 4)) & 255u) << (8 * j);
-    }
-    return make_uint2(lo, hi);
+    constexpr uint32_t kLow = 0x000A0602u, kHigh = 0x00F6FAFEu;  // t of ids 0..3 and of their negatives
+    return make_uint2(__builtin_amdgcn_perm(kHigh, kLow, spread_nibbles<0>(selector)),
+                      __builtin_amdgcn_perm(kHigh, kLow, spread_nibbles<1>(selector)));
 }
 
+// 0x01, 0xFD with the sign bit; 0x03, 0xFF at odd parity: 1 ^ 0xFC ^ 2
 __device__ __forceinline__ uint2 byte_mask_signed(uint32_t u) {
-    const uint32_t p = __popc(u) & 1u;
-    const uint32_t m = u ^ p;
-    uint32_t lo = 0, hi = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const uint32_t a = sign_bit(m, j) ? (p ? 0xFFu : 0xFDu) : (p ? 0x03u : 0x01u);
-        const uint32_t b = sign_bit(m, j + 4) ? (p ? 0xFFu : 0xFDu) : (p ? 0x03u : 0x01u);
-        lo |= a << (8 * j);
-        hi |= b << (8 * j);
-    }
-    return make_uint2(lo, hi);
+    const uint32_t p = __popc(u) & 1u, m = u ^ p, parity = 0x01010101u ^ (p * 0x02020202u);
+    const uint32_t lo = spread_signs<0>(m), hi = spread_signs<1>(m);
+    return make_uint2(((lo << 8) - (lo << 2)) ^ parity, ((hi << 8) - (hi << 2)) ^ parity);
 }
 
 // LDS tables for the byte decoders.
