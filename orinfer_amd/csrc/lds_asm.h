@@ -23,6 +23,19 @@ __device__ __forceinline__ void direct_load_16(const void* global, void* lds_wav
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)global,
                                      (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, 0);
 }
+// The same from an asm statement: a uniform base and 32 bits per lane, and no wait in front of the LDS accesses that the compiler
+// can see.  OFFSET counts on both sides; the LDS base stays set for the requests that follow with set_lds_base left out.
+template <bool SET_LDS_BASE, int OFFSET>
+__device__ __forceinline__ void request_16(uint32_t lane_offset, const void* uniform_base, uint32_t lds_wave_base) {
+    if constexpr (SET_LDS_BASE)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3" ::"v"(lane_offset), "s"(uniform_base), "s"(lds_wave_base), "n"(OFFSET)
+                     : "memory");
+    else
+        asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" ::"v"(lane_offset), "s"(uniform_base), "n"(OFFSET) : "memory");
+}
+__device__ __forceinline__ void lds_write_16(uint32_t address, v4u value) {
+    asm volatile("ds_write_b128 %0, %1" ::"v"(address), "v"(value) : "memory");
+}
 template <int OFFSET>
 __device__ __forceinline__ void lds_read_16(v4i& value, uint32_t address) {
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(value) : "v"(address), "n"(OFFSET));
@@ -40,6 +53,26 @@ __device__ __forceinline__ void load_8(v2u& value, uint32_t lane_offset, const v
 }
 __device__ __forceinline__ void load_16(v4u& value, uint32_t lane_offset, const void* uniform_base) {
     asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(value) : "v"(lane_offset), "s"(uniform_base) : "memory");
+}
+template <typename T>
+__device__ __forceinline__ void keep(T& value) { asm volatile("" : "+v"(value)); }
+// In and out in one register: left to itself the compiler moves sums about between unrolled steps, a tenth of a loop's
+// instructions.  What it would have inserted is on the caller: two instructions between the last write of an operand and the multiply,
+// and a pause (s_nop 15) in front of the first reading of a sum.
+// ACC: the sum in accumulation registers (the kernel then has half of its registers of either kind).
+template <bool ACC>
+__device__ __forceinline__ void multiply_in_place(v4i& sum, const v4i& weight, const v4i& token) {
+    if constexpr (ACC)
+        asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+a"(sum) : "v"(weight), "v"(token));
+    else
+        asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+v"(sum) : "v"(weight), "v"(token));
+}
+template <bool ACC>
+__device__ __forceinline__ void keep_sum(v4i& sum) {
+    if constexpr (ACC)
+        asm volatile("" : "+a"(sum));
+    else
+        asm volatile("" : "+v"(sum));
 }
 template <typename T>
 __device__ __forceinline__ T* uniform_pointer(T* pointer) {
@@ -80,6 +113,60 @@ struct WidePairedLookup {
         return __builtin_amdgcn_perm(code, columns, selector);
     }
 };
+// Two-stage codes: four tables (basis and mask of the coarse code, basis and mask of the fine one) share entries of BYTES, 256 or 128, in
+// copies of 8 bytes.  Of BYTES / 8 neighbouring lanes a quarter reads each table, each lane its own copy, so no two meet in a bank;
+// round r of a code reads table group ^ r: rounds 0 and 1 one stage's pair, rounds 2 and 3 the other's.
+// The entries are byte_basis_biased and byte_mask_biased, the coarse ones shifted by 2, so that
+// (e0 ^ e1) + (e2 ^ e3) = 4 (v0 + 8) + (v1 + 8) = (w + 75) / 2, between 10 and 65 in every byte: two instructions per four weights, and a
+// signed byte as it is.  sum(a w) is then 2 sum(a W) - 75 sum(a).
+constexpr int kQuadBias = 75;
+template <int BYTES>
+constexpr uint32_t kQuadTableBytes = 256 * BYTES;
+template <int BYTES>
+struct QuadLookup {
+    static_assert(BYTES == 256 || BYTES == 128, "eight or four copies");
+    uint32_t columns[BYTES == 256 ? 1 : 4], select[4];
+    __device__ __forceinline__ explicit QuadLookup(int lane) {
+        constexpr uint32_t kCopies = BYTES / 32;
+        const uint32_t group = (uint32_t)lane / kCopies & 3, copy = (uint32_t)lane % kCopies * 8;
+        if constexpr (BYTES == 256) columns[0] = 0;
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) {
+            const uint32_t table = group ^ r, column = table * (BYTES / 4) + copy, byte = table ^ 1;  // of the code, the index of the table
+            if constexpr (BYTES == 256)  // byte 0 of an address is the column, byte 1 the index: one v_perm_b32
+                columns[0] |= column << (8 * r), select[r] = 0x0C0C0000u | (4 + byte) << 8 | r;
+            else
+                columns[r] = column, select[r] = 8 * byte;
+        }
+    }
+    template <int ROUND>
+    __device__ __forceinline__ void read(v2u& entry, uint32_t code) const {  // the tables lie at LDS address 0
+        if constexpr (BYTES == 256)
+            lds_read_8<0>(entry, __builtin_amdgcn_perm(code, columns[0], select[ROUND]));
+        else
+            lds_read_8<0>(entry, (__builtin_amdgcn_ubfe(code, select[ROUND], 8) << 7) + columns[ROUND]);
+    }
+};
+// Every lane of a wave writes its own entry, whole entries apart: the order of the 16-byte slots turns with the entry, so that
+// the lanes of a write spread over the banks.
+template <int BYTES>
+__device__ __forceinline__ void write_quad_entry(int entry, uint2 coarse_basis, uint2 coarse_mask, uint2 fine_basis, uint2 fine_mask) {
+    constexpr uint32_t kSlots = BYTES / 16, kEach = kSlots / 4;  // kEach slots of a table in a row
+    uint2 value[4] = {coarse_basis, coarse_mask, fine_basis, fine_mask};
+    const uint32_t turn = BYTES == 256 ? (uint32_t)entry & 15 : (uint32_t)entry >> 1 & 7;
+    auto swap_if = [](bool swap, uint2& a, uint2& b) {
+        const uint2 x = swap ? b : a, y = swap ? a : b;
+        a = x, b = y;
+    };
+    swap_if(turn & kEach, value[0], value[1]), swap_if(turn & kEach, value[2], value[3]);
+    swap_if(turn & (2 * kEach), value[0], value[2]), swap_if(turn & (2 * kEach), value[1], value[3]);
+#pragma unroll
+    for (uint32_t i = 0; i < kSlots; ++i) {
+        const uint2 v = value[i / kEach];
+        lds_write_16((uint32_t)entry * BYTES + (i ^ turn) * 16, v4u{v.x, v.y, v.x, v.y});
+    }
+}
+
 // One half of a paired entry: SLOTS 16-byte slots of two copies each.  Every lane of a wave writes its own entry, so the slot
 // order turns with the entry: in the same order for all, the lanes, whole entries apart, would write to the same banks (the
 // 16-wave kernels spent 2 us of every launch on 64 KB of tables that way, 0.3 us now).

@@ -1580,6 +1580,23 @@ def test_channel_runs_int8_weights(rows, n, k, dtype):
     assert (gu.host(out)[rows] == 91).all() and (gu.host(out)[:, n:] == 91).all()
 
 
+# Remainders of the ring with one wave to a SIMD (slices of 3, 5 and 7 chunks), all heights of a tile from five blocks on, channels that
+# end in the middle of a store, rows of outputs at every alignment of a store.
+@pytest.mark.parametrize("rows,n,k", [(72, 5000, 1536), (96, 5000, 2560), (104, 7000, 2688), (112, 5001, 3584), (128, 12000, 1664), (240, 7000, 2560),
+                                      (130, 2562, 3456)])
+@pytest.mark.parametrize("dtype,pad", [(torch.float16, 1), (torch.float16, 4), (torch.float32, 3)], ids=["fp16-odd", "fp16-8-bytes", "fp32"])
+def test_channel_runs_two_stage_codes_remainders_and_strides(rows, n, k, dtype, pad):
+    rng = np.random.default_rng(orc.SEED + rows + n + k + pad)
+    a_q, a_s, packed, ws = q4_case(rng, rows, n, k)
+    a_q[0, :], a_q[1, :] = 127, -128  # the largest sums either way
+    stride = n + pad
+    out = torch.full((rows + 1, stride), 91, dtype=dtype, device=gu.DEV)
+    gu.q4_project(gu.dev(a_q), gu.dev(a_s), gu.dev(packed), gu.dev(ws), out=out, rows=rows, stride=stride, dtype=dtype, algorithm="runs")
+    want = orc.project(a_q, a_s, orc.q4_integers(packed, TABLE), ws, out_dtype=np.float16 if dtype == torch.float16 else np.float32)
+    np.testing.assert_array_equal(gu.host(out)[:rows, :n], want)
+    assert (gu.host(out)[rows] == 91).all() and (gu.host(out)[:, n:] == 91).all()
+
+
 # Either side of the lines where `auto` changes between the batched-decode kernels, the channel runs and the streaming kernel
 @pytest.mark.parametrize("packed_k,n,k", [(128, 1000, 3968), (128, 1000, 4096 + 128), (0, 1000, 3200), (0, 1000, 4224), (64, 1000, 4224), (128, 4112, 3072),
                                           (128, 4112, 4608), (0, 4112, 6144), (128, 8208, 4224), (0, 8208, 6272)])
