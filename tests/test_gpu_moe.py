@@ -1076,6 +1076,40 @@ def test_one_token_layer_in_three_launches_gives_the_bits_of_five(e, k, h, i):
             gu.kernel("integer_e8p_gemv", **{**dict(E=e, routes=k, N=h, K=i), **variant})
 
 
+# Routes to every split of the eight waves, channels that do not fill a workgroup, K of less than and more than one request of a wave.
+@pytest.mark.parametrize("routes,n,k", [(1, 20, 128), (1, 64, 2048), (2, 100, 384), (3, 256, 1536), (4, 8, 640), (5, 130, 512), (8, 1000, 2048), (7, 33, 1152)])
+def test_second_projection_of_one_token_with_the_sum_over_its_routes(routes, n, k):
+    e = 16
+    rng = np.random.default_rng(orc.SEED + routes * n + k)
+    codes = gu.dev(programs.codebook.q2_to_k_major(rng.integers(0, 2**16, (e, n, k // 8), dtype=np.uint16)))
+    scales = gu.dev(rng.uniform(0.005, 0.02, (e, n)).astype(np.float16))
+    rows = gu.dev(rng.normal(0, 1, (routes, 2 * k)).astype(np.float16))
+    ids = rng.permutation(e)[:routes].astype(np.int32)
+    if routes > 4:
+        ids[2] = e  # names no expert: its row and scale stay as they were, and the row counts as it is
+    d_ids, prob = gu.dev(ids), gu.dev(rng.uniform(0, 1, (1, routes)).astype(np.float32))
+    book = gu.dev(programs.codebook.raw_book())
+    shape = dict(E=e, routes=routes, N=n, K=k, shared_input=False, input_dtype="float16", fused_swiglu=True)
+    half = dict(dtype=torch.float16, device=gu.DEV)
+    got = {}
+    for combine in (False, True):
+        c, scale, out = torch.full((routes, n), 0.5, **half), torch.full((routes, 1), 0.25, **half), torch.full((1, n + 8), 7, **half)
+        args = dict(A=rows, AS=scale, Book=book, C=c, IDs=d_ids, P=codes, WS=scales)
+        if combine:
+            gu.kernel("integer_e8p_gemv", combine=True, **shape)(Output=out, Prob=prob, **args)
+        else:
+            gu.kernel("integer_e8p_gemv", **shape)(**args)
+            slots = torch.arange(routes, dtype=torch.int32, device=gu.DEV)
+            gu.kernel("moe_combine", H=n, slots=routes, M=1, E=e, top_k=routes)(Expert=c, Output=out, Prob=prob, Shared=None, SharedGate=None, SlotMap=slots)
+        gu.sync()
+        got[combine] = (c, scale, out)
+    for one, two, name in zip(got[False], got[True], ("rows", "scales", "sum")):
+        assert torch.equal(one, two), name
+    for bad in (dict(routes=9), dict(K=2176), dict(fused_swiglu=False, input_dtype="int8"), dict(route_logits=True)):
+        with pytest.raises(gu.lib.OrxError):
+            gu.kernel("integer_e8p_gemv", **{**shape, "combine": True, **bad})
+
+
 @pytest.mark.parametrize("fused_stages", [False, True], ids=["seven-launches", "five-launches"])
 def test_expert_layer_when_every_token_names_the_same_experts(fused_stages):
     """The skew a router can produce: all 150 tokens choose the same four of sixteen experts, so those
