@@ -307,4 +307,13 @@ __device__ __forceinline__ float rescale(int acc, float weight_scale, float toke
     return value;
 }
 
+// two fp32 values rounded to nearest even and packed (one v_cvt_pk_f16_f32)
+__device__ __forceinline__ uint32_t pack_halves(float low, float high) {
+    typedef float pair_f32 __attribute__((ext_vector_type(2)));
+    typedef _Float16 pair_f16 __attribute__((ext_vector_type(2)));
+    const pair_f32 pair = {low, high};
+    const pair_f16 rounded = __builtin_convertvector(pair, pair_f16);
+    return *reinterpret_cast<const uint32_t*>(&rounded);
+}
+
 }  // namespace orx

@@ -18,11 +18,12 @@
 //  * The two tables share 32 KiB without conflicts (PairedLookup); two tables of eight copies, read one after the other, had half
 //    as many conflict cycles again, and sixteen copies of each leave room for one workgroup per CU.
 // Measured at 4096 tokens x top-8 of 128 experts (H = 2048, I = 512; popularity of the experts like 1 / rank^1.1):
-// gate_up 296 -> 100 us, down 215 -> 86 us.  What bounds it now: no pipe is full (LDS 42 %, vector ALU 40 %, matrix pipe
-// 30 % of the cycles); the two waves of a SIMD wait for each other's LDS reads and barriers in a third of theirs.
+// gate_up 296 -> 100 us, down 215 -> 67 us.  What bounds it now: the loop, where two waves of a SIMD keep its matrix pipe busy
+// in 0.85 of the cycles, is 9800 of the 21000 cycles of a unit of down and 38000 of 57000 of gate_up; set-up (two dependent reads of
+// the tile lists, tables, first chunks) takes 5400, the epilogue 4600 and, with the SwiGLU's sixteen instructions a sigmoid, 11000; and
+// units of 35 us that start late leave CUs idle at the end of gate_up.
 // One persistent workgroup of eight waves per CU that requests the next unit's chunks early measured 118 and 75 us.
-// Down without its stores takes 14 us less, without the K loop 55, without either 42 (K = 512: four chunks between set-up and
-// epilogue).  A workgroup that takes 2, 4 or 8 spans of a tile in a row, the next one's chunks requested in the last steps, and 512
+// A workgroup that takes 2, 4 or 8 spans of a tile in a row, the next one's chunks requested in the last steps, and 512
 // persistent workgroups of this form with even shares both measured level or slower (whole layer 227 / 241 / 247 and 243 against
 // 226 us): what the set-up saves, the uneven ends lose.
 //  * SWIGLU: a wave owns 32 gate and the 32 matching up channels, so gate and up of one (slot, channel) meet in one
@@ -69,9 +70,6 @@ struct BulkParams {
     int n, k, tile_capacity, spans;
 };
 
-__device__ __forceinline__ uint32_t pack2(__half low, __half high) {
-    return (uint32_t)__half_as_ushort(low) | (uint32_t)__half_as_ushort(high) << 16;
-}
 template <bool GATHER, bool SWIGLU>
 __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p) {
     extern __shared__ __align__(16) uint8_t lds[];
@@ -81,10 +79,14 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
     // ---- unit: workgroups 8 apart (one XCD) take the spans of one tile, whose rows that XCD's L2 then holds ----
     const int b = (int)blockIdx.x, region = 8 * p.spans;
     const int tile = (b / region) * 8 + b % 8, span = (b / 8) % p.spans;
-    if (tile >= p.tile_capacity || tile >= p.tile_count[0]) return;
-    const uint32_t selector = p.book[tid];
-    const int expert = __builtin_amdgcn_readfirstlane(p.tile_expert[tile]);
-    const int first = __builtin_amdgcn_readfirstlane(p.tile_row[tile]);
+    if (tile >= p.tile_capacity) return;
+    uint32_t selector;
+    asm volatile("global_load_dword %0, %1, %2" : "=v"(selector) : "v"((uint32_t)tid * 4), "s"(uniform_pointer(p.book)) : "memory");
+    // the list's length and its entry in one trip; behind the end an entry is whatever the buffer holds
+    const int listed = p.tile_count[0], listed_expert = p.tile_expert[tile], listed_row = p.tile_row[tile];
+    if (tile >= listed) return;
+    const int expert = __builtin_amdgcn_readfirstlane(listed_expert);
+    const int first = __builtin_amdgcn_readfirstlane(listed_row);
     const int rows = __builtin_amdgcn_readfirstlane(min(kTileRows, p.counts[expert] - first));
     if (rows <= 0) return;
     const int row0 = __builtin_amdgcn_readfirstlane(p.offsets[expert] + first);
@@ -117,16 +119,25 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
             const int slot = row0 + min(row, rows - 1);
             const int position = (lane & 7) ^ swizzle(row);
             const int piece = ((position & 3) << 1) | (position >> 2);
-            row_offset[i] = (uint32_t)(GATHER ? p.slot_token[slot] : slot) * (uint32_t)p.k + (uint32_t)piece * 16;
+            row_offset[i] = (uint32_t)(GATHER ? p.slot_token[slot] : slot) * (uint32_t)p.k + (uint32_t)piece * 16 + 4096u - (uint32_t)i * 1024u;
         }
-        auto issue_tokens = [&](int chunk, int slot) {
-            const int8_t* base = a_base + min(chunk, chunks - 1) * 128;
-#pragma unroll
-            for (int i = 0; i < LOADS; ++i) {
-                uint32_t offset = row_offset[i];
-                asm volatile("" : "+v"(offset));  // 32 bits beside a uniform base, not a 64-bit address kept per request
-                direct_load_16(base + (uint64_t)offset, lds + kTokens + (uint32_t)slot * kSlot + (uint32_t)(wave * LOADS + i) * 1024);
-            }
+        // scales of the tile's rows and of this wave's channels (channel `lane`, in the order of its four blocks), waited for by hand like all that follows
+        uint32_t token_scale_bits = 0, channel_scale_bits;
+        {
+            const int slot = row0 + min(tid, rows - 1);
+            const uint64_t of_row = reinterpret_cast<uint64_t>(p.as + (GATHER ? p.slot_token[slot] : slot));
+            const int channel = SWIGLU && lane >= 32 ? inner + n0 + lane - 32 : n0 + lane;
+            const uint64_t of_channel = reinterpret_cast<uint64_t>(p.ws + (int64_t)expert * p.n + channel);
+            asm volatile("global_load_ushort %0, %1, off" : "=v"(token_scale_bits) : "v"(of_row) : "memory");
+            asm volatile("global_load_ushort %0, %1, off" : "=v"(channel_scale_bits) : "v"(of_channel) : "memory");
+        }
+        const uint32_t token_slots = lds_address_of(lds) + kTokens + (uint32_t)wave * (LOADS * 1024);
+        auto issue_tokens = [&](int chunk, int slot) {  // (the instruction's offset counts in memory too and is taken off the lane's)
+            const int8_t* const base = a_base + (int64_t)min(chunk, chunks - 1) * 128 - 4096;
+            const uint32_t to = token_slots + (uint32_t)slot * kSlot;
+            request_16<true, 0>(row_offset[0], base, to);
+            if constexpr (LOADS > 1) request_16<false, 1024>(row_offset[1], base, to);
+            if constexpr (LOADS > 2) request_16<false, 2048>(row_offset[2], base, to), request_16<false, 3072>(row_offset[3], base, to);
         };
         // two register sets of codes, by the parity of the chunk: four blocks of 16 channels, 8 bytes to a lane
         v2u codes[2][4];
@@ -146,17 +157,12 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
         issue_tokens(1, 1);
 
         // ---- tables, scales (beside the first loads) ----
-        {
-            write_paired_entry(lds, tid, false, byte_basis_signed(selector));
-            write_paired_entry(lds, tid, true, byte_mask_signed((uint32_t)tid));
-            if (tid < kTileRows) {
-                const int slot = row0 + min(tid, rows - 1);
-                reinterpret_cast<float*>(lds + kTokenScale)[tid] = __half2float(p.as[GATHER ? p.slot_token[slot] : slot]);
-            }
-            // channel scale `lane` of each wave, in the order of its four blocks
-            const int channel = SWIGLU && lane >= 32 ? inner + n0 + lane - 32 : n0 + lane;
-            reinterpret_cast<float*>(lds + kChannelScale)[tid] = __half2float(p.ws[(int64_t)expert * p.n + channel]);
-        }
+        constexpr int kChunkRequests = 4 + LOADS;
+        asm volatile("s_waitcnt vmcnt(%3)" : "+v"(selector), "+v"(token_scale_bits), "+v"(channel_scale_bits) : "n"(2 * kChunkRequests));
+        write_paired_entry(lds, tid, false, byte_basis_signed(selector));
+        write_paired_entry(lds, tid, true, byte_mask_signed((uint32_t)tid));
+        if (tid < kTileRows) reinterpret_cast<float*>(lds + kTokenScale)[tid] = __half2float(__ushort_as_half((unsigned short)token_scale_bits));
+        reinterpret_cast<float*>(lds + kChannelScale)[tid] = __half2float(__ushort_as_half((unsigned short)channel_scale_bits));
 
         v4i acc[NB][4];
 #pragma unroll
@@ -168,11 +174,12 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
         const uint32_t lds_base = lds_address_of(lds);
         const PairedLookup tables(lds_base, lane);
         const uint32_t frag = lds_base + kTokens + (uint32_t)(lane & 15) * 128 + (uint32_t)(((lane >> 4) ^ swizzle(lane & 15)) * 16);
+        const uint32_t frag_half = frag ^ 64u;  // of a chunk's second step
         v4i token[2][RB];  // fragments of even and odd phases
-        auto read_tokens = [&](auto phase_tag, uint32_t address) {
-            constexpr int PHASE = decltype(phase_tag)::value;
-            lds_read_16<PHASE * RB * 2048>(token[PHASE & 1][0], address);
-            if constexpr (RB > 1) lds_read_16<PHASE * RB * 2048 + 2048>(token[PHASE & 1][1], address);
+        auto read_tokens = [&](auto phase_tag, auto slot_tag, uint32_t address) {
+            constexpr int PHASE = decltype(phase_tag)::value, OFFSET = decltype(slot_tag)::value * (int)kSlot + PHASE * RB * 2048;
+            lds_read_16<OFFSET>(token[PHASE & 1][0], address);
+            if constexpr (RB > 1) lds_read_16<OFFSET + 2048>(token[PHASE & 1][1], address);
         };
         v2u looked[LB][2][2];
         auto lookup = [&](int at, uint32_t word) {  // both entries of two codes
@@ -194,7 +201,7 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
         v4i weight[2][4];  // of a chunk's two steps
         // Phase PHASE of step STEP: its multiplies (one operand changing between consecutive ones), and behind the first of them
         // the fragments of the phase after it and LB blocks of the next step's codes; all of these have come when it ends.
-        auto phase = [&](auto step_tag, auto phase_tag, uint32_t next_fragments, const v2u(&next_codes)[4], auto requests) {
+        auto phase = [&](auto step_tag, auto phase_tag, auto next_slot, uint32_t next_fragments, const v2u(&next_codes)[4], auto requests) {
             constexpr int STEP = decltype(step_tag)::value, PHASE = decltype(phase_tag)::value;
             constexpr int NEXT = (PHASE + 1) % PHASES;
 #pragma unroll
@@ -205,7 +212,7 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
                     v4i& sum = acc[PHASE * RB + i][jj];
                     sum = __builtin_amdgcn_mfma_i32_16x16x64_i8(weight[STEP][jj], token[PHASE & 1][i], sum, 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
-                    if (i == 0 && j == 0) read_tokens(std::integral_constant<int, NEXT>{}, next_fragments);
+                    if (i == 0 && j == 0) read_tokens(std::integral_constant<int, NEXT>{}, next_slot, next_fragments);
                     if (i == 0 && j >= 1 && j - 1 < LB) lookup(j - 1, next_codes[PHASE * LB + j - 1][1 - STEP]);
                     if (i == 0 && j == 3) requests();
                     __builtin_amdgcn_sched_barrier(0);
@@ -220,41 +227,44 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
         std::integral_constant<int, 3> three;
 
         // ---- prologue: chunk 0 in LDS, the weights of its first step decoded, its first fragments read ----
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)"
-                     : "+v"(codes[0][0]), "+v"(codes[0][1]), "+v"(codes[0][2]), "+v"(codes[0][3]), "+v"(codes[1][0]), "+v"(codes[1][1]),
-                       "+v"(codes[1][2]), "+v"(codes[1][3])
-                     :
+        asm volatile("s_waitcnt vmcnt(%4) lgkmcnt(0)\n\ts_barrier"
+                     : "+v"(codes[0][0]), "+v"(codes[0][1]), "+v"(codes[0][2]), "+v"(codes[0][3])
+                     : "n"(kChunkRequests)
                      : "memory");
-        __syncthreads();
-        read_tokens(zero, frag);
-        read_tokens(one, frag);
+        read_tokens(zero, zero, frag);
+        read_tokens(one, zero, frag);
 #pragma unroll
-        for (int j = 0; j < 4; j += LB) {
+        for (int j = 0; j < 4; j += 2) {  // two blocks of channels at a time
+            v2u pair[2][2][2];
 #pragma unroll
-            for (int l = 0; l < LB; ++l) lookup(l, codes[0][j + l][0]);
+            for (int l = 0; l < 2; ++l) tables.read<0>(pair[l][0], codes[0][j + l][0]), tables.read<1>(pair[l][1], codes[0][j + l][0]);
             wait_reads();
 #pragma unroll
-            for (int l = 0; l < LB; ++l) weight[0][j + l] = combine(l);
+            for (int l = 0; l < 2; ++l) {
+                keep(pair[l][0][0]), keep(pair[l][0][1]), keep(pair[l][1][0]), keep(pair[l][1][1]);
+                const v2u first = pair[l][0][0] ^ pair[l][0][1], second = pair[l][1][0] ^ pair[l][1][1];
+                weight[0][j + l] = v4i{(int)first[0], (int)first[1], (int)second[0], (int)second[1]};
+            }
         }
 
         // One chunk: two steps of 64.  In front of its last phase the workgroup meets once: chunk t + 1 has landed,
         // everybody has read chunk t, and the requests of chunk t + 2 go out into its slot and its code registers.
         auto chunk_step = [&](int t, auto set_tag) {
             constexpr int SET = decltype(set_tag)::value;
-            const uint32_t here = frag + (uint32_t)SET * kSlot, there = frag + (uint32_t)(1 - SET) * kSlot;
+            std::integral_constant<int, 1 - SET> other;
             auto meet = [&]() {
                 asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
                 __builtin_amdgcn_sched_barrier(0);
             };
             auto request = [&]() { issue_codes(t + 2, set_tag), issue_tokens(t + 2, SET); };
             if constexpr (PHASES == 4) {
-                phase(zero, zero, here, codes[SET], nothing);
-                phase(zero, one, here, codes[SET], nothing);
-                phase(zero, two, here, codes[SET], nothing);
-                phase(zero, three, here ^ 64u, codes[SET], nothing);
+                phase(zero, zero, set_tag, frag, codes[SET], nothing);
+                phase(zero, one, set_tag, frag, codes[SET], nothing);
+                phase(zero, two, set_tag, frag, codes[SET], nothing);
+                phase(zero, three, set_tag, frag_half, codes[SET], nothing);
             } else {
-                phase(zero, zero, here, codes[SET], nothing);
-                phase(zero, one, here ^ 64u, codes[SET], nothing);
+                phase(zero, zero, set_tag, frag, codes[SET], nothing);
+                phase(zero, one, set_tag, frag_half, codes[SET], nothing);
             }
             // the codes of chunk t + 1 are older than its token rows
             asm volatile("s_waitcnt vmcnt(%4)"
@@ -262,15 +272,15 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
                          : "n"(LOADS));
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (PHASES == 4) {
-                phase(one, zero, here ^ 64u, codes[1 - SET], nothing);
-                phase(one, one, here ^ 64u, codes[1 - SET], nothing);
-                phase(one, two, here ^ 64u, codes[1 - SET], nothing);
+                phase(one, zero, set_tag, frag_half, codes[1 - SET], nothing);
+                phase(one, one, set_tag, frag_half, codes[1 - SET], nothing);
+                phase(one, two, set_tag, frag_half, codes[1 - SET], nothing);
                 meet();
-                phase(one, three, there, codes[1 - SET], request);
+                phase(one, three, other, frag, codes[1 - SET], request);
             } else {
-                phase(one, zero, here ^ 64u, codes[1 - SET], nothing);
+                phase(one, zero, set_tag, frag_half, codes[1 - SET], nothing);
                 meet();
-                phase(one, one, there, codes[1 - SET], request);
+                phase(one, one, other, frag, codes[1 - SET], request);
             }
         };
         int t = 0;
@@ -286,77 +296,91 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
                      :
                      : "memory");
 
-        // ---- epilogue: a lane holds four consecutive channels of one slot in every block.  One swap of the odd rows of 16
-        // lanes of block j with the even rows of block j + 1 leaves a lane with 16 contiguous bytes of one output row ----
+        // ---- epilogue: a lane holds four consecutive channels of one slot in every block.  Stored from there, every instruction touches 16
+        // rows in an order that leaves each lane an access of its own, more than a hundred cycles apiece (128 slots of 64
+        // channels to a wave: 11300 cycles beside 9800 of the whole K loop at K = 512).  So a block of 16 rows goes through LDS, where
+        // the token rows were and private to the wave, and leaves with neighbouring lanes beside each other in a row ----
+        asm volatile("s_barrier" ::: "memory");  // nobody's token rows are on their way any more
         if (!live_wave) return;
         int own = threadIdx.x & 63;
         asm volatile("" : "+v"(own));  // nothing of the addresses below is carried through the K loop
-        const int quarter = own >> 4;
-        const float* const token_scales = reinterpret_cast<const float*>(lds + kTokenScale);
-        const float* const channel_scales = reinterpret_cast<const float*>(lds + kChannelScale) + wave * 64;
-        auto store_pair = [&](bool live, __half* row_out, const uint32_t (&first_words)[2], const uint32_t (&second_words)[2]) {
-            const v2u l = __builtin_amdgcn_permlane16_swap(first_words[0], second_words[0], false, false);
-            const v2u h = __builtin_amdgcn_permlane16_swap(first_words[1], second_words[1], false, false);
-            if (!live) return;
-            row_out += (quarter & 1) * 16 + (quarter >> 1) * 8;
-            const uint4 piece = make_uint4(l[0], h[0], l[1], h[1]);
-            if ((reinterpret_cast<uintptr_t>(row_out) & 15) == 0) {
-                *reinterpret_cast<uint4*>(row_out) = piece;
-            } else {  // an output buffer may be aligned to its elements only
-                const uint32_t words[4] = {piece.x, piece.y, piece.z, piece.w};
+        const int quarter = own >> 4, column = own & 15;
+        // the scales once, into registers: read where they are used, behind each write of a row, every value waited for an LDS read of its own
+        // (13000 of the 29000 cycles of a unit of down)
+        float token_scale[NB];
+        float4 channel_scale[4];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) row_out[e] = __ushort_as_half((unsigned short)(words[e >> 1] >> (16 * (e & 1))));
+        for (int i = 0; i < NB; ++i) token_scale[i] = reinterpret_cast<const float*>(lds + kTokenScale)[i * 16 + column];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            channel_scale[j] = *reinterpret_cast<const float4*>(lds + kChannelScale + (wave * 64 + j * 16 + 4 * quarter) * 4);
+        constexpr int kWidth = SWIGLU ? 64 : 128, kPitch = kWidth + 16, kLanes = kWidth / 16, kRowsAtOnce = 64 / kLanes;  // bytes of a row; lanes to a row
+        uint8_t* const image = lds + kTokens + wave * 8192;  // two blocks of 16 rows
+        static_assert(2 * 16 * kPitch <= 8192, "the images of four waves fit where two chunks were");
+        __half* const rows_out = (SWIGLU ? p.act : p.out) + (int64_t)row0 * (SWIGLU ? inner : p.n) + n0;
+        const int row_stride = SWIGLU ? inner : p.n;
+        const bool aligned = ((reinterpret_cast<uintptr_t>(rows_out) | (uintptr_t)row_stride * 2) & 15) == 0;  // (a buffer may be aligned to its elements only)
+        auto store_block = [&](int i) {
+            const uint8_t* const from = image + (i & 1) * (16 * kPitch);
+#pragma unroll
+            for (int h = 0; h < 16 / kRowsAtOnce; ++h) {
+                const int row = h * kRowsAtOnce + own / kLanes, local = i * 16 + row;
+                const uint4 piece = *reinterpret_cast<const uint4*>(from + row * kPitch + own % kLanes * 16);
+                if (local >= rows) continue;
+                __half* const to = rows_out + (int64_t)local * row_stride + own % kLanes * 8;
+                if (aligned) {
+                    *reinterpret_cast<uint4*>(to) = piece;
+                } else {
+                    const uint32_t words[4] = {piece.x, piece.y, piece.z, piece.w};
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) to[e] = __ushort_as_half((unsigned short)(words[e >> 1] >> (16 * (e & 1))));
+                }
             }
         };
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
-            const int local = i * 16 + (own & 15);
+            const int local = i * 16 + column;
             const bool live = local < rows;
-            const float token_scale = token_scales[local];
             const int64_t slot = row0 + local;
-            auto value = [&](int j, int r) {
-                return __float2half_rn(rescale(acc[i][j][r], channel_scales[j * 16 + 4 * quarter + r], token_scale));
+            uint8_t* const to = image + (i & 1) * (16 * kPitch) + column * kPitch + quarter * 8;
+            auto values = [&](int j) {  // of four channels, rounded to fp16 once
+                return make_uint2(pack_halves(rescale(acc[i][j][0], channel_scale[j].x, token_scale[i]), rescale(acc[i][j][1], channel_scale[j].y, token_scale[i])),
+                                  pack_halves(rescale(acc[i][j][2], channel_scale[j].z, token_scale[i]), rescale(acc[i][j][3], channel_scale[j].w, token_scale[i])));
             };
             if constexpr (!SWIGLU) {
 #pragma unroll
-                for (int pair = 0; pair < 2; ++pair) {
-                    uint32_t words[2][2];
-#pragma unroll
-                    for (int e = 0; e < 2; ++e)
-                        words[e][0] = pack2(value(2 * pair + e, 0), value(2 * pair + e, 1)),
-                        words[e][1] = pack2(value(2 * pair + e, 2), value(2 * pair + e, 3));
-                    store_pair(live, p.out + slot * p.n + n0 + 32 * pair, words[0], words[1]);
-                }
+                for (int j = 0; j < 4; ++j) *reinterpret_cast<uint2*>(to + j * 32) = values(j);
             } else {
-                uint32_t words[2][2];
                 const bool maxima = p.row_max != nullptr;
                 float amax = 0.f;
 #pragma unroll
                 for (int e = 0; e < 2; ++e) {
-                    __half gate[4], up[4], product[4];
+                    const uint2 gate = values(e), up = values(e + 2);
+                    const uint32_t gates[2] = {gate.x, gate.y}, ups[2] = {up.x, up.y};
+                    float v[4];
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        gate[r] = value(e, r), up[r] = value(e + 2, r);
-                        const float v = swiglu_value(gate[r], up[r]);
-                        product[r] = __float2half_rn(v);
-                        if (maxima) amax = fmaxf(amax, fabsf(v));
+                        auto half_of = [&](const uint32_t(&words)[2]) { return __ushort_as_half((unsigned short)(words[r >> 1] >> (16 * (r & 1)))); };
+                        v[r] = swiglu_value(half_of(gates), half_of(ups));
+                        if (maxima) amax = fmaxf(amax, fabsf(v[r]));
                     }
-                    words[e][0] = pack2(product[0], product[1]), words[e][1] = pack2(product[2], product[3]);
+                    *reinterpret_cast<uint2*>(to + e * 32) = make_uint2(pack_halves(v[0], v[1]), pack_halves(v[2], v[3]));
                     if (live && p.out != nullptr) {
                         __half* dst = p.out + slot * p.n + n0 + 16 * e + 4 * quarter;
-                        *reinterpret_cast<uint2*>(dst) = make_uint2(pack2(gate[0], gate[1]), pack2(gate[2], gate[3]));
-                        *reinterpret_cast<uint2*>(dst + inner) = make_uint2(pack2(up[0], up[1]), pack2(up[2], up[3]));
+                        *reinterpret_cast<uint2*>(dst) = gate;
+                        *reinterpret_cast<uint2*>(dst + inner) = up;
                     }
                 }
-                store_pair(live, p.act + slot * inner + n0, words[0], words[1]);
                 if (maxima) {
                     amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
                     amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
                     if (live && quarter == 0) atomicMax(p.row_max + slot, __float_as_int(amax));
                 }
             }
+            if (i > 0) store_block(i - 1);
             __builtin_amdgcn_sched_barrier(0);
         }
+        store_block(NB - 1);
     };
     if (rows > 64)
         run(std::integral_constant<int, 8>{});

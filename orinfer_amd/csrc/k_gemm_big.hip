@@ -110,16 +110,7 @@ struct TileState {
     int row0, col0, rows_here, cols_here;
 };
 
-typedef float v2f __attribute__((ext_vector_type(2)));
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef unsigned int v2u __attribute__((ext_vector_type(2)));
-
-// two fp32 values rounded to nearest even and packed (one v_cvt_pk_f16_f32)
-__device__ __forceinline__ uint32_t pack_halves(float low, float high) {
-    const v2f pair = {low, high};
-    const v2h rounded = __builtin_convertvector(pair, v2h);
-    return *reinterpret_cast<const uint32_t*>(&rounded);
-}
 
 // The four fragments pass through the statement, so no multiply that uses them can move in front of the wait: at
 // most N younger LDS requests of this wave may still be in flight behind them (they complete in order).
