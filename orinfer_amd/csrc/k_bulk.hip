@@ -19,9 +19,11 @@
 //    as many conflict cycles again, and sixteen copies of each leave room for one workgroup per CU.
 // Measured at 4096 tokens x top-8 of 128 experts (H = 2048, I = 512; popularity of the experts like 1 / rank^1.1):
 // gate_up 296 -> 100 us, down 215 -> 67 us.  What bounds it now: the loop, where two waves of a SIMD keep its matrix pipe busy
-// in 0.85 of the cycles, is 9800 of the 21000 cycles of a unit of down and 38000 of 57000 of gate_up; set-up (two dependent reads of
-// the tile lists, tables, first chunks) takes 5400, the epilogue 4600 and, with the SwiGLU's sixteen instructions a sigmoid, 11000; and
-// units of 35 us that start late leave CUs idle at the end of gate_up.
+// in 0.85 of the cycles, is 9800 of the 21000 cycles of a unit of down and 38000 of 57000 of gate_up; set-up (tile, tables, first
+// chunks) takes 5200, the epilogue 4600 and, with the SwiGLU's sixteen instructions a sigmoid, 11000.
+// With tile units the tiles come largest first and in one read: a unit of gate_up takes 30 us, and in the order of the experts the
+// last ones started when most of the chip was done (gate_up 97-107 -> 96 us over three routings, down 71-77 -> 70; the layer at 2000
+// tokens 140.7 -> 133.1 us over eight, at 4096, where two whole rounds are full, 229.6 -> 228.7).
 // One persistent workgroup of eight waves per CU that requests the next unit's chunks early measured 118 and 75 us.
 // A workgroup that takes 2, 4 or 8 spans of a tile in a row, the next one's chunks requested in the last steps, and 512
 // persistent workgroups of this form with even shares both measured level or slower (whole layer 227 / 241 / 247 and 243 against
@@ -67,6 +69,7 @@ struct BulkParams {
     const int* tile_expert;
     const int* tile_row;
     const int* tile_count;
+    const int4* tile_units;  // or null
     int n, k, tile_capacity, spans;
 };
 
@@ -83,13 +86,19 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
     uint32_t selector;
     asm volatile("global_load_dword %0, %1, %2" : "=v"(selector) : "v"((uint32_t)tid * 4), "s"(uniform_pointer(p.book)) : "memory");
     // the list's length and its entry in one trip; behind the end an entry is whatever the buffer holds
-    const int listed = p.tile_count[0], listed_expert = p.tile_expert[tile], listed_row = p.tile_row[tile];
-    if (tile >= listed) return;
-    const int expert = __builtin_amdgcn_readfirstlane(listed_expert);
-    const int first = __builtin_amdgcn_readfirstlane(listed_row);
-    const int rows = __builtin_amdgcn_readfirstlane(min(kTileRows, p.counts[expert] - first));
+    const int listed = p.tile_count[0];
+    int expert, rows, row0;
+    if (p.tile_units != nullptr) {
+        const int4 unit = p.tile_units[tile];
+        if (tile >= listed) return;
+        expert = unit.x, row0 = unit.y, rows = min(kTileRows, unit.z);
+    } else {
+        const int listed_expert = p.tile_expert[tile], first = p.tile_row[tile];
+        if (tile >= listed) return;
+        expert = listed_expert, rows = min(kTileRows, p.counts[expert] - first), row0 = p.offsets[expert] + first;
+    }
+    expert = __builtin_amdgcn_readfirstlane(expert), rows = __builtin_amdgcn_readfirstlane(rows), row0 = __builtin_amdgcn_readfirstlane(row0);
     if (rows <= 0) return;
-    const int row0 = __builtin_amdgcn_readfirstlane(p.offsets[expert] + first);
     const int inner = p.n / 2;
     const int chunks = p.k / 128;
 
@@ -428,7 +437,7 @@ int grouped_bulk_launch(const GroupedBuffers& b, int n, int k, int tiles, bool g
     p.out = reinterpret_cast<__half*>(b.out), p.act = reinterpret_cast<__half*>(b.act);
     p.row_max = swiglu ? const_cast<int*>(b.row_max) : nullptr;
     p.counts = b.counts, p.offsets = b.offsets, p.tile_expert = b.tile_expert, p.tile_row = b.tile_row;
-    p.tile_count = b.tile_count;
+    p.tile_count = b.tile_count, p.tile_units = static_cast<const int4*>(b.tile_units);
     p.n = n, p.k = k, p.tile_capacity = tiles;
     p.spans = (int)(swiglu ? ceil_div((uint32_t)n / 2, kSpan / 2) : ceil_div((uint32_t)n, kSpan));
     const dim3 grid(g.grid[0]), block(kThreads);

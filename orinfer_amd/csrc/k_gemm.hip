@@ -1730,6 +1730,7 @@ int grouped_launch(const orx_function& f, int rows, const Geometry& g, hipStream
     b.tile_row = reinterpret_cast<const int*>(buffer("TileRow")), b.ws = buffer("WS");
     b.slot_token = reinterpret_cast<const int*>(buffer("SlotToken"));
     b.row_max = reinterpret_cast<const int*>(buffer("RowMax")), b.act = buffer("Act"), b.q = buffer("Q");
+    b.tile_units = buffer("TileUnits");
     if (grouped_uses_bulk(f))
         return grouped_bulk_launch(b, f.N, f.K, f.tiles, (f.flags2 & 3) == 1, (f.flags2 >> 2) == 1, stream);
     if (grouped_uses_resident(f))
@@ -1765,6 +1766,7 @@ int make_q2_grouped(const Variant& v, orx_function* f) {
     const std::string grouped_algorithm = v.string("algorithm", "auto", &bad);
     const std::string input = v.string("input_dtype", "int8", &bad);
     const bool gather = v.boolean("gather", false, &bad);
+    const bool tile_units = f->symbol == "e8p_decode_grouped" && v.boolean("tile_units", false, &bad);
     const std::string epilogue = v.string("epilogue", "none", &bad);
     // integer_vq_grouped carries the reference's Patch buffer and its decoder options (integer_vq.py:217-258)
     const bool vq = f->symbol == "integer_vq_grouped";
@@ -1858,6 +1860,11 @@ int make_q2_grouped(const Variant& v, orx_function* f) {
     // All three are forms of the resident kernel: served where `auto` picks it, or by name.  Lists of 128-row tiles have the
     // first two on the bulk kernel, which needs no RowMax (it may be null: the rows are quantised by a launch of their own).
     const bool bulk = grouped_uses_bulk(*f);
+    // tile_units=true: TileUnits, as route_metadata lists them, in place of TileExpert, TileRow, Counts and Offsets (which stay in the list)
+    if (tile_units && !bulk) {
+        set_error("%s: tile_units is a form of the kernel that takes lists of 128-row tiles", name);
+        return ORX_ERR_BAD_VARIANT;
+    }
     if (f->flags2 != 0 && !bulk) {
         if ((f->algorithm != kAuto && f->algorithm != kResident) ||
             !grouped_resident_eligible(f->N, f->K, f->block_m, f->tiles, f->flags2 & 3, f->flags2 >> 2, f->capacity) ||
@@ -1887,6 +1894,7 @@ int make_q2_grouped(const Variant& v, orx_function* f) {
         f->args.push_back({"TileCount", ArgPointer, 4});
         f->args.push_back({"TileExpert", ArgPointer, 4});
         f->args.push_back({"TileRow", ArgPointer, 4});
+        if (tile_units) f->args.push_back({"TileUnits", ArgPointer, 16});
         f->args.push_back({"WS", ArgPointer, 2});
         if (f->dynamic_rows) f->args.push_back({"m", ArgI32, 4});
     }
@@ -2149,8 +2157,8 @@ const Registration* gemm_registrations(int* count) {
     {"int8_swiglu", make_int8_swiglu, "M, N, K, dynamic_rows=false, algorithm=tensor_core|dp4a, block_m, block_n (checked, not used)",
      "A,Gate,GateScale,Output,TokenScale,Up,UpScale[,m]"},
     {"e8p_decode_grouped", make_q2_grouped,
-     "rows, E, tiles, N, K, block_m=32|64|128|8|16 (row step of the tile list), packed_k=128|64|0, dynamic_rows=false, algorithm=auto|stream|resident|mfma, input_dtype=int8|float16, gather=false, epilogue=none|swiglu",
-     "A,AS[,Act],Book,C,Counts,Offsets,P[,Q][,RowMax][,SlotToken],TileCount,TileExpert,TileRow,WS[,m]"},
+     "rows, E, tiles, N, K, block_m=32|64|128|8|16 (row step of the tile list), packed_k=128|64|0, dynamic_rows=false, algorithm=auto|stream|resident|mfma, input_dtype=int8|float16, gather=false, epilogue=none|swiglu, tile_units=false",
+     "A,AS[,Act],Book,C,Counts,Offsets,P[,Q][,RowMax][,SlotToken],TileCount,TileExpert,TileRow[,TileUnits],WS[,m]"},
     {"integer_vq", make_vq_direct,
      "E, M (rows of every expert), N, K, block_m=16|8|32|64, packed_k=128|64|0, patched=false, shared_table=false, shortbook=false, "
      "selectorbook=false (Book: raw basis (256,2) | signed values (512,4) with shortbook | selector words (256,1) with both)",

@@ -489,9 +489,10 @@ __global__ __launch_bounds__(kMetaThreads) void segment_rank_kernel(const int* _
 __global__ __launch_bounds__(kMetaThreads) void segment_place_kernel(
     const int* __restrict__ ids, const int* __restrict__ segments, int* __restrict__ counts, int* __restrict__ relative,
     int* __restrict__ row_offsets, int* __restrict__ tile_count, int* __restrict__ tile_expert, int* __restrict__ tile_offsets,
-    int* __restrict__ tile_row, int* __restrict__ slot_map, int* __restrict__ slot_token, int* __restrict__ row_max,
-    int assignments, int experts, int top_k, int block_m) {
+    int* __restrict__ tile_row, int4* __restrict__ tile_units, int* __restrict__ slot_map, int* __restrict__ slot_token,
+    int* __restrict__ row_max, int assignments, int experts, int top_k, int block_m) {
     __shared__ int in_front[kMetaThreads], first_row[kMetaThreads], wave_rows[kMetaWaves], wave_tiles[kMetaWaves];
+    __shared__ int wave_large[kMetaWaves], wave_small[kMetaWaves];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int segment = blockIdx.x, total_segments = gridDim.x;
     const int at = segment * kSegment + tid;
@@ -508,24 +509,35 @@ __global__ __launch_bounds__(kMetaThreads) void segment_place_kernel(
         in_front[tid] = before;
     }
     const int tiles = (count + block_m - 1) / block_m;
-    int row_scan = count, tile_scan = tiles;
+    // Units: the tiles in the order of their size, so that what starts last is short: above half a tile's rows, above a quarter, the rest
+    // (an expert's last tile is the only one that is not full; tiles of the two small sizes are counted in the halves of a word)
+    const int full = count / block_m, rest = count % block_m;
+    const int size = 2 * rest > block_m ? 0 : 4 * rest > block_m ? 1 : 2;  // of the last tile
+    const int large = full + (rest > 0 && size == 0), small = rest > 0 && size > 0 ? 1 << (16 * (size - 1)) : 0;
+    int row_scan = count, tile_scan = tiles, large_scan = large, small_scan = small;
 #pragma unroll
     for (int offset = 1; offset < 64; offset <<= 1) {
         const int r = __shfl_up(row_scan, offset, 64), t = __shfl_up(tile_scan, offset, 64);
-        if (lane >= offset) row_scan += r, tile_scan += t;
+        const int l = __shfl_up(large_scan, offset, 64), m = __shfl_up(small_scan, offset, 64);
+        if (lane >= offset) row_scan += r, tile_scan += t, large_scan += l, small_scan += m;
     }
-    if (lane == 63) wave_rows[wave] = row_scan, wave_tiles[wave] = tile_scan;
+    if (lane == 63) wave_rows[wave] = row_scan, wave_tiles[wave] = tile_scan, wave_large[wave] = large_scan, wave_small[wave] = small_scan;
     __syncthreads();
-    int row_base = 0, tile_base = 0, tile_total = 0;
+    int row_base = 0, tile_base = 0, tile_total = 0, large_base = 0, large_total = 0, small_base = 0, small_total = 0;
     for (int w = 0; w < kMetaWaves; ++w) {
-        if (w < wave) row_base += wave_rows[w], tile_base += wave_tiles[w];
-        tile_total += wave_tiles[w];
+        if (w < wave) row_base += wave_rows[w], tile_base += wave_tiles[w], large_base += wave_large[w], small_base += wave_small[w];
+        tile_total += wave_tiles[w], large_total += wave_large[w], small_total += wave_small[w];
     }
     if (tid < experts) {
         const int row = row_base + row_scan - count, tile = tile_base + tile_scan - tiles;
         first_row[tid] = row;
         if (segment == 0) counts[tid] = count, row_offsets[tid] = row, tile_offsets[tid] = tile;
-        for (int t = segment; t < tiles; t += total_segments) tile_expert[tile + t] = tid, tile_row[tile + t] = t * block_m;
+        const int first_large = large_base + large_scan - large, smalls = small_base + small_scan - small;
+        const int at_rest = size == 0 ? first_large + full : large_total + (size == 1 ? smalls & 0xFFFF : (small_total & 0xFFFF) + (smalls >> 16));
+        for (int t = segment; t < tiles; t += total_segments) {
+            tile_expert[tile + t] = tid, tile_row[tile + t] = t * block_m;
+            if (tile_units != nullptr) tile_units[t < full ? first_large + t : at_rest] = make_int4(tid, row + t * block_m, t < full ? block_m : rest, 0);
+        }
     }
     if (segment == 0 && tid == 0) tile_count[0] = tile_total;
     __syncthreads();
@@ -992,8 +1004,8 @@ int make_tiles(const Variant& v, orx_function* f) {
     return ORX_OK;
 }
 
-// flags: bit0 slot_maps, bit1 segments (workspace=true: any number of assignments, two launches)
-enum { kSlotMaps = 1, kSegments = 2 };
+// flags: bit0 slot_maps, bit1 segments (workspace=true: any number of assignments, two launches), bit2 tile_units
+enum { kSlotMaps = 1, kSegments = 2, kTileUnits = 4 };
 uint64_t metadata_workspace(const orx_function& f, int rows) {
     return (uint64_t)ceil_div((uint32_t)rows * (uint32_t)f.top_k, (uint32_t)kSegment) * (uint32_t)f.E * sizeof(int);
 }
@@ -1032,7 +1044,7 @@ int metadata_launch(const orx_function& f, int rows, const Geometry& g, hipStrea
         ORX_LAUNCH(segment_place_kernel, dim3(g.grid[0]), dim3(kMetaThreads), 0, s, ids, segments, pointer_arg<int>(args, 0),
                    relative, pointer_arg<int>(args, offsets_at), pointer_arg<int>(args, tiles_at),
                    pointer_arg<int>(args, tiles_at + 1), pointer_arg<int>(args, tiles_at + 2), pointer_arg<int>(args, tiles_at + 3),
-                   pointer_arg<int>(args, 5), pointer_arg<int>(args, 6), pointer_arg<int>(args, 3), rows * f.top_k, f.E, f.top_k,
+                   f.flags & kTileUnits ? pointer_arg<int4>(args, tiles_at + 4) : nullptr, pointer_arg<int>(args, 5), pointer_arg<int>(args, 6), pointer_arg<int>(args, 3), rows * f.top_k, f.E, f.top_k,
                    f.block_m);
         return hip_check(hipGetLastError(), "launch route_metadata");
     }
@@ -1057,13 +1069,19 @@ int make_metadata(const Variant& v, orx_function* f) {
         set_error("route_metadata: workspace=true goes with slot_maps=true and at most 2^30 assignments");
         return ORX_ERR_BAD_VARIANT;
     }
+    // tile_units=true (with workspace): TileUnits (tiles, 4) int32 lists the tiles largest first: expert, first row of the sorted slots, rows, 0
+    const bool tile_units = v.boolean("tile_units", false, &bad);
+    if (bad || (tile_units && !f->takes_workspace)) {
+        set_error("route_metadata: tile_units goes with workspace=true");
+        return ORX_ERR_BAD_VARIANT;
+    }
     // one expert per thread, one route per lane; the reference's own form is decode-only (M <= 1024)
     if (f->M <= 0 || f->E <= 0 || f->E > kMetaThreads || f->top_k <= 0 || f->top_k > f->E || !valid_block_m(f->block_m) ||
         (!f->takes_workspace && (size_t)(kMetaWaves * f->E + 2 * kMetaWaves + 2 * (size_t)f->M * f->top_k) * sizeof(int) > 160 * 1024)) {
         set_error("route_metadata: need E <= 1024, top_k <= E, a valid block_m and M*top_k small enough for LDS");
         return ORX_ERR_BAD_VARIANT;
     }
-    f->flags = (slot_maps ? kSlotMaps : 0) | (f->takes_workspace ? kSegments : 0);
+    f->flags = (slot_maps ? kSlotMaps : 0) | (f->takes_workspace ? kSegments : 0) | (tile_units ? kTileUnits : 0);
     f->args = {{"Counts", ArgPointer, 4}, {"IDs", ArgPointer, 4}, {"RelativeSlot", ArgPointer, 4}};
     if (slot_maps) f->args.push_back({"RowMax", ArgPointer, f->takes_workspace ? 0x80000004u : 4u});
     f->args.push_back({"RowOffsets", ArgPointer, 4});
@@ -1071,6 +1089,7 @@ int make_metadata(const Variant& v, orx_function* f) {
     for (const ArgSpec& a : std::initializer_list<ArgSpec>{{"TileCount", ArgPointer, 4}, {"TileExpert", ArgPointer, 4},
                                                            {"TileOffsets", ArgPointer, 4}, {"TileRow", ArgPointer, 4}})
         f->args.push_back(a);
+    if (tile_units) f->args.push_back({"TileUnits", ArgPointer, 16});
     if (f->takes_workspace) f->args.push_back({"Workspace", ArgPointer, 256u | 0x80000000u}), f->workspace_need = metadata_workspace;
     if (f->dynamic_rows) f->args.push_back({"m", ArgI32, 4});
     f->geometry = metadata_geometry;
@@ -1284,8 +1303,8 @@ const Registration* moe_registrations(int* count) {
      "IDs,Offsets,Slots[,m]"},
     {"expert_offsets", make_offsets, "E=512, block_m=16", "Counts,RowOffsets,TileCount,TileOffsets"},
     {"expert_tiles", make_tiles, "M, E=512, top_k=10, block_m=16", "Counts,TileExpert,TileOffsets,TileRow"},
-    {"route_metadata", make_metadata, "M, E=512, top_k=10, block_m=8, dynamic_rows=false, slot_maps=false, workspace=false",
-     "Counts,IDs,RelativeSlot[,RowMax],RowOffsets[,SlotMap,SlotToken],TileCount,TileExpert,TileOffsets,TileRow[,Workspace][,m]"},
+    {"route_metadata", make_metadata, "M, E=512, top_k=10, block_m=8, dynamic_rows=false, slot_maps=false, workspace=false, tile_units=false",
+     "Counts,IDs,RelativeSlot[,RowMax],RowOffsets[,SlotMap,SlotToken],TileCount,TileExpert,TileOffsets,TileRow[,TileUnits][,Workspace][,m]"},
     {"single_route_metadata", make_single_metadata, "E=512, top_k=10, capacity=11",
      "Counts,IDs,Offsets,Relative,TileCount,TileExpert,TileOffsets,TileRow"},
     {"expert_partition_offsets", make_partition_offsets, "experts, hot_m, cold_m, cold_rows",

@@ -243,7 +243,7 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
             Each<CB>::run([&](auto j_tag) ORX_INLINE {
                 constexpr int j = decltype(j_tag)::value, before = (j + CB - 1) % CB;
                 constexpr int kSet = CB == 1 ? 0 : (HALF * CB + j) & 1, kHeld = CB == 1 ? 0 : 1 - kSet;
-                constexpr int kTokensHere = CB == 1 ? TB : j < CB - 1 ? (TB - j + CB - 2) / (CB - 1) : 0;  // i with i % (CB - 1) == j
+                constexpr int kTokensHere = CB == 1 ? TB : j < CB - 1 ? (TB - j + CB - 2) / (CB > 1 ? CB - 1 : 1) : 0;  // i with i % (CB - 1) == j
                 std::integral_constant<int, kSet> set;
                 std::integral_constant<int, kHeld> held;
                 Each<TB>::run([&](auto i_tag) ORX_INLINE {

@@ -157,6 +157,7 @@ struct GroupedBuffers {
     const int* tile_expert = nullptr;
     const int* tile_row = nullptr;
     const int* tile_count = nullptr;
+    const void* tile_units = nullptr;  // int4 per tile, largest first: expert, first slot, rows (128-row tiles; null: the lists above)
     const int* slot_token = nullptr;  // gathered rows: token of every slot
     const int* row_max = nullptr;     // fp32 bits of every slot's largest magnitude: read with fp16 rows, raised by the SwiGLU epilogue
     void* act = nullptr;              // SwiGLU epilogue: fp16 (slots, N/2)

@@ -201,14 +201,16 @@ class MoeLayer:
                 and not one_launch_refused and packed_k == 128 and experts <= 1024 and grouped_algorithm == "auto" and assignments >= BULK_ROWS_PER_EXPERT * experts):
             try:
                 tiles = (assignments + BULK_ROWS - 1) // BULK_ROWS + min(experts, assignments)
-                bulk = dict(rows=assignments, E=experts, tiles=tiles, block_m=BULK_ROWS)
+                bulk = dict(rows=assignments, E=experts, tiles=tiles, block_m=BULK_ROWS, tile_units=True)
                 self.k_router_a8 = Kernel("router_topk", renormalize=True, quantize_hidden=hidden, **common)
-                self.k_metadata_slots = Kernel("route_metadata", block_m=BULK_ROWS, slot_maps=True, workspace=True, **common)
+                self.k_metadata_slots = Kernel("route_metadata", block_m=BULK_ROWS, slot_maps=True, workspace=True,
+                                               tile_units=True, **common)
                 self.k_gate_up_bulk = Kernel("e8p_decode_grouped", N=2 * intermediate, K=hidden, gather=True,
                                              epilogue="swiglu", **bulk)
                 self.k_act_a8 = Kernel("activation_quantization", K=intermediate)
                 self.k_down_bulk = Kernel("e8p_decode_grouped", N=hidden, K=intermediate, **bulk)
                 self.segments = self.k_metadata_slots.workspace()
+                self.tile_units = torch.empty((tiles, 4), **i32)
                 self.slot_token = torch.empty(assignments, **i32)
                 self.act = torch.empty((assignments, intermediate), **f16)
                 if tiles > self.tile_capacity:
@@ -267,9 +269,9 @@ class MoeLayer:
         self.k_metadata_slots(stream=s, Counts=self.counts, IDs=self.ids, RelativeSlot=self.relative, RowMax=None,
                               RowOffsets=self.row_offsets, SlotMap=self.slot_map, SlotToken=self.slot_token,
                               TileCount=self.tile_count, TileExpert=self.tile_expert, TileOffsets=self.tile_offsets,
-                              TileRow=self.tile_row, Workspace=self.segments)
+                              TileRow=self.tile_row, TileUnits=self.tile_units, Workspace=self.segments)
         routed = dict(Book=self.book, Counts=self.counts, Offsets=self.row_offsets, TileCount=self.tile_count,
-                      TileExpert=self.tile_expert, TileRow=self.tile_row)
+                      TileExpert=self.tile_expert, TileRow=self.tile_row, TileUnits=self.tile_units)
         self.k_gate_up_bulk(stream=s, A=self.a_q, AS=self.a_s, Act=self.act, C=None, P=self.w1, RowMax=None,
                             SlotToken=self.slot_token, WS=self.s1, **routed)
         self.k_act_a8(stream=s, Mask=None, Q=self.h_q, S=self.h_s, X=self.act, rows=self.assignments)

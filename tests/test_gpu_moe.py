@@ -145,6 +145,32 @@ def test_route_metadata_in_segments(m, e, k, bm):
     kern(IDs=gu.dev(padded), m=m, **{**out, "RowMax": None})
 
 
+# Last tiles of every size, full ones only, none at all, more experts than a wave, segments of less than and more than one workgroup.
+@pytest.mark.parametrize("counts,bm", [([128, 0, 1, 129, 64, 65, 32, 33, 300, 0], 128), ([256, 512], 128), ([17, 16, 8, 9, 40, 4, 5], 16),
+                                       ([3] * 100 + [200] * 20 + [70] * 30, 128), ([1], 128)])
+def test_route_metadata_lists_tiles_largest_first(counts, bm):
+    counts = np.array(counts, np.int32)
+    e, m = len(counts), int(counts.sum())
+    rng = np.random.default_rng(orc.SEED + m)
+    ids = rng.permutation(np.repeat(np.arange(e, dtype=np.int32), counts)).reshape(m, 1)
+    cap = orc.tile_capacity(m, e, bm)
+    kern = gu.kernel("route_metadata", M=m, E=e, top_k=1, block_m=bm, slot_maps=True, workspace=True, tile_units=True)
+    out = {name: torch.full(shape, -1, **I32) for name, shape in
+           (("Counts", (e,)), ("RelativeSlot", (m, 1)), ("RowOffsets", (e,)), ("TileCount", (1,)), ("TileExpert", (cap,)), ("TileOffsets", (e,)),
+            ("TileRow", (cap,)), ("SlotMap", (m, 1)), ("SlotToken", (m,)), ("TileUnits", (cap, 4)))}
+    kern(IDs=gu.dev(ids), RowMax=None, **out)
+    total = int(gu.host(out["TileCount"])[0])
+    units = gu.host(out["TileUnits"])
+    assert (units[total:] == -1).all()
+    offsets = gu.host(out["RowOffsets"])
+    size = lambda rows: 0 if 2 * rows > bm else 1 if 4 * rows > bm else 2
+    tiles = [(expert, offsets[expert] + first, min(bm, counts[expert] - first), 0) for expert in range(e) for first in range(0, counts[expert], bm)]
+    want = sorted(tiles, key=lambda unit: size(unit[2]))  # (stable: by expert within a size)
+    np.testing.assert_array_equal(units[:total], np.array(want, np.int32).reshape(-1, 4))
+    with pytest.raises(gu.lib.OrxError):
+        gu.kernel("route_metadata", M=m, E=e, top_k=1, block_m=bm, slot_maps=True, tile_units=True)
+
+
 @pytest.mark.parametrize("algorithm", ["auto", "mfma"])
 @pytest.mark.parametrize("packed_k", [128, 64, 0])
 @pytest.mark.parametrize("bm", [32, 64, 128])
@@ -317,6 +343,39 @@ def test_grouped_q2_bulk_kernel(n, k, counts, form):
     lean = torch.full_like(act, 55.0)
     kern(Act=lean, RowMax=None, SlotToken=gu.dev(source), **{**args, "C": None})
     assert torch.equal(lean, act)
+
+
+@pytest.mark.parametrize("swiglu", [False, True], ids=["rows", "gathered-swiglu"])
+def test_grouped_q2_bulk_kernel_takes_its_tiles_from_units(swiglu):
+    """The same rows whether a tile comes out of TileExpert, TileRow, Counts and Offsets or out of TileUnits in any order."""
+    rng = np.random.default_rng(orc.SEED + swiglu)
+    counts = np.array([130, 0, 64, 33, 256, 1, 90], np.int32)
+    e, n, k, bm, rows, tokens = len(counts), 384, 512, 128, int(counts.sum()), 50
+    offsets, tile_offsets, total = orc.expert_offsets(counts, bm)
+    cap = orc.tile_capacity(rows, e, bm) + 3
+    te, tr = orc.expert_tiles(counts, tile_offsets, bm, cap)
+    units = np.full((cap, 4), -1, np.int32)
+    listed = [(te[t], offsets[te[t]] + tr[t], min(bm, counts[te[t]] - tr[t]), 0) for t in range(int(total[0]))]
+    units[: len(listed)] = np.array(listed, np.int32)[rng.permutation(len(listed))]
+    a_q = rng.integers(-127, 128, (tokens if swiglu else rows, k), dtype=np.int8)
+    codes = rng.integers(0, 65536, (e, n, k // 8), dtype=np.uint16)
+    args = dict(A=gu.dev(a_q), AS=gu.dev(rng.uniform(0.01, 0.03, len(a_q)).astype(np.float16)), Book=gu.book(), Counts=gu.dev(counts),
+                Offsets=gu.dev(offsets), P=gu.dev(np.stack([orc.q2_pack_k128(c) for c in codes])), TileCount=gu.dev(total), TileExpert=gu.dev(te),
+                TileRow=gu.dev(tr), WS=gu.dev(rng.uniform(0.001, 0.002, (e, n)).astype(np.float16)))
+    variant = dict(rows=rows, E=e, tiles=cap, N=n, K=k, block_m=bm)
+    if swiglu:
+        variant.update(gather=True, epilogue="swiglu")
+        args.update(C=None, RowMax=None, SlotToken=gu.dev(rng.integers(0, tokens, rows).astype(np.int32)))
+    got = []
+    for with_units in (False, True):
+        out = torch.full((rows + 1, n // 2 if swiglu else n), 55.0, dtype=torch.float16, device=gu.DEV)
+        extra = {"TileUnits": gu.dev(units)} if with_units else {}
+        kern = gu.kernel("e8p_decode_grouped", **variant, **({"tile_units": True} if with_units else {}))
+        kern(**{**args, "Act" if swiglu else "C": out}, **extra)
+        got.append(out)
+    assert torch.equal(*got) and bool((got[1][rows] == 55).all()) and not bool((got[1][:rows] == 55).all(1).any())
+    with pytest.raises(gu.lib.OrxError):
+        gu.kernel("e8p_decode_grouped", **{**variant, "block_m": 32, "gather": False, "epilogue": "none"}, tile_units=True)
 
 
 def test_grouped_resident_rejects_shapes_it_cannot_take():
