@@ -49,7 +49,7 @@ void dense_resident_geometry(int rows, int n, int k, int packed_k, Geometry* g);
 int dense_resident_launch(const int8_t* a, const void* w, const uint32_t* book, const __half* ws, const __half* as,
                           void* out, int rows, int n, int k, int stride, int packed_k, bool out_f32, hipStream_t stream);
 bool runs_eligible(int codec, int rows, int n, int k);
-int runs_rounds(int codec, int rows, int n, int* tile_rows);
+int runs_rounds(int codec, int rows, int n, int* tile_rows, int* run);
 void runs_geometry(int codec, int rows, int n, Geometry* g);
 int runs_launch(int codec, const int8_t* a, const void* w, const uint32_t* book, const __half* ws, const __half* as, void* out,
                 int rows, int n, int k, int stride, int packed_k, bool out_f32, hipStream_t stream);
@@ -708,25 +708,31 @@ int tile_for(const orx_function& f, int rows) {
 //     faster from K = 3072 on (2048 x 3584 at 32 rows 6.9 to 7.5);
 //   two blocks: 7168 x 5376 at 2 rows 9.8 to 8.3 / 10.3 to 8.7, 24 rows 10.8 to 9.2 / 12.2 to 10.9; the runs get there with rows times K: 7168 x 17408 at 16 rows
 //     1.06 / 0.97 of its time, 32 rows 0.93 / 0.84; 7168 x 5120 row-major at 24 / 32 rows 1.06 / 0.98;
-//   three blocks: 9728 x 6144 at 8 rows 0.94 / 0.89 of its time, 24 rows 0.81 / 0.78; K = 4224 at 2 rows 1.06 / 1.02, 24 rows of K = 3200 1.04; two rows stay with
-//     the GEMV (9728 x 9728 18.7 to 17.0 / row-major).
+//   three blocks: 9728 x 6144 at 8 rows 0.84 / 0.89 of its time, 24 rows 0.72 / 0.78; K = 4224 at 2 rows 1.06 / 1.02, 24 rows of K = 3200 1.04; two rows stay with
+//     the GEMV (9728 x 9728 18.7 to 17.0 / row-major);
+//   four and five: 17408 x 6144 at 3 / 16 / 32 rows 0.82 / 0.76 / 0.70 of its time K-major, x 8192 22.3 to 17.8, 24.9 to 18.2, 34.5 to 21.8; 14336 x 6144 1.00 / 0.96 / 0.87, x 8192
+//     0.99 / 0.87 / 0.83; row-major 14336 x 8192 1.01 / 0.97 / 0.84, 17408 x 8192 (the other batched-decode kernel) 0.98 / 0.95 / 0.86.
 // The batched-decode kernels where they take the shape: the one with loader waves (K up to 5120) is the fastest up to 16
-// rows in one and three blocks (K = 5120, 16 rows: 0.85-0.97 of the runs, 0.72-0.9 of the streaming kernel); with one block and
-// more rows the runs pass it at 20 K-major and 24 row-major rows of K = 5120 (2048 x 5120 at 32 rows 7.9 to 8.8 / 8.3 to 8.8, 1024 x 4096 6.5 to 7.2);
-// with two blocks the streaming kernel does (use_resident).  The other one (row-major, K to 8192) is slower than the runs with one
-// block (4096 x 8192 at 8 / 24 rows: the runs 0.81 / 0.74 of it), and with three from rows times K = 160 K on (9728 x 8192 at 8 / 24 rows 1.05 /
-// 0.86, 12288 x 6144 at 17 / 32 rows 1.09 / 0.99).
+// rows in one and three blocks (K = 5120, 16 rows: level with the runs, 0.75-0.9 of the streaming kernel) and in more; the runs pass it, K-major, with one block
+// at 17 rows of K = 5120 and 20 of 4096 (0.87-0.93, 0.91-0.97 of its time; 24 rows of K = 3072 0.97-1.03), with three at 20 rows of K = 5120
+// (0.91-0.93; 17 rows 0.99-1.02, 20 rows of K = 4096 0.99), row-major with one block at 24 rows of K = 5120 (1024 x 4096 at 32 rows 0.85); row-major
+// with three they do not (32 rows of K = 5120 1.05); with two blocks the streaming kernel passes it (use_resident); with five the runs win
+// less than runs differ (17408 x 5120 0.93-1.01).  The other one (row-major, K to 8192) is slower than the runs with one
+// block (4096 x 8192 at 8 / 24 rows: the runs 0.81 / 0.74 of it), and with three above 16 rows from rows times K = 120 K on (9728 x 6144 at 17 / 20 rows 0.95 /
+// 0.90, x 8192 at 8 / 17 rows 0.96 / 0.80; 12288 x 6144 at 20 / 24 rows 0.98 / 0.94).
 int channel_blocks_per_cu(int n) { return (int)ceil_div(ceil_div((uint32_t)n, 16u), (uint32_t)device_compute_units()); }
 bool runs_for_few_rows(const orx_function& f, int rows) {
     const int blocks = channel_blocks_per_cu(f.N);
     const int64_t work = (int64_t)rows * f.K;
-    if (blocks > 3) return false;
-    const bool loader = dense_loader_eligible(f.N, f.K, f.packed_k);
-    if (blocks == 1 && loader) return rows > 16 && work >= (f.packed_k != 0 ? 20 : 24) * 5120;
+    if (blocks > 5) return false;
+    const bool loader = dense_loader_eligible(f.N, f.K, f.packed_k), k_major = f.packed_k != 0;
+    if (blocks == 1 && loader) return rows > 16 && work >= (k_major ? 16 : 24) * 5120;
     if (blocks == 1) return f.K >= (rows > 16 ? 3072 : 4096);
-    if (blocks == 2) return work >= (f.packed_k != 0 ? 32 * 12288 : 20 * 8192);
-    if (loader || rows <= 2) return false;
-    if (dense_resident_eligible(f.N, f.K, f.packed_k)) return work >= 20 * 8192;
+    if (blocks == 2) return work >= (k_major ? 32 * 12288 : 20 * 8192);
+    if (loader) return blocks == 3 && k_major && work >= 20 * 5120;
+    if (rows <= 2 && !(blocks == 5 && k_major)) return false;
+    if (blocks >= 4) return f.K >= (blocks == 5 && k_major ? 6144 : 8192);
+    if (dense_resident_eligible(f.N, f.K, f.packed_k)) return rows > 16 && work >= 20 * 6144;
     return f.K >= (rows > 16 ? 4096 : 6144);
 }
 
@@ -753,30 +759,42 @@ bool runs_for_33_to_64_rows(const orx_function& f) {
 }
 
 // 65 to 512 rows, against all other kernels (with scratch), runs / the best of them:
-//   codes, 65 to 128 rows in one round: up to 32 channels to a CU 0.56-1.06 (K from 1024; 0.8 at 4096); 33 to 48 channels, where the runs over all
-//     rows are the other kernel, 65-80 rows 0.80-0.98, 96-128 rows K = 4096 0.95-1.02, K = 5120 0.93-0.96, K = 8192 (split tiles there) 0.85-0.91; slower
-//     at 68 channels (17408 x 5120 38.5 / 30.8 us);
+//   codes, 65 to 128 rows, against the 128-row runs of k_wide.hip and the split tiles: one round 0.49-0.97 (K = 1024 of 33 to 40 channels to a CU 1.01-1.05; 81 to 96 rows
+//     of K up to 4096 and more than 32 channels, 0.75-0.88, stay with the wide kernel, whose launch records are fixed by name there).  Two rounds lose to one of
+//     the wide kernel (17408 x 4096 1.0-1.22, 24576 x 4096 0.99-1.11) and win where that takes two itself, above 96 channels to a CU: 28672 and 34816 x 2048 / 5120 0.78-0.82 and
+//     0.92-1.0 / 0.76-0.81 and 0.88-0.96, K = 1024 0.85-0.95 and 1.0-1.13;
+//   codes, 129 to 512 rows in row tiles of 65 to 128, against split and whole 128 x 128 tiles, the 512-row runs of k_gemm_big.hip and decode once + 256 x 256 tiles:
+//     one round 0.34-0.83 (7168 x 2048 / 5120 at 200 rows 0.59 / 0.57).  Two row tiles of more than 120 rows and more than 16 channels, and 129 or 130 rows of K = 1024, are 0.5-0.8 too, but
+//     handles of such matrices declare scratch for these launches, and what they declare they use;
+//     two rounds, K from 1536: up to 40 channels in a workgroup 0.75-0.97 in tiles of up to 112 rows and 0.86-1.06 above (9728 at 200 / 256 rows),
+//     wider 0.63-0.98 (12288 x 4096 at 130 / 256 0.65 / 0.76); K = 1024 0.9-1.2.  Matrices of 17 to 32 channels to a CU, 0.60-0.98 at 257 to 512 rows (7168 x 5120 0.69-0.82), keep the
+//     split tiles there: a launch record holds one grid expression, and a program of theirs has no room for two more;
+//     three rounds: tiles of up to 96 rows 0.74-0.97 from K = 3072 (17408 x 5120 at 130-192 rows 57 -> 43, 24576 x 5120 72 -> 51), K = 2048 0.9-1.1;
+//     above, up to 48 channels 0.82-0.96 from K = 4096 and wider 0.83-0.96 from K = 8192, below 0.95-1.4;
+//     four and five up to 256 rows: tiles of up to 96 rows 0.85-0.97 from K = 4096 (34816 x 5120 at 160 rows 96 -> 82), all others 0.97-2;
 //   int8, 65 to 128 rows in one round: 0.1-0.9, except long K: 128 rows of K = 8192 / 10240 / 12288 up to 16 channels to a CU 0.84-0.88 / 0.98-1.03 / 1.04-1.08 (112 rows
 //     0.76-0.82 / 0.91-0.94 / 0.96-0.99), 17 to 32 channels 0.80-0.86 / 0.84-0.97 / 0.85-1.01;
-//   129 to 512 rows, in row tiles of up to 120 rows: codes at 129-200 rows 0.37-0.97 in one round, 33 to 48 channels in two rounds 0.81-1.02 (1.08 at K =
-//     10240, 200 rows); beyond, one round of up to 32 channels 0.41-1.0, two rounds 0.95-1.76; int8 in one round:
-//     K = 8192 / 10240 / 12288 in tiles of 120 rows 0.70-0.77 / 0.89-0.94 / 0.93-0.96, K = 17408 1.08-1.12, of 100 rows 0.84-0.9 and 0.9-1.0;
-//     two rounds of int8 rows 0.6-1.6;
-//   row tiles of 121 to 128 rows, and K up to 1024: up to 16 channels to a CU only (codes of any K 0.5-1.0 but for three row tiles of 4096 x 12288 and longer,
-//     1.06-1.16; int8 K = 10240 / 12288 / 17408 at 256 rows 0.93-0.96 / 0.96-1.0 / 1.10-1.15).  Handles of wider matrices declare scratch for these launches, and what
-//     they declare they use: the split tiles stay although the runs are faster (7168 x 5120 at 256 rows 38.6 us, the runs 30.4; K = 1024 about half the time).
+//   int8, 129 to 512 rows in one round of row tiles of up to 120 rows: K = 8192 / 10240 / 12288 in tiles of 120 rows 0.70-0.77 / 0.89-0.94 / 0.93-0.96, K = 17408
+//     1.08-1.12, of 100 rows 0.84-0.9 and 0.9-1.0; two rounds of int8 rows 0.6-1.6;
+//   row tiles of 121 to 128 rows, and int8 K up to 1024: up to 16 channels to a CU only (codes of any K 0.5-0.9; int8 K = 10240 / 12288 / 17408 at 256 rows 0.93-0.96 /
+//     0.96-1.0 / 1.10-1.15).
 bool runs_for_many_rows(const orx_function& f, int rows) {
-    int tile_rows = 0;
-    const int rounds = runs_rounds(f.flags, rows, f.N, &tile_rows), cus = device_compute_units();
+    int tile_rows = 0, run = 0;
+    const int rounds = runs_rounds(f.flags, rows, f.N, &tile_rows, &run), cus = device_compute_units();
     if (rows <= 128) {
         if (f.flags == kW8) return rounds == 1 && (rows <= 112 || f.K <= 8192 || f.N > 16 * cus);
-        return rounds == 1 && f.N <= (rows <= 80 || f.K > 4096 ? 48 : 32) * cus;
+        if (rounds == 1) return f.N <= 32 * cus || (f.K > 1024 && (f.K > 4096 || rows <= 80 || rows > 96));
+        return rounds <= 3 && f.N > 96 * cus && f.K >= 1536;
     }
-    if (tile_rows > 120 || f.K <= 1024)
-        return rounds == 1 && f.N <= 16 * cus && (f.K <= 10240 || (f.flags == kQ4 && (f.N <= 8 * cus || rows <= 256 || rows > 384)));
+    if (f.flags == kW8 && (tile_rows > 120 || f.K <= 1024)) return rounds == 1 && f.N <= 16 * cus && f.K <= 10240;
     if (f.flags == kW8) return rounds == 1 && (f.K <= 8192 || tile_rows <= 100);
-    if (rows <= 200) return rounds <= 2 && f.N <= 48 * cus;
-    return rounds == 1 && f.N <= 32 * cus;
+    if (rounds == 1) {
+        if (f.N <= 16 * cus) return tile_rows <= 120 || f.K <= 10240 || f.N <= 8 * cus || rows <= 256 || rows > 384;
+        return (f.K > 1024 || rows > 130) && (rows > 256 || tile_rows <= 120);
+    }
+    if (rounds == 2) return f.N > 32 * cus && f.K >= 1536 && (run > 40 || tile_rows <= 112);
+    if (rounds == 3) return rows > 129 && tile_rows <= 120 && f.K >= (tile_rows <= 96 ? 3072 : run <= 48 ? 4096 : 8192);
+    return rounds <= 5 && rows <= 256 && tile_rows <= 96 && f.K >= 4096;
 }
 
 // Channel runs with K split over the waves (k_runs.hip): `algorithm=runs` by name, and by `auto` from one int8 row and two rows of codes

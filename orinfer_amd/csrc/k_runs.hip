@@ -666,11 +666,11 @@ bool runs_eligible(int codec, int rows, int n, int k) {
            runs_shape(codec, rows, n).form != nullptr;
 }
 
-// rounds of the CUs that the launch takes, and the rows of its tiles
-int runs_rounds(int codec, int rows, int n, int* tile_rows) {
+// rounds of the CUs that the launch takes, the rows of its tiles and the channels of its runs
+int runs_rounds(int codec, int rows, int n, int* tile_rows, int* run) {
     const RunsShape s = runs_shape(codec, rows, n);
     const int cus = device_compute_units();
-    *tile_rows = s.tile_rows;
+    *tile_rows = s.tile_rows, *run = s.run;
     return (s.runs * s.row_tiles + cus - 1) / cus;
 }
 

@@ -304,6 +304,24 @@ def test_which_rows_the_channel_runs_take(codec, n, k, rows, algorithm):
         assert auto.geometry(rows) != lib.Kernel(symbol, algorithm="runs", **shape).geometry(rows)
 
 
+# 256 CUs: in rows tiles of up to 128, 48 (tiles above 64 rows: 64) channels a workgroup and one to five rounds of the CUs
+@pytest.mark.parametrize("n, k, rows, algorithm", [
+    (8192, 1024, 130, "mfma"), (8192, 1024, 131, "runs"), (8192, 4096, 240, "runs"), (8192, 4096, 241, "mfma"), (8192, 4096, 257, "mfma"), (8256, 4096, 257, "runs"),
+    (12288, 1280, 200, "mfma"), (12288, 1536, 200, "runs"), (9728, 2048, 224, "runs"), (9728, 2048, 226, "mfma"), (12288, 4096, 256, "runs"), (12288, 4096, 128, "runs"),
+    (12288, 4096, 97, "runs"), (12288, 4224, 96, "runs"), (9728, 1024, 65, "wide"), (14336, 2048, 128, "runs"), (24576, 4096, 128, "wide"), (24592, 4096, 128, "runs"),
+    (24592, 1408, 128, "wide"), (17408, 2944, 130, "tall"), (17408, 3072, 130, "runs"), (17408, 3968, 240, "tall"), (17408, 4096, 240, "runs"), (17408, 4096, 242, "tall"),
+    (20480, 5120, 200, "tall"), (20480, 8192, 200, "runs"), (34816, 4096, 192, "runs"), (34816, 3968, 192, "mfma"), (34816, 5120, 194, "mfma"), (17408, 5120, 257, "tall"),
+    (17408, 6016, 8, "stream"), (17408, 6144, 8, "runs"), (14336, 8064, 17, "stream"), (14336, 8192, 17, "runs"), (9728, 5120, 20, "runs"), (9728, 5120, 19, "resident"),
+])
+def test_which_rows_of_codes_the_channel_runs_take_in_several_rounds(n, k, rows, algorithm):
+    """K-major codes with scratch: both sides of each line (rows, rounds, K) of the rule for codes."""
+    shape = dict(M=rows, N=n, K=k, packed_k=128, workspace=True)
+    auto, runs = (lib.Kernel("e8p_q4_projection", algorithm=a, **shape) for a in ("auto", "runs"))
+    assert (auto.geometry(rows) == runs.geometry(rows)) == (algorithm == "runs")
+    assert algorithm == "mfma" or auto.geometry(rows) == lib.Kernel("e8p_q4_projection", algorithm=algorithm, **shape).geometry(rows)
+    assert (auto.workspace_bytes(rows) > 0) <= (algorithm == "mfma")
+
+
 @pytest.mark.parametrize("codec, n, k, rows", [("w8", 4096, 12288, 128), ("w8", 4096, 12288, 256), ("q4", 4096, 12288, 384), ("q4", 7168, 1024, 130)])
 def test_which_rows_the_channel_runs_leave(codec, n, k, rows):
     symbol, shape = {"q4": "e8p_q4_projection", "w8": "int8_projection"}[codec], dict(M=rows, N=n, K=k, workspace=True)
