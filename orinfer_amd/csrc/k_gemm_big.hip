@@ -228,7 +228,9 @@ __global__ __launch_bounds__(kPersistentThreads) void gemm_big_persistent_kernel
         f[3] = lds_read_16<3 * kBlockBytes>(a);
     };
     auto read_weights = [&](int stage, int slice) {  // into set `slice`
-        const uint32_t w = (w_frag ^ (uint32_t)(slice * 64)) + stage * (2 * kTileBytes);
+        uint32_t frag = w_frag;
+        asm volatile("" : "+v"(frag));  // (or both slices' addresses are kept in registers)
+        const uint32_t w = (frag ^ (uint32_t)(slice * 64)) + stage * (2 * kTileBytes);
         v4i(&f)[4] = fw[slice];
         f[0] = lds_read_16<0>(w);
         f[1] = lds_read_16<kBlockBytes>(w);
@@ -259,7 +261,7 @@ __global__ __launch_bounds__(kPersistentThreads) void gemm_big_persistent_kernel
     };
 
     // ---- epilogue of one tile, wave-private, in registers ----
-    auto epilogue = [&](const TileState& t) {
+    auto epilogue = [&](const TileState& t, int stage) {  // stage: the one that is free
         // the lane number is made opaque here: addresses and bounds that depend only on it would otherwise be
         // computed once in front of the K loop and held in registers (or spilled) for the whole kernel
         int lane = threadIdx.x & 63;
@@ -295,47 +297,59 @@ __global__ __launch_bounds__(kPersistentThreads) void gemm_big_persistent_kernel
             return;
         } else {
             // Weights are the MFMA row operand, so a lane holds token lane % 16 of each 16 x 16 block and four consecutive
-            // output channels 4 (lane / 16) + {0..3}: two words of fp16.  One swap of the odd rows of 16 lanes of channel
-            // block j with the even rows of block j + 1 leaves lane groups 0 and 2 with channels 0-7 and 8-15 of block j
-            // and groups 1 and 3 with those of block j + 1: 16 contiguous bytes of an output row per lane and store, and a
-            // store instruction covers 16 rows x 64 bytes.
+            // output channels 4 (lane / 16) + {0..3}.  Stored from there, neighbouring lanes would be on different rows and every
+            // store instruction would take more than a hundred cycles of the memory pipeline; so 16 rows x 64 channels at a
+            // time go through LDS, where the wave's own token rows of the stage that nobody reads any more were (2 KiB,
+            // twice; 16-byte pieces swizzled by the row), and leave with eight lanes to a row of 128 bytes.
             const bool aligned = (p.stride % 8 == 0) && ((reinterpret_cast<uintptr_t>(p.out) & 15) == 0);
             const bool whole = aligned && t.rows_here == kTile && t.cols_here == kTile;  // no bounds inside this tile
+            const int column = lane & 15;
+            // the scales once, into registers (behind each write of a row they would be read again, a wait each)
+            float4 channel_scale[4];
+            float token_scale = lds_as[wave_m * 128 + column], next_scale = 0.f;  // (of the block after, ahead of the writes)
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int local_row = wave_m * 128 + i * 16 + (lane & 15);
-                const float token_scale = lds_as[local_row];
-                __half* const row_out = reinterpret_cast<__half*>(p.out) + (int64_t)(t.row0 + local_row) * p.stride + t.col0;
+            for (int j = 0; j < 4; ++j) channel_scale[j] = *reinterpret_cast<const float4*>(lds_ws + wave_n * 64 + j * 16 + 4 * group);
+            uint8_t* const image = reinterpret_cast<uint8_t*>(stage_a(stage)) + wave * (BLOCKS_PER_WAVE * 1024);
+            uint8_t* const to = image + column * 128 + (group & 1) * 8;
+            const int piece_of_write = (group >> 1) ^ (column & 7);  // of channel block 0; block j: ^ 2 j
+            const uint8_t* const from = image + (lane >> 3) * 128 + ((lane & 7) ^ (lane >> 3)) * 16;
+            const int local_col = wave_n * 64 + (lane & 7) * 8;
+            // (a uniform row and a lane's place behind it in elements)
+            __half* const out = reinterpret_cast<__half*>(p.out) + (int64_t)(t.row0 + wave_m * 128) * p.stride + t.col0;
+            const int64_t place = (int64_t)(lane >> 3) * p.stride + local_col;
+            auto store_block = [&](int i) {
 #pragma unroll
-                for (int pair = 0; pair < 2; ++pair) {  // channel blocks (0, 1), then (2, 3)
-                    uint32_t words[2][2];
-#pragma unroll
-                    for (int b = 0; b < 2; ++b) {
-                        const int j = 2 * pair + b;
-                        const float4 wscale = *reinterpret_cast<const float4*>(lds_ws + wave_n * 64 + j * 16 + 4 * group);
-                        words[b][0] = pack_halves(rescale(acc[i][j][0], wscale.x, token_scale), rescale(acc[i][j][1], wscale.y, token_scale));
-                        words[b][1] = pack_halves(rescale(acc[i][j][2], wscale.z, token_scale), rescale(acc[i][j][3], wscale.w, token_scale));
-                    }
-                    const v2u low = __builtin_amdgcn_permlane16_swap(words[0][0], words[1][0], false, false);
-                    const v2u high = __builtin_amdgcn_permlane16_swap(words[0][1], words[1][1], false, false);
-                    const uint4 piece = make_uint4(low.x, high.x, low.y, high.y);
-                    const int local_col = wave_n * 64 + (2 * pair + (group & 1)) * 16 + (group >> 1) * 8;
+                for (int h = 0; h < 2; ++h) {
+                    const uint4 piece = *reinterpret_cast<const uint4*>(from + (i & 1) * 2048 + h * 1024);
+                    __half* const row_out = out + (int64_t)(i * 16 + h * 8) * p.stride + place;
                     if (whole) {
-                        *reinterpret_cast<uint4*>(row_out + local_col) = piece;
-                    } else if (local_row < t.rows_here && local_col < t.cols_here) {
+                        *reinterpret_cast<uint4*>(row_out) = piece;
+                    } else if (wave_m * 128 + i * 16 + h * 8 + (lane >> 3) < t.rows_here && local_col < t.cols_here) {
                         if (aligned && local_col + 8 <= t.cols_here) {
-                            *reinterpret_cast<uint4*>(row_out + local_col) = piece;
+                            *reinterpret_cast<uint4*>(row_out) = piece;
                         } else {
                             const uint32_t parts[4] = {piece.x, piece.y, piece.z, piece.w};
 #pragma unroll
                             for (int e = 0; e < 8; ++e)
                                 if (local_col + e < t.cols_here)
-                                    row_out[local_col + e] = __ushort_as_half((unsigned short)(parts[e >> 1] >> (16 * (e & 1))));
+                                    row_out[e] = __ushort_as_half((unsigned short)(parts[e >> 1] >> (16 * (e & 1))));
                         }
                     }
-                    __builtin_amdgcn_sched_barrier(0);  // one pair at a time: interleaved pairs cost registers, not time
                 }
+            };
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                if (i < 7) next_scale = lds_as[wave_m * 128 + i * 16 + 16 + column];
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    *reinterpret_cast<uint2*>(to + (i & 1) * 2048 + (piece_of_write ^ (2 * j)) * 16) =
+                        make_uint2(pack_halves(rescale(acc[i][j][0], channel_scale[j].x, token_scale), rescale(acc[i][j][1], channel_scale[j].y, token_scale)),
+                                   pack_halves(rescale(acc[i][j][2], channel_scale[j].z, token_scale), rescale(acc[i][j][3], channel_scale[j].w, token_scale)));
+                token_scale = next_scale;
+                if (i > 0) store_block(i - 1);
+                __builtin_amdgcn_sched_barrier(0);
             }
+            store_block(7);
         }
     };
 
@@ -421,7 +435,7 @@ __global__ __launch_bounds__(kPersistentThreads) void gemm_big_persistent_kernel
     for (int tile_index = 0; tile_index < my_tiles; ++tile_index) {
         for (int kt = 0; kt + 1 < k_tiles; ++kt) k_step(std::false_type{});
         k_step(std::true_type{});
-        epilogue(tile);
+        epilogue(tile, (g - 1) & 1);
         clear();
         tile = tile_state(tile_index + 1);
         const int cur = (g - 1) & 1;
