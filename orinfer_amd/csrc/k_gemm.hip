@@ -51,6 +51,10 @@ int dense_resident_launch(const int8_t* a, const void* w, const uint32_t* book, 
 bool runs_eligible(int codec, int rows, int n, int k);
 int runs_rounds(int codec, int rows, int n, int* tile_rows, int* run);
 void runs_geometry(int codec, int rows, int n, Geometry* g);
+bool panel_eligible(int rows, int n, int k);  // k_panel.hip
+void panel_geometry(int rows, int n, Geometry* g);
+int panel_launch(const uint8_t* panels, const int* sums, const void* w, const uint32_t* book, const __half* ws, const __half* as, void* out,
+                 int rows, int n, int k, int stride, int packed_k, bool out_f32, hipStream_t stream);
 int runs_launch(int codec, const int8_t* a, const void* w, const uint32_t* book, const __half* ws, const __half* as, void* out,
                 int rows, int n, int k, int stride, int packed_k, bool out_f32, hipStream_t stream);
 bool dense_wide_eligible(int n, int k, int packed_k);
@@ -1310,6 +1314,18 @@ int make_projection(const Variant& v, orx_function* f, int codec) {
     return ORX_OK;
 }
 
+// Token rows as panels (the quantiser's, of the same key): A, AS, Book, Out, S, Sums, W[, m]
+int q4_panel_geometry(const orx_function& f, int rows, Geometry* g) {
+    panel_geometry(rows, f.N, g);
+    return ORX_OK;
+}
+int q4_panel_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t stream, void** args) {
+    (void)g;
+    return panel_launch(pointer_arg<const uint8_t>(args, 0), pointer_arg<const int>(args, 5), pointer_arg<const void>(args, 6), pointer_arg<const uint32_t>(args, 2),
+                        pointer_arg<const __half>(args, 4), pointer_arg<const __half>(args, 1), pointer_arg<void>(args, 3), rows, f.N, f.K, f.stride, f.packed_k,
+                        f.out_f32, stream);
+}
+
 int make_q4_projection(const Variant& v, orx_function* f) {
     if (!two_stage_coefficients_ok(v, "e8p_q4_projection")) return ORX_ERR_BAD_VARIANT;
     int code = make_projection(v, f, kQ4);
@@ -1342,6 +1358,20 @@ int make_q4_projection(const Variant& v, orx_function* f) {
     if (bad || (f->publish_codes && !f->input_f16)) {
         set_error("e8p_q4_projection: codes=true needs input_dtype=float16");
         return ORX_ERR_BAD_VARIANT;
+    }
+    const bool panels = v.boolean("panels", false, &bad);
+    if (bad || (panels && (f->input_f16 || v.string("algorithm", "auto", &bad) != "auto" || f->tiles != 0 || f->takes_workspace ||
+                           !panel_eligible(f->capacity, f->N, f->K)))) {
+        set_error("e8p_q4_projection: panels=true serves int8 rows, up to 2048 of them, K from 256, algorithm auto, without block_m and workspace");
+        return ORX_ERR_BAD_VARIANT;
+    }
+    if (panels) {
+        f->args = {{"A", ArgPointer, 16}, {"AS", ArgPointer, 2}, {"Book", ArgPointer, 4}, {"Out", ArgPointer, 2}, {"S", ArgPointer, 2}, {"Sums", ArgPointer, 4}, {"W", ArgPointer, 16}};
+        if (f->dynamic_rows) f->args.push_back({"m", ArgI32, 4});
+        f->workspace_need = nullptr;
+        f->geometry = q4_panel_geometry;
+        f->launch = q4_panel_launch;
+        return ORX_OK;
     }
     f->args = {{"A", ArgPointer, 16}, {"AS", ArgPointer, 2}, {"Book", ArgPointer, 4}, {"Out", ArgPointer, 2}};
     if (f->publish_codes) f->args.push_back({"Q", ArgPointer, 8});
@@ -2162,9 +2192,9 @@ const Registration* gemm_registrations(int* count) {
     static const Registration rows[] = {
     {"e8p_q4_projection", make_q4_projection,
      "M, N, K, dynamic_rows=false, algorithm=auto|gemv|stream|resident|wide|tall|runs|mfma, packed_k=0|64|128, output_dtype=float16|float32, "
-     "input_dtype=int8|float16, rotate=false, codes=false, workspace=false, split_k=true, "
+     "input_dtype=int8|float16, rotate=false, codes=false, panels=false, workspace=false, split_k=true, "
      "output_stride=N, block_m=0|32|64|128|256, gemv_passes=0, decode_in_gemm=false",
-     "A,AS,Book,Out[,Q],S[,Signs],W[,Workspace][,m]"},
+     "A,AS,Book,Out[,Q],S[,Signs][,Sums],W[,Workspace][,m]"},
     {"int8_projection", make_w8_projection,
      "M, N, K, dynamic_rows=false, algorithm=auto|gemv|stream|runs|mfma, output_dtype=float16|float32, output_stride=N, "
      "block_m=0|32|64|128|256, workspace=false, split_k=true",

@@ -100,16 +100,26 @@ __device__ __forceinline__ uint2 quantise_piece(word4 piece, float scale, float 
 // What bounds it: memory with many rows (8192 x 4096: 28.1 -> 20.7 us, 4.9 TB/s; the two-pass kernel read every row twice),
 // the vector ALU beside it in the FUSED form (8192 x 17408: 416 -> 146 us; the two-pass kernel also computed every value
 // twice), the latency of one row's loads and reductions with few (FUSED, one row of 17408: 43 -> 5.9 us).
-template <bool FUSED, int WAVES, int PIECES, bool LONG>
+// PANELS (one group to a row, K a multiple of 128): the codes a second time in the order in which k_panel.hip's projection reads them, and the sum
+// of a row's codes.
+template <bool FUSED, int WAVES, int PIECES, bool LONG, bool PANELS = false>
 __global__ __launch_bounds__(WAVES == 1 ? 256 : 64 * WAVES) void a8_held_kernel(const __half* __restrict__ x,
                                                                                 int8_t* __restrict__ q,
                                                                                 __half* __restrict__ s, int k, int group,
-                                                                                int groups, int rows) {
+                                                                                int groups, int rows, uint8_t* __restrict__ panels,
+                                                                                int* __restrict__ sums) {
     constexpr int kLanes = 64 * WAVES, kTail = 4;
     __shared__ float scratch[WAVES];
     const int lane = WAVES == 1 ? threadIdx.x & 63 : threadIdx.x;
-    const int unit = WAVES == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;  // wave-uniform
-    if (unit >= rows * groups) return;  // only with one wave to a unit: nothing below waits for it
+    int unit = WAVES == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;  // wave-uniform
+    if constexpr (PANELS) {
+        // Workgroups go to the 8 XCDs in turn: the 16 rows of a panel, which share its cache lines, stay on one (a line written in pieces by all
+        // of them goes to memory from each: 512 x 5120 5.7 us, 4.3 so)
+        constexpr int kTogether = WAVES == 1 ? 4 : 16;  // workgroups to a panel
+        const int turn = blockIdx.x >> 3;
+        unit = (turn / kTogether * 8 + (blockIdx.x & 7)) * 16 + (WAVES == 1 ? turn % kTogether * 4 + (int)(threadIdx.x >> 6) : turn % kTogether);
+    }
+    if (unit >= rows * groups) return;  // whole workgroups, or one wave to a unit: nothing below waits for it
     const int row = unit / groups, g = unit % groups;
     const int first = g * group;
     const int width = min(group, k - first);
@@ -161,11 +171,23 @@ __global__ __launch_bounds__(WAVES == 1 ? 256 : 64 * WAVES) void a8_held_kernel(
     if (lane == 0) s[(int64_t)row * groups + g] = stored;
     const float scale = __half2float(stored);
     const float inverse = __frcp_rn(scale);
+    int sum = 0;
+    // byte `col` of this row in its panel: 16 rows x 64 of K, half s of a chunk of 128 holds [32 q + 16 s, +16) in its quarter q
+    auto in_panel = [&](int col) {
+        return panels + (int64_t)(row >> 4) * 16 * k + (col >> 7) * 2048 + (col >> 4 & 1) * 1024 + (col >> 5 & 3) * 256 + (row & 15) * 16 + (col & 15);
+    };
     if (vector) {
         uint2* dst = reinterpret_cast<uint2*>(q + out_base + first);
 #pragma unroll
         for (int p = 0; p < PIECES; ++p)
-            if (lane + p * kLanes < pieces) dst[lane + p * kLanes] = quantise_piece(held[p], scale, inverse);
+            if (lane + p * kLanes < pieces) {
+                const uint2 codes = quantise_piece(held[p], scale, inverse);
+                dst[lane + p * kLanes] = codes;
+                if constexpr (PANELS) {
+                    *reinterpret_cast<uint2*>(in_panel((lane + p * kLanes) * 8)) = codes;
+                    sum = __builtin_amdgcn_sdot4((int)codes.y, 0x01010101, __builtin_amdgcn_sdot4((int)codes.x, 0x01010101, sum, false), false);
+                }
+            }
         if (LONG) {
             for (int base = lane + PIECES * kLanes; base < pieces; base += kTail * kLanes) {
                 word4 more[kTail], more_up[FUSED ? kTail : 1] = {};
@@ -186,8 +208,28 @@ __global__ __launch_bounds__(WAVES == 1 ? 256 : 64 * WAVES) void a8_held_kernel(
             }
         }
     } else {
-        for (int i = lane; i < width; i += kLanes)
-            q[out_base + first + i] = quantise(load_value<FUSED>(x, in_base, k, first + i), scale, inverse);
+        for (int i = lane; i < width; i += kLanes) {
+            const int8_t code = quantise(load_value<FUSED>(x, in_base, k, first + i), scale, inverse);
+            q[out_base + first + i] = code;
+            if constexpr (PANELS) *reinterpret_cast<int8_t*>(in_panel(i)) = code, sum += code;
+        }
+    }
+    if constexpr (PANELS) {
+        // rows of 16 lanes by lane moves (the neighbour, the other pair, the mirrored half row, the mirrored row), the four rows as scalars
+        sum += __builtin_amdgcn_update_dpp(0, sum, 0xB1, 0xF, 0xF, true);
+        sum += __builtin_amdgcn_update_dpp(0, sum, 0x4E, 0xF, 0xF, true);
+        sum += __builtin_amdgcn_update_dpp(0, sum, 0x141, 0xF, 0xF, true);
+        sum += __builtin_amdgcn_update_dpp(0, sum, 0x140, 0xF, 0xF, true);
+        sum = __builtin_amdgcn_readlane(sum, 0) + __builtin_amdgcn_readlane(sum, 16) + __builtin_amdgcn_readlane(sum, 32) + __builtin_amdgcn_readlane(sum, 48);
+        if constexpr (WAVES > 1) {
+            __shared__ int wave_sums[WAVES];
+            if ((threadIdx.x & 63) == 0) wave_sums[threadIdx.x >> 6] = sum;
+            __syncthreads();
+            sum = 0;
+#pragma unroll
+            for (int w = 0; w < WAVES; ++w) sum += wave_sums[w];
+        }
+        if (lane == 0) sums[row] = sum;
     }
 }
 
@@ -687,12 +729,13 @@ __global__ __launch_bounds__(256) void swiglu_kernel(const __half* __restrict__ 
 // The forms of a8_held_kernel: waves to a group, pieces of eight values to a lane.
 struct HeldForm {
     int waves, pieces;
-    const void *plain, *fused;
+    const void *plain, *fused, *panels;  // panels: null in the form for the longest groups
 };
 const HeldForm* held_forms(int* count) {
 #define ORX_HELD(W, P)                                                                                             \
     {W, P, reinterpret_cast<const void*>(&a8_held_kernel<false, W, P, (W > 8)>),                                   \
-     reinterpret_cast<const void*>(&a8_held_kernel<true, W, P, (W > 8)>)}
+     reinterpret_cast<const void*>(&a8_held_kernel<true, W, P, (W > 8)>),                                          \
+     W > 8 ? nullptr : reinterpret_cast<const void*>(&a8_held_kernel<false, (W > 8 ? 1 : W), (W > 8 ? 1 : P), false, true>)}
     static const HeldForm forms[] = {ORX_HELD(1, 1), ORX_HELD(1, 2), ORX_HELD(1, 4), ORX_HELD(4, 1), ORX_HELD(4, 2),
                                      ORX_HELD(4, 3), ORX_HELD(4, 4), ORX_HELD(4, 6), ORX_HELD(8, 1), ORX_HELD(8, 2),
                                      ORX_HELD(8, 3), ORX_HELD(8, 5), ORX_HELD(8, 8), ORX_HELD(16, 8)};
@@ -731,6 +774,7 @@ int a8_geometry(const orx_function& f, int rows, Geometry* g) {
     if (const HeldForm* form = held_form(f, rows)) {
         const uint32_t waves = (uint32_t)form->waves, units = (uint32_t)rows * groups;
         g->grid[0] = waves == 1 ? ceil_div(units, 4u) : units;
+        if (f.flags & 4) g->grid[0] = ceil_div(units, 128u) * (waves == 1 ? 32 : 128);  // whole panels to each XCD
         g->block[0] = waves == 1 ? 256 : 64 * waves;
         return ORX_OK;
     }
@@ -741,17 +785,21 @@ int a8_geometry(const orx_function& f, int rows, Geometry* g) {
 }
 
 int a8_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t stream, void** args) {
-    const uint8_t* mask = pointer_arg<const uint8_t>(args, 0);
-    int8_t* q = pointer_arg<int8_t>(args, 1);
-    __half* s = pointer_arg<__half>(args, 2);
-    const __half* x = pointer_arg<const __half>(args, 3);
+    int next = 0;
+    const uint8_t* mask = pointer_arg<const uint8_t>(args, next++);
+    const bool to_panels = f.flags & 4;
+    uint8_t* panels = to_panels ? pointer_arg<uint8_t>(args, next++) : nullptr;
+    int8_t* q = pointer_arg<int8_t>(args, next++);
+    __half* s = pointer_arg<__half>(args, next++);
+    int* sums = to_panels ? pointer_arg<int>(args, next++) : nullptr;
+    const __half* x = pointer_arg<const __half>(args, next);
     const dim3 grid(g.grid[0], g.grid[1]), block(g.block[0]);
     const int groups = (int)ceil_div((uint32_t)f.K, (uint32_t)f.group);
     const bool fused = f.flags & 2;
     if (const HeldForm* form = held_form(f, rows)) {
-        typedef void (*Held)(const __half*, int8_t*, __half*, int, int, int, int);
-        const Held kernel = reinterpret_cast<Held>(const_cast<void*>(fused ? form->fused : form->plain));
-        ORX_LAUNCH(kernel, grid, block, 0, stream, x, q, s, f.K, f.group, groups, rows);
+        typedef void (*Held)(const __half*, int8_t*, __half*, int, int, int, int, uint8_t*, int*);
+        const Held kernel = reinterpret_cast<Held>(const_cast<void*>(to_panels ? form->panels : fused ? form->fused : form->plain));
+        ORX_LAUNCH(kernel, grid, block, 0, stream, x, q, s, f.K, f.group, groups, rows, panels, sums);
     } else if (fused)
         ORX_LAUNCH((a8_masked_kernel<true>), grid, block, 0, stream, x, mask, q, s, f.K, f.group, groups);
     else
@@ -777,11 +825,21 @@ int make_a8(const Variant& v, orx_function* f) {
         set_error("activation_quantization: threads is 128, 256 or 512");
         return ORX_ERR_BAD_VARIANT;
     }
-    f->flags = (masked ? 1 : 0) | (fused ? 2 : 0);
+    // panels=true: the codes also as panels (rows rounded up to 16 x K bytes) and every row's sum of codes, what the projection of
+    // the same key reads
+    const bool panels = v.boolean("panels", false, &bad);
+    if (bad || (panels && (masked || fused || f->group != f->K || f->K % 128 != 0 || f->K > 32768))) {
+        set_error("activation_quantization: panels=true serves one group to a row, K a multiple of 128 up to 32768, without mask and fusion");
+        return ORX_ERR_BAD_VARIANT;
+    }
+    f->flags = (masked ? 1 : 0) | (fused ? 2 : 0) | (panels ? 4 : 0);
     f->dynamic_rows = true;
     // Mask may be null unless masked (the reference ignores it then, op30:75-76)
     f->args = {{"Mask", ArgPointer, masked ? 1u : 0x80000001u}, {"Q", ArgPointer, 1}, {"S", ArgPointer, 2},
                {"X", ArgPointer, 2}, {"rows", ArgI32, 4}};
+    if (panels)
+        f->args = {{"Mask", ArgPointer, 0x80000001u}, {"Panels", ArgPointer, 16}, {"Q", ArgPointer, 1}, {"S", ArgPointer, 2},
+                   {"Sums", ArgPointer, 4}, {"X", ArgPointer, 2}, {"rows", ArgI32, 4}};
     f->device_function = nullptr;  // the kernel follows the rows and the group
     f->geometry = a8_geometry;
     f->launch = a8_launch;
@@ -1201,8 +1259,8 @@ int make_swiglu(const Variant& v, orx_function* f) {
 
 const Registration* quant_registrations(int* count) {
     static const Registration rows[] = {
-    {"activation_quantization", make_a8, "K, group_size=null, masked=false, fused=false, threads=256, M=capacity",
-     "Mask,Q,S,X,rows"},
+    {"activation_quantization", make_a8, "K, group_size=null, masked=false, fused=false, panels=false, threads=256, M=capacity",
+     "Mask[,Panels],Q,S[,Sums],X,rows"},
     {"swiglu", make_swiglu, "I, M=capacity", "X,Y,rows"},
     {"rotate_activation_a8", make_rotate_a8, "M, K, swiglu=false, reciprocal=true, dynamic_rows=false, registers=false", "Q,S,Signs,X[,m]"},
     {"rotate_expert_a8", make_rotate_expert,

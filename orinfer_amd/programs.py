@@ -20,6 +20,30 @@ def _dev(array):
     return torch.from_numpy(a.view(view) if view else a).cuda()
 
 
+PANEL_ROWS = 1024
+
+
+def panels_pay(rows, n, k, cus):
+    """Whether quantiser and projection of two-stage codes are faster over token panels than row-major (time of the pair over panels / row-major, 256 CUs):
+    65-128 rows 0.78-0.97 with 4 to 5 blocks of 16 channels to a CU, 0.9-1.3 otherwise.  Up to one block 1.0-2.1 at 129-512 rows; at 513-1024 0.44-0.95 up to
+    K = 4096, 0.75-1.5 beyond.  One to two blocks, where the channel runs fill one round (up to 240 rows; 257-384 of up to 1.3 blocks): 5120 channels 0.99-1.4, 7168 and
+    8192 at 130-160 / 200 rows 0.91-1.15 / 0.86-1.01; other rows up to 512 0.41-1.01, 513-1024 0.64-0.98 (5120 x 8192 and x 12288 at 640-768 rows 1.0-1.12).
+    Wider: 0.42-0.91 at 129-512 rows, 0.69-0.86 at 513-768 (34816 x 1024-2048 0.95-1.04), 0.66-0.99 at 1024 (K = 1024 0.66-1.13).  Beyond 1024 rows decoding once is mostly
+    faster (1280 rows 0.72-1.5)."""
+    if not 64 < rows <= PANEL_ROWS:
+        return False
+    blocks = -(-n // 16)
+    if rows <= 128:
+        return 4 * cus < blocks <= 5 * cus
+    if blocks <= cus:
+        return rows > 512 and k <= 4096
+    if rows > 768 and k < 2048 or rows > 512 and 4 * blocks <= 5 * cus and k > 5120:
+        return False
+    row_tiles = -(-rows // 128)
+    one_round = blocks <= 2 * cus and row_tiles * -(-blocks // 4) <= cus and not 240 < rows <= 256  # the channel runs take these
+    return not one_round or (rows > 176 and 4 * blocks > 6 * cus)
+
+
 class QuantizedLinear:
     """A8 quantiser + one projection (E8P-Q4 or W8A8) with a dynamic row count up to `capacity`."""
 
@@ -65,6 +89,17 @@ class QuantizedLinear:
                 if error.code != ORX_ERR_BAD_VARIANT:
                     raise
         self.workspace = self.projection.workspace()
+        # rows over panels: the quantiser leaves the int8 rows a second time, in the order of the matrix operands
+        top = min(capacity, PANEL_ROWS)
+        cus = torch.cuda.get_device_properties(self.weight.device).multi_processor_count
+        self.over_panels = [False] * (top + 1)
+        if codec == "q4" and algorithm == "auto" and not block_m and 256 <= self.k <= 32768 and self.n * self.k < 2**31:
+            self.over_panels = [panels_pay(rows, self.n, self.k, cus) for rows in range(top + 1)]
+        if any(self.over_panels):
+            self.panels = torch.empty(((top + 15) // 16 * 16, self.k), dtype=torch.int8, device="cuda")
+            self.sums = torch.empty(top, dtype=torch.int32, device="cuda")
+            self.panel_quantizer = Kernel("activation_quantization", K=self.k, panels=True)
+            self.panel_projection = Kernel("e8p_q4_projection", M=top, N=self.n, K=self.k, dynamic_rows=True, panels=True, packed_k=packed_k)
 
     def quantize(self, x16, stream=None):
         rows = x16.shape[0]
@@ -91,6 +126,12 @@ class QuantizedLinear:
         if self.single is not None and x16.shape[0] == 1 and x16.data_ptr() % 16 == 0:  # (the quantiser takes any fp16 address)
             self.single(stream=stream, A=x16, AS=self.a_s, Book=self.book, Out=self.out, Q=self.a_q, S=self.scales, W=self.weight)
             return self._rows(1)
+        rows = x16.shape[0]
+        if rows < len(self.over_panels) and self.over_panels[rows]:
+            self.panel_quantizer(stream=stream, Mask=None, Panels=self.panels, Q=self.a_q, S=self.a_s, Sums=self.sums, X=x16, rows=rows)
+            self.panel_projection(stream=stream, A=self.panels, AS=self.a_s, Book=self.book, Out=self.out, S=self.scales, Sums=self.sums,
+                                  W=self.weight, m=rows)
+            return self._rows(rows)
         return self.project(self.quantize(x16, stream), stream)
 
 

@@ -322,6 +322,18 @@ def test_which_rows_of_codes_the_channel_runs_take_in_several_rounds(n, k, rows,
     assert (auto.workspace_bytes(rows) > 0) <= (algorithm == "mfma")
 
 
+@pytest.mark.parametrize("n, k, lines", [
+    (4096, 4096, [(128, 0), (512, 0), (513, 1), (1024, 1), (1025, 0)]), (4096, 4224, [(513, 0), (1024, 0)]),
+    (5120, 5120, [(176, 0), (240, 0), (241, 1), (256, 1), (257, 0), (384, 0), (385, 1), (768, 1), (1024, 1)]), (5120, 8192, [(512, 1), (513, 0)]),
+    (7168, 5120, [(128, 0), (176, 0), (177, 1), (240, 1), (512, 1), (1024, 1)]), (12288, 1024, [(128, 0), (129, 1), (768, 1), (769, 0)]),
+    (17408, 5120, [(64, 0), (65, 1), (1024, 1), (1025, 0)]), (34816, 5120, [(128, 0), (129, 1)]),
+])
+def test_which_rows_a_linear_takes_over_panels(n, k, lines):
+    from orinfer_amd.programs import panels_pay
+    for rows, taken in lines:
+        assert panels_pay(rows, n, k, 256) == bool(taken), rows
+
+
 @pytest.mark.parametrize("codec, n, k, rows", [("w8", 4096, 12288, 128), ("w8", 4096, 12288, 256), ("q4", 4096, 12288, 384), ("q4", 7168, 1024, 130)])
 def test_which_rows_the_channel_runs_leave(codec, n, k, rows):
     symbol, shape = {"q4": "e8p_q4_projection", "w8": "int8_projection"}[codec], dict(M=rows, N=n, K=k, workspace=True)

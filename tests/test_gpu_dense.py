@@ -1675,3 +1675,104 @@ def test_auto_rows_around_the_channel_runs(rows, n, k):
         extra = {"Workspace": w8.workspace()} if scratch else {}
         w8(A=gu.dev(a_q), Output=out, TokenScale=gu.dev(a_s), Weight=gu.dev(weight), WeightScale=gu.dev(ws), m=rows, **extra)
         np.testing.assert_array_equal(gu.host(out), want8)
+
+
+# ---- token panels -----------------------------------------------------------------------------------------------------
+# Every number of waves and pieces the quantiser has, a panel that is not full, several rounds of panels over the XCDs, and rows whose
+# address leaves no 16-byte loads.
+@pytest.mark.parametrize("rows,k,shift", [(1, 128, 0), (16, 256, 0), (37, 512, 1), (130, 1280, 0), (129, 2048, 0), (2049, 2048, 0), (2100, 384, 1), (600, 5120, 0),
+                                          (200, 8192, 1), (17, 17408, 0), (3, 32768, 0)])
+def test_a8_panels(rows, k, shift):
+    rng = np.random.default_rng(orc.SEED + rows + k)
+    x = torch.empty(rows * k + 8, dtype=torch.float16, device=gu.DEV)
+    x16 = x[shift:shift + rows * k].view(rows, k)
+    x16.copy_(gu.dev(rng.normal(0, 1, (rows, k)).astype(np.float16)))
+    x16[0] = 0
+    padded = (rows + 15) // 16 * 16
+    panels = torch.full((padded + 1, k), 91, dtype=torch.int8, device=gu.DEV)
+    q = torch.empty((rows, k), dtype=torch.int8, device=gu.DEV)
+    s = torch.empty((rows, 1), dtype=torch.float16, device=gu.DEV)
+    sums = torch.full((rows + 1,), 91, dtype=torch.int32, device=gu.DEV)
+    gu.kernel("activation_quantization", K=k, panels=True)(Mask=None, Panels=panels, Q=q, S=s, Sums=sums, X=x16, rows=rows)
+    want_q, want_s = gu.a8(x16)
+    assert torch.equal(q, want_q) and torch.equal(s.view(-1), want_s.view(-1))
+    assert torch.equal(sums[:rows].long(), q.long().sum(1)) and int(sums[rows]) == 91
+    rest = torch.full((padded, k), 91, dtype=torch.int8, device=gu.DEV)
+    rest[:rows] = q
+    # block of 16 rows, chunk of 128, half, quarter, row, 16 bytes: the bytes [32 quarter + 16 half, +16) of a chunk
+    order = rest.view(padded // 16, 16, k // 128, 4, 2, 16).permute(0, 2, 4, 3, 1, 5).reshape(padded, k)
+    assert torch.equal(panels[:padded], order) and bool((panels[padded] == 91).all())
+
+
+# One to five channel blocks to a workgroup (the last ones short), two to four row blocks to a wave with rows missing, one to three row
+# tiles, phases that end early (1 to 8 chunks), and the largest sums either way.
+@pytest.mark.parametrize("rows,n,k", [(1, 16, 256), (17, 24, 384), (129, 4099, 1152), (255, 5000, 896), (257, 8200, 1280), (256, 12290, 640), (300, 9728, 384), (384, 17408, 256),
+                                      (385, 20480, 768), (512, 20600, 256), (513, 300, 1024), (1030, 1000, 640), (449, 16000, 512)])
+@pytest.mark.parametrize("packed_k", [128, 64, 0])
+def test_q4_over_panels(rows, n, k, packed_k):
+    rng = np.random.default_rng(orc.SEED + rows + n + k)
+    a_q, a_s, packed, ws = q4_case(rng, rows, n, k)
+    a_q[0, :], a_q[-1, :] = 127, -128
+    out = torch.full((rows + 1, n), 91, dtype=torch.float16, device=gu.DEV)
+    project_over_panels(a_q, a_s, packed, ws, packed_k, out)
+    np.testing.assert_array_equal(gu.host(out)[:rows], orc.project(a_q, a_s, orc.q4_integers(packed, TABLE), ws))
+    assert (gu.host(out)[rows] == 91).all()
+
+
+def project_over_panels(a_q, a_s, packed, ws, packed_k, out, **variant):
+    rows, k = a_q.shape
+    padded = np.zeros(((rows + 15) // 16 * 16, k), np.int8)
+    padded[:rows] = a_q
+    panels = np.ascontiguousarray(padded.reshape(-1, 16, k // 128, 4, 2, 16).transpose(0, 2, 4, 3, 1, 5))
+    stored = packed if packed_k == 0 else orc.q4_pack_k(packed, packed_k)
+    gu.kernel("e8p_q4_projection", M=rows, N=len(ws), K=k, packed_k=packed_k, panels=True, workspace=False, **variant)(
+        A=gu.dev(panels), AS=gu.dev(a_s), Book=gu.book(), Out=out, S=gu.dev(ws), Sums=gu.dev(a_q.astype(np.int32).sum(1).astype(np.int32)), W=gu.dev(stored))
+
+
+@pytest.mark.parametrize("dtype,pad", [(torch.float16, 1), (torch.float16, 4), (torch.float32, 3)], ids=["fp16-odd", "fp16-8-bytes", "fp32"])
+def test_q4_over_panels_strides(dtype, pad):
+    rows, n, k = 150, 9005, 512
+    a_q, a_s, packed, ws = q4_case(np.random.default_rng(orc.SEED), rows, n, k)
+    out = torch.full((rows + 1, n + pad), 91, dtype=dtype, device=gu.DEV)
+    project_over_panels(a_q, a_s, packed, ws, 0, out, output_stride=n + pad, output_dtype="float16" if dtype == torch.float16 else "float32")
+    want = orc.project(a_q, a_s, orc.q4_integers(packed, TABLE), ws, out_dtype=np.float16 if dtype == torch.float16 else np.float32)
+    np.testing.assert_array_equal(gu.host(out)[:rows, :n], want)
+    assert (gu.host(out)[rows] == 91).all() and (gu.host(out)[:, n:] == 91).all()
+
+
+def test_a_linear_over_panels_gives_the_bits_of_the_row_major_one():
+    """Rows either side of the lines, one state; the codes and scales that `run` leaves are the quantiser's; and from a graph."""
+    rng = np.random.default_rng(orc.SEED)
+    n, k = 9728, 512
+    linear = programs.QuantizedLinear("q4", rng.integers(0, 2**32, (n, k // 8), dtype=np.uint32), rng.uniform(0.005, 0.02, n).astype(np.float16), 1300, packed_k=128)
+    taken = [r for r, over in enumerate(linear.over_panels) if over]
+    assert taken and taken[0] > 64 and len(linear.over_panels) == programs.PANEL_ROWS + 1
+    for rows in (taken[0] - 1, taken[0], 512, 700, 768, 1025):
+        x = gu.dev(rng.normal(0, 1, (rows, k)).astype(np.float16))
+        got = linear.run(x).clone()
+        codes, scales = linear.a_q[:rows].clone(), linear.a_s[:rows].clone()
+        want = linear.project(linear.quantize(x))
+        assert torch.equal(got, want) and torch.equal(codes, linear.a_q[:rows]) and torch.equal(scales, linear.a_s[:rows]), rows
+    x = gu.dev(rng.normal(0, 1, (512, k)).astype(np.float16))
+    want, stream = linear.run(x).clone(), torch.cuda.Stream()
+    gu.sync()
+    with torch.cuda.stream(stream):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            got = linear.run(x)
+    for _ in range(3):
+        linear.out.zero_()
+        gu.sync()
+        graph.replay()
+        gu.sync()
+        assert torch.equal(got, want)
+
+
+def test_panels_are_refused_where_no_kernel_serves_them():
+    for symbol, variant in (("activation_quantization", dict(K=1000, panels=True)), ("activation_quantization", dict(K=256, group_size=128, panels=True)),
+                            ("activation_quantization", dict(K=256, fused=True, panels=True)), ("activation_quantization", dict(K=32896, panels=True)),
+                            ("e8p_q4_projection", dict(M=512, N=256, K=128, panels=True)), ("e8p_q4_projection", dict(M=2049, N=256, K=256, panels=True)),
+                            ("e8p_q4_projection", dict(M=64, N=256, K=256, panels=True, algorithm="runs")),
+                            ("e8p_q4_projection", dict(M=64, N=256, K=256, panels=True, workspace=True))):
+        with pytest.raises(gu.lib.OrxError):
+            gu.lib.Kernel(symbol, **variant)
