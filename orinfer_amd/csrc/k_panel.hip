@@ -10,8 +10,8 @@
 //    (113-120 GB/s per CU, all CUs reading the same rows; out of row-major memory 16 rows x 64 bytes at a time 35 GB/s).  Through LDS,
 //    as k_gemm_big.hip's 512-row runs take row-major rows, whole lines arrive as fast, but what is in flight has to have its place there: 128 of the
 //    160 KiB, which leaves the decode tables without copies and every lookup in bank conflicts.
-//  * A workgroup owns up to 512 token rows and a run of up to CB blocks of 16 channels over the whole K; wave w of eight owns TB blocks
-//    of 16 rows and all channels of the run.  The tokens of D MFMA slices of 64 are on their way in registers (TB D = 16 KiB a wave).
+//  * A workgroup owns up to 512 token rows and a run of up to CB blocks of 16 channels over the whole K; wave w of eight owns TB or TB - 1 blocks
+//    of 16 rows (w, w + 8, ...) and all channels of the run.  The tokens of D MFMA slices of 64 are on their way in registers (TB D = 16 KiB a wave).
 //  * K goes by in phases of PH chunks of 128.  While the weights of one phase are multiplied, those of the next are decoded: a unit is 16
 //    channels x 128 of K, 16 bytes of codes to a lane, four lookups a code in tables of eight copies (QuadLookup: no bank conflicts),
 //    and what a lane decodes is what a lane of the fragment reads, so both sides of the LDS are linear.  One barrier a phase, behind its
@@ -22,8 +22,8 @@
 // rows, us: 49.5; without the token requests 40.7, without the lookups 44.9, with a quarter of the multiplies 44.3.  Four waves of twice the rows (half the fragment
 // reads, sums in accumulation registers) 50-54, eight token slices instead of four, two slices to a step, a raised wave priority, lookups
 // put together later: all within 2 %.  Before, the best of all other kernels, with the A8 quantiser (here 0.1-0.7 us slower, for the second copy of the codes):
-// 17408 x 5120 at 200 / 512 rows 57.6 / 68.2 -> 36.9 / 53.8, 7168 x 5120 at 200 / 256 / 512 rows 25.1 / 41.3 / 56.1 -> 23.4 / 24.2 / 37.3, 9728 x 2560 at 200 / 512 30.4 /
-// 37.7 -> 19.0 / 27.6.
+// 17408 x 5120 at 200 / 512 rows 57.6 / 68.2 -> 35.7 / 53.2, 7168 x 5120 at 200 / 256 / 512 rows 25.1 / 41.3 / 56.1 -> 21.5 / 23.8 / 37.2, 9728 x 2560 at 200 / 512 30.4 /
+// 37.7 -> 18.0 / 26.4.
 #include <hip/hip_fp16.h>
 
 #include <algorithm>
@@ -85,7 +85,9 @@ __device__ __forceinline__ void write_16_at(uint32_t address, v4u value) {
     asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(address), "v"(value), "n"(OFFSET) : "memory");
 }
 
-template <int TB, int CB>
+// EVEN: every wave has TB blocks of rows (a branch less, and all multiplies to put the side work behind: 17408 x 5120 at 512 rows 51.2 -> 49.9; the other form leaves
+// out what is not there: 7168 x 5120 at 130 / 200 rows 18.4 / 19.2 -> 16.2 / 18.3, 17408 x 5120 at 130 rows 31.1 -> 28.1)
+template <int TB, int CB, bool EVEN>
 __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
     constexpr int PH = kPhaseChunks<CB>, S = 2 * PH;      // chunks and MFMA slices of a phase
     constexpr int D = 4;                                  // token slices on their way (eight are not faster)
@@ -133,8 +135,9 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
     const uint8_t* token_base[TB];
     Each<TB>::run([&](auto tag) ORX_INLINE {
         constexpr int i = decltype(tag)::value;
-        token_base[i] = uniform_pointer(p.panels + (int64_t)(first_row / 16 + min(wave * TB + i, row_blocks - 1)) * 16 * p.k);
+        token_base[i] = uniform_pointer(p.panels + (int64_t)(first_row / 16 + min(i * kPanelWaves + wave, row_blocks - 1)) * 16 * p.k);
     });
+    const bool last_block = EVEN || (TB - 1) * kPanelWaves + wave < row_blocks;  // (all others every wave has: row_blocks > 8 (TB - 1), see panel_shape)
     v4i token[D][TB];
     const int last_slice = 2 * chunks - 1;
     auto token_offset = [&](int slice) ORX_INLINE { return (uint32_t)lane * 16 + (uint32_t)min(slice, last_slice) * 1024; };
@@ -148,12 +151,12 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
         const uint32_t offset = token_offset(decltype(s_tag)::value);
         Each<TB>::run([&](auto i_tag) ORX_INLINE {
             constexpr int i = decltype(i_tag)::value;
-            request_token(token[decltype(s_tag)::value][i], offset, token_base[i]);
+            if (i < TB - 1 || last_block) request_token(token[decltype(s_tag)::value][i], offset, token_base[i]);
         });
     });
 
     // ---- tables: half an entry to a thread ----
-    constexpr int kLater = 2 * U + TB * D;
+    constexpr int kLater = 2 * U + (TB - 1) * D;  // at least
     asm volatile("s_waitcnt vmcnt(%4)" : "+v"(selector), "+v"(token_scale_bits), "+v"(row_sum), "+v"(channel_scale_bits) : "n"(kLater > 63 ? 63 : kLater));
     {
         const uint32_t entry = (uint32_t)tid & 255, half = (uint32_t)tid >> 8, turn = entry & 7;
@@ -204,7 +207,7 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
     std::integral_constant<int, 1> one;
     // the first phase by itself
     {
-        constexpr int kAfter = U + TB * D;
+        constexpr int kAfter = U + (TB - 1) * D;
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kAfter > 63 ? 63 : kAfter) : "memory");
         Each<U>::run([&](auto tag) ORX_INLINE { keep(first_codes[decltype(tag)::value]); });
         Each<U>::run([&](auto tag) ORX_INLINE {
@@ -248,7 +251,10 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
         constexpr bool kLooksUp = s < 2 * U, kPutsTogether = s >= 1 && s <= 2 * U;
         constexpr int u = s / 2, before = (s - 1) / 2;
         // this slice's tokens, and with them the codes, which were requested S - 1 slices ago: at most the tokens of D - 1 slices are younger
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(TB * (D - 1)) : "memory");
+        if (last_block)
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(TB * (D - 1)) : "memory");
+        else
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((TB - 1) * (D - 1)) : "memory");
         Each<CB>::run([&](auto tag) ORX_INLINE { keep(weight[set][decltype(tag)::value]); });
         Each<TB>::run([&](auto tag) ORX_INLINE { keep(token[token_set][decltype(tag)::value]); });
         if constexpr (kLooksUp) keep(codes[u]);
@@ -258,14 +264,14 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
             if (before < U - 1 || last_unit) write_16_at<((s - 1) & 1) * (CB * 1024)>(unit_weights[before] + (phase & 1 ? 0u : kPhaseBytes<CB>), combine());
         }
         const uint32_t offset = token_offset(phase * S + s + D);
-        constexpr int kMultiplies = TB * CB;
         const uint32_t next = s == S - 1 ? phase_weights + other : phase_weights;
+        // Side work behind the multiplies that every wave has, one piece each where there are that many: two codes of four lookups, then CB fragment
+        // reads (what goes out last is waited for first, at the next slice's start).
+        constexpr int kMultiplies = (EVEN ? TB : TB - 1) * CB, kSide = CB + 2, kSpan = kMultiplies < 2 * kSide ? kMultiplies : 2 * kSide;
         Each<kMultiplies>::run([&](auto m_tag) ORX_INLINE {
             constexpr int m = decltype(m_tag)::value, i = m / CB, j = (i & 1) ? CB - 1 - m % CB : m % CB;
             multiply_in_place<false>(acc[i][j], weight[set][j], token[token_set][i]);
-            // side work behind the first two thirds of the multiplies, at most one piece each where they suffice: two codes of four lookups, then CB
-            // fragment reads (what goes out last is waited for first, at the next slice's start)
-            constexpr int kSide = CB + 2, kSpan = kMultiplies < 2 * kSide ? kMultiplies : 2 * kSide, from = m * kSide / kSpan, to = (m + 1) * kSide / kSpan;
+            constexpr int from = m * kSide / kSpan, to = (m + 1) * kSide / kSpan;
             Each<kSide>::run([&](auto n_tag) ORX_INLINE {
                 constexpr int n = decltype(n_tag)::value;
                 if constexpr (n >= from && n < to) {
@@ -278,6 +284,13 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
             });
             if constexpr (m % CB == CB - 1) request_token(token[token_set][i], offset, token_base[i]);
         });
+        if (!EVEN && last_block) {
+            Each<CB>::run([&](auto j_tag) ORX_INLINE {
+                constexpr int i = TB - 1, j = (i & 1) ? CB - 1 - decltype(j_tag)::value : decltype(j_tag)::value;
+                multiply_in_place<false>(acc[i][j], weight[set][j], token[token_set][i]);
+            });
+            request_token(token[token_set][TB - 1], offset, token_base[TB - 1]);
+        }
         if constexpr (kLooksUp && (s & 1) == 1) request_codes(phase + 2, std::integral_constant<int, u>{}, codes[u]);
     };
     for (;; ++phase) {
@@ -311,13 +324,13 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
     for (int j = 0; j < CB; ++j) channel_scale[j] = *reinterpret_cast<const float4*>(lds + kPanelScales<CB> + kPanelRows * 8 + (16 * j + 4 * quarter) * 4);
 #pragma unroll
     for (int i = 0; i < TB; ++i) {
-        const int row = (wave * TB + i) * 16 + column;
+        const int row = (i * kPanelWaves + wave) * 16 + column;
         token_scale[i] = token_scales[row], bias[i] = kQuadBias * sums[row];
     }
     if (p.out_f32) {
 #pragma unroll
         for (int i = 0; i < TB; ++i) {
-            const int row = (wave * TB + i) * 16 + column;
+            const int row = (i * kPanelWaves + wave) * 16 + column;
             if (row >= rows) continue;
             float* const to = reinterpret_cast<float*>(p.out) + (int64_t)(first_row + row) * p.stride + first_channel;
 #pragma unroll
@@ -342,7 +355,7 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
 #pragma unroll
         for (int t = 0; t < (16 * kPieces + 63) / 64; ++t) {
             const int number = t * 64 + lane, local = number / kPieces, piece = number % kPieces;
-            const int row = (wave * TB + i) * 16 + local;
+            const int row = (i * kPanelWaves + wave) * 16 + local;
             if (local >= 16 || row >= rows || piece * 8 >= channels) continue;
             const uint4 value = *reinterpret_cast<const uint4*>(from + local * kPitch + piece * 16);
             __half* const to = out + (int64_t)row * p.stride + piece * 8;
@@ -376,14 +389,15 @@ struct PanelForm {
     const void* kernel;
     uint32_t shared;
 };
-// by blocks of 16 rows to a wave (2 to 4) and of channels to a workgroup (1 to 5)
-const PanelForm& panel_form(int tb, int cb) {
-#define ORX_PANEL(T, C) {reinterpret_cast<const void*>(&panel_kernel<T, C>), kPanelLds<C>}
-#define ORX_PANELS(T) {ORX_PANEL(T, 1), ORX_PANEL(T, 2), ORX_PANEL(T, 3), ORX_PANEL(T, 4), ORX_PANEL(T, 5)}
-    static const PanelForm forms[3][5] = {ORX_PANELS(2), ORX_PANELS(3), ORX_PANELS(4)};
+// by blocks of 16 rows to a wave (2 to 4), whether every wave has as many, and blocks of channels to a workgroup (1 to 5)
+const PanelForm& panel_form(int tb, bool even, int cb) {
+#define ORX_PANEL(T, E, C) {reinterpret_cast<const void*>(&panel_kernel<T, C, E>), kPanelLds<C>}
+#define ORX_PANELS(T, E) {ORX_PANEL(T, E, 1), ORX_PANEL(T, E, 2), ORX_PANEL(T, E, 3), ORX_PANEL(T, E, 4), ORX_PANEL(T, E, 5)}
+    static const PanelForm forms[6][5] = {ORX_PANELS(2, false), ORX_PANELS(2, true), ORX_PANELS(3, false),
+                                          ORX_PANELS(3, true),  ORX_PANELS(4, false), ORX_PANELS(4, true)};
 #undef ORX_PANELS
 #undef ORX_PANEL
-    return forms[tb - 2][cb - 1];
+    return forms[2 * (tb - 2) + even][cb - 1];
 }
 
 struct PanelShape {
@@ -396,7 +410,9 @@ PanelShape panel_shape(int rows, int n) {
     s.tile_rows = ((rows + s.row_tiles - 1) / s.row_tiles + 15) / 16 * 16;
     s.units = (int)gemm_tall_units(n);
     const int blocks = (n + 15) / 16, tb = std::max(2, (s.tile_rows / 16 + kPanelWaves - 1) / kPanelWaves);
-    s.form = &panel_form(tb, (blocks + s.units - 1) / s.units);
+    const int last_rows = rows - (s.row_tiles - 1) * s.tile_rows;  // of the last tile
+    const bool even = s.tile_rows == tb * kPanelWaves * 16 && last_rows > s.tile_rows - 16;
+    s.form = &panel_form(tb, even, (blocks + s.units - 1) / s.units);
     return s;
 }
 
@@ -416,13 +432,12 @@ int panel_launch(const uint8_t* panels, const int* sums, const void* w, const ui
                  int rows, int n, int k, int stride, int packed_k, bool out_f32, hipStream_t stream) {
     static DeviceOnce opted_in;  // dynamic LDS above 64 KiB needs an opt-in per kernel and device
     const int ready = opted_in.run([] {
-        for (int tb = 2; tb <= 4; ++tb)
-            for (int cb = 1; cb <= 5; ++cb) {
-                const PanelForm& form = panel_form(tb, cb);
-                const int code = hip_check(hipFuncSetAttribute(form.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)form.shared),
-                                           "hipFuncSetAttribute");
-                if (code != ORX_OK) return code;
-            }
+        for (int of = 0; of < 6 * 5; ++of) {
+            const PanelForm& form = panel_form(2 + of / 10, of / 5 % 2, 1 + of % 5);
+            const int code = hip_check(hipFuncSetAttribute(form.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)form.shared),
+                                       "hipFuncSetAttribute");
+            if (code != ORX_OK) return code;
+        }
         return (int)ORX_OK;
     });
     if (ready != ORX_OK) return ready;
