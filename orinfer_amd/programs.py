@@ -24,24 +24,34 @@ PANEL_ROWS = 1024
 
 
 def panels_pay(rows, n, k, cus):
-    """Whether quantiser and projection of two-stage codes are faster over token panels than row-major (time of the pair over panels / row-major, 256 CUs):
-    65-128 rows 0.78-0.97 with 4 to 5 blocks of 16 channels to a CU, 0.9-1.3 otherwise.  Up to one block 1.0-2.1 at 129-512 rows; at 513-1024 0.44-0.95 up to
-    K = 4096, 0.75-1.5 beyond.  One to two blocks, where the channel runs fill one round (up to 240 rows; 257-384 of up to 1.3 blocks): 5120 channels 0.99-1.4, 7168 and
-    8192 at 130-160 / 200 rows 0.91-1.15 / 0.86-1.01; other rows up to 512 0.41-1.01, 513-1024 0.64-0.98 (5120 x 8192 and x 12288 at 640-768 rows 1.0-1.12).
-    Wider: 0.42-0.91 at 129-512 rows, 0.69-0.86 at 513-768 (34816 x 1024-2048 0.95-1.04), 0.66-0.99 at 1024 (K = 1024 0.66-1.13).  Beyond 1024 rows decoding once is mostly
-    faster (1280 rows 0.72-1.5)."""
+    """Whether quantiser and projection of two-stage codes are faster over token panels than row-major (time of the pair over panels / row-major, 256 CUs,
+    by blocks of 16 channels to a CU).
+    65-128 rows: 4 to 5 blocks 0.65-0.84; more than 6 0.82-0.98 from 97 rows on, below 0.85-1.04; up to 2 blocks 0.77-0.96 above 112 rows, 0.81-0.98 above 96 up to
+    K = 5120, 0.83-0.98 at K = 1024, otherwise to 1.3; 2 to 4 blocks 0.76-0.87 at K = 1024, 0.79-0.96 at K = 2048 above 80 rows, otherwise to 1.27; 5 to 6 1.0-1.1.
+    Where the channel runs fill one round (up to 240 rows of up to 2 blocks, 257-384 of up to 1.3): up to one block 0.90-0.95 at K = 1024, 0.96-1.3 beyond;
+    1.2 to 1.5 0.87-0.97 up to K = 2048, 0.96-1.12 beyond; 1.75 and 2 0.81-0.98; 257-384 rows 1.05-1.3.
+    Elsewhere up to 512 rows: up to one block 1.1-2.2, wider 0.36-0.98 (5120 x 12288 1.01).  513-1024 rows: up to one block 0.44-1.02 up to K = 4096, 0.75-1.5
+    beyond; wider 0.64-0.99 (5120 x 8192 and x 12288 at 640-768 rows 1.0-1.12, K below 2048 at 1024 rows 0.66-1.13).  Beyond 1024 rows decoding once is mostly faster
+    (1280 rows 0.72-1.5)."""
     if not 64 < rows <= PANEL_ROWS:
         return False
     blocks = -(-n // 16)
     if rows <= 128:
-        return 4 * cus < blocks <= 5 * cus
-    if blocks <= cus:
-        return rows > 512 and k <= 4096
-    if rows > 768 and k < 2048 or rows > 512 and 4 * blocks <= 5 * cus and k > 5120:
-        return False
+        if blocks <= 2 * cus:
+            return rows > 112 or k <= (5120 if rows > 96 else 1024)
+        if blocks <= 4 * cus:
+            return k <= (2048 if rows > 80 else 1024)
+        return blocks <= 5 * cus or (blocks > 6 * cus and rows > 96)
+    if rows > 512:
+        if blocks <= cus:
+            return k <= 4096
+        return (rows <= 768 or k >= 2048) and (4 * blocks > 5 * cus or k <= 5120)
     row_tiles = -(-rows // 128)
-    one_round = blocks <= 2 * cus and row_tiles * -(-blocks // 4) <= cus and not 240 < rows <= 256  # the channel runs take these
-    return not one_round or (rows > 176 and 4 * blocks > 6 * cus)
+    if blocks <= 2 * cus and row_tiles * -(-blocks // 4) <= cus and not (240 < rows <= 256 and blocks > cus):  # the channel runs in one round
+        if rows > 256:
+            return False
+        return k <= 1024 or (blocks > cus and k <= 2048) or 2 * blocks > 3 * cus
+    return blocks > cus
 
 
 class QuantizedLinear:

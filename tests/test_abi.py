@@ -323,10 +323,11 @@ def test_which_rows_of_codes_the_channel_runs_take_in_several_rounds(n, k, rows,
 
 
 @pytest.mark.parametrize("n, k, lines", [
-    (4096, 4096, [(128, 0), (512, 0), (513, 1), (1024, 1), (1025, 0)]), (4096, 4224, [(513, 0), (1024, 0)]),
-    (5120, 5120, [(176, 0), (240, 0), (241, 1), (256, 1), (257, 0), (384, 0), (385, 1), (768, 1), (1024, 1)]), (5120, 8192, [(512, 1), (513, 0)]),
-    (7168, 5120, [(128, 0), (176, 0), (177, 1), (240, 1), (512, 1), (1024, 1)]), (12288, 1024, [(128, 0), (129, 1), (768, 1), (769, 0)]),
-    (17408, 5120, [(64, 0), (65, 1), (1024, 1), (1025, 0)]), (34816, 5120, [(128, 0), (129, 1)]),
+    (4096, 4096, [(96, 0), (97, 1), (128, 1), (129, 0), (512, 0), (513, 1), (1024, 1), (1025, 0)]), (4096, 1024, [(64, 0), (65, 1), (256, 1), (257, 0)]),
+    (4096, 4224, [(513, 0), (1024, 0)]), (4096, 5248, [(112, 0), (113, 1)]),
+    (5120, 5120, [(129, 0), (240, 0), (241, 1), (256, 1), (257, 0), (384, 0), (385, 1), (768, 1), (1024, 1)]), (5120, 8192, [(512, 1), (513, 0)]), (5120, 2048, [(129, 1)]),
+    (7168, 5120, [(96, 0), (129, 1), (512, 1), (1024, 1)]), (12288, 1024, [(65, 1), (129, 1), (768, 1), (769, 0)]), (12288, 2048, [(80, 0), (81, 1)]), (12288, 2176, [(128, 0)]),
+    (17408, 5120, [(64, 0), (65, 1), (1024, 1), (1025, 0)]), (24576, 5120, [(128, 0), (129, 1)]), (34816, 5120, [(96, 0), (97, 1)]),
 ])
 def test_which_rows_a_linear_takes_over_panels(n, k, lines):
     from orinfer_amd.programs import panels_pay
