@@ -52,8 +52,8 @@ bool runs_eligible(int codec, int rows, int n, int k);
 int runs_rounds(int codec, int rows, int n, int* tile_rows, int* run);
 void runs_geometry(int codec, int rows, int n, Geometry* g);
 bool panel_eligible(int rows, int n, int k);  // k_panel.hip
-void panel_geometry(int rows, int n, Geometry* g);
-int panel_launch(const uint8_t* panels, const int* sums, const void* w, const uint32_t* book, const __half* ws, const __half* as, void* out,
+void panel_geometry(int codec, int rows, int n, Geometry* g);  // codec: 0 two-stage codes, 1 int8
+int panel_launch(int codec, const uint8_t* panels, const int* sums, const void* w, const uint32_t* book, const __half* ws, const __half* as, void* out,
                  int rows, int n, int k, int stride, int packed_k, bool out_f32, hipStream_t stream);
 int runs_launch(int codec, const int8_t* a, const void* w, const uint32_t* book, const __half* ws, const __half* as, void* out,
                 int rows, int n, int k, int stride, int packed_k, bool out_f32, hipStream_t stream);
@@ -1314,16 +1314,35 @@ int make_projection(const Variant& v, orx_function* f, int codec) {
     return ORX_OK;
 }
 
-// Token rows as panels (the quantiser's, of the same key): A, AS, Book, Out, S, Sums, W[, m]
+// Token rows as panels (the quantiser's, of the same key): A, AS, Book, Out, S, Sums, W[, m] and A, Output, TokenScale, Weight, WeightScale[, m]
 int q4_panel_geometry(const orx_function& f, int rows, Geometry* g) {
-    panel_geometry(rows, f.N, g);
+    panel_geometry(0, rows, f.N, g);
     return ORX_OK;
 }
 int q4_panel_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t stream, void** args) {
     (void)g;
-    return panel_launch(pointer_arg<const uint8_t>(args, 0), pointer_arg<const int>(args, 5), pointer_arg<const void>(args, 6), pointer_arg<const uint32_t>(args, 2),
+    return panel_launch(0, pointer_arg<const uint8_t>(args, 0), pointer_arg<const int>(args, 5), pointer_arg<const void>(args, 6), pointer_arg<const uint32_t>(args, 2),
                         pointer_arg<const __half>(args, 4), pointer_arg<const __half>(args, 1), pointer_arg<void>(args, 3), rows, f.N, f.K, f.stride, f.packed_k,
                         f.out_f32, stream);
+}
+int w8_panel_geometry(const orx_function& f, int rows, Geometry* g) {
+    panel_geometry(1, rows, f.N, g);
+    return ORX_OK;
+}
+int w8_panel_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t stream, void** args) {
+    (void)g;
+    return panel_launch(1, pointer_arg<const uint8_t>(args, 0), nullptr, pointer_arg<const void>(args, 3), nullptr, pointer_arg<const __half>(args, 4),
+                        pointer_arg<const __half>(args, 2), pointer_arg<void>(args, 1), rows, f.N, f.K, f.stride, 0, f.out_f32, stream);
+}
+// panels=true of a projection: whether it is asked for; refuses what the panel kernel does not serve
+int panels_asked(const Variant& v, const orx_function& f, bool* asked) {
+    bool bad = false;
+    *asked = v.boolean("panels", false, &bad);
+    if (bad || (*asked && (f.input_f16 || v.string("algorithm", "auto", &bad) != "auto" || f.tiles != 0 || f.takes_workspace || !panel_eligible(f.capacity, f.N, f.K)))) {
+        set_error("%s: panels=true serves int8 rows, up to 2048 of them, K a multiple of 128 from 256, algorithm auto, without block_m and workspace", f.symbol.c_str());
+        return ORX_ERR_BAD_VARIANT;
+    }
+    return ORX_OK;
 }
 
 int make_q4_projection(const Variant& v, orx_function* f) {
@@ -1359,12 +1378,9 @@ int make_q4_projection(const Variant& v, orx_function* f) {
         set_error("e8p_q4_projection: codes=true needs input_dtype=float16");
         return ORX_ERR_BAD_VARIANT;
     }
-    const bool panels = v.boolean("panels", false, &bad);
-    if (bad || (panels && (f->input_f16 || v.string("algorithm", "auto", &bad) != "auto" || f->tiles != 0 || f->takes_workspace ||
-                           !panel_eligible(f->capacity, f->N, f->K)))) {
-        set_error("e8p_q4_projection: panels=true serves int8 rows, up to 2048 of them, K from 256, algorithm auto, without block_m and workspace");
-        return ORX_ERR_BAD_VARIANT;
-    }
+    bool panels = false;
+    code = panels_asked(v, *f, &panels);
+    if (code != ORX_OK) return code;
     if (panels) {
         f->args = {{"A", ArgPointer, 16}, {"AS", ArgPointer, 2}, {"Book", ArgPointer, 4}, {"Out", ArgPointer, 2}, {"S", ArgPointer, 2}, {"Sums", ArgPointer, 4}, {"W", ArgPointer, 16}};
         if (f->dynamic_rows) f->args.push_back({"m", ArgI32, 4});
@@ -1387,11 +1403,15 @@ int make_q4_projection(const Variant& v, orx_function* f) {
 int make_w8_projection(const Variant& v, orx_function* f) {
     int code = make_projection(v, f, kW8);
     if (code != ORX_OK) return code;
+    bool panels = false;
+    code = panels_asked(v, *f, &panels);
+    if (code != ORX_OK) return code;
     f->args = {{"A", ArgPointer, 16},     {"Output", ArgPointer, 2},      {"TokenScale", ArgPointer, 2},
                {"Weight", ArgPointer, 16}, {"WeightScale", ArgPointer, 2}};
     if (f->takes_workspace) f->args.push_back({"Workspace", ArgPointer, 256u | 0x80000000u});
     if (f->dynamic_rows) f->args.push_back({"m", ArgI32, 4});
     f->launch = w8_launch;
+    if (panels) f->workspace_need = nullptr, f->geometry = w8_panel_geometry, f->launch = w8_panel_launch;
     return ORX_OK;
 }
 
@@ -2196,7 +2216,7 @@ const Registration* gemm_registrations(int* count) {
      "output_stride=N, block_m=0|32|64|128|256, gemv_passes=0, decode_in_gemm=false",
      "A,AS,Book,Out[,Q],S[,Signs][,Sums],W[,Workspace][,m]"},
     {"int8_projection", make_w8_projection,
-     "M, N, K, dynamic_rows=false, algorithm=auto|gemv|stream|runs|mfma, output_dtype=float16|float32, output_stride=N, "
+     "M, N, K, dynamic_rows=false, algorithm=auto|gemv|stream|runs|mfma, output_dtype=float16|float32, output_stride=N, panels=false, "
      "block_m=0|32|64|128|256, workspace=false, split_k=true",
      "A,Output,TokenScale,Weight,WeightScale[,Workspace][,m]"},
     {"int8_small_projection", make_w8_small_projection,

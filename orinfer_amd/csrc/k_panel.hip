@@ -1,8 +1,8 @@
-// Projections of two-stage (Q4) codes for 129 rows to some thousand: token rows as packed panels, operands of the tokens straight into
-// registers, the weights of a workgroup decoded once through LDS.
+// Projections of two-stage (Q4) codes and of int8 weights for some dozens of rows to some thousand: token rows as packed panels, straight into
+// the operand registers, the weights of a workgroup decoded (or brought) once into LDS.
 //
 // Reference counterparts: the Tensor Core schedules of kernels/cuda/model/integer_core.py behind
-// kernels/cuda/model/e8p_q4.py:143-264.  Arithmetic: exact int32 over the full K, (float(acc) * ws) * as.
+// kernels/cuda/model/e8p_q4.py:143-264 and int8_projection.py:15-62.  Arithmetic: exact int32 over the full K, (float(acc) * ws) * as.
 //
 //  * The quantiser leaves the int8 rows as panels besides (k_quant.hip): 1 KiB for 16 rows and 64 of K, in the order in which the
 //    lanes of v_mfma_i32_16x16x64_i8 hold them: half s of a chunk of 128, lane (quarter q, row i): bytes [32 q + 16 s, +16) of row i,
@@ -16,6 +16,7 @@
 //    channels x 128 of K, 16 bytes of codes to a lane, four lookups a code in tables of eight copies (QuadLookup: no bank conflicts),
 //    and what a lane decodes is what a lane of the fragment reads, so both sides of the LDS are linear.  One barrier a phase, behind its
 //    second last slice.  Row sums (75 times them comes off, see QuadLookup) are the quantiser's.
+//  * int8 weights go to the same places by direct-to-LDS loads, two to a unit, in the first slices of the phase before.
 //
 // What bounds it: the token stream and the LDS (fragments 8 KiB x CB a slice for the eight waves, lookups 4 KiB x CB), which add up more than they overlap:
 // 64 of K take 0.08 us per 16 KiB of tokens and 0.045 us per channel block, the multiplies beside them 0.005 us per block of 16 x 16 and wave.  17408 x 5120 at 512
@@ -70,15 +71,17 @@ struct PanelParams {
     uint32_t row_stride, chunk_stride, half_stride;  // code bytes between channels, K chunks of 128, and halves of a chunk
 };
 
-constexpr uint32_t kPanelWeights = kQuadTableBytes<256>;
+enum PanelCodec { kPanelQ4 = 0, kPanelW8 = 1 };
+template <int CODEC>
+constexpr uint32_t kPanelWeights = CODEC == kPanelQ4 ? kQuadTableBytes<256> : 0;
 template <int CB>
 constexpr int kPhaseChunks = CB <= 2 ? 8 : 4;
 template <int CB>
 constexpr uint32_t kPhaseBytes = CB * kPhaseChunks<CB> * 2048;
-template <int CB>
-constexpr uint32_t kPanelScales = kPanelWeights + 2 * kPhaseBytes<CB>;  // 512 token scales, 512 sums, 16 CB channel scales
-template <int CB>
-constexpr uint32_t kPanelLds = kPanelScales<CB> + kPanelRows * 8 + CB * 64;
+template <int CODEC, int CB>
+constexpr uint32_t kPanelScales = kPanelWeights<CODEC> + 2 * kPhaseBytes<CB>;  // 512 token scales, 512 sums, 16 CB channel scales
+template <int CODEC, int CB>
+constexpr uint32_t kPanelLds = kPanelScales<CODEC, CB> + kPanelRows * 8 + CB * 64;
 
 template <int OFFSET>
 __device__ __forceinline__ void write_16_at(uint32_t address, v4u value) {
@@ -87,13 +90,15 @@ __device__ __forceinline__ void write_16_at(uint32_t address, v4u value) {
 
 // EVEN: every wave has TB blocks of rows (a branch less, and all multiplies to put the side work behind: 17408 x 5120 at 512 rows 51.2 -> 49.9; the other form leaves
 // out what is not there: 7168 x 5120 at 130 / 200 rows 18.4 / 19.2 -> 16.2 / 18.3, 17408 x 5120 at 130 rows 31.1 -> 28.1)
-template <int TB, int CB, bool EVEN>
+template <int CODEC, int TB, int CB, bool EVEN>
 __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
+    constexpr bool Q4 = CODEC == kPanelQ4;
+    constexpr uint32_t kWeights = kPanelWeights<CODEC>, kScales = kPanelScales<CODEC, CB>;
     constexpr int PH = kPhaseChunks<CB>, S = 2 * PH;      // chunks and MFMA slices of a phase
     constexpr int D = 4;                                  // token slices on their way (eight are not faster)
     constexpr int UNITS = PH * CB, U = (UNITS + kPanelWaves - 1) / kPanelWaves;
     constexpr bool kUneven = UNITS % kPanelWaves != 0;    // the last unit of a phase is some waves' only
-    static_assert(2 * U + 1 < S && S % D == 0 && S - 1 > D, "the decode of a phase ends in front of its barrier");
+    static_assert((Q4 ? 2 * U + 1 < S : U + D < S) && S % D == 0 && S - 1 > D, "the decode of a phase ends in front of its barrier");
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -105,13 +110,13 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
     const int chunks = p.k / 128;
 
     // ---- requests: what the set-up needs, the codes of two phases, the first token slices ----
-    uint32_t selector, token_scale_bits, channel_scale_bits;
-    int row_sum;
+    uint32_t selector = 0, token_scale_bits, channel_scale_bits;
+    int row_sum = 0;
     {
         const uint32_t entry_at = (uint32_t)(tid & 255) * 4, row_at = (uint32_t)min(tid, rows - 1), channel_at = (uint32_t)min(tid, channels - 1);
-        asm volatile("global_load_dword %0, %1, %2" : "=v"(selector) : "v"(entry_at), "s"(uniform_pointer(p.book)) : "memory");
+        if constexpr (Q4) asm volatile("global_load_dword %0, %1, %2" : "=v"(selector) : "v"(entry_at), "s"(uniform_pointer(p.book)) : "memory");
         asm volatile("global_load_ushort %0, %1, %2" : "=v"(token_scale_bits) : "v"(row_at * 2), "s"(uniform_pointer(p.as + first_row)) : "memory");
-        asm volatile("global_load_dword %0, %1, %2" : "=v"(row_sum) : "v"(row_at * 4), "s"(uniform_pointer(p.sums + first_row)) : "memory");
+        if constexpr (Q4) asm volatile("global_load_dword %0, %1, %2" : "=v"(row_sum) : "v"(row_at * 4), "s"(uniform_pointer(p.sums + first_row)) : "memory");
         asm volatile("global_load_ushort %0, %1, %2" : "=v"(channel_scale_bits) : "v"(channel_at * 2), "s"(uniform_pointer(p.ws + first_channel)) : "memory");
     }
     const uint8_t* const w_base = uniform_pointer(p.w + (int64_t)first_channel * p.row_stride);
@@ -122,14 +127,24 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
         constexpr int u = decltype(tag)::value;
         const int number = min(wave + kPanelWaves * u, UNITS - 1), block = number % CB;
         unit_chunk[u] = number / CB;
-        unit_codes[u] = (uint32_t)min(16 * block + column, channels - 1) * p.row_stride + (uint32_t)(quarter >> 1) * p.half_stride + (uint32_t)(quarter & 1) * 16;
-        unit_weights[u] = kPanelWeights + (uint32_t)(unit_chunk[u] * 2 * CB + block) * 1024 + (uint32_t)lane * 16;
+        unit_codes[u] = (uint32_t)min(16 * block + column, channels - 1) * p.row_stride;
+        if constexpr (Q4)
+            unit_codes[u] += (uint32_t)(quarter >> 1) * p.half_stride + (uint32_t)(quarter & 1) * 16;
+        else
+            unit_codes[u] += (uint32_t)quarter * 32;
+        unit_weights[u] = kWeights + (uint32_t)(unit_chunk[u] * 2 * CB + block) * 1024 + (Q4 ? (uint32_t)lane * 16 : 0u);
     });
     const bool last_unit = !kUneven || wave + kPanelWaves * (U - 1) < UNITS;
     v4u codes[U];
     auto request_codes = [&](int phase, auto tag, v4u& to) ORX_INLINE {
         constexpr int u = decltype(tag)::value;
         load_16(to, unit_codes[u], w_base + (uint64_t)(uint32_t)min(phase * PH + unit_chunk[u], chunks - 1) * p.chunk_stride);
+    };
+    auto bring = [&](int phase, auto tag) ORX_INLINE {  // int8: a unit of a phase to its place
+        constexpr int u = decltype(tag)::value;
+        const uint8_t* const from = w_base + (uint64_t)(uint32_t)min(phase * PH + unit_chunk[u], chunks - 1) * p.chunk_stride;
+        const uint32_t to = unit_weights[u] + (phase & 1 ? kPhaseBytes<CB> : 0u);
+        if (u < U - 1 || last_unit) request_16<true, 0>(unit_codes[u], from, to), request_16<true, 0>(unit_codes[u] + 16, from, to + CB * 1024);
     };
     const int row_blocks = (rows + 15) / 16;
     const uint8_t* token_base[TB];
@@ -145,8 +160,12 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
         asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(to) : "v"(offset), "s"(base) : "memory");
     };
     v4u first_codes[U];
-    Each<U>::run([&](auto tag) ORX_INLINE { request_codes(0, tag, first_codes[decltype(tag)::value]); });
-    Each<U>::run([&](auto tag) ORX_INLINE { request_codes(1, tag, codes[decltype(tag)::value]); });
+    if constexpr (Q4) {
+        Each<U>::run([&](auto tag) ORX_INLINE { request_codes(0, tag, first_codes[decltype(tag)::value]); });
+        Each<U>::run([&](auto tag) ORX_INLINE { request_codes(1, tag, codes[decltype(tag)::value]); });
+    } else {
+        Each<U>::run([&](auto tag) ORX_INLINE { bring(0, tag); });
+    }
     Each<D>::run([&](auto s_tag) ORX_INLINE {
         const uint32_t offset = token_offset(decltype(s_tag)::value);
         Each<TB>::run([&](auto i_tag) ORX_INLINE {
@@ -156,9 +175,9 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
     });
 
     // ---- tables: half an entry to a thread ----
-    constexpr int kLater = 2 * U + (TB - 1) * D;  // at least
+    constexpr int kLater = (Q4 ? 2 * U : 0) + (TB - 1) * D;  // at least
     asm volatile("s_waitcnt vmcnt(%4)" : "+v"(selector), "+v"(token_scale_bits), "+v"(row_sum), "+v"(channel_scale_bits) : "n"(kLater > 63 ? 63 : kLater));
-    {
+    if constexpr (Q4) {
         const uint32_t entry = (uint32_t)tid & 255, half = (uint32_t)tid >> 8, turn = entry & 7;
         const int shift = half ? 0 : 2;
         const uint2 basis = byte_basis_biased(selector, shift), mask = byte_mask_biased(entry, shift);
@@ -168,7 +187,9 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
         const uint32_t at = entry * 256 + half * 128;
 #pragma unroll
         for (uint32_t i = 0; i < 8; ++i) lds_write_16(at + ((i ^ turn) * 16), i < 4 ? low : high);
-        const uint32_t scales = kPanelScales<CB> + (uint32_t)tid * 4;
+    }
+    {
+        const uint32_t scales = kScales + (uint32_t)tid * 4;
         const float token_scale = __half2float(__ushort_as_half((unsigned short)token_scale_bits));
         asm volatile("ds_write_b32 %0, %1" ::"v"(scales), "v"(token_scale) : "memory");
         asm volatile("ds_write_b32 %0, %1" ::"v"(scales + kPanelRows * 4), "v"(row_sum) : "memory");
@@ -206,7 +227,9 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
     std::integral_constant<int, 0> zero;
     std::integral_constant<int, 1> one;
     // the first phase by itself
-    {
+    if constexpr (!Q4) {
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((TB - 1) * D) : "memory");
+    } else {
         constexpr int kAfter = U + (TB - 1) * D;
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kAfter > 63 ? 63 : kAfter) : "memory");
         Each<U>::run([&](auto tag) ORX_INLINE { keep(first_codes[decltype(tag)::value]); });
@@ -235,7 +258,7 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
             keep(acc[i][j]);
         }
     v4i weight[2][CB];
-    uint32_t phase_weights = kPanelWeights + (uint32_t)lane * 16;  // of the phase that is multiplied
+    uint32_t phase_weights = kWeights + (uint32_t)lane * 16;  // of the phase that is multiplied
     Each<CB>::run([&](auto tag) ORX_INLINE { lds_read_16<decltype(tag)::value * 1024>(weight[0][decltype(tag)::value], phase_weights); });
 #pragma unroll
     for (int w = 0; w < 2; ++w)
@@ -248,7 +271,7 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
     // multiplies.
     auto slice = [&](auto s_tag) ORX_INLINE {
         constexpr int s = decltype(s_tag)::value, set = s & 1, token_set = s % D;
-        constexpr bool kLooksUp = s < 2 * U, kPutsTogether = s >= 1 && s <= 2 * U;
+        constexpr bool kLooksUp = Q4 && s < 2 * U, kPutsTogether = Q4 && s >= 1 && s <= 2 * U;
         constexpr int u = s / 2, before = (s - 1) / 2;
         // this slice's tokens, and with them the codes, which were requested S - 1 slices ago: at most the tokens of D - 1 slices are younger
         if (last_block)
@@ -267,7 +290,7 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
         const uint32_t next = s == S - 1 ? phase_weights + other : phase_weights;
         // Side work behind the multiplies that every wave has, one piece each where there are that many: two codes of four lookups, then CB fragment
         // reads (what goes out last is waited for first, at the next slice's start).
-        constexpr int kMultiplies = (EVEN ? TB : TB - 1) * CB, kSide = CB + 2, kSpan = kMultiplies < 2 * kSide ? kMultiplies : 2 * kSide;
+        constexpr int kBefore = Q4 ? 2 : 0, kMultiplies = (EVEN ? TB : TB - 1) * CB, kSide = CB + kBefore, kSpan = kMultiplies < 2 * kSide ? kMultiplies : 2 * kSide;
         Each<kMultiplies>::run([&](auto m_tag) ORX_INLINE {
             constexpr int m = decltype(m_tag)::value, i = m / CB, j = (i & 1) ? CB - 1 - m % CB : m % CB;
             multiply_in_place<false>(acc[i][j], weight[set][j], token[token_set][i]);
@@ -275,8 +298,8 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
             Each<kSide>::run([&](auto n_tag) ORX_INLINE {
                 constexpr int n = decltype(n_tag)::value;
                 if constexpr (n >= from && n < to) {
-                    if constexpr (n >= 2) {
-                        lds_read_16<((s + 1) % S) * (CB * 1024) + (n - 2) * 1024>(weight[set ^ 1][n - 2], next);
+                    if constexpr (n >= kBefore) {
+                        lds_read_16<((s + 1) % S) * (CB * 1024) + (n - kBefore) * 1024>(weight[set ^ 1][n - kBefore], next);
                     } else if constexpr (kLooksUp) {
                         if (u < U - 1 || last_unit) read_code(std::integral_constant<int, n>{}, codes[u][2 * (s & 1) + n]);
                     }
@@ -291,6 +314,8 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
             });
             request_token(token[token_set][TB - 1], offset, token_base[TB - 1]);
         }
+        // (in front of the tokens of slice S - 1 - D, so that the wait of slice S - 1 covers them)
+        if constexpr (!Q4 && s < U) bring(phase + 1, std::integral_constant<int, (s < U ? s : 0)>{});
         if constexpr (kLooksUp && (s & 1) == 1) request_codes(phase + 2, std::integral_constant<int, u>{}, codes[u]);
     };
     for (;; ++phase) {
@@ -308,24 +333,27 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
     // what is still on its way lands before its registers are anybody else's
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     Each<D>::run([&](auto s_tag) ORX_INLINE { Each<TB>::run([&](auto tag) ORX_INLINE { keep(token[decltype(s_tag)::value][decltype(tag)::value]); }); });
-    Each<U>::run([&](auto tag) ORX_INLINE { keep(codes[decltype(tag)::value]); });
     Each<CB>::run([&](auto tag) ORX_INLINE { keep(weight[0][decltype(tag)::value]), keep(weight[1][decltype(tag)::value]); });
-    keep_entries();
+    if constexpr (Q4) {
+        Each<U>::run([&](auto tag) ORX_INLINE { keep(codes[decltype(tag)::value]); });
+        keep_entries();
+    }
     Each<TB>::run([&](auto i_tag) ORX_INLINE { Each<CB>::run([&](auto j_tag) ORX_INLINE { keep(acc[decltype(i_tag)::value][decltype(j_tag)::value]); }); });
-    asm volatile("s_barrier" ::: "memory");  // the tables are nobody's any more
+    asm volatile("s_barrier" ::: "memory");  // tables and weights are nobody's any more
 
     // ---- epilogue: blocks of 16 rows through LDS (private to the wave), whole rows of the run out ----
-    const float* const token_scales = reinterpret_cast<const float*>(lds + kPanelScales<CB>);
+    const float* const token_scales = reinterpret_cast<const float*>(lds + kScales);
     const int* const sums = reinterpret_cast<const int*>(token_scales + kPanelRows);
+    constexpr int kDouble = Q4 ? 2 : 1;
     float4 channel_scale[CB];
     float token_scale[TB];
     int bias[TB];
 #pragma unroll
-    for (int j = 0; j < CB; ++j) channel_scale[j] = *reinterpret_cast<const float4*>(lds + kPanelScales<CB> + kPanelRows * 8 + (16 * j + 4 * quarter) * 4);
+    for (int j = 0; j < CB; ++j) channel_scale[j] = *reinterpret_cast<const float4*>(lds + kScales + kPanelRows * 8 + (16 * j + 4 * quarter) * 4);
 #pragma unroll
     for (int i = 0; i < TB; ++i) {
         const int row = (i * kPanelWaves + wave) * 16 + column;
-        token_scale[i] = token_scales[row], bias[i] = kQuadBias * sums[row];
+        token_scale[i] = token_scales[row], bias[i] = Q4 ? kQuadBias * sums[row] : 0;
     }
     if (p.out_f32) {
 #pragma unroll
@@ -339,7 +367,7 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int channel = 16 * j + 4 * quarter + r;
-                    if (channel < channels) to[channel] = rescale(2 * acc[i][j][r] - bias[i], scale[r], token_scale[i]);
+                    if (channel < channels) to[channel] = rescale(kDouble * acc[i][j][r] - bias[i], scale[r], token_scale[i]);
                 }
             }
         }
@@ -347,7 +375,7 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
     }
     constexpr int kPitch = CB * 32 + 16, kPieces = 2 * CB;
     uint8_t* const image = lds + wave * (2 * 16 * kPitch);
-    static_assert(kPanelWaves * 2 * 16 * kPitch <= (int)kPanelWeights, "the images lie where the tables were");
+    static_assert(kPanelWaves * 2 * 16 * kPitch <= (int)(Q4 ? kWeights : kScales), "the images lie where the tables (the weights) were");
     __half* const out = reinterpret_cast<__half*>(p.out) + (int64_t)first_row * p.stride + first_channel;
     const bool aligned = p.stride % 8 == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0;
     auto store_block = [&](int i) {
@@ -376,8 +404,8 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
         for (int j = 0; j < CB; ++j) {
             const v4i a = acc[i][j];
             *reinterpret_cast<uint2*>(to + j * 32) =
-                make_uint2(pack_halves(rescale(2 * a[0] - bias[i], channel_scale[j].x, token_scale[i]), rescale(2 * a[1] - bias[i], channel_scale[j].y, token_scale[i])),
-                           pack_halves(rescale(2 * a[2] - bias[i], channel_scale[j].z, token_scale[i]), rescale(2 * a[3] - bias[i], channel_scale[j].w, token_scale[i])));
+                make_uint2(pack_halves(rescale(kDouble * a[0] - bias[i], channel_scale[j].x, token_scale[i]), rescale(kDouble * a[1] - bias[i], channel_scale[j].y, token_scale[i])),
+                           pack_halves(rescale(kDouble * a[2] - bias[i], channel_scale[j].z, token_scale[i]), rescale(kDouble * a[3] - bias[i], channel_scale[j].w, token_scale[i])));
         }
         if (i > 0) store_block(i - 1);
     }
@@ -389,22 +417,24 @@ struct PanelForm {
     const void* kernel;
     uint32_t shared;
 };
-// by blocks of 16 rows to a wave (2 to 4), whether every wave has as many, and blocks of channels to a workgroup (1 to 5)
-const PanelForm& panel_form(int tb, bool even, int cb) {
-#define ORX_PANEL(T, E, C) {reinterpret_cast<const void*>(&panel_kernel<T, C, E>), kPanelLds<C>}
-#define ORX_PANELS(T, E) {ORX_PANEL(T, E, 1), ORX_PANEL(T, E, 2), ORX_PANEL(T, E, 3), ORX_PANEL(T, E, 4), ORX_PANEL(T, E, 5)}
-    static const PanelForm forms[6][5] = {ORX_PANELS(2, false), ORX_PANELS(2, true), ORX_PANELS(3, false),
-                                          ORX_PANELS(3, true),  ORX_PANELS(4, false), ORX_PANELS(4, true)};
+// by codec, blocks of 16 rows to a wave (2 to 4), whether every wave has as many, and blocks of channels to a workgroup (1 to 5)
+constexpr int kPanelForms = 60;
+const PanelForm& panel_form(int index) {
+#define ORX_PANEL(K, T, E, C) {reinterpret_cast<const void*>(&panel_kernel<K, T, C, E>), kPanelLds<K, C>}
+#define ORX_PANELS(K, T, E) ORX_PANEL(K, T, E, 1), ORX_PANEL(K, T, E, 2), ORX_PANEL(K, T, E, 3), ORX_PANEL(K, T, E, 4), ORX_PANEL(K, T, E, 5)
+#define ORX_CODEC(K) ORX_PANELS(K, 2, false), ORX_PANELS(K, 2, true), ORX_PANELS(K, 3, false), ORX_PANELS(K, 3, true), ORX_PANELS(K, 4, false), ORX_PANELS(K, 4, true)
+    static const PanelForm forms[kPanelForms] = {ORX_CODEC(kPanelQ4), ORX_CODEC(kPanelW8)};
+#undef ORX_CODEC
 #undef ORX_PANELS
 #undef ORX_PANEL
-    return forms[2 * (tb - 2) + even][cb - 1];
+    return forms[index];
 }
 
 struct PanelShape {
     const PanelForm* form;
     int row_tiles, tile_rows, units;
 };
-PanelShape panel_shape(int rows, int n) {
+PanelShape panel_shape(int codec, int rows, int n) {
     PanelShape s = {};
     s.row_tiles = (rows + kPanelRows - 1) / kPanelRows;
     s.tile_rows = ((rows + s.row_tiles - 1) / s.row_tiles + 15) / 16 * 16;
@@ -412,7 +442,7 @@ PanelShape panel_shape(int rows, int n) {
     const int blocks = (n + 15) / 16, tb = std::max(2, (s.tile_rows / 16 + kPanelWaves - 1) / kPanelWaves);
     const int last_rows = rows - (s.row_tiles - 1) * s.tile_rows;  // of the last tile
     const bool even = s.tile_rows == tb * kPanelWaves * 16 && last_rows > s.tile_rows - 16;
-    s.form = &panel_form(tb, even, (blocks + s.units - 1) / s.units);
+    s.form = &panel_form(((codec * 3 + tb - 2) * 2 + even) * 5 + (blocks + s.units - 1) / s.units - 1);
     return s;
 }
 
@@ -421,19 +451,19 @@ PanelShape panel_shape(int rows, int n) {
 // (offsets of a code request are 32 bits: a run's channels times the bytes of a row)
 bool panel_eligible(int rows, int n, int k) { return rows >= 1 && rows <= kPanelMaxRows && k % 128 == 0 && k >= 256 && (int64_t)n * k < (1ll << 31); }
 
-void panel_geometry(int rows, int n, Geometry* g) {
-    const PanelShape s = panel_shape(rows, n);
+void panel_geometry(int codec, int rows, int n, Geometry* g) {
+    const PanelShape s = panel_shape(codec, rows, n);
     g->grid[0] = (uint32_t)s.units, g->grid[1] = (uint32_t)s.row_tiles, g->grid[2] = 1;
     g->block[0] = kPanelThreads;
     g->shared = s.form->shared;
 }
 
-int panel_launch(const uint8_t* panels, const int* sums, const void* w, const uint32_t* book, const __half* ws, const __half* as, void* out,
+int panel_launch(int codec, const uint8_t* panels, const int* sums, const void* w, const uint32_t* book, const __half* ws, const __half* as, void* out,
                  int rows, int n, int k, int stride, int packed_k, bool out_f32, hipStream_t stream) {
     static DeviceOnce opted_in;  // dynamic LDS above 64 KiB needs an opt-in per kernel and device
     const int ready = opted_in.run([] {
-        for (int of = 0; of < 6 * 5; ++of) {
-            const PanelForm& form = panel_form(2 + of / 10, of / 5 % 2, 1 + of % 5);
+        for (int of = 0; of < kPanelForms; ++of) {
+            const PanelForm& form = panel_form(of);
             const int code = hip_check(hipFuncSetAttribute(form.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)form.shared),
                                        "hipFuncSetAttribute");
             if (code != ORX_OK) return code;
@@ -441,11 +471,13 @@ int panel_launch(const uint8_t* panels, const int* sums, const void* w, const ui
         return (int)ORX_OK;
     });
     if (ready != ORX_OK) return ready;
-    const PanelShape s = panel_shape(rows, n);
+    const PanelShape s = panel_shape(codec, rows, n);
     PanelParams p = {};
     p.panels = panels, p.sums = sums, p.w = static_cast<const uint8_t*>(w), p.book = book, p.ws = ws, p.as = as, p.out = out;
     p.n = n, p.k = k, p.stride = stride, p.m = rows, p.out_f32 = out_f32, p.tile_rows = s.tile_rows;
-    if (packed_k == 128)
+    if (codec == kPanelW8)
+        p.row_stride = (uint32_t)k, p.chunk_stride = 128;
+    else if (packed_k == 128)
         p.row_stride = 64, p.chunk_stride = (uint32_t)n * 64, p.half_stride = 32;
     else if (packed_k == 64)
         p.row_stride = 32, p.chunk_stride = (uint32_t)n * 64, p.half_stride = (uint32_t)n * 32;

@@ -54,6 +54,37 @@ def panels_pay(rows, n, k, cus):
     return blocks > cus
 
 
+def int8_panels_pay(rows, n, k, cus):
+    """The same for int8 weights (figures as above).
+    65-128 rows: more than 5 blocks to a CU 0.55-0.94; 3 to 5 0.48-1.0 from 81 rows on, 1.0-1.3 below; 2 to 3 0.43-0.84 above 112 rows up to K = 8192, else 0.85-1.4; up to
+    two 0.78-0.96 above 112 rows (up to one K to 8192, up to two K to 2048), otherwise 0.9-1.5.
+    129-512 rows: where the channel runs fill one round 0.92-2.5 (K = 1024 of more than one block 0.39-0.5); elsewhere half to one block 0.46-0.99 up to K = 4096, 0.88-1.65
+    beyond; to 1.5 blocks 0.4-0.96 up to K = 5120, 0.92-1.5 beyond; to two 0.39-1.01 up to K = 8192, 0.53-1.2 beyond; more 0.43-1.02 (17408 x 5120 at 130 / 512 rows 0.67 /
+    0.82), but up to 256 rows of 2 to 3 blocks and K above 8192 0.83-1.1 and more than 5 blocks at 448-512 rows 0.7-1.2.
+    513-768 rows: up to 1.5 blocks 0.44-0.87 up to K = 2048, 0.77-1.8 beyond; 1.75 to 3 0.62-1.0; more 0.73-1.25.  Above: half a block 0.53-0.73 up to K = 2048, others 0.71-2.1."""
+    if not 64 < rows <= PANEL_ROWS:
+        return False
+    blocks = -(-n // 16)
+    if rows <= 128:
+        if blocks <= 3 * cus:
+            return rows > 112 and k <= (2048 if cus < blocks <= 2 * cus else 8192)
+        return blocks > 5 * cus or rows > 80
+    if rows > 512:
+        if 2 * blocks <= 3 * cus:
+            return k <= 2048 and (rows <= 768 or 2 * blocks <= cus)
+        return rows <= 768 and blocks <= 3 * cus
+    row_tiles = -(-rows // 128)
+    tile_rows = -(-rows // row_tiles)
+    most = 5 if tile_rows <= 80 else 3 if tile_rows <= 112 else 2  # blocks of the widest run
+    if row_tiles * -(-blocks // most) <= cus or 2 * blocks <= cus:
+        return k <= 1024 and blocks > cus
+    if blocks > 5 * cus:
+        return rows <= 384
+    if blocks > 2 * cus:
+        return k <= 8192 or rows > 256 or blocks >= 3 * cus
+    return k <= (4096 if blocks <= cus else 5120 if 2 * blocks <= 3 * cus else 8192)
+
+
 class QuantizedLinear:
     """A8 quantiser + one projection (E8P-Q4 or W8A8) with a dynamic row count up to `capacity`."""
 
@@ -103,13 +134,15 @@ class QuantizedLinear:
         top = min(capacity, PANEL_ROWS)
         cus = torch.cuda.get_device_properties(self.weight.device).multi_processor_count
         self.over_panels = [False] * (top + 1)
-        if codec == "q4" and algorithm == "auto" and not block_m and 256 <= self.k <= 32768 and self.n * self.k < 2**31:
-            self.over_panels = [panels_pay(rows, self.n, self.k, cus) for rows in range(top + 1)]
+        if algorithm == "auto" and not block_m and self.k % 128 == 0 and 256 <= self.k <= 32768 and self.n * self.k < 2**31:
+            pays = panels_pay if codec == "q4" else int8_panels_pay
+            self.over_panels = [pays(rows, self.n, self.k, cus) for rows in range(top + 1)]
         if any(self.over_panels):
             self.panels = torch.empty(((top + 15) // 16 * 16, self.k), dtype=torch.int8, device="cuda")
             self.sums = torch.empty(top, dtype=torch.int32, device="cuda")
             self.panel_quantizer = Kernel("activation_quantization", K=self.k, panels=True)
-            self.panel_projection = Kernel("e8p_q4_projection", M=top, N=self.n, K=self.k, dynamic_rows=True, panels=True, packed_k=packed_k)
+            variant = dict(M=top, N=self.n, K=self.k, dynamic_rows=True, panels=True)
+            self.panel_projection = Kernel("e8p_q4_projection", packed_k=packed_k, **variant) if codec == "q4" else Kernel("int8_projection", **variant)
 
     def quantize(self, x16, stream=None):
         rows = x16.shape[0]
@@ -139,8 +172,12 @@ class QuantizedLinear:
         rows = x16.shape[0]
         if rows < len(self.over_panels) and self.over_panels[rows]:
             self.panel_quantizer(stream=stream, Mask=None, Panels=self.panels, Q=self.a_q, S=self.a_s, Sums=self.sums, X=x16, rows=rows)
-            self.panel_projection(stream=stream, A=self.panels, AS=self.a_s, Book=self.book, Out=self.out, S=self.scales, Sums=self.sums,
-                                  W=self.weight, m=rows)
+            if self.codec == "q4":
+                self.panel_projection(stream=stream, A=self.panels, AS=self.a_s, Book=self.book, Out=self.out, S=self.scales, Sums=self.sums,
+                                      W=self.weight, m=rows)
+            else:
+                self.panel_projection(stream=stream, A=self.panels, Output=self.out, TokenScale=self.a_s, Weight=self.weight,
+                                      WeightScale=self.scales, m=rows)
             return self._rows(rows)
         return self.project(self.quantize(x16, stream), stream)
 

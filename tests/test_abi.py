@@ -335,6 +335,17 @@ def test_which_rows_a_linear_takes_over_panels(n, k, lines):
         assert panels_pay(rows, n, k, 256) == bool(taken), rows
 
 
+@pytest.mark.parametrize("n, k, lines", [
+    (2048, 2048, [(112, 0), (113, 1), (128, 1), (129, 0), (512, 0), (513, 1), (1024, 1), (1025, 0)]), (4096, 4096, [(256, 0), (257, 1), (512, 1), (513, 0)]), (4096, 2048, [(768, 1), (769, 0)]),
+    (5120, 5120, [(113, 0), (129, 0), (224, 0), (225, 1), (512, 1), (513, 0)]), (5120, 1024, [(129, 1)]), (7168, 8192, [(512, 1), (513, 1), (768, 1), (769, 0)]), (7168, 8320, [(400, 0)]),
+    (9728, 8320, [(256, 0), (257, 1)]), (12288, 8320, [(129, 1)]), (14336, 5120, [(80, 0), (81, 1), (512, 1), (513, 0)]), (24576, 5120, [(64, 0), (65, 1), (384, 1), (385, 0)]),
+])
+def test_which_rows_an_int8_linear_takes_over_panels(n, k, lines):
+    from orinfer_amd.programs import int8_panels_pay
+    for rows, taken in lines:
+        assert int8_panels_pay(rows, n, k, 256) == bool(taken), rows
+
+
 @pytest.mark.parametrize("codec, n, k, rows", [("w8", 4096, 12288, 128), ("w8", 4096, 12288, 256), ("q4", 4096, 12288, 384), ("q4", 7168, 1024, 130)])
 def test_which_rows_the_channel_runs_leave(codec, n, k, rows):
     symbol, shape = {"q4": "e8p_q4_projection", "w8": "int8_projection"}[codec], dict(M=rows, N=n, K=k, workspace=True)

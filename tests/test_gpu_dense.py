@@ -1719,11 +1719,34 @@ def test_q4_over_panels(rows, n, k, packed_k):
     assert (gu.host(out)[rows] == 91).all()
 
 
-def project_over_panels(a_q, a_s, packed, ws, packed_k, out, **variant):
+@pytest.mark.parametrize("rows,n,k", [(1, 16, 256), (17, 24, 384), (100, 4099, 1152), (255, 5000, 896), (257, 8200, 1280), (256, 12290, 640), (300, 9728, 384), (384, 17408, 256),
+                                      (385, 20480, 768), (512, 20600, 256), (513, 300, 1024), (1030, 1000, 640), (449, 16000, 512)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32], ids=["fp16", "fp32-strided"])
+def test_w8_over_panels(rows, n, k, dtype):
+    rng = np.random.default_rng(orc.SEED + rows + n + k)
+    weight = rng.integers(-128, 128, (n, k), dtype=np.int8)
+    a_q = rng.integers(-127, 128, (rows, k), dtype=np.int8)
+    a_q[0, :], a_q[-1, :], weight[-1, :] = 127, -128, -128
+    a_s, ws = rng.uniform(0.005, 0.02, rows).astype(np.float16), rng.uniform(0.005, 0.02, n).astype(np.float16)
+    stride = n if dtype == torch.float16 else n + 3
+    out = torch.full((rows + 1, stride), 91, dtype=dtype, device=gu.DEV)
+    gu.kernel("int8_projection", M=rows, N=n, K=k, panels=True, workspace=False, output_stride=stride, output_dtype="float16" if dtype == torch.float16 else "float32")(
+        A=gu.dev(in_panels(a_q)), Output=out, TokenScale=gu.dev(a_s), Weight=gu.dev(weight), WeightScale=gu.dev(ws))
+    want = orc.project(a_q, a_s, weight, ws, out_dtype=np.float16 if dtype == torch.float16 else np.float32)
+    np.testing.assert_array_equal(gu.host(out)[:rows, :n], want)
+    assert (gu.host(out)[rows] == 91).all() and (gu.host(out)[:, n:] == 91).all()
+
+
+def in_panels(a_q):
     rows, k = a_q.shape
     padded = np.zeros(((rows + 15) // 16 * 16, k), np.int8)
     padded[:rows] = a_q
-    panels = np.ascontiguousarray(padded.reshape(-1, 16, k // 128, 4, 2, 16).transpose(0, 2, 4, 3, 1, 5))
+    return np.ascontiguousarray(padded.reshape(-1, 16, k // 128, 4, 2, 16).transpose(0, 2, 4, 3, 1, 5))
+
+
+def project_over_panels(a_q, a_s, packed, ws, packed_k, out, **variant):
+    rows, k = a_q.shape
+    panels = in_panels(a_q)
     stored = packed if packed_k == 0 else orc.q4_pack_k(packed, packed_k)
     gu.kernel("e8p_q4_projection", M=rows, N=len(ws), K=k, packed_k=packed_k, panels=True, workspace=False, **variant)(
         A=gu.dev(panels), AS=gu.dev(a_s), Book=gu.book(), Out=out, S=gu.dev(ws), Sums=gu.dev(a_q.astype(np.int32).sum(1).astype(np.int32)), W=gu.dev(stored))
@@ -1740,11 +1763,13 @@ def test_q4_over_panels_strides(dtype, pad):
     assert (gu.host(out)[rows] == 91).all() and (gu.host(out)[:, n:] == 91).all()
 
 
-def test_a_linear_over_panels_gives_the_bits_of_the_row_major_one():
+@pytest.mark.parametrize("codec", ["q4", "w8"])
+def test_a_linear_over_panels_gives_the_bits_of_the_row_major_one(codec):
     """Rows either side of the lines, one state; the codes and scales that `run` leaves are the quantiser's; and from a graph."""
     rng = np.random.default_rng(orc.SEED)
     n, k = 9728, 512
-    linear = programs.QuantizedLinear("q4", rng.integers(0, 2**32, (n, k // 8), dtype=np.uint32), rng.uniform(0.005, 0.02, n).astype(np.float16), 1300, packed_k=128)
+    weight = rng.integers(0, 2**32, (n, k // 8), dtype=np.uint32) if codec == "q4" else rng.integers(-127, 128, (n, k), dtype=np.int8)
+    linear = programs.QuantizedLinear(codec, weight, rng.uniform(0.005, 0.02, n).astype(np.float16), 1300, packed_k=128 if codec == "q4" else 0)
     taken = [r for r, over in enumerate(linear.over_panels) if over]
     assert taken and taken[0] > 64 and len(linear.over_panels) == programs.PANEL_ROWS + 1
     for rows in (taken[0] - 1, taken[0], 512, 700, 768, 1025):
@@ -1773,6 +1798,7 @@ def test_panels_are_refused_where_no_kernel_serves_them():
                             ("activation_quantization", dict(K=256, fused=True, panels=True)), ("activation_quantization", dict(K=32896, panels=True)),
                             ("e8p_q4_projection", dict(M=512, N=256, K=128, panels=True)), ("e8p_q4_projection", dict(M=2049, N=256, K=256, panels=True)),
                             ("e8p_q4_projection", dict(M=64, N=256, K=256, panels=True, algorithm="runs")),
-                            ("e8p_q4_projection", dict(M=64, N=256, K=256, panels=True, workspace=True))):
+                            ("e8p_q4_projection", dict(M=64, N=256, K=256, panels=True, workspace=True)),
+                            ("int8_projection", dict(M=64, N=256, K=320, panels=True)), ("int8_projection", dict(M=64, N=256, K=256, panels=True, block_m=64))):
         with pytest.raises(gu.lib.OrxError):
             gu.lib.Kernel(symbol, **variant)
