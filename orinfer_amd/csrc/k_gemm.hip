@@ -712,10 +712,12 @@ int tile_for(const orx_function& f, int rows) {
 //     faster from K = 3072 on (2048 x 3584 at 32 rows 6.9 to 7.5);
 //   two blocks: 7168 x 5376 at 2 rows 9.8 to 8.3 / 10.3 to 8.7, 24 rows 10.8 to 9.2 / 12.2 to 10.9; the runs get there with rows times K: 7168 x 17408 at 16 rows
 //     1.06 / 0.97 of its time, 32 rows 0.93 / 0.84; 7168 x 5120 row-major at 24 / 32 rows 1.06 / 0.98;
-//   three blocks: 9728 x 6144 at 8 rows 0.84 / 0.89 of its time, 24 rows 0.72 / 0.78; K = 4224 at 2 rows 1.06 / 1.02, 24 rows of K = 3200 1.04; two rows stay with
-//     the GEMV (9728 x 9728 18.7 to 17.0 / row-major);
-//   four and five: 17408 x 6144 at 3 / 16 / 32 rows 0.82 / 0.76 / 0.70 of its time K-major, x 8192 22.3 to 17.8, 24.9 to 18.2, 34.5 to 21.8; 14336 x 6144 1.00 / 0.96 / 0.87, x 8192
-//     0.99 / 0.87 / 0.83; row-major 14336 x 8192 1.01 / 0.97 / 0.84, 17408 x 8192 (the other batched-decode kernel) 0.98 / 0.95 / 0.86.
+//   three blocks, 9728 to 12288 channels: K = 3200 at 24 rows 0.90 to 0.92 / 0.92 to 0.95 of its time, K = 2688 0.94 to 0.98, K = 4224 at 3 to 16 rows 0.81 to 0.94 / 0.84 to 0.95, K = 3200
+//     0.88 to 1.02 (K-major up to 16 rows only above K = 5376, 0.83 at 8 rows of it: the records of such handles name the streaming kernel); two rows stay with the GEMV
+//     (9728 x 9728 18.7 to 17.0 / row-major);
+//   four, 13312 to 16384 channels: K = 7296 at 3 / 16 rows 0.97 to 1.03 / 0.84 to 0.94, K = 6272 0.98 to 1.08 / 0.87 to 0.96; 24 rows of K = 6272 0.90 to 0.99, of 5248 0.93 to 1.03, 32 rows 0.89 to 0.93;
+//   five, 17408 to 20480: K = 4224 at 3 / 16 / 24 rows 0.84 to 0.98 / 0.81 to 0.90 / 0.84 to 0.93, K = 3200 0.94 to 1.02 / 0.90 to 0.96 / 0.92 to 1.01; 17408 x 8192 at 3 / 16 / 32 rows 22.3 to
+//     17.8, 24.9 to 18.2, 34.5 to 21.8; row-major 17408 x 6144 / 8192, where the other batched-decode kernel serves, 0.95 to 1.0 / 0.86 to 0.98.
 // The batched-decode kernels where they take the shape: the one with loader waves (K up to 5120) is the fastest up to 16
 // rows in one and three blocks (K = 5120, 16 rows: level with the runs, 0.75-0.9 of the streaming kernel) and in more; the runs pass it, K-major, with one block
 // at 17 rows of K = 5120 and 20 of 4096 (0.87-0.93, 0.91-0.97 of its time; 24 rows of K = 3072 0.97-1.03), with three at 20 rows of K = 5120
@@ -734,10 +736,12 @@ bool runs_for_few_rows(const orx_function& f, int rows) {
     if (blocks == 1) return f.K >= (rows > 16 ? 3072 : 4096);
     if (blocks == 2) return work >= (k_major ? 32 * 12288 : 20 * 8192);
     if (loader) return blocks == 3 && k_major && work >= 20 * 5120;
-    if (rows <= 2 && !(blocks == 5 && k_major)) return false;
-    if (blocks >= 4) return f.K >= (blocks == 5 && k_major ? 6144 : 8192);
-    if (dense_resident_eligible(f.N, f.K, f.packed_k)) return rows > 16 && work >= 20 * 6144;
-    return f.K >= (rows > 16 ? 4096 : 6144);
+    const bool resident = dense_resident_eligible(f.N, f.K, f.packed_k);
+    if (blocks == 5) return f.K >= (resident ? 8192 : 4096);
+    if (blocks == 4) return resident ? f.K >= 8192 : rows <= 16 ? f.K >= 7168 : work >= 24 * 6144;
+    if (rows <= 2) return false;
+    if (resident) return rows > 16 && work >= 20 * 6144;
+    return f.K >= (rows > 16 ? 3200 : k_major ? 5504 : 4096);
 }
 
 // int8 rows up to 32: channel runs against the streaming kernel, whose workgroups of 32 channels make the same difference as above

@@ -311,7 +311,8 @@ def test_which_rows_the_channel_runs_take(codec, n, k, rows, algorithm):
     (12288, 4096, 97, "runs"), (12288, 4224, 96, "runs"), (9728, 1024, 65, "wide"), (14336, 2048, 128, "runs"), (24576, 4096, 128, "wide"), (24592, 4096, 128, "runs"),
     (24592, 1408, 128, "wide"), (17408, 2944, 130, "tall"), (17408, 3072, 130, "runs"), (17408, 3968, 240, "tall"), (17408, 4096, 240, "runs"), (17408, 4096, 242, "tall"),
     (20480, 5120, 200, "tall"), (20480, 8192, 200, "runs"), (34816, 4096, 192, "runs"), (34816, 3968, 192, "mfma"), (34816, 5120, 194, "mfma"), (17408, 5120, 257, "tall"),
-    (17408, 6016, 8, "stream"), (17408, 6144, 8, "runs"), (14336, 8064, 17, "stream"), (14336, 8192, 17, "runs"), (9728, 5120, 20, "runs"), (9728, 5120, 19, "resident"),
+    (17408, 3968, 8, "stream"), (17408, 4224, 2, "runs"), (14336, 7040, 16, "stream"), (14336, 7168, 16, "runs"), (14336, 8576, 17, "stream"), (14336, 8704, 17, "runs"),
+    (9728, 3072 + 64 * 2, 17, "runs"), (9728, 2944, 32, "stream"), (9728, 5504, 3, "runs"), (9728, 5120, 20, "runs"), (9728, 5120, 19, "resident"),
 ])
 def test_which_rows_of_codes_the_channel_runs_take_in_several_rounds(n, k, rows, algorithm):
     """K-major codes with scratch: both sides of each line (rows, rounds, K) of the rule for codes."""
