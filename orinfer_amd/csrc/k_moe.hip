@@ -343,6 +343,17 @@ __global__ __launch_bounds__(256) void partition_tiles_kernel(const int* __restr
 // element, token-major stable order; a token may name an expert more than once.
 // LDS (dynamic): counters[16][E], wave-local slots[capacity assignments], scan totals.
 constexpr int kMetaWaves = 16, kMetaThreads = kMetaWaves * 64;
+// Inclusive sum over the lanes in front, by lane moves: shifts by 1, 2, 4 and 8 within a row of 16, then the last lane of rows 0 and 2 to the row
+// behind, then lane 31 to the upper half.  (A shuffle is an LDS round trip, six of them one after another.)
+__device__ __forceinline__ int wave_prefix_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
+    return v;
+}
 __global__ __launch_bounds__(kMetaThreads) void route_metadata_kernel(
     const int* __restrict__ ids, int* __restrict__ counts, int* __restrict__ relative, int* __restrict__ row_offsets,
     int* __restrict__ tile_count, int* __restrict__ tile_expert, int* __restrict__ tile_offsets, int* __restrict__ tile_row,
@@ -390,12 +401,12 @@ __global__ __launch_bounds__(kMetaThreads) void route_metadata_kernel(
     __syncthreads();
     // per expert: exclusive prefix over the 16 wave rows, total count
     int count = 0;
-    if (tid < experts) {
-        for (int w = 0; w < kMetaWaves; ++w) {
-            const int t = counters[w * experts + tid];
-            counters[w * experts + tid] = count;
-            count += t;
-        }
+    if (tid < experts) {  // (all reads in front of the writes, or each waits for the one before it)
+        int of_wave[kMetaWaves];
+#pragma unroll
+        for (int w = 0; w < kMetaWaves; ++w) of_wave[w] = counters[w * experts + tid];
+#pragma unroll
+        for (int w = 0; w < kMetaWaves; ++w) counters[w * experts + tid] = count, count += of_wave[w];
         counts[tid] = count;
     }
     __syncthreads();
@@ -407,15 +418,11 @@ __global__ __launch_bounds__(kMetaThreads) void route_metadata_kernel(
     }
     // exclusive scans of count and ceil(count / block_m) over the experts (one per thread)
     const int tiles = (count + block_m - 1) / block_m;
-    int row_scan = count, tile_scan = tiles;
-#pragma unroll
-    for (int offset = 1; offset < 64; offset <<= 1) {
-        const int r = __shfl_up(row_scan, offset, 64), t = __shfl_up(tile_scan, offset, 64);
-        if (lane >= offset) row_scan += r, tile_scan += t;
-    }
+    const int row_scan = wave_prefix_sum(count), tile_scan = wave_prefix_sum(tiles);
     if (lane == 63) wave_rows[wave] = row_scan, wave_tiles[wave] = tile_scan;
     __syncthreads();
     int row_base = 0, tile_base = 0, tile_total = 0;
+#pragma unroll
     for (int w = 0; w < kMetaWaves; ++w) {
         if (w < wave) row_base += wave_rows[w], tile_base += wave_tiles[w];
         tile_total += wave_tiles[w];
@@ -514,13 +521,7 @@ __global__ __launch_bounds__(kMetaThreads) void segment_place_kernel(
     const int full = count / block_m, rest = count % block_m;
     const int size = 2 * rest > block_m ? 0 : 4 * rest > block_m ? 1 : 2;  // of the last tile
     const int large = full + (rest > 0 && size == 0), small = rest > 0 && size > 0 ? 1 << (16 * (size - 1)) : 0;
-    int row_scan = count, tile_scan = tiles, large_scan = large, small_scan = small;
-#pragma unroll
-    for (int offset = 1; offset < 64; offset <<= 1) {
-        const int r = __shfl_up(row_scan, offset, 64), t = __shfl_up(tile_scan, offset, 64);
-        const int l = __shfl_up(large_scan, offset, 64), m = __shfl_up(small_scan, offset, 64);
-        if (lane >= offset) row_scan += r, tile_scan += t, large_scan += l, small_scan += m;
-    }
+    const int row_scan = wave_prefix_sum(count), tile_scan = wave_prefix_sum(tiles), large_scan = wave_prefix_sum(large), small_scan = wave_prefix_sum(small);
     if (lane == 63) wave_rows[wave] = row_scan, wave_tiles[wave] = tile_scan, wave_large[wave] = large_scan, wave_small[wave] = small_scan;
     __syncthreads();
     int row_base = 0, tile_base = 0, tile_total = 0, large_base = 0, large_total = 0, small_base = 0, small_total = 0;
