@@ -92,10 +92,9 @@ __device__ __forceinline__ void tile_of(int id, int tiles_m, int tiles_n, int* t
 // One workgroup per CU walks a static list of tiles (tile r of workgroup w is number w + r * gridDim.x of the
 // XCD-aware order), and the K steps of all its tiles form ONE software pipeline: the operand requests of the
 // next tile's first steps go out while the current tile's last steps multiply, so no tile after the first pays a
-// prologue.  The epilogue is private to a wave and stays in registers: lanes that hold neighbouring channels of a
-// row trade words (v_permlane16_swap), after which every lane stores 16-byte pieces of output rows.  It needs no
-// LDS, no workgroup barrier, and leaves both operand stages alone (they already hold the next tile's first
-// steps); its stores are not waited for and drain under the next tile's multiplies.
+// prologue.  The epilogue is private to a wave: blocks of 16 rows go through the wave's own part of the operand
+// stage that nobody reads any more and leave as whole rows of 128 bytes.  It needs no workgroup barrier; its stores are not
+// waited for and drain under the next tile's multiplies.
 //
 // The kernel is bound by power, not by issue slots: on random int8 data the clock inside the K loop is 1.9 GHz in a
 // sustained run (1.2-1.3 GHz in a launch that follows a pause), the same launch on zero operands is 30 % shorter, and
@@ -103,6 +102,8 @@ __device__ __forceinline__ void tile_of(int id, int tiles_m, int tiles_n, int* t
 // v_mfma_i32_32x32x32_i8 with half the accumulator traffic per multiply and sustains 3.83 POP/s on random
 // operands where the 32 x 32 shape sustains 3.37 (back-to-back issue from registers, whole chip); the fragment
 // bytes read from LDS per multiply are the same, so the tile, the stages and the swizzle stay as they were.
+// The epilogue through LDS with the channel scales in registers, against stores of 16 rows x 64 bytes after v_permlane16_swap and scales read again per
+// block: 8192 x 4096 x 4096 119.0 -> 117.9 us, 8192 x 7168 x 5120 276.6 -> 273.4, 3000 x 2048 x 1024 18.3 -> 17.3.
 constexpr uint32_t kPersistentLds = 4 * kTileBytes + 2 * kTile * 4;
 constexpr int kPersistentThreads = 512;
 
@@ -483,9 +484,9 @@ __global__ __launch_bounds__(kPersistentThreads) void gemm_big_persistent_kernel
 // lookups whose random addresses collide in the banks, and no unit is full: the matrix pipe is busy in 0.35 of
 // the cycles, the LDS pipe in about 0.6.  Taking out any one part of a step shortens the loop by 5-25 % (the
 // decode most), while lookups made cheaper (4-byte nibble tables, also stored 8 and 4 times) measure the same:
-// what a step issues has to come back within the step, and the parts queue behind one another.  The floor under
-// it is what the token rows cost: every CU reads all of them once, 2.6 MB per CU at 512 x 5120, which 256 CUs
-// together pull out of the L2 in 37 us.
+// what a step issues has to come back within the step, and the parts queue behind one another.  Every CU
+// reads all token rows once, 2.6 MB at 512 x 5120: 23 us at what the L2s give all CUs together, 37 us with the two
+// slots of 64 KiB that are in flight here (k_panel.hip has them in flight in registers, and the LDS for its tables).
 constexpr int kTallBlocks = 5;  // blocks of 16 channels per workgroup, at most
 constexpr int kTallRows = 512, kTallCols = 16 * kTallBlocks, kTallStep = 64, kTallThreads = 512, kTallStagesW = 4;
 constexpr uint32_t kTallSlotA = kTallRows * 128;  // token rows of a K chunk of 128
