@@ -18,6 +18,7 @@
 #include <hip/hip_fp16.h>
 
 #include <cstring>
+#include <type_traits>
 
 #include "a8_device.h"
 #include "e8p_device.h"
@@ -279,6 +280,57 @@ __device__ __forceinline__ float rotate_block(float (&v)[4], int l32, __half (&o
     return amax;
 }
 
+// The same stages for rows whose codes are all that is kept, in 28 vector instructions per lane and four channels where rotate_block takes 52 of a kernel's
+// 150 and an LDS trip each (rotation and A8 of 8192 x 5120, bound by them: 43.4 -> 40.1 us; 20 rows with residual and norm, where the chain counts: 5.5 -> 5.2, the
+// layer around it 91.0 -> 90.1; 8192 rows of those are bound by memory, 88 us).
+//  * A stage between lanes is one instruction per value, own + (+-1) partner: exact, for a fused multiply-add with +-1 rounds as the add does. The
+//    upper lane of a pair gets own - partner, the negative of what it should hold; so does its partner of every later stage, and the
+//    signs come back with the last multiply.  (Only the sign of a zero can differ from rotate_block, which no code shows.)
+//  * The partners are those that lane controls reach: the neighbour, the other pair, the mirrored half row, and eight lanes on.  The mirrored half
+//    row flips three bits of the lane, so lane l holds the channels 4 group .. 4 group + 3 with bits 0 and 1 of the group flipped in the upper
+//    half of eight lanes; stages then pair groups at distance 1, 2, 4, 8 and, by a swap of rows of 16 lanes, 16.
+struct RotationLane {
+    int group;
+    float sign[5], scale;  // of the five stages between lanes; 128^-1/2 with the signs of the first four
+    __device__ __forceinline__ explicit RotationLane(int l32) {
+        group = l32 ^ (l32 >> 2 & 1) * 3;
+        scale = 0.08838834764831845f;
+#pragma unroll
+        for (int bit = 0; bit < 5; ++bit) {
+            sign[bit] = group >> bit & 1 ? -1.f : 1.f;
+            if (bit < 4) scale *= sign[bit];
+        }
+    }
+};
+__device__ __forceinline__ float rotate_for_codes(float (&v)[4], const RotationLane& lane, __half (&out)[4]) {
+    const float a = v[0] + v[1], b = v[0] - v[1], c = v[2] + v[3], d = v[2] - v[3];
+    v[0] = a + c, v[2] = a - c, v[1] = b + d, v[3] = b - d;
+    // four values in turn leave the two cycles that a lane control needs behind a write of its source; the first and the last stage have a pause
+#define ORX_STAGE(SIGN, CONTROL)                                                           \
+    "v_fmac_f32_dpp %0, %0, " SIGN " " CONTROL " row_mask:0xf bank_mask:0xf\n\t"          \
+    "v_fmac_f32_dpp %1, %1, " SIGN " " CONTROL " row_mask:0xf bank_mask:0xf\n\t"          \
+    "v_fmac_f32_dpp %2, %2, " SIGN " " CONTROL " row_mask:0xf bank_mask:0xf\n\t"          \
+    "v_fmac_f32_dpp %3, %3, " SIGN " " CONTROL " row_mask:0xf bank_mask:0xf\n\t"
+    asm volatile("s_nop 1\n\t" ORX_STAGE("%4", "quad_perm:[1,0,3,2]") ORX_STAGE("%5", "quad_perm:[2,3,0,1]") ORX_STAGE("%6", "row_half_mirror")
+                     ORX_STAGE("%7", "row_ror:8") "s_nop 1"
+                 : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3])
+                 : "v"(lane.sign[0]), "v"(lane.sign[1]), "v"(lane.sign[2]), "v"(lane.sign[3]));
+#undef ORX_STAGE
+    float amax = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        typedef unsigned int pair_u32 __attribute__((ext_vector_type(2)));
+        const pair_u32 rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[j]), __float_as_uint(v[j]), false, false);  // the lower row's, the upper row's
+        const float value = __builtin_fmaf(__uint_as_float(rows[1]), lane.sign[4], __uint_as_float(rows[0]));
+        float scaled = value * lane.scale;
+        // opaque: the fp16 cast below must round the fp32 product, not a fused multiply-convert
+        asm volatile("" : "+v"(scaled));
+        out[j] = __float2half_rn(scaled);
+        amax = fmaxf(amax, fabsf(__half2float(out[j])));
+    }
+    return amax;
+}
+
 // Row scale from the largest magnitude, stored once, and the int8 codes of the fp16 row in LDS.
 __device__ __forceinline__ void quantise_row(const __half* rotated, float amax, int8_t* __restrict__ q,
                                              __half* __restrict__ s, int row, int k) {
@@ -311,7 +363,8 @@ __device__ __forceinline__ float rotate_row_to_lds(const __half* __restrict__ x,
     constexpr int kWaves = THREADS / 64;
     constexpr int kBatch = THREADS == 256 ? kRotateBatch : 2;  // steps whose loads leave together
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int half_wave = lane >> 5, l32 = lane & 31;
+    const int half_wave = lane >> 5;
+    const RotationLane rotation(lane & 31);
     const int blocks = k / 128;
     const int64_t in_base = (int64_t)row * (SWIGLU ? 2 * k : k);
     float amax = 0.f;
@@ -323,7 +376,7 @@ __device__ __forceinline__ float rotate_row_to_lds(const __half* __restrict__ x,
 #pragma unroll
         for (int u = 0; u < kBatch; ++u) {
             const int block = 2 * (base + kWaves * u) + half_wave;
-            const int first = (block < blocks ? block : 0) * 128 + 4 * l32;  // clamped, so unconditional
+            const int first = (block < blocks ? block : 0) * 128 + 4 * rotation.group;  // clamped, so unconditional
             raw[u] = *reinterpret_cast<const uint2*>(x + in_base + first);
             sign_word[u] = *reinterpret_cast<const uint32_t*>(signs + first);
             raw_up[u] = make_uint2(0u, 0u);
@@ -334,7 +387,7 @@ __device__ __forceinline__ float rotate_row_to_lds(const __half* __restrict__ x,
             if (2 * (base + kWaves * u) >= blocks) break;
             const int block = 2 * (base + kWaves * u) + half_wave;
             const bool live = block < blocks;
-            const int first = (live ? block : 0) * 128 + 4 * l32;
+            const int first = (live ? block : 0) * 128 + 4 * rotation.group;
             const __half* h = reinterpret_cast<const __half*>(&raw[u]);
             const __half* up = reinterpret_cast<const __half*>(&raw_up[u]);
             float v[4];
@@ -345,7 +398,7 @@ __device__ __forceinline__ float rotate_row_to_lds(const __half* __restrict__ x,
                 v[j] = live ? value * sign : 0.f;
             }
             __half out[4];
-            amax = fmaxf(amax, rotate_block(v, l32, out));
+            amax = fmaxf(amax, rotate_for_codes(v, rotation, out));
             if (live) *reinterpret_cast<uint2*>(rotated + first) = *reinterpret_cast<const uint2*>(out);
         }
     }
@@ -530,10 +583,19 @@ __global__ __launch_bounds__(256) void rotate_kernel(const __half* __restrict__ 
     }
 }
 
-// Sum over the first four waves, known to all.
+// Sum over the first four waves, known to all.  Halves first, then groups of channels at distance 16, 8, 4, 2, 1: the order of the fp32 sums is
+// that of the groups (RotationLane), by lane moves.
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
-#pragma unroll
-    for (int offset = 32; offset > 0; offset >>= 1) v += __shfl_xor(v, offset, 64);
+    typedef unsigned int pair_u32 __attribute__((ext_vector_type(2)));
+    const pair_u32 halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
+    const pair_u32 rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(rows[0]) + __uint_as_float(rows[1]);
+    auto partner = [&](auto control) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(control)::value, 0xF, 0xF, true)); };
+    v += partner(std::integral_constant<int, 0x128>{});  // eight lanes on
+    v += partner(std::integral_constant<int, 0x141>{});  // the mirrored half row
+    v += partner(std::integral_constant<int, 0x4E>{});   // the other pair
+    v += partner(std::integral_constant<int, 0xB1>{});   // the neighbour
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (lane == 0 && wave < 4) scratch[wave] = v;
     __syncthreads();
@@ -557,7 +619,8 @@ __global__ __launch_bounds__(THREADS) void residual_norm_rotate_a8_kernel(
     constexpr int kWaves = THREADS / 64;
     __shared__ float scratch[kWaves], sum_scratch[4];
     const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int half_wave = lane >> 5, l32 = lane & 31;
+    const int half_wave = lane >> 5;
+    const RotationLane rotation(lane & 31);
     const int blocks = k / 128;  // even: k is a multiple of 256
     const int64_t base = (int64_t)row * k;
     float squares = 0.f;
@@ -579,7 +642,7 @@ __global__ __launch_bounds__(THREADS) void residual_norm_rotate_a8_kernel(
         float4 residual[kHeld];
 #pragma unroll
         for (int u = 0; u < kHeld; ++u) {  // clamped, so unconditional (blocks is even: a pair is live or not as a whole)
-            const int first = (min(2 * (wave + kWaves * u), blocks - 2) + half_wave) * 128 + 4 * l32;
+            const int first = (min(2 * (wave + kWaves * u), blocks - 2) + half_wave) * 128 + 4 * rotation.group;
             raw[u] = *reinterpret_cast<const uint2*>(x + base + first);
             residual[u] = *reinterpret_cast<const float4*>(r + base + first);
             held_w[u] = *reinterpret_cast<const uint2*>(w + first);
@@ -588,7 +651,7 @@ __global__ __launch_bounds__(THREADS) void residual_norm_rotate_a8_kernel(
 #pragma unroll
         for (int u = 0; u < kHeld; ++u) {
             if (2 * (wave + kWaves * u) >= blocks) break;  // wave-uniform
-            const int first = (2 * (wave + kWaves * u) + half_wave) * 128 + 4 * l32;
+            const int first = (2 * (wave + kWaves * u) + half_wave) * 128 + 4 * rotation.group;
             const __half* h = reinterpret_cast<const __half*>(&raw[u]);
             float4 sum;
             sum.x = __half2float(h[0]) + residual[u].x;
@@ -604,7 +667,7 @@ __global__ __launch_bounds__(THREADS) void residual_norm_rotate_a8_kernel(
         }
     }
     for (int pair = wave + kWaves * kHeld; 2 * pair < blocks; pair += kWaves) {
-        const int first = (2 * pair + half_wave) * 128 + 4 * l32;
+        const int first = (2 * pair + half_wave) * 128 + 4 * rotation.group;
         const uint2 raw = *reinterpret_cast<const uint2*>(x + base + first);
         const __half* h = reinterpret_cast<const __half*>(&raw);
         const float4 residual = *reinterpret_cast<const float4*>(r + base + first);
@@ -640,16 +703,16 @@ __global__ __launch_bounds__(THREADS) void residual_norm_rotate_a8_kernel(
         }
         *reinterpret_cast<uint2*>(y + base + first) = *reinterpret_cast<const uint2*>(normalized);
         __half out[4];
-        amax = fmaxf(amax, rotate_block(v, l32, out));
+        amax = fmaxf(amax, rotate_for_codes(v, rotation, out));
         *reinterpret_cast<uint2*>(rotated + first) = *reinterpret_cast<const uint2*>(out);
     };
 #pragma unroll
     for (int u = 0; u < kHeld; ++u) {
         if (2 * (wave + kWaves * u) >= blocks) break;  // wave-uniform
-        second_pass((2 * (wave + kWaves * u) + half_wave) * 128 + 4 * l32, kept[u], held_w[u], held_sign[u]);
+        second_pass((2 * (wave + kWaves * u) + half_wave) * 128 + 4 * rotation.group, kept[u], held_w[u], held_sign[u]);
     }
     for (int pair = wave + kWaves * kHeld; 2 * pair < blocks; pair += kWaves) {
-        const int first = (2 * pair + half_wave) * 128 + 4 * l32;
+        const int first = (2 * pair + half_wave) * 128 + 4 * rotation.group;
         const float4 sum = *reinterpret_cast<const float4*>(ro + base + first);  // written above by this thread
         const uint2 raw_w = *reinterpret_cast<const uint2*>(w + first);
         const uint32_t sign_word = *reinterpret_cast<const uint32_t*>(signs + first);
