@@ -104,10 +104,25 @@ class QuantizedLinear:
         self.weight = _dev(stored)
         self.scales = _dev(scales)
         self.book = _dev(codebook.book() if book is None else book)
-        self.a_q = torch.empty((capacity, self.k), dtype=torch.int8, device="cuda")
+        # rows over panels: the quantiser leaves the int8 rows a second time, in the order of the matrix operands
+        top = min(capacity, PANEL_ROWS)
+        self.over_panels = [False] * (top + 1)
+        if algorithm == "auto" and not block_m and self.k % 128 == 0 and 256 <= self.k <= 32768 and self.n * self.k < 2**31:
+            pays = panels_pay if codec == "q4" else int8_panels_pay
+            cus = torch.cuda.get_device_properties(self.weight.device).multi_processor_count
+            self.over_panels = [pays(rows, self.n, self.k, cus) for rows in range(top + 1)]
+        # (both copies in one allocation: a second one, new from the driver, took 2 ms of a construction)
+        padded = (top + 15) // 16 * 16 if any(self.over_panels) else 0
+        codes = torch.empty((capacity + padded, self.k), dtype=torch.int8, device="cuda")
+        self.a_q, self.panels = codes[:capacity], codes[capacity:]
         self.a_s = torch.empty((capacity, 1), dtype=torch.float16, device="cuda")
         self.out = torch.empty((capacity, self.n), dtype=torch.float16, device="cuda")
         self.quantizer = Kernel("activation_quantization", K=self.k)
+        if padded:
+            self.sums = torch.empty(top, dtype=torch.int32, device="cuda")
+            self.panel_quantizer = Kernel("activation_quantization", K=self.k, panels=True)
+            variant = dict(M=top, N=self.n, K=self.k, dynamic_rows=True, panels=True)
+            self.panel_projection = Kernel("e8p_q4_projection", packed_k=packed_k, **variant) if codec == "q4" else Kernel("int8_projection", **variant)
         # workspace=True: the projection takes a `Workspace` buffer (allocated below, once, at the size
         # orx_workspace_bytes reports) for split tiles and decode-once launches
         variant = dict(M=capacity, N=self.n, K=self.k, dynamic_rows=True, algorithm=algorithm, workspace=True)
@@ -130,19 +145,6 @@ class QuantizedLinear:
                 if error.code != ORX_ERR_BAD_VARIANT:
                     raise
         self.workspace = self.projection.workspace()
-        # rows over panels: the quantiser leaves the int8 rows a second time, in the order of the matrix operands
-        top = min(capacity, PANEL_ROWS)
-        cus = torch.cuda.get_device_properties(self.weight.device).multi_processor_count
-        self.over_panels = [False] * (top + 1)
-        if algorithm == "auto" and not block_m and self.k % 128 == 0 and 256 <= self.k <= 32768 and self.n * self.k < 2**31:
-            pays = panels_pay if codec == "q4" else int8_panels_pay
-            self.over_panels = [pays(rows, self.n, self.k, cus) for rows in range(top + 1)]
-        if any(self.over_panels):
-            self.panels = torch.empty(((top + 15) // 16 * 16, self.k), dtype=torch.int8, device="cuda")
-            self.sums = torch.empty(top, dtype=torch.int32, device="cuda")
-            self.panel_quantizer = Kernel("activation_quantization", K=self.k, panels=True)
-            variant = dict(M=top, N=self.n, K=self.k, dynamic_rows=True, panels=True)
-            self.panel_projection = Kernel("e8p_q4_projection", packed_k=packed_k, **variant) if codec == "q4" else Kernel("int8_projection", **variant)
 
     def quantize(self, x16, stream=None):
         rows = x16.shape[0]
