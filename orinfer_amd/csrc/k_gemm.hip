@@ -1342,8 +1342,14 @@ int w8_panel_launch(const orx_function& f, int rows, const Geometry& g, hipStrea
 int panels_asked(const Variant& v, const orx_function& f, bool* asked) {
     bool bad = false;
     *asked = v.boolean("panels", false, &bad);
-    if (bad || (*asked && (f.input_f16 || v.string("algorithm", "auto", &bad) != "auto" || f.tiles != 0 || f.takes_workspace || !panel_eligible(f.capacity, f.N, f.K)))) {
-        set_error("%s: panels=true serves int8 rows, up to 2048 of them, K a multiple of 128 from 256, algorithm auto, without block_m and workspace", f.symbol.c_str());
+    if (bad || (*asked && (f.input_f16 || v.string("algorithm", "auto", &bad) != "auto" || f.takes_workspace || !panel_eligible(f.capacity, f.N, f.K)))) {
+        set_error("%s: panels=true serves int8 rows, up to 2048 of them, K a multiple of 128 from 256, algorithm auto, without workspace", f.symbol.c_str());
+        return ORX_ERR_BAD_VARIANT;
+    }
+    // keys that choose among the other kernels (as they were given: make_projection has turned row tiles of 1-8, 16, 96 and 192 into hints)
+    const bool split_named = v.has("split_k") && (v.fields.at("split_k").kind == Value::Number || !v.boolean("split_k", true, &bad));
+    if (*asked && (v.integer("block_m", 0, &bad) != 0 || v.integer("gemv_passes", 0, &bad) != 0 || v.boolean("decode_in_gemm", false, &bad) || split_named)) {
+        set_error("%s: panels=true has one kernel: block_m, gemv_passes, split_k and decode_in_gemm choose nothing there", f.symbol.c_str());
         return ORX_ERR_BAD_VARIANT;
     }
     return ORX_OK;

@@ -347,6 +347,18 @@ def test_which_rows_an_int8_linear_takes_over_panels(n, k, lines):
         assert int8_panels_pay(rows, n, k, 256) == bool(taken), rows
 
 
+@pytest.mark.parametrize("symbol", ["e8p_q4_projection", "int8_projection"])
+def test_over_panels_no_key_is_dropped(symbol):
+    """The one kernel behind panels=true serves none of the keys that choose among the others, row tiles that are hints elsewhere included."""
+    shape = dict(M=200, N=512, K=512, panels=True)
+    lib.Kernel(symbol, split_k=True, workspace=False, **shape)
+    keys = [dict(block_m=m) for m in (1, 8, 16, 32, 96, 192, 256)] + [dict(split_k=False), dict(split_k=2), dict(gemv_passes=2), dict(decode_in_gemm=True)]
+    for key in keys:
+        with pytest.raises(lib.OrxError) as err:
+            lib.Kernel(symbol, **shape, **key)
+        assert err.value.code == lib.ORX_ERR_BAD_VARIANT, key
+
+
 @pytest.mark.parametrize("codec, n, k, rows", [("w8", 4096, 12288, 128), ("w8", 4096, 12288, 256), ("q4", 4096, 12288, 384), ("q4", 7168, 1024, 130)])
 def test_which_rows_the_channel_runs_leave(codec, n, k, rows):
     symbol, shape = {"q4": "e8p_q4_projection", "w8": "int8_projection"}[codec], dict(M=rows, N=n, K=k, workspace=True)
