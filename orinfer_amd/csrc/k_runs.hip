@@ -184,7 +184,8 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
         request(1, one);
         if constexpr (D > 2) request(2, std::integral_constant<int, 2>{});
         if constexpr (D > 3) request(3, std::integral_constant<int, 3>{});
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        // (the waves that make no tables have not waited for their selector word, whose register is free from here on)
+        asm volatile("s_waitcnt vmcnt(%2) lgkmcnt(0)\n\ts_barrier" : "+v"(selector), "+v"(scale_bits) : "n"(std::min(D * kRequests, 63)) : "memory");
 
         const QuadLookup<kEntry> tables(lane);
         // Sums in accumulation registers where a wave has its SIMD to itself.  The rows' sums of codes then by a multiply with ones, of four registers

@@ -1,0 +1,146 @@
+"""What the kernels with hand-written waits and multiplies rest on, checked in the code that the compiler made of them.
+
+An asm statement that loads or multiplies hides its latency from the compiler, which takes the result as written at once: it could copy a
+register between the load and its wait, or a sum behind a multiply that is still on its way, and no source line would show it.  The check follows every
+path through the disassembly of the kernels built here and finds such a use, whatever compiler built them."""
+import re
+import subprocess
+from pathlib import Path
+
+import pytest
+
+from orinfer_amd import build, lib
+
+LLVM = Path(build.hipcc()).resolve().parents[1]
+OBJDUMP = next((p for p in (LLVM / "llvm/bin/llvm-objdump", LLVM / "lib/llvm/bin/llvm-objdump", Path("/opt/rocm/llvm/bin/llvm-objdump")) if p.exists()), None)
+FAR = 64  # wait states, or younger requests: as good as any number
+RESULT_WAIT = 8  # wait states that the compiler itself keeps between v_mfma_i32_16x16x64_i8 and another access to its sum
+
+
+def parse_registers(text):
+    """VGPRs as their numbers, accumulation registers from 1000 on."""
+    found = []
+    for kind, one, low, high in re.findall(r"\b([va])(?:(\d+)\b|\[(\d+):(\d+)\])", text):
+        numbers = range(int(one), int(one) + 1) if one else range(int(low), int(high) + 1)
+        found.extend(n + (1000 if kind == "a" else 0) for n in numbers)
+    return tuple(found)
+
+
+class Instruction:
+    def __init__(self, text):
+        self.text = text
+        self.name, _, operands = text.partition(" ")
+        first = parse_registers(operands.partition(",")[0])
+        self.all = parse_registers(operands)
+        if self.name == "v_mad_u64_u32":  # (made of 32-bit sums too: the addend's upper half is then any register, and nobody reads the result's)
+            self.all = self.all[:-1]
+        self.multiply = self.name.startswith("v_mfma")
+        self.sum = first if self.multiply else ()
+        self.memory = self.name.startswith(("global_", "buffer_", "flat_", "scratch_"))
+        self.loads = first if self.name in ("global_load_dword", "global_load_ushort") else ()
+        counted = re.search(r"vmcnt\((\d+)\)", text) if self.name == "s_waitcnt" else None
+        self.younger = int(counted.group(1)) if counted else None
+        self.states = 1 + (int(operands) if self.name == "s_nop" else 0)
+
+
+def kernels(listing):
+    """(name, [(address, Instruction)], {address of a branch: its target}) of every kernel in a disassembly."""
+    name, code, targets, base = None, [], {}, 0
+    known = {}
+    for line in listing.splitlines():
+        header = re.match(r"^([0-9a-f]+) <(.*)>:", line)
+        if header:
+            if code:
+                yield name, code, targets
+            name, code, targets, base = header.group(2), [], {}, int(header.group(1), 16)
+            continue
+        text, _, comment = line.partition("//")
+        text = " ".join(text.split())
+        if not text or not comment:
+            continue
+        address = int(comment.split(":")[0], 16)
+        target = re.search(r"<.*?(?:\+0x([0-9a-f]+))?>\s*$", comment)
+        if text.startswith(("s_cbranch", "s_branch")):
+            targets[address] = base + int(target.group(1) or "0", 16)
+            text = text.split()[0]
+        code.append((address, known.setdefault(text, Instruction(text))))
+    if code:
+        yield name, code, targets
+
+
+def faults(code, targets):
+    """Uses of a register whose set-up load or multiply may not have ended, over all paths.  (Loads of 16 bytes are left out: their waits and requests hang together
+    by uniform conditions and loop counts, which a walk over all paths does not know.)"""
+    index = {address: i for i, (address, _) in enumerate(code)}
+    starts = {0} | {index[t] for t in targets.values()} | {index[a] + 1 for a in targets}
+    found, seen, work = set(), {}, [(0, ({}, {}))]
+    while work:
+        i, state = work.pop()
+        if i in seen:  # the shortest way to every register's last event
+            merged = tuple({r: min(old.get(r, FAR), new.get(r, FAR)) for r in {*old, *new}} for old, new in zip(seen[i], state))
+            if merged == seen[i]:
+                continue
+            state = merged
+        seen[i] = state
+        loaded, multiplied = state  # younger requests; wait states since
+        while True:
+            address, ins = code[i]
+            for r in ins.all:
+                if r in loaded:
+                    found.add(f"{ins.text}: register {r} is on its way")
+                if r in multiplied and not ins.multiply:
+                    found.add(f"{ins.text}: register {r} is a sum of {multiplied[r]} wait states ago")
+            multiplied = {r: n + ins.states for r, n in multiplied.items() if n + ins.states < RESULT_WAIT}
+            if ins.multiply:
+                multiplied.update(dict.fromkeys(ins.sum, 0))
+            if ins.memory:
+                loaded = {r: n + 1 for r, n in loaded.items()}
+                loaded.update(dict.fromkeys(ins.loads, 0))
+            if ins.younger is not None:
+                loaded = {r: n for r, n in loaded.items() if n < ins.younger}
+            if ins.name == "s_endpgm":
+                break
+            if address in targets:
+                work.append((index[targets[address]], (loaded, multiplied)))
+                if ins.name == "s_branch":
+                    break
+            i += 1
+            if i == len(code):
+                break
+            if i in starts:
+                work.append((i, (loaded, multiplied)))
+                break
+    return found
+
+
+@pytest.fixture(scope="module")
+def built(tmp_path_factory):
+    """The code objects in the library, disassembled: {kernel: (code, targets)}."""
+    folder = tmp_path_factory.mktemp("code")
+    (folder / "lib.so").write_bytes(Path(lib.LIBRARY_PATH).read_bytes())
+    subprocess.run([OBJDUMP, "--offloading", "lib.so"], cwd=folder, check=True, capture_output=True)
+    out = {}
+    for part in sorted(folder.glob("*gfx950*")):
+        listing = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", part.name], cwd=folder, check=True, capture_output=True, text=True).stdout
+        out.update({name: (code, targets) for name, code, targets in kernels(listing)})
+    return out
+
+
+@pytest.mark.parametrize("family, count", [("panel_kernel", 60), ("runs_kernel", 50), ("grouped_bulk_kernel", 4)])
+def test_nothing_touches_a_register_that_is_on_its_way(built, family, count):
+    chosen = {name: code for name, code in built.items() if family in name}
+    assert len(chosen) >= count
+    for name, (code, targets) in chosen.items():
+        assert not (problems := faults(code, targets)), (name, sorted(problems)[:5])
+
+
+def test_sums_of_the_panel_kernel_stay_where_they_are(built):
+    """Its multiplies are asm statements on every side of a branch: no register moves between the first and the last, and only multiplies name the sums."""
+    for name, (code, _) in built.items():
+        if "panel_kernel" not in name:
+            continue
+        at = [i for i, (_, ins) in enumerate(code) if ins.multiply]
+        sums = {r for i in at for r in code[i][1].sum}
+        for _, ins in code[at[0]:at[-1]]:
+            assert ins.multiply or not sums & set(ins.all), (name, ins.text)
+            assert not ins.name.startswith(("v_mov", "v_accvgpr", "v_swap", "scratch_")), (name, ins.text)
