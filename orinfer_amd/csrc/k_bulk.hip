@@ -143,10 +143,7 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
         const uint32_t token_slots = lds_address_of(lds) + kTokens + (uint32_t)wave * (LOADS * 1024);
         auto issue_tokens = [&](int chunk, int slot) {  // (the instruction's offset counts in memory too and is taken off the lane's)
             const int8_t* const base = a_base + (int64_t)min(chunk, chunks - 1) * 128 - 4096;
-            const uint32_t to = token_slots + (uint32_t)slot * kSlot;
-            request_16<true, 0>(row_offset[0], base, to);
-            if constexpr (LOADS > 1) request_16<false, 1024>(row_offset[1], base, to);
-            if constexpr (LOADS > 2) request_16<false, 2048>(row_offset[2], base, to), request_16<false, 3072>(row_offset[3], base, to);
+            request_rows_16(row_offset, base, token_slots + (uint32_t)slot * kSlot);
         };
         // two register sets of codes, by the parity of the chunk: four blocks of 16 channels, 8 bytes to a lane
         v2u codes[2][4];

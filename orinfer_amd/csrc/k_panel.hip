@@ -144,7 +144,7 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
         constexpr int u = decltype(tag)::value;
         const uint8_t* const from = w_base + (uint64_t)(uint32_t)min(phase * PH + unit_chunk[u], chunks - 1) * p.chunk_stride;
         const uint32_t to = unit_weights[u] + (phase & 1 ? kPhaseBytes<CB> : 0u);
-        if (u < U - 1 || last_unit) request_16<true, 0>(unit_codes[u], from, to), request_16<true, 0>(unit_codes[u] + 16, from, to + CB * 1024);
+        if (u < U - 1 || last_unit) request_16<0>(unit_codes[u], from, to), request_16<0>(unit_codes[u] + 16, from, to + CB * 1024);
     };
     const int row_blocks = (rows + 15) / 16;
     const uint8_t* token_base[TB];

@@ -151,8 +151,10 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
             constexpr int INDEX = decltype(index_tag)::value, SLOT = decltype(slot_tag)::value, ROW = INDEX - CB;
             if constexpr (INDEX < CB)
                 load_16(codes[SLOT][INDEX], code_offset[INDEX], weights);
+            else if constexpr ((ROW & 3) == 0)
+                request_16<0>(row_offset[ROW], rows_from, ring_address + SLOT * kStage + ROW * 1024);
             else
-                request_16<(ROW & 3) == 0, (ROW & 3) * 1024>(row_offset[ROW], rows_from, ring_address + SLOT * kStage + ROW * 1024);
+                request_16_behind<(ROW & 3) * 1024>(row_offset[ROW], rows_from);
         };
         auto rows_of_chunk = [&](int index) ORX_INLINE { return reinterpret_cast<const uint8_t*>(a_base) + (int64_t)min(begin + index, last) * 128 - 4096; };
         auto codes_of_chunk = [&](int index) ORX_INLINE { return w_base + (uint64_t)min(begin + index, last) * p.chunk_stride; };

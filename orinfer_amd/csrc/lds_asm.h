@@ -24,14 +24,36 @@ __device__ __forceinline__ void direct_load_16(const void* global, void* lds_wav
                                      (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, 0);
 }
 // The same from an asm statement: a uniform base and 32 bits per lane, and no wait in front of the LDS accesses that the compiler
-// can see.  OFFSET counts on both sides; the LDS base stays set for the requests that follow with set_lds_base left out.
-template <bool SET_LDS_BASE, int OFFSET>
+// can see.  OFFSET counts on both sides.  The statements that set m0 name it: else the compiler holds what its last direct_load_16 left there for unchanged.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // (m0 is reserved: it holds nothing of the compiler's from one statement to the next)
+template <int OFFSET>
 __device__ __forceinline__ void request_16(uint32_t lane_offset, const void* uniform_base, uint32_t lds_wave_base) {
-    if constexpr (SET_LDS_BASE)
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3" ::"v"(lane_offset), "s"(uniform_base), "s"(lds_wave_base), "n"(OFFSET)
-                     : "memory");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3" ::"v"(lane_offset), "s"(uniform_base), "s"(lds_wave_base), "n"(OFFSET)
+                 : "memory", "m0");
+}
+// COUNT (1, 2 or 4) requests of 1 KiB, one behind the other in LDS.
+template <int COUNT>
+__device__ __forceinline__ void request_rows_16(const uint32_t (&lane_offset)[COUNT], const void* uniform_base, uint32_t lds_wave_base) {
+    static_assert(COUNT == 1 || COUNT == 2 || COUNT == 4, "one, two or four requests to a statement");
+    if constexpr (COUNT == 1)
+        request_16<0>(lane_offset[0], uniform_base, lds_wave_base);
+    else if constexpr (COUNT == 2)
+        asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2\n\tglobal_load_lds_dwordx4 %1, %2 offset:1024" ::"v"(lane_offset[0]), "v"(lane_offset[1]),
+                     "s"(uniform_base), "s"(lds_wave_base)
+                     : "memory", "m0");
     else
-        asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" ::"v"(lane_offset), "s"(uniform_base), "n"(OFFSET) : "memory");
+        asm volatile("s_mov_b32 m0, %5\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %4\n\tglobal_load_lds_dwordx4 %1, %4 offset:1024\n\t"
+                     "global_load_lds_dwordx4 %2, %4 offset:2048\n\tglobal_load_lds_dwordx4 %3, %4 offset:3072" ::"v"(lane_offset[0]), "v"(lane_offset[1]), "v"(lane_offset[2]),
+                     "v"(lane_offset[3]), "s"(uniform_base), "s"(lds_wave_base)
+                     : "memory", "m0");
+}
+#pragma clang diagnostic pop
+// A request OFFSET behind the last request_16, by the m0 that this one left: for a kernel whose only writes of m0 are request_16's, so for none with a
+// direct_load_16 or another builtin that needs m0 (the check of the built kernels in tests/test_codegen.py counts them).
+template <int OFFSET>
+__device__ __forceinline__ void request_16_behind(uint32_t lane_offset, const void* uniform_base) {
+    asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" ::"v"(lane_offset), "s"(uniform_base), "n"(OFFSET) : "memory");
 }
 __device__ __forceinline__ void lds_write_16(uint32_t address, v4u value) {
     asm volatile("ds_write_b128 %0, %1" ::"v"(address), "v"(value) : "memory");

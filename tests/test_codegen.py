@@ -144,3 +144,36 @@ def test_sums_of_the_panel_kernel_stay_where_they_are(built):
         for _, ins in code[at[0]:at[-1]]:
             assert ins.multiply or not sums & set(ins.all), (name, ins.text)
             assert not ins.name.startswith(("v_mov", "v_accvgpr", "v_swap", "scratch_")), (name, ins.text)
+
+
+def test_requests_that_share_an_lds_base_keep_it(built):
+    """Kernels with a request that sets no m0 of its own write m0 nowhere but in front of one that does."""
+    families = 0
+    for name, (code, _) in built.items():
+        if not ("grouped_bulk_kernel" in name or "panel_kernelILi1" in name or "runs_kernelILi0" in name):
+            continue
+        texts, families = [ins.text for _, ins in code], families + 1
+        for i, text in enumerate(texts):
+            if re.search(r"\bm0\b", text):
+                assert text.startswith("s_mov_b32 m0, ") and texts[i + 1] == "s_nop 0" and texts[i + 2].startswith("global_load_lds_dwordx4"), (name, texts[i:i + 3])
+    assert families >= 4 + 30 + 32
+
+
+def test_a_request_does_not_hide_the_lds_base_of_a_builtin(tmp_path):
+    """request_16 between two direct_load_16 to one place: the second sets its base again."""
+    source = tmp_path / "both.hip"
+    source.write_text('''#include "lds_asm.h"
+using namespace orx::lds_asm;
+extern "C" __global__ void both(const uint8_t* a, const uint8_t* b, int* out) {
+    __shared__ __align__(16) uint8_t first[1024], second[1024];
+    direct_load_16(a + threadIdx.x * 16, first);
+    request_16<REQUEST>(threadIdx.x * 16, b, lds_address_of(second));
+    direct_load_16(a + threadIdx.x * 16 + 4096, first);
+    __syncthreads();
+    out[threadIdx.x] = first[threadIdx.x] + second[threadIdx.x];
+}
+''')
+    done = subprocess.run([build.hipcc(), *build.FLAGS, "-Werror=inline-asm", f"-I{build.CSRC}", "-DREQUEST=0", "--cuda-device-only", "-S", str(source), "-o", "-"],
+                          capture_output=True, text=True, check=True)
+    order = [line.split()[0] for line in done.stdout.splitlines() if re.match(r"\s+(s_mov_b32 m0|global_load_lds)", line)]
+    assert order == ["s_mov_b32", "global_load_lds_dwordx4"] * 3
