@@ -1793,6 +1793,45 @@ def test_a_linear_over_panels_gives_the_bits_of_the_row_major_one(codec):
         assert torch.equal(got, want)
 
 
+# Every form of the panel kernel (blocks of channels to a workgroup, of rows to a wave, rows that leave waves a block short) through its steady state: four phases,
+# the last one short, so that codes requested inside the loop are multiplied and both weight buffers are written again after they were.  Sums by 64-bit products, exact.
+@pytest.mark.parametrize("codec", ["q4", "w8"])
+@pytest.mark.parametrize("blocks,n,k", [(1, 1000, 3456), (2, 5000, 3456), (3, 8200, 1920), (4, 12290, 1920), (5, 16400, 1920)])
+def test_panel_forms_through_many_phases(blocks, n, k, codec):
+    rng = np.random.default_rng(orc.SEED + n)
+    a_q = rng.integers(-127, 128, (512, k), dtype=np.int8)
+    a_s, ws = rng.uniform(0.005, 0.02, 512).astype(np.float16), rng.uniform(0.005, 0.02, n).astype(np.float16)
+    weight = rng.integers(0, 2**32, (n, k // 8), dtype=np.uint32) if codec == "q4" else rng.integers(-128, 128, (n, k), dtype=np.int8)
+    integers = orc.q4_integers(weight, TABLE) if codec == "q4" else weight
+    acc = gu.host(gu.dev(a_q).double() @ gu.dev(integers).double().T).astype(np.int32)
+    symbol, stored = ("e8p_q4_projection", gu.dev(weight)) if codec == "q4" else ("int8_projection", gu.dev(weight))
+    for rows in (200, 256, 300, 384, 450, 512):
+        kernel = gu.kernel(symbol, M=rows, N=n, K=k, panels=True, workspace=False)
+        units = kernel.geometry(rows)[0][0]
+        assert -(-(-(-n // 16)) // units) == blocks or torch.cuda.get_device_properties(0).multi_processor_count != 256
+        out = torch.full((rows + 1, n), 91, dtype=torch.float16, device=gu.DEV)
+        if codec == "q4":
+            kernel(A=gu.dev(in_panels(a_q[:rows])), AS=gu.dev(a_s), Book=gu.book(), Out=out, S=gu.dev(ws),
+                   Sums=gu.dev(a_q[:rows].astype(np.int32).sum(1).astype(np.int32)), W=stored)
+        else:
+            kernel(A=gu.dev(in_panels(a_q[:rows])), Output=out, TokenScale=gu.dev(a_s), Weight=stored, WeightScale=gu.dev(ws))
+        np.testing.assert_array_equal(gu.host(out)[:rows], orc.rescale(acc[:rows], ws, a_s[:rows], np.float16), err_msg=f"{rows} rows")
+        assert (gu.host(out)[rows] == 91).all()
+
+
+@pytest.mark.parametrize("codec, packed_k", [("q4", 0), ("q4", 128), ("w8", 0)])
+def test_a_linear_over_panels_of_a_long_k(codec, packed_k):
+    rng = np.random.default_rng(orc.SEED + 1)
+    n, k = 7168, 5120
+    weight = rng.integers(0, 2**32, (n, k // 8), dtype=np.uint32) if codec == "q4" else rng.integers(-127, 128, (n, k), dtype=np.int8)
+    linear = programs.QuantizedLinear(codec, weight, rng.uniform(0.005, 0.02, n).astype(np.float16), 512, packed_k=packed_k)
+    for rows in (200, 256, 333, 512):
+        assert linear.over_panels[rows] or torch.cuda.get_device_properties(0).multi_processor_count != 256
+        x = gu.dev(rng.normal(0, 1, (rows, k)).astype(np.float16))
+        got = linear.run(x).clone()
+        assert torch.equal(got, linear.project(linear.quantize(x))), rows
+
+
 def test_panels_are_refused_where_no_kernel_serves_them():
     for symbol, variant in (("activation_quantization", dict(K=1000, panels=True)), ("activation_quantization", dict(K=256, group_size=128, panels=True)),
                             ("activation_quantization", dict(K=256, fused=True, panels=True)), ("activation_quantization", dict(K=32896, panels=True)),
