@@ -307,6 +307,9 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelParams p) {
             });
             if constexpr (m % CB == CB - 1) request_token(token[token_set][i], offset, token_base[i]);
         });
+        // (Here and behind `done` stretches of code meet with multiplies and requests on their way, of which the compiler knows nothing: it must move no sum and no
+        // token between registers there.  It has no reason to, and tests/test_codegen.py finds it in the built kernels if it does; a pause of 16 cycles a slice would
+        // take its place.)
         if (!EVEN && last_block) {
             Each<CB>::run([&](auto j_tag) ORX_INLINE {
                 constexpr int i = TB - 1, j = (i & 1) ? CB - 1 - decltype(j_tag)::value : decltype(j_tag)::value;

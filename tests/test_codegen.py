@@ -37,7 +37,9 @@ class Instruction:
         self.multiply = self.name.startswith("v_mfma")
         self.sum = first if self.multiply else ()
         self.memory = self.name.startswith(("global_", "buffer_", "flat_", "scratch_"))
-        self.loads = first if self.name in ("global_load_dword", "global_load_ushort") else ()
+        self.wide = self.name in ("global_load_dwordx2", "global_load_dwordx4")
+        self.loads = first if self.wide or self.name in ("global_load_dword", "global_load_ushort") else ()
+        self.move = self.name.startswith(("v_mov", "v_accvgpr", "v_swap", "scratch_"))
         counted = re.search(r"vmcnt\((\d+)\)", text) if self.name == "s_waitcnt" else None
         self.younger = int(counted.group(1)) if counted else None
         self.states = 1 + (int(operands) if self.name == "s_nop" else 0)
@@ -69,8 +71,8 @@ def kernels(listing):
 
 
 def faults(code, targets):
-    """Uses of a register whose set-up load or multiply may not have ended, over all paths.  (Loads of 16 bytes are left out: their waits and requests hang together
-    by uniform conditions and loop counts, which a walk over all paths does not know.)"""
+    """Uses of a register whose load or multiply may not have ended, over all paths; of 8 and 16 bytes in flight, moves only.  (The waits for those hang together with
+    their requests by uniform conditions and loop counts, which a walk over all paths does not know.)"""
     index = {address: i for i, (address, _) in enumerate(code)}
     starts = {0} | {index[t] for t in targets.values()} | {index[a] + 1 for a in targets}
     found, seen, work = set(), {}, [(0, ({}, {}))]
@@ -82,11 +84,11 @@ def faults(code, targets):
                 continue
             state = merged
         seen[i] = state
-        loaded, multiplied = state  # younger requests; wait states since
+        loaded, multiplied = dict(state[0]), state[1]  # younger requests, by register and width; wait states since
         while True:
             address, ins = code[i]
             for r in ins.all:
-                if r in loaded:
+                if (r, False) in loaded or (ins.move and (r, True) in loaded):
                     found.add(f"{ins.text}: register {r} is on its way")
                 if r in multiplied and not ins.multiply:
                     found.add(f"{ins.text}: register {r} is a sum of {multiplied[r]} wait states ago")
@@ -95,7 +97,9 @@ def faults(code, targets):
                 multiplied.update(dict.fromkeys(ins.sum, 0))
             if ins.memory:
                 loaded = {r: n + 1 for r, n in loaded.items()}
-                loaded.update(dict.fromkeys(ins.loads, 0))
+                for r in ins.loads:
+                    loaded.pop((r, not ins.wide), None)
+                    loaded[r, ins.wide] = 0
             if ins.younger is not None:
                 loaded = {r: n for r, n in loaded.items() if n < ins.younger}
             if ins.name == "s_endpgm":
