@@ -47,17 +47,6 @@ using namespace lds_asm;
 
 constexpr int kPanelWaves = 8, kPanelThreads = kPanelWaves * 64, kPanelRows = 512;
 
-template <int COUNT>
-struct Each {
-    template <typename Body>
-    static __device__ __forceinline__ void run(Body body) {
-        if constexpr (COUNT > 0) {
-            Each<COUNT - 1>::run(body);
-            body(std::integral_constant<int, COUNT - 1>{});
-        }
-    }
-};
-
 struct PanelParams {
     const uint8_t* panels;
     const int* sums;

@@ -73,18 +73,6 @@ constexpr uint32_t runs_lds() {
     return rings > sums ? rings : sums;
 }
 
-// body(0) .. body(COUNT - 1), each with its number as a constant
-template <int COUNT>
-struct Each {
-    template <typename Body>
-    static __device__ __forceinline__ void run(Body body) {
-        if constexpr (COUNT > 0) {
-            Each<COUNT - 1>::run(body);
-            body(std::integral_constant<int, COUNT - 1>{});
-        }
-    }
-};
-
 // fragments FIRST .. FIRST + COUNT - 1 of 16 rows each
 template <int COUNT, int FIRST>
 __device__ __forceinline__ void read_fragments(v4i* to, uint32_t address) {

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 namespace orx {
 namespace lds_asm {
@@ -12,6 +13,18 @@ namespace lds_asm {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef unsigned int v2u __attribute__((ext_vector_type(2)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+
+// body(0) .. body(COUNT - 1), each with its number as a constant
+template <int COUNT>
+struct Each {
+    template <typename Body>
+    static __device__ __forceinline__ void run(Body body) {
+        if constexpr (COUNT > 0) {
+            Each<COUNT - 1>::run(body);
+            body(std::integral_constant<int, COUNT - 1>{});
+        }
+    }
+};
 
 // Rows of 128 bytes in LDS: the piece at position p of a row is kept at p ^ swizzle(row), so that the 16 rows of a
 // fragment read spread over the banks.
