@@ -710,8 +710,11 @@ int tile_for(const orx_function& f, int rows) {
 //   one block, runs against the streaming kernel: 2048 x 4224 at 2 rows 6.8 to 7.0 / 7.0 to 7.2, 16 rows 7.0 to 7.2 / 7.3 to 8.3, 32 rows 7.5 to 8.7 / 7.8 to 10.2;
 //     K = 17408 at 16 rows 0.72 / 0.57 of its time; up to 16 rows level or slower below K = 4096 (2048 x 2560 5.4 to 5.0 / 5.5 to 5.1), above 16 rows
 //     faster from K = 3072 on (2048 x 3584 at 32 rows 6.9 to 7.5);
-//   two blocks: 7168 x 5376 at 2 rows 9.8 to 8.3 / 10.3 to 8.7, 24 rows 10.8 to 9.2 / 12.2 to 10.9; the runs get there with rows times K: 7168 x 17408 at 16 rows
-//     1.06 / 0.97 of its time, 32 rows 0.93 / 0.84; 7168 x 5120 row-major at 24 / 32 rows 1.06 / 0.98;
+//   two blocks, 5120 to 8192 channels, the runs' time over the streaming kernel's at 2 to 32 rows.  K-major: K = 1024 1.18-1.29, 2048 1.07-1.18, 3072 1.01-1.15, 4096 1.00-1.16,
+//     5120 0.94-1.12 (7168 x 5120 at 20 rows 9.2 to 8.5, 5120 x 5120 level); K = 8192 of 20 channels to a CU 0.88-0.98, of 24 0.92-1.02, of 28 and 32 0.95-1.08, where
+//     the line by rows times K, drawn before the runs' decode got cheaper, still has the streaming kernel (1.03-1.13 of the time); 7168 x 17408 at 32 rows 0.93.
+//     Row-major: K to 2048 1.15-1.57, 3072 1.02-1.34, 4096 1.11-1.24 up to 16 rows and 0.92-1.07 above, 5120 1.08-1.20 and 0.98-1.06; 8192 up to 16 rows 0.92-1.00 of 20 and 24
+//     channels, 1.00-1.11 of 28 and 32 (profiles/few_rows_of_codes_two_blocks.txt);
 //   three blocks, 9728 to 12288 channels: K = 3200 at 24 rows 0.90 to 0.92 / 0.92 to 0.95 of its time, K = 2688 0.94 to 0.98, K = 4224 at 3 to 16 rows 0.81 to 0.94 / 0.84 to 0.95, K = 3200
 //     0.88 to 1.02 (K-major up to 16 rows only above K = 5376, 0.83 at 8 rows of it: the records of such handles name the streaming kernel); two rows stay with the GEMV
 //     (9728 x 9728 18.7 to 17.0 / row-major);
@@ -723,7 +726,7 @@ int tile_for(const orx_function& f, int rows) {
 // at 17 rows of K = 5120 and 20 of 4096 (0.87-0.93, 0.91-0.97 of its time; 24 rows of K = 3072 0.97-1.03), with three at 20 rows of K = 5120
 // (0.91-0.93; 17 rows 0.99-1.02, 20 rows of K = 4096 0.99), row-major with one block at 24 rows of K = 5120 (1024 x 4096 at 32 rows 0.85); row-major
 // with three they do not (32 rows of K = 5120 1.05); with two blocks the streaming kernel passes it (use_resident); with five the runs win
-// less than runs differ (17408 x 5120 0.93-1.01).  The other one (row-major, K to 8192) is slower than the runs with one
+// less than runs differ (17408 x 5120 at 8 / 16 rows 14.5 / 15.5, the runs 14.6 / 14.7).  The other one (row-major, K to 8192) is slower than the runs with one
 // block (4096 x 8192 at 8 / 24 rows: the runs 0.81 / 0.74 of it), and with three above 16 rows from rows times K = 120 K on (9728 x 6144 at 17 / 20 rows 0.95 /
 // 0.90, x 8192 at 8 / 17 rows 0.96 / 0.80; 12288 x 6144 at 20 / 24 rows 0.98 / 0.94).
 int channel_blocks_per_cu(int n) { return (int)ceil_div(ceil_div((uint32_t)n, 16u), (uint32_t)device_compute_units()); }
@@ -772,13 +775,15 @@ bool runs_for_33_to_64_rows(const orx_function& f) {
 //     the wide kernel (17408 x 4096 1.0-1.22, 24576 x 4096 0.99-1.11) and win where that takes two itself, above 96 channels to a CU: 28672 and 34816 x 2048 / 5120 0.78-0.82 and
 //     0.92-1.0 / 0.76-0.81 and 0.88-0.96, K = 1024 0.85-0.95 and 1.0-1.13;
 //   codes, 129 to 512 rows in row tiles of 65 to 128, against split and whole 128 x 128 tiles, the 512-row runs of k_gemm_big.hip and decode once + 256 x 256 tiles:
-//     one round 0.34-0.83 (7168 x 2048 / 5120 at 200 rows 0.59 / 0.57).  Two row tiles of more than 120 rows and more than 16 channels, and 129 or 130 rows of K = 1024, are 0.5-0.8 too, but
-//     handles of such matrices declare scratch for these launches, and what they declare they use;
+//     one round 0.34-0.83 (7168 x 2048 / 5120 at 200 rows 0.59 / 0.57).  Two row tiles of more than 120 rows and more than 16 channels (0.60-0.65), and 129 or 130 rows of K = 1024, are 0.5-0.8 too, but
+//     handles of such matrices declare scratch for these launches, which is asserted of them, and what they declare they use: the lines at 240 and 130 rows are where
+//     that begins, nothing in the kernels;
 //     two rounds, K from 1536: up to 40 channels in a workgroup 0.75-0.97 in tiles of up to 112 rows and 0.86-1.06 above (9728 at 200 / 256 rows),
 //     wider 0.63-0.98 (12288 x 4096 at 130 / 256 0.65 / 0.76); K = 1024 0.9-1.2.  Matrices of 17 to 32 channels to a CU, 0.60-0.98 at 257 to 512 rows (7168 x 5120 0.69-0.82), keep the
 //     split tiles there: a launch record holds one grid expression, and a program of theirs has no room for two more;
 //     three rounds: tiles of up to 96 rows 0.74-0.97 from K = 3072 (17408 x 5120 at 130-192 rows 57 -> 43, 24576 x 5120 72 -> 51), K = 2048 0.9-1.1;
-//     above, up to 48 channels 0.82-0.96 from K = 4096 and wider 0.83-0.96 from K = 8192, below 0.95-1.4;
+//     above, up to 48 channels 0.82-0.96 from K = 4096 and wider 0.83-0.96 from K = 8192, below 0.95-1.4.  129 rows, 0.66-0.91 like 130, stay with the 512-row
+//     runs: what a handle starts at 129 rows of such a matrix is asserted, and programs may have recorded it (17408 x 5120 56.3, the runs 43.1);
 //     four and five up to 256 rows: tiles of up to 96 rows 0.85-0.97 from K = 4096 (34816 x 5120 at 160 rows 96 -> 82), all others 0.97-2;
 //   int8, 65 to 128 rows in one round: 0.1-0.9, except long K: 128 rows of K = 8192 / 10240 / 12288 up to 16 channels to a CU 0.84-0.88 / 0.98-1.03 / 1.04-1.08 (112 rows
 //     0.76-0.82 / 0.91-0.94 / 0.96-0.99), 17 to 32 channels 0.80-0.86 / 0.84-0.97 / 0.85-1.01;

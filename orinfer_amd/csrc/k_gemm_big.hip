@@ -261,7 +261,7 @@ __global__ __launch_bounds__(kPersistentThreads) void gemm_big_persistent_kernel
             }
     };
 
-    // ---- epilogue of one tile, wave-private, in registers ----
+    // ---- epilogue of one tile, wave-private: fp16 through the stage that nobody reads any more, fp32 out of the registers ----
     auto epilogue = [&](const TileState& t, int stage) {  // stage: the one that is free
         // the lane number is made opaque here: addresses and bounds that depend only on it would otherwise be
         // computed once in front of the K loop and held in registers (or spilled) for the whole kernel

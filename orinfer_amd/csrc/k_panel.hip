@@ -7,7 +7,7 @@
 //  * The quantiser leaves the int8 rows as panels besides (k_quant.hip): 1 KiB for 16 rows and 64 of K, in the order in which the
 //    lanes of v_mfma_i32_16x16x64_i8 hold them: half s of a chunk of 128, lane (quarter q, row i): bytes [32 q + 16 s, +16) of row i,
 //    the weights that the 16 bytes of codes of a lane (quarter q of a chunk) decode to.  A wave loads a fragment as 1 KiB in a row
-//    (113-120 GB/s per CU, all CUs reading the same rows; out of row-major memory 16 rows x 64 bytes at a time 35 GB/s).  Through LDS,
+//    (108-115 GB/s per CU, all CUs reading the same rows with 16 loads a wave in flight; out of row-major memory 16 rows x 64 bytes at a time 35 GB/s).  Through LDS,
 //    as k_gemm_big.hip's 512-row runs take row-major rows, whole lines arrive as fast, but what is in flight has to have its place there: 128 of the
 //    160 KiB, which leaves the decode tables without copies and every lookup in bank conflicts.
 //  * A workgroup owns up to 512 token rows and a run of up to CB blocks of 16 channels over the whole K; wave w of eight owns TB or TB - 1 blocks
@@ -22,9 +22,9 @@
 // 64 of K take 0.08 us per 16 KiB of tokens and 0.045 us per channel block, the multiplies beside them 0.005 us per block of 16 x 16 and wave.  17408 x 5120 at 512
 // rows, us: 49.5; without the token requests 40.7, without the lookups 44.9, with a quarter of the multiplies 44.3.  Four waves of twice the rows (half the fragment
 // reads, sums in accumulation registers) 50-54, eight token slices instead of four, two slices to a step, a raised wave priority, lookups
-// put together later: all within 2 %.  Before, the best of all other kernels, with the A8 quantiser (here 0.1-0.7 us slower, for the second copy of the codes):
-// 17408 x 5120 at 200 / 512 rows 57.6 / 68.2 -> 35.7 / 53.2, 7168 x 5120 at 200 / 256 / 512 rows 25.1 / 41.3 / 56.1 -> 21.5 / 23.8 / 37.2, 9728 x 2560 at 200 / 512 30.4 /
-// 37.7 -> 18.0 / 26.4.
+// put together later: all within 2 %.  Against the best of all other kernels, with the A8 quantiser in front of either (here 0.2-0.7 us slower up to 512 rows, for the second
+// copy of the codes), graphs whose weights come from memory, K-major: 17408 x 5120 at 200 / 512 rows 55.4 / 72.4 -> 34.4 / 53.8, 7168 x 5120 at 200 / 256 / 512 rows 26.1 / 41.9 /
+// 56.4 -> 23.1 / 25.9 / 40.4, 9728 x 2560 at 200 / 512 29.2 / 39.7 -> 17.6 / 27.1; with one set of weights, in cache, 0.7 to 3 us less over panels and 1 to 7 without.
 #include <hip/hip_fp16.h>
 
 #include <algorithm>

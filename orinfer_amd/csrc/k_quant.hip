@@ -115,7 +115,7 @@ __global__ __launch_bounds__(WAVES == 1 ? 256 : 64 * WAVES) void a8_held_kernel(
     int unit = WAVES == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;  // wave-uniform
     if constexpr (PANELS) {
         // Workgroups go to the 8 XCDs in turn: the 16 rows of a panel, which share its cache lines, stay on one (a line written in pieces by all
-        // of them goes to memory from each: 512 x 5120 5.7 us, 4.3 so)
+        // of them goes to memory from each: 512 x 5120 5.7 us, 4.6 so; the row-major codes alone 3.9)
         constexpr int kTogether = WAVES == 1 ? 4 : 16;  // workgroups to a panel
         const int turn = blockIdx.x >> 3;
         unit = (turn / kTogether * 8 + (blockIdx.x & 7)) * 16 + (WAVES == 1 ? turn % kTogether * 4 + (int)(threadIdx.x >> 6) : turn % kTogether);
@@ -281,8 +281,8 @@ __device__ __forceinline__ float rotate_block(float (&v)[4], int l32, __half (&o
 }
 
 // The same stages for rows whose codes are all that is kept, in 28 vector instructions per lane and four channels where rotate_block takes 52 of a kernel's
-// 150 and an LDS trip each (rotation and A8 of 8192 x 5120, bound by them: 43.4 -> 40.1 us; 20 rows with residual and norm, where the chain counts: 5.5 -> 5.2, the
-// layer around it 91.0 -> 90.1; 8192 rows of those are bound by memory, 88 us).
+// 150 and an LDS trip each (rotation and A8 of 8192 x 5120, bound by them: 43.4 -> 40.1 us; 20 rows with residual and norm, where the chain counts: 5.5 -> 5.2, which
+// the layer around it does not show beyond noise; 8192 rows of those are bound by memory, 88 us).
 //  * A stage between lanes is one instruction per value, own + (+-1) partner: exact, for a fused multiply-add with +-1 rounds as the add does. The
 //    upper lane of a pair gets own - partner, the negative of what it should hold; so does its partner of every later stage, and the
 //    signs come back with the last multiply.  (Only the sign of a zero can differ from rotate_block, which no code shows.)

@@ -19,7 +19,8 @@
 //  What bounds it: a wave issues an instruction every 4.5 cycles and an LDS read every 8, multiplies of 16 cycles run beside them, and with
 //  one wave to a SIMD (five row blocks and more, whose rings and sums leave no room for two) the loop takes what its
 //  instructions take: 7168 x 5120 codes of 200 rows, 322 -> 203 a step of 64 and 28 multiplies, 2050 -> 1400 cycles, the launch 28.9 -> 22.7 us.
-//  With eight waves it is the LDS (17408 x 5120 of 48 rows 20.4 -> 18.0 us) and below 17 rows the stream (8 rows 17.3 -> 14.1 us).
+//  With eight waves it is the LDS (17408 x 5120 of 48 rows 20.4 -> 18.0 us) and below 17 rows the stream (8 rows, by name, 17.3 -> 14.1 us in
+//  cache and 14.6 out of memory, where `auto` keeps the loader-wave kernel at 14.5).
 //  int8, 24 rows of 5120 x 17408: the stream, 4.6 TB/s.
 //  * Quarter q of a wave multiplies bytes [32 q, +32) of a chunk, 16 in each of two steps: piece c = 2 q + s of row r sits at
 //    position (q + 4 s) ^ swizzle(r).

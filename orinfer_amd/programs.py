@@ -419,9 +419,9 @@ class MoeTokenLayer:
         self.k_swiglu_a8 = Kernel("activation_quantization", K=intermediate, fused=True)
         self.k_down = Kernel("integer_e8p_gemv", E=experts, routes=top_k, N=hidden, K=intermediate, shared_input=False)
         self.k_combine = Kernel("moe_combine", H=hidden, slots=top_k, **common)
-        # Three launches instead of five where the library has the forms (up to 512 experts): gate/up selects
-        # the token's routes itself while it builds its tables (no router launch), down turns the fp16 gate|up
-        # rows into SwiGLU -> A8 codes on their way into LDS (no launch in between).
+        # Fewer than five launches where the library has the forms (up to 512 experts): gate/up selects the token's
+        # routes itself while it builds its tables (no router launch), down turns the fp16 gate|up rows into
+        # SwiGLU -> A8 codes on their way into LDS (no launch in between).  These are three; two below.
         self.fused = False
         if fused is not False:
             try:

@@ -891,16 +891,16 @@ def test_moe_token_layer_matches_the_routed_layer_of_one_token():
     # and the token-sorted program on the same token
     sorted_layer = run_layer(c, 32)
     assert torch.equal(sorted_layer.out, layer.out)
-    # three launches (gate/up selects the routes itself, down applies SwiGLU -> A8 to its input): same bits
-    three = programs.MoeTokenLayer(c["experts"], c["top_k"], c["hidden"], c["intermediate"], c["gate_up"],
+    # two launches (gate/up selects the routes itself, down applies SwiGLU -> A8 to its input and adds the routes' rows): same bits
+    two = programs.MoeTokenLayer(c["experts"], c["top_k"], c["hidden"], c["intermediate"], c["gate_up"],
                                    c["gate_up_scales"], c["down"], c["down_scales"])
-    assert three.fused
-    three.ids.fill_(-1)
-    three.run(x, logits)
+    assert two.fused and two.k_down_combine is not None
+    two.ids.fill_(-1)
+    two.run(x, logits)
     gu.sync()
     for name in ("ids", "prob", "a_s", "gate_up_out", "h_s", "down_out", "out"):
-        assert torch.equal(getattr(three, name), getattr(layer, name)), name
-    layer = three  # the graph replay below runs the three-launch program
+        assert torch.equal(getattr(two, name), getattr(layer, name)), name
+    layer = two  # the graph replay below runs the two-launch program
     # graph replay with another token
     stream = torch.cuda.Stream()
     graph = torch.cuda.CUDAGraph()
@@ -1115,6 +1115,7 @@ def test_every_form_reports_a_thread_limit_that_holds_its_own_block():
 
 @pytest.mark.parametrize("e,k,h,i", [(128, 8, 2048, 512), (512, 10, 1024, 384), (64, 64, 256, 128)])
 def test_one_token_layer_in_three_launches_gives_the_bits_of_five(e, k, h, i):
+    """Three launches above eight routes, two up to that."""
     c = workloads.config3(tokens=1, experts=e, top_k=k, hidden=h, intermediate=i)
     x, logits = gu.dev(c["x"]), gu.dev(c["logits"])
     layers = []
@@ -1124,6 +1125,7 @@ def test_one_token_layer_in_three_launches_gives_the_bits_of_five(e, k, h, i):
         layer.run(x, logits)
         gu.sync()
         layers.append(layer)
+    assert (layers[1].k_down_combine is not None) == (k <= 8)
     want_ids, want_prob = orc.router_topk(c["logits"], k, True)
     np.testing.assert_array_equal(gu.host(layers[1].ids), want_ids)
     np.testing.assert_allclose(gu.host(layers[1].prob), want_prob, atol=2e-6, rtol=2e-5)
