@@ -32,13 +32,16 @@ __device__ __forceinline__ float load_value(const __half* __restrict__ x, int64_
     return FUSED ? swiglu_value(x[row_base + col], x[row_base + k + col]) : __half2float(x[row_base + col]);
 }
 
+// (The number of waves is a constant: read from the launch, it is a scalar load behind the meeting, and from another line of the arguments where a kernel has many.
+// A8 of one row of 5120: QUANT_A.)
+template <int WAVES>
 __device__ __forceinline__ float block_max(float v, float* scratch) {
     v = wave_max_magnitude(v);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (lane == 0) scratch[wave] = v;
     __syncthreads();
-    const int waves = (blockDim.x + 63) >> 6;  // 16 at most
-    return __uint_as_float(row_max_u32(__float_as_uint(scratch[min(lane & 15, waves - 1)])));
+    static_assert(WAVES <= 16, "a row of lanes holds the maxima of all waves");
+    return __uint_as_float(row_max_u32(__float_as_uint(scratch[min(lane & 15, WAVES - 1)])));
 }
 
 // Masked rows: two passes over the group, grid (rows, groups).
@@ -55,7 +58,7 @@ __global__ __launch_bounds__(256) void a8_masked_kernel(const __half* __restrict
     auto value = [&](int col) { return mask[col] != 0 ? 0.f : load_value<FUSED>(x, in_base, k, col); };
     float amax = 0.f;
     for (int i = threadIdx.x; i < width; i += 256) amax = fmaxf(amax, fabsf(value(first + i)));
-    amax = block_max(amax, scratch);
+    amax = block_max<4>(amax, scratch);
     const __half stored = a8_scale(amax);
     if (threadIdx.x == 0) s[(int64_t)row * groups + g] = stored;
     const float scale = __half2float(stored);
@@ -166,7 +169,7 @@ __global__ __launch_bounds__(WAVES == 1 ? 256 : 64 * WAVES) void a8_held_kernel(
     if (WAVES == 1) {
         amax = wave_max_magnitude(amax);
     } else {
-        amax = block_max(amax, scratch);
+        amax = block_max<WAVES>(amax, scratch);
     }
     const __half stored = a8_scale(amax);
     if (lane == 0) s[(int64_t)row * groups + g] = stored;
@@ -332,6 +335,7 @@ __device__ __forceinline__ float rotate_for_codes(float (&v)[4], const RotationL
 }
 
 // Row scale from the largest magnitude, stored once, and the int8 codes of the fp16 row in LDS.
+template <int THREADS>
 __device__ __forceinline__ void quantise_row(const __half* rotated, float amax, int8_t* __restrict__ q,
                                              __half* __restrict__ s, int row, int k) {
     const int tid = threadIdx.x;
@@ -340,7 +344,7 @@ __device__ __forceinline__ void quantise_row(const __half* rotated, float amax, 
     if (tid == 0) s[row] = stored;
     const float scale = __half2float(stored);
     const float inverse = __frcp_rn(scale);
-    for (int i = tid; i < k / 4; i += blockDim.x) {
+    for (int i = tid; i < k / 4; i += THREADS) {
         const uint2 raw = *reinterpret_cast<const uint2*>(rotated + 4 * i);
         const __half* h = reinterpret_cast<const __half*>(&raw);
         const float values[4] = {__half2float(h[0]), __half2float(h[1]), __half2float(h[2]), __half2float(h[3])};
@@ -412,8 +416,8 @@ __global__ __launch_bounds__(THREADS) void rotate_a8_kernel(const __half* __rest
     __shared__ float scratch[THREADS / 64];
     const int row = blockIdx.x;
     float amax = rotate_row_to_lds<SWIGLU, THREADS>(x, signs, rotated, row, k);
-    amax = block_max(amax, scratch);  // includes the barrier that publishes `rotated`
-    quantise_row(rotated, amax, q, s, row, k);
+    amax = block_max<THREADS / 64>(amax, scratch);  // includes the barrier that publishes `rotated`
+    quantise_row<THREADS>(rotated, amax, q, s, row, k);
 }
 
 // rotate_expert_a8 (kernels/cuda/model/rotation_a8.py:386-422, body :452-531, entry points :558-604):
@@ -447,7 +451,7 @@ __global__ __launch_bounds__(THREADS) void rotate_expert_kernel(
         slot_map[assignment] = slot;
     }
     float amax = rotate_row_to_lds<SWIGLU, THREADS>(x, signs, rotated, row, k);
-    amax = block_max(amax, scratch);  // includes the barrier that publishes `rotated` and `slot_of`
+    amax = block_max<THREADS / 64>(amax, scratch);  // includes the barrier that publishes `rotated` and `slot_of`
     const __half stored = a8_scale(amax);
     if (tid == 0) s[row] = stored;
     if (routing != 0 && tid < top_k) ds[slot_of[tid]] = stored;
@@ -529,7 +533,7 @@ __global__ __launch_bounds__(256) void rotate_tiles_kernel(const __half* __restr
         amax = fmaxf(amax, rotate_block(v, l32, out));
         if (live) *reinterpret_cast<uint2*>(rotated + (int64_t)row * k + first) = *reinterpret_cast<const uint2*>(out);
     }
-    amax = block_max(amax, scratch);
+    amax = block_max<4>(amax, scratch);
     if (tid == 0) maxima[(int64_t)row * gridDim.y + tile] = amax;
 }
 
@@ -539,7 +543,7 @@ __global__ __launch_bounds__(256) void quantize_tiles_kernel(const __half* __res
     const int row = blockIdx.x, tile = blockIdx.y, tiles = gridDim.y, tid = threadIdx.x;
     float amax = 0.f;
     for (int j = tid; j < tiles; j += 256) amax = fmaxf(amax, maxima[(int64_t)row * tiles + j]);
-    amax = block_max(amax, scratch);
+    amax = block_max<4>(amax, scratch);
     const __half stored = a8_scale(amax);
     if (tile == 0 && tid == 0) s[row] = stored;
     const float scale = __half2float(stored), inverse = __frcp_rn(scale);
@@ -718,8 +722,8 @@ __global__ __launch_bounds__(THREADS) void residual_norm_rotate_a8_kernel(
         const uint32_t sign_word = *reinterpret_cast<const uint32_t*>(signs + first);
         second_pass(first, sum, raw_w, sign_word);
     }
-    amax = block_max(amax, scratch);  // includes the barrier that publishes `rotated`
-    quantise_row(rotated, amax, q, s, row, k);
+    amax = block_max<THREADS / 64>(amax, scratch);  // includes the barrier that publishes `rotated`
+    quantise_row<THREADS>(rotated, amax, q, s, row, k);
 }
 
 // One workgroup per token; same lane layout as the rotation above (4 consecutive channels per lane,
