@@ -33,7 +33,7 @@ __device__ __forceinline__ float load_value(const __half* __restrict__ x, int64_
 }
 
 // (The number of waves is a constant: read from the launch, it is a scalar load behind the meeting, and from another line of the arguments where a kernel has many.
-// A8 of one row of 5120: QUANT_A.)
+// A8 of one row of 2048 with the word in a second line of the arguments 2.09 us, in the first 2.03, without it 2.00.)
 template <int WAVES>
 __device__ __forceinline__ float block_max(float v, float* scratch) {
     v = wave_max_magnitude(v);

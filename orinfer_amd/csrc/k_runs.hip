@@ -534,10 +534,8 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
             const bool whole = channel + kEach <= channels;
             if (p.out_f32) {
                 float* const dst = static_cast<float*>(p.out) + at;
-                if (whole && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
-#pragma unroll
-                    for (int h = 0; h < kQuads; ++h)
-                        reinterpret_cast<float4*>(dst)[h] = make_float4(value[4 * h], value[4 * h + 1], value[4 * h + 2], value[4 * h + 3]);
+                if (whole) {
+                    __builtin_memcpy(dst, value, sizeof value);
                 } else {
 #pragma unroll
                     for (int r = 0; r < kEach; ++r)
@@ -551,15 +549,16 @@ __global__ __launch_bounds__(WAVES * 64) void runs_kernel(RunsParams p) {
                 for (int r = 0; r < kEach; ++r) h[r] = __float2half_rn(value[r]);
 #pragma unroll
                 for (int r = 0; r < 2 * kQuads; ++r) words[r] = (uint32_t)__half_as_ushort(h[2 * r]) | (uint32_t)__half_as_ushort(h[2 * r + 1]) << 16;
-                if (kQuads == 2 && whole && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
-                    *reinterpret_cast<uint4*>(dst) = make_uint4(words[0], words[1], words[2 * kQuads - 2], words[2 * kQuads - 1]);
-                } else if (whole && (reinterpret_cast<uintptr_t>(dst) & 7) == 0) {
-#pragma unroll
-                    for (int q = 0; q < kQuads; ++q) reinterpret_cast<uint2*>(dst)[q] = make_uint2(words[2 * q], words[2 * q + 1]);
+                if (whole) {  // (one store at any address: a run of 38 channels, 9728 of them, leaves its rows at multiples of 4)
+                    __builtin_memcpy(dst, words, sizeof words);
                 } else {
 #pragma unroll
-                    for (int r = 0; r < kEach; ++r)
-                        if (channel + r < channels) dst[r] = h[r];
+                    for (int r = 0; r < kEach; r += 2) {
+                        if (channel + r + 2 <= channels)
+                            __builtin_memcpy(dst + r, &words[r / 2], 4);
+                        else if (channel + r < channels)
+                            dst[r] = h[r];
+                    }
                 }
             }
         }

@@ -1651,6 +1651,27 @@ def test_channel_runs_int8_weights_short_requests(rows, n, algorithm):
     assert (gu.host(out)[rows] == 91).all() and (gu.host(out)[:, n] == 91).all()
 
 
+# Runs of 37, 38 and 19 channels: rows of a run start at every multiple of 2 or 4 bytes, and its last lane holds one to seven channels.
+@pytest.mark.parametrize("codec", ["q4", "w8"])
+@pytest.mark.parametrize("n", [9472, 9728, 4752, 9701])
+@pytest.mark.parametrize("rows,dtype,pad", [(3, torch.float16, 0), (20, torch.float16, 1), (40, torch.float16, 0), (100, torch.float16, 3), (130, torch.float16, 0), (64, torch.float32, 1)])
+def test_channel_runs_whose_rows_start_anywhere(codec, n, rows, dtype, pad):
+    k = 256
+    rng = np.random.default_rng(orc.SEED + n + rows)
+    a_q = rng.integers(-127, 128, (rows, k), dtype=np.int8)
+    a_s, ws = rng.uniform(0.005, 0.02, rows).astype(np.float16), rng.uniform(0.005, 0.02, n).astype(np.float16)
+    weight = rng.integers(0, 2**32, (n, k // 8), dtype=np.uint32) if codec == "q4" else rng.integers(-128, 128, (n, k), dtype=np.int8)
+    out = torch.full((rows + 1, n + pad), 91, dtype=dtype, device=gu.DEV)
+    variant = dict(M=rows, N=n, K=k, algorithm="runs", workspace=False, output_stride=n + pad, output_dtype="float16" if dtype == torch.float16 else "float32")
+    if codec == "q4":
+        gu.kernel("e8p_q4_projection", **variant)(A=gu.dev(a_q), AS=gu.dev(a_s), Book=gu.book(), Out=out, S=gu.dev(ws), W=gu.dev(weight))
+    else:
+        gu.kernel("int8_projection", **variant)(A=gu.dev(a_q), Output=out, TokenScale=gu.dev(a_s), Weight=gu.dev(weight), WeightScale=gu.dev(ws))
+    want = orc.project(a_q, a_s, orc.q4_integers(weight, TABLE) if codec == "q4" else weight, ws, out_dtype=np.float16 if dtype == torch.float16 else np.float32)
+    np.testing.assert_array_equal(gu.host(out)[:rows, :n], want)
+    assert (gu.host(out)[rows] == 91).all() and (gu.host(out)[:, n:] == 91).all()
+
+
 # Row counts at which `auto` hands a projection to the channel runs: handles with a Workspace and without, both codecs, either side
 # of a row tile, one and two rounds of the CUs.
 @pytest.mark.parametrize("rows,n,k", [(17, 1040, 5120), (80, 8208, 1152), (81, 8208, 1152), (129, 8208, 1152), (200, 8208, 1152), (201, 8208, 1152),
