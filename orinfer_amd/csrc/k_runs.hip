@@ -626,6 +626,7 @@ constexpr int kRunsMaxRows = 512;
 struct RunsShape {
     const RunsForm* form;
     int row_tiles, tile_rows, runs, run;
+    int grid_runs;  // a row of the grid: the runs, and workgroups without one that end at once
 };
 RunsShape runs_shape(int codec, int rows, int n) {
     RunsShape s = {};
@@ -641,10 +642,15 @@ RunsShape runs_shape(int codec, int rows, int n) {
     const int rounds = (least_runs * s.row_tiles + cus - 1) / cus;
     s.runs = std::max(least_runs, rounds * cus / s.row_tiles);
     s.run = (n + s.runs - 1) / s.runs;
-    // Whole stores of 16 bytes, where that leaves no CU without work that others wait for: a wide run takes no block of 16 more (240 rows of 7000 x
-    // 2560: 55 channels 17.4 us, 56 15.7), a narrow one leaves a sixth of the CUs idle (int8, 40 rows of 5120 x 17408: 20 channels 25.8, 24 26.7).
+    // Stores that start on 16 bytes, where that leaves no CU without work that others wait for: a wide run takes no block of 16 more (240 rows of 7000 x
+    // 2560: 55 channels 16.0 us, 56 15.5), a narrow one leaves a sixth of the CUs idle (int8, 40 rows of 5120 x 17408: 20 channels 25.8, 24 26.7).
     if (rows > 32 && s.run >= 40) s.run = (s.run + 7) / 8 * 8;
     s.runs = (n + s.run - 1) / s.run;
+    // Several row tiles: rows of the grid are a multiple of the 8 XCDs, so that the workgroups of a run, a row apart, read its weights through one L2, unless an XCD
+    // would get a round more that way.  int8 9728 x 2560 at 129 / 160 rows (122 runs) 15.0 / 15.5 -> 13.7 / 14.2 us, 7000 x 2560 at 300 22.5 -> 20.5; codes, half the bytes,
+    // 7000 x 2560 at 200 / 300 rows 15.1 / 23.1 -> 14.6 / 22.3; with a round more 19000 x 2048 at 300 rows 44.4 -> 51.7.
+    const int even_runs = (s.runs + 7) / 8 * 8, rounds_here = (s.runs * s.row_tiles + cus - 1) / cus;
+    s.grid_runs = s.row_tiles > 1 && even_runs * s.row_tiles <= rounds_here * cus ? even_runs : s.runs;
     for (int i = forms.count - 1; i >= 0; --i)
         if (16 * forms.first[i].cb >= s.run) s.form = &forms.first[i];
     return s;
@@ -667,7 +673,7 @@ int runs_rounds(int codec, int rows, int n, int* tile_rows, int* run) {
 
 void runs_geometry(int codec, int rows, int n, Geometry* g) {
     const RunsShape s = runs_shape(codec, rows, n);
-    g->grid[0] = (uint32_t)s.runs, g->grid[1] = (uint32_t)s.row_tiles, g->grid[2] = 1;
+    g->grid[0] = (uint32_t)s.grid_runs, g->grid[1] = (uint32_t)s.row_tiles, g->grid[2] = 1;
     g->block[0] = (uint32_t)s.form->waves * 64;
     g->shared = kRunsLds;
 }
@@ -700,7 +706,7 @@ int runs_launch(int codec, const int8_t* a, const void* w, const uint32_t* book,
         p.row_stride = (uint32_t)k / 2, p.chunk_stride = 64, p.half_stride = 32;
     typedef void (*Runs)(RunsParams);
     const Runs kernel = reinterpret_cast<Runs>(const_cast<void*>(s.form->kernel));
-    ORX_LAUNCH(kernel, dim3(s.runs, s.row_tiles), dim3(s.form->waves * 64), kRunsLds, stream, p);
+    ORX_LAUNCH(kernel, dim3(s.grid_runs, s.row_tiles), dim3(s.form->waves * 64), kRunsLds, stream, p);
     return hip_check(hipGetLastError(), "launch projection (channel runs)");
 }
 
