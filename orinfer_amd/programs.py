@@ -388,6 +388,20 @@ class MoeLayer:
         return self.out
 
 
+def combine_pays(routes, hidden, intermediate, cus):
+    """Whether the second projection of one token with the sum over its routes is faster than projection and sum in two launches (time of the layer, one over
+    two; 256 CUs).  Every workgroup of 8 channels makes the codes of all routes itself, in turns of 512 values, and one route's are a wave's.
+    Up to 512 values 0.78-0.97, with three workgroups to a CU 1.06-1.09 up to two routes and 0.79-0.96 above.  Up to 1024: one workgroup to a CU 0.92-0.98 up to four routes
+    and 0.92-0.96 above (up to half of the CUs 1.0-1.03); two and three to a CU 0.98-1.22 up to four routes, 0.89-0.99 above.  Beyond mostly 1.0-1.33 (0.97 at best, 8 routes of
+    4096 x 1536)."""
+    per_cu = -(-hidden // (8 * cus))
+    if intermediate <= 512:
+        return per_cu <= 2 or routes > 2
+    if intermediate <= 1024:
+        return (routes <= 4 or hidden > 4 * cus) if per_cu == 1 else routes > 4
+    return False
+
+
 class MoeTokenLayer:
     """The same expert layer for ONE token: its routes index the expert banks directly
     (kernels/cuda/model/integer_vq.py:380-444), so there is no sorting, no tile list and no dispatch copy:
@@ -434,10 +448,10 @@ class MoeTokenLayer:
             except OrxError as error:
                 if fused or error.code != ORX_ERR_BAD_VARIANT:
                     raise
-        # Two launches where the sum over the routes joins the second projection (up to eight routes, intermediate up to 2048):
-        # 13.8 -> 11.6 us for 8 of 128 experts, 2048 x 512.
+        # Two launches where the sum over the routes joins the second projection and that is faster: 13.8 -> 11.6 us for 8 of 128
+        # experts, 2048 x 512.
         self.k_down_combine = None
-        if self.fused:
+        if self.fused and combine_pays(top_k, hidden, intermediate, torch.cuda.get_device_properties(self.w2.device).multi_processor_count):
             try:
                 self.k_down_combine = Kernel("integer_e8p_gemv", N=hidden, K=intermediate, shared_input=False, input_dtype="float16",
                                              fused_swiglu=True, combine=True, **routes)

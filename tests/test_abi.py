@@ -347,6 +347,16 @@ def test_which_rows_an_int8_linear_takes_over_panels(n, k, lines):
         assert int8_panels_pay(rows, n, k, 256) == bool(taken), rows
 
 
+@pytest.mark.parametrize("hidden, intermediate, lines", [
+    (2048, 512, [(1, 1), (8, 1)]), (4096, 512, [(1, 1)]), (4104, 512, [(2, 0), (3, 1)]), (1024, 640, [(4, 1), (6, 0)]), (1152, 640, [(4, 1), (6, 1)]), (2048, 1024, [(8, 1)]),
+    (2056, 1024, [(4, 0), (5, 1)]), (2048, 1152, [(1, 0), (8, 0)]), (4096, 1536, [(2, 0)]),
+])
+def test_where_the_sum_joins_the_second_projection_of_one_token(hidden, intermediate, lines):
+    from orinfer_amd.programs import combine_pays
+    for routes, taken in lines:
+        assert combine_pays(routes, hidden, intermediate, 256) == bool(taken), routes
+
+
 @pytest.mark.parametrize("symbol", ["e8p_q4_projection", "int8_projection"])
 def test_over_panels_no_key_is_dropped(symbol):
     """The one kernel behind panels=true serves none of the keys that choose among the others, row tiles that are hints elsewhere included."""
