@@ -49,8 +49,8 @@ constexpr int kThreads = 256;
 constexpr int kTileRows = 128;
 constexpr int kSpan = 256;  // output channels of a unit (SWIGLU: 128 gate + 128 up)
 constexpr uint32_t kTokens = kPairedTableBytes;
-constexpr uint32_t kSlot = kTileRows * 128;
-constexpr uint32_t kTokenScale = kTokens + 2 * kSlot;
+constexpr uint32_t kTokenBytes = 2 * kTileRows * 128;  // two chunks of 128 rows, four of 64
+constexpr uint32_t kTokenScale = kTokens + kTokenBytes;
 constexpr uint32_t kChannelScale = kTokenScale + kTileRows * 4;
 constexpr uint32_t kLds = kChannelScale + kSpan * 4;
 
@@ -72,6 +72,13 @@ struct BulkParams {
     const int4* tile_units;  // or null
     int n, k, tile_capacity, spans;
 };
+
+// until at most COUNT requests of this wave are on their way
+template <int COUNT>
+__device__ __forceinline__ void wait_requests() {
+    static_assert(COUNT < 64, "the counter has six bits");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(COUNT) : "memory");
+}
 
 template <bool GATHER, bool SWIGLU>
 __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p) {
@@ -116,55 +123,71 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
     auto run = [&](auto blocks_tag) {
         constexpr int NB = decltype(blocks_tag)::value;  // 16-row blocks
         constexpr int LOADS = NB / 2;                    // 16 NB rows are 2 NB requests of 8 rows, over four waves
-        constexpr int PHASES = NB >= 4 ? 4 : 2;          // a step of 64 in phases of RB row blocks,
+        constexpr int PHASES = NB >= 4 ? 4 : 1;          // a step of 64 in phases of RB row blocks,
         constexpr int RB = NB / PHASES, LB = 4 / PHASES; // each looking up LB of the next step's four weight blocks
+        constexpr int DEPTH = NB == 8 ? 2 : 4;           // chunks in LDS and in code registers
+        static_assert(DEPTH * NB * 16 * 128 <= kTokenBytes, "the chunks fit");
+        constexpr uint32_t SLOT = NB * 16 * 128;
+        constexpr int kChunkRequests = 4 + LOADS;
         // ---- token rows: request b of this wave brings rows 8 (LOADS wave + b) .. +7 of a chunk, 128 bytes each.  The
         // quarter q of a wave multiplies K bytes [32 q, +32) of a chunk in two steps of 16, so piece c = 2 q + s of row r sits
         // at position (q + 4 s) ^ swizzle(r): a fragment read touches four neighbouring positions of 16 rows ----
+        uint32_t slot_of[LOADS + 1];  // of this lane's row of each request, and of row `tid` for its scale; GATHER: then of their tokens
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) slot_of[i] = (uint32_t)(row0 + min((wave * LOADS + i) * 8 + (lane >> 3), rows - 1));
+        slot_of[LOADS] = (uint32_t)(row0 + min(tid, rows - 1));
+        if constexpr (GATHER) {
+            const int* const tokens_of = uniform_pointer(p.slot_token);
+            Each<LOADS + 1>::run([&](auto i) { load_4(slot_of[i], slot_of[i] * 4, tokens_of); });
+        }
+        // DEPTH register sets of codes, chunk c in set c % DEPTH: four blocks of 16 channels, 8 bytes to a lane
+        v2u codes[DEPTH][4];
+        Each<DEPTH>::run([&](auto set) { Each<4>::run([&](auto j) { anything(codes[set][j]); }); });  // (anything, but in a register)
+        // Chunks that do not exist are requested by no lane where waits behind them count requests, else not at all.
+        std::true_type counted;
+        std::bool_constant<(DEPTH > 2)> counted_in_loop;
+        auto issue_codes = [&](int chunk, auto set_tag, auto counted_tag) {
+            load_8_of_four<decltype(counted_tag)::value>(codes[decltype(set_tag)::value], code_offset, code_offset_up, codes_base + (uint64_t)chunk * chunk_stride, chunk, chunks);
+        };
+        std::integral_constant<int, 0> zero;
+        std::integral_constant<int, 1> one;
+        issue_codes(0, zero, counted);  // two chunks' are on their way while the rows' tokens are looked up
+        issue_codes(1, one, counted);
+        if constexpr (GATHER) {
+            wait_requests<8>();
+            Each<LOADS + 1>::run([&](auto i) { keep(slot_of[i]); });
+        }
         uint32_t row_offset[LOADS];
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) {
-            const int row = (wave * LOADS + i) * 8 + (lane >> 3);
-            const int slot = row0 + min(row, rows - 1);
-            const int position = (lane & 7) ^ swizzle(row);
+            const int position = (lane & 7) ^ swizzle((wave * LOADS + i) * 8 + (lane >> 3));
             const int piece = ((position & 3) << 1) | (position >> 2);
-            row_offset[i] = (uint32_t)(GATHER ? p.slot_token[slot] : slot) * (uint32_t)p.k + (uint32_t)piece * 16 + 4096u - (uint32_t)i * 1024u;
+            row_offset[i] = slot_of[i] * (uint32_t)p.k + (uint32_t)piece * 16 + 4096u - (uint32_t)i * 1024u;
         }
+        const uint32_t token_slots = lds_address_of(lds) + kTokens + (uint32_t)wave * (LOADS * 1024);
+        auto issue_tokens = [&](int chunk, int slot, auto counted_tag) {  // (the instruction's offset counts in memory too and is taken off the lane's)
+            const int8_t* const base = a_base + (int64_t)chunk * 128 - 4096;
+            request_rows_16<LOADS, decltype(counted_tag)::value>(row_offset, base, token_slots + (uint32_t)slot * SLOT, chunk, chunks);
+        };
         // scales of the tile's rows and of this wave's channels (channel `lane`, in the order of its four blocks), waited for by hand like all that follows
-        uint32_t token_scale_bits = 0, channel_scale_bits;
+        uint32_t token_scale_bits, channel_scale_bits;
         {
-            const int slot = row0 + min(tid, rows - 1);
-            const uint64_t of_row = reinterpret_cast<uint64_t>(p.as + (GATHER ? p.slot_token[slot] : slot));
+            const uint64_t of_row = reinterpret_cast<uint64_t>(p.as + slot_of[LOADS]);
             const int channel = SWIGLU && lane >= 32 ? inner + n0 + lane - 32 : n0 + lane;
             const uint64_t of_channel = reinterpret_cast<uint64_t>(p.ws + (int64_t)expert * p.n + channel);
             asm volatile("global_load_ushort %0, %1, off" : "=v"(token_scale_bits) : "v"(of_row) : "memory");
             asm volatile("global_load_ushort %0, %1, off" : "=v"(channel_scale_bits) : "v"(of_channel) : "memory");
         }
-        const uint32_t token_slots = lds_address_of(lds) + kTokens + (uint32_t)wave * (LOADS * 1024);
-        auto issue_tokens = [&](int chunk, int slot) {  // (the instruction's offset counts in memory too and is taken off the lane's)
-            const int8_t* const base = a_base + (int64_t)min(chunk, chunks - 1) * 128 - 4096;
-            request_rows_16(row_offset, base, token_slots + (uint32_t)slot * kSlot);
-        };
-        // two register sets of codes, by the parity of the chunk: four blocks of 16 channels, 8 bytes to a lane
-        v2u codes[2][4];
-        auto issue_codes = [&](int chunk, auto set_tag) {
-            constexpr int SET = decltype(set_tag)::value;
-            const uint8_t* base = codes_base + (uint64_t)min(chunk, chunks - 1) * chunk_stride;
-            load_8<0>(codes[SET][0], code_offset, base);
-            load_8<512>(codes[SET][1], code_offset, base);
-            load_8<0>(codes[SET][2], code_offset_up, base);
-            load_8<512>(codes[SET][3], code_offset_up, base);
-        };
-        std::integral_constant<int, 0> zero;
-        std::integral_constant<int, 1> one;
-        issue_codes(0, zero);
-        issue_tokens(0, 0);
-        issue_codes(1, one);
-        issue_tokens(1, 1);
+        issue_tokens(0, 0, counted);
+        issue_tokens(1, 1, counted);
+        Each<DEPTH - 2>::run([&](auto i) {
+            constexpr int CHUNK = decltype(i)::value + 2;
+            issue_codes(CHUNK, std::integral_constant<int, CHUNK>{}, counted), issue_tokens(CHUNK, CHUNK, counted);
+        });
 
         // ---- tables, scales (beside the first loads) ----
-        constexpr int kChunkRequests = 4 + LOADS;
-        asm volatile("s_waitcnt vmcnt(%3)" : "+v"(selector), "+v"(token_scale_bits), "+v"(channel_scale_bits) : "n"(2 * kChunkRequests));
+        wait_requests<2 * LOADS + (DEPTH - 2) * kChunkRequests>();
+        asm volatile("" : "+v"(selector), "+v"(token_scale_bits), "+v"(channel_scale_bits));
         write_paired_entry(lds, tid, false, byte_basis_signed(selector));
         write_paired_entry(lds, tid, true, byte_mask_signed((uint32_t)tid));
         if (tid < kTileRows) reinterpret_cast<float*>(lds + kTokenScale)[tid] = __half2float(__ushort_as_half((unsigned short)token_scale_bits));
@@ -182,10 +205,10 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
         const uint32_t frag = lds_base + kTokens + (uint32_t)(lane & 15) * 128 + (uint32_t)(((lane >> 4) ^ swizzle(lane & 15)) * 16);
         const uint32_t frag_half = frag ^ 64u;  // of a chunk's second step
         v4i token[2][RB];  // fragments of even and odd phases
-        auto read_tokens = [&](auto phase_tag, auto slot_tag, uint32_t address) {
-            constexpr int PHASE = decltype(phase_tag)::value, OFFSET = decltype(slot_tag)::value * (int)kSlot + PHASE * RB * 2048;
-            lds_read_16<OFFSET>(token[PHASE & 1][0], address);
-            if constexpr (RB > 1) lds_read_16<OFFSET + 2048>(token[PHASE & 1][1], address);
+        auto read_tokens = [&](auto phase_tag, auto set_tag, auto slot_tag, uint32_t address) {
+            constexpr int SET = decltype(set_tag)::value, OFFSET = decltype(slot_tag)::value * (int)SLOT + decltype(phase_tag)::value * RB * 2048;
+            lds_read_16<OFFSET>(token[SET][0], address);
+            if constexpr (RB > 1) lds_read_16<OFFSET + 2048>(token[SET][1], address);
         };
         v2u looked[LB][2][2];
         auto lookup = [&](int at, uint32_t word) {  // both entries of two codes
@@ -209,17 +232,18 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
         // the fragments of the phase after it and LB blocks of the next step's codes; all of these have come when it ends.
         auto phase = [&](auto step_tag, auto phase_tag, auto next_slot, uint32_t next_fragments, const v2u(&next_codes)[4], auto requests) {
             constexpr int STEP = decltype(step_tag)::value, PHASE = decltype(phase_tag)::value;
-            constexpr int NEXT = (PHASE + 1) % PHASES;
+            constexpr int NEXT = (PHASE + 1) % PHASES, TOKENS = (STEP * PHASES + PHASE) & 1;
 #pragma unroll
             for (int i = 0; i < RB; ++i)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const int jj = (i & 1) ? 3 - j : j;
                     v4i& sum = acc[PHASE * RB + i][jj];
-                    sum = __builtin_amdgcn_mfma_i32_16x16x64_i8(weight[STEP][jj], token[PHASE & 1][i], sum, 0, 0, 0);
+                    sum = __builtin_amdgcn_mfma_i32_16x16x64_i8(weight[STEP][jj], token[TOKENS][i], sum, 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
-                    if (i == 0 && j == 0) read_tokens(std::integral_constant<int, NEXT>{}, next_slot, next_fragments);
+                    if (i == 0 && j == 0) read_tokens(std::integral_constant<int, NEXT>{}, std::integral_constant<int, 1 - TOKENS>{}, next_slot, next_fragments);
                     if (i == 0 && j >= 1 && j - 1 < LB) lookup(j - 1, next_codes[PHASE * LB + j - 1][1 - STEP]);
+                    if (LB == 4 && i == 1 && j == 0) lookup(3, next_codes[3][1 - STEP]);
                     if (i == 0 && j == 3) requests();
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -233,12 +257,9 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
         std::integral_constant<int, 3> three;
 
         // ---- prologue: chunk 0 in LDS, the weights of its first step decoded, its first fragments read ----
-        asm volatile("s_waitcnt vmcnt(%4) lgkmcnt(0)\n\ts_barrier"
-                     : "+v"(codes[0][0]), "+v"(codes[0][1]), "+v"(codes[0][2]), "+v"(codes[0][3])
-                     : "n"(kChunkRequests)
-                     : "memory");
-        read_tokens(zero, zero, frag);
-        read_tokens(one, zero, frag);
+        wait_requests<LOADS + (DEPTH - 2) * kChunkRequests>();
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : "+v"(codes[0][0]), "+v"(codes[0][1]), "+v"(codes[0][2]), "+v"(codes[0][3])::"memory");
+        read_tokens(zero, zero, zero, frag);
 #pragma unroll
         for (int j = 0; j < 4; j += 2) {  // two blocks of channels at a time
             v2u pair[2][2][2];
@@ -254,59 +275,50 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
         }
 
         // One chunk: two steps of 64.  In front of its last phase the workgroup meets once: chunk t + 1 has landed,
-        // everybody has read chunk t, and the requests of chunk t + 2 go out into its slot and its code registers.
+        // everybody has read chunk t, and the requests of chunk t + DEPTH go out into its slot and its code registers.
         auto chunk_step = [&](int t, auto set_tag) {
-            constexpr int SET = decltype(set_tag)::value;
-            std::integral_constant<int, 1 - SET> other;
+            constexpr int SET = decltype(set_tag)::value, NEXT_SET = (SET + 1) % DEPTH;
+            std::integral_constant<int, NEXT_SET> other;
             auto meet = [&]() {
-                asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+                wait_requests<(DEPTH - 2) * kChunkRequests>();
+                asm volatile("s_barrier" ::: "memory");
                 __builtin_amdgcn_sched_barrier(0);
             };
-            auto request = [&]() { issue_codes(t + 2, set_tag), issue_tokens(t + 2, SET); };
+            auto request = [&]() {
+                issue_codes(t + DEPTH, set_tag, counted_in_loop), issue_tokens(t + DEPTH, SET, counted_in_loop);
+            };
             if constexpr (PHASES == 4) {
                 phase(zero, zero, set_tag, frag, codes[SET], nothing);
                 phase(zero, one, set_tag, frag, codes[SET], nothing);
                 phase(zero, two, set_tag, frag, codes[SET], nothing);
                 phase(zero, three, set_tag, frag_half, codes[SET], nothing);
             } else {
-                phase(zero, zero, set_tag, frag, codes[SET], nothing);
-                phase(zero, one, set_tag, frag_half, codes[SET], nothing);
+                phase(zero, zero, set_tag, frag_half, codes[SET], nothing);
             }
-            // the codes of chunk t + 1 are older than its token rows
-            asm volatile("s_waitcnt vmcnt(%4)"
-                         : "+v"(codes[1 - SET][0]), "+v"(codes[1 - SET][1]), "+v"(codes[1 - SET][2]), "+v"(codes[1 - SET][3])
-                         : "n"(LOADS));
+            wait_requests<(DEPTH - 2) * kChunkRequests + LOADS>();  // the codes of chunk t + 1 are older than its token rows
+            asm volatile("" : "+v"(codes[NEXT_SET][0]), "+v"(codes[NEXT_SET][1]), "+v"(codes[NEXT_SET][2]), "+v"(codes[NEXT_SET][3]));
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (PHASES == 4) {
-                phase(one, zero, set_tag, frag_half, codes[1 - SET], nothing);
-                phase(one, one, set_tag, frag_half, codes[1 - SET], nothing);
-                phase(one, two, set_tag, frag_half, codes[1 - SET], nothing);
+                phase(one, zero, set_tag, frag_half, codes[NEXT_SET], nothing);
+                phase(one, one, set_tag, frag_half, codes[NEXT_SET], nothing);
+                phase(one, two, set_tag, frag_half, codes[NEXT_SET], nothing);
                 meet();
-                phase(one, three, other, frag, codes[1 - SET], request);
+                phase(one, three, other, frag, codes[NEXT_SET], request);
             } else {
-                phase(one, zero, set_tag, frag_half, codes[1 - SET], nothing);
                 meet();
-                phase(one, one, other, frag, codes[1 - SET], request);
+                phase(one, zero, other, frag, codes[NEXT_SET], request);
             }
         };
-        int t = 0;
-        for (; t + 1 < chunks; t += 2) {
-            chunk_step(t, zero);
-            chunk_step(t + 1, one);
-        }
-        if (t < chunks) chunk_step(t, zero);
-        // requests of chunks that do not exist (clamped): their registers stay named until they have landed
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)"
-                     : "+v"(codes[0][0]), "+v"(codes[0][1]), "+v"(codes[0][2]), "+v"(codes[0][3]), "+v"(codes[1][0]), "+v"(codes[1][1]),
-                       "+v"(codes[1][2]), "+v"(codes[1][3])
-                     :
-                     : "memory");
+        for (int t = 0; t < chunks; t += DEPTH)
+            Each<DEPTH>::run([&](auto set) {
+                if (t + decltype(set)::value < chunks) chunk_step(t + decltype(set)::value, set);
+            });
 
         // ---- epilogue: a lane holds four consecutive channels of one slot in every block.  Stored from there, every instruction touches 16
         // rows in an order that leaves each lane an access of its own, more than a hundred cycles apiece (128 slots of 64
         // channels to a wave: 11300 cycles beside 9800 of the whole K loop at K = 512).  So a block of 16 rows goes through LDS, where
         // the token rows were and private to the wave, and leaves with neighbouring lanes beside each other in a row ----
-        asm volatile("s_barrier" ::: "memory");  // nobody's token rows are on their way any more
+        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");  // nobody's token rows are on their way any more
         if (!live_wave) return;
         int own = threadIdx.x & 63;
         asm volatile("" : "+v"(own));  // nothing of the addresses below is carried through the K loop

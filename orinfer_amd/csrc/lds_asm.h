@@ -45,21 +45,43 @@ __device__ __forceinline__ void request_16(uint32_t lane_offset, const void* uni
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3" ::"v"(lane_offset), "s"(uniform_base), "s"(lds_wave_base), "n"(OFFSET)
                  : "memory", "m0");
 }
-// COUNT (1, 2 or 4) requests of 1 KiB, one behind the other in LDS.
-template <int COUNT>
-__device__ __forceinline__ void request_rows_16(const uint32_t (&lane_offset)[COUNT], const void* uniform_base, uint32_t lds_wave_base) {
+// COUNT (1, 2 or 4) requests of 1 KiB, one behind the other in LDS, if index < count.  Else none, by a branch inside the statement; COUNTED: requests by no
+// lane, which bring nothing and count all the same, where requests that follow are waited for by number.
+#define ORX_BELOW_OR_SKIPPED(INDEX, COUNT, BODY) "s_cmp_lt_i32 " INDEX ", " COUNT "\n\ts_cbranch_scc0 .Lskipped%=\n\t" BODY ".Lskipped%=:"
+#define ORX_BELOW_OR_EMPTY(INDEX, COUNT, ALL, BODY) \
+    "s_mov_b64 " ALL ", exec\n\ts_cmp_lt_i32 " INDEX ", " COUNT "\n\ts_cselect_b64 exec, exec, 0\n\t" BODY "s_mov_b64 exec, " ALL
+template <int COUNT, bool COUNTED>
+__device__ __forceinline__ void request_rows_16(const uint32_t (&lane_offset)[COUNT], const void* uniform_base, uint32_t lds_wave_base, int index, int count) {
     static_assert(COUNT == 1 || COUNT == 2 || COUNT == 4, "one, two or four requests to a statement");
+    uint64_t all;
+#define ORX_REQUEST_4 \
+    "s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %5, %1\n\tglobal_load_lds_dwordx4 %6, %1 offset:1024\n\t" \
+    "global_load_lds_dwordx4 %7, %1 offset:2048\n\tglobal_load_lds_dwordx4 %8, %1 offset:3072\n\t"
+#define ORX_REQUEST_2 "s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %5, %1\n\tglobal_load_lds_dwordx4 %6, %1 offset:1024\n\t"
+#define ORX_REQUEST_1 "s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %5, %1\n\t"
+#define ORX_REQUEST(TEXT, ...)                                                                                              \
+    do {                                                                                                                    \
+        if constexpr (COUNTED)                                                                                              \
+            asm volatile(ORX_BELOW_OR_EMPTY("%3", "%4", "%0", TEXT)                                                         \
+                         : "=&s"(all)                                                                                       \
+                         : "s"(uniform_base), "s"(lds_wave_base), "s"(index), "s"(count), __VA_ARGS__                       \
+                         : "memory", "m0", "scc");                                                                          \
+        else                                                                                                                \
+            asm volatile(ORX_BELOW_OR_SKIPPED("%3", "%4", TEXT)                                                             \
+                         : "=&s"(all)                                                                                       \
+                         : "s"(uniform_base), "s"(lds_wave_base), "s"(index), "s"(count), __VA_ARGS__                       \
+                         : "memory", "m0", "scc");                                                                          \
+    } while (0)
     if constexpr (COUNT == 1)
-        request_16<0>(lane_offset[0], uniform_base, lds_wave_base);
+        ORX_REQUEST(ORX_REQUEST_1, "v"(lane_offset[0]));
     else if constexpr (COUNT == 2)
-        asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2\n\tglobal_load_lds_dwordx4 %1, %2 offset:1024" ::"v"(lane_offset[0]), "v"(lane_offset[1]),
-                     "s"(uniform_base), "s"(lds_wave_base)
-                     : "memory", "m0");
+        ORX_REQUEST(ORX_REQUEST_2, "v"(lane_offset[0]), "v"(lane_offset[1]));
     else
-        asm volatile("s_mov_b32 m0, %5\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %4\n\tglobal_load_lds_dwordx4 %1, %4 offset:1024\n\t"
-                     "global_load_lds_dwordx4 %2, %4 offset:2048\n\tglobal_load_lds_dwordx4 %3, %4 offset:3072" ::"v"(lane_offset[0]), "v"(lane_offset[1]), "v"(lane_offset[2]),
-                     "v"(lane_offset[3]), "s"(uniform_base), "s"(lds_wave_base)
-                     : "memory", "m0");
+        ORX_REQUEST(ORX_REQUEST_4, "v"(lane_offset[0]), "v"(lane_offset[1]), "v"(lane_offset[2]), "v"(lane_offset[3]));
+#undef ORX_REQUEST
+#undef ORX_REQUEST_1
+#undef ORX_REQUEST_2
+#undef ORX_REQUEST_4
 }
 #pragma clang diagnostic pop
 // A request OFFSET behind the last request_16, by the m0 that this one left: for a kernel whose only writes of m0 are request_16's, so for none with a
@@ -86,11 +108,38 @@ __device__ __forceinline__ void load_8(v2u& value, uint32_t lane_offset, const v
                  : "v"(lane_offset), "s"(uniform_base), "n"(OFFSET)
                  : "memory");
 }
+// Four times 8 bytes, at both lane offsets and 512 behind them, where index < count as above; else the registers keep what they have.
+template <bool COUNTED>
+__device__ __forceinline__ void load_8_of_four(v2u (&value)[4], uint32_t lane_offset, uint32_t other_offset, const void* uniform_base, int index, int count) {
+    uint64_t all;
+#define ORX_LOADS                                                                                                      \
+    "global_load_dwordx2 %0, %5, %7\n\tglobal_load_dwordx2 %1, %5, %7 offset:512\n\tglobal_load_dwordx2 %2, %6, %7\n\t" \
+    "global_load_dwordx2 %3, %6, %7 offset:512\n\t"
+    if constexpr (COUNTED)
+        asm volatile(ORX_BELOW_OR_EMPTY("%8", "%9", "%4", ORX_LOADS)
+                     : "+v"(value[0]), "+v"(value[1]), "+v"(value[2]), "+v"(value[3]), "=&s"(all)
+                     : "v"(lane_offset), "v"(other_offset), "s"(uniform_base), "s"(index), "s"(count)
+                     : "memory", "scc");
+    else
+        asm volatile(ORX_BELOW_OR_SKIPPED("%8", "%9", ORX_LOADS)
+                     : "+v"(value[0]), "+v"(value[1]), "+v"(value[2]), "+v"(value[3]), "=&s"(all)
+                     : "v"(lane_offset), "v"(other_offset), "s"(uniform_base), "s"(index), "s"(count)
+                     : "memory", "scc");
+#undef ORX_LOADS
+}
+#undef ORX_BELOW_OR_EMPTY
+#undef ORX_BELOW_OR_SKIPPED
+__device__ __forceinline__ void load_4(uint32_t& value, uint32_t lane_offset, const void* uniform_base) {
+    asm volatile("global_load_dword %0, %1, %2" : "=v"(value) : "v"(lane_offset), "s"(uniform_base) : "memory");
+}
 __device__ __forceinline__ void load_16(v4u& value, uint32_t lane_offset, const void* uniform_base) {
     asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(value) : "v"(lane_offset), "s"(uniform_base) : "memory");
 }
 template <typename T>
 __device__ __forceinline__ void keep(T& value) { asm volatile("" : "+v"(value)); }
+// a register of its own, whatever it holds
+template <typename T>
+__device__ __forceinline__ void anything(T& value) { asm volatile("" : "=v"(value)); }
 // In and out in one register: left to itself the compiler moves sums about between unrolled steps, a tenth of a loop's
 // instructions.  What it would have inserted is on the caller: two instructions between the last write of an operand and the multiply,
 // and a pause (s_nop 15) in front of the first reading of a sum.
