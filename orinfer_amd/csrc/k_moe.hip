@@ -460,6 +460,20 @@ __global__ __launch_bounds__(kMetaThreads) void route_metadata_kernel(
 // (Whole tiles in front of the rests, so that a projection ends on short units, made it 4 % slower: a CU runs a long and a
 // short unit together better than two of a kind.)
 constexpr int kSegment = kMetaThreads;
+// Among the lanes of a wave that hold the same expert, found one id bit at a time: how many are in front, how many there are.
+struct LaneRank {
+    int rank, group;
+};
+__device__ __forceinline__ LaneRank rank_among_lanes(int id, bool valid, int lane, int experts) {
+    const int id_bits = 32 - __builtin_clz(max(experts - 1, 1));
+    unsigned long long same = __ballot(valid);
+    for (int bit = 0; bit < id_bits; ++bit) {
+        const bool set = (id >> bit) & 1;
+        const unsigned long long with = __ballot(valid && set);
+        same &= set ? with : ~with;
+    }
+    return {(int)__popcll(same & ((1ull << lane) - 1ull)), (int)__popcll(same)};
+}
 __global__ __launch_bounds__(kMetaThreads) void segment_rank_kernel(const int* __restrict__ ids, int* __restrict__ relative,
                                                                     int* __restrict__ segments, int assignments, int experts) {
     extern __shared__ int counters[];  // [kMetaWaves][experts]
@@ -469,17 +483,9 @@ __global__ __launch_bounds__(kMetaThreads) void segment_rank_kernel(const int* _
     const bool valid = at < assignments;
     const int id = valid ? ids[at] : 0;
     for (int i = tid; i < kMetaWaves * experts; i += kMetaThreads) counters[i] = 0;
-    // the lanes of this wave that hold the same expert, found one id bit at a time
-    const int id_bits = 32 - __builtin_clz(max(experts - 1, 1));
-    unsigned long long same = __ballot(valid);
-    for (int bit = 0; bit < id_bits; ++bit) {
-        const bool set = (id >> bit) & 1;
-        const unsigned long long with = __ballot(valid && set);
-        same &= set ? with : ~with;
-    }
-    const int rank = __popcll(same & ((1ull << lane) - 1ull)), group = __popcll(same);
+    const LaneRank same = rank_among_lanes(id, valid, lane, experts);
     __syncthreads();
-    if (valid && rank == group - 1) counters[wave * experts + id] = group;
+    if (valid && same.rank == same.group - 1) counters[wave * experts + id] = same.group;
     __syncthreads();
     if (tid < experts) {  // exclusive prefix over the waves, total of the segment
         int count[kMetaWaves], before = 0;
@@ -490,21 +496,68 @@ __global__ __launch_bounds__(kMetaThreads) void segment_rank_kernel(const int* _
         segments[(int64_t)blockIdx.x * experts + tid] = before;
     }
     __syncthreads();
-    if (valid) relative[at] = counters[wave * experts + id] + rank;
+    if (valid) relative[at] = counters[wave * experts + id] + same.rank;
 }
 
-__global__ __launch_bounds__(kMetaThreads) void segment_place_kernel(
-    const int* __restrict__ ids, const int* __restrict__ segments, int* __restrict__ counts, int* __restrict__ relative,
-    int* __restrict__ row_offsets, int* __restrict__ tile_count, int* __restrict__ tile_expert, int* __restrict__ tile_offsets,
-    int* __restrict__ tile_row, int4* __restrict__ tile_units, int* __restrict__ slot_map, int* __restrict__ slot_token,
-    int* __restrict__ row_max, int assignments, int experts, int top_k, int block_m) {
-    __shared__ int in_front[kMetaThreads], first_row[kMetaThreads], wave_rows[kMetaWaves], wave_tiles[kMetaWaves];
-    __shared__ int wave_large[kMetaWaves], wave_small[kMetaWaves];
+struct SegmentOutputs {
+    int *counts, *row_offsets, *tile_count, *tile_expert, *tile_offsets, *tile_row;
+    int4* tile_units;  // or null
+    int *relative, *slot_map, *slot_token;
+    int* row_max;  // or null
+};
+struct PlaceLds {
+    int in_front[kMetaThreads], first_row[kMetaThreads];  // per expert: assignments of the segments in front, first slot
+    int wave_rows[kMetaWaves], wave_tiles[kMetaWaves], wave_large[kMetaWaves], wave_small[kMetaWaves];
+};
+// Thread `tid` has the number of assignments of expert `tid`, and of those in the segments in front: offsets, this workgroup's share of the tile lists, and
+// in `lds` what an assignment needs for its slot.  Whole workgroups; ends in a barrier.
+__device__ __forceinline__ void place_experts(PlaceLds& lds, const SegmentOutputs& out, int count, int before, int experts, int block_m) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int segment = blockIdx.x, total_segments = gridDim.x;
+    if (tid < experts) lds.in_front[tid] = before;
+    const int tiles = (count + block_m - 1) / block_m;
+    // Units: the tiles in the order of their size, so that what starts last is short: above half a tile's rows, above a quarter, the rest
+    // (an expert's last tile is the only one that is not full; tiles of the two small sizes are counted in the halves of a word)
+    const int full = count / block_m, rest = count % block_m;
+    const int size = 2 * rest > block_m ? 0 : 4 * rest > block_m ? 1 : 2;  // of the last tile
+    const int large = full + (rest > 0 && size == 0), small = rest > 0 && size > 0 ? 1 << (16 * (size - 1)) : 0;
+    const int row_scan = wave_prefix_sum(count), tile_scan = wave_prefix_sum(tiles), large_scan = wave_prefix_sum(large), small_scan = wave_prefix_sum(small);
+    if (lane == 63) lds.wave_rows[wave] = row_scan, lds.wave_tiles[wave] = tile_scan, lds.wave_large[wave] = large_scan, lds.wave_small[wave] = small_scan;
+    __syncthreads();
+    int row_base = 0, tile_base = 0, tile_total = 0, large_base = 0, large_total = 0, small_base = 0, small_total = 0;
+    for (int w = 0; w < kMetaWaves; ++w) {
+        if (w < wave) row_base += lds.wave_rows[w], tile_base += lds.wave_tiles[w], large_base += lds.wave_large[w], small_base += lds.wave_small[w];
+        tile_total += lds.wave_tiles[w], large_total += lds.wave_large[w], small_total += lds.wave_small[w];
+    }
+    if (tid < experts) {
+        const int row = row_base + row_scan - count, tile = tile_base + tile_scan - tiles;
+        lds.first_row[tid] = row;
+        if (segment == 0) out.counts[tid] = count, out.row_offsets[tid] = row, out.tile_offsets[tid] = tile;
+        const int first_large = large_base + large_scan - large, smalls = small_base + small_scan - small;
+        const int at_rest = size == 0 ? first_large + full : large_total + (size == 1 ? smalls & 0xFFFF : (small_total & 0xFFFF) + (smalls >> 16));
+        for (int t = segment; t < tiles; t += total_segments) {
+            out.tile_expert[tile + t] = tid, out.tile_row[tile + t] = t * block_m;
+            if (out.tile_units != nullptr) out.tile_units[t < full ? first_large + t : at_rest] = make_int4(tid, row + t * block_m, t < full ? block_m : rest, 0);
+        }
+    }
+    if (segment == 0 && tid == 0) out.tile_count[0] = tile_total;
+    __syncthreads();
+}
+// Assignment `at` of expert `id`, the `local`-th of its expert in its segment.
+__device__ __forceinline__ void place_assignment(const PlaceLds& lds, const SegmentOutputs& out, int at, int id, int local, int top_k) {
+    const int in_expert = lds.in_front[id] + local, slot = lds.first_row[id] + in_expert;
+    out.relative[at] = in_expert;
+    out.slot_map[at] = slot;
+    out.slot_token[slot] = at / top_k;
+    if (out.row_max != nullptr) out.row_max[at] = 0;
+}
+__global__ __launch_bounds__(kMetaThreads) void segment_place_kernel(const int* __restrict__ ids, const int* __restrict__ segments, SegmentOutputs out,
+                                                                     int assignments, int experts, int top_k, int block_m) {
+    __shared__ PlaceLds lds;
+    const int tid = threadIdx.x, segment = blockIdx.x, total_segments = gridDim.x;
     const int at = segment * kSegment + tid;
     const bool valid = at < assignments;
-    const int id = valid ? ids[at] : 0, local = valid ? relative[at] : 0;
+    const int id = valid ? ids[at] : 0, local = valid ? out.relative[at] : 0;
     int count = 0, before = 0;
     if (tid < experts) {
 #pragma unroll 8
@@ -513,42 +566,51 @@ __global__ __launch_bounds__(kMetaThreads) void segment_place_kernel(
             before += s < segment ? c : 0;
             count += c;
         }
-        in_front[tid] = before;
     }
-    const int tiles = (count + block_m - 1) / block_m;
-    // Units: the tiles in the order of their size, so that what starts last is short: above half a tile's rows, above a quarter, the rest
-    // (an expert's last tile is the only one that is not full; tiles of the two small sizes are counted in the halves of a word)
-    const int full = count / block_m, rest = count % block_m;
-    const int size = 2 * rest > block_m ? 0 : 4 * rest > block_m ? 1 : 2;  // of the last tile
-    const int large = full + (rest > 0 && size == 0), small = rest > 0 && size > 0 ? 1 << (16 * (size - 1)) : 0;
-    const int row_scan = wave_prefix_sum(count), tile_scan = wave_prefix_sum(tiles), large_scan = wave_prefix_sum(large), small_scan = wave_prefix_sum(small);
-    if (lane == 63) wave_rows[wave] = row_scan, wave_tiles[wave] = tile_scan, wave_large[wave] = large_scan, wave_small[wave] = small_scan;
+    place_experts(lds, out, count, before, experts, block_m);
+    if (valid) place_assignment(lds, out, at, id, local, top_k);
+}
+
+// Up to 16 segments in one launch: every workgroup reads the whole list and counts the other segments' assignments with LDS additions, which need no
+// order; only its own are ranked.
+constexpr int kOneLaunchSegments = 16;
+__global__ __launch_bounds__(kMetaThreads) void segment_metadata_kernel(const int* __restrict__ ids, SegmentOutputs out, int assignments, int experts,
+                                                                        int top_k, int block_m) {
+    extern __shared__ int counters[];  // [kMetaWaves][experts], then assignments in front of this segment and behind it, [experts] each
+    __shared__ PlaceLds lds;
+    int *const in_front = counters + kMetaWaves * experts, *const behind = in_front + experts;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int segment = blockIdx.x, at = segment * kSegment + tid;
+    const bool valid = at < assignments;
+    int others[kOneLaunchSegments];
+#pragma unroll
+    for (int s = 0; s < kOneLaunchSegments; ++s) {
+        const int other = s * kSegment + tid;
+        others[s] = other < assignments && s != segment ? ids[other] : -1;
+    }
+    const int id = valid ? ids[at] : 0;
+    for (int i = tid; i < (kMetaWaves + 2) * experts; i += kMetaThreads) counters[i] = 0;
     __syncthreads();
-    int row_base = 0, tile_base = 0, tile_total = 0, large_base = 0, large_total = 0, small_base = 0, small_total = 0;
-    for (int w = 0; w < kMetaWaves; ++w) {
-        if (w < wave) row_base += wave_rows[w], tile_base += wave_tiles[w], large_base += wave_large[w], small_base += wave_small[w];
-        tile_total += wave_tiles[w], large_total += wave_large[w], small_total += wave_small[w];
-    }
-    if (tid < experts) {
-        const int row = row_base + row_scan - count, tile = tile_base + tile_scan - tiles;
-        first_row[tid] = row;
-        if (segment == 0) counts[tid] = count, row_offsets[tid] = row, tile_offsets[tid] = tile;
-        const int first_large = large_base + large_scan - large, smalls = small_base + small_scan - small;
-        const int at_rest = size == 0 ? first_large + full : large_total + (size == 1 ? smalls & 0xFFFF : (small_total & 0xFFFF) + (smalls >> 16));
-        for (int t = segment; t < tiles; t += total_segments) {
-            tile_expert[tile + t] = tid, tile_row[tile + t] = t * block_m;
-            if (tile_units != nullptr) tile_units[t < full ? first_large + t : at_rest] = make_int4(tid, row + t * block_m, t < full ? block_m : rest, 0);
-        }
-    }
-    if (segment == 0 && tid == 0) tile_count[0] = tile_total;
+#pragma unroll
+    for (int s = 0; s < kOneLaunchSegments; ++s)
+        if (others[s] >= 0) atomicAdd((s < segment ? in_front : behind) + others[s], 1);
+    const LaneRank same = rank_among_lanes(id, valid, lane, experts);
+    if (valid && same.rank == same.group - 1) counters[wave * experts + id] = same.group;
     __syncthreads();
-    if (!valid) return;
-    const int in_expert = in_front[id] + local;
-    relative[at] = in_expert;
-    const int slot = first_row[id] + in_expert;
-    slot_map[at] = slot;
-    slot_token[slot] = at / top_k;
-    if (row_max != nullptr) row_max[at] = 0;
+    int count = 0, before = 0;
+    if (tid < experts) {  // exclusive prefix over the waves, total of the segment
+        int of_wave[kMetaWaves];
+        before = in_front[tid];
+        const int after = behind[tid];
+#pragma unroll
+        for (int w = 0; w < kMetaWaves; ++w) of_wave[w] = counters[w * experts + tid];
+#pragma unroll
+        for (int w = 0; w < kMetaWaves; ++w) counters[w * experts + tid] = count, count += of_wave[w];
+        count += before + after;
+    }
+    place_experts(lds, out, count, before, experts, block_m);
+    if (valid) place_assignment(lds, out, at, id, counters[wave * experts + id] + same.rank, top_k);
 }
 
 // One token: every selected expert owns one row and one tile, in expert-id order
@@ -1014,7 +1076,7 @@ int metadata_geometry(const orx_function& f, int rows, Geometry* g) {
     if (f.flags & kSegments) {
         g->grid[0] = ceil_div((uint32_t)rows * (uint32_t)f.top_k, (uint32_t)kSegment);
         g->block[0] = kMetaThreads;
-        g->shared = (uint32_t)(kMetaWaves * f.E * sizeof(int));
+        g->shared = (uint32_t)((kMetaWaves + (g->grid[0] <= kOneLaunchSegments ? 2 : 0)) * f.E * sizeof(int));
         return ORX_OK;
     }
     g->grid[0] = 1;
@@ -1028,8 +1090,9 @@ int metadata_geometry(const orx_function& f, int rows, Geometry* g) {
 int metadata_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t s, void** args) {
     static DeviceOnce opted_in;  // 64 KiB of counters at E = 1024 needs the LDS opt-in
     const int ready = opted_in.run([] {
-        for (const void* kernel : {reinterpret_cast<const void*>(&route_metadata_kernel), reinterpret_cast<const void*>(&segment_rank_kernel)}) {
-            const int code = hip_check(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024),
+        for (const void* kernel : {reinterpret_cast<const void*>(&route_metadata_kernel), reinterpret_cast<const void*>(&segment_rank_kernel),
+                                   reinterpret_cast<const void*>(&segment_metadata_kernel)}) {
+            const int code = hip_check(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (kernel == reinterpret_cast<const void*>(&segment_metadata_kernel) ? 128 : 160) * 1024),
                                        "hipFuncSetAttribute");
             if (code != ORX_OK) return code;
         }
@@ -1040,13 +1103,21 @@ int metadata_launch(const orx_function& f, int rows, const Geometry& g, hipStrea
     const int offsets_at = maps ? 4 : 3, tiles_at = maps ? 7 : 4;
     if (f.flags & kSegments) {
         const int* ids = pointer_arg<const int>(args, 1);
-        int *relative = pointer_arg<int>(args, 2), *segments = pointer_arg<int>(args, f.workspace_arg);
-        ORX_LAUNCH(segment_rank_kernel, dim3(g.grid[0]), dim3(kMetaThreads), g.shared, s, ids, relative, segments, rows * f.top_k, f.E);
-        ORX_LAUNCH(segment_place_kernel, dim3(g.grid[0]), dim3(kMetaThreads), 0, s, ids, segments, pointer_arg<int>(args, 0),
-                   relative, pointer_arg<int>(args, offsets_at), pointer_arg<int>(args, tiles_at),
-                   pointer_arg<int>(args, tiles_at + 1), pointer_arg<int>(args, tiles_at + 2), pointer_arg<int>(args, tiles_at + 3),
-                   f.flags & kTileUnits ? pointer_arg<int4>(args, tiles_at + 4) : nullptr, pointer_arg<int>(args, 5), pointer_arg<int>(args, 6), pointer_arg<int>(args, 3), rows * f.top_k, f.E, f.top_k,
-                   f.block_m);
+        SegmentOutputs out;
+        out.counts = pointer_arg<int>(args, 0), out.relative = pointer_arg<int>(args, 2), out.row_max = pointer_arg<int>(args, 3);
+        out.row_offsets = pointer_arg<int>(args, offsets_at), out.slot_map = pointer_arg<int>(args, 5), out.slot_token = pointer_arg<int>(args, 6);
+        out.tile_count = pointer_arg<int>(args, tiles_at), out.tile_expert = pointer_arg<int>(args, tiles_at + 1);
+        out.tile_offsets = pointer_arg<int>(args, tiles_at + 2), out.tile_row = pointer_arg<int>(args, tiles_at + 3);
+        out.tile_units = f.flags & kTileUnits ? pointer_arg<int4>(args, tiles_at + 4) : nullptr;
+        const int assignments = rows * f.top_k;
+        const dim3 grid(g.grid[0]), block(kMetaThreads);
+        if (g.grid[0] <= kOneLaunchSegments) {
+            ORX_LAUNCH(segment_metadata_kernel, grid, block, g.shared, s, ids, out, assignments, f.E, f.top_k, f.block_m);
+        } else {
+            int* segments = pointer_arg<int>(args, f.workspace_arg);
+            ORX_LAUNCH(segment_rank_kernel, grid, block, g.shared, s, ids, out.relative, segments, assignments, f.E);
+            ORX_LAUNCH(segment_place_kernel, grid, block, 0, s, ids, segments, out, assignments, f.E, f.top_k, f.block_m);
+        }
         return hip_check(hipGetLastError(), "launch route_metadata");
     }
     ORX_LAUNCH(route_metadata_kernel, dim3(1), dim3(kMetaThreads), g.shared, s, pointer_arg<const int>(args, 1),
@@ -1095,8 +1166,10 @@ int make_metadata(const Variant& v, orx_function* f) {
     if (f->dynamic_rows) f->args.push_back({"m", ArgI32, 4});
     f->geometry = metadata_geometry;
     f->launch = metadata_launch;
-    f->device_function = f->takes_workspace ? reinterpret_cast<const void*>(&segment_rank_kernel)
-                                            : reinterpret_cast<const void*>(&route_metadata_kernel);
+    const bool one_launch = ceil_div((uint32_t)f->M * (uint32_t)f->top_k, (uint32_t)kSegment) <= (uint32_t)kOneLaunchSegments;
+    f->device_function = !f->takes_workspace ? reinterpret_cast<const void*>(&route_metadata_kernel)
+                         : one_launch       ? reinterpret_cast<const void*>(&segment_metadata_kernel)
+                                            : reinterpret_cast<const void*>(&segment_rank_kernel);
     return ORX_OK;
 }
 

@@ -145,6 +145,12 @@ def test_route_metadata_in_segments(m, e, k, bm):
     kern(IDs=gu.dev(padded), m=m, **{**out, "RowMax": None})
 
 
+@pytest.mark.parametrize("m,e,k,bm", [(2049, 16, 8, 128), (1024, 5, 1, 32), (1025, 1024, 1, 128)])
+def test_route_metadata_in_segments_around_the_single_launch(m, e, k, bm):
+    """Up to 16 segments are one launch: 17, with one assignment of the last, one whole segment, and one and a bit over as many experts as threads."""
+    test_route_metadata_in_segments(m, e, k, bm)
+
+
 # Last tiles of every size, full ones only, none at all, more experts than a wave, segments of less than and more than one workgroup.
 @pytest.mark.parametrize("counts,bm", [([128, 0, 1, 129, 64, 65, 32, 33, 300, 0], 128), ([256, 512], 128), ([17, 16, 8, 9, 40, 4, 5], 16),
                                        ([3] * 100 + [200] * 20 + [70] * 30, 128), ([1], 128)])
