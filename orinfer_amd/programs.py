@@ -184,11 +184,22 @@ class QuantizedLinear:
         return self.project(self.quantize(x16, stream), stream)
 
 
-BULK_ROWS = 128  # tile height of the routed projections of long prompts
-# Routed rows per expert from which they beat the 32-row tiles of the seven-launch order (us, seven launches against six):
+BULK_ROWS = 128  # tile height of the routed projections of many rows
+# Routed rows per expert from which they beat the seven-launch order over tiles of 32 rows whatever the shape (us, seven launches against six):
 # 64 experts x top-6, H 3072, I 256: 73 / 76 at 24 rows, 87 / 85 at 48, 136 / 99 at 96; 16 x top-2, H 4096, I 1536: 85 / 88 at 32,
-# 121 / 93 at 64, 325 / 171 at 256.  The five-launch order is kept wherever it applies (up to 8192 routed rows).
+# 121 / 93 at 64, 325 / 171 at 256.
 BULK_ROWS_PER_EXPERT = 48
+
+
+def bulk_pays(routed, experts, hidden, intermediate, cus):
+    """Whether the order over 128-row tiles is faster than the one over tiles of 32 rows, five launches or seven (time of the layer, the latter over the former;
+    170 shapes with 10 to 70 routed rows per expert, popularity like 1 / rank^1.1, 256 CUs).  A tile of 32 rows costs a unit per 512 channels, and as long as both
+    projections together have no more than about one unit to a CU (half a tile per expert more than the rows fill), two where a unit of 256 channels reads long
+    rows, the small tiles win: 0.72-1.03.  Beyond, 24 and more rows per expert 1.01-1.67 (three in a hundred 0.98-0.99), with a uniform popularity 1.01-1.73; 16 to 24 rows of up to 64 experts
+    1.02-1.38 from 1.6 units to a CU on and 0.8-1.16 below, of 128 experts 0.83-1.51 without a line between; fewer rows 0.72-1.16."""
+    units = (routed / 32 + experts / 2) * (-(-2 * intermediate // 512) + -(-hidden // 512))
+    rows = routed / experts
+    return rows >= 24 and units >= max(1.1, hidden / 1600) * cus or rows >= 16 and experts <= 64 and units >= max(1.6, hidden / 1400) * cus
 
 
 class MoeLayer:
@@ -282,13 +293,16 @@ class MoeLayer:
             except OrxError as error:
                 if fused_stages or error.code != ORX_ERR_BAD_VARIANT:
                     raise
-        # Long prompts: six launches over tiles of 128 rows (`block_m` is the tile height of the orders above).
-        #   router top-k + A8 of every token's row, metadata in segments (two launches),
+        # Many rows: six launches over tiles of 128 rows (`block_m` is the tile height of the orders above).
+        #   router top-k + A8 of every token's row, metadata in segments (two launches above 16384 routes),
         #   gate_up that gathers the token rows and writes fp16(silu(gate) * up), A8, down, combine.
-        # A caller who asked for the quantiser and the dispatch, or the metadata, as launches of their own gets them.
+        # A caller who asked for the quantiser and the dispatch, or the metadata, as launches of their own gets them; `fused_stages` stays
+        # true where the five launches are served too.
         self.bulk = False
-        if (not self.fused_stages and fused_stages is None and not keep_intermediates and signs is None and self.fused_dispatch
-                and not one_launch_refused and packed_k == 128 and experts <= 1024 and grouped_algorithm == "auto" and assignments >= BULK_ROWS_PER_EXPERT * experts):
+        if (fused_stages is None and not keep_intermediates and signs is None and self.fused_dispatch
+                and not one_launch_refused and packed_k == 128 and experts <= 1024 and grouped_algorithm == "auto"
+                and (not self.fused_stages and assignments >= BULK_ROWS_PER_EXPERT * experts
+                     or bulk_pays(assignments, experts, hidden, intermediate, torch.cuda.get_device_properties(self.w1.device).multi_processor_count))):
             try:
                 tiles = (assignments + BULK_ROWS - 1) // BULK_ROWS + min(experts, assignments)
                 bulk = dict(rows=assignments, E=experts, tiles=tiles, block_m=BULK_ROWS, tile_units=True)
@@ -319,10 +333,10 @@ class MoeLayer:
 
     def run(self, x16, logits, stream=None):
         s = current_stream() if stream is None else stream
-        if self.fused_stages:
-            return self._run_fused(x16, logits, s)
         if self.bulk:
             return self._run_bulk(x16, logits, s)
+        if self.fused_stages:
+            return self._run_fused(x16, logits, s)
         self.k_router(stream=s, IDs=self.ids, Logits=logits, Prob=self.prob)
         if self.k_metadata is not None:
             self.k_metadata(stream=s, Counts=self.counts, IDs=self.ids, RelativeSlot=self.relative,

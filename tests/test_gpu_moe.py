@@ -351,6 +351,13 @@ def test_grouped_q2_bulk_kernel(n, k, counts, form):
     assert torch.equal(lean, act)
 
 
+@pytest.mark.parametrize("form", ["plain", "swiglu"])
+@pytest.mark.parametrize("n,k,counts", [(128, 640, [1, 32, 33, 64, 65]), (256, 768, [31, 2, 128, 40]), (128, 1152, [16, 63, 129])])
+def test_grouped_q2_bulk_kernel_over_more_chunks_than_it_holds(n, k, counts, form):
+    """5, 6 and 9 chunks of K, tiles of every form: four chunks of a small tile are on their way at once."""
+    test_grouped_q2_bulk_kernel(n, k, counts, form)
+
+
 @pytest.mark.parametrize("swiglu", [False, True], ids=["rows", "gathered-swiglu"])
 def test_grouped_q2_bulk_kernel_takes_its_tiles_from_units(swiglu):
     """The same rows whether a tile comes out of TileExpert, TileRow, Counts and Offsets or out of TileUnits in any order."""
@@ -1233,6 +1240,19 @@ def test_long_prompt_program_gives_the_bits_of_seven_launches():
         graph.replay()
         gu.sync()
         assert torch.equal(six.out, want)
+
+
+@pytest.mark.parametrize("tokens,experts,inter,five,bulk", [(1024, 128, 512, True, True), (384, 128, 512, True, True), (383, 128, 512, True, False),
+                                                            (128, 64, 768, False, True), (127, 64, 768, False, False)])
+def test_orders_for_many_rows_give_the_same_bits(tokens, experts, inter, five, bulk):
+    """From a line of rows per expert and units on the order over 128-row tiles runs, also where the five launches are served; those by name."""
+    c = workloads.config3(tokens=tokens, experts=experts, intermediate=inter)
+    args = (c["tokens"], c["experts"], c["top_k"], c["hidden"], c["intermediate"], c["gate_up"], c["gate_up_scales"], c["down"], c["down_scales"])
+    layer, other = programs.MoeLayer(*args), programs.MoeLayer(*args, fused_stages=five)
+    assert (layer.fused_stages, layer.bulk, other.fused_stages, other.bulk) == (five, bulk, five, False)
+    x, logits = gu.dev(c["x"]), gu.dev(c["logits"])
+    want = other.run(x, logits).clone()
+    assert torch.equal(layer.run(x, logits), want)
 
 
 def test_long_prompts_keep_the_launches_a_caller_asked_for():
