@@ -97,8 +97,9 @@ __device__ __forceinline__ void tile_of(int id, int tiles_m, int tiles_n, int* t
 // waited for and drain under the next tile's multiplies.
 //
 // The kernel is bound by power, not by issue slots: on random int8 data the clock inside the K loop is 1.9 GHz in a
-// sustained run (1.2-1.3 GHz in a launch that follows a pause), the same launch on zero operands is 30 % shorter, and
-// taking out stalls alone changes nothing at large K.  What pays is less energy per multiply.  v_mfma_i32_16x16x64_i8 does the same work per cycle as
+// sustained run (1.2-1.3 GHz in a launch that follows a pause), and
+// taking out the stalls that are left changes nothing with many tiles (lines brought into the L2 two steps ahead: 8192 x 34816 x 5120 1055 -> 932 us on zeros, 1158 ->
+// 1170 on random data; without any requests in the loop 945, without fragment reads 1088).  What pays is less energy per multiply.  v_mfma_i32_16x16x64_i8 does the same work per cycle as
 // v_mfma_i32_32x32x32_i8 with half the accumulator traffic per multiply and sustains 3.83 POP/s on random
 // operands where the 32 x 32 shape sustains 3.37 (back-to-back issue from registers, whole chip); the fragment
 // bytes read from LDS per multiply are the same, so the tile, the stages and the swizzle stay as they were.
@@ -238,10 +239,13 @@ __global__ __launch_bounds__(kPersistentThreads) void gemm_big_persistent_kernel
         f[2] = lds_read_16<2 * kBlockBytes>(w);
         f[3] = lds_read_16<3 * kBlockBytes>(w);
     };
-    // a wave's requests of a K step go out one at a time behind every second multiply of three phases (a wave cannot
-    // issue anything while a vector-memory instruction waits for a slot in the CU's memory pipeline)
+    // A wave's requests of a K step go out one at a time behind every second multiply of two phases (a wave cannot issue anything while a
+    // vector-memory instruction waits for a slot in the CU's memory pipeline): five in the phase behind the barrier that frees the stage, three in the next
+    // step's first.  The first wait for them is that step's barrier, so what goes out later has less than half a step to come from memory: 3 + 3 + 2
+    // over three phases, products alone, 8192 x 4096 x 4096 120.2 -> 114.1 us, 8192 x 34816 x 5120 1211 -> 1158, 8192 x 5120 x 17408 640 -> 606, 2048 x 5120 x
+    // 17408 207 -> 189; 6 + 2 and 8 + 0 0 to 3 % slower than 5 + 3.
     constexpr int LOADS = 2 * BLOCKS_PER_WAVE;
-    constexpr int PART0 = (LOADS + 2) / 3, PART1 = (LOADS - PART0 + 1) / 2, PART2 = LOADS - PART0 - PART1;
+    constexpr int PART0 = 5, PART1 = LOADS - PART0;
     auto multiply_loading = [&](int phase, int first, int count, int stage) {
         v4i(&tokens)[4] = ft[phase & 1];
         v4i(&weights)[4] = fw[phase >> 1];
@@ -373,7 +377,7 @@ __global__ __launch_bounds__(kPersistentThreads) void gemm_big_persistent_kernel
     // earlier: only the younger batch may still be in flight) and multiplies.  Behind phase 2 comes the barrier (step
     // g+1 is complete in LDS and nobody reads stage `cur` any more); then the fragments of step g+1's first phase,
     // and phase 3, whose operands are already in registers, while the requests of step g+2 start into stage `cur`.
-    // The load cursor points at step g+1 until the second group of requests is out, then at step g+2; at the end of
+    // The load cursor points at step g+1 until phase 0 has its requests out, then at step g+2; at the end of
     // the list it stays on the last step, whose repeated requests land in a stage that is not read again.  A tile's
     // last step (LAST) also brings the tile's scales into LDS and keeps its first requests of step g+2 back until the
     // epilogue has read them (a read of LDS waits for every direct-to-LDS request in flight).
@@ -405,7 +409,7 @@ __global__ __launch_bounds__(kPersistentThreads) void gemm_big_persistent_kernel
         read_weights(cur, 1);
         wait_four<8>(ft[1]);
         __builtin_amdgcn_sched_barrier(0);
-        multiply_loading(1, PART0 + PART1, PART2, nxt);
+        multiply_loading(1, 0, 0, nxt);
         __builtin_amdgcn_sched_barrier(0);
         advance();
         read_tokens(cur, 3);                  // 4 younger requests
