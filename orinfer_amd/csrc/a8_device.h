@@ -49,26 +49,26 @@ __device__ __forceinline__ int8_t quantise(float value, float scale, float inver
 }
 
 // Four codes packed into one word; one test (and, rarely, four exact quotients) for the four.
-// A product's distance from its rounded value is at most 0.5, so "within 2^-14 of a tie" is
-// "farther than 0.5 - 2^-14 from the rounded value".  The clamped integer plus 1.5 * 2^23 has the
-// integer in its low mantissa bits in two's complement: the low byte of that word is the int8 code.  The hint keeps
+// The multiply-add rounds the exact product to an integer (1.5 * 2^23 more; the code is that word's low byte in two's complement),
+// and its distance from the product is at most 0.5, so "within 2^-14 of a tie" is "farther than 0.5 - 2^-14 from the rounded value".
+// The clamp is on the word: scales below 2^-14 are rounded so coarsely that quotients pass 127; a NaN gives -127.  The hint keeps
 // the quotients behind their branch: executed for every value they cost a one-piece form a fifth of its time.
 __device__ __forceinline__ uint32_t quantise4(const float (&value)[4], float scale, float inverse) {
+    constexpr float kInteger = 12582912.0f;
     float r[4];
     float farthest = 0.f;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const float guess = value[j] * inverse;
-        r[j] = rintf(guess);
-        farthest = fmaxf(farthest, fabsf(guess - r[j]));
+        r[j] = __builtin_fmaf(value[j], inverse, kInteger);
+        farthest = fmaxf(farthest, fabsf(__builtin_fmaf(value[j], inverse, kInteger - r[j])));
     }
     if (__builtin_expect(farthest > 0.49993896484375f, 0)) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) r[j] = rintf(__fdiv_rn(value[j], scale));
+        for (int j = 0; j < 4; ++j) r[j] = rintf(__fdiv_rn(value[j], scale)) + kInteger;
     }
     uint32_t word[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) word[j] = __float_as_uint(__builtin_amdgcn_fmed3f(r[j], -127.f, 127.f) + 12582912.0f);
+    for (int j = 0; j < 4; ++j) word[j] = __float_as_uint(__builtin_amdgcn_fmed3f(r[j], kInteger - 127.f, kInteger + 127.f));
     // byte 0 of the first operand's partner (second argument), then byte 0 of the first argument
     const uint32_t low = __builtin_amdgcn_perm(word[1], word[0], 0x0C0C0400u);
     const uint32_t high = __builtin_amdgcn_perm(word[3], word[2], 0x0C0C0400u);

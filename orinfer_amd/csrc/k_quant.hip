@@ -102,7 +102,7 @@ __device__ __forceinline__ uint2 quantise_piece(word4 piece, float scale, float 
 // (us, against two passes with 16-byte loads, FUSED in brackets: 1 x 40960 12.7 -> 5.0 (81 -> 10.8), 2048 x 40960 77.5 -> 53.7
 // (263 -> 103), 512 x 131072 86 -> 49.5 (562 -> 115); four pieces held instead of eight: 5.9 (16.0), 59.5 (130), 52 (114)).
 // What bounds it: memory with many rows (8192 x 4096: 28.1 -> 20.7 us, 4.9 TB/s; the two-pass kernel read every row twice),
-// the vector ALU beside it in the FUSED form (8192 x 17408: 416 -> 146 us; the two-pass kernel also computed every value
+// the vector ALU beside it in the FUSED form (8192 x 17408: 416 -> 146 us, and 141.1 -> 135.4 with a multiply-add to a code; the two-pass kernel also computed every value
 // twice), the latency of one row's loads and reductions with few (FUSED, one row of 17408: 43 -> 5.9 us).
 // PANELS (one group to a row, K a multiple of 128): the codes a second time in the order in which k_panel.hip's projection reads them, and the sum
 // of a row's codes.
@@ -284,7 +284,7 @@ __device__ __forceinline__ float rotate_block(float (&v)[4], int l32, __half (&o
 }
 
 // The same stages for rows whose codes are all that is kept, in 28 vector instructions per lane and four channels where rotate_block takes 52 of a kernel's
-// 150 and an LDS trip each (rotation and A8 of 8192 x 5120, bound by them: 43.4 -> 40.1 us; 20 rows with residual and norm, where the chain counts: 5.5 -> 5.2, which
+// 150 and an LDS trip each (rotation and A8 of 8192 x 5120, bound by them: 43.4 -> 40.1 us, and 36.5 -> 34.3 with a multiply-add to a code; 20 rows with residual and norm, where the chain counts: 5.5 -> 5.2, which
 // the layer around it does not show beyond noise; 8192 rows of those are bound by memory, 88 us).
 //  * A stage between lanes is one instruction per value, own + (+-1) partner: exact, for a fused multiply-add with +-1 rounds as the add does. The
 //    upper lane of a pair gets own - partner, the negative of what it should hold; so does its partner of every later stage, and the

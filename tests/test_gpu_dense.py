@@ -130,6 +130,19 @@ def test_a8_held_forms(rows, k, group, fused):
     np.testing.assert_array_equal(gu.host(q), wq)
 
 
+@pytest.mark.parametrize("amax", [254.0, 127.0, 65504.0, 1.0, 3e-3, 2.0**-12, 300 * 2.0**-24, 190 * 2.0**-24, 3 * 2.0**-24])
+def test_a8_every_value_up_to_the_largest(amax):
+    """All fp16 values of a row with this largest one: ties at scales 1 and 2, quotients beyond 127 at subnormal scales."""
+    every = np.arange(65536, dtype=np.uint16).view(np.float16)
+    every = every[np.isfinite(every)]
+    x = np.where(np.abs(every.astype(np.float32)) <= np.float32(np.float16(amax)), every, np.float16(0))[None]
+    assert np.abs(x).max() == np.float16(amax)
+    q, s = gu.a8(gu.dev(x), group=None)
+    wq, ws = orc.a8(x)
+    np.testing.assert_array_equal(gu.host(s), ws)
+    np.testing.assert_array_equal(gu.host(q), wq)
+
+
 def test_swiglu_gates_without_a_finite_sigmoid_product():
     """Gates at and beyond the ends of the exponential against the formula in fp32: a gate of minus infinity has no value
     (-inf * 0), the gates down to -104 keep a sigmoid above zero, and what the products make of infinities is theirs."""
