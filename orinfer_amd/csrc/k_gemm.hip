@@ -69,6 +69,7 @@ int grouped_resident_launch(const GroupedBuffers& b, int n, int k, int tiles, in
 bool grouped_bulk_eligible(int n, int k, int block_m, int packed_k, int64_t rows);
 void grouped_bulk_geometry(int n, int tiles, bool swiglu, Geometry* g);
 int grouped_bulk_launch(const GroupedBuffers& b, int n, int k, int tiles, bool gather, bool swiglu, hipStream_t stream);
+int make_few_rows(const Variant& v, orx_function* f);  // k_few.hip
 int stream_grouped_launch(const int8_t* a, const void* w, const uint32_t* book, const __half* ws, const __half* as,
                           void* out, const int* counts, const int* offsets, const int* tile_expert, const int* tile_row,
                           const int* tile_count, int n, int k, int tiles, int block_m, int packed_k,
@@ -1839,6 +1840,7 @@ int grouped_launch(const orx_function& f, int rows, const Geometry& g, hipStream
 
 int make_q2_grouped(const Variant& v, orx_function* f) {
     bool bad = false;
+    if (f->symbol == "e8p_decode_grouped" && v.boolean("few_rows", false, &bad)) return make_few_rows(v, f);
     f->capacity = f->M = (int)v.integer("rows", 0, &bad);
     f->E = (int)v.integer("E", 0, &bad);
     f->tiles = (int)v.integer("tiles", 0, &bad);
@@ -2240,7 +2242,7 @@ const Registration* gemm_registrations(int* count) {
     {"int8_swiglu", make_int8_swiglu, "M, N, K, dynamic_rows=false, algorithm=tensor_core|dp4a, block_m, block_n (checked, not used)",
      "A,Gate,GateScale,Output,TokenScale,Up,UpScale[,m]"},
     {"e8p_decode_grouped", make_q2_grouped,
-     "rows, E, tiles, N, K, block_m=32|64|128|8|16 (row step of the tile list), packed_k=128|64|0, dynamic_rows=false, algorithm=auto|stream|resident|mfma, input_dtype=int8|float16, gather=false, epilogue=none|swiglu, tile_units=false",
+     "rows, E, tiles, N, K, block_m=32|64|128|8|16 (row step of the tile list), packed_k=128|64|0, dynamic_rows=false, algorithm=auto|stream|resident|mfma, input_dtype=int8|float16, gather=false, epilogue=none|swiglu, tile_units=false, few_rows=false",
      "A,AS[,Act],Book,C,Counts,Offsets,P[,Q][,RowMax][,SlotToken],TileCount,TileExpert,TileRow[,TileUnits],WS[,m]"},
     {"integer_vq", make_vq_direct,
      "E, M (rows of every expert), N, K, block_m=16|8|32|64, packed_k=128|64|0, patched=false, shared_table=false, shortbook=false, "

@@ -323,9 +323,32 @@ class MoeLayer:
             except OrxError as error:
                 if error.code != ORX_ERR_BAD_VARIANT:
                     raise
-        # the dispatched rows and the gate | up outputs, which the order for long prompts does without
+        # Few rows: where neither order applies, five launches over tiles of 32 rows, any hidden and intermediate width.
+        #   router top-k + A8 of every token's row, metadata with the tiles as units,
+        #   gate_up that gathers the token rows, writes fp16(silu(gate) * up) and raises every slot's largest magnitude,
+        #   down that quantises those rows on their way, combine.
+        # A caller who asked for launches of their own, for the values in between (`keep_intermediates`) or for an algorithm gets them.
+        self.few = False
+        if (fused_stages is None and not self.bulk and not self.fused_stages and not keep_intermediates and signs is None and self.fused_dispatch
+                and not one_launch_refused and packed_k == 128 and block_m == 32 and experts <= 1024 and grouped_algorithm == "auto"):
+            try:
+                few = dict(rows=assignments, E=experts, tiles=self.tile_capacity, block_m=block_m, few_rows=True)
+                self.k_router_a8 = Kernel("router_topk", renormalize=True, quantize_hidden=hidden, **common)
+                self.k_metadata_slots = Kernel("route_metadata", block_m=block_m, slot_maps=True, workspace=True, tile_units=True, **common)
+                self.k_gate_up_few = Kernel("e8p_decode_grouped", N=2 * intermediate, K=hidden, gather=True, epilogue="swiglu", **few)
+                self.k_down_few = Kernel("e8p_decode_grouped", N=hidden, K=intermediate, input_dtype="float16", **few)
+                self.segments = self.k_metadata_slots.workspace()
+                self.tile_units = torch.empty((self.tile_capacity, 4), **i32)
+                self.slot_token = torch.empty(assignments, **i32)
+                self.row_max = torch.empty(assignments, **i32)
+                self.act = torch.empty((assignments, intermediate), **f16)
+                self.few = True
+            except OrxError as error:
+                if error.code != ORX_ERR_BAD_VARIANT:
+                    raise
+        # the dispatched rows and the gate | up outputs, which the orders for long prompts and for few rows do without
         self.d = self.ds = self.gate_up_out = None
-        if not self.bulk:
+        if not self.bulk and not self.few:
             self.d = torch.empty((assignments, hidden), **i8)
             self.ds = torch.empty((assignments, 1), **f16)
             self.gate_up_out = torch.empty((assignments, 2 * intermediate), **f16)
@@ -337,6 +360,8 @@ class MoeLayer:
             return self._run_bulk(x16, logits, s)
         if self.fused_stages:
             return self._run_fused(x16, logits, s)
+        if self.few:
+            return self._run_few(x16, logits, s)
         self.k_router(stream=s, IDs=self.ids, Logits=logits, Prob=self.prob)
         if self.k_metadata is not None:
             self.k_metadata(stream=s, Counts=self.counts, IDs=self.ids, RelativeSlot=self.relative,
@@ -380,6 +405,19 @@ class MoeLayer:
                             SlotToken=self.slot_token, WS=self.s1, **routed)
         self.k_act_a8(stream=s, Mask=None, Q=self.h_q, S=self.h_s, X=self.act, rows=self.assignments)
         self.k_down_bulk(stream=s, A=self.h_q, AS=self.h_s, C=self.down_out, P=self.w2, WS=self.s2, **routed)
+        self.k_combine(stream=s, Expert=self.down_out, Output=self.out, Prob=self.prob, Shared=None, SharedGate=None,
+                       SlotMap=self.slot_map)
+        return self.out
+
+    def _run_few(self, x16, logits, s):
+        self.k_router_a8(stream=s, IDs=self.ids, Logits=logits, Prob=self.prob, Q=self.a_q, S=self.a_s, X=x16)
+        self.k_metadata_slots(stream=s, Counts=self.counts, IDs=self.ids, RelativeSlot=self.relative, RowMax=self.row_max,
+                              RowOffsets=self.row_offsets, SlotMap=self.slot_map, SlotToken=self.slot_token,
+                              TileCount=self.tile_count, TileExpert=self.tile_expert, TileOffsets=self.tile_offsets,
+                              TileRow=self.tile_row, TileUnits=self.tile_units, Workspace=self.segments)
+        routed = dict(Book=self.book, RowMax=self.row_max, TileCount=self.tile_count, TileUnits=self.tile_units)
+        self.k_gate_up_few(stream=s, A=self.a_q, AS=self.a_s, Act=self.act, P=self.w1, SlotToken=self.slot_token, WS=self.s1, **routed)
+        self.k_down_few(stream=s, A=self.act, C=self.down_out, P=self.w2, WS=self.s2, **routed)
         self.k_combine(stream=s, Expert=self.down_out, Output=self.out, Prob=self.prob, Shared=None, SharedGate=None,
                        SlotMap=self.slot_map)
         return self.out

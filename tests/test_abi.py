@@ -483,6 +483,11 @@ def test_argument_lists_of_the_fused_expert_layer_forms():
     assert names("route_metadata", M=8, E=64, top_k=4, block_m=32, slot_maps=True) == [
         "Counts", "IDs", "RelativeSlot", "RowMax", "RowOffsets", "SlotMap", "SlotToken", "TileCount", "TileExpert",
         "TileOffsets", "TileRow"]
+    few = dict(rows=64, E=16, tiles=18, few_rows=True)
+    assert names("e8p_decode_grouped", N=1024, K=4096, gather=True, epilogue="swiglu", **few) == [
+        "A", "AS", "Act", "Book", "P", "RowMax", "SlotToken", "TileCount", "TileUnits", "WS"]
+    assert names("e8p_decode_grouped", N=4096, K=512, input_dtype="float16", **few) == [
+        "A", "Book", "C", "P", "RowMax", "TileCount", "TileUnits", "WS"]
     grouped = dict(rows=2048, E=128, tiles=192, block_m=32, algorithm="resident")
     plain = ["A", "AS", "Book", "C", "Counts", "Offsets", "P", "TileCount", "TileExpert", "TileRow", "WS"]
     assert names("e8p_decode_grouped", N=1024, K=2048, **grouped) == plain
@@ -506,6 +511,11 @@ def test_argument_lists_of_the_fused_expert_layer_forms():
         "DS", "IDs", "Q", "RelativeSlot", "RowOffsets", "S", "Signs", "SlotMap", "Sum", "X"]
     assert names("rotate_expert_a8", M=4, K=256, hand_over="int8") == ["Q", "S", "Signs", "Sum", "X"]
     refused = (
+        ("e8p_decode_grouped", dict(N=1024, K=4096, **few)),                                     # neither of the two forms
+        ("e8p_decode_grouped", dict(N=1024, K=4096, gather=True, epilogue="swiglu", packed_k=0, **few)),
+        ("e8p_decode_grouped", dict(N=1040, K=4096, gather=True, epilogue="swiglu", **few)),
+        ("e8p_decode_grouped", dict(N=1024, K=4096, input_dtype="float16", **few)),              # the fp16 rows of a tile do not fit LDS
+        ("e8p_decode_grouped", dict(N=1024, K=4096, gather=True, epilogue="swiglu", algorithm="stream", **few)),
         ("e8p_decode_grouped", dict(N=1024, K=2048, gather=True, rows=8200, E=128, tiles=512, block_m=32, algorithm="resident")),
         # without the SwiGLU epilogue the kernel keeps its phase-two sums in LDS, which leaves room for fewer slots
         ("e8p_decode_grouped", dict(N=1024, K=2048, gather=True, rows=8192, E=128, tiles=512, block_m=32, algorithm="resident")),

@@ -1255,6 +1255,35 @@ def test_orders_for_many_rows_give_the_same_bits(tokens, experts, inter, five, b
     assert torch.equal(layer.run(x, logits), want)
 
 
+@pytest.mark.parametrize("tokens,experts,top_k,hidden,inter", [
+    (2, 16, 8, 3200, 256), (3, 4, 2, 128, 128),       # tiles of a row or two; K blocks fewer than the waves that share them
+    (40, 2, 2, 384, 256),                             # 40 rows to an expert: a full tile and one of eight rows
+    (17, 1, 1, 640, 128), (9, 1, 1, 1280, 384),       # one expert, tiles of 17 and 9 rows
+    (85, 32, 8, 1920, 1280), (30, 8, 4, 4096, 1536),  # long rows of down; the widest
+    (150, 64, 2, 1152, 144 * 8)])
+def test_few_rows_give_the_bits_of_seven_launches(tokens, experts, top_k, hidden, inter):
+    """Five launches over 32-row tiles where the resident kernel does not apply, eagerly and replayed; gates that leave fp16 among the values."""
+    c = workloads.config3(tokens=tokens, experts=experts, top_k=top_k, hidden=hidden, intermediate=inter)
+    scales = np.array(c["gate_up_scales"])
+    scales[:, 5] = 60000.0
+    args = (tokens, experts, top_k, hidden, inter, c["gate_up"], scales, c["down"], c["down_scales"])
+    seven, few = programs.MoeLayer(*args, fused_stages=False), programs.MoeLayer(*args)
+    assert few.few and not few.fused_stages and not few.bulk and not seven.few
+    x, logits = gu.dev(c["x"]), gu.dev(c["logits"])
+    want = gu.host(seven.run(x, logits))
+    np.testing.assert_array_equal(gu.host(few.run(x, logits)), want)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    gu.sync()
+    with torch.cuda.graph(graph, stream=stream):
+        few.run(x, logits, stream=stream.cuda_stream)
+    for _ in range(3):
+        few.out.fill_(float("nan"))
+        few.counts.fill_(-7)
+        graph.replay()
+        gu.sync()
+        np.testing.assert_array_equal(gu.host(few.out), want)
+
+
 def test_long_prompts_keep_the_launches_a_caller_asked_for():
     """fused_dispatch=False and fused_metadata=False hold whatever the row count is, and with the quantiser as a launch of its
     own the hidden rows may start at any fp16 address."""
