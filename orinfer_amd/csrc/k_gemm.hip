@@ -70,6 +70,10 @@ bool grouped_bulk_eligible(int n, int k, int block_m, int packed_k, int64_t rows
 void grouped_bulk_geometry(int n, int tiles, bool swiglu, Geometry* g);
 int grouped_bulk_launch(const GroupedBuffers& b, int n, int k, int tiles, bool gather, bool swiglu, hipStream_t stream);
 int make_few_rows(const Variant& v, orx_function* f);  // k_few.hip
+// from k_mid.hip
+int gemm_mid_launch(const int8_t* a, const void* w, const __half* ws, const __half* as, void* out, int rows, int n, int k, int stride, bool out_f32, int parts,
+                    int* partials, hipStream_t stream);
+constexpr uint64_t kMidSlotBytes = 64 * 1024;  // of `partials` for every part of a tile, if there are several
 int stream_grouped_launch(const int8_t* a, const void* w, const uint32_t* book, const __half* ws, const __half* as,
                           void* out, const int* counts, const int* offsets, const int* tile_expert, const int* tile_row,
                           const int* tile_count, int n, int k, int tiles, int block_m, int packed_k,
@@ -1015,10 +1019,10 @@ uint64_t big_rest_workspace(const orx_function& f, int rows) {
     return (uint64_t)split_groups_for_channels(f.N - main_channels, rows, f.K) * 2 * kSplitSlotInts * sizeof(int);
 }
 
-// Workspace bytes of a launch: the partial slots of a split launch, or the decoded weights of a
+// Workspace bytes of a launch without the 128 x 128 tiles below: the partial slots of a split launch, or the decoded weights of a
 // two-stage launch on the 256-row tiles (and behind them the partial slots of the channels that the
 // persistent launch leaves to the split tiles).
-uint64_t projection_workspace(const orx_function& f, int rows) {
+uint64_t workspace_without_mid(const orx_function& f, int rows) {
     if (use_runs(f, rows)) return 0;
     if (use_wide(f, rows) || use_tall(f, rows)) return 0;
     if (use_gemv(f, rows) || use_resident(f, rows) || use_stream(f, rows)) return 0;
@@ -1026,6 +1030,39 @@ uint64_t projection_workspace(const orx_function& f, int rows) {
     if (use_big(f, rows)) return f.flags == kW8 ? big_rest_workspace(f, rows) : 0;
     if (use_split(f, rows)) return (uint64_t)split_groups_for(f, rows) * 2 * kSplitSlotInts * sizeof(int);
     return 0;
+}
+
+// Parts of K of the 128 x 128 int8 tiles of k_mid.hip, 0 where others serve the launch: above 128 rows, up to two tiles to a CU, where the channel runs and the
+// kernels for fewer rows leave it; two-stage codes where they may be decoded once.  Against what ran before (256 x 256 tiles on fewer than half of the CUs, K steps of
+// older 128 x 128 tiles dealt out and summed, those tiles whole), products with the decode, us: int8 800 x 4096 x 4096 44.5 -> 18.3, 3317 x 1344 x 5248 58.3 -> 31.2, 674 x 3840 x 8960
+// 58.7 -> 37.7, 1536 x 4096 x 2048 25.9 -> 16.9; codes 1627 x 1408 x 2304 32.9 -> 18.2, 674 x 5248 x 3840 46.8 -> 34.0, 1583 x 3040 x 3072 42.9 -> 31.7; 640 to 3000 rows of 1024 to
+// 7168 channels, K 1024 to 14336, 350 shapes 1.01-2.64 times as fast (median 1.5).  Beyond two tiles to a CU the 256 x 256 tiles are (575 tiles 36 against 39, 1024 54 against 61).
+// A CU with one workgroup takes 0.44 us a step, one with two 0.78 for both.  Parts cost their sums a trip through memory and a launch, about 8 us and 0.02 for each, and pay where few tiles have long
+// rows: 704 x 1856 x 10624 49.1 -> 37.7 in four, 512 x 5120 x 17408 62.0 -> 55.5 in three.
+// A launch's Workspace is never larger than what it was before these tiles, so one that a caller has measured out once holds it; the geometry that is reported (and that a record
+// of a launch names) stays too.
+int mid_parts(const orx_function& f, int rows) {
+    if (f.algorithm != kAuto || tile_for(f, rows) != 0 || f.K % kBK != 0 || rows <= 128 || (f.flags != kW8 && f.flags != kQ4)) return 0;
+    const int64_t tiles = split_tiles(f, rows), most = 2 * (int64_t)device_compute_units(), steps = f.K / kBK;
+    if (tiles > most) return 0;
+    const bool codes = f.flags == kQ4;
+    if (codes && (!f.takes_workspace || (f.flags2 & kNoExpand))) return 0;
+    if (use_runs(f, rows) || use_wide(f, rows) || use_tall(f, rows) || use_gemv(f, rows) || use_resident(f, rows) || use_stream(f, rows)) return 0;
+    const uint64_t held = workspace_without_mid(f, rows), decoded = codes ? (uint64_t)f.N * f.K : 0;
+    if (decoded > held) return 0;
+    int best = 1;
+    double least = (2 * tiles <= most ? 0.44 : 0.78) * steps / 1.1;  // (what is gained has to be worth the launch)
+    for (int parts = 2; parts <= 8 && parts * tiles <= most && !(f.flags2 & kNoSplit); ++parts) {
+        const double time = (2 * parts * tiles <= most ? 0.44 : 0.78) * steps / parts + 8 + 0.02 * parts * tiles;
+        if (time < least && decoded + (uint64_t)tiles * parts * kMidSlotBytes <= held) best = parts, least = time;
+    }
+    return best;
+}
+
+uint64_t projection_workspace(const orx_function& f, int rows) {
+    const int parts = mid_parts(f, rows);
+    if (parts == 0) return workspace_without_mid(f, rows);
+    return (f.flags == kQ4 ? (uint64_t)f.N * f.K : 0) + (parts > 1 ? (uint64_t)split_tiles(f, rows) * parts * kMidSlotBytes : 0);
 }
 
 template <int CODEC>
@@ -1139,6 +1176,12 @@ int q4_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t st
         }
         return ORX_OK;
     }
+    if (const int parts = mid_parts(f, rows)) {
+        const int code = q4_expand_launch(p.w, p.book, workspace, f.N, f.K, f.packed_k, stream);
+        if (code != ORX_OK) return code;
+        return gemm_mid_launch(p.a, workspace, p.ws, p.as, p.out, rows, f.N, f.K, f.stride, f.out_f32, parts,
+                               reinterpret_cast<int*>(static_cast<char*>(workspace) + (size_t)f.N * f.K), stream);
+    }
     if (use_expand(f, rows)) {
         const int code = q4_expand_launch(p.w, p.book, workspace, f.N, f.K, f.packed_k, stream);
         if (code != ORX_OK) return code;
@@ -1177,6 +1220,8 @@ int w8_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t st
         }
         return ORX_OK;
     }
+    if (const int parts = mid_parts(f, rows))
+        return gemm_mid_launch(p.a, p.w, p.ws, p.as, p.out, rows, f.N, f.K, f.stride, f.out_f32, parts, static_cast<int*>(workspace), stream);
     if (use_big(f, rows)) return int8_big_launch(f, rows, g, stream, p, p.w, workspace);
     if (use_split(f, rows)) {
         p.partials = static_cast<int*>(workspace);
