@@ -581,6 +581,42 @@ def test_mid_row_projections_split_k_steps_evenly(codec, m, n, k, dtype):
     assert torch.equal(out, other)
 
 
+@pytest.mark.parametrize("codec,m,n,k,dtype,pad,parts", [
+    ("w8", 513, 144, 128, "float16", 0, 1), ("w8", 640, 257, 256, "float16", 3, 1),     # one and two K steps of four stages
+    ("w8", 600, 1000, 384, "float32", 0, 1), ("q4", 521, 528, 512, "float16", 8, 1),    # three, and as many as there are stages
+    ("w8", 700, 400, 640, "float16", 1, 1), ("q4", 650, 130, 1152, "float32", 5, 1),    # more of them
+    ("w8", 2050, 2064, 256, "float16", 0, 1), ("q4", 1100, 4112, 640, "float16", 8, 1),  # two workgroups to a CU, two stages
+    ("w8", 520, 250, 14336, "float16", 4, 8), ("q4", 770, 256, 8320, "float16", 0, 8), ("w8", 641, 1930, 14336, "float32", 2, 5)])  # tiles in parts of K
+def test_tiles_of_128_by_128(codec, m, n, k, dtype, pad, parts):
+    """The edges of tiles, steps and stages; rows that start at any address; nothing beyond the rows and channels is written."""
+    rng = np.random.default_rng(orc.SEED + m + n)
+    a = rng.integers(-128, 128, (m, k), dtype=np.int8)
+    a_s = rng.uniform(0.01, 0.03, m).astype(np.float16)
+    scales = rng.uniform(0.005, 0.02, n).astype(np.float16)
+    stride = n + pad
+    variant = dict(M=m, N=n, K=k, output_dtype=dtype, output_stride=stride, workspace=True)
+    if codec == "q4":
+        packed = rng.integers(0, 2**32, (n, k // 8), dtype=np.uint32)
+        weights, stored = orc.q4_integers(packed, TABLE), gu.dev(packed)
+        kern = gu.lib.Kernel("e8p_q4_projection", **variant)
+        call = lambda out: kern(A=gu.dev(a), AS=gu.dev(a_s), Book=gu.book(), Out=out, S=gu.dev(scales), W=stored, Workspace=kern.workspace())
+    else:
+        weights = rng.integers(-128, 128, (n, k), dtype=np.int8)
+        stored, kern = gu.dev(weights), gu.lib.Kernel("int8_projection", **variant)
+        call = lambda out: kern(A=gu.dev(a), Output=out, TokenScale=gu.dev(a_s), Weight=stored, WeightScale=gu.dev(scales), Workspace=kern.workspace())
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        tiles = -(-m // 128) * -(-n // 128)
+        assert kern.workspace_bytes(m) == (n * k if codec == "q4" else 0) + (tiles * parts * 65536 if parts > 1 else 0)
+    want = orc.project(a, a_s, weights, scales, out_dtype=np.float16 if dtype == "float16" else np.float32)
+    flat = torch.full(((m + 1) * stride + 1,), 9.0, dtype=torch.float16 if dtype == "float16" else torch.float32, device=gu.DEV)
+    for shift in (0, 1):
+        flat.fill_(9)
+        call(flat[shift : shift + (m + 1) * stride])
+        out = gu.host(flat[shift : shift + (m + 1) * stride].view(m + 1, stride))
+        np.testing.assert_array_equal(out[:m, :n], want)
+        assert (out[m] == 9).all() and (out[:, n:] == 9).all()
+
+
 @pytest.mark.parametrize("packed_k", [128, 64])
 def test_split_launches_serve_k_major_codes_and_dynamic_rows(packed_k):
     rng = np.random.default_rng(orc.SEED + 91)
