@@ -85,6 +85,29 @@ def int8_panels_pay(rows, n, k, cus):
     return k <= (4096 if blocks <= cus else 5120 if 2 * blocks <= 3 * cus else 8192)
 
 
+def tiles_pay(codec, rows, n, k, cus):
+    """Whether row-major rows over 128 x 128 tiles are faster than panels where these were the faster ones before the tiles (time of the pair over panels / row-major, 256 CUs,
+    by blocks of 16 channels to a CU).
+    Codes, 513-1024 rows: half to 1.5 blocks 1.06-1.7; to two blocks 1.01-1.15 above 768 rows, 0.88-0.99 below; wider 0.80-0.93; up to half a block 1.0-1.09 above 850 rows from K = 2048
+    on, 0.80-0.99 otherwise.  Up to 512 rows panels (where they were) 0.56-0.98.
+    int8, 129-256 rows: two to three blocks 1.02-1.09 above 208 rows, 0.92-1.03 otherwise.  257-512 rows: up to two blocks 0.99-1.37, wider 0.79-0.96 (K = 1024 1.07).  513 rows and
+    more 1.06-1.43 (a third of a block at 515 rows 0.94)."""
+    if rows <= 128 or -(-rows // 128) * -(-n // 128) > 2 * cus:
+        return False
+    blocks = -(-n // 16)
+    if codec == "q4":
+        if rows <= 512:
+            return False
+        if 2 * blocks <= cus:
+            return rows > 850 and k >= 2048
+        return 2 * blocks <= 3 * cus or (rows > 768 and blocks <= 2 * cus)
+    if rows <= 256:
+        return rows > 208 and 2 * cus < blocks <= 3 * cus
+    if rows <= 512:
+        return blocks <= 2 * cus or k <= 1024
+    return rows > 576 or 3 * blocks > cus
+
+
 class QuantizedLinear:
     """A8 quantiser + one projection (E8P-Q4 or W8A8) with a dynamic row count up to `capacity`."""
 
@@ -111,6 +134,7 @@ class QuantizedLinear:
             pays = panels_pay if codec == "q4" else int8_panels_pay
             cus = torch.cuda.get_device_properties(self.weight.device).multi_processor_count
             self.over_panels = [pays(rows, self.n, self.k, cus) for rows in range(top + 1)]
+            self.over_tiles = [tiles_pay(codec, rows, self.n, self.k, cus) for rows in range(top + 1)]
         # (both copies in one allocation: a second one, new from the driver, took 2 ms of a construction)
         padded = (top + 15) // 16 * 16 if any(self.over_panels) else 0
         codes = torch.empty((capacity + padded, self.k), dtype=torch.int8, device="cuda")
@@ -172,7 +196,7 @@ class QuantizedLinear:
             self.single(stream=stream, A=x16, AS=self.a_s, Book=self.book, Out=self.out, Q=self.a_q, S=self.scales, W=self.weight)
             return self._rows(1)
         rows = x16.shape[0]
-        if rows < len(self.over_panels) and self.over_panels[rows]:
+        if rows < len(self.over_panels) and self.over_panels[rows] and not self.over_tiles[rows]:
             self.panel_quantizer(stream=stream, Mask=None, Panels=self.panels, Q=self.a_q, S=self.a_s, Sums=self.sums, X=x16, rows=rows)
             if self.codec == "q4":
                 self.panel_projection(stream=stream, A=self.panels, AS=self.a_s, Book=self.book, Out=self.out, S=self.scales, Sums=self.sums,
