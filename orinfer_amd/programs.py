@@ -226,6 +226,12 @@ def bulk_pays(routed, experts, hidden, intermediate, cus):
     return rows >= 24 and units >= max(1.1, hidden / 1600) * cus or rows >= 16 and experts <= 64 and units >= max(1.6, hidden / 1400) * cus
 
 
+def one_launch_routes(tokens, top_k, experts):
+    """Whether router and metadata of few tokens are faster in one launch, whose workgroup has sixteen waves: a token to a wave at a time, top_k ranks one after another
+    (time of the layer, one launch over two: up to 18 ranks a wave 0.79-0.99, 24 and 32 1.01-1.11)."""
+    return tokens <= 64 and tokens * top_k <= 1024 and experts <= 512 and -(-tokens // 16) * top_k <= 18
+
+
 class MoeLayer:
     """Q2A8 expert layer: token-sort, grouped gate_up, SwiGLU->A8, grouped down, weighted combine."""
 
@@ -357,6 +363,10 @@ class MoeLayer:
                 and not one_launch_refused and packed_k == 128 and block_m == 32 and experts <= 1024 and grouped_algorithm == "auto"):
             try:
                 few = dict(rows=assignments, E=experts, tiles=self.tile_capacity, block_m=block_m, few_rows=True)
+                # four where router and metadata are one
+                self.k_routes = None
+                if one_launch_routes(tokens, top_k, experts):
+                    self.k_routes = Kernel("router_topk", renormalize=True, quantize_hidden=hidden, metadata=True, block_m=block_m, **common)
                 self.k_router_a8 = Kernel("router_topk", renormalize=True, quantize_hidden=hidden, **common)
                 self.k_metadata_slots = Kernel("route_metadata", block_m=block_m, slot_maps=True, workspace=True, tile_units=True, **common)
                 self.k_gate_up_few = Kernel("e8p_decode_grouped", N=2 * intermediate, K=hidden, gather=True, epilogue="swiglu", **few)
@@ -434,11 +444,14 @@ class MoeLayer:
         return self.out
 
     def _run_few(self, x16, logits, s):
-        self.k_router_a8(stream=s, IDs=self.ids, Logits=logits, Prob=self.prob, Q=self.a_q, S=self.a_s, X=x16)
-        self.k_metadata_slots(stream=s, Counts=self.counts, IDs=self.ids, RelativeSlot=self.relative, RowMax=self.row_max,
-                              RowOffsets=self.row_offsets, SlotMap=self.slot_map, SlotToken=self.slot_token,
-                              TileCount=self.tile_count, TileExpert=self.tile_expert, TileOffsets=self.tile_offsets,
-                              TileRow=self.tile_row, TileUnits=self.tile_units, Workspace=self.segments)
+        metadata = dict(Counts=self.counts, IDs=self.ids, RelativeSlot=self.relative, RowMax=self.row_max, RowOffsets=self.row_offsets,
+                        SlotMap=self.slot_map, SlotToken=self.slot_token, TileCount=self.tile_count, TileExpert=self.tile_expert,
+                        TileOffsets=self.tile_offsets, TileRow=self.tile_row, TileUnits=self.tile_units)
+        if self.k_routes is not None:
+            self.k_routes(stream=s, Logits=logits, Prob=self.prob, Q=self.a_q, S=self.a_s, X=x16, **metadata)
+        else:
+            self.k_router_a8(stream=s, IDs=self.ids, Logits=logits, Prob=self.prob, Q=self.a_q, S=self.a_s, X=x16)
+            self.k_metadata_slots(stream=s, Workspace=self.segments, **metadata)
         routed = dict(Book=self.book, RowMax=self.row_max, TileCount=self.tile_count, TileUnits=self.tile_units)
         self.k_gate_up_few(stream=s, A=self.a_q, AS=self.a_s, Act=self.act, P=self.w1, SlotToken=self.slot_token, WS=self.s1, **routed)
         self.k_down_few(stream=s, A=self.act, C=self.down_out, P=self.w2, WS=self.s2, **routed)

@@ -480,6 +480,9 @@ def test_argument_lists_of_the_fused_expert_layer_forms():
 
     assert names("router_topk", M=8, E=64, top_k=4, quantize_hidden=256) == ["IDs", "Logits", "Prob", "Q", "S", "X"]
     assert names("router_topk", M=8, E=64, top_k=4, dynamic_rows=True) == ["IDs", "Logits", "Prob", "m"]
+    assert names("router_topk", M=8, E=64, top_k=4, quantize_hidden=256, metadata=True) == [
+        "Counts", "IDs", "Logits", "Prob", "Q", "RelativeSlot", "RowMax", "RowOffsets", "S", "SlotMap", "SlotToken", "TileCount", "TileExpert", "TileOffsets",
+        "TileRow", "TileUnits", "X"]
     assert names("route_metadata", M=8, E=64, top_k=4, block_m=32, slot_maps=True) == [
         "Counts", "IDs", "RelativeSlot", "RowMax", "RowOffsets", "SlotMap", "SlotToken", "TileCount", "TileExpert",
         "TileOffsets", "TileRow"]
@@ -529,6 +532,11 @@ def test_argument_lists_of_the_fused_expert_layer_forms():
         ("rotate_expert_a8", dict(M=4, K=256, hand_over="fp8")),
         ("rotate_expert_a8", dict(M=4, K=256, routing="scatter", top_k=65, experts=128)),
         ("router_topk", dict(M=8, E=64, top_k=4, quantize_hidden=100)),
+        ("router_topk", dict(M=8, E=64, top_k=4, metadata=True)),                                 # goes with the quantiser
+        ("router_topk", dict(M=65, E=64, top_k=4, quantize_hidden=256, metadata=True)),
+        ("router_topk", dict(M=64, E=64, top_k=17, quantize_hidden=256, metadata=True)),
+        ("router_topk", dict(M=8, E=513, top_k=4, quantize_hidden=256, metadata=True)),
+        ("router_topk", dict(M=8, E=64, top_k=4, quantize_hidden=256, metadata=True, block_m=24)),
     )
     for symbol, variant in refused:
         with pytest.raises(lib.OrxError) as err:

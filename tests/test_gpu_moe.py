@@ -1260,7 +1260,8 @@ def test_orders_for_many_rows_give_the_same_bits(tokens, experts, inter, five, b
     (40, 2, 2, 384, 256),                             # 40 rows to an expert: a full tile and one of eight rows
     (17, 1, 1, 640, 128), (9, 1, 1, 1280, 384),       # one expert, tiles of 17 and 9 rows
     (85, 32, 8, 1920, 1280), (30, 8, 4, 4096, 1536),  # long rows of down; the widest
-    (150, 64, 2, 1152, 144 * 8)])
+    (150, 64, 2, 1152, 144 * 8),
+    (33, 100, 4, 256, 128), (16, 200, 8, 128, 128), (64, 300, 4, 128, 128)])  # routes and metadata in one launch, two to eight keys to a lane
 def test_few_rows_give_the_bits_of_seven_launches(tokens, experts, top_k, hidden, inter):
     """Five launches over 32-row tiles where the resident kernel does not apply, eagerly and replayed; gates that leave fp16 among the values."""
     c = workloads.config3(tokens=tokens, experts=experts, top_k=top_k, hidden=hidden, intermediate=inter)
@@ -1272,6 +1273,10 @@ def test_few_rows_give_the_bits_of_seven_launches(tokens, experts, top_k, hidden
     x, logits = gu.dev(c["x"]), gu.dev(c["logits"])
     want = gu.host(seven.run(x, logits))
     np.testing.assert_array_equal(gu.host(few.run(x, logits)), want)
+    for name in ("ids", "prob", "counts", "relative", "row_offsets", "slot_map", "tile_count", "tile_offsets"):
+        np.testing.assert_array_equal(gu.host(getattr(few, name)), gu.host(getattr(seven, name)), err_msg=name)
+    tiles = int(few.tile_count[0])
+    assert torch.equal(few.tile_expert[:tiles], seven.tile_expert[:tiles]) and torch.equal(few.tile_row[:tiles], seven.tile_row[:tiles])
     stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
     gu.sync()
     with torch.cuda.graph(graph, stream=stream):
