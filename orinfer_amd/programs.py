@@ -132,9 +132,8 @@ class QuantizedLinear:
         self.over_panels = [False] * (top + 1)
         if algorithm == "auto" and not block_m and self.k % 128 == 0 and 256 <= self.k <= 32768 and self.n * self.k < 2**31:
             pays = panels_pay if codec == "q4" else int8_panels_pay
-            cus = torch.cuda.get_device_properties(self.weight.device).multi_processor_count
+            cus = self.cus = torch.cuda.get_device_properties(self.weight.device).multi_processor_count
             self.over_panels = [pays(rows, self.n, self.k, cus) for rows in range(top + 1)]
-            self.over_tiles = [tiles_pay(codec, rows, self.n, self.k, cus) for rows in range(top + 1)]
         # (both copies in one allocation: a second one, new from the driver, took 2 ms of a construction)
         padded = (top + 15) // 16 * 16 if any(self.over_panels) else 0
         codes = torch.empty((capacity + padded, self.k), dtype=torch.int8, device="cuda")
@@ -196,7 +195,7 @@ class QuantizedLinear:
             self.single(stream=stream, A=x16, AS=self.a_s, Book=self.book, Out=self.out, Q=self.a_q, S=self.scales, W=self.weight)
             return self._rows(1)
         rows = x16.shape[0]
-        if rows < len(self.over_panels) and self.over_panels[rows] and not self.over_tiles[rows]:
+        if rows < len(self.over_panels) and self.over_panels[rows] and not tiles_pay(self.codec, rows, self.n, self.k, self.cus):
             self.panel_quantizer(stream=stream, Mask=None, Panels=self.panels, Q=self.a_q, S=self.a_s, Sums=self.sums, X=x16, rows=rows)
             if self.codec == "q4":
                 self.panel_projection(stream=stream, A=self.panels, AS=self.a_s, Book=self.book, Out=self.out, S=self.scales, Sums=self.sums,
