@@ -1059,6 +1059,9 @@ int mid_parts(const orx_function& f, int rows) {
     return best;
 }
 
+// (A query asks for the limits of the kernel that the reported geometry, and so a record's block, is of.)
+int mid_parts_to_launch(const orx_function& f, int rows) { return recording_launches() ? 0 : mid_parts(f, rows); }
+
 uint64_t projection_workspace(const orx_function& f, int rows) {
     const int parts = mid_parts(f, rows);
     if (parts == 0) return workspace_without_mid(f, rows);
@@ -1176,7 +1179,7 @@ int q4_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t st
         }
         return ORX_OK;
     }
-    if (const int parts = mid_parts(f, rows)) {
+    if (const int parts = mid_parts_to_launch(f, rows)) {
         const int code = q4_expand_launch(p.w, p.book, workspace, f.N, f.K, f.packed_k, stream);
         if (code != ORX_OK) return code;
         return gemm_mid_launch(p.a, workspace, p.ws, p.as, p.out, rows, f.N, f.K, f.stride, f.out_f32, parts,
@@ -1220,7 +1223,7 @@ int w8_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t st
         }
         return ORX_OK;
     }
-    if (const int parts = mid_parts(f, rows))
+    if (const int parts = mid_parts_to_launch(f, rows))
         return gemm_mid_launch(p.a, p.w, p.ws, p.as, p.out, rows, f.N, f.K, f.stride, f.out_f32, parts, static_cast<int*>(workspace), stream);
     if (use_big(f, rows)) return int8_big_launch(f, rows, g, stream, p, p.w, workspace);
     if (use_split(f, rows)) {

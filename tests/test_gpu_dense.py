@@ -607,6 +607,8 @@ def test_tiles_of_128_by_128(codec, m, n, k, dtype, pad, parts):
     if torch.cuda.get_device_properties(0).multi_processor_count == 256:
         tiles = -(-m // 128) * -(-n // 128)
         assert kern.workspace_bytes(m) == (n * k if codec == "q4" else 0) + (tiles * parts * 65536 if parts > 1 else 0)
+    threads, _ = kern.query(m)
+    assert threads == np.prod(kern.geometry(m)[1])  # a record names the reported block
     want = orc.project(a, a_s, weights, scales, out_dtype=np.float16 if dtype == "float16" else np.float32)
     flat = torch.full(((m + 1) * stride + 1,), 9.0, dtype=torch.float16 if dtype == "float16" else torch.float32, device=gu.DEV)
     for shift in (0, 1):
