@@ -31,6 +31,7 @@ int gemv_configure(orx_function* f, int codec, int passes_override);
 int gemv_prepare_device();
 bool gemv_serves_k_major(const orx_function& f, int rows);
 bool gemv_serves_fp16_input(const orx_function& f);
+int gemv_replicated_lanes(const orx_function& f);
 // from k_stream.hip
 void stream_geometry(int n, Geometry* g);
 int stream_launch(int codec, const int8_t* a, const void* w, const uint32_t* book, const __half* ws, const __half* as,
@@ -826,6 +827,24 @@ bool use_runs(const orx_function& f, int rows) {
     return (f.flags2 & kNoSplit) == 0 && runs_for_many_rows(f, rows);
 }
 
+// One row of codes in the channel runs: where the GEMV has no replicated tables (K-major not even the compact ones: the streaming kernel), or only eight lanes to a
+// K-major channel, and the matrix gives a CU one block of 16 channels.  Time of A8 and projection, runs / before, 140 shapes of 256 CUs, weights out of cache:
+//   none, one block K = 2176 / 3200 / 5376 / 8448 / 13952 0.96-1.03 / 0.87-0.95 / 0.79-0.86 / 0.62-0.77 / 0.62-0.70 (3904 x 8448 14.5 -> 10.9 us, K-major 1392 x 13952 17.4 -> 11.8); two blocks up to
+//     K = 7424 0.94-1.16, from 8448 on 0.81-0.99; three K = 3328 / 4224 / 6528 / 10368 1.01 / 0.95 / 0.86 / 0.79; four 0.96-1.24; five K = 4352 / 5888 / 7424 1.01 / 0.96 / 0.91;
+//   eight lanes, one block K = 2304 / 5888 / 11520 0.80-0.89 / 0.66 / 0.57; two K = 2304 / 3328 / 9984 0.93-0.97 / 0.9-0.93 / 0.73-0.77; three K = 3328 / 4352 / 9984 1.02 / 0.97 / 0.87; five 1.02-1.21;
+//   sixteen, one block K = 2560 / 6656 / 15872 0.82-0.85 (1.03 behind a norm in a graph) / 0.82-0.94 / 0.76-0.84 (5632 and 6144 0.86-0.99), two 0.91-1.14, more 1.03-1.45; thirty-two 1.02-1.41 (6144 0.84-0.98).
+// The reported geometry is that of the kernel before, as a record of a launch names it.
+bool runs_for_one_row(const orx_function& f) {
+    if (f.flags != kQ4 || f.algorithm != kAuto || f.input_f16 || tile_for(f, 1) != 0 || (f.flags2 & (kPreferGemv | kNoGemv)) || recording_launches() ||
+        f.K % kBK != 0 || !runs_eligible(kQ4, 1, f.N, f.K))
+        return false;
+    const int blocks = channel_blocks_per_cu(f.N), lanes = gemv_replicated_lanes(f);
+    if (lanes == 32 || blocks == 4 || blocks > 5) return false;
+    if (lanes == 16) return blocks == 1 && f.K >= 3584;
+    if (lanes == 8) return f.K >= (blocks == 1 ? 2304 : blocks == 2 ? 3072 : 4096) && blocks <= 3;
+    return f.K >= (blocks == 1 ? 2816 : blocks == 2 ? 8192 : blocks == 3 ? 4096 : 5632);
+}
+
 // Channel runs per CU over the whole K (k_wide.hip): two-stage codes, `algorithm=wide` by name, and by
 // `auto` at 65..128 rows while K is short enough.  Its time is 10 us + 0.4..0.55 us per K step of 128 whatever
 // N is (up to 96 channels per CU), where the split 128 x 128 tiles pay for N K: measured at 65-128 rows,
@@ -1152,7 +1171,7 @@ int q4_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t st
     p.w = pointer_arg<const void>(args, next);
     void* workspace = f.takes_workspace ? pointer_arg<void>(args, f.workspace_arg) : nullptr;
     p.n = f.N, p.k = f.K, p.stride = f.stride, p.m = rows, p.packed_k = f.packed_k, p.out_f32 = f.out_f32;
-    if (use_runs(f, rows))
+    if (use_runs(f, rows) || (rows == 1 && runs_for_one_row(f)))
         return runs_launch(kQ4, p.a, p.w, p.book, p.ws, p.as, p.out, rows, f.N, f.K, f.stride, f.packed_k, f.out_f32, stream);
     if (use_wide(f, rows))
         return dense_wide_launch(p.a, p.w, p.book, p.ws, p.as, p.out, rows, f.N, f.K, f.stride, f.packed_k, f.out_f32, g, stream);

@@ -1339,6 +1339,12 @@ bool gemv_serves_k_major(const orx_function& f, int rows) {
     return f.flags == kQ4 && (f.packed_k == 128 || f.packed_k == 64) && ((uint32_t)f.slots >> 8) >= (uint32_t)kKMajorLayout && use_banked(f, mr_for(rows));
 }
 
+// Lanes to a channel of the replicated-table kernel at one row, 0 where the compact-table kernel or none serves it.
+int gemv_replicated_lanes(const orx_function& f) {
+    if (!use_banked(f, 1) || (f.packed_k != 0 && !gemv_serves_k_major(f, 1))) return 0;
+    return (int)(((uint32_t)f.slots >> 8) & (uint32_t)(kKMajorLayout - 1));
+}
+
 // Launchers used by the projection factories.  Argument order is the caller's business:
 // they pass already-unmarshalled pointers.
 int gemv_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t stream, const int8_t* a,

@@ -130,9 +130,9 @@ class QuantizedLinear:
         # rows over panels: the quantiser leaves the int8 rows a second time, in the order of the matrix operands
         top = min(capacity, PANEL_ROWS)
         self.over_panels = [False] * (top + 1)
+        cus = self.cus = torch.cuda.get_device_properties(self.weight.device).multi_processor_count
         if algorithm == "auto" and not block_m and self.k % 128 == 0 and 256 <= self.k <= 32768 and self.n * self.k < 2**31:
             pays = panels_pay if codec == "q4" else int8_panels_pay
-            cus = self.cus = torch.cuda.get_device_properties(self.weight.device).multi_processor_count
             self.over_panels = [pays(rows, self.n, self.k, cus) for rows in range(top + 1)]
         # (both copies in one allocation: a second one, new from the driver, took 2 ms of a construction)
         padded = (top + 15) // 16 * 16 if any(self.over_panels) else 0
@@ -159,8 +159,11 @@ class QuantizedLinear:
             self.projection = Kernel("int8_projection", **variant)
         # one row of two-stage codes, where the GEMV serves the shape: it quantises the fp16 row itself, one launch instead of two
         # (9728 x 2560: 8.7 -> 6.4 us)
+        # (K-major codes of K = 512 i + 256 and at most 16 channels to a CU are as fast in two from K = 3072 on: 1392 x 3328 / 4352 / 5888 / 7424 7.8 / 8.9 / 11.0 / 12.4 us
+        # in one, 7.3 / 7.8 / 8.4 / 9.2 in two)
         self.single = None
-        if codec == "q4" and algorithm in ("auto", "gemv") and not block_m:
+        two_are_faster = algorithm == "auto" and packed_k and self.k % 512 == 256 and self.k >= 3072 and self.n <= 16 * cus
+        if codec == "q4" and algorithm in ("auto", "gemv") and not block_m and not two_are_faster:
             try:
                 self.single = Kernel("e8p_q4_projection", M=1, N=self.n, K=self.k, algorithm=algorithm, packed_k=packed_k,
                                      input_dtype="float16", codes=True)

@@ -619,6 +619,30 @@ def test_tiles_of_128_by_128(codec, m, n, k, dtype, pad, parts):
         assert (out[m] == 9).all() and (out[:, n:] == 9).all()
 
 
+@pytest.mark.parametrize("dtype,pad", [("float16", 0), ("float32", 3)])
+@pytest.mark.parametrize("packed_k,n,k", [
+    (0, 1, 2816), (0, 4096, 2816), (0, 4099, 8320), (0, 8208, 4224), (0, 40, 3584), (0, 16400, 5760),  # no tables, 16 lanes; one to five blocks
+    (128, 33, 2304), (128, 4112, 3328), (128, 8208, 4352), (128, 70, 3584), (128, 4096, 2944), (64, 333, 9984)])
+def test_one_row_of_codes_in_the_channel_runs(packed_k, n, k, dtype, pad):
+    """At the edges of the rule; the record of the kernel before still launches, and nothing beyond the row is written."""
+    rng = np.random.default_rng(orc.SEED + n + k)
+    packed = rng.integers(0, 2**32, (n, k // 8), dtype=np.uint32)
+    a = rng.integers(-127, 128, (1, k), dtype=np.int8)
+    a_s, scales = rng.uniform(0.01, 0.03, 1).astype(np.float16), rng.uniform(0.005, 0.02, n).astype(np.float16)
+    stored = gu.dev(codebook.q4_to_k_major(packed, packed_k) if packed_k else packed)
+    want = orc.project(a, a_s, orc.q4_integers(packed, TABLE), scales, out_dtype=np.float16 if dtype == "float16" else np.float32)
+    for rows in (1, 4):  # a handle of one row, and one that serves several
+        variant = dict(M=rows, N=n, K=k, packed_k=packed_k, output_dtype=dtype, output_stride=n + pad, dynamic_rows=rows > 1)
+        kern = gu.lib.Kernel("e8p_q4_projection", **variant)
+        out = torch.full((2, n + pad), 9.0, dtype=torch.float16 if dtype == "float16" else torch.float32, device=gu.DEV)
+        kern(A=gu.dev(a), AS=gu.dev(a_s), Book=gu.book(), Out=out, S=gu.dev(scales), W=stored, **({"m": 1} if rows > 1 else {}))
+        got = gu.host(out)
+        np.testing.assert_array_equal(got[:1, :n], want)
+        assert (got[0, n:] == 9).all() and (got[1] == 9).all()
+        threads, _ = kern.query(1)
+        assert threads == np.prod(kern.geometry(1)[1])
+
+
 @pytest.mark.parametrize("packed_k", [128, 64])
 def test_split_launches_serve_k_major_codes_and_dynamic_rows(packed_k):
     rng = np.random.default_rng(orc.SEED + 91)
