@@ -28,6 +28,7 @@
 // A workgroup that takes 2, 4 or 8 spans of a tile in a row, the next one's chunks requested in the last steps, and 512
 // persistent workgroups of this form with even shares both measured level or slower (whole layer 227 / 241 / 247 and 243 against
 // 226 us): what the set-up saves, the uneven ends lose.
+//  * Units of 128 channels where those of 256 leave CUs without one (grouped_bulk_narrow): a wave has two blocks of 16 channels instead of four.
 //  * SWIGLU: a wave owns 32 gate and the 32 matching up channels, so gate and up of one (slot, channel) meet in one
 //    lane; the epilogue writes fp16(silu(gate) * up) and, where asked, gate | up and the slots' largest magnitudes.
 #include <hip/hip_fp16.h>
@@ -47,7 +48,9 @@ using namespace lds_asm;
 
 constexpr int kThreads = 256;
 constexpr int kTileRows = 128;
-constexpr int kSpan = 256;  // output channels of a unit (SWIGLU: 128 gate + 128 up)
+// Output channels of a unit of waves with CB blocks of 16 channels (SWIGLU: half of them gate, half up).
+constexpr int span_of(int cb) { return 64 * cb; }
+constexpr int kSpan = span_of(4);
 constexpr uint32_t kTokens = kPairedTableBytes;
 constexpr uint32_t kTokenBytes = 2 * kTileRows * 128;  // two chunks of 128 rows, four of 64
 constexpr uint32_t kTokenScale = kTokens + kTokenBytes;
@@ -80,7 +83,7 @@ __device__ __forceinline__ void wait_requests() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(COUNT) : "memory");
 }
 
-template <bool GATHER, bool SWIGLU>
+template <bool GATHER, bool SWIGLU, int CB>
 __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p) {
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -111,24 +114,26 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
 
     // ---- this wave's channels: plain n0 .. n0 + 63; SWIGLU gate n0 .. n0 + 31 and up inner + n0 .. ----
     const int group = span * 4 + wave;
-    const int limit = SWIGLU ? inner / 32 : p.n / 64;
+    constexpr int kOwn = 16 * CB, kHalf = SWIGLU ? kOwn / 2 : kOwn;  // channels of a wave, and beside each other
+    const int limit = SWIGLU ? inner / kHalf : p.n / kOwn;
     const bool live_wave = group < limit;  // the others help with the token rows
-    const int n0 = (live_wave ? group : 0) * (SWIGLU ? 32 : 64);
+    const int n0 = (live_wave ? group : 0) * kHalf;
     const uint8_t* const codes_base = uniform_pointer(p.w + (int64_t)expert * p.n * (p.k / 4));
     const uint32_t chunk_stride = (uint32_t)p.n * 32;
     const uint32_t code_offset = (uint32_t)(n0 + (lane & 15)) * 32 + (uint32_t)(lane >> 4) * 8;
-    const uint32_t code_offset_up = code_offset + (SWIGLU ? (uint32_t)inner * 32 : 1024u);
+    const uint32_t code_offset_up = code_offset + (SWIGLU ? (uint32_t)inner * 32 : CB * 256u);
     const int8_t* const a_base = uniform_pointer(p.a);
 
     auto run = [&](auto blocks_tag) {
         constexpr int NB = decltype(blocks_tag)::value;  // 16-row blocks
         constexpr int LOADS = NB / 2;                    // 16 NB rows are 2 NB requests of 8 rows, over four waves
         constexpr int PHASES = NB >= 4 ? 4 : 1;          // a step of 64 in phases of RB row blocks,
-        constexpr int RB = NB / PHASES, LB = 4 / PHASES; // each looking up LB of the next step's four weight blocks
+        constexpr int RB = NB / PHASES;                  // each looking up LB of the next step's CB weight blocks, while there are any
+        constexpr int LB = CB > PHASES ? CB / PHASES : 1;
         constexpr int DEPTH = NB == 8 ? 2 : 4;           // chunks in LDS and in code registers
         static_assert(DEPTH * NB * 16 * 128 <= kTokenBytes, "the chunks fit");
         constexpr uint32_t SLOT = NB * 16 * 128;
-        constexpr int kChunkRequests = 4 + LOADS;
+        constexpr int kChunkRequests = CB + LOADS;
         // ---- token rows: request b of this wave brings rows 8 (LOADS wave + b) .. +7 of a chunk, 128 bytes each.  The
         // quarter q of a wave multiplies K bytes [32 q, +32) of a chunk in two steps of 16, so piece c = 2 q + s of row r sits
         // at position (q + 4 s) ^ swizzle(r): a fragment read touches four neighbouring positions of 16 rows ----
@@ -140,21 +145,24 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
             const int* const tokens_of = uniform_pointer(p.slot_token);
             Each<LOADS + 1>::run([&](auto i) { load_4(slot_of[i], slot_of[i] * 4, tokens_of); });
         }
-        // DEPTH register sets of codes, chunk c in set c % DEPTH: four blocks of 16 channels, 8 bytes to a lane
-        v2u codes[DEPTH][4];
-        Each<DEPTH>::run([&](auto set) { Each<4>::run([&](auto j) { anything(codes[set][j]); }); });  // (anything, but in a register)
+        // DEPTH register sets of codes, chunk c in set c % DEPTH: CB blocks of 16 channels, 8 bytes to a lane
+        v2u codes[DEPTH][CB];
+        Each<DEPTH>::run([&](auto set) { Each<CB>::run([&](auto j) { anything(codes[set][j]); }); });  // (anything, but in a register)
         // Chunks that do not exist are requested by no lane where waits behind them count requests, else not at all.
         std::true_type counted;
         std::bool_constant<(DEPTH > 2)> counted_in_loop;
         auto issue_codes = [&](int chunk, auto set_tag, auto counted_tag) {
-            load_8_of_four<decltype(counted_tag)::value>(codes[decltype(set_tag)::value], code_offset, code_offset_up, codes_base + (uint64_t)chunk * chunk_stride, chunk, chunks);
+            auto& set = codes[decltype(set_tag)::value];
+            const uint8_t* const base = codes_base + (uint64_t)chunk * chunk_stride;
+            if constexpr (CB == 4) load_8_of_four<decltype(counted_tag)::value>(set, code_offset, code_offset_up, base, chunk, chunks);
+            else load_8_of_two<decltype(counted_tag)::value>(set, code_offset, code_offset_up, base, chunk, chunks);
         };
         std::integral_constant<int, 0> zero;
         std::integral_constant<int, 1> one;
         issue_codes(0, zero, counted);  // two chunks' are on their way while the rows' tokens are looked up
         issue_codes(1, one, counted);
         if constexpr (GATHER) {
-            wait_requests<8>();
+            wait_requests<2 * CB>();
             Each<LOADS + 1>::run([&](auto i) { keep(slot_of[i]); });
         }
         uint32_t row_offset[LOADS];
@@ -169,11 +177,11 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
             const int8_t* const base = a_base + (int64_t)chunk * 128 - 4096;
             request_rows_16<LOADS, decltype(counted_tag)::value>(row_offset, base, token_slots + (uint32_t)slot * SLOT, chunk, chunks);
         };
-        // scales of the tile's rows and of this wave's channels (channel `lane`, in the order of its four blocks), waited for by hand like all that follows
+        // scales of the tile's rows and of this wave's channels (in the order of its blocks), waited for by hand like all that follows
         uint32_t token_scale_bits, channel_scale_bits;
         {
             const uint64_t of_row = reinterpret_cast<uint64_t>(p.as + slot_of[LOADS]);
-            const int channel = SWIGLU && lane >= 32 ? inner + n0 + lane - 32 : n0 + lane;
+            const int own = lane & (kOwn - 1), channel = own >= kHalf ? inner + n0 + own - kHalf : n0 + own;
             const uint64_t of_channel = reinterpret_cast<uint64_t>(p.ws + (int64_t)expert * p.n + channel);
             asm volatile("global_load_ushort %0, %1, off" : "=v"(token_scale_bits) : "v"(of_row) : "memory");
             asm volatile("global_load_ushort %0, %1, off" : "=v"(channel_scale_bits) : "v"(of_channel) : "memory");
@@ -193,11 +201,11 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
         if (tid < kTileRows) reinterpret_cast<float*>(lds + kTokenScale)[tid] = __half2float(__ushort_as_half((unsigned short)token_scale_bits));
         reinterpret_cast<float*>(lds + kChannelScale)[tid] = __half2float(__ushort_as_half((unsigned short)channel_scale_bits));
 
-        v4i acc[NB][4];
+        v4i acc[NB][CB];
 #pragma unroll
         for (int i = 0; i < NB; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = v4i{0, 0, 0, 0};
+            for (int j = 0; j < CB; ++j) acc[i][j] = v4i{0, 0, 0, 0};
 
         // ---- LDS reads ----
         const uint32_t lds_base = lds_address_of(lds);
@@ -227,29 +235,30 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
 #pragma unroll
             for (int i = 0; i < RB; ++i) asm volatile("" : "+v"(token[0][i]), "+v"(token[1][i]));
         };
-        v4i weight[2][4];  // of a chunk's two steps
+        v4i weight[2][CB];  // of a chunk's two steps
         // Phase PHASE of step STEP: its multiplies (one operand changing between consecutive ones), and behind the first of them
         // the fragments of the phase after it and LB blocks of the next step's codes; all of these have come when it ends.
-        auto phase = [&](auto step_tag, auto phase_tag, auto next_slot, uint32_t next_fragments, const v2u(&next_codes)[4], auto requests) {
+        auto phase = [&](auto step_tag, auto phase_tag, auto next_slot, uint32_t next_fragments, const v2u(&next_codes)[CB], auto requests) {
             constexpr int STEP = decltype(step_tag)::value, PHASE = decltype(phase_tag)::value;
             constexpr int NEXT = (PHASE + 1) % PHASES, TOKENS = (STEP * PHASES + PHASE) & 1;
+            constexpr bool LOOKS = PHASE * LB < CB;
 #pragma unroll
             for (int i = 0; i < RB; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int jj = (i & 1) ? 3 - j : j;
+                for (int j = 0; j < CB; ++j) {
+                    const int jj = (i & 1) ? CB - 1 - j : j;
                     v4i& sum = acc[PHASE * RB + i][jj];
                     sum = __builtin_amdgcn_mfma_i32_16x16x64_i8(weight[STEP][jj], token[TOKENS][i], sum, 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
                     if (i == 0 && j == 0) read_tokens(std::integral_constant<int, NEXT>{}, std::integral_constant<int, 1 - TOKENS>{}, next_slot, next_fragments);
-                    if (i == 0 && j >= 1 && j - 1 < LB) lookup(j - 1, next_codes[PHASE * LB + j - 1][1 - STEP]);
-                    if (LB == 4 && i == 1 && j == 0) lookup(3, next_codes[3][1 - STEP]);
-                    if (i == 0 && j == 3) requests();
+                    if (LOOKS && i == 0 && j >= 1 && j - 1 < LB) lookup(j - 1, next_codes[PHASE * LB + j - 1][1 - STEP]);
+                    if (LB == CB && i == 1 && j == 0) lookup(CB - 1, next_codes[CB - 1][1 - STEP]);
+                    if (i == 0 && j == CB - 1) requests();
                     __builtin_amdgcn_sched_barrier(0);
                 }
             wait_reads();
 #pragma unroll
-            for (int l = 0; l < LB; ++l) weight[1 - STEP][PHASE * LB + l] = combine(l);
+            for (int l = 0; l < (LOOKS ? LB : 0); ++l) weight[1 - STEP][PHASE * LB + l] = combine(l);
             __builtin_amdgcn_sched_barrier(0);
         };
         auto nothing = [] {};
@@ -258,10 +267,11 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
 
         // ---- prologue: chunk 0 in LDS, the weights of its first step decoded, its first fragments read ----
         wait_requests<LOADS + (DEPTH - 2) * kChunkRequests>();
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : "+v"(codes[0][0]), "+v"(codes[0][1]), "+v"(codes[0][2]), "+v"(codes[0][3])::"memory");
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        Each<CB>::run([&](auto j) { keep(codes[0][j]); });
         read_tokens(zero, zero, zero, frag);
 #pragma unroll
-        for (int j = 0; j < 4; j += 2) {  // two blocks of channels at a time
+        for (int j = 0; j < CB; j += 2) {  // two blocks of channels at a time
             v2u pair[2][2][2];
 #pragma unroll
             for (int l = 0; l < 2; ++l) tables.read<0>(pair[l][0], codes[0][j + l][0]), tables.read<1>(pair[l][1], codes[0][j + l][0]);
@@ -296,7 +306,7 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
                 phase(zero, zero, set_tag, frag_half, codes[SET], nothing);
             }
             wait_requests<(DEPTH - 2) * kChunkRequests + LOADS>();  // the codes of chunk t + 1 are older than its token rows
-            asm volatile("" : "+v"(codes[NEXT_SET][0]), "+v"(codes[NEXT_SET][1]), "+v"(codes[NEXT_SET][2]), "+v"(codes[NEXT_SET][3]));
+            Each<CB>::run([&](auto j) { keep(codes[NEXT_SET][j]); });
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (PHASES == 4) {
                 phase(one, zero, set_tag, frag_half, codes[NEXT_SET], nothing);
@@ -326,13 +336,13 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
         // the scales once, into registers: read where they are used, behind each write of a row, every value waited for an LDS read of its own
         // (13000 of the 29000 cycles of a unit of down)
         float token_scale[NB];
-        float4 channel_scale[4];
+        float4 channel_scale[CB];
 #pragma unroll
         for (int i = 0; i < NB; ++i) token_scale[i] = reinterpret_cast<const float*>(lds + kTokenScale)[i * 16 + column];
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < CB; ++j)
             channel_scale[j] = *reinterpret_cast<const float4*>(lds + kChannelScale + (wave * 64 + j * 16 + 4 * quarter) * 4);
-        constexpr int kWidth = SWIGLU ? 64 : 128, kPitch = kWidth + 16, kLanes = kWidth / 16, kRowsAtOnce = 64 / kLanes;  // bytes of a row; lanes to a row
+        constexpr int kWidth = 2 * kHalf, kPitch = kWidth + 16, kLanes = kWidth / 16, kRowsAtOnce = std::min(16, 64 / kLanes);  // bytes of a row; lanes to a row
         uint8_t* const image = lds + kTokens + wave * 8192;  // two blocks of 16 rows
         static_assert(2 * 16 * kPitch <= 8192, "the images of four waves fit where two chunks were");
         __half* const rows_out = (SWIGLU ? p.act : p.out) + (int64_t)row0 * (SWIGLU ? inner : p.n) + n0;
@@ -344,7 +354,7 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
             for (int h = 0; h < 16 / kRowsAtOnce; ++h) {
                 const int row = h * kRowsAtOnce + own / kLanes, local = i * 16 + row;
                 const uint4 piece = *reinterpret_cast<const uint4*>(from + row * kPitch + own % kLanes * 16);
-                if (local >= rows) continue;
+                if (local >= rows || own >= kLanes * kRowsAtOnce) continue;
                 __half* const to = rows_out + (int64_t)local * row_stride + own % kLanes * 8;
                 if (aligned) {
                     *reinterpret_cast<uint4*>(to) = piece;
@@ -367,13 +377,13 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_bulk_kernel(BulkParams p)
             };
             if constexpr (!SWIGLU) {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) *reinterpret_cast<uint2*>(to + j * 32) = values(j);
+                for (int j = 0; j < CB; ++j) *reinterpret_cast<uint2*>(to + j * 32) = values(j);
             } else {
                 const bool maxima = p.row_max != nullptr;
                 float amax = 0.f;
 #pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                    const uint2 gate = values(e), up = values(e + 2);
+                for (int e = 0; e < CB / 2; ++e) {
+                    const uint2 gate = values(e), up = values(e + CB / 2);
                     const uint32_t gates[2] = {gate.x, gate.y}, ups[2] = {up.x, up.y};
                     float v[4];
 #pragma unroll
@@ -417,24 +427,37 @@ bool grouped_bulk_eligible(int n, int k, int block_m, int packed_k, int64_t rows
 }
 
 void grouped_bulk_geometry(int n, int tiles, bool swiglu, Geometry* g) {
-    const uint32_t spans = swiglu ? ceil_div((uint32_t)n / 2, kSpan / 2) : ceil_div((uint32_t)n, kSpan);
+    const uint32_t spans = ceil_div((uint32_t)n, (uint32_t)kSpan);
     g->grid[0] = ceil_div((uint32_t)tiles, 8u) * 8u * spans;
     g->grid[1] = g->grid[2] = 1;
     g->block[0] = kThreads;
     g->shared = kLds;
 }
 
-int grouped_bulk_launch(const GroupedBuffers& b, int n, int k, int tiles, bool gather, bool swiglu, hipStream_t stream) {
+// Units of 128 channels: where units of 256 (by what the routed rows of `experts` come to, half a tile each beyond whole ones) leave CUs without one, as a unit of few blocks takes
+// as long per step of K whatever the others do.  One to a CU is bound by the chain of a step (reads of LDS, multiplies): 128 x 3200 channels and K 22 us, 256 channels 32; deeper requests
+// (three chunks of 128 rows, 80 KiB of LDS) and phases of eight and sixteen multiplies measured within 3 % of it.  gate | up, us, 256 / 128 channels: 2185 tokens of 16 experts
+// x top-2, 3200 x 384 31.6 / 22.6; 800 tokens 32.0 / 22.0; 3493 of 128 x 2, 2560 x 256 29.0 / 24.1; with both projections the layer 1500 of 16 x 2, 2048 x 1024 (248 units, the most
+// there are) 62.4 / 60.5-63.5, 600 of 32 x 4, 1280 x 512 46.7 / 38.8, 500 of 16 x 8, 4096 x 256 77.5 / 65.1.  The reported geometry is that of the units of 256, as a record of
+// a launch names it.
+bool grouped_bulk_narrow(int64_t rows, int experts, int n) {
+    return (rows / kTileRows + experts / 2) * ceil_div((uint32_t)n, (uint32_t)kSpan) <= device_compute_units();
+}
+
+template <bool GATHER, bool SWIGLU>
+const void* bulk_kernel(bool narrow) {
+    return narrow ? reinterpret_cast<const void*>(&grouped_bulk_kernel<GATHER, SWIGLU, 2>) : reinterpret_cast<const void*>(&grouped_bulk_kernel<GATHER, SWIGLU, 4>);
+}
+
+int grouped_bulk_launch(const GroupedBuffers& b, int n, int k, int tiles, bool gather, bool swiglu, bool narrow, hipStream_t stream) {
     static DeviceOnce opted_in;  // dynamic LDS above 64 KiB needs an opt-in per kernel and device
     const int ready = opted_in.run([] {
-        for (const void* kernel : {reinterpret_cast<const void*>(&grouped_bulk_kernel<false, false>),
-                                   reinterpret_cast<const void*>(&grouped_bulk_kernel<true, false>),
-                                   reinterpret_cast<const void*>(&grouped_bulk_kernel<false, true>),
-                                   reinterpret_cast<const void*>(&grouped_bulk_kernel<true, true>)}) {
-            const int code = hip_check(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds),
-                                       "hipFuncSetAttribute");
-            if (code != ORX_OK) return code;
-        }
+        for (const bool of_128 : {false, true})
+            for (const void* kernel : {bulk_kernel<false, false>(of_128), bulk_kernel<true, false>(of_128), bulk_kernel<false, true>(of_128), bulk_kernel<true, true>(of_128)}) {
+                const int code = hip_check(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds),
+                                           "hipFuncSetAttribute");
+                if (code != ORX_OK) return code;
+            }
         return (int)ORX_OK;
     });
     if (ready != ORX_OK) return ready;
@@ -448,16 +471,18 @@ int grouped_bulk_launch(const GroupedBuffers& b, int n, int k, int tiles, bool g
     p.counts = b.counts, p.offsets = b.offsets, p.tile_expert = b.tile_expert, p.tile_row = b.tile_row;
     p.tile_count = b.tile_count, p.tile_units = static_cast<const int4*>(b.tile_units);
     p.n = n, p.k = k, p.tile_capacity = tiles;
-    p.spans = (int)(swiglu ? ceil_div((uint32_t)n / 2, kSpan / 2) : ceil_div((uint32_t)n, kSpan));
-    const dim3 grid(g.grid[0]), block(kThreads);
-    if (gather && swiglu)
-        ORX_LAUNCH((grouped_bulk_kernel<true, true>), grid, block, g.shared, stream, p);
-    else if (gather)
-        ORX_LAUNCH((grouped_bulk_kernel<true, false>), grid, block, g.shared, stream, p);
-    else if (swiglu)
-        ORX_LAUNCH((grouped_bulk_kernel<false, true>), grid, block, g.shared, stream, p);
-    else
-        ORX_LAUNCH((grouped_bulk_kernel<false, false>), grid, block, g.shared, stream, p);
+    p.spans = (int)ceil_div((uint32_t)n, (uint32_t)span_of(narrow ? 2 : 4));
+    const dim3 grid(ceil_div((uint32_t)tiles, 8u) * 8u * (uint32_t)p.spans), block(kThreads);
+#define ORX_BULK(GATHER, SWIGLU)                                                                           \
+    {                                                                                                      \
+        if (narrow) ORX_LAUNCH((grouped_bulk_kernel<GATHER, SWIGLU, 2>), grid, block, g.shared, stream, p); \
+        else ORX_LAUNCH((grouped_bulk_kernel<GATHER, SWIGLU, 4>), grid, block, g.shared, stream, p);        \
+    }
+    if (gather && swiglu) ORX_BULK(true, true)
+    else if (gather) ORX_BULK(true, false)
+    else if (swiglu) ORX_BULK(false, true)
+    else ORX_BULK(false, false)
+#undef ORX_BULK
     return hip_check(hipGetLastError(), "launch routed projection (bulk)");
 }
 

@@ -69,7 +69,8 @@ int grouped_resident_launch(const GroupedBuffers& b, int n, int k, int tiles, in
                             int slots, hipStream_t stream);
 bool grouped_bulk_eligible(int n, int k, int block_m, int packed_k, int64_t rows);
 void grouped_bulk_geometry(int n, int tiles, bool swiglu, Geometry* g);
-int grouped_bulk_launch(const GroupedBuffers& b, int n, int k, int tiles, bool gather, bool swiglu, hipStream_t stream);
+bool grouped_bulk_narrow(int64_t rows, int experts, int n);
+int grouped_bulk_launch(const GroupedBuffers& b, int n, int k, int tiles, bool gather, bool swiglu, bool narrow, hipStream_t stream);
 int make_few_rows(const Variant& v, orx_function* f);  // k_few.hip
 // from k_mid.hip
 int gemm_mid_launch(const int8_t* a, const void* w, const __half* ws, const __half* as, void* out, int rows, int n, int k, int stride, bool out_f32, int parts,
@@ -1883,7 +1884,7 @@ int grouped_launch(const orx_function& f, int rows, const Geometry& g, hipStream
     b.row_max = reinterpret_cast<const int*>(buffer("RowMax")), b.act = buffer("Act"), b.q = buffer("Q");
     b.tile_units = buffer("TileUnits");
     if (grouped_uses_bulk(f))
-        return grouped_bulk_launch(b, f.N, f.K, f.tiles, (f.flags2 & 3) == 1, (f.flags2 >> 2) == 1, stream);
+        return grouped_bulk_launch(b, f.N, f.K, f.tiles, (f.flags2 & 3) == 1, (f.flags2 >> 2) == 1, grouped_bulk_narrow(f.capacity, f.E, f.N), stream);
     if (grouped_uses_resident(f))
         return grouped_resident_launch(b, f.N, f.K, f.tiles, f.packed_k, f.flags2 & 3, f.flags2 >> 2, f.capacity, stream);
     GemmParams p = {};

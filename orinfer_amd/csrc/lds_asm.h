@@ -127,6 +127,23 @@ __device__ __forceinline__ void load_8_of_four(v2u (&value)[4], uint32_t lane_of
                      : "memory", "scc");
 #undef ORX_LOADS
 }
+// The same of two, at both lane offsets.
+template <bool COUNTED>
+__device__ __forceinline__ void load_8_of_two(v2u (&value)[2], uint32_t lane_offset, uint32_t other_offset, const void* uniform_base, int index, int count) {
+    uint64_t all;
+#define ORX_LOADS "global_load_dwordx2 %0, %3, %5\n\tglobal_load_dwordx2 %1, %4, %5\n\t"
+    if constexpr (COUNTED)
+        asm volatile(ORX_BELOW_OR_EMPTY("%6", "%7", "%2", ORX_LOADS)
+                     : "+v"(value[0]), "+v"(value[1]), "=&s"(all)
+                     : "v"(lane_offset), "v"(other_offset), "s"(uniform_base), "s"(index), "s"(count)
+                     : "memory", "scc");
+    else
+        asm volatile(ORX_BELOW_OR_SKIPPED("%6", "%7", ORX_LOADS)
+                     : "+v"(value[0]), "+v"(value[1]), "=&s"(all)
+                     : "v"(lane_offset), "v"(other_offset), "s"(uniform_base), "s"(index), "s"(count)
+                     : "memory", "scc");
+#undef ORX_LOADS
+}
 #undef ORX_BELOW_OR_EMPTY
 #undef ORX_BELOW_OR_SKIPPED
 __device__ __forceinline__ void load_4(uint32_t& value, uint32_t lane_offset, const void* uniform_base) {

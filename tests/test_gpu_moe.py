@@ -358,6 +358,14 @@ def test_grouped_q2_bulk_kernel_over_more_chunks_than_it_holds(n, k, counts, for
     test_grouped_q2_bulk_kernel(n, k, counts, form)
 
 
+@pytest.mark.parametrize("form", ["plain", "swiglu"])
+@pytest.mark.parametrize("n,k,counts,empty", [(128, 128, [0, 1, 16, 17, 33, 65, 0, 2], 520), (320, 384, [128, 129, 64, 0, 300, 32], 260),
+                                              (576, 256, [127, 31, 257, 5, 96], 180), (2176, 640, [48, 0, 130], 60)])
+def test_grouped_q2_bulk_kernel_with_units_of_256_channels(n, k, counts, empty, form):
+    """The experts of a list choose the channels of a unit: few ones (the tests above) 128, so many that every CU has a unit 256."""
+    test_grouped_q2_bulk_kernel(n, k, counts + [0] * empty, form)
+
+
 @pytest.mark.parametrize("swiglu", [False, True], ids=["rows", "gathered-swiglu"])
 def test_grouped_q2_bulk_kernel_takes_its_tiles_from_units(swiglu):
     """The same rows whether a tile comes out of TileExpert, TileRow, Counts and Offsets or out of TileUnits in any order."""
