@@ -218,14 +218,15 @@ BULK_ROWS_PER_EXPERT = 48
 
 
 def bulk_pays(routed, experts, hidden, intermediate, cus):
-    """Whether the order over 128-row tiles is faster than the one over tiles of 32 rows, five launches or seven (time of the layer, the latter over the former;
-    170 shapes with 10 to 70 routed rows per expert, popularity like 1 / rank^1.1, 256 CUs).  A tile of 32 rows costs a unit per 512 channels, and as long as both
-    projections together have no more than about one unit to a CU (half a tile per expert more than the rows fill), two where a unit of 256 channels reads long
-    rows, the small tiles win: 0.72-1.03.  Beyond, 24 and more rows per expert 1.01-1.67 (three in a hundred 0.98-0.99), with a uniform popularity 1.01-1.73; 16 to 24 rows of up to 64 experts
-    1.02-1.38 from 1.6 units to a CU on and 0.8-1.16 below, of 128 experts 0.83-1.51 without a line between; fewer rows 0.72-1.16."""
-    units = (routed / 32 + experts / 2) * (-(-2 * intermediate // 512) + -(-hidden // 512))
+    """Whether the order over 128-row tiles is faster than the one over tiles of 32 rows, five launches of either kind (time of the layer, the latter over the former; 600 shapes
+    with 6 to 48 routed rows per expert, popularity like 1 / rank^1.1, 256 CUs).  What counts is the small tiles' work: units of 32 rows (half a tile per expert more than the rows
+    fill) x 512 channels to a CU, those of the second projection by the length of its rows.  From 24 rows per expert and half a unit on 0.95-1.64 (median 1.2), of up to 64 experts from 16 rows
+    (32 experts: 12) and 0.7 on 0.97-1.35, of up to 32 experts with 896 and more channels between, where the small tiles of the second projection hold the fewest rows, from 7 rows and 0.4 on
+    0.96-1.33; otherwise 0.64-1.1 (of 128 experts with fewer rows 0.75-1.29 without a line between)."""
+    work = (routed / 32 + experts / 2) * (-(-2 * intermediate // 512) + -(-hidden // 512) * intermediate / hidden)
     rows = routed / experts
-    return rows >= 24 and units >= max(1.1, hidden / 1600) * cus or rows >= 16 and experts <= 64 and units >= max(1.6, hidden / 1400) * cus
+    return (rows >= 24 and work >= 0.5 * cus or experts <= 64 and rows >= (12 if experts <= 32 else 16) and work >= 0.7 * cus
+            or experts <= 32 and intermediate >= 896 and rows >= 7 and work >= 0.4 * cus)
 
 
 def one_launch_routes(tokens, top_k, experts):

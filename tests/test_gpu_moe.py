@@ -1267,7 +1267,7 @@ def test_orders_for_many_rows_give_the_same_bits(tokens, experts, inter, five, b
     (2, 16, 8, 3200, 256), (3, 4, 2, 128, 128),       # tiles of a row or two; K blocks fewer than the waves that share them
     (40, 2, 2, 384, 256),                             # 40 rows to an expert: a full tile and one of eight rows
     (17, 1, 1, 640, 128), (9, 1, 1, 1280, 384),       # one expert, tiles of 17 and 9 rows
-    (85, 32, 8, 1920, 1280), (30, 8, 4, 4096, 1536),  # long rows of down; the widest
+    (25, 32, 8, 1920, 1280), (13, 8, 4, 4096, 1536),  # long rows of down; the widest
     (150, 64, 2, 1152, 144 * 8),
     (33, 100, 4, 256, 128), (16, 200, 8, 128, 128), (64, 300, 4, 128, 128)])  # routes and metadata in one launch, two to eight keys to a lane
 def test_few_rows_give_the_bits_of_seven_launches(tokens, experts, top_k, hidden, inter):
