@@ -31,7 +31,7 @@ int gemv_configure(orx_function* f, int codec, int passes_override);
 int gemv_prepare_device();
 bool gemv_serves_k_major(const orx_function& f, int rows);
 bool gemv_serves_fp16_input(const orx_function& f);
-int gemv_replicated_lanes(const orx_function& f);
+int gemv_replicated_lanes(const orx_function& f, int rows);
 // from k_stream.hip
 void stream_geometry(int n, Geometry* g);
 int stream_launch(int codec, const int8_t* a, const void* w, const uint32_t* book, const __half* ws, const __half* as,
@@ -834,16 +834,49 @@ bool use_runs(const orx_function& f, int rows) {
 //     K = 7424 0.94-1.16, from 8448 on 0.81-0.99; three K = 3328 / 4224 / 6528 / 10368 1.01 / 0.95 / 0.86 / 0.79; four 0.96-1.24; five K = 4352 / 5888 / 7424 1.01 / 0.96 / 0.91;
 //   eight lanes, one block K = 2304 / 5888 / 11520 0.80-0.89 / 0.66 / 0.57; two K = 2304 / 3328 / 9984 0.93-0.97 / 0.9-0.93 / 0.73-0.77; three K = 3328 / 4352 / 9984 1.02 / 0.97 / 0.87; five 1.02-1.21;
 //   sixteen, one block K = 2560 / 6656 / 15872 0.82-0.85 (1.03 behind a norm in a graph) / 0.82-0.94 / 0.76-0.84 (5632 and 6144 0.86-0.99), two 0.91-1.14, more 1.03-1.45; thirty-two 1.02-1.41 (6144 0.84-0.98).
-// The reported geometry is that of the kernel before, as a record of a launch names it.
 bool runs_for_one_row(const orx_function& f) {
-    if (f.flags != kQ4 || f.algorithm != kAuto || f.input_f16 || tile_for(f, 1) != 0 || (f.flags2 & (kPreferGemv | kNoGemv)) || recording_launches() ||
-        f.K % kBK != 0 || !runs_eligible(kQ4, 1, f.N, f.K))
-        return false;
-    const int blocks = channel_blocks_per_cu(f.N), lanes = gemv_replicated_lanes(f);
-    if (lanes == 32 || blocks == 4 || blocks > 5) return false;
+    const int blocks = channel_blocks_per_cu(f.N), lanes = gemv_replicated_lanes(f, 1);
+    if (f.flags != kQ4 || lanes == 32 || blocks == 4 || blocks > 5) return false;
     if (lanes == 16) return blocks == 1 && f.K >= 3584;
     if (lanes == 8) return f.K >= (blocks == 1 ? 2304 : blocks == 2 ? 3072 : 4096) && blocks <= 3;
     return f.K >= (blocks == 1 ? 2816 : blocks == 2 ? 8192 : blocks == 3 ? 4096 : 5632);
+}
+
+// More rows in the channel runs, where use_runs leaves them to others.  Time of the projection, runs / others, 2600 shapes of 256 CUs drawn over 1024 to 34816 channels and K to 17408:
+//   codes, 2 to 32 rows: one block without the loader-wave kernel up to 16 rows K = 2816 to 3328 / 4096 0.87-0.95 / 0.84-0.9 (below 0.94-1.29), 17 rows and more from K = 2304 on
+//     0.88-0.96; two blocks up to 16 rows from K = 8192 on 0.81-0.95, more from 12288 on 0.91-0.98; three at two rows without replicated tables from K = 4096 on 0.56-0.9;
+//   codes, 65 to 128 rows in one round 0.78-0.89 from K = 2048 on; 129 to 256 in tiles of more than 120 and one round 0.56-0.94 from K = 2048 on; 257 to 384 in tiles of up to 96
+//     and two rounds 0.77-0.95 from K = 1536 on;
+//   int8, 65 to 128 rows in two and three rounds 0.44-0.91 up to K = 8192 (above 1.0); in one round 113 to 120 rows of long K 0.83-0.94.
+// The reported geometry is that of the kernel before, here and at one row, as a record of a launch names it.
+bool runs_instead(const orx_function& f, int rows) {
+    if (f.algorithm != kAuto || f.input_f16 || tile_for(f, rows) != 0 || (f.flags2 & (kPreferGemv | kNoGemv)) || recording_launches() || f.K % kBK != 0 ||
+        (f.flags != kQ4 && f.flags != kW8) || !runs_eligible(f.flags, rows, f.N, f.K))
+        return false;
+    if (rows == 1) return runs_for_one_row(f);
+    if (rows <= 32) {
+        const int blocks = channel_blocks_per_cu(f.N);
+        if (f.flags != kQ4) return false;
+        if (blocks == 1) return f.K >= (rows <= 16 ? 2816 : 2304) && !dense_loader_eligible(f.N, f.K, f.packed_k);
+        if (blocks == 2) return f.K >= (rows <= 16 ? 8192 : 12288);
+        return blocks == 3 && rows == 2 && f.K >= 4096 && gemv_replicated_lanes(f, 2) == 0;
+    }
+    if (rows <= 64 || (f.flags2 & kNoSplit)) return false;
+    int tile_rows = 0, run = 0;
+    const int rounds = runs_rounds(f.flags, rows, f.N, &tile_rows, &run);
+    if (f.flags == kW8) return rows <= 128 && (rounds == 1 ? rows <= 120 : rounds <= 3 && f.K <= 8192);
+    if (rows <= 128) return rounds == 1 && f.K >= 2048;
+    if (rows <= 256) return rounds == 1 && tile_rows > 120 && f.K >= 2048;
+    return rows <= 384 && rounds == 2 && tile_rows <= 96 && f.K >= 1536;
+}
+
+// Two to four rows of row-major codes without replicated tables: the streaming kernel where the compact-table GEMV is reported (kept as above).  From three blocks of 16 channels to a
+// CU on, streaming kernel / GEMV: 2 rows 0.73-0.99 (five blocks once 1.05), 3 and 4 rows 0.53-0.67; 23632 x 3840 at 4 rows 27.4 -> 16.0 us, 25616 x 1152 at 2 12.8 -> 8.7.
+bool use_gemv(const orx_function& f, int rows);
+bool use_stream(const orx_function& f, int rows);
+bool stream_instead(const orx_function& f, int rows) {
+    return f.flags == kQ4 && f.algorithm == kAuto && !f.input_f16 && rows > 1 && rows <= 4 && f.packed_k == 0 && !(f.flags2 & kPreferGemv) && !recording_launches() &&
+           use_gemv(f, rows) && gemv_replicated_lanes(f, rows) == 0 && use_stream(f, rows);
 }
 
 // Channel runs per CU over the whole K (k_wide.hip): two-stage codes, `algorithm=wide` by name, and by
@@ -1172,14 +1205,15 @@ int q4_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t st
     p.w = pointer_arg<const void>(args, next);
     void* workspace = f.takes_workspace ? pointer_arg<void>(args, f.workspace_arg) : nullptr;
     p.n = f.N, p.k = f.K, p.stride = f.stride, p.m = rows, p.packed_k = f.packed_k, p.out_f32 = f.out_f32;
-    if (use_runs(f, rows) || (rows == 1 && runs_for_one_row(f)))
+    if (use_runs(f, rows) || runs_instead(f, rows))
         return runs_launch(kQ4, p.a, p.w, p.book, p.ws, p.as, p.out, rows, f.N, f.K, f.stride, f.packed_k, f.out_f32, stream);
     if (use_wide(f, rows))
         return dense_wide_launch(p.a, p.w, p.book, p.ws, p.as, p.out, rows, f.N, f.K, f.stride, f.packed_k, f.out_f32, g, stream);
     if (use_tall(f, rows))
         return gemm_tall_launch(p.a, p.w, p.book, p.ws, p.as, p.out, rows, f.N, f.K, f.stride, f.packed_k, f.out_f32, g, stream);
-    if (use_gemv(f, rows)) return gemv_launch(f, rows, g, stream, p.a, p.w, p.book, p.ws, p.as, p.out, signs, codes);
-    if (use_resident(f, rows)) {
+    const bool streams = stream_instead(f, rows);
+    if (!streams && use_gemv(f, rows)) return gemv_launch(f, rows, g, stream, p.a, p.w, p.book, p.ws, p.as, p.out, signs, codes);
+    if (!streams && use_resident(f, rows)) {
         for (int first = 0; first < rows; first += 32) {
             const size_t out_offset = (size_t)first * f.stride * (f.out_f32 ? 4 : 2);
             const int code = dense_resident_launch(p.a + (size_t)first * f.K, p.w, p.book, p.ws, p.as + first,
@@ -1230,7 +1264,7 @@ int w8_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t st
     p.book = nullptr;
     void* workspace = f.takes_workspace ? pointer_arg<void>(args, f.workspace_arg) : nullptr;
     p.n = f.N, p.k = f.K, p.stride = f.stride, p.m = rows, p.packed_k = 0, p.out_f32 = f.out_f32;
-    if (use_runs(f, rows))
+    if (use_runs(f, rows) || runs_instead(f, rows))
         return runs_launch(kW8, p.a, p.w, nullptr, p.ws, p.as, p.out, rows, f.N, f.K, f.stride, 0, f.out_f32, stream);
     if (use_gemv(f, rows)) return gemv_launch(f, rows, g, stream, p.a, p.w, p.book, p.ws, p.as, p.out);
     if (use_stream(f, rows)) {

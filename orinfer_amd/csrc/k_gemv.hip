@@ -1339,9 +1339,9 @@ bool gemv_serves_k_major(const orx_function& f, int rows) {
     return f.flags == kQ4 && (f.packed_k == 128 || f.packed_k == 64) && ((uint32_t)f.slots >> 8) >= (uint32_t)kKMajorLayout && use_banked(f, mr_for(rows));
 }
 
-// Lanes to a channel of the replicated-table kernel at one row, 0 where the compact-table kernel or none serves it.
-int gemv_replicated_lanes(const orx_function& f) {
-    if (!use_banked(f, 1) || (f.packed_k != 0 && !gemv_serves_k_major(f, 1))) return 0;
+// Lanes to a channel of the replicated-table kernel at that many rows, 0 where the compact-table kernel or none serves them.
+int gemv_replicated_lanes(const orx_function& f, int rows) {
+    if (!use_banked(f, mr_for(rows)) || (f.packed_k != 0 && !gemv_serves_k_major(f, rows))) return 0;
     return (int)(((uint32_t)f.slots >> 8) & (uint32_t)(kKMajorLayout - 1));
 }
 

@@ -643,6 +643,35 @@ def test_one_row_of_codes_in_the_channel_runs(packed_k, n, k, dtype, pad):
         assert threads == np.prod(kern.geometry(1)[1])
 
 
+@pytest.mark.parametrize("codec,packed_k,rows,n,k", [
+    ("q4", 0, 2, 4096, 2816), ("q4", 128, 16, 1030, 3456), ("q4", 128, 17, 333, 2304), ("q4", 0, 32, 70, 2432),      # one block of channels to a CU
+    ("q4", 128, 16, 4112, 8192), ("q4", 0, 32, 4100, 12288), ("q4", 0, 2, 8208, 4224),                                  # two, three
+    ("q4", 0, 2, 8200, 1152), ("q4", 0, 4, 16400, 1152), ("q4", 0, 3, 20500, 1408),                                     # the streaming kernel
+    ("q4", 0, 96, 8300, 2048), ("q4", 128, 128, 4130, 2176), ("q4", 128, 247, 5904, 2304), ("q4", 64, 256, 4300, 2048), ("q4", 0, 270, 8192, 1536),
+    ("w8", 0, 65, 14960, 1152), ("w8", 0, 128, 9000, 1024), ("w8", 0, 120, 1000, 8320)])
+def test_rows_that_leave_the_reported_kernel(codec, packed_k, rows, n, k):
+    """Shapes at the edges of the rules by which a launch takes the channel runs or the streaming kernel while its records name another."""
+    rng = np.random.default_rng(orc.SEED + rows + n + k)
+    a = rng.integers(-127, 128, (rows, k), dtype=np.int8)
+    a_s, scales = rng.uniform(0.01, 0.03, rows).astype(np.float16), rng.uniform(0.005, 0.02, n).astype(np.float16)
+    out = torch.full((rows + 1, n), 9.0, dtype=torch.float16, device=gu.DEV)
+    if codec == "q4":
+        packed = rng.integers(0, 2**32, (n, k // 8), dtype=np.uint32)
+        weights = orc.q4_integers(packed, TABLE)
+        kern = gu.kernel("e8p_q4_projection", M=512, N=n, K=k, packed_k=packed_k, dynamic_rows=True)
+        kern(A=gu.dev(a), AS=gu.dev(a_s), Book=gu.book(), Out=out, S=gu.dev(scales), W=gu.dev(codebook.q4_to_k_major(packed, packed_k) if packed_k else packed),
+             Workspace=kern.workspace(), m=rows)
+    else:
+        weights = rng.integers(-127, 128, (n, k), dtype=np.int8)
+        kern = gu.kernel("int8_projection", M=512, N=n, K=k, dynamic_rows=True)
+        kern(A=gu.dev(a), Output=out, TokenScale=gu.dev(a_s), Weight=gu.dev(weights), WeightScale=gu.dev(scales), Workspace=kern.workspace(), m=rows)
+    got = gu.host(out)
+    np.testing.assert_array_equal(got[:rows], orc.project(a, a_s, weights, scales, out_dtype=np.float16))
+    assert (got[rows] == 9).all()
+    threads, _ = kern.query(rows)
+    assert threads == np.prod(kern.geometry(rows)[1])
+
+
 @pytest.mark.parametrize("packed_k", [128, 64])
 def test_split_launches_serve_k_major_codes_and_dynamic_rows(packed_k):
     rng = np.random.default_rng(orc.SEED + 91)
