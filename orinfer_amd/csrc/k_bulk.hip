@@ -6,7 +6,7 @@
 // With hundreds of rows per expert the projection is a matrix product: 4096 tokens x top-8 of 128 experts are 137 GOP in
 // gate_up and 69 GOP in down, which the 32-row tiles of the weight-streaming kernels ran at 460 TOP/s, decoding every code
 // once per 32 rows.
-//  * A unit is (tile of up to 128 slots, 256 output channels), a workgroup four waves, two workgroups to a CU, so that the
+//  * A unit is (tile of up to 128 slots, 256 output channels or, see below, 128), a workgroup four waves, two workgroups to a CU, so that the
 //    set-up and the epilogue of one run beside the K loop of the other.
 //  * A wave owns 64 channels and all rows of the tile, 8 x 4 blocks of v_mfma_i32_16x16x64_i8 (128 accumulator
 //    registers).  Its codes go from memory into registers (8 bytes per lane, block of 16 channels and 128 of K) and through

@@ -1008,7 +1008,7 @@ bool use_expand(const orx_function& f, int rows) {
 }
 
 // Split launches serve the 128-row tiles when whole tiles would not spread evenly: up to two tiles
-// per CU.  The partial slots are in the caller's Workspace.
+// per CU, and what mid_parts leaves of them: up to 128 rows, handles by name, channels beyond a persistent round.  The partial slots are in the caller's Workspace.
 // two workgroups per CU: a single workgroup of four waves leaves every load latency exposed
 int split_groups() { return 2 * device_compute_units(); }
 // 128-row tiles of this launch, and whether their count suits a split launch: measured at K = 5120
