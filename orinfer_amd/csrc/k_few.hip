@@ -1,5 +1,5 @@
 // The two routed single-stage (Q2) projections of an expert layer where the routed tiles are too few for workgroups that own 512 channels
-// (k_grouped.hip): decode batches and short prompts, any K.
+// (k_grouped.hip): decode batches and short prompts, any K whose sums int32 holds.
 //
 // Reference counterpart: the warp-owned routed decode kernels/cuda/model/e8p_decode.py:36-245 behind the tile metadata of
 // kernels/cuda/model/routing.py.  Arithmetic: exact int32 over the full K, (float(acc) * ws) * as, rounded to fp16 once; fp16(silu(gate) * up).
@@ -323,10 +323,11 @@ int make_few_rows(const Variant& v, orx_function* f) {
     const bool act = v.string("input_dtype", "int8", &bad) == "float16", gather = v.boolean("gather", false, &bad);
     const std::string epilogue = v.string("epilogue", "none", &bad), algorithm = v.string("algorithm", "auto", &bad);
     if (bad) return ORX_ERR_BAD_VARIANT;
-    if (f->M <= 0 || f->E <= 0 || f->tiles <= 0 || f->tiles > 65535 || f->N <= 0 || f->N % 32 || f->K <= 0 || f->K % 128 || f->block_m != 32 ||
-        f->packed_k != 128 || algorithm != "auto" || (act ? gather || epilogue != "none" : !gather || epilogue != "swiglu")) {
-        set_error("%s: few_rows=true serves lists of up to 65535 32-row tiles, packed_k=128, N a multiple of 32, K of 128, algorithm auto: gather=true with "
-                  "epilogue=swiglu, or input_dtype=float16", f->symbol.c_str());
+    if (f->M <= 0 || f->E <= 0 || f->tiles <= 0 || f->tiles > 65535 || f->N <= 0 || f->N % 32 || f->K <= 0 || f->K % 128 ||
+        (int64_t)f->K * 128 * 128 > 2147483647LL || f->block_m != 32 || f->packed_k != 128 || algorithm != "auto" ||
+        (act ? gather || epilogue != "none" : !gather || epilogue != "swiglu")) {
+        set_error("%s: few_rows=true serves lists of up to 65535 32-row tiles, packed_k=128, N a multiple of 32, K of 128 with K * 2^14 < 2^31, algorithm auto: gather=true "
+                  "with epilogue=swiglu, or input_dtype=float16", f->symbol.c_str());
         return ORX_ERR_BAD_VARIANT;
     }
     f->flags = act ? 1 : 0;

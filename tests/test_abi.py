@@ -519,6 +519,7 @@ def test_argument_lists_of_the_fused_expert_layer_forms():
         ("e8p_decode_grouped", dict(N=1040, K=4096, gather=True, epilogue="swiglu", **few)),
         ("e8p_decode_grouped", dict(N=1024, K=4096, input_dtype="float16", **few)),              # the fp16 rows of a tile do not fit LDS
         ("e8p_decode_grouped", dict(N=1024, K=4096, gather=True, epilogue="swiglu", algorithm="stream", **few)),
+        ("e8p_decode_grouped", dict(N=256, K=131072, gather=True, epilogue="swiglu", **few)),    # a sum of 131072 products of -128 is 2^31
         ("e8p_decode_grouped", dict(N=1024, K=2048, gather=True, rows=8200, E=128, tiles=512, block_m=32, algorithm="resident")),
         # without the SwiGLU epilogue the kernel keeps its phase-two sums in LDS, which leaves room for fewer slots
         ("e8p_decode_grouped", dict(N=1024, K=2048, gather=True, rows=8192, E=128, tiles=512, block_m=32, algorithm="resident")),
