@@ -48,7 +48,7 @@ struct FewParams {
     __half* out;            // gate | up: (slots, N / 2); down: (slots, N)
     const int4* units;      // expert, first slot, rows
     const int* tile_count;
-    int n, k;
+    int n, k, tile_rows;    // the most of a tile
     int64_t expert_stride;  // bytes of codes of an expert
 };
 
@@ -71,7 +71,8 @@ __global__ __launch_bounds__(kThreads) void few_rows_kernel(FewParams p) {
     const uint32_t selector = p.book[tid & 255];
     const int4 unit = p.units[blockIdx.y];  // (nothing there behind the last tile)
     if ((int)blockIdx.y >= p.tile_count[0]) return;
-    const int expert = unit.x, row0 = unit.y, rows = unit.z;
+    const int expert = unit.x, row0 = unit.y, rows = min(p.tile_rows, unit.z);  // (a list of taller tiles: the rows that LDS holds)
+    if (rows <= 0) return;
     const int inner = p.n / 2;
 
     // weight row of this lane (clamped: channels beyond the last are computed and not stored)
@@ -258,13 +259,16 @@ int splits_for(const orx_function& f) {
     return best;
 }
 
+// rows of a tile, for which down has LDS
+int most_rows(const orx_function& f) { return std::min(kRows, f.capacity); }
+
 int few_geometry(const orx_function& f, int, Geometry* g) {
     const bool act = f.flags & 1;
     const int channels = (kWaves / splits_for(f)) * (act ? 32 : 16);
     g->grid[0] = ceil_div((uint32_t)(act ? f.N : f.N / 2), (uint32_t)channels);
     g->grid[1] = (uint32_t)f.tiles;
     g->block[0] = kThreads;
-    g->shared = kWaves * kRegion + (uint32_t)sizeof(Q2ByteTables) + (act ? (uint32_t)std::min(kRows, f.capacity) * (f.K + kRowPad) : 0u);
+    g->shared = kWaves * kRegion + (uint32_t)sizeof(Q2ByteTables) + (act ? (uint32_t)most_rows(f) * (f.K + kRowPad) : 0u);
     return ORX_OK;
 }
 
@@ -292,7 +296,7 @@ int few_launch(const orx_function& f, int, const Geometry& g, hipStream_t stream
     p.tile_count = pointer_arg<const int>(args, next++);
     p.units = pointer_arg<const int4>(args, next++);
     p.ws = pointer_arg<const __half>(args, next++);
-    p.n = f.N, p.k = f.K, p.expert_stride = (int64_t)f.N * (f.K / 8) * 2;
+    p.n = f.N, p.k = f.K, p.tile_rows = most_rows(f), p.expert_stride = (int64_t)f.N * (f.K / 8) * 2;
     const dim3 grid(g.grid[0], g.grid[1]), block(kThreads);
 #define ORX_FEW(ACT, S) ORX_LAUNCH((few_rows_kernel<ACT, S>), grid, block, g.shared, stream, p)
     const int splits = splits_for(f);

@@ -399,6 +399,53 @@ def test_grouped_q2_bulk_kernel_takes_its_tiles_from_units(swiglu):
         gu.kernel("e8p_decode_grouped", **{**variant, "block_m": 32, "gather": False, "epilogue": "none"}, tile_units=True)
 
 
+@pytest.mark.parametrize("slots,units,written", [
+    (75, [(1, 0, 40), (0, 40, 0), (2, 41, -3), (2, 43, 7), (0, 50, 25)], [(1, 0, 32), (2, 43, 7), (0, 50, 25)]),  # taller than a tile, none, fewer than none
+    (64, [(2, 0, 64)], [(2, 0, 32)]),                                                                              # as a list of 64-row tiles has them
+    (9, [(1, 0, 32)], [(1, 0, 9)])])                                                                               # LDS for the rows that there are
+def test_few_rows_takes_no_more_of_a_unit_than_a_tile_has(slots, units, written):
+    """Lists that this kernel is not handed by the metadata of its own tile height: nothing beyond a tile's rows is staged or written."""
+    rng = np.random.default_rng(orc.SEED + slots)
+    e, hidden, inter, tokens = 3, 384, 256, 21
+    scale = lambda n, k: rng.uniform(0.5, 1.5, (e, n)).astype(np.float16) * np.float16(0.05 / np.sqrt(k))
+    codes = {n: rng.integers(0, 65536, (e, n, k // 8), dtype=np.uint16) for n, k in ((2 * inter, hidden), (hidden, inter))}
+    stored = {n: gu.dev(np.stack([orc.q2_pack_k128(one) for one in c])) for n, c in codes.items()}
+    w1, w2 = (np.stack([orc.q2_integers(one, TABLE) for one in codes[n]]) for n in (2 * inter, hidden))
+    s1, s2 = scale(2 * inter, hidden), scale(hidden, inter)
+    a_q, a_s = rng.integers(-127, 128, (tokens, hidden), dtype=np.int8), rng.uniform(0.01, 0.03, tokens).astype(np.float16)
+    source = rng.integers(0, tokens, slots).astype(np.int32)
+    live = np.concatenate([np.arange(row, row + rows) for _, row, rows in written])
+    one = lambda array: array[None]  # a tile's expert by itself
+    project = lambda x, xs, w, ws: np.concatenate([orc.grouped_project(x[r : r + m], xs[r : r + m], one(w[ex]), one(ws[ex]), np.array([m], np.int32), np.array([0], np.int32))
+                                                   for ex, r, m in written])
+    common = dict(Book=gu.book(), TileCount=gu.dev(np.array([len(units)], np.int32)), TileUnits=gu.dev(np.array([u + (0,) for u in units], np.int32)))
+    few = dict(rows=slots, E=e, tiles=len(units) + 2, few_rows=True)
+    common["TileUnits"] = torch.cat([common["TileUnits"], torch.full((2, 4), -1, dtype=torch.int32, device=gu.DEV)])
+
+    act = torch.full((slots + 1, inter), 55.0, dtype=torch.float16, device=gu.DEV)
+    row_max = torch.zeros(slots + 1, dtype=torch.int32, device=gu.DEV)
+    gu.kernel("e8p_decode_grouped", N=2 * inter, K=hidden, gather=True, epilogue="swiglu", **few)(
+        A=gu.dev(a_q), AS=gu.dev(a_s), Act=act, P=stored[2 * inter], RowMax=row_max, SlotToken=gu.dev(source), WS=gu.dev(s1), **common)
+    gate_up = gu.dev(project(a_q[source], a_s[source][:, None], w1, s1))
+    product = torch.empty((len(live), inter), dtype=torch.float16, device=gu.DEV)
+    gu.kernel("swiglu", I=inter)(X=gate_up, Y=product, rows=len(live))
+    want = torch.full_like(act, 55.0)
+    want[live] = product
+    assert torch.equal(act, want)
+    want_max = torch.zeros_like(row_max)
+    want_max[live] = product.abs().amax(1).float().view(torch.int32)
+    assert torch.equal(row_max, want_max)
+
+    values = rng.normal(size=(slots, inter)).astype(np.float16)
+    out = torch.full((slots + 1, hidden), 55.0, dtype=torch.float16, device=gu.DEV)
+    gu.kernel("e8p_decode_grouped", N=hidden, K=inter, input_dtype="float16", **few)(
+        A=gu.dev(values), C=out, P=stored[hidden], RowMax=gu.dev(np.abs(values).max(1).astype(np.float32).view(np.int32)), WS=gu.dev(s2), **common)
+    q, q_s = orc.a8(values)
+    want = torch.full_like(out, 55.0)
+    want[live] = gu.dev(project(q, q_s, w2, s2))
+    assert torch.equal(out, want)
+
+
 def test_grouped_resident_rejects_shapes_it_cannot_take():
     for bad in (dict(N=200, K=384), dict(N=256, K=128), dict(N=256, K=3072), dict(N=256, K=512, block_m=64)):
         variant = dict(rows=64, E=4, tiles=6, block_m=32, packed_k=128, algorithm="resident")
