@@ -88,7 +88,7 @@ def int8_panels_pay(rows, n, k, cus):
 def tiles_pay(codec, rows, n, k, cus):
     """Whether row-major rows over 128 x 128 tiles are faster than panels where these were the faster ones before the tiles (time of the pair over panels / row-major, 256 CUs,
     by blocks of 16 channels to a CU).
-    Codes, 513-1024 rows: half to 1.5 blocks 1.06-1.7; to two blocks 1.01-1.15 above 768 rows, 0.88-0.99 below; wider 0.80-0.93; up to half a block 1.0-1.09 above 850 rows from K = 2048
+    Codes, 513-1024 rows: half to 1.5 blocks 1.06-1.7 where the tiles are there (split_pays); to two blocks 1.01-1.15 above 768 rows, 0.88-0.99 below; wider 0.80-0.93; up to half a block 1.0-1.09 above 850 rows from K = 2048
     on, 0.80-0.99 otherwise.  Up to 512 rows panels (where they were) 0.56-0.98.
     int8, 129-256 rows: two to three blocks 1.02-1.09 above 208 rows, 0.92-1.03 otherwise.  257-512 rows: up to two blocks 0.99-1.37, wider 0.79-0.96 (K = 1024 1.07).  513 rows and
     more 1.06-1.43 (a third of a block at 515 rows 0.94)."""
@@ -106,6 +106,13 @@ def tiles_pay(codec, rows, n, k, cus):
     if rows <= 512:
         return blocks <= 2 * cus or k <= 1024
     return rows > 576 or 3 * blocks > cus
+
+
+def split_pays(rows, n, cus):
+    """The same for codes without the 128 x 128 int8 tiles: these are decoded for them once, into a Workspace that is never larger than the launch's without them, and
+    the older split tiles hold 64 MiB (513 to 896 rows of 5121 to 6144 channels and K from 11008 on).  Time over panels / split tiles: rows that fill 15/16 of their row tiles of up to
+    22 channels to a CU 0.98-1.10, rows that fill less 0.90-1.06 there, wider 0.87-1.02."""
+    return 16 * rows >= 15 * 128 * -(-rows // 128) and n <= 22 * cus
 
 
 class QuantizedLinear:
@@ -134,6 +141,7 @@ class QuantizedLinear:
         if algorithm == "auto" and not block_m and self.k % 128 == 0 and 256 <= self.k <= 32768 and self.n * self.k < 2**31:
             pays = panels_pay if codec == "q4" else int8_panels_pay
             self.over_panels = [pays(rows, self.n, self.k, cus) for rows in range(top + 1)]
+        self.over_tiles = {}  # of row counts that have come: whether row-major is faster after all
         # (both copies in one allocation: a second one, new from the driver, took 2 ms of a construction)
         padded = (top + 15) // 16 * 16 if any(self.over_panels) else 0
         codes = torch.empty((capacity + padded, self.k), dtype=torch.int8, device="cuda")
@@ -191,6 +199,16 @@ class QuantizedLinear:
         host time beside the launch, slicing 1.4; a kept slice and detach() take 0.5, but 12 more on a first call.)"""
         return self.out.as_strided((rows, self.n), (self.n, 1))
 
+    def _row_major(self, rows):
+        """Whether row-major rows are faster than panels, asked when such rows first come (0.2 us, of codes 1.5; for every row count at construction it was 3 ms)."""
+        known = self.over_tiles.get(rows)
+        if known is None:
+            known = tiles_pay(self.codec, rows, self.n, self.k, self.cus)
+            if known and self.codec == "q4" and self.projection.workspace_bytes(rows) < self.n * self.k:
+                known = split_pays(rows, self.n, self.cus)
+            self.over_tiles[rows] = known
+        return known
+
     def run(self, x16, stream=None):
         if stream is None:
             stream = current_stream()
@@ -198,7 +216,7 @@ class QuantizedLinear:
             self.single(stream=stream, A=x16, AS=self.a_s, Book=self.book, Out=self.out, Q=self.a_q, S=self.scales, W=self.weight)
             return self._rows(1)
         rows = x16.shape[0]
-        if rows < len(self.over_panels) and self.over_panels[rows] and not tiles_pay(self.codec, rows, self.n, self.k, self.cus):
+        if rows < len(self.over_panels) and self.over_panels[rows] and not self._row_major(rows):
             self.panel_quantizer(stream=stream, Mask=None, Panels=self.panels, Q=self.a_q, S=self.a_s, Sums=self.sums, X=x16, rows=rows)
             if self.codec == "q4":
                 self.panel_projection(stream=stream, A=self.panels, AS=self.a_s, Book=self.book, Out=self.out, S=self.scales, Sums=self.sums,

@@ -336,6 +336,32 @@ def test_which_rows_a_linear_takes_over_panels(n, k, lines):
         assert panels_pay(rows, n, k, 256) == bool(taken), rows
 
 
+@pytest.mark.parametrize("n, k, lines", [  # rows, and whether they go over panels
+    (6144, 11008, [(513, 1), (640, 1), (768, 1), (769, 0), (896, 0)]), (6144, 10880, [(513, 0), (768, 0)]),     # more than 64 MiB of weights, fewer
+    (5184, 17408, [(513, 1), (599, 1), (600, 0), (640, 0), (641, 1), (719, 1), (720, 0), (768, 0), (769, 1), (839, 1), (840, 0), (896, 0), (897, 0)]),
+    (5632, 13056, [(600, 0), (599, 1)]), (5640, 13056, [(640, 1)]), (5120, 17408, [(513, 0), (1024, 0)]), (6160, 17408, [(513, 1), (768, 1), (769, 0)])])
+def test_a_linear_leaves_panels_only_for_tiles_that_are_there(n, k, lines):
+    """Codes are decoded for the 128 x 128 tiles, into a Workspace that is never larger than without them: where it does not hold the weights, the split tiles would
+    run, which are slower than panels for the most part."""
+    from orinfer_amd import lib, programs
+
+    linear = object.__new__(programs.QuantizedLinear)  # (its construction takes a device)
+    linear.codec, linear.n, linear.k, linear.cus, linear.single, linear.over_tiles = "q4", n, k, 256, None, {}
+    linear.projection = lib.Kernel("e8p_q4_projection", M=1024, N=n, K=k, dynamic_rows=True, workspace=True)
+    linear.over_panels = [programs.panels_pay(rows, n, k, 256) for rows in range(1025)]
+    for name in ("panels", "a_s", "a_q", "sums", "book", "out", "scales", "weight"):
+        setattr(linear, name, None)
+    taken = []
+    linear.panel_quantizer = lambda **args: taken.append("panels")
+    linear.panel_projection = linear._rows = lambda *args, **named: None
+    linear.quantize = lambda x, stream: taken.append("rows")
+    linear.project = lambda rows, stream: None
+    for rows, panels in lines + lines:  # the second time from what is known
+        taken.clear()
+        linear.run(np.empty((rows, 0), np.float16), stream=0)
+        assert taken == ["panels" if panels else "rows"], rows
+
+
 @pytest.mark.parametrize("n, k, lines", [
     (2048, 2048, [(112, 0), (113, 1), (128, 1), (129, 0), (512, 0), (513, 1), (1024, 1), (1025, 0)]), (4096, 4096, [(256, 0), (257, 1), (512, 1), (513, 0)]), (4096, 2048, [(768, 1), (769, 0)]),
     (5120, 5120, [(113, 0), (129, 0), (224, 0), (225, 1), (512, 1), (513, 0)]), (5120, 1024, [(129, 1)]), (7168, 8192, [(512, 1), (513, 1), (768, 1), (769, 0)]), (7168, 8320, [(400, 0)]),
