@@ -357,13 +357,14 @@ class MoeLayer:
             try:
                 tiles = (assignments + BULK_ROWS - 1) // BULK_ROWS + min(experts, assignments)
                 bulk = dict(rows=assignments, E=experts, tiles=tiles, block_m=BULK_ROWS, tile_units=True)
-                self.k_router_a8 = Kernel("router_topk", renormalize=True, quantize_hidden=hidden, **common)
-                self.k_metadata_slots = Kernel("route_metadata", block_m=BULK_ROWS, slot_maps=True, workspace=True,
-                                               tile_units=True, **common)
-                self.k_gate_up_bulk = Kernel("e8p_decode_grouped", N=2 * intermediate, K=hidden, gather=True,
-                                             epilogue="swiglu", **bulk)
-                self.k_act_a8 = Kernel("activation_quantization", K=intermediate)
-                self.k_down_bulk = Kernel("e8p_decode_grouped", N=hidden, K=intermediate, **bulk)
+                # (all of them before the first is kept: the five launches have kernels of the same names)
+                served = dict(
+                    k_router_a8=Kernel("router_topk", renormalize=True, quantize_hidden=hidden, **common),
+                    k_metadata_slots=Kernel("route_metadata", block_m=BULK_ROWS, slot_maps=True, workspace=True, tile_units=True, **common),
+                    k_gate_up_bulk=Kernel("e8p_decode_grouped", N=2 * intermediate, K=hidden, gather=True, epilogue="swiglu", **bulk),
+                    k_act_a8=Kernel("activation_quantization", K=intermediate),
+                    k_down_bulk=Kernel("e8p_decode_grouped", N=hidden, K=intermediate, **bulk))
+                vars(self).update(served)
                 self.segments = self.k_metadata_slots.workspace()
                 self.tile_units = torch.empty((tiles, 4), **i32)
                 self.slot_token = torch.empty(assignments, **i32)

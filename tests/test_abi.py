@@ -498,6 +498,49 @@ def test_workload_sizes_and_algorithmic_bytes():
     assert small["x"].shape == (8, 256) and np.array_equal(small["packed"], workloads.config1(1, n=256, k=256)["packed"])
 
 
+@pytest.mark.parametrize("refused", [None, "gate_up", "a8", "down"])
+def test_an_expert_layer_keeps_its_order_where_a_kernel_of_another_is_refused(monkeypatch, refused):
+    """1024 tokens of 16 experts x top-8: the order over 128-row tiles, where all of its kernels are served; else the five launches, with the kernels that were theirs."""
+    import types
+
+    import torch
+
+    from orinfer_amd import lib, programs
+
+    tokens, experts, top_k, hidden, inter = 1024, 16, 8, 512, 256
+    launched = []
+
+    class Recorder(lib.Kernel):
+        def __init__(self, symbol, **variant):
+            grouped = symbol == "e8p_decode_grouped" and variant.get("block_m") == 128
+            a8 = symbol == "activation_quantization" and variant == dict(K=inter)
+            if {"gate_up": grouped and variant["K"] == hidden, "down": grouped and variant["K"] == inter, "a8": a8}.get(refused, False):
+                raise lib.OrxError(lib.ORX_ERR_BAD_VARIANT, "refused")
+            super().__init__(symbol, **variant)
+
+        def workspace(self):
+            return None
+
+        def __call__(self, stream=None, **named):
+            assert set(named) == set(self.arg_names), self.symbol
+            launched.append(self)
+
+    on_host = types.SimpleNamespace(
+        **{name: getattr(torch, name) for name in ("int32", "int8", "float16", "float32")},
+        empty=lambda *shape, device=None, **named: torch.empty(*shape, **named),
+        cuda=types.SimpleNamespace(get_device_properties=lambda device: types.SimpleNamespace(multi_processor_count=256)))
+    monkeypatch.setattr(programs, "torch", on_host)
+    monkeypatch.setattr(programs, "_dev", lambda array: torch.from_numpy(np.ascontiguousarray(np.asarray(array)).view(np.uint8)))
+    monkeypatch.setattr(programs, "Kernel", Recorder)
+    bank = lambda n, k: (np.zeros((experts, n, k // 8), np.uint16), np.zeros((experts, n), np.float16))
+    layer = programs.MoeLayer(tokens, experts, top_k, hidden, inter, *bank(2 * inter, hidden), *bank(hidden, inter))
+    assert (layer.fused_stages, layer.bulk, layer.few) == (True, refused is None, False)
+    layer.run(None, None, stream=0)
+    assert [k.symbol for k in launched] == ["router_topk", "route_metadata", "e8p_decode_grouped"] + ([] if refused else ["activation_quantization"]) + [
+        "e8p_decode_grouped", "moe_combine"]
+    assert {k.variant["block_m"] for k in launched if "block_m" in k.variant} == {32 if refused else 128}
+
+
 def test_argument_lists_of_the_fused_expert_layer_forms():
     """Buffer names stay in ASCII order when a form adds buffers, and forms the resident expert kernel
     does not serve are refused at resolve time (so a program can fall back to the separate launches)."""
