@@ -92,18 +92,21 @@ int orx_release(orx_fn f);
  * (kernels.rs:150-170): limits the caller validates its launch record against. */
 int orx_query(orx_fn f, uint32_t* max_threads_per_block, uint32_t* static_lds_bytes);
 
-/* The same for the kernel that a launch of `rows` live rows starts (rows <= 0: the variant's own M,
- * which is what orx_query reports).  A projection handle picks its kernel by the live rows (one-row
- * GEMV, batched-decode kernels, MFMA tiles): the attributes are read from that kernel, the one whose
+/* The same for the kernel that a record of `rows` live rows names (rows <= 0: the variant's own M,
+ * which is what orx_query reports).  A projection handle has a kernel per range of live rows (one-row
+ * GEMV, batched-decode kernels, MFMA tiles): the attributes are read from the one whose
  * grid, block and LDS bytes orx_geometry returns for the same rows, so a record per row range
  * (crates/orinfer-model-sdk/src/operators/rows.rs:14-58) is validated against its own function as
- * kernels.rs:150-170 validates a cubin's.  Enqueues nothing. */
+ * kernels.rs:150-170 validates a cubin's.  What a launch starts may be another kernel (orx_launch): its
+ * limits are the library's own business and are not reported.  Enqueues nothing. */
 int orx_query_rows(orx_fn f, int32_t rows, uint32_t* max_threads_per_block, uint32_t* static_lds_bytes);
 
 /* The launch geometry a package would record for this kernel: the static grid of a
  * fixed-row kernel, or the RowExpression result of a dynamic one for `rows` live rows
  * (crates/orinfer-model-sdk/src/operators/dynamic.rs:93-118).  rows <= 0 means the
- * variant's own M.  Fails with ORX_ERR_ROWS when rows exceeds the capacity. */
+ * variant's own M.  Fails with ORX_ERR_ROWS when rows exceeds the capacity.  It is what a record holds and
+ * orx_launch checks, and stays the same where a faster kernel has taken the place of the one that it
+ * belongs to: no measure of the workgroups or the LDS of a launch. */
 int orx_geometry(orx_fn f, int32_t rows, uint32_t grid[3], uint32_t block[3], uint32_t* shared_bytes);
 
 /* Scratch the engine provides (AGENTS.md:41 "the engine owns every buffer"; the reference's
@@ -111,7 +114,8 @@ int orx_geometry(orx_fn f, int32_t rows, uint32_t grid[3], uint32_t block[3], ui
  * crates/orinfer-model-sdk/src/artifact.rs:60-72 in which the engine would list it).  A
  * projection resolved with `"workspace": true` takes one more buffer, `Workspace`, after its
  * weights (256-byte aligned; contents need not be kept between launches; launches that overlap
- * in time need distinct ones).  *bytes = what a launch of `rows` rows reads and writes there;
+ * in time need distinct ones).  *bytes = the most that a launch of `rows` rows reads and writes there
+ * (a launch asks for a buffer wherever that is not 0, also where the kernel that it starts leaves it alone);
  * rows <= 0 asks for the largest need of any row count up to the capacity, which is what an
  * engine allocates once.  0 means the launch uses none and the pointer may be null.  Handles
  * resolved without the key never use scratch (whole tiles, decode inside the GEMM). */
@@ -128,8 +132,10 @@ int orx_arg_kind(orx_fn f, int index);
  * orx_geometry() returns for the row count passed in `m` (validated; the reference
  * validates records in kernels.rs:47-61).  Never blocks, never allocates.  A launch may
  * enqueue more than one kernel (weight expansion + GEMM, split tiles + their sum, row slices
- * of a batched-decode kernel): the recorded grid/block/shared are those of its main kernel and
- * the whole launch is one node sequence under graph capture. */
+ * of a batched-decode kernel), and another main kernel than the recorded grid/block/shared belong to, where one
+ * that came later is faster for the rows (channel runs, the streaming kernel, 128 x 128 int8 tiles, units of 128
+ * channels of a routed projection): with a geometry of its own, the same bytes as result, the same arguments and
+ * no more Workspace.  The whole launch is one node sequence under graph capture. */
 int orx_launch(orx_fn f, const uint32_t grid[3], const uint32_t block[3], uint32_t shared_bytes,
                void* hip_stream, void** args);
 

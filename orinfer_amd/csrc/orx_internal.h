@@ -99,7 +99,8 @@ int hip_check(hipError_t code, const char* operation);
 
 // Every kernel launch of the library goes through ORX_LAUNCH.  While a thread records (orx_query_rows), a launch
 // enqueues nothing and leaves its function, grid, block and dynamic LDS bytes in that thread's list instead: the
-// query then reads the attributes of the very kernel a launch of that row count would start.
+// query then reads the attributes of the kernel that a record of that row count names.  A rule that starts another kernel behind
+// such a record (runs_instead, stream_instead, mid_parts_to_launch) does not hold while a thread records.
 struct LaunchRecord {
     const void* function;
     uint32_t grid, block, shared;

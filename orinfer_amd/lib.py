@@ -141,7 +141,7 @@ class Kernel:
             self._handle = None
 
     def query(self, rows=0):
-        """(thread limit, static LDS bytes) of the kernel that a launch of `rows` rows starts (0: the variant's M)."""
+        """(thread limit, static LDS bytes) of the kernel that a record of `rows` rows names (0: the variant's M); a launch may start a faster one."""
         threads, lds = ctypes.c_uint32(), ctypes.c_uint32()
         _check(library().orx_query_rows(self._handle, int(rows), ctypes.byref(threads), ctypes.byref(lds)))
         return threads.value, lds.value
