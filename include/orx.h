@@ -134,7 +134,7 @@ int orx_arg_kind(orx_fn f, int index);
  * enqueue more than one kernel (weight expansion + GEMM, split tiles + their sum, row slices
  * of a batched-decode kernel), and another main kernel than the recorded grid/block/shared belong to, where one
  * that came later is faster for the rows (channel runs, the streaming kernel, 128 x 128 int8 tiles, units of 128
- * channels of a routed projection): with a geometry of its own, the same bytes as result, the same arguments and
+ * channels of a routed projection, segmented metadata in one launch): with a geometry of its own, the same bytes as result, the same arguments and
  * no more Workspace.  The whole launch is one node sequence under graph capture. */
 int orx_launch(orx_fn f, const uint32_t grid[3], const uint32_t block[3], uint32_t shared_bytes,
                void* hip_stream, void** args);

@@ -1169,7 +1169,7 @@ int metadata_geometry(const orx_function& f, int rows, Geometry* g) {
     if (f.flags & kSegments) {
         g->grid[0] = ceil_div((uint32_t)rows * (uint32_t)f.top_k, (uint32_t)kSegment);
         g->block[0] = kMetaThreads;
-        g->shared = (uint32_t)((kMetaWaves + (g->grid[0] <= kOneLaunchSegments ? 2 : 0)) * f.E * sizeof(int));
+        g->shared = (uint32_t)(kMetaWaves * f.E * sizeof(int));  // of segment_rank_kernel: a record holds one size for all row counts
         return ORX_OK;
     }
     g->grid[0] = 1;
@@ -1205,7 +1205,8 @@ int metadata_launch(const orx_function& f, int rows, const Geometry& g, hipStrea
         const int assignments = rows * f.top_k;
         const dim3 grid(g.grid[0]), block(kMetaThreads);
         if (g.grid[0] <= kOneLaunchSegments) {
-            ORX_LAUNCH(segment_metadata_kernel, grid, block, g.shared, s, ids, out, assignments, f.E, f.top_k, f.block_m);
+            const uint32_t counters = (uint32_t)((kMetaWaves + 2) * f.E * sizeof(int));
+            ORX_LAUNCH(segment_metadata_kernel, grid, block, counters, s, ids, out, assignments, f.E, f.top_k, f.block_m);
         } else {
             int* segments = pointer_arg<int>(args, f.workspace_arg);
             ORX_LAUNCH(segment_rank_kernel, grid, block, g.shared, s, ids, out.relative, segments, assignments, f.E);
@@ -1259,10 +1260,8 @@ int make_metadata(const Variant& v, orx_function* f) {
     if (f->dynamic_rows) f->args.push_back({"m", ArgI32, 4});
     f->geometry = metadata_geometry;
     f->launch = metadata_launch;
-    const bool one_launch = ceil_div((uint32_t)f->M * (uint32_t)f->top_k, (uint32_t)kSegment) <= (uint32_t)kOneLaunchSegments;
-    f->device_function = !f->takes_workspace ? reinterpret_cast<const void*>(&route_metadata_kernel)
-                         : one_launch       ? reinterpret_cast<const void*>(&segment_metadata_kernel)
-                                            : reinterpret_cast<const void*>(&segment_rank_kernel);
+    f->device_function = f->takes_workspace ? reinterpret_cast<const void*>(&segment_rank_kernel)
+                                            : reinterpret_cast<const void*>(&route_metadata_kernel);
     return ORX_OK;
 }
 

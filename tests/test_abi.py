@@ -541,6 +541,14 @@ def test_an_expert_layer_keeps_its_order_where_a_kernel_of_another_is_refused(mo
     assert {k.variant["block_m"] for k in launched if "block_m" in k.variant} == {32 if refused else 128}
 
 
+@pytest.mark.parametrize("experts", [4, 128, 1024])
+def test_a_record_of_the_segmented_metadata_fits_at_every_length(experts):
+    """One dynamic LDS size per handle, which a record fixes: counters of sixteen waves, whether a list of up to 16 segments is one launch or more are two."""
+    handle = lib.Kernel("route_metadata", M=40000, E=experts, top_k=1, block_m=32, slot_maps=True, workspace=True, dynamic_rows=True)
+    for rows in (1, 1024, 1025, 16384, 16385, 40000):
+        assert handle.geometry(rows) == ((-(-rows // 1024), 1, 1), (1024, 1, 1), 16 * experts * 4)
+
+
 def test_argument_lists_of_the_fused_expert_layer_forms():
     """Buffer names stay in ASCII order when a form adds buffers, and forms the resident expert kernel
     does not serve are refused at resolve time (so a program can fall back to the separate launches)."""
