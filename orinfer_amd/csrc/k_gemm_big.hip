@@ -107,6 +107,7 @@ __device__ __forceinline__ void tile_of(int id, int tiles_m, int tiles_n, int* t
 // block: 8192 x 4096 x 4096 119.0 -> 117.9 us, 8192 x 7168 x 5120 276.6 -> 273.4, 3000 x 2048 x 1024 18.3 -> 17.3.
 constexpr uint32_t kPersistentLds = 4 * kTileBytes + 2 * kTile * 4;
 constexpr int kPersistentThreads = 512;
+constexpr int kShortK = 384;  // up to here SHORT
 
 struct TileState {
     int row0, col0, rows_here, cols_here;
@@ -133,13 +134,13 @@ __device__ __forceinline__ const int8_t* uniform_pointer(const int8_t* pointer) 
     return reinterpret_cast<const int8_t*>(((uint64_t)high << 32) | low);
 }
 
-// F32: fp32 output (heads); its own instantiation, so that either kernel holds one epilogue.
+// F32: fp32 output (heads); its own instantiation, so that either kernel holds one epilogue.  SHORT: K of up to kShortK.
 //
 // Eight waves share the 256 x 256 tile, 128 token rows x 64 channels each: 8 x 4 blocks of 16 x 16, 128 accumulator
 // registers.  A K step of 128 is two MFMA K slices of 64; a slice is multiplied in two phases of 16 multiplies
 // (token blocks 0-3, then 4-7, against the slice's four channel blocks), so that only four token fragments and four
 // weight fragments are live per phase and a second set is on its way from LDS: 64 fragment registers.
-template <bool F32>
+template <bool F32, bool SHORT>
 __global__ __launch_bounds__(kPersistentThreads) void gemm_big_persistent_kernel(BigParams p) {
     constexpr int WAVES_N = 4, BLOCKS_PER_WAVE = 4;
     extern __shared__ __align__(16) int8_t lds[];  // [2 stages][A 32 KiB | W 32 KiB], 512 scales
@@ -244,8 +245,10 @@ __global__ __launch_bounds__(kPersistentThreads) void gemm_big_persistent_kernel
     // step's first.  The first wait for them is that step's barrier, so what goes out later has less than half a step to come from memory: 3 + 3 + 2
     // over three phases, products alone, 8192 x 4096 x 4096 120.2 -> 114.1 us, 8192 x 34816 x 5120 1211 -> 1158, 8192 x 5120 x 17408 640 -> 606, 2048 x 5120 x
     // 17408 207 -> 189; 6 + 2 and 8 + 0 0 to 3 % slower than 5 + 3.
+    // SHORT, two or three steps to a tile: 3 + 3 + 2, measured the faster one with operands out of cache (which of a tile's two ends costs it was not looked into; 5 + 3 / 3 + 3 + 2: 1224 x
+    // 18784 x 256 20.76 / 20.45 us, 2048 x 34816 x 256 46.8 / 46.3, 1224 x 18784 x 384 24.7 / 24.5; four steps are level, 1224 x 18784 x 512 29.4 / 29.3, 3000 x 16384 x 512 40.0 / 40.5).
     constexpr int LOADS = 2 * BLOCKS_PER_WAVE;
-    constexpr int PART0 = 5, PART1 = LOADS - PART0;
+    constexpr int PART0 = SHORT ? 3 : 5, PART1 = 3, PART2 = LOADS - PART0 - PART1;
     auto multiply_loading = [&](int phase, int first, int count, int stage) {
         v4i(&tokens)[4] = ft[phase & 1];
         v4i(&weights)[4] = fw[phase >> 1];
@@ -409,7 +412,7 @@ __global__ __launch_bounds__(kPersistentThreads) void gemm_big_persistent_kernel
         read_weights(cur, 1);
         wait_four<8>(ft[1]);
         __builtin_amdgcn_sched_barrier(0);
-        multiply_loading(1, 0, 0, nxt);
+        multiply_loading(1, PART0 + PART1, PART2, nxt);
         __builtin_amdgcn_sched_barrier(0);
         advance();
         read_tokens(cur, 3);                  // 4 younger requests
@@ -854,14 +857,12 @@ __global__ __launch_bounds__(kTallThreads) void gemm_q4_tall_kernel(BigParams p)
 }
 
 int prepare_device() {
-    int code = hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_big_persistent_kernel<false>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPersistentLds),
-                         "hipFuncSetAttribute");
-    if (code != ORX_OK) return code;
-    code = hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_big_persistent_kernel<true>),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPersistentLds),
-                     "hipFuncSetAttribute");
-    if (code != ORX_OK) return code;
+    int code = ORX_OK;
+    for (const void* kernel : {reinterpret_cast<const void*>(&gemm_big_persistent_kernel<false, false>), reinterpret_cast<const void*>(&gemm_big_persistent_kernel<true, false>),
+                               reinterpret_cast<const void*>(&gemm_big_persistent_kernel<false, true>), reinterpret_cast<const void*>(&gemm_big_persistent_kernel<true, true>)}) {
+        code = hip_check(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPersistentLds), "hipFuncSetAttribute");
+        if (code != ORX_OK) return code;
+    }
     code = hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_q4_tall_kernel<false>),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTallLds),
                      "hipFuncSetAttribute");
@@ -942,10 +943,15 @@ int gemm_big_launch(const int8_t* a, const void* w, const __half* ws, const __ha
         set_error("projection (mfma 256x256): the persistent int8 kernel needs K >= 256");
         return ORX_ERR_BAD_VARIANT;
     }
-    if (out_f32)
-        ORX_LAUNCH((gemm_big_persistent_kernel<true>), dim3(g.grid[0]), dim3(kPersistentThreads), g.shared, stream, p);
-    else
-        ORX_LAUNCH((gemm_big_persistent_kernel<false>), dim3(g.grid[0]), dim3(kPersistentThreads), g.shared, stream, p);
+    const dim3 grid(g.grid[0]), block(kPersistentThreads);
+    const bool short_k = k <= kShortK;
+    if (out_f32) {
+        if (short_k) ORX_LAUNCH((gemm_big_persistent_kernel<true, true>), grid, block, g.shared, stream, p);
+        else ORX_LAUNCH((gemm_big_persistent_kernel<true, false>), grid, block, g.shared, stream, p);
+    } else {
+        if (short_k) ORX_LAUNCH((gemm_big_persistent_kernel<false, true>), grid, block, g.shared, stream, p);
+        else ORX_LAUNCH((gemm_big_persistent_kernel<false, false>), grid, block, g.shared, stream, p);
+    }
     return hip_check(hipGetLastError(), "launch projection (mfma 256x256)");
 }
 

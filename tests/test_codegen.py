@@ -143,7 +143,7 @@ def built(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("family, count", [("panel_kernel", 60), ("runs_kernel", 50), ("grouped_bulk_kernel", 8), ("gemm_mid_kernel", 2), ("gemm_big_persistent_kernel", 2)])
+@pytest.mark.parametrize("family, count", [("panel_kernel", 60), ("runs_kernel", 50), ("grouped_bulk_kernel", 8), ("gemm_mid_kernel", 2), ("gemm_big_persistent_kernel", 4)])
 def test_nothing_touches_a_register_that_is_on_its_way(built, family, count):
     chosen = {name: code for name, code in built.items() if family in name}
     assert len(chosen) >= count

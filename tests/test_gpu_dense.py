@@ -619,6 +619,23 @@ def test_tiles_of_128_by_128(codec, m, n, k, dtype, pad, parts):
         assert (out[m] == 9).all() and (out[:, n:] == 9).all()
 
 
+@pytest.mark.parametrize("m,n,k,dtype,pad", [
+    (1224, 18784, 256, "float16", 0), (1224, 18784, 384, "float32", 0), (2100, 17000, 512, "float16", 3), (1224, 18784, 640, "float16", 0)])
+def test_persistent_tiles_of_short_k(m, n, k, dtype, pad):
+    """Two and three K steps, whose requests are spread over three phases, four and five, over two; more tiles than workgroups, ragged ones among them."""
+    generator = torch.Generator(device=gu.DEV).manual_seed(orc.SEED + m + k)
+    a, weights = (torch.randint(-128, 128, (rows, k), generator=generator, device=gu.DEV, dtype=torch.int8) for rows in (m, n))
+    a_s, scales = (torch.rand(rows, generator=generator, device=gu.DEV).add(0.5).mul(0.01).half() for rows in (m, n))
+    # sums of up to 640 products of 2^14 at most are integers below 2^24: exact in float32, in any order
+    want = (((a.float() @ weights.float().t()) * scales.float()) * a_s.float()[:, None]).to(getattr(torch, dtype))
+    kern = gu.kernel("int8_projection", M=m, N=n, K=k, output_dtype=dtype, output_stride=n + pad)
+    out = torch.full((m + 1, n + pad), 9.0, dtype=want.dtype, device=gu.DEV)
+    for _ in range(2):
+        kern(A=a, Output=out, TokenScale=a_s, Weight=weights, WeightScale=scales)
+        assert torch.equal(out[:m, :n], want)
+        assert (out[m] == 9).all() and (out[:, n:] == 9).all()
+
+
 @pytest.mark.parametrize("dtype,pad", [("float16", 0), ("float32", 3)])
 @pytest.mark.parametrize("packed_k,n,k", [
     (0, 1, 2816), (0, 4096, 2816), (0, 4099, 8320), (0, 8208, 4224), (0, 40, 3584), (0, 16400, 5760),  # no tables, 16 lanes; one to five blocks
