@@ -850,7 +850,7 @@ bool runs_for_one_row(const orx_function& f) {
 //   int8, 65 to 128 rows in two and three rounds 0.44-0.91 up to K = 8192 (above 1.0); in one round 113 to 120 rows of long K 0.83-0.94.
 // The reported geometry is that of the kernel before, here and at one row, as a record of a launch names it.
 bool runs_instead(const orx_function& f, int rows) {
-    if (f.algorithm != kAuto || f.input_f16 || tile_for(f, rows) != 0 || (f.flags2 & (kPreferGemv | kNoGemv)) || recording_launches() || f.K % kBK != 0 ||
+    if (f.algorithm != kAuto || f.input_f16 || tile_for(f, rows) != 0 || (f.flags2 & (kPreferGemv | kNoGemv)) || recording_reported_kernels() || f.K % kBK != 0 ||
         (f.flags != kQ4 && f.flags != kW8) || !runs_eligible(f.flags, rows, f.N, f.K))
         return false;
     if (rows == 1) return runs_for_one_row(f);
@@ -875,7 +875,7 @@ bool runs_instead(const orx_function& f, int rows) {
 bool use_gemv(const orx_function& f, int rows);
 bool use_stream(const orx_function& f, int rows);
 bool stream_instead(const orx_function& f, int rows) {
-    return f.flags == kQ4 && f.algorithm == kAuto && !f.input_f16 && rows > 1 && rows <= 4 && f.packed_k == 0 && !(f.flags2 & kPreferGemv) && !recording_launches() &&
+    return f.flags == kQ4 && f.algorithm == kAuto && !f.input_f16 && rows > 1 && rows <= 4 && f.packed_k == 0 && !(f.flags2 & kPreferGemv) && !recording_reported_kernels() &&
            use_gemv(f, rows) && gemv_replicated_lanes(f, rows) == 0 && use_stream(f, rows);
 }
 
@@ -1113,7 +1113,7 @@ int mid_parts(const orx_function& f, int rows) {
 }
 
 // (A query asks for the limits of the kernel that the reported geometry, and so a record's block, is of.)
-int mid_parts_to_launch(const orx_function& f, int rows) { return recording_launches() ? 0 : mid_parts(f, rows); }
+int mid_parts_to_launch(const orx_function& f, int rows) { return recording_reported_kernels() ? 0 : mid_parts(f, rows); }
 
 uint64_t projection_workspace(const orx_function& f, int rows) {
     const int parts = mid_parts(f, rows);

@@ -26,6 +26,7 @@ void set_error(const char* format, ...) {
 
 int hip_check(hipError_t code, const char* operation) {
     if (code == hipSuccess) return ORX_OK;
+    if (code == hipErrorNoDevice && recording_started_kernels()) return ORX_OK;  // (nothing was asked of one)
     // Same text shape as the reference's check(): "<op>: CUDA error <code>" (mod.rs:48-55).
     set_error("%s: HIP error %d (%s)", operation, (int)code, hipGetErrorName(code));
     return (int)code;
@@ -33,8 +34,11 @@ int hip_check(hipError_t code, const char* operation) {
 
 namespace {
 thread_local std::vector<LaunchRecord>* g_recording = nullptr;
+thread_local bool g_as_reported = false;
 }
 bool recording_launches() { return g_recording != nullptr; }
+bool recording_reported_kernels() { return g_recording != nullptr && g_as_reported; }
+bool recording_started_kernels() { return g_recording != nullptr && !g_as_reported; }
 void record_launch(const void* function, dim3 grid, dim3 block, uint32_t shared) {
     g_recording->push_back({function, grid.x, block.x * block.y * block.z, shared});
 }
@@ -559,6 +563,23 @@ int launch_checked(const orx_function* f, int rows, const Geometry& want, void* 
     return f->launch(*f, rows, want, reinterpret_cast<hipStream_t>(hip_stream), args);
 }
 
+// Runs the launch of `live` rows with recording on: nothing is enqueued, no argument is dereferenced.
+int record_kernels(const orx_function* f, int live, const Geometry& want, bool as_reported, std::vector<LaunchRecord>* seen) {
+    uint64_t zero[64] = {};
+    void* args[64];
+    if (f->args.size() > 64) {
+        set_error("%s: too many arguments", f->symbol.c_str());
+        return (int)ORX_ERR_INTERNAL;
+    }
+    for (size_t i = 0; i < f->args.size(); ++i) args[i] = &zero[i];
+    if (f->dynamic_rows) *reinterpret_cast<int32_t*>(&zero[f->args.size() - 1]) = live;
+    struct Recording {
+        Recording(std::vector<LaunchRecord>* seen, bool as_reported) { g_recording = seen, g_as_reported = as_reported; }
+        ~Recording() { g_recording = nullptr; }
+    } recording(seen, as_reported);
+    return f->launch(*f, live, want, nullptr, args);
+}
+
 }  // namespace
 
 extern "C" {
@@ -596,23 +617,8 @@ int orx_query_rows(orx_fn f, int32_t rows, uint32_t* max_threads_per_block, uint
             Geometry want;
             int code = f->geometry(*f, live, &want);
             if (code != ORX_OK) return code;
-            uint64_t zero[64] = {};
-            void* args[64];
-            if (f->args.size() > 64) {
-                set_error("orx_query %s: too many arguments", f->symbol.c_str());
-                return (int)ORX_ERR_INTERNAL;
-            }
-            for (size_t i = 0; i < f->args.size(); ++i) args[i] = &zero[i];
-            if (f->dynamic_rows) *reinterpret_cast<int32_t*>(&zero[f->args.size() - 1]) = live;
             std::vector<LaunchRecord> seen;
-            g_recording = &seen;
-            try {
-                code = f->launch(*f, live, want, nullptr, args);
-            } catch (...) {
-                g_recording = nullptr;
-                throw;
-            }
-            g_recording = nullptr;
+            code = record_kernels(f, live, want, true, &seen);
             if (code != ORX_OK) return code;
             for (const LaunchRecord& r : seen)
                 if (function == nullptr && r.grid == want.grid[0] && r.block == want.block[0] * want.block[1] * want.block[2] &&
@@ -630,6 +636,24 @@ int orx_query_rows(orx_fn f, int32_t rows, uint32_t* max_threads_per_block, uint
         if (code != ORX_OK) return code;
         if (max_threads_per_block) *max_threads_per_block = (uint32_t)attr.maxThreadsPerBlock;
         if (static_lds_bytes) *static_lds_bytes = (uint32_t)attr.sharedSizeBytes;
+        return (int)ORX_OK;
+    });
+}
+
+// What a launch of `rows` rows enqueues (orx_internal.h).
+int orx_started_kernels(orx_fn f, int32_t rows, uint32_t (*kernels)[3], int32_t capacity, int32_t* count) {
+    return guard("orx_started_kernels", [&] {
+        const int live = rows <= 0 ? f->capacity : rows;
+        if (live > f->capacity || (!f->dynamic_rows && live != f->capacity)) return (int)ORX_ERR_ROWS;
+        HeldUnits held;
+        Geometry want;
+        int code = f->geometry(*f, live, &want);
+        if (code != ORX_OK) return code;
+        std::vector<LaunchRecord> seen;
+        code = record_kernels(f, live, want, false, &seen);
+        if (code != ORX_OK) return code;
+        *count = (int32_t)seen.size();
+        for (int i = 0; i < std::min(*count, capacity); ++i) kernels[i][0] = seen[i].grid, kernels[i][1] = seen[i].block, kernels[i][2] = seen[i].shared;
         return (int)ORX_OK;
     });
 }

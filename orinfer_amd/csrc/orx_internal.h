@@ -97,15 +97,18 @@ namespace orx {
 void set_error(const char* format, ...);
 int hip_check(hipError_t code, const char* operation);
 
-// Every kernel launch of the library goes through ORX_LAUNCH.  While a thread records (orx_query_rows), a launch
-// enqueues nothing and leaves its function, grid, block and dynamic LDS bytes in that thread's list instead: the
-// query then reads the attributes of the kernel that a record of that row count names.  A rule that starts another kernel behind
-// such a record (runs_instead, stream_instead, mid_parts_to_launch) does not hold while a thread records.
+// Every kernel launch of the library goes through ORX_LAUNCH.  While a thread records, a launch
+// enqueues nothing and leaves its function, grid, block and dynamic LDS bytes in that thread's list instead.
+// orx_query_rows records the kernels that orx_geometry reports and reads the attributes of the one that a record of
+// that row count names: a rule that starts another kernel behind such a record (runs_instead, stream_instead,
+// mid_parts_to_launch) does not hold meanwhile.  orx_started_kernels records what a launch starts.
 struct LaunchRecord {
     const void* function;
     uint32_t grid, block, shared;
 };
 bool recording_launches();
+bool recording_reported_kernels();
+bool recording_started_kernels();
 void record_launch(const void* function, dim3 grid, dim3 block, uint32_t shared);
 #define ORX_LAUNCH(kernel, grid, block, shared, stream, ...)                                                          \
     do {                                                                                                              \
@@ -173,6 +176,7 @@ struct DeviceOnce {
     int run(F&& setup) {
         const uint64_t bit = 1ull << (current_device() & 63);
         if (done.load(std::memory_order_acquire) & bit) return ORX_OK;
+        if (recording_started_kernels()) return ORX_OK;  // (there need be no device)
         const int code = setup();
         if (code == ORX_OK) done.fetch_or(bit, std::memory_order_release);
         return code;

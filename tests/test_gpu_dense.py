@@ -13,6 +13,7 @@ from oracle import reference as orc
 from orinfer_amd import codebook, programs, workloads
 
 from . import gpu_util as gu
+from .started_util import MID_2, MID_4, RUNS, reported, started
 
 pytestmark = pytest.mark.gpu
 TABLE = orc.basis()
@@ -607,6 +608,7 @@ def test_tiles_of_128_by_128(codec, m, n, k, dtype, pad, parts):
     if torch.cuda.get_device_properties(0).multi_processor_count == 256:
         tiles = -(-m // 128) * -(-n // 128)
         assert kern.workspace_bytes(m) == (n * k if codec == "q4" else 0) + (tiles * parts * 65536 if parts > 1 else 0)
+        assert started(kern, m)[codec == "q4"] == (tiles * parts, 256, MID_4 if tiles * parts <= 256 else MID_2)
     threads, _ = kern.query(m)
     assert threads == np.prod(kern.geometry(m)[1])  # a record names the reported block
     want = orc.project(a, a_s, weights, scales, out_dtype=np.float16 if dtype == "float16" else np.float32)
@@ -656,6 +658,7 @@ def test_one_row_of_codes_in_the_channel_runs(packed_k, n, k, dtype, pad):
         got = gu.host(out)
         np.testing.assert_array_equal(got[:1, :n], want)
         assert (got[0, n:] == 9).all() and (got[1] == 9).all()
+        assert started(kern, 1)[0][1:] == (512, RUNS)
         threads, _ = kern.query(1)
         assert threads == np.prod(kern.geometry(1)[1])
 
@@ -665,9 +668,10 @@ def test_one_row_of_codes_in_the_channel_runs(packed_k, n, k, dtype, pad):
     ("q4", 128, 16, 4112, 8192), ("q4", 0, 32, 4100, 12288), ("q4", 0, 2, 8208, 4224),                                  # two, three
     ("q4", 0, 2, 8200, 1152), ("q4", 0, 4, 16400, 1152), ("q4", 0, 3, 20500, 1408),                                     # the streaming kernel
     ("q4", 0, 96, 8300, 2048), ("q4", 128, 128, 4130, 2176), ("q4", 128, 247, 5904, 2304), ("q4", 64, 256, 4300, 2048), ("q4", 0, 270, 8192, 1536),
-    ("w8", 0, 65, 14960, 1152), ("w8", 0, 128, 9000, 1024), ("w8", 0, 120, 1000, 8320)])
+    ("w8", 0, 65, 14960, 1152), ("w8", 0, 128, 9000, 1024), ("w8", 0, 120, 1000, 8320),
+    ("q4", 128, 24, 4100, 12288), ("q4", 0, 2, 12289, 1152), ("q4", 128, 82, 9928, 2176), ("w8", 0, 65, 23909, 256)])
 def test_rows_that_leave_the_reported_kernel(codec, packed_k, rows, n, k):
-    """Shapes at the edges of the rules by which a launch takes the channel runs or the streaming kernel while its records name another."""
+    """Shapes at the edges of the rules by which a launch takes the channel runs or the streaming kernel while its records name another; of four the records name it too."""
     rng = np.random.default_rng(orc.SEED + rows + n + k)
     a = rng.integers(-127, 128, (rows, k), dtype=np.int8)
     a_s, scales = rng.uniform(0.01, 0.03, rows).astype(np.float16), rng.uniform(0.005, 0.02, n).astype(np.float16)
@@ -685,6 +689,9 @@ def test_rows_that_leave_the_reported_kernel(codec, packed_k, rows, n, k):
     got = gu.host(out)
     np.testing.assert_array_equal(got[:rows], orc.project(a, a_s, weights, scales, out_dtype=np.float16))
     assert (got[rows] == 9).all()
+    (only,) = started(kern, rows)
+    assert only[2] == RUNS or (only == (-(-n // 32), 512, 0) and rows <= 4)  # the channel runs, or the streaming kernel
+    assert (only == reported(kern, rows)) == ((codec, rows, n, k) in {("q4", 32, 4100, 12288), ("q4", 2, 8200, 1152), ("q4", 128, 4130, 2176), ("w8", 65, 14960, 1152)})
     threads, _ = kern.query(rows)
     assert threads == np.prod(kern.geometry(rows)[1])
 
