@@ -542,8 +542,8 @@ def test_q4_fp16_input_is_refused_where_no_kernel_serves_it():
                                                ("q4", 256, 17408, 256, "float16"), ("w8", 40, 2048, 1024, "float16"),
                                                ("w8", 17, 5120, 512, "float32")])
 def test_mid_row_projections_split_k_steps_evenly(codec, m, n, k, dtype):
-    """65-384 rows on the 128-row tiles: the K steps of the tiles are dealt evenly to one workgroup per
-    CU, runs that do not cover a whole tile meet as int32 partial sums.  Same bytes as whole tiles."""
+    """The 128-row tiles by name: the K steps of the tiles are dealt evenly to one workgroup per CU, runs that
+    do not cover a whole tile meet as int32 partial sums.  Same bytes as whole tiles in one launch."""
     rng = np.random.default_rng(orc.SEED + m + n)
     a = rng.integers(-128, 128, (m, k), dtype=np.int8)
     a_s = rng.uniform(0.01, 0.03, m).astype(np.float16)
@@ -560,14 +560,14 @@ def test_mid_row_projections_split_k_steps_evenly(codec, m, n, k, dtype):
         symbol, stored = "int8_projection", gu.dev(weights)
         call = lambda kern, out: kern(A=gu.dev(a), Output=out, TokenScale=gu.dev(a_s), Weight=stored, WeightScale=gu.dev(scales))
     variant = dict(M=m, N=n, K=k, output_dtype=dtype, output_stride=stride)
-    if m <= 64 or codec == "q4":
-        # `auto` gives so few rows of so small a matrix to the streaming kernel, 65..128 rows of two-stage codes with a
-        # short K to the channel-run kernel, and more rows of a matrix this wide to the 512-row channel runs
-        variant["algorithm"] = "mfma"
+    # by name: `auto` gives few rows to the streaming kernel or the channel runs, and more int8 rows to the 128 x 128 tiles of k_mid.hip, split or not
+    variant["algorithm"] = "mfma"
     split = gu.kernel(symbol, **variant)
     whole = gu.kernel(symbol, split_k=False, **variant)
     grid_split, grid_whole = tuple(split.geometry()[0]), tuple(whole.geometry()[0])
     assert grid_split[1] == 1 and grid_whole[0] == -(-n // 128) and grid_whole[1] == -(-m // 128)
+    assert started(split, m)[0] == (grid_split[0], 256, 0) and len(started(split, m)) == 2  # the steps, the sums
+    assert started(whole, m) == [(grid_whole[0], 256, 0)]
     out = torch.full((m + 1, stride), 9.0, dtype=torch_dtype, device=gu.DEV)
     other = torch.full((m + 1, stride), 9.0, dtype=torch_dtype, device=gu.DEV)
     call(split, out)
