@@ -7,6 +7,8 @@ device memory and the stream), so `run()` only enqueues and can be captured in a
 Program order of the expert layer follows python/orinfer_build/models/flash_next (router top-k,
 histogram, offsets, tiles, A8, dispatch, grouped gate_up, SwiGLU->A8, grouped down, combine).
 """
+import math
+
 import numpy as np
 import torch
 
@@ -253,6 +255,21 @@ def one_launch_routes(tokens, top_k, experts):
     return tokens <= 64 and tokens * top_k <= 1024 and experts <= 512 and -(-tokens // 16) * top_k <= 18
 
 
+def few_pays(tokens, top_k, experts, hidden, intermediate, cus):
+    """Whether five launches over tiles of 32 rows (few_rows) are faster than the seven, where the resident kernel is not there (time of the layer, seven over five, 2500 shapes, popularity
+    like 1 / rank^0.9, 256 CUs; weights in cache, and in brackets out of it).  Every workgroup of their second projection quantises its tile's rows again, which few or short rows pay for.
+    Rows of all tiles together (routed x intermediate) up to 65536 0.92-1.80, median 1.33 (1.00-1.72); up to 768 channels between and 4000 tiles x 128 channels of hidden x channels
+    between to a CU 0.90-1.55, 95 of 100 above 1.02 (0.92-1.37), beyond 0.90-1.24, median 0.99 (0.96-1.20, 1.07); up to 1152 where gate | up has at most 2.5 workgroups of 64 channels
+    to a CU 0.90-1.23, 1.04 (0.93-1.24, 1.07), beyond 0.77-1.17, 0.97 (0.82-1.22, 1.02); longer ones 0.66-1.06, 0.88 (0.73-1.16, 0.97)."""
+    routed = tokens * top_k
+    if routed * intermediate <= 65536:
+        return True
+    tiles = max(experts * (1 - math.exp(-routed / experts)), routed / 32)  # of uniform popularity
+    if intermediate <= 768:
+        return tiles * -(-hidden // 128) * intermediate <= 4000 * cus
+    return intermediate <= 1152 and tiles * -(-intermediate // 32) <= 2.5 * cus
+
+
 class MoeLayer:
     """Q2A8 expert layer: token-sort, grouped gate_up, SwiGLU->A8, grouped down, weighted combine."""
 
@@ -375,14 +392,15 @@ class MoeLayer:
             except OrxError as error:
                 if error.code != ORX_ERR_BAD_VARIANT:
                     raise
-        # Few rows: where neither order applies, five launches over tiles of 32 rows, any hidden and intermediate width.
+        # Few rows: where neither order applies, five launches over tiles of 32 rows, any hidden and intermediate width, where they are the faster ones.
         #   router top-k + A8 of every token's row, metadata with the tiles as units,
         #   gate_up that gathers the token rows, writes fp16(silu(gate) * up) and raises every slot's largest magnitude,
         #   down that quantises those rows on their way, combine.
         # A caller who asked for launches of their own, for the values in between (`keep_intermediates`) or for an algorithm gets them.
         self.few = False
         if (fused_stages is None and not self.bulk and not self.fused_stages and not keep_intermediates and signs is None and self.fused_dispatch
-                and not one_launch_refused and packed_k == 128 and block_m == 32 and experts <= 1024 and grouped_algorithm == "auto"):
+                and not one_launch_refused and packed_k == 128 and block_m == 32 and experts <= 1024 and grouped_algorithm == "auto"
+                and few_pays(tokens, top_k, experts, hidden, intermediate, torch.cuda.get_device_properties(self.w1.device).multi_processor_count)):
             try:
                 few = dict(rows=assignments, E=experts, tiles=self.tile_capacity, block_m=block_m, few_rows=True)
                 # four where router and metadata are one
