@@ -572,8 +572,13 @@ __global__ __launch_bounds__(kMetaThreads) void segment_place_kernel(const int* 
 }
 
 // Up to 16 segments in one launch: every workgroup reads the whole list and counts the other segments' assignments with LDS additions, which need no
-// order; only its own are ranked.
+// order; only its own are ranked.  Additions to one counter are served one after another, so lists of many segments over few experts stay with the two launches (these over one, 470 lists of
+// uniform to 1 / rank popularity: 4 and 8 experts up to 6 segments 0.96-1.13, to 8 0.83-1.08, above 0.74-1.05, median 0.9; 16 experts up to 12 segments 0.94-1.17, above 0.72-1.03; 32 and more
+// 0.85-1.26, median 1.1.  7889 tokens of 16 x 2, 1 / rank, 10.1 us in one, 7.3 in two).
 constexpr int kOneLaunchSegments = 16;
+bool metadata_in_one_launch(uint32_t segments, int experts) {
+    return segments <= (experts <= 8 ? 8u : experts <= 16 ? 12u : (uint32_t)kOneLaunchSegments);
+}
 __global__ __launch_bounds__(kMetaThreads) void segment_metadata_kernel(const int* __restrict__ ids, SegmentOutputs out, int assignments, int experts,
                                                                         int top_k, int block_m) {
     extern __shared__ int counters[];  // [kMetaWaves][experts], then assignments in front of this segment and behind it, [experts] each
@@ -1204,7 +1209,7 @@ int metadata_launch(const orx_function& f, int rows, const Geometry& g, hipStrea
         out.tile_units = f.flags & kTileUnits ? pointer_arg<int4>(args, tiles_at + 4) : nullptr;
         const int assignments = rows * f.top_k;
         const dim3 grid(g.grid[0]), block(kMetaThreads);
-        if (g.grid[0] <= kOneLaunchSegments) {
+        if (metadata_in_one_launch(g.grid[0], f.E)) {
             const uint32_t counters = (uint32_t)((kMetaWaves + 2) * f.E * sizeof(int));
             ORX_LAUNCH(segment_metadata_kernel, grid, block, counters, s, ids, out, assignments, f.E, f.top_k, f.block_m);
         } else {

@@ -366,7 +366,7 @@ class MoeLayer:
                 if fused_stages or error.code != ORX_ERR_BAD_VARIANT:
                     raise
         # Many rows: six launches over tiles of 128 rows (`block_m` is the tile height of the orders above).
-        #   router top-k + A8 of every token's row, metadata in segments (two launches above 16384 routes),
+        #   router top-k + A8 of every token's row, metadata in segments (two launches above 16384 routes, of few experts above 8192 or 12288),
         #   gate_up that gathers the token rows and writes fp16(silu(gate) * up), A8, down, combine.
         # A caller who asked for the quantiser and the dispatch, or the metadata, as launches of their own gets them; `fused_stages` stays
         # true where the five launches are served too.

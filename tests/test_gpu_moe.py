@@ -145,9 +145,11 @@ def test_route_metadata_in_segments(m, e, k, bm):
     kern(IDs=gu.dev(padded), m=m, **{**out, "RowMax": None})
 
 
-@pytest.mark.parametrize("m,e,k,bm", [(2049, 16, 8, 128), (1024, 5, 1, 32), (1025, 1024, 1, 128)])
+@pytest.mark.parametrize("m,e,k,bm", [(2049, 16, 8, 128), (1024, 5, 1, 32), (1025, 1024, 1, 128), (2045, 17, 8, 32), (2046, 17, 8, 32), (1021, 8, 8, 128), (1022, 8, 8, 128),
+                                      (1533, 16, 8, 32), (1534, 16, 8, 32)])
 def test_route_metadata_in_segments_around_the_single_launch(m, e, k, bm):
-    """Up to 16 segments are one launch: 17, with one assignment of the last, one whole segment, and one and a bit over as many experts as threads."""
+    """Up to 16 segments are one launch (12 of up to 16 experts, 8 of up to 8): 17, with one assignment of the last, one whole segment, one and a bit over as many experts as threads, and
+    either side of the lines."""
     test_route_metadata_in_segments(m, e, k, bm)
 
 

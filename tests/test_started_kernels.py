@@ -67,6 +67,13 @@ def test_launches_that_take_the_128_by_128_tiles(codec, rows, n, k, variant, til
     assert kernel.workspace_bytes(rows) == (n * k if codec == "q4" else 0) + (tiles * parts * 65536 if parts > 1 else 0)
 
 
+@pytest.mark.parametrize("experts,segments", [(4, 8), (8, 8), (9, 12), (16, 12), (17, 16), (1024, 16)])
+def test_segmented_metadata_in_one_launch_up_to_a_line(experts, segments):
+    kernel = lib.Kernel("route_metadata", M=40000, E=experts, top_k=1, block_m=32, slot_maps=True, workspace=True, dynamic_rows=True)
+    assert started(kernel, 1024 * segments) == [(segments, 1024, 18 * experts * 4)]
+    assert started(kernel, 1024 * segments + 1) == [(segments + 1, 1024, 16 * experts * 4), (segments + 1, 1024, 0)]
+
+
 def test_a_launch_by_record_starts_what_is_reported():
     """Kernels by name and rows that no rule takes elsewhere."""
     for kernel, rows in ((projection("w8", 513, 16384, 512), 513), (projection("q4", 40, 8300, 2048), 40), (projection("q4", 128, 8704, 512, algorithm="wide", M=128), 128),
