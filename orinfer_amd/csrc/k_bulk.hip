@@ -437,11 +437,14 @@ void grouped_bulk_geometry(int n, int tiles, bool swiglu, Geometry* g) {
 // Units of 128 channels: where units of 256 (by what the routed rows of `experts` come to, half a tile each beyond whole ones) leave CUs without one, as a unit of few blocks takes
 // as long per step of K whatever the others do.  One to a CU is bound by the chain of a step (reads of LDS, multiplies): 128 x 3200 channels and K 22 us, 256 channels 32; deeper requests
 // (three chunks of 128 rows, 80 KiB of LDS) and phases of eight and sixteen multiplies measured within 3 % of it.  gate | up, us, 256 / 128 channels: 2185 tokens of 16 experts
-// x top-2, 3200 x 384 31.6 / 22.6; 800 tokens 32.0 / 22.0; 3493 of 128 x 2, 2560 x 256 29.0 / 24.1; with both projections the layer 1500 of 16 x 2, 2048 x 1024 (248 units, the most
-// there are) 62.4 / 60.5-63.5, 600 of 32 x 4, 1280 x 512 46.7 / 38.8, 500 of 16 x 8, 4096 x 256 77.5 / 65.1.  The reported geometry is that of the units of 256, as a record of
+// x top-2, 3200 x 384 31.6 / 22.6; 800 tokens 32.0 / 22.0; 3493 of 128 x 2, 2560 x 256 29.0 / 24.1; with both projections the layer 600 of 32 x 4, 1280 x 512 46.7 / 38.8, 500 of 16 x 8, 4096 x 256 77.5 / 65.1.  The reported geometry is that of the units of 256, as a record of
 // a launch names it.
+// Tiles go to the eight XCDs in turn, so what counts is the XCD with the most of them: the line is at one unit of 256 to a CU of it (820 projections, time of 256 over 128 channels: up to there
+// 0.91-1.56, median 1.32, three of 591 below 0.98; up to a fourth more 0.81-1.20, median 0.99, then 0.80-1.17, 0.93; by the tiles that came, which a launch does not know, 574 of 574 are 1.00
+// or more.  Units summed over the chip had 1890 tokens of 8 x 1, 3200 x 1536, in 216 of 36 to an XCD: 37 -> 43 us).
 bool grouped_bulk_narrow(int64_t rows, int experts, int n) {
-    return (rows / kTileRows + experts / 2) * ceil_div((uint32_t)n, (uint32_t)kSpan) <= device_compute_units();
+    const int64_t tiles = (rows / kTileRows + experts / 2 + 7) / 8 * 8;
+    return tiles * ceil_div((uint32_t)n, (uint32_t)kSpan) <= device_compute_units();
 }
 
 int grouped_bulk_launch(const GroupedBuffers& b, int n, int k, int tiles, bool gather, bool swiglu, bool narrow, hipStream_t stream) {

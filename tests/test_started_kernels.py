@@ -74,6 +74,16 @@ def test_segmented_metadata_in_one_launch_up_to_a_line(experts, segments):
     assert started(kernel, 1024 * segments + 1) == [(segments + 1, 1024, 16 * experts * 4), (segments + 1, 1024, 0)]
 
 
+@pytest.mark.parametrize("rows,n,k,narrow", [  # tiles of the routed rows and half of the experts, eight XCDs
+    (28 * 128 + 127, 2048, 1024, True), (29 * 128, 2048, 1024, False), (20 * 128, 2304, 512, True), (21 * 128, 2304, 512, False), (12 * 128, 4096, 256, True), (13 * 128, 4096, 256, False),
+    (252 * 128, 256, 128, True), (253 * 128, 256, 128, False)])
+def test_units_of_128_channels_up_to_a_line(rows, n, k, narrow):
+    tiles = rows // 128 + 8
+    kernel = lib.Kernel("e8p_decode_grouped", rows=rows, E=8, tiles=tiles, N=n, K=k, block_m=128, tile_units=True)
+    assert [grid for grid, _, _ in started(kernel)] == [-(-tiles // 8) * 8 * -(-n // (128 if narrow else 256))]
+    assert reported(kernel)[0] == -(-tiles // 8) * 8 * -(-n // 256)
+
+
 def test_a_launch_by_record_starts_what_is_reported():
     """Kernels by name and rows that no rule takes elsewhere."""
     for kernel, rows in ((projection("w8", 513, 16384, 512), 513), (projection("q4", 40, 8300, 2048), 40), (projection("q4", 128, 8704, 512, algorithm="wide", M=128), 128),
