@@ -554,11 +554,13 @@ uint64_t workspace_need(const orx_function* f, int rows) {
 
 // A checked launch with the Workspace the caller gave.
 int launch_checked(const orx_function* f, int rows, const Geometry& want, void* hip_stream, void** args) {
-    const uint64_t need = workspace_need(f, rows);
-    if (need != 0 && *reinterpret_cast<uint64_t*>(args[f->workspace_arg]) == 0) {
-        set_error("launch %s: %d rows need a Workspace of %llu bytes (orx_workspace_bytes), the buffer is null",
-                  f->symbol.c_str(), rows, (unsigned long long)need);
-        return (int)ORX_ERR_WORKSPACE;
+    // (only without a buffer is it asked what the rows need: 0.1 to 0.3 us)
+    if (f->takes_workspace && *reinterpret_cast<uint64_t*>(args[f->workspace_arg]) == 0) {
+        if (const uint64_t need = workspace_need(f, rows)) {
+            set_error("launch %s: %d rows need a Workspace of %llu bytes (orx_workspace_bytes), the buffer is null",
+                      f->symbol.c_str(), rows, (unsigned long long)need);
+            return (int)ORX_ERR_WORKSPACE;
+        }
     }
     return f->launch(*f, rows, want, reinterpret_cast<hipStream_t>(hip_stream), args);
 }
