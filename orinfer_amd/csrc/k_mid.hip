@@ -178,18 +178,26 @@ __global__ __launch_bounds__(kThreads, STAGES == 2 ? 2 : 1) void gemm_mid_kernel
             for (int r = 0; r < 4; ++r) channel_scale[j][r] = __half2float(p.ws[col0 + min(wave_n * 64 + j * 16 + 4 * quarter + r, cols - 1)]);
         }
         if (p.out_f32) {
+            // (a lane's four channels in one store: 249 x 19456 x 512 24.0 -> 12.4 us, value by value)
+            const bool aligned = p.stride % 4 == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int row = wave_m * 64 + i * 16 + frag_row;
                 if (row >= rows) continue;
                 float* const to = reinterpret_cast<float*>(p.out) + (int64_t)(row0 + row) * p.stride + col0;
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
+                for (int j = 0; j < 4; ++j) {
+                    const int col = wave_n * 64 + j * 16 + 4 * quarter;
+                    const float value[4] = {rescale(acc[i][j][0], channel_scale[j][0], token_scale[i]), rescale(acc[i][j][1], channel_scale[j][1], token_scale[i]),
+                                            rescale(acc[i][j][2], channel_scale[j][2], token_scale[i]), rescale(acc[i][j][3], channel_scale[j][3], token_scale[i])};
+                    if (aligned && col + 4 <= cols) {
+                        *reinterpret_cast<float4*>(to + col) = make_float4(value[0], value[1], value[2], value[3]);
+                    } else {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int col = wave_n * 64 + j * 16 + 4 * quarter + r;
-                        if (col < cols) to[col] = rescale(acc[i][j][r], channel_scale[j][r], token_scale[i]);
+                        for (int r = 0; r < 4; ++r)
+                            if (col + r < cols) to[col + r] = value[r];
                     }
+                }
             }
         } else {
             // 16 rows x 64 channels at a time through the wave's own LDS (nobody reads the stages any more), whole rows of 128 bytes out
@@ -245,7 +253,7 @@ __global__ __launch_bounds__(kThreads) void mid_finish_kernel(MidParams p) {
     const int row = (wave >> 1) * 64 + i * 16 + (lane & 15);
     if (row >= rows) return;
     const float token_scale = __half2float(p.as[row0 + row]);
-    const bool aligned = p.stride % 4 == 0 && (reinterpret_cast<uintptr_t>(p.out) & 7) == 0;
+    const bool aligned = p.stride % 4 == 0 && (reinterpret_cast<uintptr_t>(p.out) & (p.out_f32 ? 15 : 7)) == 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int col = (wave & 1) * 64 + j * 16 + 4 * (lane >> 4);
@@ -254,7 +262,9 @@ __global__ __launch_bounds__(kThreads) void mid_finish_kernel(MidParams p) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) value[r] = rescale(acc[j][r], __half2float(p.ws[col0 + min(col + r, cols - 1)]), token_scale);
         const int64_t at = (int64_t)(row0 + row) * p.stride + col0 + col;
-        if (!p.out_f32 && aligned && col + 4 <= cols) {
+        if (p.out_f32 && aligned && col + 4 <= cols) {
+            *reinterpret_cast<float4*>(reinterpret_cast<float*>(p.out) + at) = make_float4(value[0], value[1], value[2], value[3]);
+        } else if (aligned && col + 4 <= cols) {
             *reinterpret_cast<uint2*>(reinterpret_cast<__half*>(p.out) + at) = make_uint2(pack_halves(value[0], value[1]), pack_halves(value[2], value[3]));
         } else {
 #pragma unroll
