@@ -1090,8 +1090,6 @@ uint64_t workspace_without_mid(const orx_function& f, int rows) {
 // older 128 x 128 tiles dealt out and summed, those tiles whole), products with the decode, us: int8 800 x 4096 x 4096 44.5 -> 18.3, 3317 x 1344 x 5248 58.3 -> 31.2, 674 x 3840 x 8960
 // 58.7 -> 37.7, 1536 x 4096 x 2048 25.9 -> 16.9; codes 1627 x 1408 x 2304 32.9 -> 18.2, 674 x 5248 x 3840 46.8 -> 34.0, 1583 x 3040 x 3072 42.9 -> 31.7; 640 to 3000 rows of 1024 to
 // 7168 channels, K 1024 to 14336, 350 shapes 1.01-2.64 times as fast (median 1.5).  Beyond two tiles to a CU the 256 x 256 tiles are (575 tiles 36 against 39, 1024 54 against 61).
-// fp32 rows that are not a multiple of four channels apart leave them a value at a time, which short K does not hide: 370 x 20089 x 256 19.7 -> 23.7, 326 x 20638 x 384 21.4 -> 24.8 (380 x 18718
-// x 1792 34.1 -> 34.8); whole pieces 249 x 19456 x 512 20.1 -> 12.4.
 // A CU with one workgroup takes 0.44 us a step, one with two 0.78 for both.  Parts cost their sums a trip through memory and a launch, about 8 us and 0.02 for each, and pay where few tiles have long
 // rows: 704 x 1856 x 10624 49.1 -> 37.7 in four, 512 x 5120 x 17408 62.0 -> 55.5 in three.
 // A launch's Workspace is never larger than what it was before these tiles, so one that a caller has measured out once holds it; the geometry that is reported (and that a record
@@ -1100,7 +1098,6 @@ int mid_parts(const orx_function& f, int rows) {
     if (f.algorithm != kAuto || tile_for(f, rows) != 0 || f.K % kBK != 0 || rows <= 128 || (f.flags != kW8 && f.flags != kQ4)) return 0;
     const int64_t tiles = split_tiles(f, rows), most = 2 * (int64_t)device_compute_units(), steps = f.K / kBK;
     if (tiles > most) return 0;
-    if (f.out_f32 && f.stride % 4 != 0 && steps <= 4 && 2 * tiles > most) return 0;
     const bool codes = f.flags == kQ4;
     if (codes && (!f.takes_workspace || (f.flags2 & kNoExpand))) return 0;
     if (use_runs(f, rows) || use_wide(f, rows) || use_tall(f, rows) || use_gemv(f, rows) || use_resident(f, rows) || use_stream(f, rows)) return 0;

@@ -89,13 +89,12 @@ def int8_panels_pay(rows, n, k, cus):
 
 def tiles_pay(codec, rows, n, k, cus):
     """Whether row-major rows over 128 x 128 tiles are faster than panels where these were the faster ones before the tiles (time of the pair over panels / row-major, 256 CUs,
-    by blocks of 16 channels to a CU; weights in cache, both layouts of codes).
-    Codes, 513-1024 rows, half to 1.5 blocks 0.92-1.64, median 1.17, where the tiles are there (split_pays); of K = 769 to 2048 up to 544 rows 0.87-1.16, 0.97, and above 1.25 blocks up to 736
-    rows 0.91-1.14, 0.97; to two blocks 1.07-1.38 above 896 rows, 0.84-1.14, 0.97 below; wider 0.80-0.93; up to half a block 0.94-1.10, 1.04 above 896 rows from K = 2048 on, 0.85-1.04,
-    0.97 below, 0.80-0.99 otherwise.  Up to 512 rows panels (where they were) 0.56-0.98.
-    int8, 129-256 rows: two to three blocks 0.97-1.11 above 208 rows, 0.92-1.03 otherwise.  257-512 rows: up to two blocks 0.96-1.43, wider 0.79-0.96 except K up to 1024: to 2.5 blocks
-    0.99-1.18, K = 256 or above 420 rows 1.00-1.13, otherwise 0.88-1.10, 1.00.  513 rows and more: above half a block 0.97-1.57 (once 0.88), up to it 0.98-1.22 above 680 rows, 0.91-1.08, 0.97
-    below."""
+    by blocks of 16 channels to a CU; 2600 shapes with weights in cache, both layouts of codes; median behind the range).
+    Codes, 513-1024 rows: half to 1.5 blocks 0.94-1.60, 1.22, where the tiles are there (split_pays); to two blocks 0.90-1.33, 1.14 above 768 rows, 0.77-1.29, 1.02 below; wider 0.77-1.23, 0.97;
+    up to half a block 0.96-1.11, 1.03 above 896 rows from K = 2048 on, 0.70-1.04, 0.86 otherwise.  Up to 512 rows panels (where they were) 0.56-0.98.
+    int8, 129-256 rows: two to three blocks 1.01-1.12, 1.06 above 208 rows, up to 208 0.85-1.14, 0.99.  257-512 rows: up to two blocks 0.97-1.41, 1.15, wider 0.89-1.18, 1.05 up to K = 1024,
+    0.84-1.26, 1.02 above.  513 rows and more: above half a block 1.07-1.67, 1.31; a third to half 0.97-1.26, 1.10 above 640 rows, 0.90-1.08, 0.98 below; up to a third 0.98-1.17, 1.06 above
+    704, 0.88-1.05, 0.95 below."""
     if rows <= 128 or -(-rows // 128) * -(-n // 128) > 2 * cus:
         return False
     blocks = -(-n // 16)
@@ -104,14 +103,12 @@ def tiles_pay(codec, rows, n, k, cus):
             return False
         if 2 * blocks <= cus:
             return rows > 896 and k >= 2048
-        if 2 * blocks <= 3 * cus:
-            return not (768 < k <= 2048 and (rows <= 544 or rows <= 736 and 4 * blocks > 5 * cus))
-        return rows > 896 and blocks <= 2 * cus
+        return 2 * blocks <= 3 * cus or (rows > 768 and blocks <= 2 * cus)
     if rows <= 256:
         return rows > 208 and 2 * cus < blocks <= 3 * cus
     if rows <= 512:
-        return blocks <= 2 * cus or k <= 1024 and (2 * blocks <= 5 * cus or rows > 420 or k <= 256)
-    return rows > 680 or 2 * blocks > cus
+        return blocks <= 2 * cus or k <= 1024
+    return 2 * blocks > cus or rows > (640 if 3 * blocks > cus else 704)
 
 
 def split_pays(rows, n, cus):

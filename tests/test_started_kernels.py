@@ -52,8 +52,6 @@ def test_few_rows_of_codes_that_take_the_streaming_kernel(rows, n, k, instead):
     ("w8", 520, 250, 14336, {}, 10, 8), ("w8", 520, 250, 14336, dict(split_k=False), 10, 1), ("w8", 520, 250, 14336, dict(workspace=False), 10, 1),
     ("w8", 641, 1930, 14336, {}, 96, 5), ("q4", 770, 256, 8320, {}, 14, 8), ("q4", 513, 528, 512, {}, 25, 1), ("q4", 512, 528, 512, {}, 0, 0),
     ("q4", 513, 528, 512, dict(workspace=False), 0, 0), ("q4", 1100, 4112, 640, dict(packed_k=64), 297, 1),
-    ("w8", 370, 20089, 256, dict(output_dtype="float32"), 0, 0), ("w8", 370, 20089, 640, dict(output_dtype="float32"), 471, 1), ("w8", 370, 20089, 256, {}, 471, 1),   # fp32 values one by one
-    ("w8", 370, 20089, 256, dict(output_dtype="float32", output_stride=20092), 471, 1), ("w8", 370, 10241, 256, dict(output_dtype="float32"), 243, 1),
     ("q4", 513, 6144, 10880, {}, 240, 1), ("q4", 513, 6144, 11008, {}, 0, 0)])                                                     # what the Workspace holds
 def test_launches_that_take_the_128_by_128_tiles(codec, rows, n, k, variant, tiles, parts):
     kernel = projection(codec, rows, n, k, **variant)
