@@ -257,18 +257,16 @@ def one_launch_routes(tokens, top_k, experts):
 
 
 def few_pays(tokens, top_k, experts, hidden, intermediate, cus):
-    """Whether five launches over tiles of 32 rows (few_rows) are faster than the seven, where the resident kernel is not there (time of the layer, seven over five, 2500 shapes, popularity
-    like 1 / rank^0.9, 256 CUs; weights in cache, and in brackets out of it).  Every workgroup of their second projection quantises its tile's rows again, which few or short rows pay for.
-    Rows of all tiles together (routed x intermediate) up to 65536 0.92-1.80, median 1.33 (1.00-1.72); up to 768 channels between and 4000 tiles x 128 channels of hidden x channels
-    between to a CU 0.90-1.55, 95 of 100 above 1.02 (0.92-1.37), beyond 0.90-1.24, median 0.99 (0.96-1.20, 1.07); up to 1152 where gate | up has at most 2.5 workgroups of 64 channels
-    to a CU 0.90-1.23, 1.04 (0.93-1.24, 1.07), beyond 0.77-1.17, 0.97 (0.82-1.22, 1.02); longer ones 0.66-1.06, 0.88 (0.73-1.16, 0.97)."""
+    """Whether five launches over tiles of 32 rows (few_rows) are faster than the seven, where the resident kernel is not there (time of the layer, seven over five, 3700 shapes, popularity
+    like 1 / rank^0.9, 256 CUs, the median behind the range; weights in cache, and in brackets out of it).  Every workgroup of their second projection quantises its tile's rows again,
+    which few or short rows pay for.  Rows of all tiles together (routed x intermediate) up to 80000 0.85-1.80, 1.30 (0.98-1.72, 1.31); above, up to 640 channels between 0.87-1.55, 1.12
+    (0.92-1.35, 1.11); up to 1152 where gate | up has at most seven workgroups of 64 channels to a CU 0.85-1.26, 1.02 (0.90-1.27, 1.05), beyond 0.77-1.31, 0.94 (0.82-1.25, 1.01); longer ones
+    0.66-1.11, 0.89 (0.72-1.16, 0.97)."""
     routed = tokens * top_k
-    if routed * intermediate <= 65536:
+    if intermediate <= 640 or routed * intermediate <= 80000:
         return True
     tiles = max(experts * (1 - math.exp(-routed / experts)), routed / 32)  # of uniform popularity
-    if intermediate <= 768:
-        return tiles * -(-hidden // 128) * intermediate <= 4000 * cus
-    return intermediate <= 1152 and tiles * -(-intermediate // 32) <= 2.5 * cus
+    return intermediate <= 1152 and tiles * -(-intermediate // 32) <= 7 * cus
 
 
 class MoeLayer:

@@ -554,9 +554,9 @@ def test_an_expert_layer_keeps_its_order_where_a_kernel_of_another_is_refused(mo
 
 
 @pytest.mark.parametrize("shape, pays", [  # tokens, top_k, experts, hidden, intermediate
-    ((2, 4, 32, 4096, 3584), True), ((42, 1, 64, 1920, 1536), True), ((43, 1, 64, 1920, 1536), False), ((832, 1, 64, 1920, 1536), False),  # rows of all tiles together
-    ((416, 1, 128, 2688, 384), True), ((416, 1, 128, 2816, 384), False), ((1000, 8, 128, 1152, 768), False), ((1000, 8, 128, 640, 768), True), ((135, 6, 128, 3968, 512), False),  # tiles x channels of the second projection
-    ((20, 8, 8, 3328, 896), True), ((60, 8, 16, 1024, 1152), True), ((75, 8, 32, 1024, 1024), False), ((60, 8, 16, 1024, 1280), False)])  # workgroups of the first
+    ((22, 1, 64, 4096, 3584), True), ((52, 1, 64, 1920, 1536), True), ((53, 1, 64, 1920, 1536), False), ((832, 1, 64, 1920, 1536), False),      # rows of all tiles together
+    ((1000, 8, 128, 4096, 640), True), ((1000, 8, 128, 4096, 768), False), ((60, 8, 16, 1024, 1152), True), ((60, 8, 16, 1024, 1280), False),      # channels between
+    ((75, 8, 56, 1024, 1024), True), ((75, 8, 57, 1024, 1024), False)])                                                                              # workgroups of the first projection
 def test_which_layers_take_the_few_rows_order(shape, pays):
     """At the lines: long rows that every workgroup of the second projection would quantise again are left to seven launches."""
     from orinfer_amd.programs import few_pays
