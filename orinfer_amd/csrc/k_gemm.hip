@@ -65,6 +65,10 @@ int dense_wide_launch(const int8_t* a, const void* w, const uint32_t* book, cons
 bool grouped_resident_eligible(int n, int k, int block_m, int tiles, int input, int epilogue, int slots);
 bool grouped_resident_preferred(int rows, int experts, int n);
 void grouped_resident_geometry(int k, int input, int epilogue, int slots, Geometry* g);
+// k_routed.hip
+bool routed_gate_up_eligible(int n, int k, int block_m, int experts, int routes);
+void routed_gate_up_geometry(int k, Geometry* g);
+int routed_gate_up_launch(const GroupedBuffers& b, int n, int k, int packed_k, int routes, hipStream_t stream);
 int grouped_resident_launch(const GroupedBuffers& b, int n, int k, int tiles, int packed_k, int input, int epilogue,
                             int slots, hipStream_t stream);
 bool grouped_bulk_eligible(int n, int k, int block_m, int packed_k, int64_t rows);
@@ -1874,10 +1878,17 @@ bool grouped_uses_resident(const orx_function& f) {
            grouped_resident_preferred(f.capacity, f.E, f.N);
 }
 
+// Input form 3: from the ids of the routes.
+bool grouped_from_routes(const orx_function& f) { return (f.flags2 & 3) == 3; }
+
 int grouped_geometry(const orx_function& f, int rows, Geometry* g) {
     (void)rows;
     if (grouped_uses_bulk(f)) {
         grouped_bulk_geometry(f.N, f.tiles, (f.flags2 >> 2) == 1, g);
+        return ORX_OK;
+    }
+    if (grouped_from_routes(f)) {
+        routed_gate_up_geometry(f.K, g);
         return ORX_OK;
     }
     if (grouped_uses_resident(f)) {
@@ -1917,8 +1928,16 @@ int grouped_launch(const orx_function& f, int rows, const Geometry& g, hipStream
     b.slot_token = reinterpret_cast<const int*>(buffer("SlotToken"));
     b.row_max = reinterpret_cast<const int*>(buffer("RowMax")), b.act = buffer("Act"), b.q = buffer("Q");
     b.tile_units = buffer("TileUnits");
+    if (grouped_from_routes(f)) {
+        auto list = [&](const char* name) { return static_cast<int*>(buffer(name)); };
+        b.routed.ids = list("IDs"), b.routed.counts = list("Counts"), b.routed.row_offsets = list("Offsets"), b.routed.tile_count = list("TileCount");
+        b.routed.tile_expert = list("TileExpert"), b.routed.tile_offsets = list("TileOffsets"), b.routed.tile_row = list("TileRow");
+        b.routed.tile_units = static_cast<int4*>(buffer("TileUnits")), b.routed.relative = list("RelativeSlot");
+        b.routed.slot_map = list("SlotMap"), b.routed.slot_token = list("SlotToken"), b.routed.experts = f.E, b.routed.top_k = f.top_k;
+    }
     if (grouped_uses_bulk(f))
         return grouped_bulk_launch(b, f.N, f.K, f.tiles, (f.flags2 & 3) == 1, (f.flags2 >> 2) == 1, grouped_bulk_narrow(f.capacity, f.E, f.N), stream);
+    if (grouped_from_routes(f)) return routed_gate_up_launch(b, f.N, f.K, f.packed_k, f.capacity, stream);
     if (grouped_uses_resident(f))
         return grouped_resident_launch(b, f.N, f.K, f.tiles, f.packed_k, f.flags2 & 3, f.flags2 >> 2, f.capacity, stream);
     GemmParams p = {};
@@ -1953,7 +1972,9 @@ int make_q2_grouped(const Variant& v, orx_function* f) {
     const std::string grouped_algorithm = v.string("algorithm", "auto", &bad);
     const std::string input = v.string("input_dtype", "int8", &bad);
     const bool gather = v.boolean("gather", false, &bad);
-    const bool tile_units = f->symbol == "e8p_decode_grouped" && v.boolean("tile_units", false, &bad);
+    const bool routes = f->symbol == "e8p_decode_grouped" && v.boolean("routes", false, &bad);
+    const bool tile_units = f->symbol == "e8p_decode_grouped" && (v.boolean("tile_units", false, &bad) || routes);
+    if (routes) f->top_k = (int)v.integer("top_k", 10, &bad);
     const std::string epilogue = v.string("epilogue", "none", &bad);
     // integer_vq_grouped carries the reference's Patch buffer and its decoder options (integer_vq.py:217-258)
     const bool vq = f->symbol == "integer_vq_grouped";
@@ -1991,7 +2012,13 @@ int make_q2_grouped(const Variant& v, orx_function* f) {
                   name);
         return ORX_ERR_BAD_VARIANT;
     }
-    f->flags2 = (input == "float16" ? 2 : gather ? 1 : 0) + (epilogue == "swiglu" ? 4 : 0);
+    f->flags2 = (input == "float16" ? 2 : routes ? 3 : gather ? 1 : 0) + (epilogue == "swiglu" ? 4 : 0);
+    // routes=true: nobody has listed the tiles; the launch reads the IDs of all rows (top_k to a token, rows of them) and leaves the metadata for those behind it
+    if (routes && (input != "int8" || !gather || epilogue != "swiglu" || f->block_m != 32 || f->E > 1024 || f->top_k <= 0 || f->top_k > 64 || f->M % f->top_k ||
+                   f->tiles < (f->M + 31) / 32 + std::min(f->E, f->M))) {
+        set_error("%s: routes=true goes with gather=true, epilogue=swiglu, block_m=32, up to 1024 experts and 64 routes to a token, and tiles for all of them", name);
+        return ORX_ERR_BAD_VARIANT;
+    }
     if (grouped_algorithm != "auto" && grouped_algorithm != "mfma" && grouped_algorithm != "stream" &&
         grouped_algorithm != "resident") {
         set_error("%s: algorithm must be auto, stream, resident or mfma", name);
@@ -2034,7 +2061,7 @@ int make_q2_grouped(const Variant& v, orx_function* f) {
                   "(algorithm auto or mfma, int8 rows, plain epilogue)", name);
         return ORX_ERR_BAD_VARIANT;
     }
-    if (f->algorithm == kResident && !grouped_resident_eligible(f->N, f->K, f->block_m, f->tiles, 0, 0, f->capacity)) {
+    if (f->algorithm == kResident && !routes && !grouped_resident_eligible(f->N, f->K, f->block_m, f->tiles, 0, 0, f->capacity)) {
         set_error("%s: algorithm=resident needs block_m=32, at most 1024 tiles, N a multiple of 32 and K/128 even or a multiple of 3, K <= 2304",
                   name);
         return ORX_ERR_BAD_VARIANT;
@@ -2048,13 +2075,14 @@ int make_q2_grouped(const Variant& v, orx_function* f) {
     // first two on the bulk kernel, which needs no RowMax (it may be null: the rows are quantised by a launch of their own).
     const bool bulk = grouped_uses_bulk(*f);
     // tile_units=true: TileUnits, as route_metadata lists them, in place of TileExpert, TileRow, Counts and Offsets (which stay in the list)
-    if (tile_units && !bulk) {
-        set_error("%s: tile_units is a form of the kernel that takes lists of 128-row tiles", name);
+    if (tile_units && !bulk && f->flags2 != 2 && !routes) {
+        set_error("%s: tile_units is a form of the kernel that takes lists of 128-row tiles, and of float16 rows", name);
         return ORX_ERR_BAD_VARIANT;
     }
     if (f->flags2 != 0 && !bulk) {
         if ((f->algorithm != kAuto && f->algorithm != kResident) ||
-            !grouped_resident_eligible(f->N, f->K, f->block_m, f->tiles, f->flags2 & 3, f->flags2 >> 2, f->capacity) ||
+            !(routes ? routed_gate_up_eligible(f->N, f->K, f->block_m, f->E, f->M)
+                     : grouped_resident_eligible(f->N, f->K, f->block_m, f->tiles, f->flags2 & 3, f->flags2 >> 2, f->capacity)) ||
             (f->algorithm == kAuto && !grouped_resident_preferred(f->capacity, f->E, f->N))) {
             set_error("%s: gather, epilogue=swiglu and input_dtype=float16 are forms of the resident kernel (block_m=32, "
                       "gathered slots that fit LDS beside the staged rows, K <= 1024 for float16 rows) where the routed rows fill the chip", name);
@@ -2063,7 +2091,7 @@ int make_q2_grouped(const Variant& v, orx_function* f) {
     }
     {
         const uint32_t nullable = 0x80000000u;
-        const bool rows16 = (f->flags2 & 3) == 2, gathered = (f->flags2 & 3) == 1, swiglu = (f->flags2 >> 2) == 1;
+        const bool rows16 = (f->flags2 & 3) == 2, gathered = (f->flags2 & 1) == 1, swiglu = (f->flags2 >> 2) == 1;
         f->args.clear();
         f->args.push_back({"A", ArgPointer, 16});
         f->args.push_back({"AS", ArgPointer, rows16 ? nullable | 2u : 2u});
@@ -2071,15 +2099,19 @@ int make_q2_grouped(const Variant& v, orx_function* f) {
         f->args.push_back({"Book", ArgPointer, 4});
         f->args.push_back({"C", ArgPointer, swiglu ? nullable | 8u : 2u});
         f->args.push_back({"Counts", ArgPointer, 4});
+        if (routes) f->args.push_back({"IDs", ArgPointer, 4});
         f->args.push_back({"Offsets", ArgPointer, 4});
         f->args.push_back({"P", ArgPointer, 16});
         // (E, K/128, N) u16 when patched; the reference binds a one-element dummy otherwise: never read, may be null
         if (vq) f->args.push_back({"Patch", ArgPointer, patched ? 2u : nullable | 2u});
         if (rows16) f->args.push_back({"Q", ArgPointer, nullable | 8u});
+        if (routes) f->args.push_back({"RelativeSlot", ArgPointer, 4});
         if (rows16 || swiglu) f->args.push_back({"RowMax", ArgPointer, bulk ? nullable | 4u : 4u});
+        if (routes) f->args.push_back({"SlotMap", ArgPointer, 4});
         if (gathered) f->args.push_back({"SlotToken", ArgPointer, 4});
         f->args.push_back({"TileCount", ArgPointer, 4});
         f->args.push_back({"TileExpert", ArgPointer, 4});
+        if (routes) f->args.push_back({"TileOffsets", ArgPointer, 4});
         f->args.push_back({"TileRow", ArgPointer, 4});
         if (tile_units) f->args.push_back({"TileUnits", ArgPointer, 16});
         f->args.push_back({"WS", ArgPointer, 2});
@@ -2344,8 +2376,8 @@ const Registration* gemm_registrations(int* count) {
     {"int8_swiglu", make_int8_swiglu, "M, N, K, dynamic_rows=false, algorithm=tensor_core|dp4a, block_m, block_n (checked, not used)",
      "A,Gate,GateScale,Output,TokenScale,Up,UpScale[,m]"},
     {"e8p_decode_grouped", make_q2_grouped,
-     "rows, E, tiles, N, K, block_m=32|64|128|8|16 (row step of the tile list), packed_k=128|64|0, dynamic_rows=false, algorithm=auto|stream|resident|mfma, input_dtype=int8|float16, gather=false, epilogue=none|swiglu, tile_units=false, few_rows=false",
-     "A,AS[,Act],Book,C,Counts,Offsets,P[,Q][,RowMax][,SlotToken],TileCount,TileExpert,TileRow[,TileUnits],WS[,m]"},
+     "rows, E, tiles, N, K, block_m=32|64|128|8|16 (row step of the tile list), packed_k=128|64|0, dynamic_rows=false, algorithm=auto|stream|resident|mfma, input_dtype=int8|float16, gather=false, epilogue=none|swiglu, tile_units=false, routes=false, top_k=10, few_rows=false",
+     "A,AS[,Act],Book,C,Counts[,IDs],Offsets,P[,Q][,RelativeSlot][,RowMax][,SlotMap][,SlotToken],TileCount,TileExpert[,TileOffsets],TileRow[,TileUnits],WS[,m]"},
     {"integer_vq", make_vq_direct,
      "E, M (rows of every expert), N, K, block_m=16|8|32|64, packed_k=128|64|0, patched=false, shared_table=false, shortbook=false, "
      "selectorbook=false (Book: raw basis (256,2) | signed values (512,4) with shortbook | selector words (256,1) with both)",

@@ -88,6 +88,7 @@ struct GroupedParams {
     const int* tile_expert;
     const int* tile_row;
     const int* tile_count;
+    const int4* tile_units;        // in place of the four lists in front: expert, first slot, rows of every tile; or null
     int n, k, k_major, tile_capacity;
     int64_t expert_weight_stride;  // bytes
 };
@@ -120,7 +121,8 @@ __global__ __launch_bounds__(kThreads) void grouped_resident_kernel(GroupedParam
     // channels a unit covers: 512 outputs, or 256 gate + the 256 matching up channels
     const int inner = p.n / 2;  // kEpilogueSwiglu: N = gate | up
     const int spans = EPILOGUE == kEpilogueSwiglu ? (inner + kSpan / 2 - 1) / (kSpan / 2) : (p.n + kSpan - 1) / kSpan;
-    const int groups = (int)gridDim.x, group = (int)blockIdx.x;
+    const int groups = (int)gridDim.x;  // each XCD gets a stretch of neighbours: tiles of one expert meet in one L2
+    const int group = groups % 8 == 0 ? ((int)blockIdx.x % 8) * (groups / 8) + (int)blockIdx.x / 8 : (int)blockIdx.x;
     const Split split = phase_two_split(kb_count);
     // forms without a phase two (see below) have no sum blocks, and the staged rows start where those would
     constexpr bool kPhaseTwo = INPUT != kInputAct && EPILOGUE == kEpiloguePlain;
@@ -139,11 +141,17 @@ __global__ __launch_bounds__(kThreads) void grouped_resident_kernel(GroupedParam
     if (wave < 4) selector = p.book[tid];
     const int listed = min(p.tile_capacity, kMaxTiles);
     const int my_tile = min(tid, listed - 1);
-    const int my_expert = p.tile_expert[my_tile], my_first = p.tile_row[my_tile];
     const int tile_count = min(p.tile_count[0], listed);
     const bool listed_here = tid < tile_count;
-    const int safe_expert = listed_here ? my_expert : 0;  // entries beyond the count are not initialised
-    const int my_count = p.counts[safe_expert], my_offset = p.offsets[safe_expert];
+    Tile my_info;
+    if (p.tile_units != nullptr) {  // one trip
+        const int4 unit = p.tile_units[my_tile];
+        my_info = {unit.x, unit.y, unit.z};
+    } else {
+        const int my_expert = p.tile_expert[my_tile], my_first = p.tile_row[my_tile];
+        const int safe_expert = listed_here ? my_expert : 0;  // entries beyond the count are not initialised
+        my_info = {my_expert, p.offsets[safe_expert] + my_first, p.counts[safe_expert] - my_first};
+    }
     if (wave < 8) {
         const int entry = tid & 255;
         const uint2 value = wave < 4 ? byte_basis_signed(selector) : byte_mask_signed((uint32_t)entry);
@@ -155,7 +163,7 @@ __global__ __launch_bounds__(kThreads) void grouped_resident_kernel(GroupedParam
         for (int i = tid; i < p.slots; i += kThreads) slot_tokens[i] = (uint16_t)p.slot_token[i];
     if (listed_here) {
         int* info = reinterpret_cast<int*>(lds + kInfoBase) + 3 * tid;
-        info[0] = my_expert, info[1] = my_offset + my_first, info[2] = min(32, my_count - my_first);
+        info[0] = my_info.expert, info[1] = my_info.row0, info[2] = min(32, my_info.rows);
     }
     __syncthreads();
     auto tile_info = [&](int tile) {
@@ -633,7 +641,7 @@ int grouped_resident_launch(const GroupedBuffers& b, int n, int k, int tiles, in
     p.w = reinterpret_cast<const uint8_t*>(b.w), p.book = b.book, p.ws = reinterpret_cast<const __half*>(b.ws);
     p.out = reinterpret_cast<__half*>(b.out);
     p.counts = b.counts, p.offsets = b.offsets, p.tile_expert = b.tile_expert, p.tile_row = b.tile_row;
-    p.tile_count = b.tile_count;
+    p.tile_count = b.tile_count, p.tile_units = static_cast<const int4*>(b.tile_units);
     p.n = n, p.k = k, p.k_major = packed_k != 0, p.tile_capacity = tiles;
     p.expert_weight_stride = (int64_t)n * (k / 8) * 2;
     Geometry g;

@@ -66,7 +66,7 @@ constexpr int router_threads() { return QUANT && LOCAL <= 8 ? 512 : 256; }
 template <int LOCAL, bool QUANT>  // LOCAL keys per lane: ceil(E / 64) rounded up to a power of two
 __global__ __launch_bounds__((router_threads<LOCAL, QUANT>())) void router_topk_kernel(
     const float* __restrict__ logits, int* __restrict__ ids, float* __restrict__ prob, int m, int e, int top_k,
-    int renormalize, const __half* __restrict__ x, int8_t* __restrict__ q, __half* __restrict__ s, int h) {
+    int renormalize, const __half* __restrict__ x, int8_t* __restrict__ q, __half* __restrict__ s, int h, int* __restrict__ row_max) {
     constexpr bool kQuantiserWaves = router_threads<LOCAL, QUANT>() == 512;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -78,6 +78,7 @@ __global__ __launch_bounds__((router_threads<LOCAL, QUANT>())) void router_topk_
     }
     float values[LOCAL];
     load_route_logits<LOCAL>(values, logits + (int64_t)row * e, e, lane);
+    if (row_max != nullptr && lane < top_k) row_max[(int64_t)row * top_k + lane] = 0;
     select_routes<LOCAL>(values, ids + (int64_t)row * top_k, prob + (int64_t)row * top_k, e, top_k, renormalize, lane);
     if (QUANT && !kQuantiserWaves) wave_quantise_row(x, q, s, row, h, lane);
 }
@@ -343,17 +344,6 @@ __global__ __launch_bounds__(256) void partition_tiles_kernel(const int* __restr
 // element, token-major stable order; a token may name an expert more than once.
 // LDS (dynamic): counters[16][E], wave-local slots[capacity assignments], scan totals.
 constexpr int kMetaWaves = 16, kMetaThreads = kMetaWaves * 64;
-// Inclusive sum over the lanes in front, by lane moves: shifts by 1, 2, 4 and 8 within a row of 16, then the last lane of rows 0 and 2 to the row
-// behind, then lane 31 to the upper half.  (A shuffle is an LDS round trip, six of them one after another.)
-__device__ __forceinline__ int wave_prefix_sum(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
-    return v;
-}
 __global__ __launch_bounds__(kMetaThreads) void route_metadata_kernel(
     const int* __restrict__ ids, int* __restrict__ counts, int* __restrict__ relative, int* __restrict__ row_offsets,
     int* __restrict__ tile_count, int* __restrict__ tile_expert, int* __restrict__ tile_offsets, int* __restrict__ tile_row,
@@ -875,23 +865,25 @@ int rows_geometry_router(const orx_function& f, int rows, Geometry* g) {
     g->block[0] = f.H > 0 && f.E <= 512 ? 512 : 256;
     return ORX_OK;
 }
-// IDs, Logits, Prob[, Q, S, X][, m]
+// IDs, Logits, Prob[, Q[, RowMax], S, X][, m]
 int router_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t s, void** args) {
     const float* logits = pointer_arg<const float>(args, 1);
     int* ids = pointer_arg<int>(args, 0);
     float* prob = pointer_arg<float>(args, 2);
-    const __half* x = f.H > 0 ? pointer_arg<const __half>(args, 5) : nullptr;
+    const int clears = f.flags2;  // row_max
+    const __half* x = f.H > 0 ? pointer_arg<const __half>(args, 5 + clears) : nullptr;
     int8_t* q = f.H > 0 ? pointer_arg<int8_t>(args, 3) : nullptr;
-    __half* scale = f.H > 0 ? pointer_arg<__half>(args, 4) : nullptr;
+    __half* scale = f.H > 0 ? pointer_arg<__half>(args, 4 + clears) : nullptr;
+    int* row_max = clears ? pointer_arg<int>(args, 4) : nullptr;
     const dim3 grid(g.grid[0]), block(g.block[0]);
 #define ORX_ROUTER(LOCAL)                                                                                              \
     do {                                                                                                               \
         if (f.H > 0)                                                                                                   \
             ORX_LAUNCH((router_topk_kernel<LOCAL, true>), grid, block, 0, s, logits, ids, prob, rows, f.E,     \
-                               f.top_k, f.flags, x, q, scale, f.H);                                                    \
+                               f.top_k, f.flags, x, q, scale, f.H, row_max);                                           \
         else                                                                                                           \
             ORX_LAUNCH((router_topk_kernel<LOCAL, false>), grid, block, 0, s, logits, ids, prob, rows, f.E,    \
-                               f.top_k, f.flags, x, q, scale, f.H);                                                    \
+                               f.top_k, f.flags, x, q, scale, f.H, row_max);                                           \
     } while (0)
     if (f.E <= 64) ORX_ROUTER(1);
     else if (f.E <= 128) ORX_ROUTER(2);
@@ -961,8 +953,16 @@ int make_router(const Variant& v, orx_function* f) {
                                            : reinterpret_cast<const void*>(&few_tokens_kernel<8>);
         return ORX_OK;
     }
+    // row_max=true: the launch also clears RowMax (M, top_k), the maxima that a projection with the SwiGLU epilogue raises
+    f->flags2 = v.boolean("row_max", false, &bad) ? 1 : 0;
+    if (bad || (f->flags2 && f->H == 0)) {
+        set_error("router_topk: row_max goes with quantize_hidden");
+        return ORX_ERR_BAD_VARIANT;
+    }
     f->args = {{"IDs", ArgPointer, 4}, {"Logits", ArgPointer, 4}, {"Prob", ArgPointer, 4}};
-    if (f->H > 0) f->args.push_back({"Q", ArgPointer, 8}), f->args.push_back({"S", ArgPointer, 2}), f->args.push_back({"X", ArgPointer, 16});
+    if (f->H > 0) f->args.push_back({"Q", ArgPointer, 8});
+    if (f->flags2) f->args.push_back({"RowMax", ArgPointer, 4});
+    if (f->H > 0) f->args.push_back({"S", ArgPointer, 2}), f->args.push_back({"X", ArgPointer, 16});
     if (f->dynamic_rows) f->args.push_back({"m", ArgI32, 4});
     f->geometry = rows_geometry_router;
     f->launch = router_launch;
@@ -1460,7 +1460,7 @@ int make_combine(const Variant& v, orx_function* f) {
 
 const Registration* moe_registrations(int* count) {
     static const Registration rows[] = {
-    {"router_topk", make_router, "M, E=512, top_k=10, renormalize=true, dynamic_rows=false, quantize_hidden=0, metadata=false, block_m=32",
+    {"router_topk", make_router, "M, E=512, top_k=10, renormalize=true, dynamic_rows=false, quantize_hidden=0, row_max=false, metadata=false, block_m=32",
      "[Counts,]IDs,Logits,Prob[,Q][,RelativeSlot,RowMax,RowOffsets][,S][,SlotMap,SlotToken,TileCount,TileExpert,TileOffsets,TileRow,TileUnits][,X][,m]"},
     {"router_projection", make_router_projection, "M, H, E, dynamic_rows=false, block_m=16, block_n=32, block_k=128, stages=2",
      "Logits,SharedGate,W,X[,m]"},

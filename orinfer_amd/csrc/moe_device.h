@@ -27,6 +27,18 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
+// Inclusive sum over the lanes in front, by lane moves: shifts by 1, 2, 4 and 8 within a row of 16, then the last lane of rows 0 and 2 to the row
+// behind, then lane 31 to the upper half.  (A shuffle is an LDS round trip, six of them one after another.)
+__device__ __forceinline__ int wave_prefix_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
+    return v;
+}
+
 // The logits of one row as one wave holds them: LOCAL = ceil(E/64) (rounded up to a power of two) per lane.
 template <int LOCAL>
 __device__ __forceinline__ void load_route_logits(float (&values)[LOCAL], const float* __restrict__ logits, int e, int lane) {

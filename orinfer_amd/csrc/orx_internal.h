@@ -148,6 +148,16 @@ int current_device();
 // Compute units of the current device (256 where no device answers).  Cached per device.
 int device_compute_units();
 
+// What a projection that works out its tiles by itself reads and writes: the ids of all assignments in token-major order, and the metadata that route_metadata writes
+// with slot_maps (tile_units in the order of the tiles).
+struct RoutedOutputs {
+    const int* ids = nullptr;
+    int *counts = nullptr, *row_offsets = nullptr, *tile_count = nullptr, *tile_expert = nullptr, *tile_offsets = nullptr, *tile_row = nullptr;
+    int4* tile_units = nullptr;
+    int *relative = nullptr, *slot_map = nullptr, *slot_token = nullptr;
+    int experts = 0, top_k = 1;
+};
+
 // Buffers of a routed expert projection as the resident kernel takes them (null where a form has none).
 struct GroupedBuffers {
     const void* a = nullptr;        // rows: int8 (slots, K); gathered: int8 (tokens, K); fp16 (slots, K) values to quantise
@@ -161,11 +171,12 @@ struct GroupedBuffers {
     const int* tile_expert = nullptr;
     const int* tile_row = nullptr;
     const int* tile_count = nullptr;
-    const void* tile_units = nullptr;  // int4 per tile, largest first: expert, first slot, rows (128-row tiles; null: the lists above)
+    const void* tile_units = nullptr;  // int4 per tile: expert, first slot, rows (null: the lists above)
     const int* slot_token = nullptr;  // gathered rows: token of every slot
     const int* row_max = nullptr;     // fp32 bits of every slot's largest magnitude: read with fp16 rows, raised by the SwiGLU epilogue
     void* act = nullptr;              // SwiGLU epilogue: fp16 (slots, N/2)
     void* q = nullptr;                // fp16 rows: the codes, optional
+    RoutedOutputs routed;
 };
 
 // One-time set-up that has to happen once per DEVICE (function attributes are per device), safe to

@@ -238,13 +238,25 @@ BULK_ROWS = 128  # tile height of the routed projections of many rows
 BULK_ROWS_PER_EXPERT = 48
 
 
+def small_tile_work(routed, experts, hidden, intermediate):
+    """Units of 32 rows (half a tile per expert more than the rows fill) x 512 channels that the projections of a layer come to, those of the second by the length of its rows."""
+    return (routed / 32 + experts / 2) * (-(-2 * intermediate // 512) + -(-hidden // 512) * intermediate / hidden)
+
+
+def routes_pay(routed, experts, hidden, intermediate, cus):
+    """Whether the four launches over 32-row tiles whose first projection works out its tiles by itself are faster than the order over 128-row tiles where that was the faster one (time of the
+    layer, the latter over the former; 75 layers of up to 4096 routes, popularity like 1 / rank^1.1, 256 CUs, by the small tiles' work to a CU).  Up to 1.5 units 0.96-1.36, median 1.08 (two of 58
+    below 0.98); above 0.87-1.19, median 0.96."""
+    return 2 * small_tile_work(routed, experts, hidden, intermediate) <= 3 * cus
+
+
 def bulk_pays(routed, experts, hidden, intermediate, cus):
     """Whether the order over 128-row tiles is faster than the one over tiles of 32 rows, five launches of either kind (time of the layer, the latter over the former; 600 shapes
     with 6 to 48 routed rows per expert, popularity like 1 / rank^1.1, 256 CUs).  What counts is the small tiles' work: units of 32 rows (half a tile per expert more than the rows
     fill) x 512 channels to a CU, those of the second projection by the length of its rows.  From 24 rows per expert and half a unit on 0.95-1.64 (median 1.2), of up to 64 experts from 16 rows
     (32 experts: 12) and 0.7 on 0.97-1.35, of up to 32 experts with 896 and more channels between, where the small tiles of the second projection hold the fewest rows, from 7 rows and 0.4 on
     0.96-1.33; otherwise 0.64-1.1 (of 128 experts with fewer rows 0.75-1.29 without a line between)."""
-    work = (routed / 32 + experts / 2) * (-(-2 * intermediate // 512) + -(-hidden // 512) * intermediate / hidden)
+    work = small_tile_work(routed, experts, hidden, intermediate)
     rows = routed / experts
     return (rows >= 24 and work >= 0.5 * cus or experts <= 64 and rows >= (12 if experts <= 32 else 16) and work >= 0.7 * cus
             or experts <= 32 and intermediate >= 896 and rows >= 7 and work >= 0.4 * cus)
@@ -310,6 +322,7 @@ class MoeLayer:
         # one launch for all routing metadata where the fused kernel applies (kernels/cuda/model/moe.py:713-764),
         # the three-kernel form otherwise
         one_launch_refused = fused_metadata is False
+        fused_metadata_asked = fused_metadata
         if fused_metadata is None:
             fused_metadata = experts <= 1024 and (16 * experts + 32 + 2 * tokens * top_k) * 4 <= 160 * 1024
         self.k_metadata = Kernel("route_metadata", block_m=block_m, **common) if fused_metadata else None
@@ -343,21 +356,35 @@ class MoeLayer:
         #   down that quantises those fp16 rows while it stages a tile (no SwiGLU->A8 launch),
         #   combine.
         # The library refuses the variants it does not serve that way, and the seven-launch program stays.
-        self.fused_stages = False
+        # Four where gate_up also works out its tiles from the ids (up to 4096 routes): no launch for the metadata, which it leaves for down and combine; the router then
+        # clears the maxima.
+        self.fused_stages = self.routes_inside = False
         self.keep_intermediates = keep_intermediates
         if fused_stages is not False and fused_metadata and signs is None and hidden % 8 == 0:
             try:
-                self.k_router_a8 = Kernel("router_topk", renormalize=True, quantize_hidden=hidden, **common)
-                self.k_metadata_slots = Kernel("route_metadata", block_m=block_m, slot_maps=True, **common)
-                self.k_gate_up_fused = Kernel("e8p_decode_grouped", N=2 * intermediate, K=hidden, gather=True,
-                                              epilogue="swiglu", **grouped)
+                if fused_metadata_asked is None:
+                    try:
+                        self.k_gate_up_routes = Kernel("e8p_decode_grouped", N=2 * intermediate, K=hidden, gather=True, epilogue="swiglu", routes=True,
+                                                       top_k=top_k, **grouped)
+                        self.k_router_clear = Kernel("router_topk", renormalize=True, quantize_hidden=hidden, row_max=True, **common)
+                        self.tile_units = torch.empty((self.tile_capacity, 4), **i32)
+                        self.routes_inside = True
+                    except OrxError as error:
+                        if error.code != ORX_ERR_BAD_VARIANT:
+                            raise
+                if not self.routes_inside:
+                    self.k_router_a8 = Kernel("router_topk", renormalize=True, quantize_hidden=hidden, **common)
+                    self.k_metadata_slots = Kernel("route_metadata", block_m=block_m, slot_maps=True, **common)
+                    self.k_gate_up_fused = Kernel("e8p_decode_grouped", N=2 * intermediate, K=hidden, gather=True,
+                                                  epilogue="swiglu", **grouped)
                 self.k_down_fused = Kernel("e8p_decode_grouped", N=hidden, K=intermediate, input_dtype="float16",
-                                           **grouped)
+                                           tile_units=self.routes_inside, **grouped)
                 self.slot_token = torch.empty(assignments, **i32)
                 self.row_max = torch.empty(assignments, **i32)
                 self.act = torch.empty((assignments, intermediate), **f16)
                 self.fused_stages = True
             except OrxError as error:
+                self.routes_inside = False
                 if fused_stages or error.code != ORX_ERR_BAD_VARIANT:
                     raise
         # Many rows: six launches over tiles of 128 rows (`block_m` is the tile height of the orders above).
@@ -419,9 +446,35 @@ class MoeLayer:
             except OrxError as error:
                 if error.code != ORX_ERR_BAD_VARIANT:
                     raise
+        # The four launches also where nothing but the seven is left (1.12-1.28 times as fast, 5 layers), and over the order for many rows where they are the faster ones.  `bulk` says that that
+        # one is served and would run; `routes_first` that these run before either.
+        self.routes_first = False
+        if (fused_stages is None and not self.few and not keep_intermediates and signs is None and self.fused_dispatch and fused_metadata and fused_metadata_asked is None
+                and packed_k == 128 and block_m == 32 and grouped_algorithm == "auto"
+                and (routes_pay(assignments, experts, hidden, intermediate, torch.cuda.get_device_properties(self.w1.device).multi_processor_count) if self.bulk
+                     else not self.fused_stages)):
+            if not self.routes_inside:
+                try:
+                    resident = dict(grouped, algorithm="resident")
+                    served = dict(
+                        k_gate_up_routes=Kernel("e8p_decode_grouped", N=2 * intermediate, K=hidden, gather=True, epilogue="swiglu", routes=True, top_k=top_k, **resident),
+                        k_router_clear=Kernel("router_topk", renormalize=True, quantize_hidden=hidden, row_max=True, **common),
+                        k_down_fused=Kernel("e8p_decode_grouped", N=hidden, K=intermediate, input_dtype="float16", tile_units=True, **resident))
+                    vars(self).update(served)
+                    if not self.bulk:
+                        self.slot_token, self.act = torch.empty(assignments, **i32), torch.empty((assignments, intermediate), **f16)
+                        self.tile_units = torch.empty((self.tile_capacity, 4), **i32)
+                    elif self.tile_units.shape[0] < self.tile_capacity:
+                        self.tile_units = torch.empty((self.tile_capacity, 4), **i32)
+                    self.row_max = torch.empty(assignments, **i32)
+                    self.routes_inside = True
+                except OrxError as error:
+                    if error.code != ORX_ERR_BAD_VARIANT:
+                        raise
+            self.routes_first = self.routes_inside
         # the dispatched rows and the gate | up outputs, which the orders for long prompts and for few rows do without
         self.d = self.ds = self.gate_up_out = None
-        if not self.bulk and not self.few:
+        if not self.bulk and not self.few and not self.routes_first:
             self.d = torch.empty((assignments, hidden), **i8)
             self.ds = torch.empty((assignments, 1), **f16)
             self.gate_up_out = torch.empty((assignments, 2 * intermediate), **f16)
@@ -429,6 +482,8 @@ class MoeLayer:
 
     def run(self, x16, logits, stream=None):
         s = current_stream() if stream is None else stream
+        if self.routes_first:
+            return self._run_routes_inside(x16, logits, s)
         if self.bulk:
             return self._run_bulk(x16, logits, s)
         if self.fused_stages:
@@ -500,6 +555,8 @@ class MoeLayer:
 
     def _run_fused(self, x16, logits, s):
         keep = self.keep_intermediates
+        if self.routes_inside:
+            return self._run_routes_inside(x16, logits, s)
         self.k_router_a8(stream=s, IDs=self.ids, Logits=logits, Prob=self.prob, Q=self.a_q, S=self.a_s, X=x16)
         self.k_metadata_slots(stream=s, Counts=self.counts, IDs=self.ids, RelativeSlot=self.relative, RowMax=self.row_max,
                               RowOffsets=self.row_offsets, SlotMap=self.slot_map, SlotToken=self.slot_token,
@@ -511,6 +568,18 @@ class MoeLayer:
                              P=self.w1, RowMax=self.row_max, SlotToken=self.slot_token, WS=self.s1, **routed)
         self.k_down_fused(stream=s, A=self.act, AS=self.h_s if keep else None, C=self.down_out, P=self.w2,
                           Q=self.h_q if keep else None, RowMax=self.row_max, WS=self.s2, **routed)
+        self.k_combine(stream=s, Expert=self.down_out, Output=self.out, Prob=self.prob, Shared=None, SharedGate=None,
+                       SlotMap=self.slot_map)
+        return self.out
+
+    def _run_routes_inside(self, x16, logits, s):
+        keep = self.keep_intermediates
+        self.k_router_clear(stream=s, IDs=self.ids, Logits=logits, Prob=self.prob, Q=self.a_q, RowMax=self.row_max, S=self.a_s, X=x16)
+        routed = dict(Book=self.book, Counts=self.counts, Offsets=self.row_offsets, RowMax=self.row_max, TileCount=self.tile_count,
+                      TileExpert=self.tile_expert, TileRow=self.tile_row, TileUnits=self.tile_units)
+        self.k_gate_up_routes(stream=s, A=self.a_q, AS=self.a_s, Act=self.act, C=self.gate_up_out if keep else None, IDs=self.ids, P=self.w1,
+                              RelativeSlot=self.relative, SlotMap=self.slot_map, SlotToken=self.slot_token, TileOffsets=self.tile_offsets, WS=self.s1, **routed)
+        self.k_down_fused(stream=s, A=self.act, AS=self.h_s if keep else None, C=self.down_out, P=self.w2, Q=self.h_q if keep else None, WS=self.s2, **routed)
         self.k_combine(stream=s, Expert=self.down_out, Output=self.out, Prob=self.prob, Shared=None, SharedGate=None,
                        SlotMap=self.slot_map)
         return self.out

@@ -448,6 +448,93 @@ def test_few_rows_takes_no_more_of_a_unit_than_a_tile_has(slots, units, written)
     assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("tokens,e,top_k,hidden,inter,spread", [
+    (1, 1, 1, 256, 16, 1), (33, 3, 1, 384, 48, 1),         # the least; an odd number of K blocks, a wave with one block of channels and waves with none
+    (256, 128, 8, 512, 272, 2), (257, 129, 8, 256, 32, 2),   # 2048 routes of 128 experts, and beyond either
+    (512, 512, 8, 256, 256, 1), (64, 64, 64, 256, 32, 1),    # the most routes and experts; every expert names every token
+    (680, 8, 6, 384, 304, 8), (90, 300, 3, 896, 528, 0)])    # experts of many tiles, units of both parts of one; experts without rows
+@pytest.mark.parametrize("packed_k", [128, 0])
+def test_gate_up_from_routes(tokens, e, top_k, hidden, inter, spread, packed_k):
+    """Tiles worked out by the projection itself: gate | up, its product and the maxima are what oracle and quantiser say, the metadata what the oracle lists."""
+    rng = np.random.default_rng(orc.SEED + tokens + e)
+    rank = np.log(rng.permutation(e) + 1.0)
+    ids = np.argsort(-(rng.normal(size=(tokens, e)) - spread * rank), axis=1)[:, :top_k].astype(np.int32)
+    routes = tokens * top_k
+    codes = rng.integers(0, 65536, (e, 2 * inter, hidden // 8), dtype=np.uint16)
+    w = np.stack([orc.q2_integers(one, TABLE) for one in codes])
+    ws = (rng.uniform(0.5, 1.5, (e, 2 * inter)) * 0.05 / np.sqrt(hidden)).astype(np.float16)
+    a_q, a_s = rng.integers(-127, 128, (tokens, hidden), dtype=np.int8), rng.uniform(0.01, 0.03, (tokens, 1)).astype(np.float16)
+    counts, rel = orc.expert_histogram(ids, e)
+    rows, first_tile, total = orc.expert_offsets(counts, 32)
+    d, ds, slot = orc.expert_dispatch(a_q, a_s, ids, rel, rows)
+    capacity = -(-routes // 32) + min(e, routes)
+    stored = codes if packed_k == 0 else np.stack([orc.q2_pack_k128(one) for one in codes])
+    ints = lambda *shape: torch.full(shape, -5, dtype=torch.int32, device=gu.DEV)
+    out = dict(Counts=ints(e), Offsets=ints(e), RelativeSlot=ints(tokens, top_k), SlotMap=ints(tokens, top_k), SlotToken=ints(routes + 1), TileCount=ints(1),
+               TileExpert=ints(capacity + 1), TileOffsets=ints(e), TileRow=ints(capacity + 1), TileUnits=ints(capacity + 1, 4))
+    act = torch.full((routes + 1, inter), 55.0, dtype=torch.float16, device=gu.DEV)
+    both = torch.full((routes + 1, 2 * inter), 55.0, dtype=torch.float16, device=gu.DEV)
+    variant = dict(rows=routes, E=e, tiles=capacity, N=2 * inter, K=hidden, block_m=32, packed_k=packed_k, gather=True, epilogue="swiglu", algorithm="resident")
+    kern = gu.kernel("e8p_decode_grouped", routes=True, top_k=top_k, **variant)
+    for kept in (both, None):
+        row_max = torch.zeros(routes + 1, dtype=torch.int32, device=gu.DEV)
+        act.fill_(55.0)
+        kern(A=gu.dev(a_q), AS=gu.dev(a_s), Act=act, Book=gu.book(), C=kept, IDs=gu.dev(ids), P=gu.dev(stored), RowMax=row_max, WS=gu.dev(ws), **out)
+        want = torch.full_like(both, 55.0)
+        want[:routes] = gu.dev(orc.grouped_project(d, ds, w, ws, counts, rows))
+        assert torch.equal(both, want)
+        product = torch.empty((routes, inter), dtype=torch.float16, device=gu.DEV)
+        gu.kernel("swiglu", I=inter)(X=want[:routes].contiguous(), Y=product, rows=routes)
+        assert torch.equal(act[:routes], product) and bool((act[routes] == 55).all())
+        assert torch.equal(row_max[:routes], product.abs().amax(1).float().view(torch.int32)) and int(row_max[routes]) == 0
+    host = {name: gu.host(t) for name, t in out.items()}
+    tiles = int(host["TileCount"][0])
+    assert tiles == int(np.asarray(total).ravel()[0])
+    for name, value in (("Counts", counts), ("Offsets", rows), ("RelativeSlot", rel), ("SlotMap", slot), ("TileOffsets", first_tile)):
+        np.testing.assert_array_equal(host[name], value, err_msg=name)
+    token_of = np.full(routes + 1, -5, np.int32)
+    token_of[slot.ravel()] = np.repeat(np.arange(tokens, dtype=np.int32), top_k)
+    np.testing.assert_array_equal(host["SlotToken"], token_of)
+    listed = [(x, rows[x] + r, min(32, counts[x] - r), 0) for x in range(e) for r in range(0, counts[x], 32)]
+    np.testing.assert_array_equal(host["TileUnits"][:tiles], np.array(listed, np.int32))
+    np.testing.assert_array_equal(host["TileExpert"][:tiles], [x for x, _, _, _ in listed])
+    np.testing.assert_array_equal(host["TileRow"][:tiles], [row - rows[x] for x, row, _, _ in listed])
+    for name in ("TileUnits", "TileExpert", "TileRow"):
+        assert (host[name][tiles:] == -5).all()
+
+
+def test_gate_up_from_routes_refuses_what_it_cannot_take():
+    good = dict(rows=64, E=8, tiles=10, N=64, K=256, block_m=32, gather=True, epilogue="swiglu", algorithm="resident", routes=True, top_k=4)
+    gu.kernel("e8p_decode_grouped", **good)
+    for bad in (dict(tiles=9), dict(top_k=5), dict(top_k=0), dict(gather=False), dict(epilogue="none"), dict(block_m=64), dict(N=48), dict(K=128), dict(K=2944), dict(E=513, tiles=66),
+                dict(rows=4100, tiles=137)):
+        with pytest.raises(gu.lib.OrxError):
+            gu.kernel("e8p_decode_grouped", **{**good, **bad})
+
+
+@pytest.mark.parametrize("tokens,experts,top_k,hidden,inter,bulk", [(477, 64, 2, 1024, 1024, False), (200, 32, 8, 1792, 768, True), (230, 64, 6, 1152, 768, True)])
+def test_four_launches_first_give_the_bits_of_seven(tokens, experts, top_k, hidden, inter, bulk):
+    """Where the seven launches were left and in front of the order for many rows, eagerly and replayed with new routing."""
+    c = workloads.config3(tokens=tokens, experts=experts, top_k=top_k, hidden=hidden, intermediate=inter)
+    args = (tokens, experts, top_k, hidden, inter, c["gate_up"], c["gate_up_scales"], c["down"], c["down_scales"])
+    seven, four = programs.MoeLayer(*args, fused_stages=False), programs.MoeLayer(*args)
+    assert four.routes_first and four.bulk == bulk and four.d is None
+    x, logits = gu.dev(c["x"]), gu.dev(c["logits"])
+    assert torch.equal(four.run(x, logits), seven.run(x, logits))
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    gu.sync()
+    with torch.cuda.graph(graph, stream=stream):
+        four.run(x, logits, stream=stream.cuda_stream)
+    for step in range(3):
+        logits.copy_(gu.dev(np.random.default_rng(step).normal(size=c["logits"].shape).astype(np.float32)))
+        four.counts.fill_(-7)
+        gu.sync()
+        graph.replay()
+        gu.sync()
+        replayed = four.out.clone()
+        assert torch.equal(seven.run(x, logits), replayed)
+
+
 def test_grouped_resident_rejects_shapes_it_cannot_take():
     for bad in (dict(N=200, K=384), dict(N=256, K=128), dict(N=256, K=3072), dict(N=256, K=512, block_m=64)):
         variant = dict(rows=64, E=4, tiles=6, block_m=32, packed_k=128, algorithm="resident")
