@@ -837,11 +837,12 @@ bool use_runs(const orx_function& f, int rows) {
 //   none, one block K = 2176 / 3200 / 5376 / 8448 / 13952 0.96-1.03 / 0.87-0.95 / 0.79-0.86 / 0.62-0.77 / 0.62-0.70 (3904 x 8448 14.5 -> 10.9 us, K-major 1392 x 13952 17.4 -> 11.8); two blocks up to
 //     K = 7424 0.94-1.16, from 8448 on 0.81-0.99; three K = 3328 / 4224 / 6528 / 10368 1.01 / 0.95 / 0.86 / 0.79; four 0.96-1.24; five K = 4352 / 5888 / 7424 1.01 / 0.96 / 0.91;
 //   eight lanes, one block K = 2304 / 5888 / 11520 0.80-0.89 / 0.66 / 0.57; two K = 2304 / 3328 / 9984 0.93-0.97 / 0.9-0.93 / 0.73-0.77; three K = 3328 / 4352 / 9984 1.02 / 0.97 / 0.87; five 1.02-1.21;
-//   sixteen, one block K = 2560 / 6656 / 15872 0.82-0.85 (1.03 behind a norm in a graph) / 0.82-0.94 / 0.76-0.84 (5632 and 6144 0.86-0.99), two 0.91-1.14, more 1.03-1.45; thirty-two 1.02-1.41 (6144 0.84-0.98).
+//   sixteen, one block K = 2560 / 6656 / 15872 0.82-0.85 (1.03 behind a norm in a graph) / 0.82-0.94 / 0.76-0.84 (5632 and 6144 0.86-0.99), two 0.91-1.14, more 1.03-1.45; thirty-two 1.02-1.41 (6144 0.84-0.98), K-major, where the launch
+//     takes them in the place of sixteen, K = 4096 and 5120 0.99-1.13, 6144 and more 0.86-1.0.
 bool runs_for_one_row(const orx_function& f) {
     const int blocks = channel_blocks_per_cu(f.N), lanes = gemv_replicated_lanes(f, 1);
     if (f.flags != kQ4 || lanes == 32 || blocks == 4 || blocks > 5) return false;
-    if (lanes == 16) return blocks == 1 && f.K >= 3584;
+    if (lanes == 16) return blocks == 1 && f.K >= 3584 && (f.packed_k == 0 || f.K % 1024 != 0 || f.K > 5120);
     if (lanes == 8) return f.K >= (blocks == 1 ? 2304 : blocks == 2 ? 3072 : 4096) && blocks <= 3;
     return f.K >= (blocks == 1 ? 2816 : blocks == 2 ? 8192 : blocks == 3 ? 4096 : 5632);
 }

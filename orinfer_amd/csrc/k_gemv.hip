@@ -515,6 +515,7 @@ __global__ __launch_bounds__(kBankedThreads) void gemv_banked_kernel(
         amax = wave_max_magnitude(amax);
         if (lane == 0) wave_max[wave] = amax;
         __syncthreads();
+        prefetch(2, D);  // (everybody's small reads are back: 0.7 us before the barrier that publishes the planes)
         // the 16 wave maxima, one per lane of a row, reduced with lane controls (no LDS round trips):
         // quad permutes, then the mirror of each half row, then the mirror of the row
         amax = wave_max[lane & 15];
@@ -600,7 +601,7 @@ __global__ __launch_bounds__(kBankedThreads) void gemv_banked_kernel(
         for (int r = 0; r < MR; ++r) wave_sums[r * 16 + wave] = wave_total[r];
     }
     __syncthreads();
-    prefetch(2, D);
+    if (!X16) prefetch(2, D);
 
     const uint32_t column = kMskBase + 4u * (uint32_t)lane;
     // sum of each activation row (scalar), the steps at which this lane's column holds an
@@ -610,9 +611,13 @@ __global__ __launch_bounds__(kBankedThreads) void gemv_banked_kernel(
     for (int r = 0; r < MR; ++r)
         row_sum[r] = __builtin_amdgcn_readlane(wave_sum_to_last_lane(lane < 16 ? wave_sums[r * 16 + lane] : 0), 63);
     uint32_t flag_lo = 0, flag_hi = 0;
-    for (int step = 0; step < steps; ++step) {
-        const uint32_t bit = chunk_flags[sub + step * LPR];
-        if (step < 32) flag_lo |= bit << step; else flag_hi |= bit << (step - 32);
+    constexpr int kFlagsAtOnce = HOLD ? D : 8;  // (one read after another is an LDS latency a step in front of the first codes)
+    for (int first = 0; first < steps; first += kFlagsAtOnce) {
+        uint32_t bits = 0;
+#pragma unroll
+        for (int i = 0; i < kFlagsAtOnce; ++i) bits |= (uint32_t)chunk_flags[sub + min(first + i, steps - 1) * LPR] << i;
+        // (beyond the last step: set and not looked at; a group of eight does not cross the halves)
+        if (first < 32) flag_lo |= bits << first; else flag_hi |= bits << (first - 32);
     }
     const uint64_t flagged = (uint64_t)flag_lo | (uint64_t)flag_hi << 32;
     const uint64_t any_flagged = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)wave_or_to_last_lane(flag_lo), 63) |
@@ -755,21 +760,49 @@ int gemv_geometry(const orx_function& f, int rows, Geometry* g) {
 static thread_local const int8_t* pending_signs = nullptr;
 static thread_local int8_t* pending_codes = nullptr;
 
+// The ring depth in {6,5,4} that pads a row's step count the least.
+int ring_depth_for(int steps) {
+    int best_pad = 1 << 30, depth = 4;
+    for (int candidate : {6, 5, 4}) {
+        const int pad = (int)ceil_div((uint32_t)steps, (uint32_t)candidate) * candidate - steps;
+        if (pad < best_pad) best_pad = pad, depth = candidate;
+    }
+    return depth;
+}
+
+// The lanes to a channel that a launch takes at one row, by the channels that a CU gets (the reported geometry is the same for all, and so is what `slots` says to other rules).  With few
+// channels wide ones leave no wave without a task and put a whole row into the ring at once; with many, narrow ones keep four or five steps to a row, which are held.  Time of
+// narrow over wide, fp16 rows / int8 rows, weights out of cache:
+//   K-major, 16 over 32: K = 3072 1.08-1.17 / 1.05-1.18; 4096 to 8192 up to 20 channels 1.10-1.30 / 1.15-1.43, to 40 0.99-1.18 / 0.98-1.13, 48 1.01-1.10 / 0.95-0.98, 56 and more 0.91-1.04 /
+//     0.87-0.99; 2048 0.83-1.03 / 0.86-1.03.  5120 x 5120 8.6 -> 7.0 us with the rotation.
+//   K-major, 8 over 16: K = 1024 0.88-1.0 / 0.89-0.99 (34816 channels 7.7 -> 6.9 us); 1536 and 2048 1.0-1.23 / 0.98-1.31.
+//   row-major, 16 over 32: K = 2048 0.82-0.98 / 0.86-0.99; 1024 up to 16 channels 1.04 / 1.03-1.06, from 28 on 0.86-0.99 / 0.84-0.99; 3072 and more 0.98-1.29 / 0.95-1.42.
+int launch_layout(const orx_function& f, int rows) {
+    const int layout = f.slots >> 8, lanes = layout & (kKMajorLayout - 1);
+    if (rows != 1 || f.K % 1024 != 0) return layout;
+    const int cus = device_cus();
+    if (layout == lanes) return f.K == 2048 || (f.K == 1024 && f.N > 24 * cus) ? 16 : layout;
+    if (f.K == 1024) return kKMajorLayout + 8;
+    return f.K >= 3072 && f.N <= (f.K == 3072 ? 80 : f.input_f16 ? 48 : 40) * cus ? kKMajorLayout + 32 : layout;
+}
+
 template <int D, int LPR>  // LPR: the kernel's LAYOUT (lanes per row, + 64 for K-major codes)
 int gemv_launch_banked(const orx_function& f, int rows, const Geometry& g, hipStream_t stream, const int8_t* a,
                        const uint4* w, const uint32_t* book, const __half* ws, const __half* as, void* out) {
     const dim3 grid(g.grid[0]), block(kBankedThreads);
-    const bool hold = f.K / 32 / (LPR & (kKMajorLayout - 1)) == D;  // a row's steps fill the ring exactly
+    // a row's steps fill the ring exactly; six held chunks spill (K-major 17408 x 3072 15.2 us, without 9.9)
+    constexpr bool kHolds = D <= 5;
+    const bool hold = kHolds && f.K / 32 / (LPR & (kKMajorLayout - 1)) == D;
     switch (mr_for(rows)) {
         case 1:
             if (f.input_f16 && hold)
-                ORX_LAUNCH((gemv_banked_kernel<kQ4, 1, D, LPR, true, true>), grid, block, g.shared, stream, a, w,
+                ORX_LAUNCH((gemv_banked_kernel<kQ4, 1, D, LPR, kHolds, true>), grid, block, g.shared, stream, a, w,
                                    book, ws, as, out, f.N, f.K, f.stride, rows, (int)f.out_f32 | (f.packed_k == 64 ? 2 : 0), pending_signs, pending_codes);
             else if (f.input_f16)
                 ORX_LAUNCH((gemv_banked_kernel<kQ4, 1, D, LPR, false, true>), grid, block, g.shared, stream, a, w,
                                    book, ws, as, out, f.N, f.K, f.stride, rows, (int)f.out_f32 | (f.packed_k == 64 ? 2 : 0), pending_signs, pending_codes);
             else if (hold)
-                ORX_LAUNCH((gemv_banked_kernel<kQ4, 1, D, LPR, true>), grid, block, g.shared, stream, a, w, book,
+                ORX_LAUNCH((gemv_banked_kernel<kQ4, 1, D, LPR, kHolds>), grid, block, g.shared, stream, a, w, book,
                                    ws, as, out, f.N, f.K, f.stride, rows, (int)f.out_f32 | (f.packed_k == 64 ? 2 : 0), pending_signs, pending_codes);
             else
                 ORX_LAUNCH((gemv_banked_kernel<kQ4, 1, D, LPR, false>), grid, block, g.shared, stream, a, w, book,
@@ -790,7 +823,7 @@ int gemv_launch_banked(const orx_function& f, int rows, const Geometry& g, hipSt
 template <int LPR>
 int gemv_launch_banked_depth(const orx_function& f, int rows, const Geometry& g, hipStream_t stream, const int8_t* a,
                              const uint4* w, const uint32_t* book, const __half* ws, const __half* as, void* out) {
-    switch (f.slots & 255) {
+    switch (ring_depth_for(f.K / 32 / (LPR & (kKMajorLayout - 1)))) {
         case 4: return gemv_launch_banked<4, LPR>(f, rows, g, stream, a, w, book, ws, as, out);
         case 5: return gemv_launch_banked<5, LPR>(f, rows, g, stream, a, w, book, ws, as, out);
         default: return gemv_launch_banked<6, LPR>(f, rows, g, stream, a, w, book, ws, as, out);
@@ -804,7 +837,8 @@ int gemv_launch_codec(const orx_function& f, int rows, const Geometry& g, hipStr
     const uint4* wp = reinterpret_cast<const uint4*>(w);
     if constexpr (CODEC == kQ4) {
         if (use_banked(f, mr_for(rows))) {
-            switch (f.slots >> 8) {
+            switch (launch_layout(f, rows)) {
+                case kKMajorLayout + 32: return gemv_launch_banked_depth<kKMajorLayout + 32>(f, rows, g, stream, a, wp, book, ws, as, out);
                 case 32: return gemv_launch_banked_depth<32>(f, rows, g, stream, a, wp, book, ws, as, out);
                 case kKMajorLayout + 16: return gemv_launch_banked_depth<kKMajorLayout + 16>(f, rows, g, stream, a, wp, book, ws, as, out);
                 case kKMajorLayout + 8: return gemv_launch_banked_depth<kKMajorLayout + 8>(f, rows, g, stream, a, wp, book, ws, as, out);
@@ -1401,12 +1435,7 @@ int gemv_configure(orx_function* f, int codec, int passes_override) {
         // and 15.0 with 32), 8 for a K that is a multiple of 256 only
         if (f->packed_k != 0) lanes_per_row = chunks % 16 == 0 ? 16 : chunks % 8 == 0 ? 8 : 0;
         if (lanes_per_row) {
-            const int steps = chunks / lanes_per_row;
-            int best_pad = 1 << 30, depth = 4;
-            for (int candidate : {6, 5, 4}) {
-                const int pad = ceil_div(steps, candidate) * candidate - steps;
-                if (pad < best_pad) best_pad = pad, depth = candidate;
-            }
+            const int steps = chunks / lanes_per_row, depth = ring_depth_for(steps);
             // the overflow flags hold one bit per step in a 64-bit word per lane column
             if (steps <= 64) f->slots = depth | (lanes_per_row + (f->packed_k != 0 ? kKMajorLayout : 0)) << 8;
         }
@@ -1440,15 +1469,16 @@ static int gemv_opt_in_current_device() {
     ORX_OPT_IN((gemv_rowmajor_kernel<kW8, 4>))
     limit = (int)kBankedLdsLimit;
 #define ORX_OPT_IN_BANKED(depth, lanes)                       \
-    ORX_OPT_IN((gemv_banked_kernel<kQ4, 1, depth, lanes, true>))     \
+    ORX_OPT_IN((gemv_banked_kernel<kQ4, 1, depth, lanes, (depth <= 5)>))     \
     ORX_OPT_IN((gemv_banked_kernel<kQ4, 1, depth, lanes, false>))    \
-    ORX_OPT_IN((gemv_banked_kernel<kQ4, 1, depth, lanes, true, true>))  \
+    ORX_OPT_IN((gemv_banked_kernel<kQ4, 1, depth, lanes, (depth <= 5), true>))  \
     ORX_OPT_IN((gemv_banked_kernel<kQ4, 1, depth, lanes, false, true>)) \
     ORX_OPT_IN((gemv_banked_kernel<kQ4, 2, depth, lanes, false>))    \
     ORX_OPT_IN((gemv_banked_kernel<kQ4, 4, depth, lanes, false>))
     ORX_OPT_IN_BANKED(4, 16) ORX_OPT_IN_BANKED(5, 16) ORX_OPT_IN_BANKED(6, 16)
     ORX_OPT_IN_BANKED(4, 32) ORX_OPT_IN_BANKED(5, 32) ORX_OPT_IN_BANKED(6, 32)
     ORX_OPT_IN_BANKED(4, kKMajorLayout + 8) ORX_OPT_IN_BANKED(5, kKMajorLayout + 8) ORX_OPT_IN_BANKED(6, kKMajorLayout + 8)
+    ORX_OPT_IN_BANKED(4, kKMajorLayout + 32) ORX_OPT_IN_BANKED(5, kKMajorLayout + 32) ORX_OPT_IN_BANKED(6, kKMajorLayout + 32)
     ORX_OPT_IN_BANKED(4, kKMajorLayout + 16) ORX_OPT_IN_BANKED(5, kKMajorLayout + 16) ORX_OPT_IN_BANKED(6, kKMajorLayout + 16)
 #undef ORX_OPT_IN_BANKED
 #undef ORX_OPT_IN

@@ -489,6 +489,33 @@ def test_q4_gemv_rotates_and_quantises_fp16_input(n, k, packed_k):
         gu.kernel("e8p_q4_projection", M=1, N=n, K=k, rotate=True)
 
 
+@pytest.mark.parametrize("n,k,packed_k", [
+    (1027, 5120, 128), (515, 5120, 64), (517, 3072, 128), (35, 6144, 128), (34, 8192, 64),                        # 32 lanes to a K-major channel: 5, 3, 6 and 8 steps
+    (10240, 4096, 128), (10241, 4096, 128), (12289, 4096, 128), (20481, 3072, 128), (258, 3072, 0), (35, 6144, 0),  # both sides of its lines; six steps, which nothing holds
+    (70, 1024, 128), (71, 1024, 64), (6144, 1024, 0), (6145, 1024, 0), (67, 2048, 0), (66, 2048, 128)])             # 8 lanes; 16 where 32 divide
+def test_one_row_with_other_lanes_than_the_handle_says(n, k, packed_k):
+    """The lanes to a channel that a launch takes by the channels that a CU gets, int8 and rotated fp16 rows, codes on both sides of the overflow plane."""
+    rng = np.random.default_rng(orc.SEED + n + k)
+    packed = rng.integers(0, 2**32, (n, k // 8), dtype=np.uint32)
+    scales = rng.uniform(0.005, 0.02, n).astype(np.float16)
+    weights = orc.q4_integers(packed, TABLE)
+    stored = gu.dev(packed if packed_k == 0 else orc.q4_pack_k(packed, packed_k))
+    q = rng.integers(-128, 128, (1, k), dtype=np.int8)
+    q[0, k // 2 :] = np.clip(q[0, k // 2 :], -127, 119)  # (chunks without an overflow)
+    ones = np.ones(1, np.float16)
+    got = gu.q4_project(gu.dev(q), gu.dev(ones), stored, gu.dev(scales), algorithm="gemv", packed_k=packed_k)
+    np.testing.assert_array_equal(gu.host(got), orc.project(q, ones[:, None], weights, scales))
+    signs = rng.choice(np.array([-1, 1], np.int8), k)
+    x = rng.normal(size=(1, k)).astype(np.float16)
+    kern = gu.kernel("e8p_q4_projection", M=1, N=n, K=k, packed_k=packed_k, input_dtype="float16", rotate=True)
+    out = torch.full((2, n), 9.0, dtype=torch.float16, device=gu.DEV)
+    scale = torch.empty(1, dtype=torch.float16, device=gu.DEV)
+    kern(A=gu.dev(x), AS=scale, Book=gu.book(), Out=out, S=gu.dev(scales), Signs=gu.dev(signs), W=stored)
+    a_q, a_s = orc.rotate_a8(x, signs)
+    np.testing.assert_array_equal(gu.host(out)[:1], orc.project(a_q, a_s, weights, scales))
+    assert (gu.host(out)[1] == 9).all()
+
+
 @pytest.mark.parametrize("n,k,packed_k,single", [(200, 1024, 0, True), (136, 2048, 128, True), (48, 8192, 0, True), (40, 8704, 0, False), (64, 1152, 128, False)])
 def test_one_row_program_gives_the_bits_of_two_launches(n, k, packed_k, single):
     """One launch quantises the row, publishes its codes and projects; shapes and addresses it does not take keep the two launches."""
