@@ -918,22 +918,28 @@ __device__ __forceinline__ int route_dot_two_codes(uint32_t word, const uint4& v
 }
 
 // Two launches of the one-token expert layer can run inside this kernel's set-up:
-//   LOCAL > 0 (route_logits): `ids` is an output.  Wave 0 of every workgroup selects the token's
-//     routes from `logits` (the router's rule, moe_device.h) while the others build the tables; the
-//     first workgroup writes ids and probabilities for the combine.  Selecting eight routes of one
-//     token costs a wave about a microsecond; a router launch in front costs three to four.
+//   LOCAL > 0 (route_logits): `ids` is an output.  Every workgroup selects the token's
+//     routes from `logits` (the router's rule, moe_device.h) beside its tables: up to 256 experts each wave counts for a share of them
+//     who comes in front of whom, above that wave 0 selects rank after rank; the
+//     first workgroup writes ids and probabilities for the combine.  A router launch in front costs three to four microseconds.
 //   x16 == 2 (fused_swiglu): `a` holds fp16 gate|up rows, one per route; the row becomes
 //     fp16(silu(gate) * up), then A8 codes, on its way into LDS (the SwiGLU -> A8 launch between the
 //     two projections disappears); the first workgroup of a route writes its scale.
+// act (epilogue=swiglu): the rows are gate | up and a workgroup owns 16 gate and the 16 matching up channels, so that it also writes fp16(silu(gate) * up): the second projection
+// then finds the values that its workgroups would each make again (8 routes of 512: 1 us of 5 in 256 workgroups).
 template <int LOCAL>
 __global__ __launch_bounds__(kRouteThreads) void route_gemv_kernel(
     const int8_t* __restrict__ a, const __half* __restrict__ as, const uint32_t* __restrict__ book, __half* __restrict__ c,
     const int32_t* __restrict__ ids, const uint16_t* __restrict__ p, const __half* __restrict__ ws, int experts, int n,
-    int k, int shared_input, int x16, const float* __restrict__ logits, float* __restrict__ prob, int renormalize) {
+    int k, int shared_input, int x16, const float* __restrict__ logits, float* __restrict__ prob, int renormalize, __half* __restrict__ act) {
     extern __shared__ __align__(16) uint8_t route_lds[];
     __shared__ float route_wave_max[kRouteWaves];
     __shared__ int selected_ids[64];
     __shared__ float selected_prob[64];
+    constexpr bool kCounts = LOCAL > 0 && LOCAL <= 4;
+    __shared__ uint2 in_front[kCounts ? LOCAL * 64 : 1];  // of every expert, a byte to a wave
+    __shared__ __align__(16) uint32_t route_keys[kCounts ? LOCAL * 64 : 1];
+    __shared__ uint32_t selected_keys[kCounts ? 64 : 1];
     uint4* table = reinterpret_cast<uint4*>(route_lds);                                    // entry, negated entry
     uint2* masks = reinterpret_cast<uint2*>(route_lds + kRouteTableBytes);                  // per u
     int* partial = reinterpret_cast<int*>(route_lds + kRouteTableBytes + kRouteMaskBytes);  // [waves][channels]
@@ -948,7 +954,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_gemv_kernel(
     const bool swiglu_rows = x16 == 2;
     constexpr int kSelected = LOCAL == 0 ? 1 : LOCAL;
     float route_logits[kSelected];
-    if (LOCAL > 0 && wave == 0) load_route_logits<kSelected>(route_logits, logits, experts, lane);
+    if (kCounts || (LOCAL > 0 && wave == 0)) load_route_logits<kSelected>(route_logits, logits, experts, lane);
     int expert = LOCAL > 0 ? 0 : ids[route];
     const uint2 entry = reinterpret_cast<const uint2*>(book)[tid & 255];
     const __half* x = reinterpret_cast<const __half*>(a) + (swiglu_rows ? (int64_t)route * 2 * k : 0);
@@ -967,7 +973,11 @@ __global__ __launch_bounds__(kRouteThreads) void route_gemv_kernel(
     if (LOCAL == 0 && (unsigned)expert >= (unsigned)experts) return;  // nothing to index: the row stays as it was
     const int row = shared_input ? 0 : route;
     const int blocks = k / 128;
-    const int channel = blockIdx.x * kRouteChannels + (lane >> 1);
+    auto channel_of = [&](int local) {
+        if (act == nullptr) return (int)blockIdx.x * kRouteChannels + local;
+        return (int)blockIdx.x * (kRouteChannels / 2) + (local & (kRouteChannels / 2 - 1)) + (local < kRouteChannels / 2 ? 0 : n / 2);
+    };
+    const int channel = channel_of(lane >> 1);
     const int half = lane & 1;
     const bool live = channel < n;
     // codes of this lane: 16 bytes per K block, K blocks wave, wave + 8, ...; the first kRouteDepth loads leave as soon as the
@@ -976,7 +986,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_gemv_kernel(
     const uint4* codes = nullptr;
     uint4 held[kRouteDepth];
     unsigned short scale_bits = 0;
-    const int out_channel = blockIdx.x * kRouteChannels + (tid & (kRouteChannels - 1));
+    const int out_channel = channel_of(tid & (kRouteChannels - 1));
     auto request_codes = [&]() {
         codes = reinterpret_cast<const uint4*>(p + (((int64_t)expert * blocks) * n + (live ? channel : 0)) * 16) + half;
 #pragma unroll
@@ -987,7 +997,12 @@ __global__ __launch_bounds__(kRouteThreads) void route_gemv_kernel(
         scale_bits = reinterpret_cast<const unsigned short*>(ws)[(int64_t)expert * n + min(out_channel, n - 1)];
     };
     if (LOCAL == 0) request_codes();
-    if (LOCAL > 0 && wave == 0)  // (one workgroup writes the probabilities)
+    if constexpr (kCounts) {
+        uint32_t counts[kSelected];
+        count_in_front<kSelected, kRouteWaves>(route_logits, counts, route_keys, experts, wave, lane);
+#pragma unroll
+        for (int j = 0; j < kSelected; ++j) reinterpret_cast<uint8_t*>(in_front + j * 64 + lane)[wave] = (uint8_t)counts[j];
+    } else if (LOCAL > 0 && wave == 0)  // (one workgroup writes the probabilities)
         select_routes<kSelected>(route_logits, selected_ids, blockIdx.x == 0 && blockIdx.y == 0 ? selected_prob : nullptr, experts,
                                  routes, renormalize, lane);
     if (tid < 256) {
@@ -1001,6 +1016,31 @@ __global__ __launch_bounds__(kRouteThreads) void route_gemv_kernel(
     // the routes are known after the next barrier (the one of the row maximum where there is one)
     auto routes_published = [&]() {
         if (LOCAL == 0) return;
+        if constexpr (kCounts) {
+            const bool writes = blockIdx.x == 0 && blockIdx.y == 0 && wave == 0;
+            int rank[kSelected];
+            expert = 0;
+#pragma unroll
+            for (int j = 0; j < kSelected; ++j) {
+                const uint2 of_waves = in_front[j * 64 + lane];
+                rank[j] = j * 64 + lane < experts ? (int)__builtin_amdgcn_udot4(of_waves.x, 0x01010101u, __builtin_amdgcn_udot4(of_waves.y, 0x01010101u, 0u, false), false) : experts;
+                const unsigned long long here = __ballot(rank[j] == route);
+                if (here != 0) expert = j * 64 + (int)__builtin_ctzll(here);
+            }
+            expert = __builtin_amdgcn_readfirstlane(expert);
+            request_codes();
+            if (writes) {  // (one wave by itself: LDS serves it in order)
+                float local_max = -INFINITY;
+#pragma unroll
+                for (int j = 0; j < kSelected; ++j) {
+                    if (rank[j] < routes) selected_keys[rank[j]] = ordered_key(route_logits[j]), const_cast<int32_t*>(ids)[rank[j]] = j * 64 + lane;
+                    if (j * 64 + lane < experts) local_max = fmaxf(local_max, route_logits[j]);
+                }
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                route_probabilities<kSelected>(route_logits, local_max, selected_keys[lane], prob, experts, routes, renormalize, lane);
+            }
+            return;
+        }
         expert = selected_ids[route];
         request_codes();
         if (blockIdx.x == 0 && blockIdx.y == 0 && tid < routes) {
@@ -1024,6 +1064,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_gemv_kernel(
                     for (int e = 0; e < 8; ++e) gate[e] = __float2half_rn(swiglu_value(gate[e], up[e]));
                 }
             }
+            if (j * kRouteThreads >= k / 8) continue;  // uniform
             const __half2* pairs = reinterpret_cast<const __half2*>(&kept[j]);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -1096,7 +1137,12 @@ __global__ __launch_bounds__(kRouteThreads) void route_gemv_kernel(
         for (int w = 0; w < kRouteWaves; ++w) total += partial[w * kRouteChannels + tid];
         const float token_scale = x16 ? row_scale : __half2float(as[row]);
         const float scaled = ((float)total * __half2float(__ushort_as_half(scale_bits))) * token_scale;
-        c[(int64_t)route * n + out_channel] = __float2half_rn(scaled);
+        const __half value = __float2half_rn(scaled);
+        c[(int64_t)route * n + out_channel] = value;
+        if (act != nullptr) {
+            const __half up = __ushort_as_half((unsigned short)__shfl_down((int)__half_as_ushort(value), kRouteChannels / 2, 64));
+            if (tid < kRouteChannels / 2) act[(int64_t)route * (n / 2) + out_channel] = __float2half_rn(swiglu_value(value, up));
+        }
     }
 }
 
@@ -1105,10 +1151,12 @@ __global__ __launch_bounds__(kRouteThreads) void route_gemv_kernel(
 // route.  Each wave turns its route's gate | up row into A8 codes in registers and leaves them in an LDS area of its own, so nothing but the
 // decode tables is waited for; the rows' fp16 results meet in LDS and are added in the order of the ranks as moe_combine
 // does.  What bounds it is a chain: ids, codes of the chosen experts (requested before the SwiGLU, which runs under their
-// way), lookups, two meetings.  One token, 8 of 128 experts, 2048 x 512: projection 5.4 us and
+// way), lookups, two meetings.  With rows that the first projection has made of gate and up already (what is above goes without the SwiGLU: the layer 11.3 -> 10.9 us).  One token, 8 of 128 experts, 2048 x 512: projection 5.4 us and
 // combine 2.4 us in two launches, 5.1 in one, the layer 13.8 -> 11.6 us (16 channels to a workgroup, half of the CUs: 12.3).
 // SwiGLU, row maximum, quantiser, dots and rescale are those of route_gemv_kernel, in its order wherever the order can be seen.
+// SWIGLU: the rows are gate | up of 2 k values; else what their projection made of them.
 constexpr int kCombineChannels = 8, kCombineMaxK = 2048, kCombineRoutes = 8;
+template <bool SWIGLU>
 __global__ __launch_bounds__(kRouteThreads) void route_combine_kernel(
     const __half* __restrict__ a, __half* __restrict__ as, const uint32_t* __restrict__ book, __half* __restrict__ c,
     const int32_t* __restrict__ ids, __half* __restrict__ output, const uint16_t* __restrict__ p, const float* __restrict__ prob,
@@ -1131,14 +1179,14 @@ __global__ __launch_bounds__(kRouteThreads) void route_combine_kernel(
     const uint2 entry = reinterpret_cast<const uint2*>(book)[tid & 255];
     const int pieces = k / 8;
     constexpr int kPieces = kCombineMaxK / 512;
-    uint4 kept[kPieces], up_kept[kPieces];
-    const __half* const row = a + (int64_t)(live_wave ? route : 0) * 2 * k;
+    uint4 kept[kPieces], up_kept[SWIGLU ? kPieces : 1];
+    const __half* const row = a + (int64_t)(live_wave ? route : 0) * (SWIGLU ? 2 : 1) * k;
 #pragma unroll
     for (int j = 0; j < kPieces; ++j) {
-        kept[j] = up_kept[j] = make_uint4(0u, 0u, 0u, 0u);
+        kept[j] = make_uint4(0u, 0u, 0u, 0u);
         if (lane + 64 * j < pieces) {
             kept[j] = reinterpret_cast<const uint4*>(row)[lane + 64 * j];
-            up_kept[j] = reinterpret_cast<const uint4*>(row + k)[lane + 64 * j];
+            if constexpr (SWIGLU) up_kept[j] = reinterpret_cast<const uint4*>(row + k)[lane + 64 * j];
         }
     }
     // scale and weight of what this thread adds at the end
@@ -1175,10 +1223,10 @@ __global__ __launch_bounds__(kRouteThreads) void route_combine_kernel(
         for (int j = 0; j < kPieces; ++j) {
             if (lane + 64 * j >= pieces) continue;
             __half* gate = reinterpret_cast<__half*>(&kept[j]);
-            const __half* up = reinterpret_cast<const __half*>(&up_kept[j]);
+            const __half* up = reinterpret_cast<const __half*>(&up_kept[SWIGLU ? j : 0]);
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                gate[e] = __float2half_rn(swiglu_value(gate[e], up[e]));
+                if constexpr (SWIGLU) gate[e] = __float2half_rn(swiglu_value(gate[e], up[e]));
                 amax = fmaxf(amax, fabsf(__half2float(gate[e])));
             }
         }
@@ -1267,27 +1315,33 @@ int route_gemv_geometry(const orx_function& f, int rows, Geometry* g) {
 int route_gemv_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t stream, void** args) {
     (void)rows;
     if (f.flags & 16) {
-        ORX_LAUNCH(route_combine_kernel, dim3(g.grid[0]), dim3(kRouteThreads), g.shared, stream, pointer_arg<const __half>(args, 0),
-                   pointer_arg<__half>(args, 1), pointer_arg<const uint32_t>(args, 2), pointer_arg<__half>(args, 3), pointer_arg<const int32_t>(args, 4),
-                   pointer_arg<__half>(args, 5), pointer_arg<const uint16_t>(args, 6), pointer_arg<const float>(args, 7), pointer_arg<const __half>(args, 8),
-                   f.E, f.M, f.N, f.K);
+#define ORX_ROUTE_COMBINE(SWIGLU)                                                                                                                                     \
+    ORX_LAUNCH(route_combine_kernel<SWIGLU>, dim3(g.grid[0]), dim3(kRouteThreads), g.shared, stream, pointer_arg<const __half>(args, 0),                              \
+               pointer_arg<__half>(args, 1), pointer_arg<const uint32_t>(args, 2), pointer_arg<__half>(args, 3), pointer_arg<const int32_t>(args, 4),                 \
+               pointer_arg<__half>(args, 5), pointer_arg<const uint16_t>(args, 6), pointer_arg<const float>(args, 7), pointer_arg<const __half>(args, 8), f.E, f.M, \
+               f.N, f.K)
+        if (f.flags & 2) ORX_ROUTE_COMBINE(true);
+        else ORX_ROUTE_COMBINE(false);
+#undef ORX_ROUTE_COMBINE
         return hip_check(hipGetLastError(), "launch integer_e8p_gemv (combine)");
     }
     const bool routing = f.flags & 4;
     const int8_t* a = pointer_arg<const int8_t>(args, 0);
     const __half* as = pointer_arg<const __half>(args, 1);
-    const uint32_t* book = pointer_arg<const uint32_t>(args, 2);
-    __half* c = pointer_arg<__half>(args, 3);
-    const int32_t* ids = pointer_arg<const int32_t>(args, 4);
-    const float* logits = routing ? pointer_arg<const float>(args, 5) : nullptr;
-    const uint16_t* p = pointer_arg<const uint16_t>(args, routing ? 6 : 5);
-    float* prob = routing ? pointer_arg<float>(args, 7) : nullptr;
-    const __half* ws = pointer_arg<const __half>(args, routing ? 8 : 6);
+    const int more = f.flags & 32 ? 1 : 0;  // Act behind AS
+    __half* act = more ? pointer_arg<__half>(args, 2) : nullptr;
+    const uint32_t* book = pointer_arg<const uint32_t>(args, 2 + more);
+    __half* c = pointer_arg<__half>(args, 3 + more);
+    const int32_t* ids = pointer_arg<const int32_t>(args, 4 + more);
+    const float* logits = routing ? pointer_arg<const float>(args, 5 + more) : nullptr;
+    const uint16_t* p = pointer_arg<const uint16_t>(args, (routing ? 6 : 5) + more);
+    float* prob = routing ? pointer_arg<float>(args, 7 + more) : nullptr;
+    const __half* ws = pointer_arg<const __half>(args, (routing ? 8 : 6) + more);
     const int x16 = f.input_f16 ? ((f.flags & 2) ? 2 : 1) : 0;
     const dim3 grid(g.grid[0], g.grid[1]), block(kRouteThreads);
 #define ORX_ROUTE_GEMV(LOCAL)                                                                                      \
     ORX_LAUNCH(route_gemv_kernel<LOCAL>, grid, block, g.shared, stream, a, as, book, c, ids, p, ws, f.E, f.N, f.K, \
-                       f.flags & 1, x16, logits, prob, (f.flags >> 3) & 1)
+                       f.flags & 1, x16, logits, prob, (f.flags >> 3) & 1, act)
     if (!routing) ORX_ROUTE_GEMV(0);
     else if (f.E <= 64) ORX_ROUTE_GEMV(1);
     else if (f.E <= 128) ORX_ROUTE_GEMV(2);
@@ -1321,8 +1375,9 @@ int make_route_gemv(const Variant& v, orx_function* f) {
     // gate|up row of 2K values per route, which becomes fp16(silu(gate) * up) and then A8 codes.
     const std::string input = v.string("input_dtype", "int8", &bad);
     const bool fused_swiglu = v.boolean("fused_swiglu", false, &bad);
+    const bool combine = v.boolean("combine", false, &bad);
     if (bad || (input != "int8" && input != "float16") || (input == "float16" && f->K > 16384) ||
-        (input == "float16" && shared_input == fused_swiglu) || (fused_swiglu && input != "float16")) {
+        (input == "float16" && shared_input == fused_swiglu && !(combine && !shared_input)) || (fused_swiglu && input != "float16")) {
         set_error("integer_e8p_gemv: input_dtype must be int8 or float16 (float16: the shared row, or with fused_swiglu "
                   "one gate|up row per route; K up to 16384)");
         return ORX_ERR_BAD_VARIANT;
@@ -1338,22 +1393,30 @@ int make_route_gemv(const Variant& v, orx_function* f) {
         return ORX_ERR_BAD_VARIANT;
     }
     if (route_logits) f->flags |= 4 | (renormalize ? 8 : 0);
-    // combine=true (with fused_swiglu): Output (1, N) fp16 is the sum of the routes' rows times Prob, in the order of the routes; C is
-    // written as well
-    const bool combine = v.boolean("combine", false, &bad);
-    if (bad || (combine && (!fused_swiglu || route_logits || f->M > kCombineRoutes || f->K > kCombineMaxK))) {
-        set_error("integer_e8p_gemv: combine needs fused_swiglu, ids that are given, up to 8 routes and K up to 2048");
+    // combine=true: Output (1, N) fp16 is the sum of the routes' rows times Prob, in the order of the routes; C is
+    // written as well.  A holds gate|up rows with fused_swiglu, else the fp16 rows that are made of them
+    if (bad || (combine && (input != "float16" || shared_input || route_logits || f->M > kCombineRoutes || f->K > kCombineMaxK))) {
+        set_error("integer_e8p_gemv: combine needs fp16 rows of their own, ids that are given, up to 8 routes and K up to 2048");
         return ORX_ERR_BAD_VARIANT;
     }
     if (combine) f->flags |= 16;
+    // epilogue=swiglu: N = gate | up; Act (routes, N/2) fp16 receives fp16(silu(gate) * up) beside C
+    const std::string epilogue = v.string("epilogue", "none", &bad);
+    if (bad || (epilogue != "none" && epilogue != "swiglu") || (epilogue == "swiglu" && (f->N % 32 || combine))) {
+        set_error("integer_e8p_gemv: epilogue is none or swiglu (N a multiple of 32, no combine)");
+        return ORX_ERR_BAD_VARIANT;
+    }
+    if (epilogue == "swiglu") f->flags |= 32;
     // 16-byte loads of A rows and P, 8-byte loads of Book
-    f->args = {{"A", ArgPointer, 16}, {"AS", ArgPointer, 2}, {"Book", ArgPointer, 8}, {"C", ArgPointer, 2}, {"IDs", ArgPointer, 4}};
+    f->args = {{"A", ArgPointer, 16}, {"AS", ArgPointer, 2}};
+    if (epilogue == "swiglu") f->args.push_back({"Act", ArgPointer, 2});
+    f->args.push_back({"Book", ArgPointer, 8}), f->args.push_back({"C", ArgPointer, 2}), f->args.push_back({"IDs", ArgPointer, 4});
     if (route_logits) f->args.push_back({"Logits", ArgPointer, 4});
     if (combine) f->args.push_back({"Output", ArgPointer, 2});
     f->args.push_back({"P", ArgPointer, 16});
     if (route_logits || combine) f->args.push_back({"Prob", ArgPointer, 4});
     f->args.push_back({"WS", ArgPointer, 2});
-    f->device_function = combine ? reinterpret_cast<const void*>(&route_combine_kernel)
+    f->device_function = combine ? (fused_swiglu ? reinterpret_cast<const void*>(&route_combine_kernel<true>) : reinterpret_cast<const void*>(&route_combine_kernel<false>))
                          : !route_logits  ? reinterpret_cast<const void*>(&route_gemv_kernel<0>)
                          : f->E <= 64  ? reinterpret_cast<const void*>(&route_gemv_kernel<1>)
                          : f->E <= 128 ? reinterpret_cast<const void*>(&route_gemv_kernel<2>)
@@ -1493,8 +1556,8 @@ int gemv_prepare_device() {
 const Registration* gemv_registrations(int* count) {
     static const Registration rows[] = {
     {"integer_e8p_gemv", make_route_gemv,
-     "E, routes, N, K, shared_input, block_n=8, input_dtype=int8|float16, fused_swiglu=false, route_logits=false, renormalize=true, combine=false",
-     "A,AS,Book,C,IDs[,Logits][,Output],P[,Prob],WS"},
+     "E, routes, N, K, shared_input, block_n=8, input_dtype=int8|float16, fused_swiglu=false, route_logits=false, renormalize=true, combine=false, epilogue=none|swiglu",
+     "A,AS[,Act],Book,C,IDs[,Logits][,Output],P[,Prob],WS"},
     };
     *count = (int)(sizeof(rows) / sizeof(rows[0]));
     return rows;

@@ -645,23 +645,31 @@ class MoeTokenLayer:
             except OrxError as error:
                 if fused or error.code != ORX_ERR_BAD_VARIANT:
                     raise
-        # Two launches where the sum over the routes joins the second projection and that is faster: 13.8 -> 11.6 us for 8 of 128
-        # experts, 2048 x 512.
-        self.k_down_combine = None
-        if self.fused and combine_pays(top_k, hidden, intermediate, torch.cuda.get_device_properties(self.w2.device).multi_processor_count):
+        # Two launches where the sum over the routes joins the second projection: 13.8 -> 11.6 us for 8 of 128 experts, 2048 x 512, and 10.9 since the first one leaves
+        # fp16(silu(gate) * up), which every workgroup of the second made again, beside gate | up.  Three launches over two (140 shapes of up to 2048 channels between): up to two workgroups to a CU
+        # 0.99-1.37, median 1.13.  `k_down_combine` names it where it also paid with the SwiGLU in front.
+        self.k_down_combine = self.k_down_act = None
+        cus = torch.cuda.get_device_properties(self.w2.device).multi_processor_count
+        pays = combine_pays(top_k, hidden, intermediate, cus)
+        if self.fused and (pays or hidden <= 16 * cus):
             try:
-                self.k_down_combine = Kernel("integer_e8p_gemv", N=hidden, K=intermediate, shared_input=False, input_dtype="float16",
-                                             fused_swiglu=True, combine=True, **routes)
+                served = dict(
+                    k_gate_up_act=Kernel("integer_e8p_gemv", N=2 * intermediate, K=hidden, shared_input=True, input_dtype="float16", route_logits=True,
+                                         renormalize=True, epilogue="swiglu", **routes),
+                    k_down_act=Kernel("integer_e8p_gemv", N=hidden, K=intermediate, shared_input=False, input_dtype="float16", combine=True, **routes))
+                vars(self).update(served)
+                self.act = torch.empty((top_k, intermediate), **f16)
+                self.k_down_combine = self.k_down_act if pays else None
             except OrxError as error:
                 if error.code != ORX_ERR_BAD_VARIANT:
                     raise
 
     def run(self, x16, logits, stream=None):
         s = current_stream() if stream is None else stream
-        if self.k_down_combine is not None:
-            self.k_gate_up_routing(stream=s, A=x16, AS=self.a_s, Book=self.book, C=self.gate_up_out, IDs=self.ids,
-                                   Logits=logits, P=self.w1, Prob=self.prob, WS=self.s1)
-            self.k_down_combine(stream=s, A=self.gate_up_out, AS=self.h_s, Book=self.book, C=self.down_out, IDs=self.ids,
+        if self.k_down_act is not None:
+            self.k_gate_up_act(stream=s, A=x16, AS=self.a_s, Act=self.act, Book=self.book, C=self.gate_up_out, IDs=self.ids,
+                               Logits=logits, P=self.w1, Prob=self.prob, WS=self.s1)
+            self.k_down_act(stream=s, A=self.act, AS=self.h_s, Book=self.book, C=self.down_out, IDs=self.ids,
                                 Output=self.out, P=self.w2, Prob=self.prob, WS=self.s2)
             return self.out
         if self.fused:

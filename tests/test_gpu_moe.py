@@ -1294,6 +1294,32 @@ def test_one_token_layer_in_three_launches_gives_the_bits_of_five(e, k, h, i):
             gu.kernel("integer_e8p_gemv", **{**dict(E=e, routes=k, N=h, K=i), **variant})
 
 
+@pytest.mark.parametrize("e,k,h,i", [(16, 2, 4096, 1536), (16, 8, 128, 128), (64, 1, 256, 640), (65, 7, 384, 384), (100, 8, 1024, 2048), (256, 5, 512, 256), (130, 8, 256, 128)])
+def test_two_launches_of_one_token_give_the_bits_of_five(e, k, h, i):
+    """Routes counted by all waves, the product of gate and up left by the first projection; ties, zeros of both signs and an infinity among the logits."""
+    c = workloads.config3(tokens=1, experts=e, top_k=k, hidden=h, intermediate=i)
+    args = (e, k, h, i, c["gate_up"], c["gate_up_scales"], c["down"], c["down_scales"])
+    five, two = programs.MoeTokenLayer(*args, fused=False), programs.MoeTokenLayer(*args)
+    assert two.k_down_act is not None
+    x, rng = gu.dev(c["x"]), np.random.default_rng(orc.SEED + e)
+    for case in range(4):
+        logits = np.array(c["logits"])
+        if case == 1:
+            logits[0, rng.permutation(e)[: e // 2]] = logits[0, e - 1]  # ties
+        if case == 2:
+            logits[0] = np.where(rng.random(e) < 0.5, 0.0, -0.0)
+        if case == 3:
+            logits[0, rng.integers(e)], logits[0, 0] = -np.inf, -3e38
+        for layer in (five, two):
+            layer.run(x, gu.dev(logits.astype(np.float32)))
+        gu.sync()
+        for name in ("ids", "prob", "a_s", "gate_up_out", "h_s", "down_out", "out"):
+            assert torch.equal(getattr(two, name), getattr(five, name)), (case, name)
+        product = torch.empty_like(two.act)
+        gu.kernel("swiglu", I=i)(X=two.gate_up_out, Y=product, rows=k)
+        assert torch.equal(two.act, product)
+
+
 # Routes to every split of the eight waves, channels that do not fill a workgroup, K of less than and more than one request of a wave.
 @pytest.mark.parametrize("routes,n,k", [(1, 20, 128), (1, 64, 2048), (2, 100, 384), (3, 256, 1536), (4, 8, 640), (5, 130, 512), (8, 1000, 2048), (7, 33, 1152)])
 def test_second_projection_of_one_token_with_the_sum_over_its_routes(routes, n, k):
