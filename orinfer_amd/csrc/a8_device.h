@@ -75,6 +75,43 @@ __device__ __forceinline__ uint32_t quantise4(const float (&value)[4], float sca
     return low | (high << 16);
 }
 
+typedef _Float16 half_pair __attribute__((ext_vector_type(2)));
+// Largest magnitude of `count` pieces of eight fp16 values.  NaN does not count: as largest and smallest value by three-operand instructions that hand a
+// NaN on, one instruction to a pair (without its sign through the maximum that drops NaN it is three), and that way only where a NaN came out.
+template <int COUNT, typename WORDS>
+__device__ __forceinline__ float largest_magnitude(const WORDS (&pieces)[COUNT]) {
+    half_pair high = {(_Float16)0.f, (_Float16)0.f}, low = high;
+#pragma unroll
+    for (int p = 0; p < COUNT; ++p)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const half_pair pair = __builtin_bit_cast(half_pair, (uint32_t)pieces[p][j]);
+            high = __builtin_elementwise_maximum(high, pair), low = __builtin_elementwise_minimum(low, pair);
+        }
+    half_pair largest = __builtin_elementwise_maximum(high, -low);
+    if (__builtin_expect(largest[0] != largest[0] || largest[1] != largest[1], 0)) {
+        largest = half_pair{(_Float16)0.f, (_Float16)0.f};
+#pragma unroll
+        for (int p = 0; p < COUNT; ++p)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) largest = __builtin_elementwise_max(largest, __builtin_bit_cast(half_pair, (uint32_t)(pieces[p][j] & 0x7FFF7FFFu)));
+    }
+    return fmaxf((float)largest[0], (float)largest[1]);
+}
+
+// The codes of such a piece.
+template <typename WORDS>
+__device__ __forceinline__ uint2 quantise_eight(const WORDS& piece, float scale, float inverse) {
+    float value[8];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const half_pair pair = __builtin_bit_cast(half_pair, (uint32_t)piece[j]);
+        value[2 * j] = (float)pair[0], value[2 * j + 1] = (float)pair[1];
+    }
+    const float low[4] = {value[0], value[1], value[2], value[3]}, high[4] = {value[4], value[5], value[6], value[7]};
+    return make_uint2(quantise4(low, scale, inverse), quantise4(high, scale, inverse));
+}
+
 // A stable sigmoid in fp32: e = exp(-|gate|), (gate >= 0 ? 1 : e) / (1 + e).
 // exp(x) = 2^whole 2^part, whole = rint(x log2 e) (the sum with 1.5 * 2^23 has it in its low bits), part = x log2 e - whole by
 // two fused multiply-adds over log2 e as a pair of fp32 numbers: |part| is at most a half, so its rounding is below that of

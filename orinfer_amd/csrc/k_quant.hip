@@ -66,7 +66,6 @@ __global__ __launch_bounds__(256) void a8_masked_kernel(const __half* __restrict
     for (int i = threadIdx.x; i < width; i += 256) q[out_base + first + i] = quantise(value(first + i), scale, inverse);
 }
 
-typedef _Float16 half_pair __attribute__((ext_vector_type(2)));
 typedef uint32_t word4 __attribute__((ext_vector_type(4)));  // eight fp16 values
 
 // Eight values of a row as the quantiser sees them (FUSED: fp16(silu(gate) * up), eight of each) and their magnitudes, as two
@@ -84,16 +83,6 @@ __device__ __forceinline__ void take_piece(word4& piece, word4 ups, half_pair& l
         largest = __builtin_elementwise_max(largest, __builtin_bit_cast(half_pair, (uint32_t)(piece[j] & 0x7FFF7FFFu)));
     }
 }
-__device__ __forceinline__ uint2 quantise_piece(word4 piece, float scale, float inverse) {
-    float value[8];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const half_pair pair = __builtin_bit_cast(half_pair, (uint32_t)piece[j]);
-        value[2 * j] = (float)pair[0], value[2 * j + 1] = (float)pair[1];
-    }
-    const float low[4] = {value[0], value[1], value[2], value[3]}, high[4] = {value[4], value[5], value[6], value[7]};
-    return make_uint2(quantise4(low, scale, inverse), quantise4(high, scale, inverse));
-}
 
 // One pass: WAVES waves hold a (row, group) in registers as 16-byte pieces of eight fp16 values, PIECES to a lane,
 // between the maximum and the codes; FUSED values are fp16(silu(gate) * up), computed once.  All loads of a wave leave
@@ -101,7 +90,8 @@ __device__ __forceinline__ uint2 quantise_piece(word4 piece, float scale, float 
 // LONG: what lies beyond the held pieces is read for the maximum and again for the codes, four pieces of a lane at a time
 // (us, against two passes with 16-byte loads, FUSED in brackets: 1 x 40960 12.7 -> 5.0 (81 -> 10.8), 2048 x 40960 77.5 -> 53.7
 // (263 -> 103), 512 x 131072 86 -> 49.5 (562 -> 115); four pieces held instead of eight: 5.9 (16.0), 59.5 (130), 52 (114)).
-// What bounds it: memory with many rows (8192 x 4096: 28.1 -> 20.7 us, 4.9 TB/s; the two-pass kernel read every row twice),
+// What bounds it: memory with many rows (8192 x 4096: 28.1 -> 20.7 us; the two-pass kernel read every row twice; 19.1 -> 17.8 us, 5.6 TB/s, with a third of
+// the instructions for the maximum and a wave's addresses, its unit and its row as scalars, and 32768 x 512 13.6 -> 11.8),
 // the vector ALU beside it in the FUSED form (8192 x 17408: 416 -> 146 us, and 141.1 -> 135.4 with a multiply-add to a code; the two-pass kernel also computed every value
 // twice), the latency of one row's loads and reductions with few (FUSED, one row of 17408: 43 -> 5.9 us).
 // PANELS (one group to a row, K a multiple of 128): the codes a second time in the order in which k_panel.hip's projection reads them, and the sum
@@ -115,16 +105,17 @@ __global__ __launch_bounds__(WAVES == 1 ? 256 : 64 * WAVES) void a8_held_kernel(
     constexpr int kLanes = 64 * WAVES, kTail = 4;
     __shared__ float scratch[WAVES];
     const int lane = WAVES == 1 ? threadIdx.x & 63 : threadIdx.x;
-    int unit = WAVES == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;  // wave-uniform
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    int unit = WAVES == 1 ? blockIdx.x * 4 + wave : blockIdx.x;
     if constexpr (PANELS) {
         // Workgroups go to the 8 XCDs in turn: the 16 rows of a panel, which share its cache lines, stay on one (a line written in pieces by all
         // of them goes to memory from each: 512 x 5120 5.7 us, 4.6 so; the row-major codes alone 3.9)
         constexpr int kTogether = WAVES == 1 ? 4 : 16;  // workgroups to a panel
         const int turn = blockIdx.x >> 3;
-        unit = (turn / kTogether * 8 + (blockIdx.x & 7)) * 16 + (WAVES == 1 ? turn % kTogether * 4 + (int)(threadIdx.x >> 6) : turn % kTogether);
+        unit = (turn / kTogether * 8 + (blockIdx.x & 7)) * 16 + (WAVES == 1 ? turn % kTogether * 4 + wave : turn % kTogether);
     }
     if (unit >= rows * groups) return;  // whole workgroups, or one wave to a unit: nothing below waits for it
-    const int row = unit / groups, g = unit % groups;
+    const int row = groups == 1 ? unit : unit / groups, g = unit - row * groups;
     const int first = g * group;
     const int width = min(group, k - first);
     const int64_t in_base = (int64_t)row * (FUSED ? 2 * k : k);
@@ -145,9 +136,11 @@ __global__ __launch_bounds__(WAVES == 1 ? 256 : 64 * WAVES) void a8_held_kernel(
             if (FUSED) up[p] = src_up[i];
         }
         half_pair largest = {(_Float16)0.f, (_Float16)0.f};
+        if (FUSED || LONG) {
 #pragma unroll
-        for (int p = 0; p < PIECES; ++p) {
-            if (lane + p * kLanes < pieces) take_piece<FUSED>(held[p], up[FUSED ? p : 0], largest);
+            for (int p = 0; p < PIECES; ++p) {
+                if (lane + p * kLanes < pieces) take_piece<FUSED>(held[p], up[FUSED ? p : 0], largest);
+            }
         }
         if (LONG) {
             for (int base = lane + PIECES * kLanes; base < pieces; base += kTail * kLanes) {
@@ -162,7 +155,8 @@ __global__ __launch_bounds__(WAVES == 1 ? 256 : 64 * WAVES) void a8_held_kernel(
                 for (int u = 0; u < kTail; ++u) take_piece<FUSED>(more[u], more_up[FUSED ? u : 0], largest);
             }
         }
-        amax = fmaxf((float)largest[0], (float)largest[1]);
+        // (a repeated last piece does not change it; computed values are compared as they come, and long rows lost 3 % to the test for a NaN)
+        amax = FUSED || LONG ? fmaxf((float)largest[0], (float)largest[1]) : largest_magnitude(held);
     } else {
         for (int i = lane; i < width; i += kLanes) amax = fmaxf(amax, fabsf(load_value<FUSED>(x, in_base, k, first + i)));
     }
@@ -185,7 +179,7 @@ __global__ __launch_bounds__(WAVES == 1 ? 256 : 64 * WAVES) void a8_held_kernel(
 #pragma unroll
         for (int p = 0; p < PIECES; ++p)
             if (lane + p * kLanes < pieces) {
-                const uint2 codes = quantise_piece(held[p], scale, inverse);
+                const uint2 codes = quantise_eight(held[p], scale, inverse);
                 dst[lane + p * kLanes] = codes;
                 if constexpr (PANELS) {
                     *reinterpret_cast<uint2*>(in_panel((lane + p * kLanes) * 8)) = codes;
@@ -206,7 +200,7 @@ __global__ __launch_bounds__(WAVES == 1 ? 256 : 64 * WAVES) void a8_held_kernel(
                     if (base + u * kLanes < pieces) {
                         half_pair unused = {(_Float16)0.f, (_Float16)0.f};
                         take_piece<FUSED>(more[u], more_up[FUSED ? u : 0], unused);
-                        dst[base + u * kLanes] = quantise_piece(more[u], scale, inverse);
+                        dst[base + u * kLanes] = quantise_eight(more[u], scale, inverse);
                     }
                 }
             }

@@ -197,6 +197,21 @@ def test_a8_of_gates_without_a_value(rows, k):
         assert np.isinf(s[2:4]).all() and (q[2:4][live[2:4]] == 0).all()
 
 
+@pytest.mark.parametrize("rows,k", [(2049, 512), (5, 8), (5, 2048), (5, 12296), (5, 32776)])
+def test_a8_largest_beside_a_nan(rows, k):
+    """The lane that holds a row's largest magnitude, a negative one, holds a NaN too (either sign, either half of a pair); rows of zeros and of NaN alone."""
+    rng = np.random.default_rng(orc.SEED + rows + k)
+    x = (rng.normal(size=(rows, k)) * 2).astype(np.float16)
+    x[:3, -1] = -77
+    x[0, -2], x[1, -3], x[2, -8] = np.nan, np.float16(-np.float32(np.nan)), np.nan
+    x[3], x[4] = -0.0, np.nan
+    q, s = (gu.host(t) for t in gu.a8(gu.dev(x)))
+    live = ~np.isnan(x)
+    wq, ws = orc.a8(np.where(live, x, np.float16(0)))
+    np.testing.assert_array_equal(s, ws)
+    np.testing.assert_array_equal(q[live], wq[live])
+
+
 def test_swiglu_rounds_as_an_unbiased_exponential_does():
     """Share of fp16 results that differ from the correctly rounded product, where the exponential's argument is large: the
     fp32 roundings alone (sigmoid within 1.6e-7, two products) cost 0.85e-4 of them there, an exponential that is off by the
