@@ -21,6 +21,9 @@
 // to 8192 in steps of 1024: sixteen waves, each loading its own codes through a register ring).
 #include <hip/hip_fp16.h>
 
+#include <type_traits>
+
+#include "a8_device.h"
 #include "e8p_device.h"
 #include "lds_asm.h"
 #include "orx_internal.h"
@@ -49,6 +52,7 @@ struct DenseParams {
     const __half* as;
     void* out;
     int n, k, stride, m, out_f32, k_major;
+    const __half* x;  // fp16 rows that the launch quantises itself (a and as are written then), or null
 };
 
 // W: waves per workgroup (K is split over them); S: 64-wide K steps per wave (K = 64 W S); CB: token
@@ -217,7 +221,13 @@ __device__ __forceinline__ void direct_load_16(const void* global, void* lds_wav
 
 // S: 64-wide K steps per decoder wave (K = 512 S); CB: token tiles of 16; KM: K-major codes (K/128
 // blocks of N rows x 64 bytes; S is even then, so a decoder wave owns whole K blocks).
-template <int S, int CB, bool KM>
+// XR: 0, or the workgroup quantises up to XR (4 or 8) fp16 rows itself.  Every decoder wave holds its K slice of them, the waves' maxima meet at the barrier that
+// the tables need anyway, and the codes are made a pair of steps at a time while the first block's lookups are on their way, through 1 KiB of LDS a
+// wave into operand order.  All workgroups make all codes, which is what bounds it: 41 k values of 8 x 5120 take the vector ALU 2 us a CU, so rows up
+// to four have a form of their own, with half of that (17408 x 5120, 4 rows, 15.7 us in the form of eight, 14.5).  Quantiser and projection -> one launch,
+// weights out of memory: 17408 x 5120 at 8 / 4 rows 17.1 / 16.6 -> 16.3 / 14.5 us, 9728 x 2560 9.4 / 9.1 -> 7.7 / 7.0, 2048 x 512 at 8 rows 4.7 -> 3.3.
+// (Codes first and then the first block, with the second block requested meanwhile: level at 8 rows, 0.3 us more at 4.)
+template <int S, int CB, bool KM, int XR = 0>
 __global__ __launch_bounds__(kSpecThreads) void dense_specialized_kernel(DenseParams p) {
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -303,15 +313,26 @@ __global__ __launch_bounds__(kSpecThreads) void dense_specialized_kernel(DensePa
         return s < 2 * kPairs ? 128 * (s >> 1) + 32 * quarter + 16 * (s & 1) : 64 * s + 16 * quarter;
     };
     v4u tokens[CB][S];
+    // X16: 64 / XR neighbouring lanes hold consecutive values of a row, 1 KiB of XR rows to a request
+    constexpr bool X16 = XR != 0;
+    constexpr int kRowLanes = X16 ? 64 / XR : 1, kHeldPieces = X16 ? (8 * S + kRowLanes - 1) / kRowLanes : 1;
+    v4u values[kHeldPieces];
+    const int own_row = lane / kRowLanes, own_piece = lane % kRowLanes;  // (a piece is eight values)
+    if constexpr (X16) {
+        const __half* row = p.x + (int64_t)min(own_row, p.m - 1) * p.k + wave * kSlice;
 #pragma unroll
-    for (int c = 0; c < CB; ++c) {
-        const int8_t* row = p.a + (int64_t)min(16 * c + column, p.m - 1) * p.k + wave * kSlice;
+        for (int i = 0; i < kHeldPieces; ++i) values[i] = *reinterpret_cast<const v4u*>(row + min(i * kRowLanes + own_piece, 8 * S - 1) * 8);
+    } else {
 #pragma unroll
-        for (int s = 0; s < S; ++s) tokens[c][s] = *reinterpret_cast<const v4u*>(row + step_offset(s));
+        for (int c = 0; c < CB; ++c) {
+            const int8_t* row = p.a + (int64_t)min(16 * c + column, p.m - 1) * p.k + wave * kSlice;
+#pragma unroll
+            for (int s = 0; s < S; ++s) tokens[c][s] = *reinterpret_cast<const v4u*>(row + step_offset(s));
+        }
     }
     const int out_channel = tid & 15, out_token = tid >> 4;  // 512 decoder threads: 32 tokens x 16 channels
     const bool finalises = out_token < p.m && out_token < 16 * CB;
-    const float token_scale = __half2float(p.as[min(out_token, p.m - 1)]);
+    float token_scale = X16 ? 0.f : __half2float(p.as[min(out_token, p.m - 1)]);
     for (int i = tid; i < rows_here; i += kDecoders * 64) scales[i] = p.ws[first_row + i];
     {
         const int entry = tid & 255;
@@ -319,7 +340,53 @@ __global__ __launch_bounds__(kSpecThreads) void dense_specialized_kernel(DensePa
         lds_asm::write_paired_entry<8>(lds, entry, wave >= 4, value);
     }
     for (int i = tid; i < 2 * kSumBuffer; i += kDecoders * 64) sums[i] = 0;
+    // X16, behind the two buffers of sums: 1 KiB a wave on the codes' way from eight lanes of a row to operand order, and every wave's maxima
+    constexpr uint32_t kStage = kSumBase + 2 * kSumBuffer * 4, kMaxima = kStage + kDecoders * 1024;
+    static_assert(kStage % 16 == 0 && kMaxima + 8 * kDecoders * 4 <= kScaleBase, "what the third buffers of the other kernel leave");
+    uint32_t* maxima = reinterpret_cast<uint32_t*>(lds + kMaxima);
+    if constexpr (X16) {
+        uint32_t key = __float_as_uint(largest_magnitude(values));
+        key = dpp_max_step<0xB1, 0xF>(key);
+        key = dpp_max_step<0x4E, 0xF>(key);
+        key = dpp_max_step<0x141, 0xF>(key);  // of eight lanes
+        if constexpr (kRowLanes == 16) key = dpp_max_step<0x140, 0xF>(key);
+        if (own_piece == 0) maxima[own_row * kDecoders + wave] = key;
+    }
     __syncthreads();
+
+    float scale = 0.f, inverse = 0.f;
+    if constexpr (X16) {
+        const v4u low = *reinterpret_cast<const v4u*>(maxima + own_row * kDecoders), high = *reinterpret_cast<const v4u*>(maxima + own_row * kDecoders + 4);
+        const uint32_t row_key = max(max(max(low.x, low.y), max(low.z, low.w)), max(max(high.x, high.y), max(high.z, high.w)));
+        const __half stored = a8_scale(__uint_as_float(row_key));
+        scale = __half2float(stored), inverse = __frcp_rn(scale);
+        if (group == 0 && wave == 0 && own_piece == 0 && own_row < p.m) const_cast<__half*>(p.as)[own_row] = stored;
+        token_scale = __shfl(scale, (out_token & (XR - 1)) * kRowLanes, 64);
+    }
+    const int writers = min((p.n + run - 1) / run, S);  // workgroups with channels
+    // X16: this wave's values of steps s and (two) s + 1 as token operands
+    auto quantise_steps = [&](int s, int two) __attribute__((always_inline)) {
+        uint8_t* stage = lds + kStage + wave * 1024;
+#pragma unroll
+        for (int i = 8 * s / kRowLanes; i < (8 * (s + two + 1) + kRowLanes - 1) / kRowLanes; ++i) {
+            const uint2 codes = quantise_eight(values[X16 ? i : 0], scale, inverse);
+            const int piece = i * kRowLanes + own_piece;
+            if (kRowLanes * kHeldPieces == 8 * S || piece < 8 * S) {
+                if (i % writers == group && own_row < p.m)  // a workgroup writes one piece of every lane
+                    *reinterpret_cast<uint2*>(const_cast<int8_t*>(p.a) + (int64_t)own_row * p.k + wave * kSlice + piece * 8) = codes;
+                // unit u of row r at (u ^ r): the units that the rows read together lie in different groups of banks
+                const int unit = (piece - 8 * s) >> 1;
+                *reinterpret_cast<uint2*>(stage + own_row * 128 + ((unit ^ own_row) << 4) + (lane & 1) * 8) = codes;
+            }
+        }
+        asm volatile("" ::: "memory");  // (a wave's LDS accesses stay in order)
+#pragma unroll
+        for (int t = 0; t <= two; ++t) {  // of this lane's K positions
+            const int unit = two ? 2 * quarter + t : quarter, row = column & (XR - 1);
+            tokens[0][s + t] = *reinterpret_cast<const v4u*>(stage + row * 128 + ((unit ^ row) << 4));
+        }
+        asm volatile("" ::: "memory");
+    };
 
     const lds_asm::WidePairedLookup tables(lane);
     // The tables start at LDS address 0 (the kernel has no static LDS), so the permuted bytes are the
@@ -356,7 +423,9 @@ __global__ __launch_bounds__(kSpecThreads) void dense_specialized_kernel(DensePa
                               : column * kPitch + wave * (kSlice / 2) + 16 * quarter;
     constexpr int kPairBytes = KM ? 1024 : 64;
 
-    for (int block = 0; block < blocks; ++block) {
+    // (X16: the first block's lookups are on their way while its tokens are made)
+    auto decode = [&](int block, auto makes_tokens) __attribute__((always_inline)) {
+        constexpr bool kMakes = decltype(makes_tokens)::value;
         const uint8_t* src = buffer(block) + lane_codes;
         v4i acc[CB];
 #pragma unroll
@@ -365,12 +434,14 @@ __global__ __launch_bounds__(kSpecThreads) void dense_specialized_kernel(DensePa
         for (int d = 0; d < kPairs; ++d) {
             const v4u pair = *reinterpret_cast<const v4u*>(src + kPairBytes * d);
             const Looked l0 = request(pair.x), l1 = request(pair.y), l2 = request(pair.z), l3 = request(pair.w);
+            if constexpr (kMakes) quantise_steps(2 * d, 1);
             multiply(acc, combine(l0), combine(l1), 2 * d);
             multiply(acc, combine(l2), combine(l3), 2 * d + 1);
         }
         if (kOdd) {
             const v2u last = *reinterpret_cast<const v2u*>(src + 32 * (S - 1) - 8 * quarter);  // lane_codes holds 16 * quarter
             const Looked l0 = request(last.x), l1 = request(last.y);
+            if constexpr (kMakes) quantise_steps(S - 1, 0);
             multiply(acc, combine(l0), combine(l1), S - 1);
         }
         int* block_sums = sums + (block & 1) * kSumBuffer;
@@ -393,9 +464,10 @@ __global__ __launch_bounds__(kSpecThreads) void dense_specialized_kernel(DensePa
             else
                 reinterpret_cast<__half*>(p.out)[index] = __float2half_rn(value);
         }
-    }
+    };
+    if constexpr (X16) decode(0, std::true_type{});
+    for (int block = X16; block < blocks; ++block) decode(block, std::false_type{});
 }
-
 
 // Channel blocks whose codes a lane holds at once: 3 (2 where the token fragments of a long K leave
 // less room); ring depths beyond that only delay the first MFMA.
@@ -443,22 +515,28 @@ bool specialized_fits(int n, int k, int packed_k) {
     return packed_k == 0 || ((packed_k == 128 || packed_k == 64) && k % 1024 == 0);
 }
 
-template <int S, int CB, bool KM>
+template <int S, int CB, bool KM, int XR = 0>
 int launch_specialized_shape(const DenseParams& p, hipStream_t stream) {
     static DeviceOnce opted_in;  // dynamic LDS above 64 KiB needs an opt-in per kernel and device
     const int ready = opted_in.run([] {
-        return hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(&dense_specialized_kernel<S, CB, KM>),
+        return hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(&dense_specialized_kernel<S, CB, KM, XR>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsLimit),
                          "hipFuncSetAttribute");
     });
     if (ready != ORX_OK) return ready;
-    ORX_LAUNCH((dense_specialized_kernel<S, CB, KM>), dim3(device_compute_units()), dim3(kSpecThreads),
+    ORX_LAUNCH((dense_specialized_kernel<S, CB, KM, XR>), dim3(device_compute_units()), dim3(kSpecThreads),
                        specialized_lds_bytes(p.n, p.k), stream, p);
     return hip_check(hipGetLastError(), "launch projection (resident, loader waves)");
 }
 
 template <int S>
 int launch_specialized(const DenseParams& p, hipStream_t stream) {
+    if (p.x != nullptr) {
+        if constexpr (S % 2 == 0) {
+            if (p.k_major) return p.m <= 4 ? launch_specialized_shape<S, 1, true, 4>(p, stream) : launch_specialized_shape<S, 1, true, 8>(p, stream);
+        }
+        return p.m <= 4 ? launch_specialized_shape<S, 1, false, 4>(p, stream) : launch_specialized_shape<S, 1, false, 8>(p, stream);
+    }
     if constexpr (S % 2 == 0) {
         if (p.k_major)
             return p.m <= 16 ? launch_specialized_shape<S, 1, true>(p, stream) : launch_specialized_shape<S, 2, true>(p, stream);
@@ -498,13 +576,18 @@ void dense_resident_geometry(int rows, int n, int k, int packed_k, Geometry* g) 
 }
 
 int dense_resident_launch(const int8_t* a, const void* w, const uint32_t* book, const __half* ws, const __half* as,
-                          void* out, int rows, int n, int k, int stride, int packed_k, bool out_f32, hipStream_t stream) {
+                          void* out, int rows, int n, int k, int stride, int packed_k, bool out_f32, hipStream_t stream, const __half* x) {
+    if (x != nullptr && (rows > 8 || !specialized_fits(n, k, packed_k))) {
+        set_error("projection (resident): fp16 rows need at most 8 of them and K a multiple of 512 up to 5120");
+        return ORX_ERR_BAD_VARIANT;
+    }
     if (rows < 1 || rows > 32 || !dense_resident_eligible(n, k, packed_k)) {
         set_error("projection (resident): needs 1..32 rows and K a multiple of 512 up to 5120 or of 1024 up to 8192");
         return ORX_ERR_BAD_VARIANT;
     }
     DenseParams p = {};
     p.a = a, p.w = reinterpret_cast<const uint8_t*>(w), p.book = book, p.ws = ws, p.as = as, p.out = out;
+    p.x = x;
     p.n = n, p.k = k, p.stride = stride, p.m = rows, p.out_f32 = out_f32, p.k_major = packed_k == 64 ? 2 : packed_k != 0;  // 1: blocks of 128, 2: blocks of 64
     if (specialized_fits(n, k, packed_k)) {
         switch (k / 512) {

@@ -48,7 +48,7 @@ bool dense_resident_eligible(int n, int k, int packed_k);
 bool dense_loader_eligible(int n, int k, int packed_k);
 void dense_resident_geometry(int rows, int n, int k, int packed_k, Geometry* g);
 int dense_resident_launch(const int8_t* a, const void* w, const uint32_t* book, const __half* ws, const __half* as,
-                          void* out, int rows, int n, int k, int stride, int packed_k, bool out_f32, hipStream_t stream);
+                          void* out, int rows, int n, int k, int stride, int packed_k, bool out_f32, hipStream_t stream, const __half* x = nullptr);
 bool runs_eligible(int codec, int rows, int n, int k);
 int runs_rounds(int codec, int rows, int n, int* tile_rows, int* run);
 void runs_geometry(int codec, int rows, int n, Geometry* g);
@@ -1451,6 +1451,17 @@ int w8_panel_launch(const orx_function& f, int rows, const Geometry& g, hipStrea
     return panel_launch(1, pointer_arg<const uint8_t>(args, 0), nullptr, pointer_arg<const void>(args, 3), nullptr, pointer_arg<const __half>(args, 4),
                         pointer_arg<const __half>(args, 2), pointer_arg<void>(args, 1), rows, f.N, f.K, f.stride, 0, f.out_f32, stream);
 }
+// quantize=true: A holds up to eight fp16 rows; their codes and scales are written to Q and AS
+int q4_rows_geometry(const orx_function& f, int rows, Geometry* g) {
+    dense_resident_geometry(rows, f.N, f.K, f.packed_k, g);
+    return ORX_OK;
+}
+int q4_rows_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t stream, void** args) {
+    (void)g;
+    return dense_resident_launch(pointer_arg<const int8_t>(args, 4), pointer_arg<const void>(args, 6), pointer_arg<const uint32_t>(args, 2), pointer_arg<const __half>(args, 5),
+                                 pointer_arg<const __half>(args, 1), pointer_arg<void>(args, 3), rows, f.N, f.K, f.stride, f.packed_k, f.out_f32, stream,
+                                 pointer_arg<const __half>(args, 0));
+}
 // panels=true of a projection: whether it is asked for; refuses what the panel kernel does not serve
 int panels_asked(const Variant& v, const orx_function& f, bool* asked) {
     bool bad = false;
@@ -1473,6 +1484,22 @@ int make_q4_projection(const Variant& v, orx_function* f) {
     int code = make_projection(v, f, kQ4);
     if (code != ORX_OK) return code;
     bool bad = false;
+    const bool quantizes = v.boolean("quantize", false, &bad);
+    if (quantizes && !bad) {
+        const bool named = v.has("input_dtype") || v.has("rotate") || v.has("codes") || v.has("panels") || v.has("workspace") || v.has("split_k") || v.has("block_m") ||
+                           v.has("gemv_passes") || v.has("decode_in_gemm");
+        if (named || v.string("algorithm", "auto", &bad) != "auto" || bad || f->capacity > 8 || !dense_loader_eligible(f->N, f->K, f->packed_k)) {
+            set_error("e8p_q4_projection: quantize=true serves up to 8 fp16 rows of codes with K a multiple of 512 (K-major: of 1024) up to 5120, algorithm auto, and no key of "
+                      "another kernel");
+            return ORX_ERR_BAD_VARIANT;
+        }
+        f->args = {{"A", ArgPointer, 16}, {"AS", ArgPointer, 2}, {"Book", ArgPointer, 4}, {"Out", ArgPointer, 2}, {"Q", ArgPointer, 8}, {"S", ArgPointer, 2}, {"W", ArgPointer, 16}};
+        if (f->dynamic_rows) f->args.push_back({"m", ArgI32, 4});
+        f->workspace_need = nullptr;
+        f->geometry = q4_rows_geometry;
+        f->launch = q4_rows_launch;
+        return ORX_OK;
+    }
     // input_dtype=float16: A is the fp16 row and AS is written, not read (the kernel quantises the row)
     const std::string input = v.string("input_dtype", "int8", &bad);
     if (bad || (input != "int8" && input != "float16")) {
@@ -2364,7 +2391,7 @@ const Registration* gemm_registrations(int* count) {
     static const Registration rows[] = {
     {"e8p_q4_projection", make_q4_projection,
      "M, N, K, dynamic_rows=false, algorithm=auto|gemv|stream|resident|wide|tall|runs|mfma, packed_k=0|64|128, output_dtype=float16|float32, "
-     "input_dtype=int8|float16, rotate=false, codes=false, panels=false, workspace=false, split_k=true, "
+     "input_dtype=int8|float16, rotate=false, codes=false, panels=false, quantize=false, workspace=false, split_k=true, "
      "output_stride=N, block_m=0|32|64|128|256, gemv_passes=0, decode_in_gemm=false",
      "A,AS,Book,Out[,Q],S[,Signs][,Sums],W[,Workspace][,m]"},
     {"int8_projection", make_w8_projection,

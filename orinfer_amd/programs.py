@@ -118,6 +118,9 @@ def split_pays(rows, n, cus):
     return 16 * rows >= 15 * 128 * -(-rows // 128) and n <= 22 * cus
 
 
+FEW_ROWS = 8  # rows that a projection of two-stage codes quantises itself
+
+
 class QuantizedLinear:
     """A8 quantiser + one projection (E8P-Q4 or W8A8) with a dynamic row count up to `capacity`."""
 
@@ -181,6 +184,16 @@ class QuantizedLinear:
             except OrxError as error:
                 if error.code != ORX_ERR_BAD_VARIANT:
                     raise
+        # two to eight rows, where the loader-wave kernel serves the shape: it quantises the fp16 rows itself.  Time against quantiser and projection, 600 shapes of 1000 to 34816
+        # channels, weights out of cache: 2 and 4 rows 0.65 (K = 512) to 0.93, 5 and 8 rows 0.68 to 0.98 (17408 x 5120 at 8 rows 17.1 -> 16.3 us, at 4 16.6 -> 14.5;
+        # 9728 x 2560 9.4 -> 7.7)
+        self.few = None
+        if codec == "q4" and algorithm == "auto" and not block_m and capacity > 1:
+            try:
+                self.few = Kernel("e8p_q4_projection", M=min(capacity, FEW_ROWS), N=self.n, K=self.k, packed_k=packed_k, dynamic_rows=True, quantize=True)
+            except OrxError as error:
+                if error.code != ORX_ERR_BAD_VARIANT:
+                    raise
         self.workspace = self.projection.workspace()
 
     def quantize(self, x16, stream=None):
@@ -219,6 +232,9 @@ class QuantizedLinear:
             self.single(stream=stream, A=x16, AS=self.a_s, Book=self.book, Out=self.out, Q=self.a_q, S=self.scales, W=self.weight)
             return self._rows(1)
         rows = x16.shape[0]
+        if 1 < rows <= FEW_ROWS and self.few is not None and x16.data_ptr() % 16 == 0:
+            self.few(stream=stream, A=x16, AS=self.a_s, Book=self.book, Out=self.out, Q=self.a_q, S=self.scales, W=self.weight, m=rows)
+            return self._rows(rows)
         if rows < len(self.over_panels) and self.over_panels[rows] and not self._row_major(rows):
             self.panel_quantizer(stream=stream, Mask=None, Panels=self.panels, Q=self.a_q, S=self.a_s, Sums=self.sums, X=x16, rows=rows)
             if self.codec == "q4":

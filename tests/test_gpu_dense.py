@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from oracle import reference as orc
-from orinfer_amd import codebook, programs, workloads
+from orinfer_amd import codebook, lib, programs, workloads
 
 from . import gpu_util as gu
 from .started_util import MID_2, MID_4, RUNS, reported, started
@@ -551,6 +551,53 @@ def test_one_row_program_gives_the_bits_of_two_launches(n, k, packed_k, single):
         assert (gu.host(linear.a_q)[1:] == 99).all()
         np.testing.assert_array_equal(gu.host(linear.a_s)[:1], a_s)
         np.testing.assert_array_equal(out, orc.project(a_q, a_s, weights, scales))
+
+
+@pytest.mark.parametrize("n,k,packed_k", [
+    (17, 512, 0), (300, 1536, 0), (4097, 2560, 0), (5, 4608, 0), (2000, 5120, 0),            # odd and even steps to a wave; fewer workgroups than steps
+    (17, 1024, 128), (4200, 3072, 128), (33, 5120, 128), (258, 2048, 64), (8448, 5120, 64)])
+@pytest.mark.parametrize("rows", [1, 2, 4, 5, 8])
+def test_few_rows_quantised_by_the_projection(rows, n, k, packed_k):
+    """One launch leaves the codes, scales and outputs of the quantiser and the projection, of rows with a NaN, an infinity and zeros too, and nothing behind its rows."""
+    rng = np.random.default_rng(orc.SEED + rows + n + k)
+    stored = torch.from_numpy(rng.integers(-(2**31), 2**31, n * k // 8).astype(np.int32)).to(gu.DEV)
+    scales = gu.dev(rng.uniform(0.005, 0.02, n).astype(np.float16))
+    x = (rng.normal(size=(rows, k)) * 3).astype(np.float16)
+    x[rows - 1, -1] = 500
+    if rows > 4:
+        x[0], x[1, k // 2], x[2, 3], x[2, -2] = 0, np.inf, np.nan, -900
+    f16 = dict(dtype=torch.float16, device=gu.DEV)
+    out, a_s, a_q = torch.full((rows + 1, n + 8), 9.0, **f16), torch.full((rows + 1,), 7.0, **f16), torch.full((rows + 1, k), 99, dtype=torch.int8, device=gu.DEV)
+    few = lib.Kernel("e8p_q4_projection", M=rows, N=n, K=k, packed_k=packed_k, output_stride=n + 8, quantize=True)
+    few(A=gu.dev(x), AS=a_s, Book=gu.book(), Out=out, Q=a_q, S=scales, W=stored)
+    want_q, want_s = gu.a8(gu.dev(x))
+    want = gu.q4_project(want_q, want_s.view(-1), stored, scales, packed_k=packed_k)
+    assert torch.equal(a_q[:rows], want_q) and torch.equal(a_s[:rows], want_s[:, 0])
+    np.testing.assert_array_equal(gu.host(out)[:rows, :n], gu.host(want))
+    assert (a_q[rows:] == 99).all() and (a_s[rows:] == 7).all() and (out[rows:] == 9).all() and (out[:, n:] == 9).all()
+
+
+@pytest.mark.parametrize("k,packed_k,served", [(1024, 128, True), (2560, 0, True), (1536, 128, False), (5632, 0, False)])
+def test_few_rows_of_a_linear(k, packed_k, served):
+    """Which rows and addresses a linear hands to the projection as they are; all of them give the bits of two launches, rows after others as well."""
+    rng = np.random.default_rng(orc.SEED + k)
+    linear = programs.QuantizedLinear("q4", rng.integers(0, 2**32, (200, k // 8), dtype=np.uint32), rng.uniform(0.005, 0.02, 200).astype(np.float16), 12, packed_k=packed_k)
+    assert (linear.few is not None) == served
+    for rows, offset in ((2, 0), (9, 0), (8, 0), (3, 1), (4, 8)):
+        x = torch.zeros(rows * k + 8, dtype=torch.float16, device=gu.DEV)[offset : offset + rows * k].view(rows, k)
+        x.copy_(torch.from_numpy((rng.normal(size=(rows, k)) * 3).astype(np.float16)))
+        got, codes, a_s = linear.run(x).clone(), linear.a_q[:rows].clone(), linear.a_s[:rows].clone()
+        want = linear.project(linear.quantize(x))
+        assert torch.equal(got, want) and torch.equal(codes, linear.a_q[:rows]) and torch.equal(a_s, linear.a_s[:rows])
+
+
+def test_quantize_is_refused_beside_keys_of_other_kernels():
+    good = dict(M=8, N=256, K=1024, quantize=True)
+    lib.Kernel("e8p_q4_projection", **good)
+    for other in (dict(M=9), dict(K=1152), dict(K=6144), dict(K=1536, packed_k=128), dict(workspace=True), dict(algorithm="runs"), dict(block_m=32), dict(panels=True),
+                  dict(input_dtype="float16"), dict(split_k=True), dict(decode_in_gemm=True), dict(quantize=3)):
+        with pytest.raises(Exception):
+            lib.Kernel("e8p_q4_projection", **{**good, **other})
 
 
 @pytest.mark.parametrize("codec", ["q4", "w8"])
