@@ -13,8 +13,8 @@ namespace orx {
 // broadcasts carry it across rows into lane 63, which is then read back as a scalar.
 template <int CTRL, int ROW_MASK>
 __device__ __forceinline__ uint32_t dpp_max_step(uint32_t v) {
-    // lanes outside ROW_MASK receive their own value back
-    return max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, ROW_MASK, 0xF, false));
+    // lanes outside ROW_MASK receive 0, which raises nothing: the move is part of the maximum then (their own value back was three instructions)
+    return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROW_MASK, 0xF, ROW_MASK == 0xF));
 }
 __device__ __forceinline__ uint32_t row_max_u32(uint32_t v) {  // over each row of 16 lanes, known to the row
     v = dpp_max_step<0xB1, 0xF>(v);      // quad_perm [1,0,3,2]

@@ -1030,14 +1030,11 @@ __global__ __launch_bounds__(kRouteThreads) void route_gemv_kernel(
             expert = __builtin_amdgcn_readfirstlane(expert);
             request_codes();
             if (writes) {  // (one wave by itself: LDS serves it in order)
-                float local_max = -INFINITY;
 #pragma unroll
-                for (int j = 0; j < kSelected; ++j) {
+                for (int j = 0; j < kSelected; ++j)
                     if (rank[j] < routes) selected_keys[rank[j]] = ordered_key(route_logits[j]), const_cast<int32_t*>(ids)[rank[j]] = j * 64 + lane;
-                    if (j * 64 + lane < experts) local_max = fmaxf(local_max, route_logits[j]);
-                }
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                route_probabilities<kSelected>(route_logits, local_max, selected_keys[lane], prob, experts, routes, renormalize, lane);
+                route_probabilities<kSelected>(route_logits, selected_keys[lane], prob, experts, routes, renormalize, lane);
             }
             return;
         }

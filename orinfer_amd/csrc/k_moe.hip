@@ -23,37 +23,28 @@ __device__ __forceinline__ void wave_quantise_row(const __half* __restrict__ x, 
                                                   __half* __restrict__ s, int row, int h, int lane) {
     constexpr int kHeldPieces = 4;  // 16-byte pieces a lane keeps in registers (the whole row up to h = 2048)
     const int pieces = h / 8;
-    const uint4* row_pieces = reinterpret_cast<const uint4*>(x + (int64_t)row * h);
-    uint4 held[kHeldPieces];
+    typedef uint32_t word4 __attribute__((ext_vector_type(4)));
+    const word4* row_pieces = reinterpret_cast<const word4*>(x + (int64_t)row * h);
+    word4 held[kHeldPieces];
 #pragma unroll
     for (int i = 0; i < kHeldPieces; ++i) held[i] = row_pieces[min(lane + 64 * i, pieces - 1)];
     // (the held pieces are counted at compile time: an array indexed by a loop's counter lives in scratch memory)
-    float amax = 0.f;
-    auto raise = [&](const uint4& raw) {
-        const __half2* pairs = reinterpret_cast<const __half2*>(&raw);
+    float amax = largest_magnitude(held);  // (repeats of the last piece among them)
+    half_pair rest = {(_Float16)0.f, (_Float16)0.f};
+    for (int at = lane + 64 * kHeldPieces; at < pieces; at += 64) {
+        const word4 more = row_pieces[at];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const float2 f = __half22float2(pairs[j]);
-            amax = fmaxf(amax, fmaxf(fabsf(f.x), fabsf(f.y)));
-        }
-    };
-#pragma unroll
-    for (int i = 0; i < kHeldPieces; ++i) raise(held[i]);  // (repeats of the last piece among them)
-    for (int at = lane + 64 * kHeldPieces; at < pieces; at += 64) raise(row_pieces[at]);
-    amax = wave_max_magnitude(amax);
+        for (int j = 0; j < 4; ++j) rest = __builtin_elementwise_max(rest, __builtin_bit_cast(half_pair, (uint32_t)(more[j] & 0x7FFF7FFFu)));
+    }
+    amax = wave_max_magnitude(fmaxf(amax, fmaxf((float)rest[0], (float)rest[1])));
     const __half stored = a8_scale(amax);
     if (lane == 0) s[row] = stored;
     const float scale = __half2float(stored), inverse = __frcp_rn(scale);
-    auto quantise = [&](const uint4& raw, int at) {
-        const __half* v = reinterpret_cast<const __half*>(&raw);
-        const float low[4] = {__half2float(v[0]), __half2float(v[1]), __half2float(v[2]), __half2float(v[3])};
-        const float high[4] = {__half2float(v[4]), __half2float(v[5]), __half2float(v[6]), __half2float(v[7])};
-        reinterpret_cast<uint2*>(q + (int64_t)row * h)[at] = make_uint2(quantise4(low, scale, inverse), quantise4(high, scale, inverse));
-    };
+    uint2* const codes = reinterpret_cast<uint2*>(q + (int64_t)row * h);
 #pragma unroll
     for (int i = 0; i < kHeldPieces; ++i)
-        if (lane + 64 * i < pieces) quantise(held[i], lane + 64 * i);
-    for (int at = lane + 64 * kHeldPieces; at < pieces; at += 64) quantise(row_pieces[at], at);
+        if (lane + 64 * i < pieces) codes[lane + 64 * i] = quantise_eight(held[i], scale, inverse);
+    for (int at = lane + 64 * kHeldPieces; at < pieces; at += 64) codes[at] = quantise_eight(row_pieces[at], scale, inverse);
 }
 
 // QUANT (quantize_hidden): four more waves per workgroup quantise the same four tokens' hidden rows
@@ -69,7 +60,7 @@ __global__ __launch_bounds__((router_threads<LOCAL, QUANT>())) void router_topk_
     int renormalize, const __half* __restrict__ x, int8_t* __restrict__ q, __half* __restrict__ s, int h, int* __restrict__ row_max) {
     constexpr bool kQuantiserWaves = router_threads<LOCAL, QUANT>() == 512;
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int row = blockIdx.x * 4 + (wave & 3);
     if (row >= m) return;
     if (kQuantiserWaves && wave >= 4) {

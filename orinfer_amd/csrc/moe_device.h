@@ -6,6 +6,7 @@
 
 #include <cmath>
 #include <cstdint>
+#include <type_traits>
 
 #include "a8_device.h"
 
@@ -21,9 +22,18 @@ __device__ __forceinline__ float key_value(uint32_t ordered) {
     return __uint_as_float((ordered & 0x80000000u) ? ordered ^ 0x80000000u : ~ordered);
 }
 
+// Sums of lanes 32, 16, 8, 4, 2 and 1 apart, in this order, by lane moves: the swap of two copies' halves (rows) puts a lane's value beside that of its
+// partner, and once all are alike 8 apart a turn by 4 within a row is the exchange.  (As shuffles, six LDS round trips one after another.)
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int offset = 32; offset > 0; offset >>= 1) v += __shfl_xor(v, offset, 64);
+    auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
+    auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(rows[0]) + __uint_as_float(rows[1]);
+    auto from = [](float x, auto control) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(control)::value, 0xF, 0xF, true)); };
+    v += from(v, std::integral_constant<int, 0x128>{});  // row_ror:8
+    v += from(v, std::integral_constant<int, 0x124>{});  // row_ror:4
+    v += from(v, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+    v += from(v, std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
     return v;
 }
 
@@ -48,10 +58,8 @@ __device__ __forceinline__ void load_route_logits(float (&values)[LOCAL], const 
 
 // What depends on the selected scores alone: lane `rank` has the key of that rank and writes prob[rank].
 template <int LOCAL>
-__device__ __forceinline__ void route_probabilities(const float (&values)[LOCAL], float local_max, uint32_t my_key, float* prob, int e, int top_k, int renormalize, int lane) {
-    float global_max = local_max;
-#pragma unroll
-    for (int offset = 32; offset > 0; offset >>= 1) global_max = fmaxf(global_max, __shfl_xor(global_max, offset, 64));
+__device__ __forceinline__ void route_probabilities(const float (&values)[LOCAL], uint32_t my_key, float* prob, int e, int top_k, int renormalize, int lane) {
+    const float global_max = key_value((uint32_t)__builtin_amdgcn_readfirstlane((int)my_key));  // of rank 0
     float all_exp = 0.f;
     if (!renormalize) {
 #pragma unroll
@@ -64,44 +72,57 @@ __device__ __forceinline__ void route_probabilities(const float (&values)[LOCAL]
     if (lane < top_k) prob[lane] = __fdiv_rn(mine, renormalize ? selected_sum : all_exp);
 }
 
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // (m0 is reserved: it holds nothing of the compiler's from one statement to the next)
 // The routes of one row, by one wave: the largest score first, the lowest id on ties.  A rank is one maximum of 32-bit keys and
 // one ballot per held key for the lowest id that has it; what depends on the score alone waits for the end.  (64-bit keys of
 // score and id, with the exponential inside the loop, took 0.3 us a rank.)  Lane `rank` writes ids[rank] and, where `prob` is
 // not null, prob[rank].
+// With many rows this is bound by its instructions: which keys are taken is kept as scalar masks, and a rank's id and key are put into their lane as
+// they are, 15 vector instructions a rank with two keys a lane instead of 45.
 template <int LOCAL>
 __device__ __forceinline__ void select_routes(const float (&values)[LOCAL], int* ids, float* prob, int e, int top_k, int renormalize,
                                               int lane) {
     uint32_t keys[LOCAL];
-    uint32_t open = 0;  // bit j: key j is there and not taken yet
-    float local_max = -INFINITY;
+    uint64_t open[LOCAL];  // lanes whose key j is there and not taken yet
 #pragma unroll
     for (int j = 0; j < LOCAL; ++j) {
         const bool live = j * 64 + lane < e;
         keys[j] = live ? ordered_key(values[j]) : 0u;
-        open |= live ? 1u << j : 0u;
-        if (live) local_max = fmaxf(local_max, values[j]);
+        open[j] = __ballot(live);
     }
-    int my_id = e;
-    uint32_t my_key = 0;  // of rank == lane
-    for (int rank = 0; rank < top_k; ++rank) {
+    uint32_t my_id = (uint32_t)e, my_key = 0;  // of rank == lane
+    const int ranks = __builtin_amdgcn_readfirstlane(top_k);
+    for (int rank = 0; rank < ranks; ++rank) {
         uint32_t best = keys[0];
 #pragma unroll
         for (int j = 1; j < LOCAL; ++j) best = max(best, keys[j]);
         best = wave_max_u32(best);
-        int id = e;  // (never more ranks than ids)
+        int chosen = -1;  // (never more ranks than ids)
+        uint64_t lowest = 0;
 #pragma unroll
         for (int j = LOCAL - 1; j >= 0; --j) {
-            const unsigned long long having = __ballot(keys[j] == best && (open >> j & 1u));
-            if (having != 0) id = j * 64 + __builtin_ctzll(having);
+            const uint64_t having = __ballot(keys[j] == best) & open[j];
+            if (having != 0) chosen = j, lowest = having;
         }
+        lowest &= 0 - lowest;
+        const uint32_t id = chosen < 0 ? (uint32_t)e : (uint32_t)(chosen * 64 + __builtin_ctzll(lowest));
 #pragma unroll
-        for (int j = 0; j < LOCAL; ++j)
-            if (j * 64 + lane == id) keys[j] = 0u, open &= ~(1u << j);
-        if (lane == rank) my_id = id, my_key = best;
+        for (int j = 0; j < LOCAL; ++j) {
+            const uint64_t taken = j == chosen ? lowest : 0;
+            open[j] &= ~taken;
+            asm("v_cndmask_b32_e64 %0, %0, 0, %1" : "+v"(keys[j]) : "s"(taken));
+        }
+        // (an instruction reads one scalar register: the lane's number goes by m0)
+        asm("s_mov_b32 m0, %4\n\ts_nop 0\n\tv_writelane_b32 %0, %2, m0\n\tv_writelane_b32 %1, %3, m0"
+            : "+v"(my_id), "+v"(my_key)
+            : "s"(id), "s"(best), "s"(__builtin_amdgcn_readfirstlane(rank))
+            : "m0");
     }
-    if (lane < top_k) ids[lane] = my_id;
-    if (prob != nullptr) route_probabilities<LOCAL>(values, local_max, my_key, prob, e, top_k, renormalize, lane);
+    if (lane < top_k) ids[lane] = (int)my_id;
+    if (prob != nullptr) route_probabilities<LOCAL>(values, my_key, prob, e, top_k, renormalize, lane);
 }
+#pragma clang diagnostic pop
 
 // The same selection by all waves of a workgroup: a wave counts, for every expert, those of its own share (kShare experts from wave * kShare on) that come in front of it, so a
 // rank is the sum over the waves and no rank waits for the one before it.  (One wave, rank after rank: the projection of one token was ready to name

@@ -1227,6 +1227,26 @@ def test_router_quantises_the_hidden_rows_in_the_same_launch(m, e, k, h):
     assert (gu.host(q)[m:] == 7).all() and (gu.host(s)[m:] == 3).all() and (gu.host(ids)[m:] == -1).all()
 
 
+@pytest.mark.parametrize("e,k,h", [(32, 32, 8), (64, 8, 2048), (96, 32, 2056), (200, 20, 4096), (1000, 32, 520)])
+def test_router_takes_all_and_alike_experts_and_rows_with_a_nan(e, k, h):
+    """Ranks down to the last expert and among few different scores; a NaN in a hidden row leaves its scale and other codes alone, in the held pieces and behind them."""
+    rng = np.random.default_rng(orc.SEED + e + h)
+    m = 9
+    logits = rng.integers(-2, 3, (m, e)).astype(np.float32)
+    x = (rng.normal(size=(m, h)) * 2).astype(np.float16)
+    x[0, 0], x[1, -1], x[2, h // 2], x[3] = np.nan, np.nan, -np.float16(np.nan), np.nan
+    ids, prob = torch.full((m, k), -1, **I32), torch.empty((m, k), dtype=torch.float32, device=gu.DEV)
+    q, s = torch.empty((m, h), dtype=torch.int8, device=gu.DEV), torch.empty(m, dtype=torch.float16, device=gu.DEV)
+    gu.kernel("router_topk", M=m, E=e, top_k=k, quantize_hidden=h)(IDs=ids, Logits=gu.dev(logits), Prob=prob, Q=q, S=s, X=gu.dev(x))
+    want_ids, want_prob = orc.router_topk(logits, k, True)
+    np.testing.assert_array_equal(gu.host(ids), want_ids)
+    np.testing.assert_allclose(gu.host(prob), want_prob, atol=2e-6, rtol=2e-5)
+    live = ~np.isnan(x)
+    wq, ws = orc.a8(np.where(live, x, np.float16(0)))
+    np.testing.assert_array_equal(gu.host(s), ws[:, 0])
+    np.testing.assert_array_equal(gu.host(q)[live], wq[live])
+
+
 def test_every_form_reports_a_thread_limit_that_holds_its_own_block():
     """`orx_query` is what an engine checks a record's block against before it accepts the record
     (backend/cuda/kernels.rs:150-170): every form's limit must hold the block its geometry asks for."""
