@@ -31,6 +31,25 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
 // of magnitudes (never NaN, never -0): their bits order as they do
 __device__ __forceinline__ float wave_max_magnitude(float v) { return __uint_as_float(wave_max_u32(__float_as_uint(v))); }
 
+// Sum over groups of LANES neighbouring lanes, known to all of them, without an LDS round trip: pairs, quads, mirrored half rows and rows of 16, then the
+// swap of two copies' rows and halves, which puts a lane's sum beside its partner's.  All lanes of the wave take part.
+template <int FIRST, int LANES>
+__device__ __forceinline__ int group_sum(int v) {  // of lanes FIRST, 2 FIRST .. LANES / 2 apart
+    if constexpr (FIRST <= 1 && LANES > 1) v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true);
+    if constexpr (FIRST <= 2 && LANES > 2) v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, true);
+    if constexpr (FIRST <= 1 && LANES > 4) v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, true);
+    if constexpr (FIRST <= 1 && LANES > 8) v += __builtin_amdgcn_update_dpp(0, v, 0x140, 0xF, 0xF, true);
+    if constexpr (FIRST <= 16 && LANES > 16) {
+        auto rows = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
+        v = (int)(rows[0] + rows[1]);
+    }
+    if constexpr (LANES > 32) {
+        auto halves = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
+        v = (int)(halves[0] + halves[1]);
+    }
+    return v;
+}
+
 // fp16 scale of a group from its largest magnitude: max(amax / 127, 2^-24), or 1 for an all-zero group.
 __device__ __forceinline__ __half a8_scale(float amax) {
     const float raw_scale = fmaxf(__fdiv_rn(amax, 127.0f), 5.9604644775390625e-08f);

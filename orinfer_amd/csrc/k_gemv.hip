@@ -131,8 +131,7 @@ __global__ __launch_bounds__(kThreads) void gemv_rowmajor_kernel(
                     partial = sdot4(v.x, 0x01010101u, partial);
                     partial = sdot4(v.y, 0x01010101u, partial);
                 }
-#pragma unroll
-                for (int offset = 32; offset > 0; offset >>= 1) partial += __shfl_xor(partial, offset, 64);
+                partial = group_sum<1, 64>(partial);
                 if (lane == 0 && partial != 0) atomicAdd(&sums[r], partial);
             }
         }
@@ -241,8 +240,7 @@ __global__ __launch_bounds__(kThreads) void gemv_rowmajor_kernel(
                 total = 2 * (16 * acc_h0[r] + acc_l0[r] + 8 * acc_v0);
             else
                 total = acc_h0[r];
-#pragma unroll
-            for (int offset = kLanesPerRow / 2; offset > 0; offset >>= 1) total += __shfl_xor(total, offset, 64);
+            total = group_sum<1, kLanesPerRow>(total);
             if (live && sub == 0 && r < m) {
                 if (CODEC == kQ4) total += 5 * sums[r];
                 if (CODEC == kQ2) total += sums[r];
@@ -698,8 +696,7 @@ __global__ __launch_bounds__(kBankedThreads) void gemv_banked_kernel(
         for (int r = 0; r < MR; ++r) {
             // w = 4*q0 + q1 = 8*v0 + 2*v1 + 5 and a = 16*hi + lo + 256*ov
             int total = 8 * (16 * acc_h0[r] + acc_l0[r] + 256 * acc_o0[r]) + 2 * (16 * acc_h1[r] + acc_l1[r] + 256 * acc_o1[r]);
-#pragma unroll
-            for (int offset = LPR / 2; offset > 0; offset >>= 1) total += __shfl_xor(total, offset, 64);
+            total = group_sum<1, LPR>(total);
             if (live && sub == 0 && r < m) {
                 total += 5 * row_sum[r];
                 const float value = rescale(total, __half2float(__ushort_as_half(ws_bits)),
@@ -1125,7 +1122,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_gemv_kernel(
             }
         }
     }
-    acc += __shfl_xor(acc, 1, 64);
+    acc = group_sum<1, 2>(acc);
     if (half == 0) partial[wave * kRouteChannels + (lane >> 1)] = acc;
     __syncthreads();
     if (tid < kRouteChannels && out_channel < n) {
@@ -1268,9 +1265,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_combine_kernel(
             }
         }
     }
-    acc += __shfl_xor(acc, 1, 64);
-    acc += __shfl_xor(acc, 16, 64);
-    acc += __shfl_xor(acc, 32, 64);
+    acc = group_sum<16, 64>(group_sum<1, 2>(acc));
     if (live_wave && lane < 16 && half == 0) partial[wave][channel] = acc;
     __syncthreads();
     if (adds) {
