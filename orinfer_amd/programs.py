@@ -383,7 +383,6 @@ class MoeLayer:
                         self.k_gate_up_routes = Kernel("e8p_decode_grouped", N=2 * intermediate, K=hidden, gather=True, epilogue="swiglu", routes=True,
                                                        top_k=top_k, **grouped)
                         self.k_router_clear = Kernel("router_topk", renormalize=True, quantize_hidden=hidden, row_max=True, **common)
-                        self.tile_units = torch.empty((self.tile_capacity, 4), **i32)
                         self.routes_inside = True
                     except OrxError as error:
                         if error.code != ORX_ERR_BAD_VARIANT:
@@ -395,9 +394,6 @@ class MoeLayer:
                                                   epilogue="swiglu", **grouped)
                 self.k_down_fused = Kernel("e8p_decode_grouped", N=hidden, K=intermediate, input_dtype="float16",
                                            tile_units=self.routes_inside, **grouped)
-                self.slot_token = torch.empty(assignments, **i32)
-                self.row_max = torch.empty(assignments, **i32)
-                self.act = torch.empty((assignments, intermediate), **f16)
                 self.fused_stages = True
             except OrxError as error:
                 self.routes_inside = False
@@ -408,28 +404,21 @@ class MoeLayer:
         #   gate_up that gathers the token rows and writes fp16(silu(gate) * up), A8, down, combine.
         # A caller who asked for the quantiser and the dispatch, or the metadata, as launches of their own gets them; `fused_stages` stays
         # true where the five launches are served too.
-        self.bulk = False
+        self.bulk, bulk_tiles, bulk_kernels = False, 0, {}
         if (fused_stages is None and not keep_intermediates and signs is None and self.fused_dispatch
                 and not one_launch_refused and packed_k == 128 and experts <= 1024 and grouped_algorithm == "auto"
                 and (not self.fused_stages and assignments >= BULK_ROWS_PER_EXPERT * experts
                      or bulk_pays(assignments, experts, hidden, intermediate, torch.cuda.get_device_properties(self.w1.device).multi_processor_count))):
             try:
-                tiles = (assignments + BULK_ROWS - 1) // BULK_ROWS + min(experts, assignments)
-                bulk = dict(rows=assignments, E=experts, tiles=tiles, block_m=BULK_ROWS, tile_units=True)
+                bulk_tiles = (assignments + BULK_ROWS - 1) // BULK_ROWS + min(experts, assignments)
+                bulk = dict(rows=assignments, E=experts, tiles=bulk_tiles, block_m=BULK_ROWS, tile_units=True)
                 # (all of them before the first is kept: the five launches have kernels of the same names)
-                served = dict(
+                bulk_kernels = dict(
                     k_router_a8=Kernel("router_topk", renormalize=True, quantize_hidden=hidden, **common),
                     k_metadata_slots=Kernel("route_metadata", block_m=BULK_ROWS, slot_maps=True, workspace=True, tile_units=True, **common),
                     k_gate_up_bulk=Kernel("e8p_decode_grouped", N=2 * intermediate, K=hidden, gather=True, epilogue="swiglu", **bulk),
                     k_act_a8=Kernel("activation_quantization", K=intermediate),
                     k_down_bulk=Kernel("e8p_decode_grouped", N=hidden, K=intermediate, **bulk))
-                vars(self).update(served)
-                self.segments = self.k_metadata_slots.workspace()
-                self.tile_units = torch.empty((tiles, 4), **i32)
-                self.slot_token = torch.empty(assignments, **i32)
-                self.act = torch.empty((assignments, intermediate), **f16)
-                if tiles > self.tile_capacity:
-                    self.tile_expert, self.tile_row = torch.empty(tiles, **i32), torch.empty(tiles, **i32)
                 self.bulk = True
             except OrxError as error:
                 if error.code != ORX_ERR_BAD_VARIANT:
@@ -453,11 +442,6 @@ class MoeLayer:
                 self.k_metadata_slots = Kernel("route_metadata", block_m=block_m, slot_maps=True, workspace=True, tile_units=True, **common)
                 self.k_gate_up_few = Kernel("e8p_decode_grouped", N=2 * intermediate, K=hidden, gather=True, epilogue="swiglu", **few)
                 self.k_down_few = Kernel("e8p_decode_grouped", N=hidden, K=intermediate, input_dtype="float16", **few)
-                self.segments = self.k_metadata_slots.workspace()
-                self.tile_units = torch.empty((self.tile_capacity, 4), **i32)
-                self.slot_token = torch.empty(assignments, **i32)
-                self.row_max = torch.empty(assignments, **i32)
-                self.act = torch.empty((assignments, intermediate), **f16)
                 self.few = True
             except OrxError as error:
                 if error.code != ORX_ERR_BAD_VARIANT:
@@ -477,17 +461,27 @@ class MoeLayer:
                         k_router_clear=Kernel("router_topk", renormalize=True, quantize_hidden=hidden, row_max=True, **common),
                         k_down_fused=Kernel("e8p_decode_grouped", N=hidden, K=intermediate, input_dtype="float16", tile_units=True, **resident))
                     vars(self).update(served)
-                    if not self.bulk:
-                        self.slot_token, self.act = torch.empty(assignments, **i32), torch.empty((assignments, intermediate), **f16)
-                        self.tile_units = torch.empty((self.tile_capacity, 4), **i32)
-                    elif self.tile_units.shape[0] < self.tile_capacity:
-                        self.tile_units = torch.empty((self.tile_capacity, 4), **i32)
-                    self.row_max = torch.empty(assignments, **i32)
                     self.routes_inside = True
                 except OrxError as error:
                     if error.code != ORX_ERR_BAD_VARIANT:
                         raise
             self.routes_first = self.routes_inside
+        # What the order that `run` takes needs between its launches, behind all decisions: orders that are served and not taken leave no buffer and no length of a list.
+        takes_bulk = self.bulk and not self.routes_first
+        if takes_bulk:
+            vars(self).update(bulk_kernels)
+        if takes_bulk or self.few or self.fused_stages or self.routes_first:
+            tiles = bulk_tiles if takes_bulk else self.tile_capacity
+            if tiles > self.tile_capacity:
+                self.tile_expert, self.tile_row = torch.empty(tiles, **i32), torch.empty(tiles, **i32)
+            if takes_bulk or self.few or self.routes_inside:
+                self.tile_units = torch.empty((tiles, 4), **i32)
+            if not takes_bulk:
+                self.row_max = torch.empty(assignments, **i32)
+            self.slot_token = torch.empty(assignments, **i32)
+            self.act = torch.empty((assignments, intermediate), **f16)
+        if takes_bulk or self.few:
+            self.segments = self.k_metadata_slots.workspace()
         # the dispatched rows and the gate | up outputs, which the orders for long prompts and for few rows do without
         self.d = self.ds = self.gate_up_out = None
         if not self.bulk and not self.few and not self.routes_first:

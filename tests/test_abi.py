@@ -553,6 +553,78 @@ def test_an_expert_layer_keeps_its_order_where_a_kernel_of_another_is_refused(mo
     assert {k.variant["block_m"] for k in launched if "block_m" in k.variant} == {32 if refused else 128}
 
 
+def expert_layer_needs(kernel):
+    """Bytes that a launch of an expert layer's kernel may touch of every buffer that its handle is given (weights, scales of weights, inputs of the layer and workspaces aside)."""
+    v, name = kernel.variant, kernel.symbol
+    get = lambda key, default=0: v.get(key, default)
+    need = {}
+    if name in ("router_topk", "route_metadata", "expert_dispatch", "moe_combine"):
+        routes, experts = v["M"] * v["top_k"], v["E"]
+        tiles = -(-routes // get("block_m", 32)) + min(experts, routes)
+        width = get("quantize_hidden") or get("H")
+        need = dict(IDs=routes * 4, Prob=routes * 4, Q=v["M"] * width, S=v["M"] * 2, Counts=experts * 4, RelativeSlot=routes * 4, RowMax=routes * 4, RowOffsets=experts * 4,
+                    SlotMap=routes * 4, SlotToken=routes * 4, TileCount=4, TileExpert=tiles * 4, TileOffsets=experts * 4, TileRow=tiles * 4, TileUnits=tiles * 16,
+                    D=routes * width, DS=routes * 2, Expert=routes * width * 2, Output=v["M"] * width * 2)
+    elif name == "e8p_decode_grouped":
+        rows, experts, tiles, swiglu = v["rows"], v["E"], v["tiles"], get("epilogue") == "swiglu"
+        need = dict(Act=rows * v["N"], C=rows * v["N"] * 2, Counts=experts * 4, IDs=rows * 4, Offsets=experts * 4, Q=rows * v["K"], RelativeSlot=rows * 4, RowMax=rows * 4,
+                    SlotMap=rows * 4, SlotToken=rows * 4, TileCount=4, TileExpert=tiles * 4, TileOffsets=experts * 4, TileRow=tiles * 4, TileUnits=tiles * 16)
+        if not get("gather"):
+            need.update(A=rows * v["K"] * (2 if get("input_dtype") == "float16" else 1), AS=rows * 2)
+        assert swiglu or "Act" not in kernel.arg_names
+    return {key: size for key, size in need.items() if key in kernel.arg_names}
+
+
+def test_every_list_of_an_expert_layer_holds_what_its_launches_may_write(monkeypatch):
+    """Layers of the whole range, whichever order they take: every buffer of a launch is as long as its handle says, where several orders are served as well."""
+    import random
+    import types
+
+    import torch
+
+    from orinfer_amd import codebook, lib, programs
+
+    rng = random.Random(1)
+    launched = []
+
+    class Recorder(lib.Kernel):
+        def workspace(self):
+            return None
+
+        def __call__(self, stream=None, **named):
+            assert set(named) == set(self.arg_names), self.symbol
+            launched.append((self, named))
+
+    on_host = types.SimpleNamespace(
+        **{name: getattr(torch, name) for name in ("int32", "int8", "float16", "float32")},
+        empty=lambda *shape, device=None, **named: torch.empty(*shape, device="meta", **named),
+        cuda=types.SimpleNamespace(get_device_properties=lambda device: types.SimpleNamespace(multi_processor_count=256)))
+    monkeypatch.setattr(programs, "torch", on_host)
+    monkeypatch.setattr(programs, "_dev", lambda array: torch.empty(1, device="meta"))
+    monkeypatch.setattr(programs, "Kernel", Recorder)
+    monkeypatch.setattr(codebook, "q2_to_k_major", lambda codes: codes)
+    spread = lambda low, high: int(round(low * (high / low) ** rng.random()))
+    layers = [(578, 32, 6, 1280, 384), (431, 16, 4, 1920, 1024), (1742, 32, 2, 1152, 384), (616, 16, 6, 1792, 384), (893, 16, 4, 1408, 512),
+              (477, 64, 2, 1024, 1024), (200, 32, 8, 1792, 768), (256, 128, 8, 2048, 512), (4096, 128, 8, 2048, 512), (20, 64, 6, 3072, 256)]
+    while len(layers) < 300:
+        experts = spread(4, 512)
+        layers.append((spread(1, 4096), experts, rng.randint(1, min(experts, 10)), 128 * spread(2, 32), 128 * spread(1, 16)))
+    orders = set()
+    for tokens, experts, top_k, hidden, inter in layers:
+        bank = np.zeros(1, np.float16)
+        layer = programs.MoeLayer(tokens, experts, top_k, hidden, inter, bank, bank, bank, bank)
+        launched.clear()
+        layer.run(None, None, stream=0)
+        orders.add((layer.fused_stages, layer.bulk, layer.few, layer.routes_first))
+        for kernel, named in launched:
+            for name, size in expert_layer_needs(kernel).items():
+                tensor = named[name]
+                assert tensor is None or tensor.numel() * tensor.element_size() >= size, ((tokens, experts, top_k, hidden, inter), kernel.symbol, name)
+        written = [k.variant for k, named in launched if "TileUnits" in named]
+        assert len({v.get("block_m", 32) for v in written}) <= 1
+    assert {(True, True, False, True), (True, True, False, False), (False, True, False, True), (True, False, False, False), (False, False, True, False)} <= orders
+
+
 @pytest.mark.parametrize("shape, pays", [  # tokens, top_k, experts, hidden, intermediate
     ((22, 1, 64, 4096, 3584), True), ((52, 1, 64, 1920, 1536), True), ((53, 1, 64, 1920, 1536), False), ((832, 1, 64, 1920, 1536), False),      # rows of all tiles together
     ((1000, 8, 128, 4096, 640), True), ((1000, 8, 128, 4096, 768), False), ((60, 8, 16, 1024, 1152), True), ((60, 8, 16, 1024, 1280), False),      # channels between

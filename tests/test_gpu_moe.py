@@ -512,7 +512,8 @@ def test_gate_up_from_routes_refuses_what_it_cannot_take():
             gu.kernel("e8p_decode_grouped", **{**good, **bad})
 
 
-@pytest.mark.parametrize("tokens,experts,top_k,hidden,inter,bulk", [(477, 64, 2, 1024, 1024, False), (200, 32, 8, 1792, 768, True), (230, 64, 6, 1152, 768, True)])
+@pytest.mark.parametrize("tokens,experts,top_k,hidden,inter,bulk", [(477, 64, 2, 1024, 1024, False), (200, 32, 8, 1792, 768, True), (230, 64, 6, 1152, 768, True),
+                                                                   (578, 32, 6, 1280, 384, True)])  # the five launches of the resident kernels are served as well
 def test_four_launches_first_give_the_bits_of_seven(tokens, experts, top_k, hidden, inter, bulk):
     """Where the seven launches were left and in front of the order for many rows, eagerly and replayed with new routing."""
     c = workloads.config3(tokens=tokens, experts=experts, top_k=top_k, hidden=hidden, intermediate=inter)
