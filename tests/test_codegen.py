@@ -3,6 +3,7 @@
 An asm statement that loads or multiplies hides its latency from the compiler, which takes the result as written at once: it could copy a
 register between the load and its wait, or a sum behind a multiply that is still on its way, and no source line would show it.  The check follows every
 path through the disassembly of the kernels built here and finds such a use, whatever compiler built them."""
+import functools
 import re
 import subprocess
 from pathlib import Path
@@ -130,6 +131,56 @@ def faults(code, targets, by_condition=False):
     return found
 
 
+SCALAR_WAIT = 2  # wait states that the compiler itself keeps between a vector instruction that writes a scalar register and one that reads it
+TO_MEMORY_WAIT = 5  # and before a memory instruction that reads it
+
+
+def scalar_registers(text):
+    found = set()
+    for name, one, low, high in re.findall(r"\b(?:(vcc)\b|s(\d+)\b|s\[(\d+):(\d+)\])", text):
+        found |= {"vcc"} if name else {int(one)} if one else set(range(int(low), int(high) + 1))
+    return found
+
+
+@functools.lru_cache(maxsize=None)
+def scalars_of(text):
+    """(scalar registers that a vector instruction writes, those that it or a memory instruction reads)."""
+    name, _, operands = text.partition(" ")
+    if name.startswith(("global_", "buffer_", "flat_", "scratch_")):
+        return set(), scalar_registers(operands)
+    if not name.startswith("v_"):
+        return set(), set()
+    parts = re.split(r",(?![^\[]*\])", operands.replace("vcc_lo", "vcc").replace("vcc_hi", "vcc"))
+    results = 2 if re.match("v_(add|sub|subrev|addc|subb|subbrev)_co_|v_div_scale|v_mad_[ui]64", name) else 1
+    writes, reads = scalar_registers(",".join(parts[:results])), scalar_registers(",".join(parts[results:]))
+    if re.match("v_div_fmas|v_cndmask_b32_(e32|dpp|sdwa)", name):
+        reads |= {"vcc"}
+    return writes, reads
+
+
+def early_scalars(code, targets):
+    """Vector and memory instructions that read a scalar register too soon behind the vector instruction that writes it, on any path.  The compiler spaces its own instructions and
+    does not look into asm statements."""
+    index, found = {address: i for i, (address, _) in enumerate(code)}, set()
+    for start, (_, writer) in enumerate(code):
+        written = scalars_of(writer.text)[0]
+        if not written:
+            continue
+        following = lambda i: ([index[targets[code[i][0]]]] if code[i][0] in targets else []) + ([i + 1] if code[i][1].name not in ("s_branch", "s_endpgm") and i + 1 < len(code) else [])
+        work = [(i, 0, written) for i in following(start)]
+        while work:
+            i, states, left = work.pop()
+            ins = code[i][1]
+            writes, reads = scalars_of(ins.text)
+            if reads & left and states < (TO_MEMORY_WAIT if ins.memory else SCALAR_WAIT):
+                found.add(f"{ins.text}: {states} wait states behind {writer.text}")
+            left = left - writes - (scalar_registers(ins.text.partition(" ")[2].partition(",")[0]) if ins.name.startswith("s_") else set())
+            states += ins.states
+            if left and states < TO_MEMORY_WAIT:
+                work.extend((next_one, states, left) for next_one in following(i))
+    return found
+
+
 @pytest.fixture(scope="module")
 def built(tmp_path_factory):
     """The code objects in the library, disassembled: {kernel: (code, targets)}."""
@@ -166,6 +217,29 @@ def test_nothing_touches_a_register_that_is_on_its_way(built, family, count):
 def test_the_walk_finds_a_use_in_front_of_its_wait(lines, found):
     code = [(4 * i, Instruction(text)) for i, text in enumerate(lines + ["s_endpgm"])]
     assert bool(faults(code, {})) == bool(faults(code, {}, True)) == found
+
+
+def test_no_instruction_reads_a_scalar_register_too_soon_behind_a_vector_instruction(built):
+    assert len(built) > 400
+    for name, (code, targets) in built.items():
+        assert not (problems := early_scalars(code, targets)), (name, sorted(problems)[:5])
+
+
+@pytest.mark.parametrize("lines, found", [
+    (["v_subb_co_u32_e64 v0, vcc, v1, v2, s[0:1]", "v_addc_co_u32_e32 v3, vcc, 0, v3, vcc"], True),
+    (["v_subb_co_u32_e64 v0, vcc, v1, v2, s[0:1]", "s_nop 1", "v_addc_co_u32_e32 v3, vcc, 0, v3, vcc"], False),
+    (["v_subb_co_u32_e64 v0, vcc, v1, v2, s[0:1]", "s_nop 0", "v_addc_co_u32_e32 v3, vcc, 0, v3, vcc"], True),
+    (["v_subb_co_u32_e64 v0, s[4:5], v1, v2, s[0:1]", "v_mov_b32_e32 v9, v8", "v_addc_co_u32_e64 v3, s[4:5], 0, v3, s[4:5]"], True),
+    (["v_subb_co_u32_e64 v0, s[4:5], v1, v2, s[0:1]", "v_subb_co_u32_e64 v0, s[6:7], v1, v4, s[2:3]", "v_mov_b32_e32 v9, v8", "v_addc_co_u32_e64 v3, s[4:5], 0, v3, s[4:5]"], False),
+    (["v_cmp_lt_u32_e64 s[4:5], v1, v2", "s_and_b64 s[4:5], s[4:5], s[6:7]", "v_cndmask_b32_e64 v0, v0, 0, s[4:5]"], False),  # a scalar instruction's result
+    (["v_cmp_lt_u32_e32 vcc, v1, v2", "v_cndmask_b32_e32 v0, v0, v3, vcc"], True),
+    (["v_readfirstlane_b32 s4, v1", "s_nop 1", "v_add_u32_e32 v0, s4, v0"], False),
+    (["v_readfirstlane_b32 s4, v1", "s_nop 3", "global_load_dword v0, v1, s[4:5]"], True),
+    (["v_readfirstlane_b32 s4, v1", "s_nop 4", "global_load_dword v0, v1, s[4:5]"], False)])
+def test_the_walk_finds_a_scalar_register_that_is_read_too_soon(lines, found):
+    code = [(4 * i, Instruction(text)) for i, text in enumerate(lines + ["s_endpgm"])]
+    assert bool(early_scalars(code, {})) == found
+    assert bool(early_scalars([(0, Instruction("s_branch"))] + [(4 * i + 4, Instruction(text)) for i, text in enumerate(lines + ["s_endpgm"])], {0: 4})) == found
 
 
 def test_the_walk_follows_a_read_around_a_loop():

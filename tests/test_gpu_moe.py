@@ -1341,6 +1341,29 @@ def test_two_launches_of_one_token_give_the_bits_of_five(e, k, h, i):
         assert torch.equal(two.act, product)
 
 
+@pytest.mark.parametrize("e,k", [(8, 8), (64, 3), (70, 8), (128, 8), (193, 7), (256, 8), (300, 5)])
+def test_routes_of_one_token_among_logits_without_a_value(e, k):
+    """A NaN ranks by its bits, the sign of it and the lowest id of equal ones included, as the router ranks it: the same experts, also where no other is left."""
+    c = workloads.config3(tokens=1, experts=e, top_k=k, hidden=128, intermediate=128)
+    args = (e, k, 128, 128, c["gate_up"], c["gate_up_scales"], c["down"], c["down_scales"])
+    five, two = programs.MoeTokenLayer(*args, fused=False), programs.MoeTokenLayer(*args)
+    assert two.k_down_act is not None
+    x, rng = gu.dev(c["x"]), np.random.default_rng(orc.SEED + e)
+    for words in ((0x7FC00000,), (0xFFC00000,), (0xFFFFFFFF,), (0x7FFFFFFF, 0x7FC00000, 0xFFFFFFFF, 0xFFC00001), (0xFFFFFFFF, 0xFFFFFFFE, 0x7F800000, 0xFF800000, 0, 0x80000000)):
+        for share in (0.1, 0.6, 1.0):
+            bits = np.array(c["logits"], np.float32).view(np.uint32)
+            at = rng.random(e) < share
+            bits[0, at] = rng.choice(np.array(words, np.uint32), int(at.sum()))
+            for layer in (five, two):
+                layer.run(x, gu.dev(bits.view(np.float32)))
+            for name in ("ids", "prob", "a_s", "gate_up_out", "h_s", "down_out", "out"):
+                got, want = getattr(two, name), getattr(five, name)
+                assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num()), (words, share, name)
+            word = np.where(bits[0] == 0x80000000, np.uint32(0), bits[0])  # (zeros of both signs are one score)
+            key = np.where(word >> 31, ~word, word | np.uint32(0x80000000)).astype(np.int64)
+            np.testing.assert_array_equal(gu.host(two.ids)[0], np.argsort(-key, kind="stable")[:k])
+
+
 # Routes to every split of the eight waves, channels that do not fill a workgroup, K of less than and more than one request of a wave.
 @pytest.mark.parametrize("routes,n,k", [(1, 20, 128), (1, 64, 2048), (2, 100, 384), (3, 256, 1536), (4, 8, 640), (5, 130, 512), (8, 1000, 2048), (7, 33, 1152)])
 def test_second_projection_of_one_token_with_the_sum_over_its_routes(routes, n, k):
