@@ -1941,7 +1941,10 @@ int grouped_arg(const orx_function& f, const char* name) {
 }
 
 int grouped_launch(const orx_function& f, int rows, const Geometry& g, hipStream_t stream, void** args) {
-    (void)rows;
+    if (grouped_from_routes(f) && rows % f.top_k) {  // (the other forms get their rows from the tile lists)
+        set_error("launch %s: %d routes are no whole number of tokens with %d routes each", f.symbol.c_str(), rows, f.top_k);
+        return ORX_ERR_ROWS;
+    }
     auto buffer = [&](const char* name) -> void* {
         const int at = grouped_arg(f, name);
         return at < 0 ? nullptr : pointer_arg<void>(args, at);
@@ -1965,7 +1968,7 @@ int grouped_launch(const orx_function& f, int rows, const Geometry& g, hipStream
     }
     if (grouped_uses_bulk(f))
         return grouped_bulk_launch(b, f.N, f.K, f.tiles, (f.flags2 & 3) == 1, (f.flags2 >> 2) == 1, grouped_bulk_narrow(f.capacity, f.E, f.N), stream);
-    if (grouped_from_routes(f)) return routed_gate_up_launch(b, f.N, f.K, f.packed_k, f.capacity, stream);
+    if (grouped_from_routes(f)) return routed_gate_up_launch(b, f.N, f.K, f.packed_k, rows, stream);
     if (grouped_uses_resident(f))
         return grouped_resident_launch(b, f.N, f.K, f.tiles, f.packed_k, f.flags2 & 3, f.flags2 >> 2, f.capacity, stream);
     GemmParams p = {};
@@ -2020,8 +2023,8 @@ int make_q2_grouped(const Variant& v, orx_function* f) {
     for (const char* hint : {"block_n", "num_stages", "stages", "group_n", "warp_decode", "split_k", "parity_xor", "warp_private"})
         v.accept(hint);
     // dynamic_rows: the reference's kernel then takes the live row count as a trailing `m` (integer_vq.py:234-258
-    // with kernels/shared/rows.py); the tile lists already bound every row these kernels touch, so `m` is taken
-    // and only checked against the capacity
+    // with kernels/shared/rows.py).  The tile lists already bound every row that the kernels touch, so `m` is only checked
+    // against the capacity, except with routes=true, which makes the lists: it reads the IDs of `m` rows
     f->dynamic_rows = v.boolean("dynamic_rows", false, &bad);
     if (bad) return ORX_ERR_BAD_VARIANT;
     const char* name = f->symbol.c_str();

@@ -503,6 +503,40 @@ def test_gate_up_from_routes(tokens, e, top_k, hidden, inter, spread, packed_k):
         assert (host[name][tiles:] == -5).all()
 
 
+@pytest.mark.parametrize("capacity,top_k,live", [(96, 4, 1), (96, 4, 31), (96, 1, 33), (96, 4, 95), (96, 4, 96), (64, 64, 20), (64, 64, 40)])  # (up to 2048 routes and above are two kernels)
+def test_gate_up_from_routes_takes_the_live_rows(capacity, top_k, live):
+    """dynamic_rows: ids, rows and scales behind the live tokens are not there for the launch, and what it leaves is that of a handle for the live rows alone."""
+    rng = np.random.default_rng(orc.SEED + capacity + top_k + live)
+    e, hidden, inter = 70, 256, 48
+    ids = np.argsort(rng.random((capacity, e)), axis=1)[:, :top_k].astype(np.int32)
+    rows, m = capacity * top_k, live * top_k
+    a_q, a_s = rng.integers(-127, 128, (capacity, hidden), dtype=np.int8), rng.uniform(0.01, 0.03, (capacity, 1)).astype(np.float16)
+    a_s[live:] = np.nan
+    codes = gu.dev(np.stack([orc.q2_pack_k128(rng.integers(0, 65536, (2 * inter, hidden // 8), dtype=np.uint16)) for _ in range(e)]))
+    ws = gu.dev((rng.uniform(0.5, 1.5, (e, 2 * inter)) * 0.05 / np.sqrt(hidden)).astype(np.float16))
+    ints = lambda *shape: torch.full(shape, -5, dtype=torch.int32, device=gu.DEV)
+    halves = lambda *shape: torch.full(shape, 55.0, dtype=torch.float16, device=gu.DEV)
+    tiles = lambda routes: -(-routes // 32) + min(e, routes)
+    variant = dict(E=e, N=2 * inter, K=hidden, block_m=32, gather=True, epilogue="swiglu", algorithm="resident", routes=True, top_k=top_k)
+    kern = gu.kernel("e8p_decode_grouped", rows=rows, tiles=tiles(rows), dynamic_rows=True, **variant)
+    assert kern.arg_names[-1] == "m"
+    left = []
+    for kernel, more in ((kern, dict(m=m)), (gu.kernel("e8p_decode_grouped", rows=m, tiles=tiles(m), **variant), {})):
+        out = dict(Act=halves(rows, inter), C=halves(rows, 2 * inter), Counts=ints(e), Offsets=ints(e), RelativeSlot=ints(rows), SlotMap=ints(rows), SlotToken=ints(rows),
+                   TileCount=ints(1), TileExpert=ints(tiles(rows)), TileOffsets=ints(e), TileRow=ints(tiles(rows)), TileUnits=ints(tiles(rows), 4),
+                   RowMax=torch.zeros(rows, dtype=torch.int32, device=gu.DEV))
+        args = dict(A=gu.dev(a_q), AS=gu.dev(a_s), Book=gu.book(), IDs=gu.dev(ids), P=codes, WS=ws, **out, **more)
+        kernel(**args)
+        left.append(out)
+    np.testing.assert_array_equal(gu.host(left[0]["Counts"]), np.bincount(ids[:live].ravel(), minlength=e))
+    for name, value in left[0].items():
+        assert torch.equal(value, left[1][name]), name
+    assert bool((left[0]["Act"][m:] == 55).all()) and bool((left[0]["SlotMap"][m:] == -5).all()) and not left[0]["RowMax"][m:].any()
+    for bad in (0, rows + top_k) + ((m - 1,) if top_k > 1 else ()):
+        with pytest.raises(gu.lib.OrxError):
+            kern(**{**args, "m": bad})
+
+
 def test_gate_up_from_routes_refuses_what_it_cannot_take():
     good = dict(rows=64, E=8, tiles=10, N=64, K=256, block_m=32, gather=True, epilogue="swiglu", algorithm="resident", routes=True, top_k=4)
     gu.kernel("e8p_decode_grouped", **good)
