@@ -2045,9 +2045,10 @@ int make_q2_grouped(const Variant& v, orx_function* f) {
     }
     f->flags2 = (input == "float16" ? 2 : routes ? 3 : gather ? 1 : 0) + (epilogue == "swiglu" ? 4 : 0);
     // routes=true: nobody has listed the tiles; the launch reads the IDs of all rows (top_k to a token, rows of them) and leaves the metadata for those behind it
-    if (routes && (input != "int8" || !gather || epilogue != "swiglu" || f->block_m != 32 || f->E > 1024 || f->top_k <= 0 || f->top_k > 64 || f->M % f->top_k ||
-                   f->tiles < (f->M + 31) / 32 + std::min(f->E, f->M))) {
-        set_error("%s: routes=true goes with gather=true, epilogue=swiglu, block_m=32, up to 1024 experts and 64 routes to a token, and tiles for all of them", name);
+    if (routes && (input != "int8" || !gather || epilogue != "swiglu" || f->top_k <= 0 || f->top_k > 64 || f->M % f->top_k || f->tiles < (f->M + 31) / 32 + std::min(f->E, f->M) ||
+                   !routed_gate_up_eligible(f->N, f->K, f->block_m, f->E, f->M))) {
+        set_error("%s: routes=true goes with gather=true, epilogue=swiglu, block_m=32, up to 512 experts, 4096 routes and 64 of them to a token, tiles for all of them, N a multiple of 32 "
+                  "and K one of 128 from 256 on whose rows fit LDS", name);
         return ORX_ERR_BAD_VARIANT;
     }
     if (grouped_algorithm != "auto" && grouped_algorithm != "mfma" && grouped_algorithm != "stream" &&
@@ -2112,8 +2113,7 @@ int make_q2_grouped(const Variant& v, orx_function* f) {
     }
     if (f->flags2 != 0 && !bulk) {
         if ((f->algorithm != kAuto && f->algorithm != kResident) ||
-            !(routes ? routed_gate_up_eligible(f->N, f->K, f->block_m, f->E, f->M)
-                     : grouped_resident_eligible(f->N, f->K, f->block_m, f->tiles, f->flags2 & 3, f->flags2 >> 2, f->capacity)) ||
+            (!routes && !grouped_resident_eligible(f->N, f->K, f->block_m, f->tiles, f->flags2 & 3, f->flags2 >> 2, f->capacity)) ||
             (f->algorithm == kAuto && !grouped_resident_preferred(f->capacity, f->E, f->N))) {
             set_error("%s: gather, epilogue=swiglu and input_dtype=float16 are forms of the resident kernel (block_m=32, "
                       "gathered slots that fit LDS beside the staged rows, K <= 1024 for float16 rows) where the routed rows fill the chip", name);

@@ -553,6 +553,15 @@ def test_an_expert_layer_keeps_its_order_where_a_kernel_of_another_is_refused(mo
     assert {k.variant["block_m"] for k in launched if "block_m" in k.variant} == {32 if refused else 128}
 
 
+@pytest.mark.parametrize("bad", [dict(E=513, tiles=515), dict(E=1024, tiles=1026), dict(rows=4100, tiles=137), dict(K=2944), dict(K=128), dict(N=48), dict(top_k=65), dict(top_k=3)])
+def test_projections_from_routes_say_what_they_serve(bad):
+    good = dict(rows=64, E=8, tiles=10, N=64, K=256, block_m=32, gather=True, epilogue="swiglu", algorithm="resident", routes=True, top_k=4)
+    lib.Kernel("e8p_decode_grouped", **good)
+    with pytest.raises(lib.OrxError) as err:
+        lib.Kernel("e8p_decode_grouped", **{**good, **bad})
+    assert err.value.code == lib.ORX_ERR_BAD_VARIANT and "up to 512 experts, 4096 routes" in str(err.value)
+
+
 def expert_layer_needs(kernel):
     """Bytes that a launch of an expert layer's kernel may touch of every buffer that its handle is given (weights, scales of weights, inputs of the layer and workspaces aside)."""
     v, name = kernel.variant, kernel.symbol
