@@ -121,8 +121,7 @@ __global__ __launch_bounds__(kThreads) void grouped_resident_kernel(GroupedParam
     // channels a unit covers: 512 outputs, or 256 gate + the 256 matching up channels
     const int inner = p.n / 2;  // kEpilogueSwiglu: N = gate | up
     const int spans = EPILOGUE == kEpilogueSwiglu ? (inner + kSpan / 2 - 1) / (kSpan / 2) : (p.n + kSpan - 1) / kSpan;
-    const int groups = (int)gridDim.x;  // each XCD gets a stretch of neighbours: tiles of one expert meet in one L2
-    const int group = groups % 8 == 0 ? ((int)blockIdx.x % 8) * (groups / 8) + (int)blockIdx.x / 8 : (int)blockIdx.x;
+    const int groups = (int)gridDim.x;
     const Split split = phase_two_split(kb_count);
     // forms without a phase two (see below) have no sum blocks, and the staged rows start where those would
     constexpr bool kPhaseTwo = INPUT != kInputAct && EPILOGUE == kEpiloguePlain;
@@ -181,6 +180,11 @@ __global__ __launch_bounds__(kThreads) void grouped_resident_kernel(GroupedParam
     // a run mostly stays inside one tile and its staged rows are reused.
     const int units = tile_count * spans;
     const int full = units / groups;
+    // Each XCD gets a stretch of neighbours: tiles of one expert meet in one L2 (layer, workgroups in turn over the XCDs -> stretches: 700 tokens of 512 x 8, 2048 x 256 81.2 -> 79.4 us, 100 of
+    // 128 x 8, 2048 x 512 38.9 -> 38.1, 256 and 500 of these within 0.5 %; in seven launches 600 of 256 x 8 101.9 -> 100.2).  Fewer units than workgroups, and the split rest, would leave whole XCDs without
+    // work that way (seven launches, 60 tokens of 128 x 8, 1536 x 384 37.3 us in turn, 37.9 in stretches); the forms without a split rest were level there.
+    const bool spread = groups % 8 != 0 || (kPhaseTwo && full == 0);
+    const int group = spread ? (int)blockIdx.x : ((int)blockIdx.x % 8) * (groups / 8) + (int)blockIdx.x / 8;
     int leftover = units - full * groups;
     const int passes = (leftover * kWaves + groups * split.per_pass - 1) / (groups * split.per_pass);
     int my_units = full, first_unit = group * full;
@@ -396,7 +400,7 @@ __global__ __launch_bounds__(kThreads) void grouped_resident_kernel(GroupedParam
     };
     auto piece_of = [&](int pass) {
         Piece piece = {0, 0, 0, {0, 0, 0}, false};
-        const int block = (pass * groups + group) * split.per_pass + local;
+        const int block = (pass * groups + (int)blockIdx.x) * split.per_pass + local;
         if (local < split.per_pass && block < blocks) {
             const int unit = first_leftover + block / kWaves;
             const int tile = unit / spans;
@@ -498,8 +502,8 @@ __global__ __launch_bounds__(kThreads) void grouped_resident_kernel(GroupedParam
     // ---- phase two: the rest, 32-channel blocks split over K between waves ----------------------
     if (leftover == 0) return;
     const bool early_loaded = my_units > 0 && unit_at(my_units - 1).rows > 0;
-    for (int pass = 0; (pass * groups + group) * split.per_pass < blocks; ++pass) {
-        const int first_block = (pass * groups + group) * split.per_pass;
+    for (int pass = 0; (pass * groups + (int)blockIdx.x) * split.per_pass < blocks; ++pass) {
+        const int first_block = (pass * groups + (int)blockIdx.x) * split.per_pass;
         if (pass > 0) {
             __syncthreads();  // the previous pass's sums have been read
             for (int i = tid; i < split.per_pass * kSumBlock; i += kThreads) sums[i] = 0;
