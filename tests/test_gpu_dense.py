@@ -577,6 +577,23 @@ def test_few_rows_quantised_by_the_projection(rows, n, k, packed_k):
     assert (a_q[rows:] == 99).all() and (a_s[rows:] == 7).all() and (out[rows:] == 9).all() and (out[:, n:] == 9).all()
 
 
+@pytest.mark.parametrize("rows,n,k,packed_k", [(1, 40, 512, 0), (3, 300, 2560, 0), (4, 17, 1024, 128), (5, 272, 3072, 64), (8, 1000, 5120, 128), (7, 33, 4608, 0)])
+def test_few_rows_quantised_by_the_projection_against_the_oracle(rows, n, k, packed_k):
+    rng = np.random.default_rng(orc.SEED + rows + k)
+    packed = rng.integers(0, 2**32, (n, k // 8), dtype=np.uint32)
+    scales = rng.uniform(0.005, 0.02, n).astype(np.float16)
+    x = (rng.normal(size=(rows, k)) * np.where(rng.random((1, k)) < 0.01, 40, 1)).astype(np.float16)
+    x[0, :64] = 0
+    f16 = dict(dtype=torch.float16, device=gu.DEV)
+    out, a_s, a_q = torch.empty((rows, n), **f16), torch.empty(rows, **f16), torch.empty((rows, k), dtype=torch.int8, device=gu.DEV)
+    lib.Kernel("e8p_q4_projection", M=rows, N=n, K=k, packed_k=packed_k, quantize=True)(
+        A=gu.dev(x), AS=a_s, Book=gu.book(), Out=out, Q=a_q, S=gu.dev(scales), W=gu.dev((orc.q4_pack_k(packed, packed_k) if packed_k else packed).view(np.int32)))
+    want_q, want_s = orc.a8(x)
+    np.testing.assert_array_equal(gu.host(a_q), want_q)
+    np.testing.assert_array_equal(gu.host(a_s), want_s[:, 0])
+    np.testing.assert_array_equal(gu.host(out), orc.project(want_q, want_s, orc.q4_integers(packed, TABLE), scales))
+
+
 @pytest.mark.parametrize("k,packed_k,served", [(1024, 128, True), (2560, 0, True), (1536, 128, False), (5632, 0, False)])
 def test_few_rows_of_a_linear(k, packed_k, served):
     """Which rows and addresses a linear hands to the projection as they are; all of them give the bits of two launches, rows after others as well."""

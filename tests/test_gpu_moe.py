@@ -1375,6 +1375,24 @@ def test_two_launches_of_one_token_give_the_bits_of_five(e, k, h, i):
         assert torch.equal(two.act, product)
 
 
+@pytest.mark.parametrize("e,k,h,i,launches", [(16, 2, 4096, 1536, 2), (16, 2, 8192, 1536, 3), (16, 8, 4224, 1152, 3), (16, 3, 8192, 512, 2), (16, 9, 1024, 256, 3), (16, 4, 1024, 2176, 3)])
+def test_launches_of_one_token_by_its_shape(monkeypatch, e, k, h, i, launches):
+    """Two launches up to 16 channels to a CU and where the sum over the routes paid on its own, three where it does not or is not served; the bits of five."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("lines drawn for 256 CUs")
+    c = workloads.config3(tokens=1, experts=e, top_k=k, hidden=h, intermediate=i)
+    args = (e, k, h, i, c["gate_up"], c["gate_up_scales"], c["down"], c["down_scales"])
+    five, layer = programs.MoeTokenLayer(*args, fused=False), programs.MoeTokenLayer(*args)
+    x, logits, started = gu.dev(c["x"]), gu.dev(c["logits"]), []
+    five.run(x, logits)
+    enqueue = programs.Kernel.__call__
+    monkeypatch.setattr(programs.Kernel, "__call__", lambda self, stream=None, **named: (started.append(self.symbol), enqueue(self, stream, **named))[1])
+    layer.run(x, logits)
+    assert len(started) == launches
+    for name in ("ids", "prob", "a_s", "gate_up_out", "h_s", "down_out", "out"):
+        assert torch.equal(getattr(layer, name), getattr(five, name)), name
+
+
 @pytest.mark.parametrize("e,k", [(8, 8), (64, 3), (70, 8), (128, 8), (193, 7), (256, 8), (300, 5)])
 def test_routes_of_one_token_among_logits_without_a_value(e, k):
     """A NaN ranks by its bits, the sign of it and the lowest id of equal ones included, as the router ranks it: the same experts, also where no other is left."""
