@@ -739,8 +739,9 @@ int gemv_geometry(const orx_function& f, int rows, Geometry* g) {
     if (use_banked(f, mr)) {
         const uint32_t lanes_per_row = ((uint32_t)f.slots >> 8) & (uint32_t)(kKMajorLayout - 1);
         const uint32_t tasks = ceil_div((uint32_t)f.N, 64u / lanes_per_row);
-        // every CU gets a workgroup as soon as there is a task for each: a small matrix then runs with
-        // some idle waves per CU rather than with idle CUs
+        // Every CU gets a workgroup as soon as the reported lanes make a task for each: a small matrix then runs with
+        // some idle waves per CU rather than with idle CUs.  (A launch of one row with other lanes keeps this grid: with 32 lanes instead
+        // of 16 a workgroup has two tasks below four channels to a CU, with fewer lanes than reported some have none.)
         g->grid[0] = std::min<uint32_t>((uint32_t)device_cus(), tasks);
         g->block[0] = kBankedThreads;
         g->shared = banked_lds_bytes(f, mr);

@@ -48,10 +48,11 @@ constexpr int kDepth = 2;                       // pairs of K blocks whose codes
 constexpr int kRowPad = 16;
 constexpr int kMaxExperts = 512;
 constexpr uint32_t kLdsLimit = 160 * 1024;
-// LDS: 256 entries x (16 copies of basis, 16 of mask) x 8 bytes; scales of the tile's rows; the waves' matches; the routes of the tile's rows; the staged rows, which lie
-// where the experts' counts were
+// LDS: 256 entries x (16 copies of basis, 16 of mask) x 8 bytes; scales of the tile's rows; the waves' matches; the routes of the tile's rows; the experts' counts, which
+// are read again for every tile above 128 experts; the staged rows behind them
 constexpr uint32_t kRowScale = 65536, kMatches = kRowScale + kRows * 4, kTileRoutes = kMatches + kWaves * 16, kCounts = kTileRoutes + kRows * 2,
                    kStaged = kCounts + kMaxExperts * 4;
+static_assert(kMatches % 16 == 0 && kStaged % 16 == 0, "whole requests, and pairs of words for the matches");
 
 struct RoutedParams {
     const int8_t* a;       // (tokens, K)

@@ -596,8 +596,8 @@ class MoeLayer:
 
 
 def combine_pays(routes, hidden, intermediate, cus):
-    """Whether the second projection of one token with the sum over its routes is faster than projection and sum in two launches (time of the layer, one over
-    two; 256 CUs).  Every workgroup of 8 channels makes the codes of all routes itself, in turns of 512 values, and one route's are a wave's.
+    """Whether the second projection of one token with the SwiGLU in front and the sum over its routes behind is faster than projection and sum in two launches (time of the layer, one over
+    two; 256 CUs; without the SwiGLU it also is where `MoeTokenLayer` says).  Every workgroup of 8 channels makes the codes of all routes itself, in turns of 512 values, and one route's are a wave's.
     Up to 512 values 0.78-0.97, with three workgroups to a CU 1.06-1.09 up to two routes and 0.79-0.96 above.  Up to 1024: one workgroup to a CU 0.92-0.98 up to four routes
     and 0.92-0.96 above (up to half of the CUs 1.0-1.03); two and three to a CU 0.98-1.22 up to four routes, 0.89-0.99 above.  Beyond mostly 1.0-1.33 (0.97 at best, 8 routes of
     4096 x 1536)."""
