@@ -446,7 +446,7 @@ class MoeLayer:
             except OrxError as error:
                 if error.code != ORX_ERR_BAD_VARIANT:
                     raise
-        # The four launches also where nothing but the seven is left (1.12-1.28 times as fast, 5 layers), and over the order for many rows where they are the faster ones.  `bulk` says that that
+        # The four launches also where nothing but the seven is left (1.06-1.28 times as fast, 11 layers), and over the order for many rows where they are the faster ones.  `bulk` says that that
         # one is served and would run; `routes_first` that these run before either.
         self.routes_first = False
         if (fused_stages is None and not self.few and not keep_intermediates and signs is None and self.fused_dispatch and fused_metadata and fused_metadata_asked is None
